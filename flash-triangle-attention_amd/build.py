@@ -15,10 +15,14 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "libfta.so")
 SOURCES = ["fta_api.hip", "fta_fwd.hip", "fta_fwd1.hip", "fta_fwd2.hip", "fta_fwd_feat.hip", "fta_bwd.hip", "fta_bwd_feat.hip", "fta_bwd_dq1.hip",
-           "fta_bwd_dkdv1.hip"]
+           "fta_bwd_dkdv1.hip", "fta_block.hip"]
 
 DEMO_SOURCE = "fta_c_demo.cpp"
 DEMO = os.path.join(HERE, "fta_c_demo")
+
+# the C++ host path between torch and the library: a Python extension module
+NATIVE_SOURCE = "fta_torch.cpp"
+NATIVE = os.path.join(HERE, "fta_native.so")
 
 OBJDIR = os.path.join(HERE, "build")
 
@@ -31,11 +35,30 @@ FLAGS = [
 
 
 def needs_build() -> bool:
-    if not os.path.exists(LIB) or not os.path.exists(DEMO):
+    if not os.path.exists(LIB) or not os.path.exists(DEMO) or not os.path.exists(NATIVE):
         return True
-    t = os.path.getmtime(LIB)
+    t = min(os.path.getmtime(LIB), os.path.getmtime(NATIVE))
     deps = [os.path.join(CSRC, f) for f in os.listdir(CSRC)] + [os.path.join(INCLUDE, "fta.h")]
     return any(os.path.getmtime(d) > t for d in deps)
+
+
+def native_commands(hipcc: str, obj: str) -> tuple[list, list]:
+    """Compile and link commands of the extension module (host code only)."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"], os.path.join(os.path.dirname(os.path.dirname(hipcc)), "include"), INCLUDE]
+    compile_cmd = [hipcc, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=fta_native",
+                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-everything"]
+    for d in inc:
+        compile_cmd += ["-I", d]
+    compile_cmd += ["-c", os.path.join(CSRC, NATIVE_SOURCE), "-o", obj]
+    lib = os.path.join(root, "lib")
+    link_cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", NATIVE, obj, "-L", HERE, "-lfta", "-L", lib, "-lc10", "-lc10_hip", "-ltorch",
+                "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN", "-Wl,--no-as-needed"]
+    return compile_cmd, link_cmd
 
 
 def build(force: bool = True, verbose: bool = False) -> str:
@@ -49,6 +72,9 @@ def build(force: bool = True, verbose: bool = False) -> str:
     if verbose:
         for c in cmds:
             print(" ".join(c))
+    native_obj = os.path.join(OBJDIR, "fta_torch.o")
+    native_compile, native_link = native_commands(hipcc, native_obj)
+    cmds.append(native_compile)
     procs = [subprocess.Popen(c, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True) for c in cmds]
     failed = False
     for pr in procs:
@@ -65,6 +91,10 @@ def build(force: bool = True, verbose: bool = False) -> str:
     if res.returncode != 0:
         sys.stderr.write(res.stdout + res.stderr)
         raise RuntimeError("hipcc failed linking libfta.so")
+    res = subprocess.run(native_link, capture_output=True, text=True)
+    if res.returncode != 0:
+        sys.stderr.write(res.stdout + res.stderr)
+        raise RuntimeError("linking fta_native.so failed")
     # the C-ABI demo: a plain C++ program (HIP runtime only) linked against the library next to it
     demo = [hipcc, "--offload-arch=gfx950", "-O2", "-std=c++17", "-Wno-unused-command-line-argument", "-I", INCLUDE,
             os.path.join(CSRC, DEMO_SOURCE), "-o", DEMO, "-L", HERE, "-lfta", "-Wl,-rpath,$ORIGIN"]

@@ -46,6 +46,22 @@ hipError_t ensure_dynamic_lds(const void* kern, size_t smem) {
   return e;
 }
 
+// The kernels are gfx950 code objects: anything else cannot run them.  Checked once per device.
+int check_device() {
+  static std::atomic<int> state[64];  // 0 unknown, 1 usable, 2 not usable
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return FTA_ERR_NO_DEVICE; }
+  if (dev < 0 || dev >= 64) return FTA_OK;
+  int st = state[dev].load(std::memory_order_relaxed);
+  if (st == 0) {
+    hipDeviceProp_t prop;
+    if (hipGetDeviceProperties(&prop, dev) != hipSuccess) { (void)hipGetLastError(); return FTA_ERR_NO_DEVICE; }
+    st = (strncmp(prop.gcnArchName, "gfx950", 6) == 0) ? 1 : 2;
+    state[dev].store(st, std::memory_order_relaxed);
+  }
+  return (st == 1) ? FTA_OK : FTA_ERR_NO_DEVICE;
+}
+
 }  // namespace fta
 
 // Scratch of fta_bwd_noalloc: one copy per device, inside the code object's own data segment, held
@@ -194,22 +210,6 @@ int bwd_level(const Opts& opt, int B, int H, int L1, int L2, int D, float sm_sca
   return opt.feat;
 }
 
-// The kernels are gfx950 code objects: anything else cannot run them.  Checked once per device.
-int check_device() {
-  static std::atomic<int> state[64];  // 0 unknown, 1 usable, 2 not usable
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) { (void)hipGetLastError(); return FTA_ERR_NO_DEVICE; }
-  if (dev < 0 || dev >= 64) return FTA_OK;
-  int st = state[dev].load(std::memory_order_relaxed);
-  if (st == 0) {
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, dev) != hipSuccess) { (void)hipGetLastError(); return FTA_ERR_NO_DEVICE; }
-    st = (strncmp(prop.gcnArchName, "gfx950", 6) == 0) ? 1 : 2;
-    state[dev].store(st, std::memory_order_relaxed);
-  }
-  return (st == 1) ? FTA_OK : FTA_ERR_NO_DEVICE;
-}
-
 int check_dims(int B, int H, int L1, int L2, int D, float sm_scale) {
   if (D != 32 && D != 64) return FTA_ERR_HEAD_DIM;
   if (B < 1 || H < 1) return FTA_ERR_BATCH;
@@ -316,6 +316,7 @@ const char* fta_strerror(int status) {
     case FTA_ERR_NO_DEVICE: return "no usable gfx950 device";
     case FTA_ERR_DTYPE: return "fta_options.dtype is neither FTA_DTYPE_F16 nor FTA_DTYPE_BF16";
     case FTA_ERR_DROPOUT: return "fta_options.dropout_p must be in [0, 1)";
+    case FTA_ERR_BLOCK_SHAPE: return "fta_block needs C and H*D of 64 or 128";
     case FTA_ERR_STATIC_WORKSPACE: return "these sizes need more scratch than the built-in buffer of fta_bwd_noalloc holds (FTA_STATIC_WORKSPACE_BYTES); use fta_bwd with a workspace";
     default: break;
   }
@@ -417,7 +418,7 @@ int fta_fwd_ex(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor5* v,
   if (rc != FTA_OK) return rc;
   rc = check_fwd_impl(q, k, v, bias, o, lse, B, H, L1, L2, D, sm_scale, opt.feat_fwd);
   if (rc != FTA_OK) return rc;
-  if ((rc = check_device()) != FTA_OK) return rc;
+  if ((rc = fta::check_device()) != FTA_OK) return rc;
   fta::FwdParams p{};
   p.q = static_cast<const half_t*>(q->ptr);
   p.k = static_cast<const half_t*>(k->ptr);
@@ -507,7 +508,7 @@ static int bwd_impl(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor
                       B, H, L1, L2, D, sm_scale, level);
   if (rc != FTA_OK) return rc;
   if (opt.dbias_f32 && reinterpret_cast<uintptr_t>(dbias->ptr) % 4 != 0) return FTA_ERR_MISALIGNED;
-  if ((rc = check_device()) != FTA_OK) return rc;
+  if ((rc = fta::check_device()) != FTA_OK) return rc;
   const fta::BwdPlan pl = cached_plan_bwd(B, H, L1, L2, D, level);
   fta::BwdParams p{};
   p.q = static_cast<const half_t*>(q->ptr);
@@ -566,7 +567,7 @@ int fta_dropout_mask(const fta_options* options, int B, int H, int L1, int L2, u
   if (mask == nullptr) return FTA_ERR_NULL_POINTER;
   if (B < 1 || H < 1) return FTA_ERR_BATCH;
   if (L1 < 1 || L2 < 1 || L2 > FTA_MAX_L2) return FTA_ERR_SEQ_LEN;
-  if ((rc = check_device()) != FTA_OK) return rc;
+  if ((rc = fta::check_device()) != FTA_OK) return rc;
   const int64_t rows = (int64_t)B * H * L1;
   const int64_t n = rows * L2 * ((L2 + 3) / 4);
   hipLaunchKernelGGL(fta_dropout_mask_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),

@@ -173,6 +173,9 @@ hipError_t launch_bwd_feat(const BwdParams& p, const BwdPlan& pl, int D, int dty
 // feat: the plan is for bf16 inputs or dropout, which have a smaller set of kernel instances
 FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, bool feat);
 
+// The kernels are gfx950 code objects: FTA_OK if the current device can run them (fta_api.hip).
+int check_device();
+
 // Launch helper shared by all kernels: raises the kernel's dynamic-LDS limit to `smem` bytes once
 // per (kernel, device) -- the attribute call is not free and the limit only ever has to grow --
 // then launches.  Defined in fta_api.hip.

@@ -134,6 +134,10 @@ def _seq_len_supported(lib, L2: int, D: int, opt_key: tuple) -> bool:
     return ok
 
 
+def _draw_seed() -> int:
+    return int(torch.randint(0, 2 ** 62, (1,)).item())
+
+
 class _attention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, b_pw, sm_scale, *extra):
@@ -151,7 +155,7 @@ class _attention(torch.autograd.Function):
         if len(extra) > 1:
             seed = extra[1]
         else:
-            seed = int(torch.randint(0, 2 ** 62, (1,)).item()) if float(dropout_p) > 0.0 else 0
+            seed = _draw_seed() if float(dropout_p) > 0.0 else 0
         ctx.n_extra = len(extra)
         # same preconditions as upstream forward (:557-561)
         HEAD_DIM_Q, HEAD_DIM_K = q.shape[-1], k.shape[-1]

@@ -2,10 +2,12 @@
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libfta.so")
+NATIVE_PATH = os.path.join(HERE, "fta_native.so")
 MAX_L2 = 4096  # FTA_MAX_L2 of include/fta.h
 STATIC_WORKSPACE_BYTES = 128 * 1024 * 1024  # FTA_STATIC_WORKSPACE_BYTES of include/fta.h
 
@@ -23,7 +25,20 @@ class Options(ctypes.Structure):
                 ("precise", ctypes.c_int)]
 
 
-DTYPE_F16, DTYPE_BF16 = 0, 1
+_WEIGHTS = [(n, ctypes.c_void_p) for n in ("norm_weight", "norm_bias", "wq", "wk", "wv", "wb", "wg", "bg", "wo", "bo")]
+
+
+class Block(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("B", "L", "C", "H", "D", "dtype")] + [
+        ("eps", ctypes.c_float), ("sm_scale", ctypes.c_float), ("dropout_p", ctypes.c_float), ("seed", ctypes.c_uint64),
+        ("precise", ctypes.c_int), ("z", ctypes.c_void_p), ("z_stride", ctypes.c_int64 * 3), ("mask", ctypes.c_void_p)] + _WEIGHTS
+
+
+class BlockGrads(ctypes.Structure):
+    _fields_ = [("z", ctypes.c_void_p), ("z_stride", ctypes.c_int64 * 3)] + _WEIGHTS
+
+
+DTYPE_F16, DTYPE_BF16, DTYPE_F32 = 0, 1, 2
 
 
 class FtaError(RuntimeError):
@@ -37,6 +52,8 @@ _lib = None
 PO = ctypes.POINTER(Options)
 P5 = ctypes.POINTER(Tensor5)
 P4 = ctypes.POINTER(Tensor4)
+PB = ctypes.POINTER(Block)
+_S3 = ctypes.POINTER(ctypes.c_int64)
 _DIMS = [ctypes.c_int] * 5
 
 SIGNATURES = {
@@ -65,6 +82,12 @@ SIGNATURES = {
     "fta_bwd_profile": (ctypes.c_int, [P5, P5, P5, P4, P5, ctypes.c_void_p, P5, P5, P5, P5, P4, ctypes.c_void_p,
                                        ctypes.c_size_t] + _DIMS + [ctypes.c_float, ctypes.c_void_p,
                                                                    ctypes.POINTER(ctypes.c_float)]),
+    "fta_block_check": (ctypes.c_int, [PB]),
+    "fta_block_state_bytes": (ctypes.c_size_t, [PB]),
+    "fta_block_bwd_workspace_bytes": (ctypes.c_size_t, [PB]),
+    "fta_block_fwd": (ctypes.c_int, [PB, ctypes.c_void_p, _S3, ctypes.c_void_p, ctypes.c_void_p]),
+    "fta_block_bwd": (ctypes.c_int, [PB, ctypes.c_void_p, ctypes.c_void_p, _S3, ctypes.POINTER(BlockGrads), ctypes.c_void_p,
+                                     ctypes.c_size_t, ctypes.c_void_p]),
 }
 
 
@@ -83,6 +106,23 @@ def load() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The C++ host path (csrc/fta_torch.cpp), a Python extension module next to the library."""
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise ImportError(f"{NATIVE_PATH} is missing: build it with `python flash-triangle-attention_amd/build.py`")
+        spec = importlib.util.spec_from_file_location("fta_native", NATIVE_PATH)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _native = mod
+    return _native
 
 
 def strerror(status: int) -> str:

@@ -24,14 +24,22 @@ import math
 
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
-from flash_tt_attn import attention, reference_tt_attn
+import fta_lib
+from flash_tt_attn import _attention, attention, reference_tt_attn
 
 __all__ = ["TriangleAttention"]
 
 # Added to the bias of padded key positions: its exponent underflows to exactly 0 in fp16 and fp32
 # (attention() also takes -inf there; a finite value keeps the naive reference free of inf - inf).
 _KEY_MASK_BIAS = -30000.0
+
+
+# Submodules in the order in which the fused path takes their weights, and whether it takes a bias with them.
+_SUBMODULES = (("layer_norm", nn.LayerNorm, True), ("linear_q", nn.Linear, False), ("linear_k", nn.Linear, False),
+               ("linear_v", nn.Linear, False), ("linear_b", nn.Linear, False), ("linear_g", nn.Linear, True),
+               ("linear_o", nn.Linear, True))
 
 
 class TriangleAttention(nn.Module):
@@ -72,7 +80,39 @@ class TriangleAttention(nn.Module):
         out = self.linear_o(gate * o).to(dtype)
         return out if self.starting else out.transpose(1, 2)
 
+    def _fused(self, z, key_mask, seed):
+        """The whole block in the kernels of csrc/fta_block.hip (three launches forward, eleven backward), for
+        plain fp16, bf16 or fp32 modules of the sizes built there; None where this does not apply: other
+        sizes, autocast, mixed types, hooked, parametrised or replaced submodules, a subclass."""
+        if type(self) is not TriangleAttention or not z.is_cuda or _has_any_global_hook():
+            return None
+        weights = []
+        for name, kind, has_bias in _SUBMODULES:
+            m = self._modules.get(name)
+            if type(m) is not kind or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+                return None
+            weights.append(m._parameters.get("weight"))
+            if has_bias:
+                weights.append(m._parameters.get("bias"))
+            elif m._parameters.get("bias") is not None:
+                return None
+        norm = self._modules["layer_norm"]
+        if norm.normalized_shape != (z.shape[-1],):
+            return None
+        scope = _attention.forward.__globals__  # (the module that holds the PRECISE_BACKWARD switch)
+        p = self.dropout_p if self.training else 0.0
+        if p > 0.0 and seed is None:
+            seed = scope["_draw_seed"]()
+        try:
+            return fta_lib.native().block(z, key_mask, weights, self.n_heads, self.c_hidden, self.starting, norm.eps, p,
+                                          seed if p > 0.0 else 0, scope)
+        except TypeError:  # (a seed beyond 63 bits, a mask that is no tensor)
+            return None
+
     def forward(self, z: torch.Tensor, key_mask: torch.Tensor | None = None, seed: int | None = None) -> torch.Tensor:
+        out = self._fused(z, key_mask, seed)
+        if out is not None:
+            return out
         q, k, v, bias, gate = self._operands(z, key_mask)
         sm = 1.0 / math.sqrt(self.c_hidden)
         if self.training and self.dropout_p > 0.0:

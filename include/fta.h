@@ -68,7 +68,8 @@ typedef enum fta_status {
   FTA_ERR_NO_DEVICE = -9,      /* no gfx950 device is current */
   FTA_ERR_STATIC_WORKSPACE = -10, /* fta_bwd_noalloc: the sizes need more than FTA_STATIC_WORKSPACE_BYTES of scratch */
   FTA_ERR_DTYPE = -11,         /* fta_options.dtype unknown */
-  FTA_ERR_DROPOUT = -12        /* fta_options.dropout_p outside [0, 1) */
+  FTA_ERR_DROPOUT = -12,       /* fta_options.dropout_p outside [0, 1) */
+  FTA_ERR_BLOCK_SHAPE = -13    /* fta_block_*: C is not 64 or 128, or H*D is not 64 or 128 */
 } fta_status;
 
 /* One fp16 tensor of logical shape (B,H,L1,L2,D): base pointer and element strides (b,h,l1,l2). */
@@ -109,6 +110,7 @@ typedef struct fta_tensor4 {
  *              or when asked for (2e-3 to 5e-3). */
 #define FTA_DTYPE_F16 0
 #define FTA_DTYPE_BF16 1
+#define FTA_DTYPE_F32 2  /* fta_block only: fp32 pair tensor and weights around an fp16 attention */
 typedef struct fta_options {
   int dtype;
   int dbias_f32;
@@ -229,6 +231,47 @@ int fta_bwd_profile(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor
                     const fta_tensor5* dv, const fta_tensor4* dbias, void* workspace,
                     size_t workspace_bytes, int B, int H, int L1, int L2, int D, float sm_scale,
                     void* stream, float stage_ms[4]);
+
+/* ---- the AlphaFold2 block around the attention (Alg. 13/14) -------------------------------------------
+ *
+ *   x = layer_norm(z);  q, k, v = x Wq^T, x Wk^T, x Wv^T;  bias = x Wb^T (+ -30000 on padded keys);
+ *   g = sigmoid(x Wg^T + bg);  out = (g * attention(q, k, v, bias)) Wo^T + bo
+ *
+ * No counterpart upstream, which has the op only.  All tensors of one call have the type `dtype`; the
+ * attention runs in fp16, or in bf16 for bf16 tensors.  z, out, dout, dz: logical (B, L, L, C), unit
+ * stride for the channels, element strides (b, i, j) that are multiples of 8, where i is the attention's
+ * row and j its key: the ending node is the same call with the last two swapped.  Weights are contiguous in
+ * torch's (out features, in features) order, 16-byte aligned; mask (B, L), 1 for keys that exist, or NULL; bg and
+ * bo may be NULL.  C and H*D are 64 or 128. */
+typedef struct fta_block {
+  int B, L, C, H, D, dtype;
+  float eps;       /* of the layer norm */
+  float sm_scale;
+  float dropout_p; /* as in fta_options */
+  uint64_t seed;
+  int precise;
+  const void* z;
+  int64_t z_stride[3];
+  const void* mask;
+  const void *norm_weight, *norm_bias, *wq, *wk, *wv, *wb, *wg, *bg, *wo, *bo;
+} fta_block;
+/* Where the gradients go: dz (strides as z) and one tensor per weight; bg and bo may be NULL. */
+typedef struct fta_block_grads {
+  void* z;
+  int64_t z_stride[3];
+  void *norm_weight, *norm_bias, *wq, *wk, *wv, *wb, *wg, *bg, *wo, *bo;
+} fta_block_grads;
+
+/* Argument checks only (no GPU call). */
+int fta_block_check(const fta_block* b);
+/* Bytes of the forward state (q, k, v, bias, gate, o, lse), which the backward reads: caller-provided, 16-byte aligned.
+ * A forward without a backward uses it as scratch. */
+size_t fta_block_state_bytes(const fta_block* b);
+size_t fta_block_bwd_workspace_bytes(const fta_block* b);
+int fta_block_fwd(const fta_block* b, void* out, const int64_t out_stride[3], void* state, void* stream);
+/* All gradients from the forward's state; deterministic (partial sums are added in a fixed order). */
+int fta_block_bwd(const fta_block* b, const void* state, const void* dout, const int64_t dout_stride[3],
+                  const fta_block_grads* grads, void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -113,6 +113,49 @@ def test_block_at_the_crop_shape_against_the_oracle(starting, zdtype):
             assert _rel_l2(res["hip"][n], res["oracle"][n]) <= g_tol, n
 
 
+class _Unfused(TriangleAttention):
+    """The block as separate torch operations around attention() (a subclass does not take the fused kernels)."""
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("C,H,D,B,L,starting,masked,dropout_p", [
+    (128, 4, 32, 1, 1, True, False, 0.0),      # one pair
+    (128, 4, 32, 2, 5, False, True, 0.0),      # 25 rows of a 32-row block, two batch entries
+    (128, 4, 32, 1, 33, True, True, 0.0),      # 1089 rows: a last block of one row
+    (128, 4, 32, 2, 64, False, False, 0.0),    # whole blocks
+    (128, 4, 32, 1, 200, True, False, 0.2),    # enough rows for the weights in LDS, several chunks of the weight gradients
+    (64, 2, 32, 1, 40, True, False, 0.0), (64, 4, 32, 1, 41, False, True, 0.0),
+    (128, 1, 64, 1, 40, True, True, 0.0), (128, 2, 64, 1, 39, False, False, 0.0), (64, 1, 64, 1, 9, True, False, 0.0)])
+def test_fused_block_kernels_against_separate_operations(C, H, D, B, L, starting, masked, dropout_p, dtype):
+    torch.manual_seed(4)
+    fused = TriangleAttention(C, D, H, starting=starting, dropout_p=dropout_p).to("cuda:0")
+    with torch.no_grad():
+        fused.layer_norm.weight.add_(0.3 * torch.randn(C, device="cuda:0"))
+        fused.layer_norm.bias.add_(0.3 * torch.randn(C, device="cuda:0"))
+    plain = _Unfused(C, D, H, starting=starting, dropout_p=dropout_p).to("cuda:0")
+    plain.load_state_dict(fused.state_dict())
+    z = torch.randn(B, L, L, C, device="cuda:0").to(dtype) + 0.5
+    dout = torch.randn_like(z)
+    km = None
+    if masked:
+        km = torch.ones(B, L, device="cuda:0")
+        km[:, L - max(1, L // 8):] = 0
+    res = []
+    for blk in (fused.to(dtype), plain.to(dtype)):
+        zz = z.clone().requires_grad_(True)
+        out = blk(zz, km, 7)
+        res.append({"out": out, "z": torch.autograd.grad(out, [zz, *blk.parameters()], dout)})
+        torch.cuda.synchronize()
+    assert fused._fused(z, km, 7) is not None and plain._fused(z, km, 7) is None
+    tol = {torch.float16: 3e-3, torch.bfloat16: 2e-2, torch.float32: 1e-3}[dtype]
+    names = ["z", *(n for n, _ in fused.named_parameters())]
+    assert _rel_l2(res[0]["out"], res[1]["out"]) <= tol
+    for n, a, b in zip(names, res[0]["z"], res[1]["z"]):
+        # (one pair: every softmax is over one key, the gradients of q, k and the bias are zero up to rounding)
+        assert _rel_l2(a, b) <= tol or (L == 1 and b.abs().max() < 1e-2), n
+
+
 @pytest.mark.gpu
 def test_block_dropout_draws_a_fresh_mask_per_call_and_replays_a_given_seed():
     torch.manual_seed(3)
