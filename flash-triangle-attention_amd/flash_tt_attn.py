@@ -138,7 +138,34 @@ def _draw_seed() -> int:
     return int(torch.randint(0, 2 ** 62, (1,)).item())
 
 
+_GLOBALS = globals()
+_native = None
+
+
+def _load_native():
+    global _native
+    _native = fta_lib.native().attention
+    return _native
+
+
 class _attention(torch.autograd.Function):
+    @staticmethod
+    def apply(*args):
+        """The operator.  Tensors that the kernels read in place go through the C++ host path (an autograd
+        function of its own, csrc/fta_torch.cpp): the interpreted path below costs 15 us a call, as much as
+        the kernel at 64 keys.  What that path does not take -- and the precise mode -- comes here."""
+        if 5 <= len(args) <= 7 and not PRECISE_BACKWARD:
+            if len(args) == 6 and float(args[5]) > 0.0:
+                args = args + (_draw_seed(),)
+            native = _native or _load_native()
+            try:
+                o = native(*args[:4], *map(float, args[4:6]), *args[6:], globals=_GLOBALS)
+            except TypeError:  # (not tensors, or a seed beyond 63 bits)
+                o = None
+            if o is not None:
+                return o
+        return super(_attention, _attention).apply(*args)
+
     @staticmethod
     def forward(ctx, q, k, v, b_pw, sm_scale, *extra):
         """Upstream's five positional arguments (:556), plus two optional positional ones for what
