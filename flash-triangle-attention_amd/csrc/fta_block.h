@@ -6,8 +6,6 @@
 
 namespace fta {
 
-constexpr int kWgradChunksMax = 64;  // chunks of pair rows whose weight-gradient partials are summed in order
-
 // All element strides are of the NODE's view of the pair tensors: index (b, i, j) is row i, key j of the
 // attention, so that the ending node only swaps two strides.  q, k, v, gate, o and their gradients are
 // laid out (B, H, L, L, D) contiguously, bias and dbias (B, H, L, L).
@@ -24,8 +22,8 @@ struct BlockParams {
   void* dog; void* dgp;                   // dO (16-bit type), gradient of the gate before the sigmoid (block's type)
   const void* dqkv[3]; const void* db;    // attention gradients
   void* wt;                               // packed transposed projection weights, in MFMA operand order
-  float* part;                            // weight-gradient partial sums, see wgrad_part()
-  float* red;                             // reduced: G (4*HD + H, C), then the sums over the rows (4*HD + H)
+  float* part;                            // weight-gradient partial sums, one block of wgrad_part_floats() per section and chunk
+  float* red;                             // contributions to the layer norm's gradients, (groups, 2, C)
   void* dw[4]; void* dwb; void* dbg; void* dwo; void* dbo; void* dgamma; void* dbeta;
   int B, L, H, D, HD;
   int64_t LL;                             // L * L
@@ -33,7 +31,6 @@ struct BlockParams {
   int cg;                                 // column groups a row block's output tiles are dealt to
   int nwg;                                // workgroups of the work proper (the ones behind them pack weights)
   int nchunks;                            // chunks of the weight-gradient kernel
-  int wlds;                               // packed weights are staged in LDS (else read from the cache each time)
   float eps;
 };
 

@@ -28,6 +28,8 @@
 // launch functions at the end of this file.
 #include "fta_block.h"
 
+#include <type_traits>
+
 #include "fta.h"
 
 #include "fta_common.h"
@@ -176,6 +178,15 @@ __device__ __forceinline__ float sigmoid(float x) {
   else return __builtin_amdgcn_rcpf(1.0f + exp2_fast(-kLog2e * x));
 }
 
+// q / L for q < 2^24 (L <= 4096): the fp32 quotient is off by one at most.
+__device__ __forceinline__ uint32_t div_by_length(uint32_t q, uint32_t L, float inv_l) {
+  uint32_t i = (uint32_t)((float)q * inv_l);
+  const int r = (int)(q - i * L);
+  i -= r < 0 ? 1u : 0u;
+  i += r >= (int)L ? 1u : 0u;
+  return i;
+}
+
 // 32 pair rows of one batch entry: which ones, and where this lane's row is.
 struct RowBlock {
   int b;          // batch entry (wave-uniform)
@@ -189,7 +200,7 @@ __device__ __forceinline__ RowBlock row_block(const BlockParams& p, int blk, int
   const uint32_t p0 = (uint32_t)(blk - r.b * p.nper) * 32u + (uint32_t)(lane & 31);
   r.valid = p0 < (uint32_t)p.LL;
   r.p = r.valid ? p0 : (uint32_t)p.LL - 1u;
-  r.i = r.p / (uint32_t)p.L;
+  r.i = div_by_length(r.p, (uint32_t)p.L, 1.0f / (float)p.L);
   r.j = r.p - r.i * (uint32_t)p.L;
   return r;
 }
@@ -199,130 +210,177 @@ __device__ __forceinline__ int64_t head_off(const BlockParams& p, const RowBlock
   return (((int64_t)r.b * p.H + h) * p.LL + r.p) * p.D;
 }
 
-// Layer-norm statistics of this lane's row from its half of the row (C/16 fragments) and its partner's,
-// in two passes over the registers, as mean and sum of squared deviations.
-template <class A, bool F32, int KS>
-__device__ __forceinline__ void row_stats(const Frag<F32> (&z)[KS], float eps, float& mean, float& rstd) {
+// Sum over the 8 or 16 neighbouring lanes that hold a pair row of 64 or 128 channels (DPP moves: quads, then
+// mirrored half rows, then mirrored rows).
+template <int LANES>
+__device__ __forceinline__ float row_sum(float x) {
+  auto add = [](float v, auto sel) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(sel)::value, 0xF, 0xF, true));
+  };
+  x = add(x, std::integral_constant<int, 0xB1>{});   // lanes 1 0 3 2
+  x = add(x, std::integral_constant<int, 0x4E>{});   // lanes 2 3 0 1
+  x = add(x, std::integral_constant<int, 0x141>{});  // half row mirrored
+  if constexpr (LANES == 16) x = add(x, std::integral_constant<int, 0x140>{});  // row mirrored
+  return x;
+}
+
+// Layer norm without its parameters: v holds 8 of the row's C channels, the neighbouring lanes the others.
+// Mean first, then the squared deviations, in fp32.
+template <int C>
+__device__ __forceinline__ void normalise(float (&v)[8], float eps, float& mean, float& rstd) {
   float s = 0.f;
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    float x[8];
-    unpack<A>(z[ks], x);
+  for (int e = 0; e < 8; ++e) s += v[e];
+  mean = row_sum<C / 8>(s) * (1.0f / C);
+  s = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) s += x[e];
-  }
-  mean = sum_both_halves(s) * (1.0f / (16 * KS));
-  float v = 0.f;
+  for (int e = 0; e < 8; ++e) { v[e] -= mean; s = __builtin_fmaf(v[e], v[e], s); }
+  rstd = 1.0f / __builtin_sqrtf(row_sum<C / 8>(s) * (1.0f / C) + eps);
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    float x[8];
-    unpack<A>(z[ks], x);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { const float d = x[e] - mean; v = __builtin_fmaf(d, d, v); }
-  }
-  v = sum_both_halves(v) * (1.0f / (16 * KS));
-  rstd = 1.0f / __builtin_sqrtf(v + eps);
+  for (int e = 0; e < 8; ++e) v[e] *= rstd;
+}
+
+// ---- staged row tiles ---------------------------------------------------------------------------------
+// The kernels whose weights fill the registers (proj, dx) share the rows between the waves instead: a stage of
+// rows is loaded in whole 128-byte lines (a thread takes 8 consecutive elements of a row, neighbouring threads the
+// next ones), and sits in LDS as MFMA B operands, one 16-byte slot per (row, 8 elements) and plane.  Slot
+// of row r, piece c of a 32-row sub-block: ((c / 2) * 64 + (r ^ (c % 16)) + 32 * (c % 2)): the XOR spreads the
+// pieces of a row, which neighbouring threads write at once, over the banks.
+template <bool F32>
+__device__ __forceinline__ void piece_write(char* blk, int r, int c, const Frag<F32>& f) {
+  frag_write<F32>(blk, c / 2, (r ^ (c % 16)) + 32 * (c % 2), f);
+}
+template <bool F32>
+__device__ __forceinline__ Frag<F32> piece_frag(const char* blk, int ks, int l32, int hh) {
+  return frag_read<F32>(blk, ks, (l32 ^ ((2 * ks + hh) % 16)) + 32 * hh);
 }
 
 // ---- forward: layer norm and projections --------------------------------------------------------------
-// Output tiles of 32 channels: 4*HD/32 of q, k, v, gate, then the heads of the bias (padded to 32).
-template <class A, bool F32, int C>
+// A wave keeps the weights of one or two tiles of 32 output channels (4*HD/32 tiles of q, k, v, gate over eight
+// waves) in registers, 64 or 128 of them; the bias heads are one more tile, its weights in LDS, that the waves take
+// turns at.  The next stage's loads and its layer norm overlap this stage's products (two stage buffers).
+template <class A, bool F32, int C, int HD>
 __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
-  constexpr int KS = C / 16;
+  constexpr int KS = C / 16, NT = HD / 64;           // NT: tiles per wave
+  constexpr int TR = F32 ? 32 : 64, RS = TR / 32;    // rows per stage (fp32: half, so that few rows still load the CUs evenly)
+  constexpr int NP = (TR * C / 8 + 511) / 512;       // pieces per thread
+  constexpr int SUB = KS * kFragBytes<F32>, BUF = RS * SUB;
   extern __shared__ char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
-  const int nw = blockDim.x >> 6;
-  const int nt4 = 4 * p.HD / 32, ntiles = nt4 + (p.H + 31) / 32;
-  const int per = (ntiles + gridDim.y - 1) / gridDim.y;  // tiles of this workgroup's column range
-  const int t0 = blockIdx.y * per, t1 = min(ntiles, t0 + per);
-  // weights -> LDS in operand order; layer-norm parameters and gate biases as fp32 behind them
-  float* gam = reinterpret_cast<float*>(smem + (size_t)per * KS * kFragBytes<F32>);
-  float* bet = gam + C;
-  float* bgs = bet + C;
-  for (int idx = wave; idx < (t1 - t0) * KS; idx += nw) {
-    const int t = t0 + idx / KS, ks = idx % KS;
-    const int n = t * 32 + l32;
-    Frag<F32> f = frag_zero<F32>();
-    if (t < nt4) {
-      const int s = n / p.HD;
-      f = load8<F32>(p.w[s], (int64_t)(n - s * p.HD) * C + ks * 16 + hh * 8);
-    } else if (n - 32 * nt4 < p.H) {
-      f = load8<F32>(p.wb, (int64_t)(n - 32 * nt4) * C + ks * 16 + hh * 8);
-    }
-    frag_write<F32>(smem, idx, lane, f);
-  }
-  for (int c = tid; c < C; c += blockDim.x) {
-    gam[c] = load1<A, F32>(p.gamma, c);
-    bet[c] = load1<A, F32>(p.beta, c);
-  }
-  for (int c = tid; c < p.HD; c += blockDim.x) bgs[c] = p.bg != nullptr ? load1<A, F32>(p.bg, c) : 0.f;
-  __syncthreads();
-
-  const int nitems = p.B * p.nper * p.cg, step = (int)gridDim.x * nw;
-  int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * nw + wave);
-  if (item >= nitems) return;
-  Frag<F32> z[KS];
-  RowBlock rb = row_block(p, item / p.cg, lane);
-  auto fetch = [&]() {
-    const int64_t zo = pair_off(p.zs, rb) + hh * 8;
+  char* wbf = smem + 2 * BUF;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
+  float* bgs = reinterpret_cast<float*>(wbf + SUB);
+  float* msk = bgs + HD;  // what the mask adds to the bias of a stage's rows, two buffers
+  Frag<F32> w[NT][KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) z[ks] = load8<F32>(p.z, zo + ks * 16);
-  };
-  fetch();
-  for (; item < nitems; item += step) {
-    const RowBlock cur = rb;
-    const int g = item % p.cg;
-    float mean, rstd;
-    row_stats<A, F32, KS>(z, p.eps, mean, rstd);
-    Frag<F32> x[KS];
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      float v[8];
-      unpack<A>(z[ks], v);
+      const int n = (wave * NT + t) * 32 + l32, sec = n / HD;
+      w[t][ks] = load8<F32>(p.w[sec], (int64_t)(n - sec * HD) * C + ks * 16 + hh * 8);
+    }
+  for (int ks = wave; ks < KS; ks += 8)
+    frag_write<F32>(wbf, ks, lane, l32 < p.H ? load8<F32>(p.wb, (int64_t)l32 * C + ks * 16 + hh * 8) : frag_zero<F32>());
+  const int c8 = (tid % (C / 8)) * 8;
+  float gam[8], bet[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int c = ks * 16 + hh * 8 + e;
-        v[e] = __builtin_fmaf((v[e] - mean) * rstd, gam[c], bet[c]);
+  for (int e = 0; e < 8; ++e) { gam[e] = load1<A, F32>(p.gamma, c8 + e); bet[e] = load1<A, F32>(p.beta, c8 + e); }
+
+  const int LL = (int)p.LL, nst = (LL + TR - 1) / TR, ntot = p.B * nst;
+  const float inv_l = 1.0f / (float)p.L;
+  Frag<F32> z[NP];
+  float mrow;
+  const void* mask = p.mask != nullptr ? p.mask : p.gamma;  // (loaded either way, see the stores)
+  for (int c = tid; c < HD; c += 512) bgs[c] = p.bg != nullptr ? load1<A, F32>(p.bg, c) : 0.f;
+  auto fetch = [&](int st) {
+    const int b = st / nst, p0 = (st - b * nst) * TR;
+    {
+      const uint32_t q = (uint32_t)min(p0 + tid % TR, LL - 1), i = div_by_length(q, (uint32_t)p.L, inv_l);
+      mrow = load1<A, F32>(mask, p.mask != nullptr ? (int64_t)b * p.L + (q - i * (uint32_t)p.L) : 0);
+    }
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      const uint32_t q = (uint32_t)min(p0 + (tid + 512 * n) / (C / 8), LL - 1);
+      const uint32_t i = div_by_length(q, (uint32_t)p.L, inv_l), j = q - i * (uint32_t)p.L;
+      z[n] = load8<F32>(p.z, b * p.zs[0] + (int64_t)i * p.zs[1] + (int64_t)j * p.zs[2] + c8);
+    }
+  };
+  auto put = [&](int buffer) {
+    char* buf = smem + buffer * BUF;
+    // 0 marks padded key positions, which no query may attend to
+    if (tid < TR) msk[buffer * TR + tid] = p.mask != nullptr ? (mrow - 1.0f) * 30000.0f : 0.f;
+#pragma unroll
+    for (int n = 0; n < NP; ++n) {
+      const int row = (tid + 512 * n) / (C / 8);
+      float v[8], mean, rstd;
+      unpack<A>(z[n], v);
+      normalise<C>(v, p.eps, mean, rstd);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = __builtin_fmaf(v[e], gam[e], bet[e]);
+      Frag<F32> f;
+      pack<A>(v, f);
+      if (TR * C / 8 >= 512 || row < TR) piece_write<F32>(buf + (row / 32) * SUB, row % 32, c8 / 8, f);
+    }
+  };
+  int st = (int)blockIdx.x;
+  if (st < ntot) {
+    fetch(st);
+    put(0);
+    fetch(min(st + (int)gridDim.x, ntot - 1));
+  }
+  __syncthreads();
+  for (int it = 0; st < ntot; st += (int)gridDim.x, ++it) {
+    const char* buf = smem + (it & 1) * BUF;
+    const int b = st / nst, p0 = (st - b * nst) * TR;
+#pragma unroll
+    for (int rs = 0; rs < RS; ++rs) {
+      // (rows beyond the end repeat the last one, and store the same values to the same place: with no branch
+      // around the stores the waits for the next stage's loads do not have to wait for them as well)
+      const int q = min(p0 + rs * 32 + l32, LL - 1);
+      floatx16 acc[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = zero16();
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const Frag<F32> x = piece_frag<F32>(buf + rs * SUB, ks, l32, hh);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = mma<A>(w[t][ks], x, acc[t]);
       }
-      pack<A>(v, x[ks]);
-    }
-    if (item + step < nitems) {  // the next row block's loads fly during this one's products
-      rb = row_block(p, (item + step) / p.cg, lane);
-      fetch();
-    }
-    for (int t = t0 + g; t < t1; t += p.cg) {
-      floatx16 acc = zero16();
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) acc = mma<A>(frag_read<F32>(smem, (t - t0) * KS + ks, lane), x[ks], acc);
-      if (t < nt4) {
-        const int n = t * 32, s = n / p.HD, col = n - s * p.HD, h = col / p.D;
-        const int64_t off = head_off(p, cur, h) + (col - h * p.D) + hh * 8;
+      for (int t = 0; t < NT; ++t) {
+        const int n = (wave * NT + t) * 32, sec = n / HD, col = n - sec * HD, h = col / p.D;
+        const int64_t off = (((int64_t)b * p.H + h) * LL + q) * p.D + (col - h * p.D) + hh * 8;
         float y[2][8];
-        rows8(acc, y);
+        rows8(acc[t], y);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          if (s == 3) {
+          if (sec == 3) {
+            Frag<F32> f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) y[u][e] = sigmoid<F32>(y[u][e] + bgs[col + 16 * u + 8 * hh + e]);
-            Frag<F32> f;
             pack<A>(y[u], f);
-            if (cur.valid) store8<F32>(p.gate, off + 16 * u, f);
+            store8<F32>(p.gate, off + 16 * u, f);
           } else {
             Frag<false> f;
             pack<A>(y[u], f);
-            if (cur.valid) store8<false>(p.qkv[s], off + 16 * u, f);
+            store8<false>(p.qkv[sec], off + 16 * u, f);
           }
         }
-      } else {
-        float add = 0.f;  // 0 marks padded key positions, which no query may attend to
-        if (p.mask != nullptr) add = (load1<A, F32>(p.mask, (int64_t)cur.b * p.L + cur.j) - 1.0f) * 30000.0f;
+      }
+      if (wave == ((RS * it + rs) & 7)) {
+        floatx16 ab = zero16();
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int h = (t - nt4) * 32 + 8 * (r / 4) + 4 * hh + r % 4;
-          if (h < p.H && cur.valid) store1<A, false>(p.bias, ((int64_t)cur.b * p.H + h) * p.LL + cur.p, acc[r] + add);
-        }
+        for (int ks = 0; ks < KS; ++ks)
+          ab = mma<A>(frag_read<F32>(wbf, ks, lane), piece_frag<F32>(buf + rs * SUB, ks, l32, hh), ab);
+        const float add = msk[(it & 1) * TR + rs * 32 + l32];
+        if (hh == 0)
+#pragma unroll
+          for (int h = 0; h < 4; ++h)
+            if (h < p.H) store1<A, false>(p.bias, ((int64_t)b * p.H + h) * LL + q, ab[h] + add);
       }
     }
+    put((it + 1) & 1);  // (behind the last stage: once more the last rows, into the buffer nobody reads)
+    fetch(min(st + 2 * (int)gridDim.x, ntot - 1));
+    __syncthreads();
   }
 }
 
@@ -331,7 +389,7 @@ template <class A, bool F32, int C, int HD>
 __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
   constexpr int KS = HD / 16, NT = C / 32;
   extern __shared__ char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
   const int nw = blockDim.x >> 6;
   float* bos = reinterpret_cast<float*>(smem + (size_t)NT * KS * kFragBytes<F32>);
   for (int idx = wave; idx < NT * KS; idx += nw)
@@ -398,10 +456,10 @@ template <class A, bool F32, int C, int HD>
 __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
   constexpr int KS = C / 16, NT = HD / 32;
   extern __shared__ char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
   const int nw = blockDim.x >> 6;
   if ((int)blockIdx.x >= p.nwg) {
-    const int ksall = 4 * HD / 16 + (p.H + 15) / 16;
+    constexpr int ksall = 4 * HD / 16 + 1;
     const int npack = (int)gridDim.x - p.nwg;
     for (int idx = ((int)blockIdx.x - p.nwg) * nw + wave; idx < (C / 32) * ksall; idx += npack * nw) {
       const int ct = idx / ksall, ks = idx % ksall, c = ct * 32 + l32;
@@ -482,120 +540,160 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
 }
 
 // ---- backward: input gradient and layer norm ----------------------------------------------------------
-template <class A, bool F32, int C, int HD, bool WLDS>
+// dx = sum of the five projections' input gradients, one product with 4*HD + 16 contraction elements (the bias
+// heads padded to one 16-wide step).  A wave keeps the transposed weights of 32 channels in registers (132 of them in
+// bf16; fp32: half of the contraction, 136), the rows' gradients go through LDS once, and dx comes back
+// through LDS in fp32 (one plane per share of the contraction) to the threads that hold the rows of z in the layer norm's layout: 8 channels
+// of a row each, so that dz leaves in whole lines.
+template <class A, bool F32, int C, int HD>
 __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
-  constexpr int KS = C / 16, NT = C / 32, KH = HD / 16;
+  constexpr int TR = F32 ? 32 : 64, RS = TR / 32, NT = C / 32;
+  constexpr int SPLIT = 8 / (RS * NT);                   // shares of the contraction
+  constexpr int KH = HD / 16, KALL = 4 * KH + 1, KW = (KALL + SPLIT - 1) / SPLIT;
+  constexpr int NP = TR * HD / 8 / 512;                  // pieces per thread of a section
+  constexpr int NZ = (TR * C / 8 + 511) / 512;           // pieces of z
+  constexpr int SUB = KALL * kFragBytes<F32>;
+  constexpr int XROW = C + 4;                            // floats per row of a dx plane
+  static_assert(NP >= 1 || F32, "pieces");
+  constexpr int NPP = NP > 0 ? NP : 1;
   extern __shared__ char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, hh = lane >> 5;
-  const int nw = blockDim.x >> 6;
-  const int kb = (p.H + 15) / 16, ksall = 4 * KH + kb;
-  float* gam = reinterpret_cast<float*>(smem + (WLDS ? (size_t)NT * ksall * kFragBytes<F32> : 0));
-  const char* wt = WLDS ? smem : static_cast<const char*>(p.wt);
-  if (WLDS)
-    for (int idx = tid; idx < NT * ksall * kFragBytes<F32> / 16; idx += blockDim.x)
-      reinterpret_cast<u32x4*>(smem)[idx] = static_cast<const u32x4*>(p.wt)[idx];
-  for (int c = tid; c < C; c += blockDim.x) gam[c] = load1<A, F32>(p.gamma, c);
-  __syncthreads();
+  float* dxs = reinterpret_cast<float*>(smem + RS * SUB);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
+  const int ct = wave % NT, rs = (wave / NT) % RS, share = wave / (NT * RS);
+  Frag<F32> w[KW];
+#pragma unroll
+  for (int k = 0; k < KW; ++k) {
+    const int ks = share * KW + k;
+    w[k] = ks < KALL ? frag_read<F32>(static_cast<const char*>(p.wt), ct * KALL + ks, lane) : frag_zero<F32>();
+  }
+  const int c8 = (tid % (C / 8)) * 8;
+  float gam[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) gam[e] = load1<A, F32>(p.gamma, c8 + e);
 
-  const int nitems = p.B * p.nper, step = (int)gridDim.x * nw;
-  for (int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * nw + wave); item < nitems; item += step) {
-    const RowBlock cur = row_block(p, item, lane);
-    Frag<F32> z[KS];
-    const int64_t zo = pair_off(p.zs, cur) + hh * 8;
+  const int LL = (int)p.LL, nst = (LL + TR - 1) / TR, ntot = p.B * nst;
+  const float inv_l = 1.0f / (float)p.L;
+  Frag<F32> z[NZ], dg[NPP];
+  Frag<false> d[3][NPP];
+  uint16_t rd[4];
+  auto fetch = [&](int st) {
+    const int b = st / nst, p0 = (st - b * nst) * TR;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) z[ks] = load8<F32>(p.z, zo + ks * 16);
-    floatx16 acc[NT];
+    for (int n = 0; n < NPP; ++n) {
+      const int pc = tid + 512 * n, e8 = (pc % (HD / 8)) * 8, h = e8 / p.D;
+      const int q = min(p0 + pc / (HD / 8), LL - 1);
+      const int64_t off = (((int64_t)b * p.H + h) * LL + q) * p.D + (e8 - h * p.D);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) acc[t] = zero16();
-    auto step16 = [&](const Frag<F32>& d, int ks) {
+      for (int s = 0; s < 3; ++s) d[s][n] = load8<false>(p.dqkv[s], off);
+      dg[n] = load8<F32>(p.dgp, off);
+    }
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = mma<A>(frag_read<F32>(wt, t * ksall + ks, lane), d, acc[t]);
-    };
-    for (int s = 0; s < 3; ++s) {
-      Frag<false> d[KH];
+    for (int h = 0; h < 4; ++h) rd[h] = static_cast<const uint16_t*>(p.db)[((int64_t)b * p.H + min(h, p.H - 1)) * LL + min(p0 + tid % TR, LL - 1)];
+  };
+  // (rows beyond the end, or beyond the stage, repeat the last one and store the same values there)
+  auto pair_off_of = [&](const int64_t (&s)[3], int st, int n) {
+    const int b = st / nst, r = (st - b * nst) * TR + min((tid + 512 * n) / (C / 8), TR - 1);
+    const uint32_t q = (uint32_t)min(r, LL - 1), i = div_by_length(q, (uint32_t)p.L, inv_l), j = q - i * (uint32_t)p.L;
+    return b * s[0] + (int64_t)i * s[1] + (int64_t)j * s[2] + c8;
+  };
+  auto put = [&]() {
 #pragma unroll
-      for (int k = 0; k < KH; ++k) {
-        const int h = k * 16 / p.D;
-        d[k] = load8<false>(p.dqkv[s], head_off(p, cur, h) + (k * 16 - h * p.D) + hh * 8);
-      }
+    for (int n = 0; n < NPP; ++n) {
+      const int pc = tid + 512 * n, row = pc / (HD / 8), c = pc % (HD / 8);
+      if (NP >= 1 || row < TR) {
+        char* blk = smem + (row / 32) * SUB;
 #pragma unroll
-      for (int k = 0; k < KH; ++k) {
-        Frag<F32> f;
-        if constexpr (F32) unpack<A>(d[k], f.v);
-        else f = d[k];
-        step16(f, s * KH + k);
+        for (int s = 0; s < 3; ++s) {
+          Frag<F32> f;
+          if constexpr (F32) unpack<A>(d[s][n], f.v);
+          else f = d[s][n];
+          piece_write<F32>(blk, row % 32, s * (HD / 8) + c, f);
+        }
+        piece_write<F32>(blk, row % 32, 3 * (HD / 8) + c, dg[n]);
       }
     }
-    {
-      Frag<F32> d[KH];
+    if (tid < 2 * TR) {  // (the second half of the step: zeros)
+      float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (tid < TR)
 #pragma unroll
-      for (int k = 0; k < KH; ++k) {
-        const int h = k * 16 / p.D;
-        d[k] = load8<F32>(p.dgp, head_off(p, cur, h) + (k * 16 - h * p.D) + hh * 8);
-      }
-#pragma unroll
-      for (int k = 0; k < KH; ++k) step16(d[k], 3 * KH + k);
-    }
-    for (int k = 0; k < kb; ++k) {
-      float v[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int h = k * 16 + hh * 8 + e;
-        v[e] = h < p.H ? load1<A, false>(p.db, ((int64_t)cur.b * p.H + h) * p.LL + cur.p) : 0.f;
-      }
+        for (int h = 0; h < 4; ++h) v[h] = h < p.H ? A::lo((uint32_t)rd[h]) : 0.f;
       Frag<F32> f;
       pack<A>(v, f);
-      step16(f, 4 * KH + k);
+      const int row = tid % TR;
+      piece_write<F32>(smem + (row / 32) * SUB, row % 32, 4 * (HD / 8) + tid / TR, f);
     }
-    float mean, rstd;
-    row_stats<A, F32, KS>(z, p.eps, mean, rstd);
+  };
+  int st = (int)blockIdx.x;
+  if (st < ntot) { fetch(st); put(); }
+  __syncthreads();
+  for (; st < ntot; st += (int)gridDim.x) {
+    const int next = st + (int)gridDim.x;
+#pragma unroll
+    for (int n = 0; n < NZ; ++n) z[n] = load8<F32>(p.z, pair_off_of(p.zs, st, n));
+    fetch(min(next, ntot - 1));
+    floatx16 acc = zero16();
+#pragma unroll
+    for (int k = 0; k < KW; ++k) {
+      const int ks = share * KW + k;
+      if (ks < KALL) acc = mma<A>(w[k], piece_frag<F32>(smem + rs * SUB, ks, l32, hh), acc);
+    }
+    float* plane = dxs + ((size_t)share * TR + rs * 32 + l32) * XROW + ct * 32 + 4 * hh;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) *reinterpret_cast<float4*>(plane + 8 * g) = make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
+    __syncthreads();
     // dz = rstd * (g - mean(g) - xhat * mean(g * xhat)), g = dx * gamma
-    float s1 = 0.f, s2 = 0.f;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      float y[2][8];
-      rows8(acc[t], y);
+    for (int n = 0; n < NZ; ++n) {
+      const int row = min((tid + 512 * n) / (C / 8), TR - 1);
+      float x[8], g[8], mean, rstd;
+      unpack<A>(z[n], x);
+      normalise<C>(x, p.eps, mean, rstd);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        float x[8];
-        unpack<A>(z[2 * t + u], x);
+      for (int e = 0; e < 8; ++e) g[e] = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float gx = y[u][e] * gam[t * 32 + 16 * u + 8 * hh + e];
-          s1 += gx;
-          s2 = __builtin_fmaf(gx, (x[e] - mean) * rstd, s2);
-          acc[t][8 * u + e] = gx;  // (from here on in runs of eight channels)
-        }
+      for (int s = 0; s < SPLIT; ++s) {
+        const float* src = dxs + ((size_t)s * TR + row) * XROW + c8;
+        const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
+        g[0] += a.x; g[1] += a.y; g[2] += a.z; g[3] += a.w;
+        g[4] += b.x; g[5] += b.y; g[6] += b.z; g[7] += b.w;
       }
+      float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        g[e] *= gam[e];
+        s1 += g[e];
+        s2 = __builtin_fmaf(g[e], x[e], s2);
+      }
+      s1 = row_sum<C / 8>(s1) * (1.0f / C);
+      s2 = row_sum<C / 8>(s2) * (1.0f / C);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[e] = rstd * (g[e] - s1 - x[e] * s2);
+      Frag<F32> f;
+      pack<A>(x, f);
+      store8<F32>(p.dz, pair_off_of(p.dzs, st, n), f);
     }
-    s1 = sum_both_halves(s1) * (1.0f / C);
-    s2 = sum_both_halves(s2) * (1.0f / C);
-    const int64_t dzo = pair_off(p.dzs, cur) + hh * 8;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        float x[8];
-        unpack<A>(z[2 * t + u], x);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = rstd * (acc[t][8 * u + e] - s1 - (x[e] - mean) * rstd * s2);
-        Frag<F32> f;
-        pack<A>(x, f);
-        if (cur.valid) store8<F32>(p.dz, dzo + t * 32 + 16 * u, f);
-      }
+    put();
+    __syncthreads();
   }
 }
 
 // ---- backward: weight gradients -----------------------------------------------------------------------
-// Five products with the pair rows as contraction: section s = 0..3 is (d of projection s)^T xhat, with xhat
+// Six products with the pair rows as contraction: section s = 0..3 is (d of projection s)^T xhat, with xhat
 // the normalised row without gamma and beta (the reduction applies those: one product serves the weight, gamma
-// and beta), section 4 is dout^T (gate * o).  Section 0 takes the bias projection along.  A workgroup works
-// off one chunk of rows of one section: 32-row tiles (two per stage) are formed in registers, written to LDS as 32-column
+// and beta), section 4 is dout^T (gate * o), section 5 the bias projection's.  A workgroup works off one chunk of
+// rows of one section: stages of 64 rows (32 in fp32) are formed in registers, written to LDS as 32-column
 // sub-tiles and read back transposed as MFMA operands; its waves own up to two 32 x 32 tiles of the result
-// each.  The sums over the rows (bias gradients) come from one more product with a column of ones.
-// One chunk's partial: NA*NB*1024 floats of the result tiles, row-major [a][b], then NA*32 row sums; for section 0
-// also H*C and H floats of the bias projection.
-__host__ __device__ inline size_t wgrad_part_floats(int C, int HD, int H) { return (size_t)C * HD + (C > HD ? C : HD) + (size_t)H * C + H; }
+// each.  The sums over the rows (bias gradients) are kept by the threads that load the rows.  The
+// sections of a chunk sit on one die, whose L2 serves z to five of them.
+//
+// Bound by memory latency and the vector ALU rather than bandwidth: a stage has 8 MFMAs per wave.  So all
+// addresses are a base plus the row, the next stage's loads are in flight during a stage, and two workgroups
+// share a CU.  Sections in separate workgroups keep a partial sum at 64 KB (one workgroup for all six: 264 KB, 67 MB to
+// write and read back over the chip, as much as the inputs at 384 x 384 pairs).
+//
+// One chunk's partial: the result tiles row-major [a][b], then (at C * HD) the row sums.
+__host__ __device__ inline size_t wgrad_part_floats(int C, int HD) { return (size_t)C * HD + (C > HD ? C : HD); }
+constexpr int kWgradSections = 6;
 
 // Sub-tile of 32 columns in LDS: 16-bit rows of 64 bytes, swizzled as the attention's staged tiles; fp32 rows
 // of 128 bytes as they are.
@@ -624,286 +722,291 @@ __device__ __forceinline__ Frag<F32> sub_frag_t(const char* tile, int rowbase, c
   return f;
 }
 
-template <class A, bool F32, int C, int HD>
-__global__ void __launch_bounds__(512) blk_wgrad_kernel(BlockParams p) {
-  constexpr int W = (C > HD) ? C : HD;      // columns a stage buffer holds
-  constexpr int TR = F32 ? 32 : 64;         // rows per stage
-  constexpr int NP = (TR * W / 8 + 511) / 512;  // 8-element pieces per thread and operand
-  constexpr int SUB = TR * kSubRow<F32>;    // bytes of a sub-tile
-  constexpr int BUF = 2 * (W / 32) * SUB;   // both operands
-  extern __shared__ char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hh = lane >> 5;
-  const int sec = (int)blockIdx.x % 5, chunk = (int)blockIdx.x / 5;
-  const int na = (sec == 4 ? C : HD) / 32, nb = (sec == 4 ? HD : C) / 32;
-  const int nst = (int)((p.LL + TR - 1) / TR);               // stages per batch entry
+enum WgradKind { kWgradQkv, kWgradGate, kWgradOut, kWgradBias };
+
+template <class A, bool F32, int C, int HD, int KIND>
+__device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int chunk, char* smem) {
+  constexpr int NA = KIND == kWgradOut ? C / 32 : KIND == kWgradBias ? 1 : HD / 32;
+  constexpr int NB = KIND == kWgradOut ? HD / 32 : C / 32;
+  constexpr int NT = (NA * NB + 7) / 8;                 // result tiles per wave
+  constexpr int TR = F32 ? 32 : 64;                     // rows per stage
+  constexpr int PA = KIND == kWgradBias ? 0 : (TR * NA * 4 + 511) / 512;   // 8-element pieces per thread
+  constexpr int PB = (TR * NB * 4 + 511) / 512;
+  constexpr int PD = KIND == kWgradBias ? 4 : 0;        // dbias entries per thread (H <= 32)
+  constexpr int SUB = TR * kSubRow<F32>;                // bytes of a sub-tile
+  constexpr int DROW = TR + 8;                          // dbias: one row of TR entries per head
+  constexpr int ABYTES = KIND == kWgradBias ? 32 * DROW * 2 : NA * SUB;
+  constexpr int BUF = ABYTES + NB * SUB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
+  const int LL = (int)p.LL, nst = (LL + TR - 1) / TR;   // stages per batch entry
   const int ntot = p.B * nst, per = (ntot + p.nchunks - 1) / p.nchunks;
   const int first = chunk * per, last = min(ntot, first + per);
   FragOffsets<32> fo;
   fo.init(lane);
 
-  Frag<F32> ra[NP], rx[NP];
-  Frag<false> ro[NP];
-  bool rv[NP];
-  const int ca = na * 4, cb = nb * 4;  // 8-element pieces per row of the two operands
-  // this thread's pieces of stage st: operand A (the gradient rows) and what operand B is formed from
-  auto fetch = [&](int st) {
-    const int b = st / nst;
-    const uint32_t p0 = (uint32_t)(st - b * nst) * TR;
+  const void* srca = KIND == kWgradQkv ? p.dqkv[sec] : KIND == kWgradGate ? p.dgp : KIND == kWgradOut ? p.dout : p.db;
+  Frag<F32> ra[PA > 0 ? PA : 1], rx[PB];
+  Frag<false> ro[PB];
+  uint16_t rd[PD > 0 ? PD : 1];
+  // where this thread's pieces sit: row of the stage, and the offset of their first element inside row 0
+  auto head_part = [&](int c8) { const int h = c8 / p.D; return ((int64_t)h * LL) * p.D + (c8 - h * p.D); };
+  int64_t ao[PA > 0 ? PA : 1], bo[PB];
 #pragma unroll
-    for (int n = 0; n < NP; ++n) {
-      const int pc = tid + 512 * n;
-      {
-        const uint32_t row = pc / ca, c8 = (pc % ca) * 8;
-        if (row < (uint32_t)TR) {
-          uint32_t q = p0 + row;
-          q = q < (uint32_t)p.LL ? q : (uint32_t)p.LL - 1u;
-          if (sec == 4) {
-            const uint32_t i = q / (uint32_t)p.L, j = q - i * (uint32_t)p.L;
-            ra[n] = load8<F32>(p.dout, b * p.douts[0] + i * p.douts[1] + j * p.douts[2] + c8);
-          } else {
-            const int h = c8 / p.D;
-            const int64_t off = (((int64_t)b * p.H + h) * p.LL + q) * p.D + (c8 - h * p.D);
-            if (sec == 3) {
-              ra[n] = load8<F32>(p.dgp, off);
-            } else {
-              const Frag<false> d = load8<false>(p.dqkv[sec], off);
-              if constexpr (F32) unpack<A>(d, ra[n].v);
-              else ra[n] = d;
-            }
-          }
-        }
+  for (int n = 0; n < PA; ++n) {
+    const int c8 = ((tid + 512 * n) % (NA * 4)) * 8;
+    ao[n] = KIND == kWgradOut ? c8 : head_part(c8);
+  }
+#pragma unroll
+  for (int n = 0; n < PB; ++n) {
+    const int c8 = ((tid + 512 * n) % (NB * 4)) * 8;
+    bo[n] = KIND == kWgradOut ? head_part(c8) : c8;
+  }
+  const float inv_l = 1.0f / (float)p.L;
+  auto pair_row = [&](const int64_t (&s)[3], int b, int q) {
+    const uint32_t i = div_by_length((uint32_t)q, (uint32_t)p.L, inv_l), j = (uint32_t)q - i * (uint32_t)p.L;
+    return b * s[0] + (int64_t)i * s[1] + (int64_t)j * s[2];
+  };
+  auto fetch = [&](int st) {
+    const int b = st / nst, p0 = (st - b * nst) * TR;
+    const int64_t hb = (int64_t)b * p.H * LL * p.D;
+#pragma unroll
+    for (int n = 0; n < PA; ++n) {
+      const int q = min(p0 + (tid + 512 * n) / (NA * 4), LL - 1);
+      if constexpr (KIND == kWgradOut) ra[n] = load8<F32>(srca, pair_row(p.douts, b, q) + ao[n]);
+      else if constexpr (KIND == kWgradGate) ra[n] = load8<F32>(srca, hb + (int64_t)q * p.D + ao[n]);
+      else if constexpr (F32) unpack<A>(load8<false>(srca, hb + (int64_t)q * p.D + ao[n]), ra[n].v);
+      else ra[n] = load8<false>(srca, hb + (int64_t)q * p.D + ao[n]);
+    }
+#pragma unroll
+    for (int n = 0; n < PB; ++n) {
+      const int q = min(p0 + (tid + 512 * n) / (NB * 4), LL - 1);
+      if constexpr (KIND == kWgradOut) {
+        rx[n] = load8<F32>(p.gate, hb + (int64_t)q * p.D + bo[n]);
+        ro[n] = load8<false>(p.o, hb + (int64_t)q * p.D + bo[n]);
+      } else {
+        rx[n] = load8<F32>(p.z, pair_row(p.zs, b, q) + bo[n]);
       }
-      {
-        const uint32_t row = pc / cb, c8 = (pc % cb) * 8;
-        rv[n] = false;
-        if (row < (uint32_t)TR) {
-          uint32_t q = p0 + row;
-          rv[n] = q < (uint32_t)p.LL;
-          q = rv[n] ? q : (uint32_t)p.LL - 1u;
-          if (sec == 4) {
-            const int h = c8 / p.D;
-            const int64_t off = (((int64_t)b * p.H + h) * p.LL + q) * p.D + (c8 - h * p.D);
-            rx[n] = load8<F32>(p.gate, off);
-            ro[n] = load8<false>(p.o, off);
-          } else {
-            const uint32_t i = q / (uint32_t)p.L, j = q - i * (uint32_t)p.L;
-            rx[n] = load8<F32>(p.z, b * p.zs[0] + i * p.zs[1] + j * p.zs[2] + c8);
-          }
-        }
-      }
+    }
+#pragma unroll
+    for (int n = 0; n < PD; ++n) {
+      const int e = tid + 512 * n, h = e / TR, q = min(p0 + e % TR, LL - 1);
+      if (h < p.H) rd[n] = static_cast<const uint16_t*>(srca)[((int64_t)b * p.H + h) * LL + q];
     }
   };
   // forms operand B (gate * o, or the normalised row: the lanes of a row are neighbours) and writes both to LDS;
   // rows beyond the end are zero in operand B
-  auto put = [&](char* buf) {
+  float csum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // of this thread's columns of operand A (dbias: of its entry)
+  auto put = [&](char* buf, int st) {
+    const int left = LL - (st % nst) * TR;
 #pragma unroll
-    for (int n = 0; n < NP; ++n) {
-      const int pc = tid + 512 * n;
-      {
-        const int row = pc / ca, c = pc % ca;
-        if (row < TR) sub_write<F32>(buf + (c / 4) * SUB, row, c % 4, ra[n]);
+    for (int n = 0; n < PA; ++n) {
+      const int pc = tid + 512 * n, row = pc / (NA * 4), c = pc % (NA * 4);
+      if (TR * NA * 4 >= 512 || row < TR) {
+        sub_write<F32>(buf + (c / 4) * SUB, row, c % 4, ra[n]);
+        float v[8];
+        unpack<A>(ra[n], v);
+        const float one = row < left ? 1.0f : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) csum[e] = __builtin_fmaf(v[e], one, csum[e]);
       }
-      const int row = pc / cb, c = pc % cb;
+    }
+#pragma unroll
+    for (int n = 0; n < PD; ++n) {
+      const int e = tid + 512 * n, h = e / TR;
+      if (h < p.H) {
+        reinterpret_cast<uint16_t*>(buf)[h * DROW + e % TR] = rd[n];
+        csum[n] += e % TR < left ? A::lo((uint32_t)rd[n]) : 0.f;
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < PB; ++n) {
+      const int pc = tid + 512 * n, row = pc / (NB * 4), c = pc % (NB * 4);
       float v[8];
       unpack<A>(rx[n], v);
-      if (sec == 4) {
+      if constexpr (KIND == kWgradOut) {
         float w[8];
         unpack<A>(ro[n], w);
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] *= w[e];
       } else {
-        float s = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += v[e];
-#pragma unroll
-        for (int m = 1; m < C / 8; m *= 2) s += __shfl_xor(s, m, 64);
-        const float mean = s * (1.0f / C);
-        s = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) { v[e] -= mean; s = __builtin_fmaf(v[e], v[e], s); }
-#pragma unroll
-        for (int m = 1; m < C / 8; m *= 2) s += __shfl_xor(s, m, 64);
-        const float rstd = 1.0f / __builtin_sqrtf(s * (1.0f / C) + p.eps);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] *= rstd;
+        float mean, rstd;
+        normalise<C>(v, p.eps, mean, rstd);
       }
-      if (row < TR) {
-        Frag<F32> f;
-        pack<A>(v, f);
-        if (!rv[n]) f = frag_zero<F32>();
-        sub_write<F32>(buf + (W / 32 + c / 4) * SUB, row, c % 4, f);
+      Frag<F32> f;
+      pack<A>(v, f);
+      if (row >= left) f = frag_zero<F32>();
+      if (TR * NB * 4 >= 512 || row < TR) sub_write<F32>(buf + ABYTES + (c / 4) * SUB, row, c % 4, f);
+    }
+  };
+  auto frag_a = [&](const char* buf, int at, int k) {
+    if constexpr (KIND == kWgradBias) {
+      const char* s = buf + ((size_t)(l32 < p.H ? l32 : 0) * DROW + k * 16 + 4 * hh) * 2;
+      const u32x2 lo = *reinterpret_cast<const u32x2*>(s), hi = *reinterpret_cast<const u32x2*>(s + 16);
+      Frag<false> d;
+      d.w = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      if (l32 >= p.H) d = frag_zero<false>();
+      if constexpr (F32) {
+        Frag<true> f;
+        unpack<A>(d, f.v);
+        return f;
+      } else {
+        return d;
       }
+    } else {
+      return sub_frag_t<F32>(buf + at * SUB, k * 16, fo, l32, hh);
     }
   };
 
-  floatx16 acc[2], sums = zero16(), accb = zero16(), sumb = zero16();
-  acc[0] = zero16();
-  acc[1] = zero16();
-  const int at = wave % na;                                        // (na is 2 or 4: the same rows for both tiles of a wave)
-  const int bt[2] = {wave / na, wave / na + 8 / na};
-  const bool own[2] = {bt[0] < nb, bt[1] < nb};
-  const bool own_sum = wave < na;
-  const bool own_bias = (sec == 0) && wave >= 4 && wave - 4 < nb;  // bias projection: columns of sub-tile wave - 4
-  Frag<F32> ones;
-  {
-    float v[8];
+  floatx16 acc[NT];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = 1.0f;
-    pack<A>(v, ones);
-  }
-  // (double buffered: stage st is multiplied while the next one's loads are in flight)
+  for (int n = 0; n < NT; ++n) acc[n] = zero16();
+  const int at = wave % NA;             // (NA divides 8: the same rows for both tiles of a wave)
+  const bool own = wave < NA * NB;      // (fewer than eight tiles: the other waves only help staging)
   if (first < last) {
     fetch(first);
-    put(smem);
+    put(smem, first);
     if (first + 1 < last) fetch(first + 1);
     __syncthreads();
     for (int st = first; st < last; ++st) {
       const char* buf = smem + ((st - first) & 1) * BUF;
-      Frag<F32> dbf[TR / 16];
-      if (own_bias) {
-        const int b = st / nst;
-        const uint32_t p0 = (uint32_t)(st - b * nst) * TR;
+      if (own) {
 #pragma unroll
         for (int k = 0; k < TR / 16; ++k) {
-          float v[8];
+          const Frag<F32> fa = frag_a(buf, at, k);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const uint32_t q = p0 + k * 16 + 8 * (e / 4) + 4 * hh + e % 4;
-            v[e] = (l32 < p.H && q < (uint32_t)p.LL) ? load1<A, false>(p.db, ((int64_t)b * p.H + l32) * p.LL + q) : 0.f;
-          }
-          pack<A>(v, dbf[k]);
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < TR / 16; ++k) {
-        const Frag<F32> fa = sub_frag_t<F32>(buf + at * SUB, k * 16, fo, l32, hh);
-#pragma unroll
-        for (int n = 0; n < 2; ++n)
-          if (own[n]) acc[n] = mma<A>(fa, sub_frag_t<F32>(buf + (W / 32 + bt[n]) * SUB, k * 16, fo, l32, hh), acc[n]);
-        if (own_sum) {
-          // (rows beyond the end repeat the last one here: the ones are zero there)
-          Frag<F32> o1 = ones;
-          const int b = st / nst;
-          const uint32_t left = (uint32_t)p.LL - (uint32_t)(st - b * nst) * TR;
-          if (left < (uint32_t)TR) {
-            float v[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = (uint32_t)(k * 16 + 8 * (e / 4) + 4 * hh + e % 4) < left ? 1.0f : 0.0f;
-            pack<A>(v, o1);
-          }
-          sums = mma<A>(fa, o1, sums);
-        }
-        if (own_bias) {
-          accb = mma<A>(dbf[k], sub_frag_t<F32>(buf + (W / 32 + wave - 4) * SUB, k * 16, fo, l32, hh), accb);
-          if (wave == 4) sumb = mma<A>(dbf[k], ones, sumb);
+          for (int n = 0; n < NT; ++n)
+            acc[n] = mma<A>(fa, sub_frag_t<F32>(buf + ABYTES + (wave / NA + n * (8 / NA)) * SUB, k * 16, fo, l32, hh), acc[n]);
         }
       }
       if (st + 1 < last) {
-        put(smem + ((st + 1 - first) & 1) * BUF);
+        put(smem + ((st + 1 - first) & 1) * BUF, st + 1);
         if (st + 2 < last) fetch(st + 2);
       }
       __syncthreads();
     }
   }
   // partial of this chunk
-  float* out = p.part + ((size_t)sec * p.nchunks + chunk) * wgrad_part_floats(C, HD, p.H);
-  const int ncol = nb * 32;
+  float* out = p.part + ((size_t)sec * p.nchunks + chunk) * wgrad_part_floats(C, HD);
+  const int rows = KIND == kWgradBias ? p.H : NA * 32;
 #pragma unroll
-  for (int n = 0; n < 2; ++n)
-    if (own[n])
+  for (int r = 0; r < 16; ++r) {
+    const int a = at * 32 + 8 * (r / 4) + 4 * hh + r % 4;
+    if (a >= rows || !own) continue;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) out[(size_t)(at * 32 + 8 * (r / 4) + 4 * hh + r % 4) * ncol + bt[n] * 32 + l32] = acc[n][r];
-  float* osum = out + (size_t)C * HD;
-  if (own_sum && l32 == 0)
+    for (int n = 0; n < NT; ++n) out[(size_t)a * (NB * 32) + (wave / NA + n * (8 / NA)) * 32 + l32] = acc[n][r];
+  }
+  float* ssum = reinterpret_cast<float*>(smem);  // (the last stage has been read: every wave is past its barrier)
+  constexpr int PER = KIND == kWgradBias ? TR : 512 / (NA * 4);
+  if constexpr (KIND == kWgradBias) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) osum[at * 32 + 8 * (r / 4) + 4 * hh + r % 4] = sums[r];
-  if (own_bias) {
-    float* ob = osum + W;
+    for (int n = 0; n < PD; ++n) ssum[tid + 512 * n] = csum[n];
+  } else {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int h = 8 * (r / 4) + 4 * hh + r % 4;
-      if (h < p.H) {
-        ob[(size_t)h * C + (wave - 4) * 32 + l32] = accb[r];
-        if (wave == 4 && l32 == 0) ob[(size_t)p.H * C + h] = sumb[r];
-      }
+    for (int e = 0; e < 8; ++e) ssum[((tid % (NA * 4)) * 8 + e) * (PER + 1) + tid / (NA * 4)] = csum[e];
+  }
+  __syncthreads();
+  if (tid < rows) {
+    float s = 0.f;
+    for (int k = 0; k < PER; ++k) s += ssum[KIND == kWgradBias ? tid * TR + k : tid * (PER + 1) + k];
+    out[(size_t)C * HD + tid] = s;
+  }
+}
+
+template <class A, bool F32, int C, int HD>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) blk_wgrad_kernel(BlockParams p) {
+  extern __shared__ char smem[];
+  const int slot = (int)blockIdx.x / kXcds;
+  const int sec = slot % kWgradSections, chunk = (slot / kWgradSections) * kXcds + (int)blockIdx.x % kXcds;
+  if (sec < 3) wgrad_body<A, F32, C, HD, kWgradQkv>(p, sec, chunk, smem);
+  else if (sec == 3) wgrad_body<A, F32, C, HD, kWgradGate>(p, sec, chunk, smem);
+  else if (sec == 4) wgrad_body<A, F32, C, HD, kWgradOut>(p, sec, chunk, smem);
+  else wgrad_body<A, F32, C, HD, kWgradBias>(p, sec, chunk, smem);
+}
+
+// Sums the chunks in a fixed order: a workgroup takes four rows of the projections' gradients (4*HD, then H of the
+// bias projection) or of the output projection's (C), its threads four columns of a row and a group of chunks each.
+// The rows' contributions to dgamma[c] = sum_n W[n][c] G[n][c] and dbeta[c] = sum_n W[n][c] * (sum over the
+// pair rows of d[n]) go to p.red, one pair of rows of C floats per workgroup.
+__host__ __device__ inline int reduce_proj_groups(int HD, int H) { return (4 * HD + H + 3) / 4; }
+template <class A, bool F32, int C, int HD>
+__global__ void __launch_bounds__(1024) blk_reduce_kernel(BlockParams p) {
+  __shared__ float4 part[1024];
+  __shared__ float psum[1024];
+  const int tid = threadIdx.x, ngp = reduce_proj_groups(HD, p.H);
+  const bool proj = (int)blockIdx.x < ngp;
+  const int quads = (proj ? C : HD) / 4, groups = 256 / quads;
+  const int row = tid / (quads * groups), grp = (tid / quads) % groups, c = (tid % quads) * 4;
+  const int n = (proj ? (int)blockIdx.x : (int)blockIdx.x - ngp) * 4 + row, nall = 4 * HD + p.H;
+  const bool valid = !proj || n < nall;
+  const int sec = !proj ? 4 : n < 4 * HD ? n / HD : 5, r = !proj ? n : n < 4 * HD ? n % HD : n - 4 * HD;
+  const size_t pf = wgrad_part_floats(C, HD);
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+  float sum = 0.f;
+  if (valid) {
+    const float* src = p.part + (size_t)sec * p.nchunks * pf;
+#pragma unroll 8
+    for (int k = grp; k < p.nchunks; k += groups) {
+      const float4 v = *reinterpret_cast<const float4*>(src + (size_t)k * pf + (size_t)r * (quads * 4) + c);
+      a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
+      sum += src[(size_t)k * pf + (size_t)C * HD + r];
     }
   }
-}
-
-// Sums the chunks in order, four columns per thread: rows [0, 4*HD) the projections, then H of the bias
-// projection, then C of the output projection.
-template <class A, bool F32>
-__global__ void __launch_bounds__(256) blk_reduce_kernel(BlockParams p, int C) {
-  const int HD = p.HD, H = p.H, W = C > HD ? C : HD;
-  const size_t pf = wgrad_part_floats(C, HD, H);
-  const int cq = C / 4, nproj = (4 * HD + H) * cq, nout = C * (HD / 4);
-  const int t = (int)(blockIdx.x * 256 + threadIdx.x);
-  if (t >= nproj + nout) return;
-  const float* src;
-  const float* ssum;
-  int n, c;
-  if (t < nproj) {
-    n = t / cq;
-    c = (t % cq) * 4;
-    const int s = n < 4 * HD ? n / HD : 0;
-    src = p.part + (size_t)s * p.nchunks * pf;
-    if (n < 4 * HD) { ssum = src + (size_t)C * HD + n % HD; src += (size_t)(n % HD) * C + c; }
-    else { src += (size_t)C * HD + W; ssum = src + (size_t)H * C + (n - 4 * HD); src += (size_t)(n - 4 * HD) * C + c; }
-  } else {
-    const int u = t - nproj;
-    n = u / (HD / 4);
-    c = (u % (HD / 4)) * 4;
-    src = p.part + (size_t)4 * p.nchunks * pf;
-    ssum = src + (size_t)C * HD + n;
-    src += (size_t)n * HD + c;
+  part[tid] = a;
+  psum[tid] = sum;
+  __syncthreads();
+  float dg[4] = {0.f, 0.f, 0.f, 0.f}, db[4] = {0.f, 0.f, 0.f, 0.f};
+  if (grp == 0 && valid) {
+    float g[4] = {a.x, a.y, a.z, a.w};
+    for (int k = 1; k < groups; ++k) {
+      const float4 v = part[tid + k * quads];
+      g[0] += v.x; g[1] += v.y; g[2] += v.z; g[3] += v.w;
+      sum += psum[tid + k * quads];
+    }
+    if (proj) {
+      void* dst = sec < 4 ? p.dw[sec] : p.dwb;
+      const void* w = sec < 4 ? p.w[sec] : p.wb;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float wv = load1<A, F32>(w, (int64_t)r * C + c + e);
+        store1<A, F32>(dst, (int64_t)r * C + c + e, load1<A, F32>(p.gamma, c + e) * g[e] + load1<A, F32>(p.beta, c + e) * sum);
+        dg[e] = wv * g[e];
+        db[e] = wv * sum;
+      }
+      if (c == 0 && sec == 3 && p.dbg != nullptr) store1<A, F32>(p.dbg, r, sum);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) store1<A, F32>(p.dwo, (int64_t)r * HD + c + e, g[e]);
+      if (c == 0 && p.dbo != nullptr) store1<A, F32>(p.dbo, r, sum);
+    }
   }
-  float a[4] = {0.f, 0.f, 0.f, 0.f}, sum = 0.f;
-  for (int k = 0; k < p.nchunks; ++k) {
-    const float* s = src + (size_t)k * pf;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) a[e] += s[e];
-    sum += ssum[(size_t)k * pf];
+  if (!proj) return;
+  // over the workgroup's four rows
+  __shared__ float4 sg[4 * (C / 4)], sb[4 * (C / 4)];
+  if (grp == 0) {
+    sg[row * quads + c / 4] = make_float4(dg[0], dg[1], dg[2], dg[3]);
+    sb[row * quads + c / 4] = make_float4(db[0], db[1], db[2], db[3]);
   }
-  if (t < nproj) {
-    float* g = p.red + (size_t)n * C + c;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) g[e] = a[e];
-    if (c == 0) p.red[(size_t)(4 * HD + H) * C + n] = sum;
-    void* dst = n < 4 * HD ? p.dw[n / HD] : p.dwb;
-    const int64_t off = (int64_t)(n < 4 * HD ? n % HD : n - 4 * HD) * C + c;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      store1<A, F32>(dst, off + e, load1<A, F32>(p.gamma, c + e) * a[e] + load1<A, F32>(p.beta, c + e) * sum);
-    if (c == 0 && n >= 3 * HD && n < 4 * HD && p.dbg != nullptr) store1<A, F32>(p.dbg, n - 3 * HD, sum);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) store1<A, F32>(p.dwo, (int64_t)n * HD + c + e, a[e]);
-    if (c == 0 && p.dbo != nullptr) store1<A, F32>(p.dbo, n, sum);
+  __syncthreads();
+  const float* f = reinterpret_cast<const float*>(tid < C ? sg : sb);
+  if (tid < 2 * C) {
+    const int col = tid % C;
+    p.red[((size_t)blockIdx.x * 2 + tid / C) * C + col] = f[col] + f[C + col] + f[2 * C + col] + f[3 * C + col];
   }
 }
 
-// dgamma[c] = sum_n W[n][c] G[n][c], dbeta[c] = sum_n W[n][c] * (sum over the rows of d[n]): 16 columns per workgroup.
+// dgamma and dbeta from the workgroups' contributions: 16 columns per workgroup.
 template <class A, bool F32>
-__global__ void __launch_bounds__(512) blk_norm_grad_kernel(BlockParams p, int C) {
-  __shared__ float sg[512], sb[512];
-  const int tid = threadIdx.x, c = (int)blockIdx.x * 16 + tid % 16, nall = 4 * p.HD + p.H;
-  float g = 0.f, b = 0.f;
-  for (int n = tid / 16; n < nall; n += 32) {
-    const float w = n < 4 * p.HD ? load1<A, F32>(p.w[n / p.HD], (int64_t)(n % p.HD) * C + c)
-                                 : load1<A, F32>(p.wb, (int64_t)(n - 4 * p.HD) * C + c);
-    g = __builtin_fmaf(w, p.red[(size_t)n * C + c], g);
-    b = __builtin_fmaf(w, p.red[(size_t)nall * C + n], b);
-  }
-  sg[tid] = g;
-  sb[tid] = b;
-  for (int s = 256; s >= 16; s /= 2) {
+__global__ void __launch_bounds__(1024) blk_norm_grad_kernel(BlockParams p, int C) {
+  __shared__ float sm[1024];
+  const int tid = threadIdx.x, col = (int)blockIdx.x * 16 + tid % 16, ngp = reduce_proj_groups(p.HD, p.H);
+  float s = 0.f;  // (columns 0 .. C-1: dgamma, C .. 2C-1: dbeta)
+  for (int n = tid / 16; n < ngp; n += 64) s += p.red[(size_t)n * 2 * C + col];
+  sm[tid] = s;
+  for (int w = 512; w >= 16; w /= 2) {
     __syncthreads();
-    if (tid < s) { sg[tid] += sg[tid + s]; sb[tid] += sb[tid + s]; }
+    if (tid < w) sm[tid] += sm[tid + w];
   }
-  if (tid < 16) {
-    store1<A, F32>(p.dgamma, c, sg[tid]);
-    store1<A, F32>(p.dbeta, c, sb[tid]);
-  }
+  if (tid < 16) store1<A, F32>(col < C ? p.dgamma : p.dbeta, col < C ? col : col - C, sm[tid]);
 }
 
 }  // namespace
@@ -916,8 +1019,6 @@ constexpr int kCus = 256;
 // (element type, fp32 block) instances
 #define FTA_BLOCK_TYPES(X, ...) \
   if (dtype == kF16) X(F16, false, __VA_ARGS__) else if (dtype == kBF16) X(BF16, false, __VA_ARGS__) else X(F16, true, __VA_ARGS__)
-#define FTA_BLOCK_C(X) \
-  if (C == 64) { FTA_BLOCK_TYPES(X, 64) } else { FTA_BLOCK_TYPES(X, 128) }
 #define FTA_BLOCK_C_HD(X)                                                                         \
   if (C == 64 && p.HD == 64) { FTA_BLOCK_TYPES(X, 64, 64) } else if (C == 64) { FTA_BLOCK_TYPES(X, 64, 128) } \
   else if (p.HD == 64) { FTA_BLOCK_TYPES(X, 128, 64) } else { FTA_BLOCK_TYPES(X, 128, 128) }
@@ -939,16 +1040,12 @@ int workgroups(long items, int waves, int most) {
 }  // namespace
 
 hipError_t launch_block_proj(BlockParams p, int C, int dtype, hipStream_t st) {
-  const long blocks = (long)p.B * p.nper;
-  const int ntiles = 4 * p.HD / 32 + (p.H + 31) / 32, KS = C / 16;
-  const size_t extra = (size_t)(2 * C + p.HD) * sizeof(float);
-  int gy = 1;
-  while ((size_t)((ntiles + gy - 1) / gy) * KS * frag_bytes(dtype) + extra > 160 * 1024) ++gy;
-  const size_t smem = (size_t)((ntiles + gy - 1) / gy) * KS * frag_bytes(dtype) + extra;
-  p.cg = column_groups(blocks * gy, 8);
-  const dim3 grid((unsigned)workgroups(blocks * p.cg, 8, kCus / gy), (unsigned)gy), block(512);
-#define FTA_BLOCK_CASE(AA, FF, CC) return launch_kernel(blk_proj_kernel<AA, FF, CC>, p, grid, block, smem, st);
-  FTA_BLOCK_C(FTA_BLOCK_CASE)
+  // two stage buffers of 64 rows (fp32: 32) and the bias projection's weights
+  const int rows = dtype == 2 ? 32 : 64;
+  const size_t smem = (size_t)(2 * rows / 32 + 1) * (C / 16) * frag_bytes(dtype) + (p.HD + 2 * rows) * sizeof(float);
+  const dim3 grid((unsigned)workgroups((long)p.B * ((p.LL + rows - 1) / rows), 1, kCus)), block(512);
+#define FTA_BLOCK_CASE(AA, FF, CC, HH) return launch_kernel(blk_proj_kernel<AA, FF, CC, HH>, p, grid, block, smem, st);
+  FTA_BLOCK_C_HD(FTA_BLOCK_CASE)
 #undef FTA_BLOCK_CASE
 }
 
@@ -974,46 +1071,31 @@ hipError_t launch_block_dout(BlockParams p, int C, int dtype, hipStream_t st) {
 }
 
 hipError_t launch_block_dx(BlockParams p, int C, int dtype, hipStream_t st) {
-  const long blocks = (long)p.B * p.nper;
-  const size_t wbytes = (size_t)(C / 32) * (4 * p.HD / 16 + (p.H + 15) / 16) * frag_bytes(dtype);
-  // Weights in LDS where they fit and a workgroup has a row block for each of its eight waves; few row blocks
-  // run as many small workgroups that read the weights from the cache.
-  const bool wlds = wbytes + C * sizeof(float) <= 160 * 1024 && blocks >= 4 * kCus;
-  int nw = 8;
-  while (nw > 1 && blocks < (long)nw * kCus) nw /= 2;
-  const dim3 grid((unsigned)workgroups(blocks, nw, wlds ? kCus : 2 * kCus * 8 / nw)), block((unsigned)(64 * nw));
-  const size_t smem = (wlds ? wbytes : 0) + C * sizeof(float);
-#define FTA_BLOCK_CASE(AA, FF, CC, HH)                                                                      \
-  {                                                                                                         \
-    if constexpr (!FF)                                                                                      \
-      if (wlds) return launch_kernel(blk_dx_kernel<AA, FF, CC, HH, true>, p, grid, block, smem, st);        \
-    return launch_kernel(blk_dx_kernel<AA, FF, CC, HH, false>, p, grid, block, smem, st);                   \
-  }
+  const int rows = dtype == 2 ? 32 : 64, split = 8 / (rows / 32 * (C / 32));
+  const size_t smem = (size_t)(rows / 32) * (4 * p.HD / 16 + 1) * frag_bytes(dtype) + (size_t)split * rows * (C + 4) * sizeof(float);
+  const dim3 grid((unsigned)workgroups((long)p.B * ((p.LL + rows - 1) / rows), 1, kCus)), block(512);
+#define FTA_BLOCK_CASE(AA, FF, CC, HH) return launch_kernel(blk_dx_kernel<AA, FF, CC, HH>, p, grid, block, smem, st);
   FTA_BLOCK_C_HD(FTA_BLOCK_CASE)
 #undef FTA_BLOCK_CASE
 }
 
 hipError_t launch_block_wgrad(BlockParams p, int C, int dtype, hipStream_t st) {
-  const int W = C > p.HD ? C : p.HD;
-  const size_t smem = (size_t)2 * 2 * (W / 32) * (dtype == 2 ? 32 * 128 : 64 * 64);
-  const dim3 grid((unsigned)(5 * p.nchunks)), block(512);
-#define FTA_BLOCK_CASE(AA, FF, CC, HH)                                                          \
-  {                                                                                             \
-    hipError_t e = launch_kernel(blk_wgrad_kernel<AA, FF, CC, HH>, p, grid, block, smem, st);   \
-    if (e != hipSuccess) return e;                                                              \
+  // (the largest section: both operands C or HD columns wide; the bias section has one row per head)
+  const int sub = dtype == 2 ? 32 * 128 : 64 * 64, n = (p.HD + C) / 32;
+  const size_t smem = (size_t)2 * n * sub;
+  const dim3 grid((unsigned)(kWgradSections * p.nchunks)), block(512);
+  const dim3 rgrid((unsigned)(reduce_proj_groups(p.HD, p.H) + C / 4));
+#define FTA_BLOCK_CASE(AA, FF, CC, HH)                                                                       \
+  {                                                                                                          \
+    hipError_t e = launch_kernel(blk_wgrad_kernel<AA, FF, CC, HH>, p, grid, block, smem, st);                \
+    if (e != hipSuccess) return e;                                                                           \
+    hipLaunchKernelGGL((blk_reduce_kernel<AA, FF, CC, HH>), rgrid, dim3(1024), 0, st, p);                    \
+    e = hipGetLastError();                                                                                   \
+    if (e != hipSuccess) return e;                                                                           \
+    hipLaunchKernelGGL((blk_norm_grad_kernel<AA, FF>), dim3((unsigned)(2 * CC / 16)), dim3(1024), 0, st, p, CC); \
+    return hipGetLastError();                                                                                \
   }
   FTA_BLOCK_C_HD(FTA_BLOCK_CASE)
-#undef FTA_BLOCK_CASE
-  const int nred = (4 * p.HD + p.H) * (C / 4) + C * (p.HD / 4);
-#define FTA_BLOCK_CASE(AA, FF, UNUSED)                                                                                    \
-  {                                                                                                                       \
-    hipLaunchKernelGGL((blk_reduce_kernel<AA, FF>), dim3((unsigned)((nred + 255) / 256)), dim3(256), 0, st, p, C);        \
-    hipError_t e = hipGetLastError();                                                                                     \
-    if (e != hipSuccess) return e;                                                                                        \
-    hipLaunchKernelGGL((blk_norm_grad_kernel<AA, FF>), dim3((unsigned)(C / 16)), dim3(512), 0, st, p, C);                 \
-    return hipGetLastError();                                                                                             \
-  }
-  FTA_BLOCK_TYPES(FTA_BLOCK_CASE, 0)
 #undef FTA_BLOCK_CASE
 }
 
@@ -1051,13 +1133,14 @@ BlockLayout block_layout(const fta_block& b) {
   l.state = at;
   at = 0;
   l.dog = take(2 * n); l.dgp = take(es * n); l.dq = take(2 * n); l.dk = take(2 * n); l.dv = take(2 * n); l.db = take(2 * m);
-  l.wt = take((size_t)(b.C / 32) * (4 * HD / 16 + (b.H + 15) / 16) * frag_bytes(b.dtype));
-  // Chunks of the weight-gradient kernel: 51 x 5 sections fill the chip once; a chunk keeps at least four stages,
-  // so that its partial sums (64 KB at C = H*D = 128) are not what the launch spends its time on.
+  l.wt = take((size_t)(b.C / 32) * (4 * HD / 16 + 1) * frag_bytes(b.dtype));
+  // Chunks of the weight-gradient kernel, a multiple of the dies: six sections of 80 are 480 workgroups, of which two
+  // fit a CU (56: 118 us at 384 x 384 pairs in bf16, 40: 110, 80: 91).  A chunk keeps at least four stages, so that its partial sums (64 KB at C = H*D = 128) are not
+  // what the launch spends its time on.
   const size_t rows = b.dtype == FTA_DTYPE_F32 ? 32 : 64, stages = b.B * ((LL + rows - 1) / rows);
-  l.nchunks = (int)(stages / 4 < 1 ? 1 : stages / 4 > 51 ? 51 : stages / 4);
-  l.part = take((size_t)5 * l.nchunks * wgrad_part_floats(b.C, (int)HD, b.H) * sizeof(float));
-  l.red = take((4 * HD + b.H) * (b.C + 1) * sizeof(float));
+  l.nchunks = kXcds * (int)(stages < 64 ? 1 : stages > 32 * 10 ? 10 : stages / 32);
+  l.part = take((size_t)kWgradSections * l.nchunks * wgrad_part_floats(b.C, (int)HD) * sizeof(float));
+  l.red = take((size_t)reduce_proj_groups((int)HD, b.H) * 2 * b.C * sizeof(float));
   const fta_options opt = attn_options(b);
   l.attn_bytes = fta_bwd_workspace_bytes_ex(b.B, b.H, b.L, b.L, b.D, &opt);
   l.attn = take(l.attn_bytes);
