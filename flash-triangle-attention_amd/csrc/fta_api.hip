@@ -116,7 +116,7 @@ struct PlanKey {
   int B, H, L1, L2, D, mask;
   bool operator==(const PlanKey& o) const { return B == o.B && H == o.H && L1 == o.L1 && L2 == o.L2 && D == o.D && mask == o.mask; }
 };
-// The length the tiles of one direction cover for rows of L2 keys: the smallest multiple of 128 that is at
+// The length the tiles of one direction cover for rows of L2 keys: the smallest multiple of 128 (forward: 64) that is at
 // least L2 and that the direction has a workgroup shape for (0 if there is none up to FTA_MAX_L2).  The
 // two directions need not agree (nothing they exchange is laid out by it: lse has the row's true length):
 // the backward has a shape for every multiple of 128, the forward skips a few (D = 32: 11 and 25 blocks
@@ -124,8 +124,10 @@ struct PlanKey {
 // (`feat`: 1 for the backward's vector-ALU instances, 2 for dropout, which has fewer instances in both
 // directions)
 int padded_len_fwd(int L2, int D, int feat) {
-  for (int lp = (L2 + 127) / 128 * 128; lp <= FTA_MAX_L2; lp += 128)
-    if (fta::plan_fwd(1, 1, 1, lp, D, feat == 2).valid) return lp;
+  for (int lp = (L2 + 63) / 64 * 64; lp <= FTA_MAX_L2; lp += 64) {
+    const fta::FwdPlan pl = fta::plan_fwd(1, 1, 1, lp, D, feat == 2);
+    if (pl.valid && (lp % 128 == 0 || pl.fwd1 == 1)) return lp;  // (only the hand-scheduled kernel has shapes in between)
+  }
   return 0;
 }
 int padded_len_bwd(int L2, int D, int feat) {

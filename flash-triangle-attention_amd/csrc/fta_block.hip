@@ -634,8 +634,8 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
     floatx16 acc = zero16();
 #pragma unroll
     for (int k = 0; k < KW; ++k) {
-      const int ks = share * KW + k;
-      if (ks < KALL) acc = mma<A>(w[k], piece_frag<F32>(smem + rs * SUB, ks, l32, hh), acc);
+      const int ks = SPLIT == 1 ? k : min(share * KW + k, KALL - 1);  // (a share's steps beyond the end: the last one again, with zero weights)
+      acc = mma<A>(w[k], piece_frag<F32>(smem + rs * SUB, ks, l32, hh), acc);
     }
     float* plane = dxs + ((size_t)share * TR + rs * 32 + l32) * XROW + ct * 32 + 4 * hh;
 #pragma unroll

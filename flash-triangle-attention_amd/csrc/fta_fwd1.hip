@@ -1,4 +1,4 @@
-// Forward, hand-scheduled variant for rows of one key slab (D = 32, tiled length 128 ... 512).
+// Forward, hand-scheduled variant for rows of one key slab (D = 32, tiled length 64 ... 512).
 // Same mathematics and the same decomposition as fta_fwd_kernel (fta_fwd_kernel.h): a wave owns 32
 // queries and all keys of a (b,h), keeps its bias tile in registers and walks a chunk of L1 rows;
 // replaces upstream's _attn_fwd / _attn_fwd_inner (flash_tt_attn.py:49-109, :128-264).  What differs
@@ -23,9 +23,10 @@
 
 namespace fta {
 
-// T: element type; NKT: 32-key tiles per row (4, 8, 12 or 16); TAIL: the row's true length L2 is shorter
-// than the 32*NKT keys the tiles cover (keys beyond it masked, queries beyond it computed on copies of
-// the last one and not stored); W: waves (query blocks of 32) per workgroup, 4 or 8.
+// T: element type; NKT: 32-key tiles per row (even, 2 to 16: the score tiles alternate between two register
+// tuples, so an odd count would end a row on the wrong one); TAIL: the row's true length L2 is shorter
+// than the 32*NKT keys the tiles cover, or than the workgroups' query blocks (keys beyond it masked, queries
+// beyond it computed on copies of the last one and not stored); W: waves (query blocks of 32) per workgroup, 4 or 8.
 // Two waves share a SIMD either way.  With W = 4 they belong to two independent workgroups, and the
 // hardware lets the older one issue first whenever both are ready, which in a kernel bound by the
 // vector ALU is nearly always: measured with a clock around every workgroup, the older workgroup of a CU
@@ -34,16 +35,33 @@ namespace fta {
 // stage barrier, so neither runs ahead, and the K/V stage is copied into LDS once for eight query blocks.
 template <class T, int NKT, bool TAIL, int W, int G = 4>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_waves_per_eu(2, 2))) fta_fwd1_kernel(const FwdParams p) {
-  static_assert(W == 4 || W == 8, "one or two waves per SIMD from the same workgroup");
-  static_assert(G == 4 || (G == 8 && W == 8), "stages of 128 keys, or of 256 where one workgroup has the CU's LDS to itself");
+  static_assert(W == 2 || W == 4 || W == 8, "one or two waves per SIMD from the same workgroup (rows of up to 64 keys: two waves)");
+  static_assert(G == 4 || (G == 8 && W == 8) || (G == 2 && NKT == 2), "stages of 128 keys, of 256 where one workgroup has the CU's LDS to itself, of 64 for such rows");
   constexpr int D = 32, KS = 2;
   constexpr int NCU = 2 * G / W;               // copies per wave and stage of K, and of V (a stage has 2*G pieces of 1 KB of each)
   constexpr int KT = 32 * G;                   // keys per stage
-  constexpr int NST = NKT / G;                 // stages per row
+  constexpr int NST = (NKT + G - 1) / G;       // stages per row, the last one of NKT % G tiles where that is not 0
   constexpr int R = 4;                         // ring slots
   constexpr uint32_t TILE_B = KT * D * 2;      // bytes of a staged K (or V) tile
   constexpr uint32_t SLOT_B = 2 * TILE_B;      // K tile, then V tile
-  static_assert(NKT % G == 0 && NKT >= 4 && NKT <= 16, "whole stages, bias within the register budget");
+  static_assert(NKT % 2 == 0 && NKT >= 2 && NKT <= 16, "an even number of tiles, bias within the register budget");
+  // Stage w of a row: its tiles, and the copies a wave issues for it (of K, and as many of V).
+  constexpr auto tiles_of = [](int w) { return (w + 1) * G <= NKT ? G : NKT - w * G; };
+  constexpr auto ncu_of = [=](int w) { return (2 * tiles_of(w) + W - 1) / W; };
+  // Iteration t issues the scores of tile tn = (t + 1) % NKT, and the tn % G-th share of the copies of the stage two
+  // behind tile tn's: `first` to `end`, the K copies before the V copies.
+  struct Share { int stage, first, end; };
+  constexpr auto share_of = [=](int tn) {
+    const int w = tn / G, fill = (w + 2) % NST, total = 2 * ncu_of(fill), per = (total + tiles_of(w) - 1) / tiles_of(w);
+    const int a = (tn % G) * per;
+    return Share{fill, a < total ? a : total, a + per < total ? a + per : total};
+  };
+  // copies issued between the request for the next row's Q and the last barrier of the row
+  constexpr auto behind_q = [=]() {
+    int n = 0;
+    for (int tn = 1; tn < NKT; ++tn) n += share_of(tn).end - share_of(tn).first;
+    return n;
+  };
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
 
@@ -105,13 +123,14 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
   // ---- stage copies: a stage is 32*G K rows and 32*G V rows of 64 bytes, 1 KB per wave instruction,
   // NCU K and NCU V copies per wave; copy u of wave w carries the 16-byte pieces (w + W*u)*64 .. +63.
   uint32_t goffk[NCU], goffv[NCU];
-  [[maybe_unused]] uint32_t goffk_t[NCU], goffv_t[NCU];  // TAIL: the row's last stage (rows beyond the last key are copies of it)
+  constexpr bool CLAMP = TAIL || NKT % G != 0;
+  [[maybe_unused]] uint32_t goffk_t[NCU], goffv_t[NCU];  // CLAMP: the row's last stage (rows beyond the last key are copies of it)
 #pragma unroll
   for (int u = 0; u < NCU; ++u) {
     const int pidx = (wave + W * u) * 64 + lane, row = pidx >> 2, chunkk = swz_slot<D>(row, pidx & 3);
     goffk[u] = (uint32_t)(((int64_t)row * p.ks[3] + chunkk * 8) * 2);
     goffv[u] = (uint32_t)(((int64_t)row * p.vs[3] + chunkk * 8) * 2);
-    if constexpr (TAIL) {
+    if constexpr (CLAMP) {
       const int grow = min((NST - 1) * KT + row, last) - (NST - 1) * KT;
       goffk_t[u] = (uint32_t)(((int64_t)grow * p.ks[3] + chunkk * 8) * 2);
       goffv_t[u] = (uint32_t)(((int64_t)grow * p.vs[3] + chunkk * 8) * 2);
@@ -147,13 +166,18 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
     fill_lds = lds0 + wofs + (uint32_t)fill_slot * SLOT_B;
     fill_slot = (fill_slot + 1) & (R - 1);
   };
-  // copy c (first the K copies, then the V copies; nothing for c >= 2*NCU) of the stage begun last,
-  // which is stage number w of its row
+  // copy c (first the K copies, then the V copies) of the stage begun last, which is stage number w of
+  // its row
   auto fill_copy = [&](auto wc, auto cc) {
-    constexpr int w = decltype(wc)::value, c = decltype(cc)::value;
-    constexpr bool TL = TAIL && (w == NST - 1);
-    if constexpr (c < NCU) dma16s_at<(uint32_t)c * W * 1024u>(TL ? goffk_t[c] : goffk[c], kst, fill_lds);
-    else if constexpr (c < 2 * NCU) dma16s_at<TILE_B + (uint32_t)(c - NCU) * W * 1024u>(TL ? goffv_t[c - NCU] : goffv[c - NCU], vst, fill_lds);
+    constexpr int w = decltype(wc)::value, c = decltype(cc)::value, nk = ncu_of(w);
+    constexpr bool TL = CLAMP && (w == NST - 1);
+    static_assert(c < 2 * nk, "a copy of the stage");
+    if constexpr (c < nk) dma16s_at<(uint32_t)c * W * 1024u>(TL ? goffk_t[c] : goffk[c], kst, fill_lds);
+    else dma16s_at<TILE_B + (uint32_t)(c - nk) * W * 1024u>(TL ? goffv_t[c - nk] : goffv[c - nk], vst, fill_lds);
+  };
+  auto fill_share = [&](auto tc) {
+    constexpr Share sh = share_of(decltype(tc)::value);
+    static_for<sh.first, sh.end>([&](auto cc) { fill_copy(std::integral_constant<int, sh.stage>{}, cc); });
   };
 
   // ---- Q^T B-operand fragments of one row, straight into registers (contraction step ks holds
@@ -188,15 +212,15 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
   const float lg2e = kLog2e;
   const uint32_t ones = T::is_bf16 ? 0x3F803F80u : 0x3C003C00u;
 
-  // ---- prologue: stages 0 and 1 whole, the first copy of stage 2 (the one the iteration "before the
+  // ---- prologue: stages 0 and 1 whole, the first share of stage 2 (the one the iteration "before the
   // first" would have issued), Q of row 0; then the scores of tile 0
   static_for<0, 2>([&](auto nc) {
     constexpr int n = decltype(nc)::value;
     fill_begin(std::integral_constant<int, n % NST>{}, n > 0);
-    static_for<0, 2 * NCU>([&](auto cc) { fill_copy(std::integral_constant<int, n % NST>{}, cc); });
+    static_for<0, 2 * ncu_of(n % NST)>([&](auto cc) { fill_copy(std::integral_constant<int, n % NST>{}, cc); });
   });
   fill_begin(std::integral_constant<int, 2 % NST>{}, true);
-  fill_copy(std::integral_constant<int, 2 % NST>{}, std::integral_constant<int, 0>{});
+  fill_share(std::integral_constant<int, 0>{});
   q_issue(false);
   wait_vmem_all();
   __builtin_amdgcn_s_barrier();
@@ -278,28 +302,26 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
     static_for<0, NKT>([&](auto tc) {
       constexpr int t = decltype(tc)::value;
       constexpr int tn = (t + 1) % NKT;           // the tile whose scores this iteration produces
-      constexpr bool PUB = ((t + 1) % G == 0);    // tile t+1 opens a stage: publish it first
-      constexpr int c = (t + 1) % G;              // the copy this iteration issues
-      constexpr int fw = ((t + 1) / G + 2) % NST;  // number, in its row, of the stage being filled
+      constexpr bool PUB = (tn % G == 0);         // tile t+1 opens a stage: publish it first
       floatx16& sc = s[t & 1];
       floatx16& sn = s[(t + 1) & 1];
 
       if constexpr (PUB) {
-        // everything but the copies of the stage after it has landed (copies retire in order; in a row of
-        // one stage fewer copies separate the Q loads of the next row from this wait)
-        static_assert(W == 4 || NKT > G, "rows of one stage run the four-wave instances");
-        constexpr int allowed = (W == 8) ? 2 * NCU : (t == NKT - 1 && NKT - 1 < G) ? NKT - 1 : G;
+        // everything but the copies of the stage after it has landed (copies retire in order; the last wait of
+        // a row also covers the Q loads of the next row, which fewer copies may separate from it)
+        constexpr int ahead = 2 * ncu_of((tn / G + 1) % NST);
+        constexpr int allowed = (t == NKT - 1 && behind_q() < ahead) ? behind_q() : ahead;
         __builtin_amdgcn_s_waitcnt(0x0F70 | allowed);
         __builtin_amdgcn_s_barrier();
         kslot = (kslot + 1) & (R - 1);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) aKc[ks] = aK[ks] + (uint32_t)kslot * SLOT_B;
-        fill_begin(std::integral_constant<int, fw>{}, true);  // into the slot the barrier has freed
+        fill_begin(std::integral_constant<int, share_of(tn).stage>{}, true);  // into the slot the barrier has freed
       }
       // K operands of tile t+1
       kf[0] = lds_issue_b128<(tn % G) * 32 * D * 2>(aKc[0]);
       kf[1] = lds_issue_b128<(tn % G) * 32 * D * 2>(aKc[1]);
-      fill_copy(std::integral_constant<int, fw>{}, std::integral_constant<int, c>{});
+      fill_share(std::integral_constant<int, tn>{});
 
       // O^T += V^T P^T of tile t-1, first 16 keys (the V^T operands were read one iteration ago)
       asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(vtl[0]), "+v"(vth[0]), "+v"(vtl[1]), "+v"(vth[1]));
@@ -419,23 +441,26 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
 // ---- host side ---------------------------------------------------------------------------------
 
 bool plan_fwd1(int B, int H, int L1, int L2, int D, FwdPlan& pl) {
-  if (D != 32 || L2 % 128 != 0 || L2 < 128 || L2 > 512) return false;
+  if (D != 32 || L2 % 64 != 0 || L2 < 64 || L2 > 512) return false;
   pl = FwdPlan{};
   pl.NKT = L2 / 32;
   pl.S = 1;
   // eight waves per workgroup where the queries divide that way and such workgroups still fill the chip
   // (see the kernel's comment; same-run A/B at B4 H8: 1.020 against 1.078 ms at L2 = 512, 0.183 against
-  // 0.194 at 256; four-wave workgroups in four rounds instead of two gain 4 %), else four
+  // 0.194 at 256; four-wave workgroups in four rounds instead of two gain 4 %), else four; rows of up to
+  // 64 queries have two query blocks
   const bool fills = (long)B * H * (L2 / 256) * ((L1 + 7) / 8) >= 256;
-  pl.QB = (L2 % 256 == 0 && fills) ? 8 : 4;
-  pl.nqg = L2 / (32 * pl.QB);
+  pl.QB = (L2 % 256 == 0 && fills) ? 8 : L2 <= 64 ? 2 : 4;
+  pl.nqg = (L2 + 32 * pl.QB - 1) / (32 * pl.QB);
   pl.threads = 64 * pl.QB;
   // (stages of 256 keys, which an eight-wave workgroup has the LDS for, halve the barriers and measured
   // the same: 1.040-1.043 against 1.044-1.047 ms at B4 H8 L512; not instantiated)
-  pl.KT = 128;
+  pl.KT = L2 <= 64 ? 64 : 128;
   pl.smem = (size_t)4 * 2 * pl.KT * 32 * 2;  // four slots of a K and a V tile of KT keys
   pl.alias_scratch = 0;
-  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, pl.QB == 8 ? 256 : 512);  // one or two workgroups per CU
+  // two waves per SIMD: one, two or four workgroups per CU.  At least a row per 64 keys in a chunk: a workgroup's set-up
+  // loads one bias row per query, so short rows can be spread thinner (B1 H4 L64: 14.9 us with 8 rows, 5 with 1)
+  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, 256 * 8 / pl.QB, L2 <= 64 ? 1 : L2 / 64);
   pl.rows_per_chunk = (L1 + nch - 1) / nch;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   pl.fwd1 = 1;
@@ -444,7 +469,7 @@ bool plan_fwd1(int B, int H, int L1, int L2, int D, FwdPlan& pl) {
 }
 
 hipError_t launch_fwd1(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 grid, dim3 block, hipStream_t st) {
-  const bool tl = (p.L2 != p.L2p) || p.odd_bias;  // (the instances that mask a row's tail also read the bias entry by entry where they must)
+  const bool tl = (p.L2 % (32 * pl.QB) != 0) || p.odd_bias;  // (the instances that mask a row's tail also read the bias entry by entry where they must)
 #define FTA_FWD1_CASE(NN, WW, GG)                                                                           \
   if (pl.NKT == NN && pl.QB == WW && pl.KT == 32 * GG) {                                                    \
     if (dtype == kBF16)                                                                                     \
@@ -453,7 +478,9 @@ hipError_t launch_fwd1(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 gr
     return tl ? launch_kernel(fta_fwd1_kernel<F16, NN, true, WW, GG>, p, grid, block, pl.smem, st)          \
               : launch_kernel(fta_fwd1_kernel<F16, NN, false, WW, GG>, p, grid, block, pl.smem, st);        \
   }
-  FTA_FWD1_CASE(4, 4, 4) FTA_FWD1_CASE(8, 4, 4) FTA_FWD1_CASE(12, 4, 4) FTA_FWD1_CASE(16, 4, 4)
+  FTA_FWD1_CASE(2, 2, 2)
+  FTA_FWD1_CASE(4, 4, 4) FTA_FWD1_CASE(6, 4, 4) FTA_FWD1_CASE(8, 4, 4) FTA_FWD1_CASE(10, 4, 4)
+  FTA_FWD1_CASE(12, 4, 4) FTA_FWD1_CASE(14, 4, 4) FTA_FWD1_CASE(16, 4, 4)
   FTA_FWD1_CASE(8, 8, 4) FTA_FWD1_CASE(16, 8, 4)
 #undef FTA_FWD1_CASE
   return hipErrorInvalidConfiguration;

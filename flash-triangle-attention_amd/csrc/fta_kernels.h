@@ -52,10 +52,10 @@ struct FwdPlan {
 // workgroups run on the chip at once (256 CUs times the workgroups of this kernel that fit a CU).
 // The launch takes (rounds of workgroups) x (rows per chunk + what a workgroup spends before its
 // first row: bias tile, pipeline fill, measured at about 5 rows' worth); the count that minimises
-// that wins, with at least 8 rows per chunk so that the stationary bias pays off.  (A launch of
-// 2.25 rounds runs as long as one of 3; two rounds of half-length chunks lose to one round.)
-inline int balanced_chunks(long base, int L1, long slots) {
-  const int maxch = (L1 + 7) / 8 > 0 ? (L1 + 7) / 8 : 1;
+// that wins, with at least `least` rows per chunk.  (A launch of 2.25 rounds runs as long as one of 3;
+// two rounds of half-length chunks lose to one round.)
+inline int balanced_chunks(long base, int L1, long slots, int least = 8) {
+  const int maxch = (L1 + least - 1) / least;
   int best = 1;
   long best_cost = -1;
   for (int nch = 1; nch <= maxch; ++nch) {
@@ -192,7 +192,7 @@ inline hipError_t launch_kernel(K kern, const P& p, dim3 grid, dim3 block, size_
 // same for dK/dV (set through fta_debug_select_kernels, for tests of the general kernels).
 int forced_general_mask();
 hipError_t launch_fwd(FwdParams p, const FwdPlan& pl, int D, int dtype, hipStream_t st);
-// The hand-scheduled forward (fta_fwd1.hip): D = 32, tiled length 128 ... 512, no dropout.
+// The hand-scheduled forward (fta_fwd1.hip): D = 32, tiled length 64 ... 512, no dropout.
 bool plan_fwd1(int B, int H, int L1, int L2, int D, FwdPlan& pl);
 hipError_t launch_fwd1(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 grid, dim3 block, hipStream_t st);
 bool plan_fwd2(int B, int H, int L1, int L2, int D, FwdPlan& pl);

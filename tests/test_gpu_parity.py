@@ -329,6 +329,14 @@ def test_rows_of_a_single_key():
         assert got[n].float().abs().max().item() <= 2e-3, n
 
 
+@pytest.mark.parametrize("sm", [1.0 / math.sqrt(32), 1.3])
+@pytest.mark.parametrize("L1,L2", [(7, 33), (64, 64), (5, 65), (9, 192), (3, 193), (40, 320), (6, 321), (17, 448), (2, 449)])
+def test_forward_rows_of_a_number_of_64_key_pairs_of_tiles(L1, L2, sm):
+    """The hand-scheduled D=32 forward tiles a row in steps of 64 keys: a last stage of two tiles instead of four, one stage
+    of two tiles per row (two-wave workgroups) up to 64 keys, query blocks beyond the row's end."""
+    _case(1, 2, L1, L2, 32, sm, seed=23)
+
+
 @pytest.mark.parametrize("L2", [200, 203])
 def test_no_padded_copies_for_lengths_that_are_not_multiples_of_128(L2):
     """L2 = 200 (or 203) is tiled as 256 inside the kernels: peak memory of forward + backward stays within 5 %
