@@ -132,7 +132,7 @@ int padded_len_fwd(int L2, int D, int feat) {
 }
 int padded_len_bwd(int L2, int D, int feat) {
   for (int lp = (L2 + 127) / 128 * 128; lp <= FTA_MAX_L2; lp += 128)
-    if (fta::plan_bwd(1, 1, 1, lp, D, false, feat).valid) return lp;
+    if (fta::plan_bwd(1, 1, 1, lp, D, lp, feat).valid) return lp;
   return 0;
 }
 bool len_supported(int L2, int D, int feat) { return padded_len_fwd(L2, D, feat) != 0 && padded_len_bwd(L2, D, feat) != 0; }
@@ -154,7 +154,7 @@ const fta::BwdPlan& cached_plan_bwd(int B, int H, int L1, int L2, int D, int fea
   const PlanKey k{B, H, L1, L2, D, fta::forced_general_mask() | (feat * 4)};
   if (!(key == k)) {
     const int lp = len_supported(L2, D, feat) ? padded_len_bwd(L2, D, feat) : 0;
-    plan = (lp != 0) ? fta::plan_bwd(B, H, L1, lp, D, lp != L2, feat) : fta::BwdPlan{};
+    plan = (lp != 0) ? fta::plan_bwd(B, H, L1, lp, D, L2, feat) : fta::BwdPlan{};
     plan.L2p = lp;
     key = k;
   }
@@ -361,13 +361,17 @@ int fta_describe_plan_ex(int B, int H, int L1, int L2, int D, float sm_scale, co
   const long bh = (long)B * H;
   const char* tn = (opt.dtype == fta::kBF16) ? "BF16" : "F16";
   char dq[160], dkdv[160];
-  if (b.use_dq1)
+  if (b.use_short) {
+    snprintf(dq, sizeof dq, "fta_bwd_short_kernel<%d,%d> launches=1 grid=%ld block=%d lds=%zu", D, b.sh.NT, bh * b.sh.nchunks, b.sh.threads, b.sh.smem);
+    memcpy(dkdv, dq, sizeof dkdv);
+  } else if (b.use_dq1)
     snprintf(dq, sizeof dq, "fta_bwd_dq1_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, b.dq1.SK, b.dq1.nlaunch,
              bh * b.dq1.nqg * b.dq1.nchunks, b.dq1.threads, b.dq1.smem);
   else
     snprintf(dq, sizeof dq, "fta_bwd_dq_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, (D == 32) ? 2 : 1, b.nlaunch,
              bh * b.nqg * b.nchunks, b.threads, b.smem);
-  if (b.use_dkdv1)
+  if (b.use_short) {
+  } else if (b.use_dkdv1)
     snprintf(dkdv, sizeof dkdv, "fta_bwd_dkdv1_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, b.dkdv1.NJT,
              b.dkdv1.nlaunch, bh * b.dkdv1.nkg * b.dkdv1.nchunks, b.dkdv1.threads, b.dkdv1.smem);
   else

@@ -10,8 +10,7 @@ namespace fta {
 // ------------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------------
-BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, bool tail, int feat) {
-  (void)tail;  // (every kernel of the plan has instances that mask the tail of a row: the launch picks them)
+BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
   BwdPlan pl{};
   const int nqb = L2 / 32;
   const size_t lds_max = 160 * 1024;
@@ -80,13 +79,14 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, bool tail, int feat) {
   pl.rows_per_chunk2 = (L1 + pl.nchunks2 - 1) / pl.nchunks2;
   pl.nchunks2 = (L1 + pl.rows_per_chunk2 - 1) / pl.rows_per_chunk2;
 
+  pl.use_short = forced_general_mask() == 0 && plan_short(B, H, L1, row, D, pl.sh);
   pl.use_dq1 = !feat && plan_dq1(B, H, L1, L2, D, pl.dq1);
   // (the pipelined dQ kernel makes delta itself and hands it on inside the packed constants)
-  pl.delta_bytes = pl.use_dq1 ? 0 : (size_t)B * H * L1 * L2 * sizeof(float);
+  pl.delta_bytes = (pl.use_dq1 || pl.use_short) ? 0 : (size_t)B * H * L1 * L2 * sizeof(float);
   pl.use_dkdv1 = !feat && plan_dkdv1(B, H, L1, L2, D, pl.dkdv1);
-  const int maxchunks = pl.use_dq1 ? pl.dq1.nchunks : pl.nchunks;  // of the dQ/dBias kernel that runs
+  const int maxchunks = pl.use_short ? pl.sh.nchunks : pl.use_dq1 ? pl.dq1.nchunks : pl.nchunks;  // of the dQ/dBias kernel that runs
   pl.partial_bytes = (size_t)maxchunks * B * H * L2 * L2 * sizeof(float);
-  pl.aux_bytes = (size_t)B * H * L1 * L2 * 2 * sizeof(uint32_t);
+  pl.aux_bytes = pl.use_short ? 0 : (size_t)B * H * L1 * L2 * 2 * sizeof(uint32_t);
   pl.valid = ok2 && (pl.SK * pl.QB <= 8) && (pl.ring >= 3);
   pl.feat = feat != 0;
   return pl;
@@ -114,6 +114,23 @@ hipError_t launch_bwd(BwdParams p, const BwdPlan& pl, int D, int dtype, hipStrea
   const bool nat = (p.nat != 0);  // (fp16, precise mode, D = 32, a plan with both hand-scheduled kernels)
   const bool hilo = (fast_bf16 && bf16_scale_needs_split(p.scale)) || nat;
   mark(0);
+  if (pl.use_short) {
+    // rows of up to 128 keys, any options: one kernel
+    p.partial_scale = 1.0f;
+    mark(1);
+    e = launch_short(p, pl.sh, D, dtype, st);
+    if (e != hipSuccess) return e;
+    p.nchunks = pl.sh.nchunks;
+    mark(2);
+    mark(3);
+    const int64_t total4 = (int64_t)p.B * p.H * p.L2 * ((p.L2 + 3) / 4);
+    dim3 grid((unsigned)((total4 + 255) / 256)), block(256);
+    if (dtype == kBF16) hipLaunchKernelGGL(fta_dbias_reduce_kernel<BF16>, grid, block, 0, st, p);
+    else hipLaunchKernelGGL(fta_dbias_reduce_kernel<F16>, grid, block, 0, st, p);
+    e = hipGetLastError();
+    mark(4);
+    return e;
+  }
   if (feat) {
     e = launch_bwd_feat(p, pl, D, dtype, st, ev);
     return e;

@@ -129,6 +129,12 @@ struct Dkdv1Plan {
   size_t smem;                    // the largest
 };
 
+// Geometry of the one-kernel backward for rows of up to 128 keys (a workgroup holds a whole row).
+struct ShortPlan {
+  int NT, nchunks, rows_per_chunk, threads;
+  size_t smem;
+};
+
 struct BwdPlan {
   // dQ/dBias kernel
   int SK, QB, nqg, nchunks, rows_per_chunk, threads, KR, nlaunch, ring, nb;
@@ -141,6 +147,8 @@ struct BwdPlan {
   Dq1Plan dq1;
   bool use_dkdv1;      // the dK/dV stage runs the one-wave-per-SIMD kernel
   Dkdv1Plan dkdv1;
+  bool use_short;      // rows of up to 128 keys: all gradients in one kernel
+  ShortPlan sh;
   int L2p;             // the length the tiles cover (filled in by the C-ABI layer)
   bool feat;           // planned for the feature instances (bf16, dropout, precise fp16)
   bool valid;
@@ -159,14 +167,16 @@ inline bool bf16_scale_needs_split(float sm_scale) { return !(fabsf(sm_scale) * 
 bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl);
 hipError_t launch_dq1(BwdParams p, const Dq1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st);
 
+bool plan_short(int B, int H, int L1, int L2, int D, ShortPlan& pl);
+hipError_t launch_short(BwdParams p, const ShortPlan& pl, int D, int dtype, hipStream_t st);
+
 bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl);
 hipError_t launch_dkdv1(BwdParams p, const Dkdv1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st);
 
-// L2 is the length the tiles cover (a multiple of 128); `tail`: the true row length is shorter, which
-// only the general kernels handle.
+// L2 is the length the tiles cover (a multiple of 128), `row` the true row length.
 // `feat`: 0 the fp16 kernels; 1 the plan is for bf16 inputs or the precise mode, 2 for dropout (general
 // kernels only, smaller instance sets).
-BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, bool tail, int feat);
+BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat);
 hipError_t launch_bwd(BwdParams p, const BwdPlan& pl, int D, int dtype, hipStream_t st, hipEvent_t* ev = nullptr);
 hipError_t launch_bwd_feat(const BwdParams& p, const BwdPlan& pl, int D, int dtype, hipStream_t st, hipEvent_t* ev);
 

@@ -295,6 +295,23 @@ def test_dropout_against_the_oracle_with_the_same_mask(B, H, L1, L2, D, p, dtype
     assert not torch.equal(got["o"], other["o"])
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("L1,L2,p", [(3, 2, 0.0), (5, 32, 0.0), (4, 33, 0.25), (6, 64, 0.1), (3, 65, 0.0), (7, 96, 0.25), (9, 97, 0.0), (40, 128, 0.1)])
+def test_one_kernel_backward_of_short_rows(L1, L2, p, D, dtype):
+    """Rows of up to 128 keys: all gradients in one kernel of one to four waves, with and without dropout, at the edges
+    of its 32-key blocks."""
+    import fta_lib
+    assert fta_lib.describe_plan(1, 2, L1, L2, D)["dq"]["kernel"] == f"fta_bwd_short_kernel<{D},{(L2 + 31) // 32}>"
+    B, H, sm = 1, 2, 1.0 / math.sqrt(D)
+    q, k, v, b, do = _inputs(B, H, L1, L2, D, 29, dtype)
+    extra, kw = (), {}
+    if p:
+        keep, scale = dm.keep_mask(1234, p, B, H, L1, L2)
+        extra, kw = (p, 1234), dict(keep=torch.from_numpy(keep).to(DEV), keep_scale=scale)
+    _compare(_run(q, k, v, b, sm, do, *extra), _oracle(q, k, v, b, sm, do, **kw), dtype, f"short {L1}x{L2}")
+
+
 def test_dropout_zero_is_the_plain_path_and_lse_ignores_the_mask():
     import fta_lib, flash_tt_attn as fta
     lib = fta_lib.load()
