@@ -118,7 +118,7 @@ hipError_t launch_bwd(BwdParams p, const BwdPlan& pl, int D, int dtype, hipStrea
     // rows of up to 128 keys, any options: one kernel
     p.partial_scale = 1.0f;
     mark(1);
-    e = launch_short(p, pl.sh, D, dtype, st);
+    e = launch_short(p, pl.sh, D, dtype, pl.feat, st);  // (fp16 without dropout is planned at that level in precise mode only)
     if (e != hipSuccess) return e;
     p.nchunks = pl.sh.nchunks;
     mark(2);

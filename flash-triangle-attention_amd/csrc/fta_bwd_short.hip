@@ -13,8 +13,9 @@
 // works on keys (w + r) % NT, writes P and dS as 16-bit row-major tiles into its slot of the exchange buffer, and after
 // the round's barrier reads those of wave (w - r) % NT with transposing LDS reads.  Two buffers, so one barrier per round.
 //
-// Everything per score is in fp32 on the vector ALU (scale, bias, row constants unrounded), so the precise mode is this
-// kernel as it is; dropout replays the forward's mask.
+// Everything per score is in fp32 on the vector ALU (scale, bias, row constants unrounded).  The precise mode of fp16
+// is an instance that rounds P and dS to nearest on their way into the matrix core instead of toward zero; dropout
+// replays the forward's mask.
 //
 // Bound: memory (eight tensors of 64 bytes per pair and head against some 130 vector instructions per 32 x 32 tile,
 // about half of the memory time at 128 keys).  Two workgroups of four waves share a CU, one's loads under the other's
@@ -25,7 +26,7 @@
 namespace fta {
 
 // NT: blocks of 32 queries (and keys) that a row takes, one wave each.
-template <class T, int D, int NT, bool DROP>
+template <class T, int D, int NT, bool DROP, bool NEAREST>
 __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(D == 32 ? 2 : 1))) fta_bwd_short_kernel(const BwdParams p) {
   constexpr int KS = D / 16, DT = D / 32;
   constexpr int ROWS = 32 * NT;
@@ -166,8 +167,8 @@ __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(D 
         const float d0 = p0 * (e0 - delta), d1 = p1 * (e1 - delta);
         dbacc[r][e] += d0;
         dbacc[r][e + 1] += d1;
-        pp[e >> 1] = T::pack(w0, w1);
-        ds[e >> 1] = T::pack(d0, d1);
+        pp[e >> 1] = NEAREST ? T::pack(w0, w1) : T::pack_fast(w0, w1);
+        ds[e >> 1] = NEAREST ? T::pack(d0, d1) : T::pack_fast(d0, d1);
       }
       // dQ^T += K^T dS^T
 #pragma unroll
@@ -253,18 +254,19 @@ bool plan_short(int B, int H, int L1, int L2, int D, ShortPlan& pl) {
   return true;
 }
 
-hipError_t launch_short(BwdParams p, const ShortPlan& pl, int D, int dtype, hipStream_t st) {
+hipError_t launch_short(BwdParams p, const ShortPlan& pl, int D, int dtype, bool precise, hipStream_t st) {
   p.nchunks = pl.nchunks;
   p.rows_per_chunk = pl.rows_per_chunk;
   const dim3 grid((unsigned)(p.B * p.H * pl.nchunks)), block((unsigned)pl.threads);
   const bool drop = p.drop.thresh != 0;
-#define FTA_SHORT_CASE(DD, NN)                                                                                       \
-  if (D == DD && pl.NT == NN) {                                                                                      \
-    if (dtype == kBF16)                                                                                              \
-      return drop ? launch_kernel(fta_bwd_short_kernel<BF16, DD, NN, true>, p, grid, block, pl.smem, st)             \
-                  : launch_kernel(fta_bwd_short_kernel<BF16, DD, NN, false>, p, grid, block, pl.smem, st);           \
-    return drop ? launch_kernel(fta_bwd_short_kernel<F16, DD, NN, true>, p, grid, block, pl.smem, st)                \
-                : launch_kernel(fta_bwd_short_kernel<F16, DD, NN, false>, p, grid, block, pl.smem, st);              \
+#define FTA_SHORT_CASE(DD, NN)                                                                                             \
+  if (D == DD && pl.NT == NN) {                                                                                            \
+    if (dtype == kBF16)                                                                                                    \
+      return drop ? launch_kernel(fta_bwd_short_kernel<BF16, DD, NN, true, true>, p, grid, block, pl.smem, st)             \
+                  : launch_kernel(fta_bwd_short_kernel<BF16, DD, NN, false, true>, p, grid, block, pl.smem, st);           \
+    if (drop) return launch_kernel(fta_bwd_short_kernel<F16, DD, NN, true, true>, p, grid, block, pl.smem, st);            \
+    return precise ? launch_kernel(fta_bwd_short_kernel<F16, DD, NN, false, true>, p, grid, block, pl.smem, st)            \
+                   : launch_kernel(fta_bwd_short_kernel<F16, DD, NN, false, false>, p, grid, block, pl.smem, st);          \
   }
   FTA_SHORT_CASE(32, 1) FTA_SHORT_CASE(32, 2) FTA_SHORT_CASE(32, 3) FTA_SHORT_CASE(32, 4)
   FTA_SHORT_CASE(64, 1) FTA_SHORT_CASE(64, 2) FTA_SHORT_CASE(64, 3) FTA_SHORT_CASE(64, 4)

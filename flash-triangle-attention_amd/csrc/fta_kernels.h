@@ -168,7 +168,7 @@ bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl);
 hipError_t launch_dq1(BwdParams p, const Dq1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st);
 
 bool plan_short(int B, int H, int L1, int L2, int D, ShortPlan& pl);
-hipError_t launch_short(BwdParams p, const ShortPlan& pl, int D, int dtype, hipStream_t st);
+hipError_t launch_short(BwdParams p, const ShortPlan& pl, int D, int dtype, bool precise, hipStream_t st);
 
 bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl);
 hipError_t launch_dkdv1(BwdParams p, const Dkdv1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st);
