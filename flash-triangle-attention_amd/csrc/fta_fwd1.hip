@@ -88,38 +88,6 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
   const half_t* vbase = p.v + b * p.vs[0] + h * p.vs[1];
   half_t* obase = p.o + b * p.os[0] + h * p.os[1];
 
-  // ---- stationary bias: tile tt, register pair rg holds keys 32*tt + 8*rg + 4*hh + 0..3 of query l32
-  uint32_t bias_reg[NKT][8];
-  {
-    const half_t* bbh = p.bias + b * p.bs[0] + h * p.bs[1];
-    if constexpr (!TAIL) {
-      // whole rows of 8-byte aligned quads: plain loads, all of them in flight before the first is used
-      // (one at a time they cost a workgroup 64 trips to memory before its first row)
-      const half_t* bp = bbh + (int64_t)(q0 + l32) * p.bs[2] + 4 * hh;
-      u32x2 raw[NKT][4];
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) raw[tt][rg] = *reinterpret_cast<const u32x2*>(bp + tt * 32 + rg * 8);
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          bias_reg[tt][2 * rg] = fwd1_bias_pair<T>(raw[tt][rg][0]);
-          bias_reg[tt][2 * rg + 1] = fwd1_bias_pair<T>(raw[tt][rg][1]);
-        }
-    } else {
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          const u32x2 v = load_bias4(bbh, p.bs[2], q0 + l32, 4 * hh + tt * 32 + rg * 8, p.L2, T::kNegInf2);
-          bias_reg[tt][2 * rg] = fwd1_bias_pair<T>(v[0]);
-          bias_reg[tt][2 * rg + 1] = fwd1_bias_pair<T>(v[1]);
-        }
-    }
-  }
-
   // ---- stage copies: a stage is 32*G K rows and 32*G V rows of 64 bytes, 1 KB per wave instruction,
   // NCU K and NCU V copies per wave; copy u of wave w carries the 16-byte pieces (w + W*u)*64 .. +63.
   uint32_t goffk[NCU], goffv[NCU];
@@ -212,18 +180,26 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
   const float lg2e = kLog2e;
   const uint32_t ones = T::is_bf16 ? 0x3F803F80u : 0x3C003C00u;
 
-  // ---- prologue: stages 0 and 1 whole, the first share of stage 2 (the one the iteration "before the
-  // first" would have issued), Q of row 0; then the scores of tile 0
+  // ---- prologue: stages 0 and 1 whole; the stationary bias (tile tt, register pair rg holds keys 32*tt + 8*rg +
+  // 4*hh + 0..3 of query l32), which changes lanes in the ring slots that nothing is copied to yet; Q of row 0; behind
+  // the barrier the first share of stage 2 (the one the iteration "before the first" would have issued)
   static_for<0, 2>([&](auto nc) {
     constexpr int n = decltype(nc)::value;
     fill_begin(std::integral_constant<int, n % NST>{}, n > 0);
     static_for<0, 2 * ncu_of(n % NST)>([&](auto cc) { fill_copy(std::integral_constant<int, n % NST>{}, cc); });
   });
-  fill_begin(std::integral_constant<int, 2 % NST>{}, true);
-  fill_share(std::integral_constant<int, 0>{});
+  uint32_t bias_reg[NKT][8];
+  static_assert(W * 4096 <= 2 * SLOT_B, "4 KB for every wave's bias");
+  load_bias_tiles<NKT, TAIL>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], q0, 0, p.L2, T::kNegInf2, smem_raw + 2 * SLOT_B + wave * 4096, lane,
+                             [&](int tt, int rg, u32x2 v) {
+                               bias_reg[tt][2 * rg] = fwd1_bias_pair<T>(v[0]);
+                               bias_reg[tt][2 * rg + 1] = fwd1_bias_pair<T>(v[1]);
+                             });
   q_issue(false);
   wait_vmem_all();
-  __builtin_amdgcn_s_barrier();
+  __syncthreads();
+  fill_begin(std::integral_constant<int, 2 % NST>{}, true);
+  fill_share(std::integral_constant<int, 0>{});
 
   u32x4 qf[KS];
 #pragma unroll
