@@ -186,39 +186,10 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
   // the scores through the matrix core, with the same one-hot selectors that accumulate dBias
   u32x4 bias4[NKT][2];  // [tile][16-key contraction step]: B operands of S^T += E_u * bias^T_u
   floatx16 dbacc[NKT];
-  {
-    const half_t* bias_bh = p.bias + b * p.bs[0] + h * p.bs[1];
-    const half_t* bp = bias_bh + (int64_t)(q0 + l32) * p.bs[2] + key0 + 4 * hh;
-    // (whole, aligned rows: every load is issued before the first value is parked, which is an opaque
-    // statement that would otherwise put a trip to memory between one pair of loads and the next)
-    [[maybe_unused]] u32x2 raw[TAIL ? 1 : NKT][4];
-    if constexpr (!TAIL) {
 #pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
+  for (int tt = 0; tt < NKT; ++tt)
 #pragma unroll
-        for (int x = 0; x < 4; ++x) raw[tt][x] = *reinterpret_cast<const u32x2*>(bp + tt * 32 + x * 8);
-    }
-#pragma unroll
-    for (int tt = 0; tt < NKT; ++tt) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        u32x2 v0, v1;
-        if constexpr (TAIL) {
-          const int kk = key0 + 4 * hh + tt * 32 + 16 * u;
-          v0 = load_bias4(bias_bh, p.bs[2], q0 + l32, kk, p.L2, T::kNegInf2);
-          v1 = load_bias4(bias_bh, p.bs[2], q0 + l32, kk + 8, p.L2, T::kNegInf2);
-        } else {
-          v0 = raw[tt][2 * u];
-          v1 = raw[tt][2 * u + 1];
-        }
-        if constexpr (NAT) bias4[tt][u] = u32x4{T::bias_nat(v0[0]), T::bias_nat(v0[1]), T::bias_nat(v1[0]), T::bias_nat(v1[1])};
-        else bias4[tt][u] = u32x4{T::bias_log2(v0[0]), T::bias_log2(v0[1]), T::bias_log2(v1[0]), T::bias_log2(v1[1])};
-        asm volatile("" : "+a"(bias4[tt][u]));  // parked in accumulation registers for the whole kernel
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dbacc[tt][r] = 0.f;
-    }
-  }
+    for (int r = 0; r < 16; ++r) dbacc[tt][r] = 0.f;
   // one-hot selectors: E[u] (A operand, 32 rows x 16 slots) has a 1 where accumulator row l32 is
   // the key that contraction slot (hh, e) of step u carries: key = 16u + 8*(e/4) + 4*hh + e%4
   half8_t E[2];
@@ -448,6 +419,20 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
     constexpr int n = decltype(nc)::value;
     stage_issue(std::integral_constant<int, n % 2>{}, n == 0);
   });
+  {
+    // the bias, while those copies fly; it changes lanes in the ring slot that nothing is copied to yet
+    static_assert(4 * 4096 <= SLOT_H * 2, "4 KB for every wave's bias");
+    u32x2 even = {0u, 0u};
+    load_bias_tiles<NKT / 2, 2, TAIL, false>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], q0, p.L2, T::kNegInf2,
+                                             smem_raw + (R - 1) * SLOT_H * 2 + wave * 4096, lane, [=](int c) { return key0 + 64 * c; },
+                                             [&](int tt, int g, u32x2 v) {
+                                               if (g % 2 == 0) { even = v; return; }
+                                               u32x4& d = bias4[tt][g / 2];
+                                               if constexpr (NAT) d = u32x4{T::bias_nat(even[0]), T::bias_nat(even[1]), T::bias_nat(v[0]), T::bias_nat(v[1])};
+                                               else d = u32x4{T::bias_log2(even[0]), T::bias_log2(even[1]), T::bias_log2(v[0]), T::bias_log2(v[1])};
+                                               asm volatile("" : "+a"(d));  // parked in accumulation registers for the whole kernel
+                                             });
+  }
   rowconst_issue(0);
   {
     wait_vmem_all();

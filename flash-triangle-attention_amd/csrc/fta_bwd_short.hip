@@ -60,21 +60,16 @@ __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(D 
   // stationary bias, in the order of the rounds: tile r holds keys of block (wave + r) % NT
   uint32_t bias_reg[NT][8];
   float dbacc[NT][16];
-  {
-    const half_t* bbh = p.bias + b * p.bs[0] + h * p.bs[1];
+  load_bias_tiles<NT, 1, true, true>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], wave * 32, p.L2, T::kNegInf2,
+                                     reinterpret_cast<char*>(xchg + wave * 2 * XT), lane, [=](int c) { return (wave + c) % NT * 32; },
+                                     [&](int r, int g, u32x2 v) {
+                                       bias_reg[r][2 * g] = v[0];
+                                       bias_reg[r][2 * g + 1] = v[1];
+                                     });
 #pragma unroll
-    for (int r = 0; r < NT; ++r) {
-      const int kb = (wave + r) % NT;
+  for (int r = 0; r < NT; ++r)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const u32x2 v = load_bias4(bbh, p.bs[2], j, kb * 32 + 8 * g + 4 * hh, p.L2, T::kNegInf2);
-        bias_reg[r][2 * g] = v[0];
-        bias_reg[r][2 * g + 1] = v[1];
-      }
-#pragma unroll
-      for (int e = 0; e < 16; ++e) dbacc[r][e] = 0.f;
-    }
-  }
+    for (int e = 0; e < 16; ++e) dbacc[r][e] = 0.f;
 
   // copies of one row: TILE / 512 pieces of 1 KB per tensor, dealt to the waves; rows beyond the last are copies of it
   constexpr int NC = TILE / 512 / NT;    // per wave and tensor

@@ -537,70 +537,71 @@ __device__ __forceinline__ u32x2 load_bias4(const half_t* bias_bh, int64_t jstri
   return u32x2{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
 }
 
-// The stationary bias of a wave: 32 queries from q0 against 32*NT keys from key0, handed to `sink(tile, group, pair)` in
-// the S^T accumulator layout (keys 32*tile + 8*group + 4*hh + 0..3 of query l%32, as two packed pairs).  Loaded that
-// way, 8 bytes per lane, an instruction touches 32 rows and every 128-byte line is asked for by eight of them, more
-// lines than the L1 holds between two: at 512 keys the set-up of a workgroup took 16 us.  Instead eight lanes load a
-// row's 64 keys as one line, all of them in flight at once, and the pieces change lanes through 4 KB of LDS that belong
-// to the wave (no barrier: a wave's LDS operations are executed in order).
-// TAIL: rows of L2 keys that end inside the tile (keys beyond it read as -inf, queries beyond it as the last query's
-// row), on any 2-byte boundary.
-template <int NT, bool TAIL, class Sink>
-__device__ __forceinline__ void load_bias_tiles(const half_t* bias_bh, int64_t jstride, int q0, int key0, int L2, uint32_t neg_inf2,
-                                                char* lds, int lane, Sink&& sink) {
-  static_assert(NT % 2 == 0, "chunks of 64 keys");
-  constexpr int NC = NT / 2;
-  const int row8 = lane >> 3, piece = lane & 7, l32 = lane & 31, hh = lane >> 5;
-  u32x4 raw[NC][4];
+// Eight consecutive bias entries from key k of a row, as whole-row loads want them: entries k .. k+7 of a row that holds
+// them, any other piece (TAIL) as the row's last eight entries, which bias_piece_fix() shifts into place; keys at or
+// beyond L2 come out as -inf.  Any 2-byte boundary.  (Rows of fewer than eight keys are read entry by entry.)
+template <bool TAIL>
+__device__ __forceinline__ u32x4 bias_piece_load(const half_t* row, int k, int L2, uint32_t neg_inf2, bool short_rows) {
+  u32x4 v;
+  if constexpr (!TAIL) {
+    v = *reinterpret_cast<const u32x4*>(row + k);
+  } else if (!short_rows || L2 >= 8) {
+    __builtin_memcpy(&v, row + (k + 8 <= L2 ? k : L2 - 8), 16);
+  } else {
+    uint32_t e[8];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int j = q0 + 8 * i + row8;
+    for (int n = 0; n < 8; ++n) e[n] = k + n < L2 ? (uint32_t)reinterpret_cast<const uint16_t*>(row)[k + n] : (neg_inf2 & 0xFFFFu);
+    v = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+  }
+  return v;
+}
+__device__ __forceinline__ u32x4 bias_piece_fix(u32x4 v, int k, int L2, uint32_t neg_inf2) {
+  const int sh = k + 8 <= L2 ? 0 : (k - (L2 - 8) < 8 ? k - (L2 - 8) : 8);  // entries to drop at the front
+  if (sh & 4) v = u32x4{v[2], v[3], neg_inf2, neg_inf2};
+  if (sh & 2) v = u32x4{v[1], v[2], v[3], neg_inf2};
+  if (sh & 1)
+    v = u32x4{__builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16), __builtin_amdgcn_alignbit(v[3], v[2], 16),
+              __builtin_amdgcn_alignbit(neg_inf2, v[3], 16)};
+  if (sh & 8) v = u32x4{neg_inf2, neg_inf2, neg_inf2, neg_inf2};
+  return v;
+}
+
+// The stationary bias of a wave: 32 queries from q0 against NC chunks of 32*CT keys (chunk c from key first_key(c)),
+// handed to `sink(tile, group, pair)` in the S^T accumulator layout (keys 8*group + 4*hh + 0..3 of the tile's 32, of query
+// l%32, as two packed pairs; tile c*CT + t).  Loaded that way, 8 bytes per lane, an instruction touches 32 rows and every
+// 128-byte line is asked for by eight of them, more lines than the L1 holds between two: at 512 keys the set-up of a
+// workgroup took 16 us.  Instead four or eight lanes load a row's keys as one piece of a line, all of them in flight at
+// once, and the pieces change lanes through 2 or 4 KB (CT) of LDS that belong to the wave (no barrier: a wave's LDS operations are
+// executed in order).
+// TAIL: rows of L2 keys that may end inside the tile (keys beyond it read as -inf, queries beyond it as the last query's
+// row), on any 2-byte boundary; SHORT: of fewer than eight keys, too.
+template <int NC, int CT, bool TAIL, bool SHORT, class Key, class Sink>
+__device__ __forceinline__ void load_bias_tiles(const half_t* bias_bh, int64_t jstride, int q0, int L2, uint32_t neg_inf2, char* lds, int lane,
+                                                Key&& first_key, Sink&& sink) {
+  static_assert(CT == 1 || CT == 2, "chunks of 32 or 64 keys");
+  constexpr int PR = 4 * CT, RI = 64 / PR, NI = 32 / RI;  // pieces per row, rows per instruction, instructions per chunk
+  const int rowi = lane / PR, piece = lane % PR, l32 = lane & 31, hh = lane >> 5;
+  auto slot = [](int row, int pc) { return row * (16 * PR) + ((pc ^ (CT == 2 ? row & 7 : (row >> 1) & 3)) << 4); };
+  u32x4 raw[NC][NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int j = q0 + RI * i + rowi;
     const half_t* row = bias_bh + (int64_t)(TAIL ? (j < L2 ? j : L2 - 1) : j) * jstride;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      const int k = key0 + 64 * c + 8 * piece;
-      if constexpr (!TAIL) {
-        raw[c][i] = *reinterpret_cast<const u32x4*>(row + k);
-      } else {
-        // a whole piece that lies in the row, shifted into place below (the tiles of longer rows are only taken for rows
-        // that reach into the last pair of tiles)
-        if (NT > 2 || L2 >= 8) {
-          __builtin_memcpy(&raw[c][i], row + (k + 8 <= L2 ? k : L2 - 8), 16);
-        } else {
-          uint32_t e[8];
-#pragma unroll
-          for (int n = 0; n < 8; ++n) e[n] = k + n < L2 ? (uint32_t)reinterpret_cast<const uint16_t*>(row)[k + n] : (neg_inf2 & 0xFFFFu);
-          raw[c][i] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
-        }
-      }
-    }
+    for (int c = 0; c < NC; ++c) raw[c][i] = bias_piece_load<TAIL>(row, first_key(c) + 8 * piece, L2, neg_inf2, SHORT);
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     if constexpr (TAIL)
-      if (key0 + 64 * c + 64 > L2 && L2 >= 8) {
-        // the row ends in this chunk: entries L2-8 .. L2-1 were loaded for every piece that reaches beyond it
-        const int k = key0 + 64 * c + 8 * piece;
-        const int sh = k + 8 <= L2 ? 0 : (k - (L2 - 8) < 8 ? k - (L2 - 8) : 8);  // entries to drop at the front
+      if (first_key(c) + 32 * CT > L2 && (!SHORT || L2 >= 8))  // the row ends in this chunk, or before it
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          u32x4 v = raw[c][i];
-          if (sh & 4) v = u32x4{v[2], v[3], neg_inf2, neg_inf2};
-          if (sh & 2) v = u32x4{v[1], v[2], v[3], neg_inf2};
-          if (sh & 1)
-            v = u32x4{__builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16), __builtin_amdgcn_alignbit(v[3], v[2], 16),
-                      __builtin_amdgcn_alignbit(neg_inf2, v[3], 16)};
-          if (sh & 8) v = u32x4{neg_inf2, neg_inf2, neg_inf2, neg_inf2};
-          raw[c][i] = v;
-        }
-      }
+        for (int i = 0; i < NI; ++i) raw[c][i] = bias_piece_fix(raw[c][i], first_key(c) + 8 * piece, L2, neg_inf2);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(lds + (8 * i + row8) * 128 + ((piece ^ row8) << 4)) = raw[c][i];
+    for (int i = 0; i < NI; ++i) *reinterpret_cast<u32x4*>(lds + slot(RI * i + rowi, piece)) = raw[c][i];
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < CT; ++t)
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        sink(2 * c + t, g, *reinterpret_cast<const u32x2*>(lds + l32 * 128 + (((4 * t + g) ^ (l32 & 7)) << 4) + 8 * hh));
+      for (int g = 0; g < 4; ++g) sink(c * CT + t, g, *reinterpret_cast<const u32x2*>(lds + slot(l32, 4 * t + g) + 8 * hh));
   }
 }
 

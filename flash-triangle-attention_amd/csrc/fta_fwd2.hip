@@ -67,37 +67,6 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_wav
   const half_t* vbase = p.v + b * p.vs[0] + h * p.vs[1];
   half_t* obase = p.o + b * p.os[0] + h * p.os[1];
 
-  // ---- stationary bias: tile tt, register pair rg holds keys key0 + 32*tt + 8*rg + 4*hh + 0..3 of query l32
-  uint32_t bias_reg[NKT][8];
-  {
-    const half_t* bbh = p.bias + b * p.bs[0] + h * p.bs[1];
-    if constexpr (!TAIL) {
-      // whole rows of 8-byte aligned quads: plain loads, all of them in flight before the first is used
-      const half_t* bp = bbh + (int64_t)(q0 + l32) * p.bs[2] + key0 + 4 * hh;
-      u32x2 raw[NKT][4];
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) raw[tt][rg] = *reinterpret_cast<const u32x2*>(bp + tt * 32 + rg * 8);
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          bias_reg[tt][2 * rg] = fwd1_bias_pair<T>(raw[tt][rg][0]);
-          bias_reg[tt][2 * rg + 1] = fwd1_bias_pair<T>(raw[tt][rg][1]);
-        }
-    } else {
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          const u32x2 v = load_bias4(bbh, p.bs[2], q0 + l32, key0 + 4 * hh + tt * 32 + rg * 8, p.L2, T::kNegInf2);
-          bias_reg[tt][2 * rg] = fwd1_bias_pair<T>(v[0]);
-          bias_reg[tt][2 * rg + 1] = fwd1_bias_pair<T>(v[1]);
-        }
-    }
-  }
-
   // ---- stage copies: per slab 64 K rows and 64 V rows of 128 bytes; one wave instruction moves 1 KB =
   // 8 rows, and wave w moves rows 8w .. 8w+7 of each of the stage's 2*S tiles (copy u: slab u/2, K or V).
   const int crow = 8 * wave + (lane >> 3);  // row of this lane inside a 64-row tile
@@ -196,18 +165,27 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_wav
   const float lg2e = kLog2e;
   const uint32_t ones = T::is_bf16 ? 0x3F803F80u : 0x3C003C00u;
 
-  // ---- prologue: stages 0 and 1 whole, the first iteration's share of stage 2, Q of row 0; then the
-  // scores of tile 0
+  // ---- prologue: stages 0 and 1 whole; the stationary bias (tile tt, register pair rg holds keys key0 + 32*tt + 8*rg +
+  // 4*hh + 0..3 of query l32), which changes lanes in ring slots that nothing is copied to yet; Q of row 0; behind the
+  // barrier the first iteration's share of stage 2; then the scores of tile 0
   static_for<0, 2>([&](auto nc) {
     constexpr int n = decltype(nc)::value;
     fill_begin(std::integral_constant<int, n % NST>{}, n > 0);
     static_for<0, NCPY>([&](auto uc) { fill_copy(std::integral_constant<int, n % NST>{}, uc); });
   });
-  fill_begin(std::integral_constant<int, 2 % NST>{}, true);
-  static_for<0, S>([&](auto uc) { fill_copy(std::integral_constant<int, 2 % NST>{}, uc); });
+  uint32_t bias_reg[NKT][8];
+  static_assert(8 * 4096 <= 2 * SLOT_B, "4 KB for every wave's bias");
+  load_bias_tiles<NKT / 2, 2, TAIL, false>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], q0, p.L2, T::kNegInf2, smem_raw + 2 * SLOT_B + wave * 4096,
+                                           lane, [=](int c) { return key0 + 64 * c; },
+                                           [&](int tt, int rg, u32x2 v) {
+                                             bias_reg[tt][2 * rg] = fwd1_bias_pair<T>(v[0]);
+                                             bias_reg[tt][2 * rg + 1] = fwd1_bias_pair<T>(v[1]);
+                                           });
   q_issue(false);
   wait_vmem_all();
-  __builtin_amdgcn_s_barrier();
+  __syncthreads();
+  fill_begin(std::integral_constant<int, 2 % NST>{}, true);
+  static_for<0, S>([&](auto uc) { fill_copy(std::integral_constant<int, 2 % NST>{}, uc); });
 
   u32x4 qf[KS];
 #pragma unroll

@@ -88,33 +88,17 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
   const int last = p.L2 - 1;
   uint32_t bias_reg[NKT][8];
   {
+    // (it changes lanes in the second stage buffer, which nothing is copied to before the first row's barrier; a row's
+    // end that is no tile's end, or rows off the 8-byte boundary, take the instance that looks)
     const half_t* bbh = p.bias + b * p.bs[0] + h * p.bs[1];
-    if (!tail && !p.odd_bias) {
-      // whole rows of 8-byte aligned quads: plain loads, all of them in flight before the first is used
-      // (one at a time they cost a workgroup as many trips to memory before its first row)
-      const half_t* bp = bbh + (int64_t)(q0 + l32) * p.bs[2] + slab * KW + 4 * hh;
-      u32x2 raw[NKT][4];
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) raw[tt][rg] = *reinterpret_cast<const u32x2*>(bp + tt * 32 + rg * 8);
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          bias_reg[tt][2 * rg] = T::finite2(raw[tt][rg][0]);
-          bias_reg[tt][2 * rg + 1] = T::finite2(raw[tt][rg][1]);
-        }
-    } else {
-#pragma unroll
-      for (int tt = 0; tt < NKT; ++tt)
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-          u32x2 v = load_bias4(bbh, p.bs[2], q0 + l32, slab * KW + 4 * hh + tt * 32 + rg * 8, p.L2, T::kNegInf2);
-          bias_reg[tt][2 * rg] = T::finite2(v[0]);
-          bias_reg[tt][2 * rg + 1] = T::finite2(v[1]);
-        }
-    }
+    char* turn = reinterpret_cast<char*>(smem + buf_halfs) + wave * 2048;
+    auto key = [=](int c) { return slab * KW + 32 * c; };
+    auto keep = [&](int tt, int rg, u32x2 v) {
+      bias_reg[tt][2 * rg] = T::finite2(v[0]);
+      bias_reg[tt][2 * rg + 1] = T::finite2(v[1]);
+    };
+    if (!tail && !p.odd_bias) load_bias_tiles<NKT, 1, false, false>(bbh, p.bs[2], q0, p.L2, T::kNegInf2, turn, lane, key, keep);
+    else load_bias_tiles<NKT, 1, true, NKT == 4>(bbh, p.bs[2], q0, p.L2, T::kNegInf2, turn, lane, key, keep);
   }
 
   // ---- global -> LDS staging of one (row, step): S slabs x KT keys of K and V, copied
@@ -144,7 +128,8 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
   auto stage = [&](int buf_ct) {
     const int cur_buf = (STEPS & 1) ? buf_ct : buf_rt;
     buf_rt ^= 1;
-    if (PLAN && !tail) {
+    // (stages that end inside the row in every slab take the offsets computed once)
+    if (PLAN && (!tail || (S - 1) * KW + (cur_t + 1) * KT <= p.L2)) {
       dma_issue(plk, kcur + cur_t * kstep, ldsK[cur_buf]);
       dma_issue(plv, vcur + cur_t * vstep, ldsV[cur_buf]);
     } else {
