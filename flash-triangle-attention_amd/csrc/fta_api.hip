@@ -437,6 +437,7 @@ int fta_fwd_ex(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor5* v,
   const fta::FwdPlan pl = cached_plan_fwd(B, H, L1, L2, D, opt.feat_fwd);
   p.B = B; p.H = H; p.L1 = L1; p.L2 = L2; p.L2p = pl.L2p;
   p.odd_bias = bias_rows_unaligned(bias) ? 1 : 0;
+  p.head_inner = (H > 1 && k->stride[1] < k->stride[3]) ? 1 : 0;
   p.scale = sm_scale;
   p.drop = opt.drop;
   return static_cast<int>(fta::launch_fwd(p, pl, D, opt.dtype, static_cast<hipStream_t>(stream)));
@@ -538,6 +539,7 @@ static int bwd_impl(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor
   p.scale = sm_scale;
   p.drop = opt.drop;
   p.dbias_f32 = opt.dbias_f32;
+  p.head_inner = (H > 1 && k->stride[1] < k->stride[3]) ? 1 : 0;
   p.nat = (opt.f16_precise && level == 0) ? 1 : 0;
   p.odd_bias = bias_rows_unaligned(bias) ? 1 : 0;  // (the reduction looks at the address of every dBias group itself)
   return static_cast<int>(fta::launch_bwd(p, pl, D, opt.dtype, static_cast<hipStream_t>(stream), ev));

@@ -155,11 +155,8 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hh = lane >> 5, l32 = lane & 31;
 
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int kg = lid % p.nkg;
-  const int chunk = (lid / p.nkg) % p.nchunks2;
-  const int bh = lid / (p.nkg * p.nchunks2);
-  const int b = bh / p.H, h = bh % p.H;
+  const WorkId id = work_id(p.nkg, p.nchunks2, p.H, p.head_inner);
+  const int kg = id.group, chunk = id.chunk, b = id.b, h = id.h, bh = b * p.H + h;
   const int i0 = chunk * p.rows_per_chunk2;
   const int nrows = min(p.rows_per_chunk2, p.L1 - i0);
   if (nrows <= 0) return;

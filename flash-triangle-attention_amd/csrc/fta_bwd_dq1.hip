@@ -158,11 +158,8 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
   const int slab = wave % SK, qb = wave / SK;
   const int hh = lane >> 5, l32 = lane & 31;
 
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int qg = lid % p.nqg;
-  const int chunk = (lid / p.nqg) % p.nchunks;
-  const int bh = lid / (p.nqg * p.nchunks);
-  const int b = bh / p.H, h = bh % p.H;
+  const WorkId id = work_id(p.nqg, p.nchunks, p.H, p.head_inner);
+  const int qg = id.group, chunk = id.chunk, b = id.b, h = id.h, bh = b * p.H + h;
   const int i0 = chunk * p.rows_per_chunk;
   const int nrows = min(p.rows_per_chunk, p.L1 - i0);
   if (nrows <= 0) return;

@@ -96,11 +96,8 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   const int slab = wave % SK, qb = wave / SK;
   const int hh = lane >> 5, l32 = lane & 31;
 
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int qg = lid % p.nqg;
-  const int chunk = (lid / p.nqg) % p.nchunks;
-  const int bh = lid / (p.nqg * p.nchunks);
-  const int b = bh / p.H, h = bh % p.H;
+  const WorkId id = work_id(p.nqg, p.nchunks, p.H, p.head_inner);
+  const int qg = id.group, chunk = id.chunk, b = id.b, h = id.h, bh = b * p.H + h;
   const int i0 = chunk * p.rows_per_chunk;
   const int nrows = min(p.rows_per_chunk, p.L1 - i0);
   if (nrows <= 0) return;
@@ -435,11 +432,8 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   const int jslab = wave % SJ, kb = wave / SJ;
   const int hh = lane >> 5, l32 = lane & 31;
 
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int kg = lid % p.nkg;
-  const int chunk = (lid / p.nkg) % p.nchunks2;
-  const int bh = lid / (p.nkg * p.nchunks2);
-  const int b = bh / p.H, h = bh % p.H;
+  const WorkId id = work_id(p.nkg, p.nchunks2, p.H, p.head_inner);
+  const int kg = id.group, chunk = id.chunk, b = id.b, h = id.h, bh = b * p.H + h;
   const int i0 = chunk * p.rows_per_chunk2;
   const int nrows = min(p.rows_per_chunk2, p.L1 - i0);
   if (nrows <= 0) return;

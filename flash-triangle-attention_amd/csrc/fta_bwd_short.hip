@@ -40,9 +40,8 @@ __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(D 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hh = lane >> 5, l32 = lane & 31;
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int chunk = lid % p.nchunks, bh = lid / p.nchunks;
-  const int b = bh / p.H, h = bh % p.H;
+  const WorkId id = work_id(1, p.nchunks, p.H, p.head_inner);
+  const int chunk = id.chunk, b = id.b, h = id.h, bh = b * p.H + h;
   const int i0 = chunk * p.rows_per_chunk;
   const int nrows = min(p.rows_per_chunk, p.L1 - i0);
   if (nrows <= 0) return;  // whole workgroup leaves together

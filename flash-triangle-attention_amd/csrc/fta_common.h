@@ -658,10 +658,35 @@ __device__ __forceinline__ half8_t lds_frag_t(const half_t* tile, int rowbase, c
 
 // XCD-aware decode: hardware deals consecutive workgroup ids round-robin over the 8 dies, so
 // id n lands on die n%8.  Re-number so that logically consecutive workgroups (which share K/V
-// rows and the bias in that die's L2) sit on the same die.
+// rows and the bias in that die's L2) sit on the same die, also where the count is no multiple of 8 (the first dies
+// then have one more).
 __device__ __forceinline__ int xcd_remap(int n, int total) {
-  if (total % kXcds != 0) return n;
-  return (n % kXcds) * (total / kXcds) + n / kXcds;
+  const int die = n % kXcds, each = total / kXcds, more = total % kXcds;
+  return die * each + min(die, more) + n / kXcds;
+}
+
+// What a workgroup works on: `group` of queries (or keys) of one (b,h), a chunk of L1 rows.  Logically consecutive
+// workgroups take the groups of a chunk (they read the same rows), then the chunks of a (b,h) (the same bias); where
+// the heads of a row are interleaved in memory (`head_inner`: a projection's (.., H*D) layout) the heads come
+// before the chunks, since a 128-byte line then holds two heads' rows and would else be fetched by two dies.
+struct WorkId { int group, chunk, b, h; };
+__device__ __forceinline__ WorkId work_id(int ngroups, int nchunks, int H, int head_inner) {
+  int lid = xcd_remap(blockIdx.x, gridDim.x);
+  WorkId w;
+  w.group = lid % ngroups;
+  lid /= ngroups;
+  if (head_inner) {
+    w.h = lid % H;
+    lid /= H;
+    w.chunk = lid % nchunks;
+    w.b = lid / nchunks;
+  } else {
+    w.chunk = lid % nchunks;
+    lid /= nchunks;
+    w.h = lid % H;
+    w.b = lid / H;
+  }
+  return w;
 }
 
 }  // namespace fta

@@ -48,11 +48,8 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_wav
   const int slab = wave % S, qb = wave / S;
   const int hh = lane >> 5, l32 = lane & 31;
 
-  const int lid = xcd_remap(blockIdx.x, gridDim.x);
-  const int qg = lid % p.nqg;
-  const int chunk = (lid / p.nqg) % p.nchunks;
-  const int bh = lid / (p.nqg * p.nchunks);
-  const int b = bh / p.H, h = bh % p.H;
+  const WorkId id = work_id(p.nqg, p.nchunks, p.H, p.head_inner);
+  const int qg = id.group, chunk = id.chunk, b = id.b, h = id.h, bh = b * p.H + h;
   const int i0 = chunk * p.rows_per_chunk;
   const int nrows = min(p.rows_per_chunk, p.L1 - i0);
   if (nrows <= 0) return;  // whole workgroup leaves together

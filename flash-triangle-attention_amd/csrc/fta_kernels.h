@@ -28,6 +28,7 @@ struct FwdParams {
   int L2p;             // the length the tiles cover: the next supported multiple of 128 (== L2 where that is one)
   int odd_bias;        // bias rows may start off an 8-byte boundary (strides that are not multiples of 4): the bias
                        // is then read entry by entry where it must be, like the tail of a row
+  int head_inner;      // the heads of a row are interleaved in memory (see work_id)
   int S;               // key slabs (waves sharing one query block)
   int QB;              // query blocks of 32 per workgroup
   int nqg;             // query groups = L2 / (32*QB)
@@ -104,6 +105,7 @@ struct BwdParams {
   int ring2;           // LDS ring slots of the Q/dO stage buffers
   int nb2;             // LDS buffers for the per-row K/V tiles
   DropParams drop;
+  int head_inner;      // the heads of a row are interleaved in memory (see work_id)
   int odd_bias;        // bias rows may start off an 8-byte boundary (strides that are not multiples of 4): the
                        // instances that mask a row's tail run, which read the bias entry by entry where they must
   int nat;             // (host side) the hand-scheduled backward kernels' precise instances run: exponents in
