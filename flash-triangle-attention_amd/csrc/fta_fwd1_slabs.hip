@@ -1,0 +1,12 @@
+// Forward, hand-scheduled (D = 32): the instances for rows of two and four key slabs.
+#include "fta_fwd1_kernel.h"
+
+namespace fta {
+
+hipError_t launch_fwd1_slabs(const FwdParams& p, const FwdPlan& pl, int dtype, bool tl, dim3 grid, dim3 block, hipStream_t st) {
+  FTA_FWD1_CASE(10, 8, 2, 2) FTA_FWD1_CASE(12, 8, 2, 2) FTA_FWD1_CASE(14, 8, 2, 2) FTA_FWD1_CASE(16, 8, 2, 2)
+  FTA_FWD1_CASE(10, 8, 2, 4) FTA_FWD1_CASE(12, 8, 2, 4) FTA_FWD1_CASE(14, 8, 2, 4)
+  return hipErrorInvalidConfiguration;
+}
+
+}  // namespace fta

@@ -337,6 +337,14 @@ def test_forward_rows_of_a_number_of_64_key_pairs_of_tiles(L1, L2, sm):
     _case(1, 2, L1, L2, 32, sm, seed=23)
 
 
+@pytest.mark.parametrize("sm", [1.0 / math.sqrt(32), 1.3])
+@pytest.mark.parametrize("L1,L2", [(3, 513), (9, 640), (4, 703), (2, 1024), (4, 1025), (9, 1280), (3, 1409), (2, 1729), (2, 1792)])
+def test_forward_rows_in_key_slabs(L1, L2, sm):
+    """The hand-scheduled D=32 forward cuts rows beyond 512 keys into two slabs, beyond 1024 into four, and merges them
+    per row; the last slab may end anywhere in its last two (four) stages of 64 keys."""
+    _case(1, 1, L1, L2, 32, sm, seed=29)
+
+
 @pytest.mark.parametrize("L2", [200, 203])
 def test_no_padded_copies_for_lengths_that_are_not_multiples_of_128(L2):
     """L2 = 200 (or 203) is tiled as 256 inside the kernels: peak memory of forward + backward stays within 5 %
