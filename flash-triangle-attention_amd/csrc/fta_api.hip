@@ -126,7 +126,8 @@ struct PlanKey {
 int padded_len_fwd(int L2, int D, int feat) {
   for (int lp = (L2 + 63) / 64 * 64; lp <= FTA_MAX_L2; lp += 64) {
     const fta::FwdPlan pl = fta::plan_fwd(1, 1, 1, lp, D, feat == 2);
-    if (pl.valid && (lp % 128 == 0 || pl.fwd1 == 1)) return lp;  // (only the hand-scheduled kernel has shapes in between)
+    // (shapes in between: the hand-scheduled kernel's, and rows of one slab with dropout at D = 32)
+    if (pl.valid && (lp % 128 == 0 || pl.fwd1 == 1 || (feat == 2 && D == 32 && pl.S == 1))) return lp;
   }
   return 0;
 }

@@ -316,6 +316,21 @@ __device__ __forceinline__ u32pair keep_block(const DP& d, uint32_t row, int j, 
 }
 template <class DP>
 __device__ __forceinline__ bool keep_byte(const DP& d, uint32_t bits, int n) { return ((bits >> (8 * n)) & 0xFFu) >= d.thresh; }
+// The keep bytes of four consecutive keys as masks of the packed pairs (keys 0, 1) and (2, 3): a kept weight's 16 bits
+// all ones.  The four bytes are compared at once: bit 7 of d says whether the low seven bits reach the threshold's,
+// and the bytes' own bit 7 decides together with it (or for thresholds below 128, and from there on); v_perm
+// spreads the bits of bytes 1 and 3 of either operand (selectors 8 to 11).  Nine instructions for four weights, where a
+// compare and a select per weight take eight and keep the pair from being converted by one instruction.
+struct KeepMasks {
+  uint32_t low, either;
+  template <class DP>
+  __device__ __forceinline__ explicit KeepMasks(const DP& d) : low((d.thresh & 0x7Fu) * 0x01010101u), either(d.thresh < 128u ? ~0u : 0u) {}
+  __device__ __forceinline__ u32pair pairs(uint32_t bits) const {
+    const uint32_t d = (bits | 0x80808080u) - low, x = bits ^ d;
+    const uint32_t g = (x & either) | (~x & d);
+    return u32pair{__builtin_amdgcn_perm(g << 8, g, 0x08080A0Au), __builtin_amdgcn_perm(g << 8, g, 0x09090B0Bu)};
+  }
+};
 // Neighbouring lanes need the same blocks: a value from another lane of the own group of four
 // (v_mov_b32 with a DPP quad permutation; lane i of a quad reads lane (SEL >> 2i) & 3).
 template <int SEL>

@@ -40,7 +40,8 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int
   // waves per workgroup: with one slab per row two independent workgroups of 4 waves share a CU
   // (their barriers do not couple: measured 5 to 20 % faster than one of 8); several slabs want the
   // 8 waves of one workgroup behind each staged tile.
-  const int maxw = (pl.S == 1 && D == 32) ? 4 : 8;
+  // (D = 32 with a number of query blocks that four does not divide: workgroups of two waves, four to a CU)
+  const int maxw = (pl.S == 1 && D == 32) ? (nqb % 4 == 0 ? 4 : 2) : 8;
   int qb = maxw / pl.S;
   if (qb < 1) qb = 1;
   while (qb > 1 && nqb % qb != 0) --qb;
@@ -89,7 +90,7 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int
     }
   // L1-row chunks: enough workgroups to fill 256 CUs a few times over, rows >= 8 per chunk
   // (two of the 4-wave workgroups fit a CU, one of the larger ones)
-  const long slots = (pl.threads <= 256 && pl.smem <= 80 * 1024) ? 512 : 256;
+  const long slots = (pl.threads <= 128 && pl.smem <= 40 * 1024) ? 1024 : (pl.threads <= 256 && pl.smem <= 80 * 1024) ? 512 : 256;
   const int nch = balanced_chunks((long)B * H * pl.nqg, L1, slots);
   pl.rows_per_chunk = (L1 + nch - 1) / nch;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
@@ -98,7 +99,7 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int
 }
 
 FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, bool feat) {
-  // L2 here is the length the tiles cover (a multiple of 128).  Slab widths are tried in this order,
+  // L2 here is the length the tiles cover (a multiple of 128, or of 64 where a rule below takes it).  Slab widths are tried in this order,
   // the first that has a built instance and a stage length that fits is taken:
   const int kwmax = (D == 32) ? 512 : 256;  // the widest that keeps the stationary bias within the register budget
   FwdPlan pl{};
@@ -115,6 +116,9 @@ FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, bool feat) {
   if (D == 64 && !feat)
     for (int c = 448; c >= 320; c -= 64)
       if (L2 % c == 0 && (L2 / c == 2 || L2 / c == 4)) take(c, true);
+  // Dropout at D=32: one slab of an odd number of 64-key steps (the only lengths in between the multiples of 128
+  // that these instances take: a slab count of one keeps the waves even)
+  if (D == 32 && feat && L2 % 128 == 64 && L2 < 512) take(L2);
   // 1. multiples of 128 keys from 256 on (longer stages, fewer barriers per row) with a slab count that
   //    is a power of two (fills the four SIMDs evenly: preferred over a wider slab)
   for (int c = kwmax; c >= 256; c -= 128)

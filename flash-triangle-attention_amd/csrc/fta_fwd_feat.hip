@@ -1,5 +1,8 @@
 // Forward: the kernel instances for bf16 tensors (the same tile shapes as fp16) and for dropout (fp16
 // and bf16: a smaller set, 64 keys per staged tile, 32 for the longest rows at D = 64; plan_fwd knows).
+// The dropout instances are bound by the vector ALU: the generator is a third of a tile's instructions, so neighbouring
+// lanes share its blocks and whole packed pairs are masked (KeepMasks).  B1 H4 L300 D32 bf16: 136 us with a generator
+// call per four weights, a select per weight and the row tiled as 384 keys, 87 us with these and 320 keys.
 #include "fta_fwd_kernel.h"
 
 namespace fta {

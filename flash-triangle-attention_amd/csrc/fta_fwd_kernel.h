@@ -26,7 +26,7 @@
   X(64, 4, 64) X(64, 8, 64) X(64, 8, 32) X(64, 10, 64) X(64, 12, 64) X(64, 12, 32) X(64, 14, 64)
 
 // The (D, NKT) instances built with dropout (64 keys per staged tile).
-#define FTA_FWD_FEAT_INSTANCES(X) X(32, 4) X(32, 8) X(32, 10) X(32, 12) X(32, 14) X(32, 16) X(64, 4) X(64, 8)
+#define FTA_FWD_FEAT_INSTANCES(X) X(32, 4) X(32, 6) X(32, 8) X(32, 10) X(32, 12) X(32, 14) X(32, 16) X(64, 4) X(64, 8)
 // (and with 32 keys per staged tile, for the five to eight slabs of rows beyond 1024 keys at D = 64)
 #define FTA_FWD_FEAT_INSTANCES_KT32(X) X(64, 8)
 
@@ -155,6 +155,10 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
   __syncthreads();
 
   const float scale = p.scale;
+  // DROP: the factor 1/(1 - p) of the kept weights is part of the exponent (the row sum carries it too and is freed of it
+  // at the end of the row), and whole packed pairs are masked.
+  [[maybe_unused]] const KeepMasks kept(p.drop);
+  [[maybe_unused]] const float drop_log2 = DROP ? __builtin_amdgcn_logf(p.drop.scale) : 0.f;
   [[maybe_unused]] const uint32_t rid = (uint32_t)(bh * p.L1 + i0);  // DROP: number of the first (b,h,i) row of the chunk
 
   // Stage n of the chunk lives in buffer n % 2.  With an odd number of stages per row that parity
@@ -235,17 +239,14 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
             for (int r = 0; r < 16; ++r) acc[dt][r] *= alpha;
           m = mnew;
         }
-        const float nm = -m * kLog2e;
+        const float nm = DROP ? __builtin_fmaf(-m, kLog2e, drop_log2) : -m * kLog2e;
 #pragma unroll
         for (int g = 0; g < 2 && gp + g < G; ++g) {
           uint32_t ph[8];
           [[maybe_unused]] uint32_t kb[4];  // DROP: the keep bytes of this lane's four groups of four keys
           if constexpr (DROP) {
             const int key = slab * KW + (t * G + gp + g) * 32 + 4 * hh;
-            // (every lane computes its four blocks: sharing them with the neighbouring lane, as the backward
-            // kernels do, costs this kernel more in spilled registers than the two calls it saves)
-#pragma unroll
-            for (int rg = 0; rg < 4; ++rg) kb[rg] = keep_bits(p.drop, rid + (uint32_t)ir, q0 + l32, key + 8 * rg);
+            keep_bits4_shared(p.drop, rid + (uint32_t)ir, q0 + l32, key, kb);
           }
 #pragma unroll
           for (int r = 0; r < 16; r += 2) {
@@ -253,9 +254,8 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
             float p1 = exp2_fast(__builtin_fmaf(s[g][r + 1], kLog2e, nm));
             if constexpr (DROP) {
               l += p0 + p1;
-              p0 = keep_byte(p.drop, kb[r >> 2], r & 3) ? p0 * p.drop.scale : 0.f;
-              p1 = keep_byte(p.drop, kb[r >> 2], (r & 3) + 1) ? p1 * p.drop.scale : 0.f;
-              ph[r >> 1] = T::pack_fast(p0, p1);
+              const u32pair mk = kept.pairs(kb[r >> 2]);
+              ph[r >> 1] = T::pack_fast(p0, p1) & ((r & 2) ? mk.y : mk.x);
             } else {
               ph[r >> 1] = T::pack_fast(p0, p1);
               l = T::sum2(ph[r >> 1], l);
@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
       if (p.alias_scratch) __syncthreads();
     }
     if (slab == 0 && q0 + l32 <= last) {
-      const float inv = 1.0f / l;
+      const float inv = (DROP ? p.drop.scale : 1.0f) / l;
       // The two lanes of a query (hh = 0, 1) hold alternating runs of four d values; one exchange per
       // register pair (v_permlane32_swap; both lanes are inside this branch together) gives each of them
       // eight consecutive ones, so the row goes out in 16-byte pieces: d = 32 dt + 16 pr + 8 hh .. +7.
@@ -329,7 +329,7 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
           *reinterpret_cast<u32x4*>(orow + 32 * dt + 16 * pr) = u32x4{(uint32_t)r0[0], (uint32_t)r1[0], (uint32_t)r0[1], (uint32_t)r1[1]};
         }
       if (hh == 0)
-        p.lse[((int64_t)bh * p.L1 + (i0 + ir)) * p.L2 + q0 + l32] = m * kLog2e + __builtin_amdgcn_logf(l);
+        p.lse[((int64_t)bh * p.L1 + (i0 + ir)) * p.L2 + q0 + l32] = m * kLog2e + __builtin_amdgcn_logf(l) - (DROP ? drop_log2 : 0.f);
     }
   }
   }

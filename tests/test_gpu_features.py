@@ -296,6 +296,23 @@ def test_dropout_against_the_oracle_with_the_same_mask(B, H, L1, L2, D, p, dtype
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L1,L2,p", [(4, 129, 0.1), (9, 192, 0.5), (5, 193, 0.75), (20, 300, 0.25), (3, 320, 0.9), (6, 321, 0.1), (5, 384, 0.6),
+                                     (7, 385, 0.25), (3, 448, 0.5), (4, 449, 0.1), (2, 700, 0.25), (2, 768, 0.4)])
+def test_dropout_at_the_tiled_lengths_of_head_dim_32(L1, L2, p, dtype):
+    """The dropout instances at the edges of the lengths they tile a row as, at keep thresholds below 128 (of 256), at it
+    and above, against the oracle with the mask rebuilt on the host."""
+    B, H, sm = 1, 2, 0.6
+    q, k, v, b, do = _inputs(B, H, L1, L2, 32, 31, dtype)
+    keep, scale = dm.keep_mask(77 + L2, p, B, H, L1, L2)
+    ref = _oracle(q, k, v, b, sm, do, keep=torch.from_numpy(keep).to(DEV), keep_scale=scale)
+    got = _run(q, k, v, b, sm, do, p, 77 + L2)
+    # (kept weights are 1/(1-p) times larger, and with them O and the rounding error of the weights (2^-10 of each in fp16,
+    # 2^-9 in bf16) and of O: the absolute tolerance of O is for weights that sum to one, i.e. for (1-p) O)
+    got["o"], ref["o"] = (got["o"].float() / scale).to(dtype), ref["o"] / scale
+    _compare(got, ref, dtype, f"dropout {L1}x{L2} p{p}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("D", [32, 64])
 @pytest.mark.parametrize("L1,L2,p", [(3, 2, 0.0), (5, 32, 0.0), (4, 33, 0.25), (6, 64, 0.1), (3, 65, 0.0), (7, 96, 0.25), (9, 97, 0.0), (40, 128, 0.1)])
 def test_one_kernel_backward_of_short_rows(L1, L2, p, D, dtype):
