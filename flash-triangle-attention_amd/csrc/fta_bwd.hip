@@ -20,17 +20,22 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
     if (L2 % c == 0) { kr = c; break; }
   pl.KR = kr;
   pl.nlaunch = L2 / kr;
-  pl.SK = kr / 128;
+  // Dropout at D = 32, key ranges of 384 keys: four slabs of 96 keys instead of three of 128, so that eight waves and
+  // not six share a CU's four SIMDs, and the query (key) blocks that hold nothing of the row have no workgroup.
+  const bool three = (feat == 2 && D == 32 && kr == 384);
+  const int nblk = (feat == 2) ? (row + 31) / 32 : nqb;
+  pl.NKT = three ? 3 : 4;
+  pl.SK = kr / (32 * pl.NKT);
   int qb = 8 / pl.SK;
   if (qb < 1) qb = 1;
   while (qb > 1 && nqb % qb != 0) --qb;
   pl.QB = qb;
-  pl.nqg = nqb / qb;
+  pl.nqg = (nblk + qb - 1) / qb;
   pl.threads = 64 * pl.SK * pl.QB;
-  const int G1 = (D == 32) ? 2 : 1;
+  const int G1 = (D == 32 && !three) ? 2 : 1;
   const int stage_rows = pl.SK * G1 * 32;
   const size_t slot1 = (size_t)2 * stage_rows * D * 2;
-  const int steps1 = 4 / G1;
+  const int steps1 = pl.NKT / G1;
   const size_t part1 = (pl.SK > 1) ? (size_t)(pl.threads / 64) * 16 * (D / 32) * 64 * ((D == 32) ? 4 : 2) : 0;
   const size_t qtile1 = (size_t)2 * pl.QB * 32 * D * 2;  // Q and dO rows of the workgroup, one L1 row
   pl.ring = 0;
@@ -49,10 +54,14 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
   int jw = 0;
   for (int c = jwmax; c >= 128; c -= 128)
     if (L2 % c == 0) { jw = c; break; }
+  // (dropout, lengths that three slabs of 128 queries would cut: two slabs of 192, for eight waves instead of six)
+  const bool two192 = (feat == 2 && D == 32 && jw == 128 && L2 % 384 == 0);
+  if (two192) jw = 192;
   pl.NJT = jw / 32;
   const int nslab = L2 / jw;
+  const int sjmax = two192 ? 2 : 4;
   bool ok2 = false;
-  for (int sj = (nslab < 4 ? nslab : 4); sj >= 1 && !ok2; --sj) {
+  for (int sj = (nslab < sjmax ? nslab : sjmax); sj >= 1 && !ok2; --sj) {
     if (nslab % sj != 0) continue;
     int kb = 8 / sj;
     if (kb < 1) continue;
@@ -68,7 +77,7 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
       for (int r = 4; r >= 3 && !ok2; --r) {
         const int nb = (r + steps2 - 1) / steps2;
         if (r * slot2 + nb * ktile2 + scratch2 > lds_max) continue;
-        pl.SJ = sj; pl.KB = kb; pl.nkg = nqb / kb; pl.threads2 = 64 * sj * kb; pl.JT = jt;
+        pl.SJ = sj; pl.KB = kb; pl.nkg = (nblk + kb - 1) / kb; pl.threads2 = 64 * sj * kb; pl.JT = jt;
         pl.ring2 = r; pl.nb2 = nb; pl.smem2 = r * slot2 + nb * ktile2 + scratch2;
         pl.JR = sj * jw; pl.nlaunch2 = L2 / pl.JR;
         ok2 = true;

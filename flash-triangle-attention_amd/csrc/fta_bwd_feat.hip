@@ -3,6 +3,12 @@
 // on their way into the matrix core).  Same four stages
 // as launch_bwd; the row constants and the bias are applied on the vector ALU (no MFMA folding), the
 // tail handling is always compiled in, and dK/dV has 64 or 32 queries per staged tile (plan_bwd knows).
+//
+// Dropout is bound by the vector ALU (the mask alone is two generator calls and 16 compares per tile and lane), so what
+// counts is instructions per score and that all four SIMDs of a CU have two waves.  B1 H4 L300 D32 bf16, dropout 0.25:
+// dQ/dBias 223 us with three slabs of 128 keys (six waves) and 1/(1 - p) multiplied in per score, 161 with four slabs
+// of 96 and the factor in the row constants; dK/dV 256 us with three slabs of 128 queries, each keep byte fetched from the
+// lane that made it, 145 with two slabs of 192 and the bytes of a key group transposed once per tile.
 #include "fta_bwd_kernels.h"
 
 namespace fta {
@@ -24,7 +30,8 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
     dim3 grid((unsigned)(p.B * p.H * pl.nqg * pl.nchunks)), block((unsigned)pl.threads);
     for (int n = 0; n < pl.nlaunch; ++n) {
       p.kr0 = n * pl.KR;
-      if (D == 32) e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2, 0, 512, true>, p, grid, block, pl.smem, st);
+      if (DROP && pl.NKT == 3) e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 1, 0, 512, true, 3>, p, grid, block, pl.smem, st);
+      else if (D == 32) e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2, 0, 512, true>, p, grid, block, pl.smem, st);
       else e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 64, 1, 0, 512, true>, p, grid, block, pl.smem, st);
       if (e != hipSuccess) return e;
     }
@@ -40,6 +47,7 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
   if (D == DD && pl.NJT == NN && pl.JT == JJ) e = launch_kernel(fta_bwd_dkdv_kernel<T, false, DROP, DD, NN, JJ, true>, p, grid, block, pl.smem2, st);
       FTA_DKDV_FEAT_CASE(32, 8, 64) FTA_DKDV_FEAT_CASE(32, 4, 64) FTA_DKDV_FEAT_CASE(32, 8, 32) FTA_DKDV_FEAT_CASE(32, 4, 32)
       FTA_DKDV_FEAT_CASE(64, 4, 64) FTA_DKDV_FEAT_CASE(64, 4, 32)
+      if constexpr (DROP) { FTA_DKDV_FEAT_CASE(32, 6, 64) }
 #undef FTA_DKDV_FEAT_CASE
       if (e != hipSuccess) return e;
     }

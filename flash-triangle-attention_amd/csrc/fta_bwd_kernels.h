@@ -63,8 +63,10 @@ __global__ void __launch_bounds__(256) fta_bwd_delta_kernel(const BwdParams p) {
     // the folded per-query constants of the dK/dV kernel: fp16 (hi, lo) splits of -lse (log2 domain)
     // and -delta, see split_2048().  A query beyond the row's true length gets -lse = kBiasFloorLog2:
     // its P is exactly 0, so the rows staged for it (copies of the last real query) add nothing to dK, dV.
+    // Dropout's factor c = 1/(1 - p) (1 without) goes into the raw pair: with P' = c P = exp(t - (lse - log c)), a kept
+    // weight is P' and dS = P' (mask dP - delta / c), so that neither takes a multiplication per score.
     if constexpr (RAW)
-      *reinterpret_cast<float2*>(p.aux + row * 2) = float2{real ? p.lse[lrow] : -kBiasFloorLog2, d};
+      *reinterpret_cast<float2*>(p.aux + row * 2) = float2{(real ? p.lse[lrow] : -kBiasFloorLog2) - __builtin_amdgcn_logf(p.drop.scale), d / p.drop.scale};
     else
       *reinterpret_cast<u32x2*>(p.aux + row * 2) = u32x2{split_2048(real ? -p.lse[lrow] : kBiasFloorLog2), split_2048(-d)};
   }
@@ -73,7 +75,7 @@ __global__ void __launch_bounds__(256) fta_bwd_delta_kernel(const BwdParams p) {
 // ------------------------------------------------------------------------------------------------
 // 1. dQ + dBias partials
 // ------------------------------------------------------------------------------------------------
-template <class T, bool DROP, int D, int G1, int AUGC, int MAXT, bool TAIL>
+template <class T, bool DROP, int D, int G1, int AUGC, int MAXT, bool TAIL, int NKT = 4>
 __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   // T: element type.  The MFMA folding of the row constants and of the pre-scaled bias is an fp16
   // device; bf16 inputs and DROP (whose mask sits between dP and the subtraction of delta) use AUGC = 0.
@@ -82,7 +84,7 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   // nothing for the clamped copies and predicated stores)
   // AUGC: which per-query constants are folded into the MFMAs here: 0 none, 1 -delta, 2 -delta and -lse
   constexpr bool AUG = (AUGC == 2);
-  constexpr int NKT = 4;            // 32-key tiles per wave slab (128 keys)
+  // NKT: 32-key tiles per wave slab (128 keys; with dropout also 96, where that makes four slabs of a key range)
   constexpr int STEPS = NKT / G1;   // stages per row (>= 2: the LDS reduction buffer relies on it)
   constexpr int KS = D / 16;
   constexpr int DT = D / 32;
@@ -91,7 +93,7 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
   const int SK = p.SK;
   const int slab = wave % SK, qb = wave / SK;
   const int hh = lane >> 5, l32 = lane & 31;
@@ -103,7 +105,7 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   if (nrows <= 0) return;
 
   const int q0 = (qg * p.QB + qb) * 32;
-  const int key0 = p.kr0 + slab * 128;
+  const int key0 = p.kr0 + slab * (NKT * 32);
   const int stage_rows = SK * G1 * 32;       // K (and V) rows per stage: G1 tiles for every slab
   const int buf_halfs = 2 * stage_rows * D;  // one ring slot: K tile then V tile
   const int R = p.ring;                      // ring slots; R - 2 stages are in flight beyond the next one
@@ -153,8 +155,8 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   // K/V staging: asynchronous global -> LDS copies into a ring of stage buffers
   const int nstage = nrows * STEPS;
   DmaPlan<2> plk, plv;
-  dma_plan<D, 2>(plk, stage_rows, G1 * 32, 128, p.ks[3], wave, lane, nwaves);
-  dma_plan<D, 2>(plv, stage_rows, G1 * 32, 128, p.vs[3], wave, lane, nwaves);
+  dma_plan<D, 2>(plk, stage_rows, G1 * 32, NKT * 32, p.ks[3], wave, lane, nwaves);
+  dma_plan<D, 2>(plv, stage_rows, G1 * 32, NKT * 32, p.vs[3], wave, lane, nwaves);
   const int ndma = plk.n + plv.n;  // K/V copies this wave issues per stage
   const int nqdma = 2 * dma_rows_count(QR, D, wave, nwaves);  // extra copies in a row's first stage
   const uint32_t lds0 = lds_addr_of(smem);
@@ -185,9 +187,9 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
     } else {
       // (kcur and vcur point at key kr0 of the row, qcur and docur at the workgroup's first query:
       // the clamped copies count rows from the start of the row)
-      dma_tile_clamped<D>(kcur - (int64_t)p.kr0 * p.ks[3], p.ks[3], stage_rows, G1 * 32, 128, p.kr0 + cur_t * (G1 * 32), last, dst,
+      dma_tile_clamped<D>(kcur - (int64_t)p.kr0 * p.ks[3], p.ks[3], stage_rows, G1 * 32, NKT * 32, p.kr0 + cur_t * (G1 * 32), last, dst,
                           wave, lane, nwaves);
-      dma_tile_clamped<D>(vcur - (int64_t)p.kr0 * p.vs[3], p.vs[3], stage_rows, G1 * 32, 128, p.kr0 + cur_t * (G1 * 32), last,
+      dma_tile_clamped<D>(vcur - (int64_t)p.kr0 * p.vs[3], p.vs[3], stage_rows, G1 * 32, NKT * 32, p.kr0 + cur_t * (G1 * 32), last,
                           dst + (uint32_t)(stage_rows * D) * 2u, wave, lane, nwaves);
       if (cur_t == 0) {
         dma_tile_clamped<D>(qcur - (int64_t)(qg * QR) * p.qs[3], p.qs[3], QR, QR, 0, qg * QR, last, qd, wave, lane, nwaves);
@@ -221,6 +223,7 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
 
   const float scale = p.scale;
   const float sl2 = p.scale * kLog2e;
+  [[maybe_unused]] const float drop_log2 = __builtin_amdgcn_logf(p.drop.scale), drop_inv = 1.0f / p.drop.scale;
   int cur = 0;                    // ring slot of the stage being read
   int fill = (ahead + 1) % R;     // ring slot the next issued stage goes to
 
@@ -256,7 +259,9 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
-    const float nl = -lse_c;
+    // DROP: P' = P / (1 - p), dS = P' (mask dP - (1 - p) delta)
+    const float nl = DROP ? drop_log2 - lse_c : -lse_c;
+    if constexpr (DROP) delta_c *= drop_inv;
 
 #pragma unroll
     for (int t = 0; t < STEPS; ++t) {
@@ -296,9 +301,9 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
             p0 = exp2_fast(__builtin_fmaf(t0, kLog2e, nl));
             p1 = exp2_fast(__builtin_fmaf(t1, kLog2e, nl));
             float e0 = dp[r], e1 = dp[r + 1];
-            if constexpr (DROP) {  // dP = mask/(1-p) * dP_dropped
-              e0 = keep_byte(p.drop, kb[r >> 2], r & 3) ? e0 * p.drop.scale : 0.f;
-              e1 = keep_byte(p.drop, kb[r >> 2], (r & 3) + 1) ? e1 * p.drop.scale : 0.f;
+            if constexpr (DROP) {  // (1 - p) dP
+              e0 = keep_byte(p.drop, kb[r >> 2], r & 3) ? e0 : 0.f;
+              e1 = keep_byte(p.drop, kb[r >> 2], (r & 3) + 1) ? e1 : 0.f;
             }
             d0 = (AUGC == 1) ? p0 * e0 : p0 * (e0 - delta_c);
             d1 = (AUGC == 1) ? p1 * e1 : p1 * (e1 - delta_c);
@@ -396,7 +401,7 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
     }
   }
 
-  // stage one of the dBias reduction: this chunk's sums for the wave's 32 x 128 tile
+  // stage one of the dBias reduction: this chunk's sums for the wave's 32 queries and its slab of keys
   float* part = p.partial + (((int64_t)chunk * p.B * p.H + bh) * p.L2p + (q0 + l32)) * p.L2p + key0 + 4 * hh;
 #pragma unroll
   for (int tt = 0; tt < NKT; ++tt)
@@ -427,7 +432,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
   const int SJ = p.SJ;
   const int jslab = wave % SJ, kb = wave / SJ;
   const int hh = lane >> 5, l32 = lane & 31;
@@ -642,13 +647,18 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
           const float* cF = reinterpret_cast<const float*>(cL) + (g * 32 + 4 * hh) * 2;
           // DROP: the eight blocks of this tile (query pairs m = 0..7: accumulator rows 2m, 2m+1) are the
           // same for the four lanes of a key group; each lane computes pairs q and q + 4 (q = its place in
-          // the group) and the others are read from the lane that has them
-          [[maybe_unused]] u32pair blkA{0u, 0u}, blkB{0u, 0u};
+          // the group) and the bytes change lanes: kb[w] holds this lane's key, byte s of word w (the even and the
+          // odd query of pairs s, then of pairs s + 4)
+          [[maybe_unused]] uint32_t kb[4];
           if constexpr (DROP) {
             const int qd = l32 & 3, jtile = p.jr0 + jslab * JW + jt * 32 + 4 * hh;
             const uint32_t rowid = (uint32_t)(bh * p.L1 + i0 + ir);
-            blkA = keep_block(p.drop, rowid, jtile + 8 * (qd >> 1) + 2 * (qd & 1), k0 + l32);          // pair m = q
-            blkB = keep_block(p.drop, rowid, jtile + 8 * ((qd + 4) >> 1) + 2 * (qd & 1), k0 + l32);    // pair m = q + 4
+            const u32pair blkA = keep_block(p.drop, rowid, jtile + 8 * (qd >> 1) + 2 * (qd & 1), k0 + l32);          // pair m = q
+            const u32pair blkB = keep_block(p.drop, rowid, jtile + 8 * ((qd + 4) >> 1) + 2 * (qd & 1), k0 + l32);    // pair m = q + 4
+            kb[0] = quad_transpose_bytes(blkA.x, lane);
+            kb[1] = quad_transpose_bytes(blkA.y, lane);
+            kb[2] = quad_transpose_bytes(blkB.x, lane);
+            kb[3] = quad_transpose_bytes(blkB.y, lane);
           }
 #pragma unroll
           for (int rg = 0; rg < 4; ++rg) {
@@ -664,19 +674,13 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
               float e0 = dp[r], e1 = dp[r + 1];
               float w0 = p0, w1 = p1;  // the weights that dV sees
               if constexpr (DROP) {
-                // rows r, r+1 are the queries 2*(j/2), 2*(j/2)+1 of one block; this lane's key picks the byte
-                const int m = 2 * rg + e / 2;  // the pair: its block is held by lane m & 3 of the group
-                const u32pair src = (m < 4) ? blkA : blkB;
-                u32pair blk;
-                if ((m & 3) == 0) blk = u32pair{quad_perm<0x00>(src.x), quad_perm<0x00>(src.y)};
-                else if ((m & 3) == 1) blk = u32pair{quad_perm<0x55>(src.x), quad_perm<0x55>(src.y)};
-                else if ((m & 3) == 2) blk = u32pair{quad_perm<0xAA>(src.x), quad_perm<0xAA>(src.y)};
-                else blk = u32pair{quad_perm<0xFF>(src.x), quad_perm<0xFF>(src.y)};
-                const bool k0b = keep_byte(p.drop, blk.x, (k0 + l32) & 3), k1b = keep_byte(p.drop, blk.y, (k0 + l32) & 3);
-                w0 = k0b ? p0 * p.drop.scale : 0.f;
-                w1 = k1b ? p1 * p.drop.scale : 0.f;
-                e0 = k0b ? e0 * p.drop.scale : 0.f;
-                e1 = k1b ? e1 * p.drop.scale : 0.f;
+                const int m = 2 * rg + e / 2;  // the query pair of rows r, r+1
+                const bool k0b = keep_byte(p.drop, kb[m < 4 ? 0 : 2], m & 3), k1b = keep_byte(p.drop, kb[m < 4 ? 1 : 3], m & 3);
+                w0 = k0b ? p0 : 0.f;
+                w1 = k1b ? p1 : 0.f;
+                e0 = k0b ? e0 : 0.f;
+                e1 = k1b ? e1 : 0.f;
+                asm("" : "+v"(w0), "+v"(w1));  // (otherwise each is converted by itself, selected and packed: twice the instructions)
               }
               pp[r >> 1] = T::pack_fast(w0, w1);
               dsp[r >> 1] = T::pack_fast(p0 * (e0 - del4[e]), p1 * (e1 - del4[e + 1]));

@@ -337,6 +337,12 @@ template <int SEL>
 __device__ __forceinline__ uint32_t quad_perm(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, SEL, 0xF, 0xF, true);
 }
+// Four lanes with a word each, transposed as a 4 x 4 matrix of bytes: byte s of the result is byte q of lane s's word,
+// q and s counted inside the group of four.  Two exchanges, with the neighbour and with the other pair.
+__device__ __forceinline__ uint32_t quad_transpose_bytes(uint32_t v, int lane) {
+  const uint32_t a = __builtin_amdgcn_perm(v, quad_perm<0xB1>(v), (lane & 1) ? 0x07030501u : 0x02060004u);
+  return __builtin_amdgcn_perm(a, quad_perm<0x4E>(a), (lane & 2) ? 0x07060302u : 0x01000504u);
+}
 // Transposed score layout (the forward and the dQ kernel: a lane owns one query and, per tile, four
 // groups of four keys: kfirst + 8g .. +3, g = 0..3).  The two lanes of a query pair (adjacent lanes:
 // query and lane have the same parity) need the same four blocks, each its own word of them; each

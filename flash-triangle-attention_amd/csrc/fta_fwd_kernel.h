@@ -50,7 +50,7 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nthreads = blockDim.x;
   const int S = p.S;
   const int slab = wave % S;

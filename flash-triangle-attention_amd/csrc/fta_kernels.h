@@ -140,6 +140,7 @@ struct ShortPlan {
 struct BwdPlan {
   // dQ/dBias kernel
   int SK, QB, nqg, nchunks, rows_per_chunk, threads, KR, nlaunch, ring, nb;
+  int NKT;             // 32-key tiles of a wave's slab
   size_t smem;
   // dK/dV kernel
   int NJT, JT, SJ, KB, nkg, nchunks2, rows_per_chunk2, threads2, JR, nlaunch2, ring2, nb2;
