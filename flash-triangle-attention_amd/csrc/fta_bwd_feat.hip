@@ -8,7 +8,9 @@
 // counts is instructions per score and that all four SIMDs of a CU have two waves.  B1 H4 L300 D32 bf16, dropout 0.25:
 // dQ/dBias 223 us with three slabs of 128 keys (six waves) and 1/(1 - p) multiplied in per score, 161 with four slabs
 // of 96 and the factor in the row constants; dK/dV 256 us with three slabs of 128 queries, each keep byte fetched from the
-// lane that made it, 145 with two slabs of 192 and the bytes of a key group transposed once per tile.
+// lane that made it, 145 with two slabs of 192 and the bytes of a key group transposed once per tile.  With the geometry
+// fixed at compile time where eight waves share the row: training passes of 386 to 325 us there (dQ/dBias 118), 350 to 299
+// at B2 H4 L256 and 2.41 to 2.18 ms at B1 H8 L512 (dK/dV alone).
 #include "fta_bwd_kernels.h"
 
 namespace fta {
@@ -30,9 +32,16 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
     dim3 grid((unsigned)(p.B * p.H * pl.nqg * pl.nchunks)), block((unsigned)pl.threads);
     for (int n = 0; n < pl.nlaunch; ++n) {
       p.kr0 = n * pl.KR;
-      if (DROP && pl.NKT == 3) e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 1, 0, 512, true, 3>, p, grid, block, pl.smem, st);
-      else if (D == 32) e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2, 0, 512, true>, p, grid, block, pl.smem, st);
-      else e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 64, 1, 0, 512, true>, p, grid, block, pl.smem, st);
+      e = hipErrorInvalidConfiguration;
+      if (pl.NKT == 3) {  // key ranges of 384 keys with dropout: fixed geometry
+        if constexpr (DROP)
+          if (D == 32 && pl.threads == 512 && pl.SK == 4 && pl.ring == dq_ring(32, 3, 1, 4).r && pl.nb == dq_ring(32, 3, 1, 4).nb)
+            e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 0, 512, true, 3, 4>, p, grid, block, pl.smem, st);
+      } else if (D == 32) {
+        e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2, 0, 512, true>, p, grid, block, pl.smem, st);
+      } else {
+        e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 64, 1, 0, 512, true>, p, grid, block, pl.smem, st);
+      }
       if (e != hipSuccess) return e;
     }
     p.kr0 = 0;
@@ -44,10 +53,18 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
       p.jr0 = n * pl.JR;
       e = hipErrorInvalidConfiguration;
 #define FTA_DKDV_FEAT_CASE(DD, NN, JJ) \
-  if (D == DD && pl.NJT == NN && pl.JT == JJ) e = launch_kernel(fta_bwd_dkdv_kernel<T, false, DROP, DD, NN, JJ, true>, p, grid, block, pl.smem2, st);
+  if (e == hipErrorInvalidConfiguration && D == DD && pl.NJT == NN && pl.JT == JJ) \
+    e = launch_kernel(fta_bwd_dkdv_kernel<T, false, DROP, DD, NN, JJ, true>, p, grid, block, pl.smem2, st);
+      if constexpr (DROP) {  // fixed geometry: query ranges of 256, 384, 512 and 1024 queries
+#define FTA_DKDV_FIX_CASE(NN, SS)                                                                                        \
+  if (D == 32 && pl.threads2 == 512 && pl.NJT == NN && pl.JT == 64 && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, 64, SS).r &&  \
+      pl.nb2 == dkdv_ring(32, NN, 64, SS).nb)                                                                            \
+    e = launch_kernel(fta_bwd_dkdv_kernel<T, false, true, 32, NN, 64, true, SS>, p, grid, block, pl.smem2, st);
+        FTA_DKDV_FIX_CASE(6, 2) FTA_DKDV_FIX_CASE(8, 1) FTA_DKDV_FIX_CASE(8, 2) FTA_DKDV_FIX_CASE(8, 4)
+#undef FTA_DKDV_FIX_CASE
+      }
       FTA_DKDV_FEAT_CASE(32, 8, 64) FTA_DKDV_FEAT_CASE(32, 4, 64) FTA_DKDV_FEAT_CASE(32, 8, 32) FTA_DKDV_FEAT_CASE(32, 4, 32)
       FTA_DKDV_FEAT_CASE(64, 4, 64) FTA_DKDV_FEAT_CASE(64, 4, 32)
-      if constexpr (DROP) { FTA_DKDV_FEAT_CASE(32, 6, 64) }
 #undef FTA_DKDV_FEAT_CASE
       if (e != hipSuccess) return e;
     }

@@ -22,6 +22,7 @@
 
 #include "fta_common.h"
 #include "fta_kernels.h"
+#include "fta_pipe.h"
 
 namespace fta {
 
@@ -75,7 +76,7 @@ __global__ void __launch_bounds__(256) fta_bwd_delta_kernel(const BwdParams p) {
 // ------------------------------------------------------------------------------------------------
 // 1. dQ + dBias partials
 // ------------------------------------------------------------------------------------------------
-template <class T, bool DROP, int D, int G1, int AUGC, int MAXT, bool TAIL, int NKT = 4>
+template <class T, bool DROP, int D, int G1, int AUGC, int MAXT, bool TAIL, int NKT = 4, int SKC = 0>
 __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   // T: element type.  The MFMA folding of the row constants and of the pre-scaled bias is an fp16
   // device; bf16 inputs and DROP (whose mask sits between dP and the subtraction of delta) use AUGC = 0.
@@ -84,6 +85,13 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   // nothing for the clamped copies and predicated stores)
   // AUGC: which per-query constants are folded into the MFMAs here: 0 none, 1 -delta, 2 -delta and -lse
   constexpr bool AUG = (AUGC == 2);
+  // SKC: the number of slabs where it is known at compile time (eight waves, TAIL): the geometry is then constant, every
+  // wave issues the same number of copies per stage, and their offsets are formed from two registers.  With the geometry
+  // in kernel arguments a third of the instructions per tile moved or made scalars (slabs of 96 keys, B1 H4 L300 with
+  // dropout: 162 against 118 us).  Slabs of 128 keys have no registers for it: 70 spilled, 2.41 against 2.51 ms a training
+  // pass at B1 H8 L512, so those keep the run-time geometry.
+  constexpr bool FIX = (SKC != 0);
+  static_assert(!FIX || (TAIL && D == 32), "fixed geometry");
   // NKT: 32-key tiles per wave slab (128 keys; with dropout also 96, where that makes four slabs of a key range)
   constexpr int STEPS = NKT / G1;   // stages per row (>= 2: the LDS reduction buffer relies on it)
   constexpr int KS = D / 16;
@@ -93,8 +101,8 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
-  const int SK = p.SK;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = FIX ? 8 : blockDim.x >> 6;
+  const int SK = FIX ? SKC : p.SK, QB = FIX ? 8 / (FIX ? SKC : 1) : p.QB;
   const int slab = wave % SK, qb = wave / SK;
   const int hh = lane >> 5, l32 = lane & 31;
 
@@ -104,14 +112,14 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   const int nrows = min(p.rows_per_chunk, p.L1 - i0);
   if (nrows <= 0) return;
 
-  const int q0 = (qg * p.QB + qb) * 32;
+  const int q0 = (qg * QB + qb) * 32;
   const int key0 = p.kr0 + slab * (NKT * 32);
   const int stage_rows = SK * G1 * 32;       // K (and V) rows per stage: G1 tiles for every slab
   const int buf_halfs = 2 * stage_rows * D;  // one ring slot: K tile then V tile
-  const int R = p.ring;                      // ring slots; R - 2 stages are in flight beyond the next one
+  const int R = FIX ? dq_ring(D, NKT, G1, SKC).r : p.ring;  // ring slots; R - 2 stages are in flight beyond the next one
   const int ahead = R - 2;
-  const int QR = p.QB * 32;                  // query rows of the workgroup
-  const int NB = p.nb;                       // row-operand buffers (rows whose Q/dO tiles are in flight)
+  const int QR = QB * 32;                    // query rows of the workgroup
+  const int NB = FIX ? dq_ring(D, NKT, G1, SKC).nb : p.nb;  // row-operand buffers (rows whose Q/dO tiles are in flight)
   half_t* qtiles = smem + R * buf_halfs;     // [NB][Q tile | dO tile], QR x D each
   // cross-slab dQ partials: fp32 for D=32; fp16 for D=64, where fp32 would not fit in LDS
   typedef typename std::conditional<D == 32, float, half_t>::type part_t;
@@ -165,10 +173,10 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   // workgroup's Q and dO rows of that row (read as B operands at the start of the row)
   // Stages are issued in order; the cursor keeps the row pointers so that issuing costs scalar adds.
   int cur_ir = 0, cur_t = 0;  // (row, step) of the next stage to issue
-  const half_t* kcur = kbase + (int64_t)i0 * p.ks[2] + (int64_t)p.kr0 * p.ks[3];
-  const half_t* vcur = vbase + (int64_t)i0 * p.vs[2] + (int64_t)p.kr0 * p.vs[3];
-  const half_t* qcur = qbase + (int64_t)i0 * p.qs[2] + (int64_t)(qg * p.QB * 32) * p.qs[3];
-  const half_t* docur = dobase + (int64_t)i0 * p.dos[2] + (int64_t)(qg * p.QB * 32) * p.dos[3];
+  const half_t* kcur = kbase + (int64_t)i0 * p.ks[2] + (int64_t)(FIX ? 0 : p.kr0) * p.ks[3];
+  const half_t* vcur = vbase + (int64_t)i0 * p.vs[2] + (int64_t)(FIX ? 0 : p.kr0) * p.vs[3];
+  const half_t* qcur = qbase + (int64_t)i0 * p.qs[2] + (int64_t)(FIX ? 0 : qg * QB * 32) * p.qs[3];
+  const half_t* docur = dobase + (int64_t)i0 * p.dos[2] + (int64_t)(FIX ? 0 : qg * QB * 32) * p.dos[3];
   const int64_t kstep = (int64_t)(G1 * 32) * p.ks[3], vstep = (int64_t)(G1 * 32) * p.vs[3];
   // (a row length that is not a multiple of the tile: rows beyond it are copies of the last real
   // key or query; such keys are masked through the bias, such queries are never stored)
@@ -203,6 +211,38 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
       kcur += p.ks[2]; vcur += p.vs[2]; qcur += p.qs[2]; docur += p.dos[2];
     }
   };
+  // FIX: pieces of 16 rows (one copy each), dealt to the eight waves; the cursors stand at the start of the row
+  constexpr int PK = FIX ? SKC * G1 * 2 / 8 : 0, PQ = FIX ? 32 / (FIX ? SKC : 1) / 8 : 0;  // per wave: K (and V) pieces of a stage; Q and dO pieces of a row
+  const uint32_t crow = (uint32_t)lane >> 2, ccol = (uint32_t)swz_slot<D>(lane >> 2, lane & 3) * 16u;
+  auto piece = [&](const half_t* row, uint32_t stride2, int first, uint32_t dst) {
+    uint32_t cr = crow;
+    asm volatile("" : "+v"(cr));  // (offsets kept over the rows would take the registers of the tiles)
+    dma16s(min((uint32_t)first + cr, (uint32_t)last) * stride2 + ccol, uniform_ptr(row), __builtin_amdgcn_readfirstlane(dst));
+  };
+  auto stage_fix = [&](auto tc, int slot) {
+    constexpr int t = decltype(tc)::value;
+    const uint32_t dst = lds0 + (uint32_t)(slot * buf_halfs) * 2u;
+#pragma unroll
+    for (int u = 0; u < PK; ++u) {
+      const int tr = (wave + 8 * u) * 16, first = p.kr0 + tr / (G1 * 32) * (NKT * 32) + t * (G1 * 32) + tr % (G1 * 32);
+      piece(kcur, (uint32_t)(2 * p.ks[3]), first, dst + (uint32_t)tr * (D * 2));
+      piece(vcur, (uint32_t)(2 * p.vs[3]), first, dst + (uint32_t)(stage_rows + tr) * (D * 2));
+    }
+    if constexpr (t == 0) {
+      const uint32_t qd = ldsq + (uint32_t)((cur_ir % NB) * 2 * QR * D) * 2u;
+#pragma unroll
+      for (int u = 0; u < PQ; ++u) {
+        const int tr = (wave + 8 * u) * 16;  // of the Q rows and then the dO rows
+        const bool isq = tr < QR;
+        const int w = isq ? tr : tr - QR;
+        piece(isq ? qcur : docur, (uint32_t)(2 * (isq ? p.qs[3] : p.dos[3])), qg * QR + w, qd + (uint32_t)tr * (D * 2));
+      }
+    }
+    if constexpr (t == STEPS - 1) {
+      ++cur_ir;
+      kcur += p.ks[2]; vcur += p.vs[2]; qcur += p.qs[2]; docur += p.dos[2];
+    }
+  };
   auto stage_copies = [&](int sidx) { return ndma + ((sidx % STEPS == 0) ? nqdma : 0); };
 
   // per-row operands of this wave's 32 queries: Q^T and dO^T B-operand fragments (from the staged
@@ -216,7 +256,13 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
     delta_n = p.delta[((int64_t)bh * p.L1 + i) * p.L2p + q0 + l32];
   };
 
-  for (int s0 = 0; s0 <= ahead && s0 < nstage; ++s0) stage(s0);
+  if constexpr (FIX) {
+    static_for<0, dq_ring(D, NKT, G1, SKC).r - 1>([&](auto sc) {
+      if (decltype(sc)::value < nstage) stage_fix(std::integral_constant<int, decltype(sc)::value % STEPS>{}, decltype(sc)::value);
+    });
+  } else {
+    for (int s0 = 0; s0 <= ahead && s0 < nstage; ++s0) stage(s0);
+  }
   rowload(0);
   wait_vmem_all();
   __syncthreads();
@@ -263,8 +309,8 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
     const float nl = DROP ? drop_log2 - lse_c : -lse_c;
     if constexpr (DROP) delta_c *= drop_inv;
 
-#pragma unroll
-    for (int t = 0; t < STEPS; ++t) {
+    static_for<0, STEPS>([&](auto tc) {
+      constexpr int t = decltype(tc)::value;
       const int sidx = ir * STEPS + t;
       const half_t* cK = smem + cur * buf_halfs;
       const half_t* cV = cK + stage_rows * D;
@@ -272,6 +318,7 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
 #pragma unroll
       for (int g = 0; g < G1; ++g) {
         const int tt = t * G1 + g;
+        if constexpr (FIX) __builtin_amdgcn_sched_barrier(0);  // (tiles interleaved need more registers than there are)
         floatx16 s, dp;
 #pragma unroll
         for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
@@ -284,7 +331,9 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
         uint32_t dsp[8];
         [[maybe_unused]] uint32_t kb[4];  // DROP: the keep bytes of this lane's four groups of four keys
         if constexpr (DROP) {
-          keep_bits4_shared(p.drop, (uint32_t)(bh * p.L1 + i0 + ir), q0 + l32, key0 + tt * 32 + 4 * hh, kb);
+          int jl = q0 + l32, kl = key0 + 4 * hh;
+          if constexpr (FIX) asm volatile("" : "+v"(jl), "+v"(kl));  // (nor are the generator's counters kept over the rows)
+          keep_bits4_shared(p.drop, (uint32_t)(bh * p.L1 + i0 + ir), jl, kl + tt * 32, kb);
         }
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
@@ -331,16 +380,28 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
       }
       // keep `ahead` stages in flight beyond the one the next step reads
       const int nxt = sidx + 1 + ahead;
-      if (nxt < nstage) {
-        stage(fill);
-        fill = (fill + 1 == R) ? 0 : fill + 1;
-      }
       cur = (cur + 1 == R) ? 0 : cur + 1;
-      int pending = 0;  // copies of the stages issued after the one the next step reads
-      for (int s2 = sidx + 2; s2 <= nxt && s2 < nstage; ++s2) pending += stage_copies(s2);
-      wait_vmem_leq(pending);
+      if constexpr (FIX) {
+        constexpr int AHEAD = dq_ring(D, NKT, G1, SKC).r - 2;
+        if (nxt < nstage) {
+          stage_fix(std::integral_constant<int, (t + 1 + AHEAD) % STEPS>{}, fill);
+          fill = (fill + 1 == R) ? 0 : fill + 1;
+          constexpr int firsts = (AHEAD >= 1 && (t + 2) % STEPS == 0 ? 1 : 0) + (AHEAD >= 2 && (t + 3) % STEPS == 0 ? 1 : 0);
+          wait_vmem_leq(AHEAD * 2 * PK + firsts * PQ);
+        } else {
+          wait_vmem_all();
+        }
+      } else {
+        if (nxt < nstage) {
+          stage(fill);
+          fill = (fill + 1 == R) ? 0 : fill + 1;
+        }
+        int pending = 0;  // copies of the stages issued after the one the next step reads
+        for (int s2 = sidx + 2; s2 <= nxt && s2 < nstage; ++s2) pending += stage_copies(s2);
+        wait_vmem_leq(pending);
+      }
       __syncthreads();
-    }
+    });
 
     // dQ: the SK slab waves of a query block each finish a share of the 8-byte output groups
     half_t* dqr = dqbase + (int64_t)(i0 + ir) * p.dqs[2] + (int64_t)(q0 + l32) * p.dqs[3] + 4 * hh;
@@ -419,9 +480,12 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
 // core (an fp16 device: pre-scaled K, one-hot bias steps, fp16 splits in aux); without it they are
 // applied on the vector ALU in fp32 from the raw {lse, delta} pairs in aux, which is what bf16
 // inputs and DROP (whose mask sits between dP and the subtraction of delta) need.
-template <class T, bool FOLD, bool DROP, int D, int NJT, int JT, bool TAIL>
+// SJC: the number of query slabs where it is known at compile time, as in the dQ kernel.
+template <class T, bool FOLD, bool DROP, int D, int NJT, int JT, bool TAIL, int SJC = 0>
 __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   static_assert(!FOLD || (!T::is_bf16 && !DROP), "folded constants: fp16 without dropout only");
+  constexpr bool FIX = (SJC != 0);
+  static_assert(!FIX || (TAIL && D == 32 && JT == 64), "fixed geometry");
   constexpr int G = JT / 32;                // 32-query tiles per stage (JT queries per slab and stage)
   constexpr int STEPS = NJT / G;
   constexpr int JW = NJT * 32;              // queries per wave slab
@@ -432,8 +496,8 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
-  const int SJ = p.SJ;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = FIX ? 8 : blockDim.x >> 6;
+  const int SJ = FIX ? SJC : p.SJ, KB = FIX ? 8 / (FIX ? SJC : 1) : p.KB;
   const int jslab = wave % SJ, kb = wave / SJ;
   const int hh = lane >> 5, l32 = lane & 31;
 
@@ -443,14 +507,14 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   const int nrows = min(p.rows_per_chunk2, p.L1 - i0);
   if (nrows <= 0) return;
 
-  const int k0 = (kg * p.KB + kb) * 32;  // first key of this wave
+  const int k0 = (kg * KB + kb) * 32;  // first key of this wave
   const int stage_rows = SJ * JT;
   // one ring slot: Q tile, dO tile (halfs), then lse and delta of the same rows (floats)
   const int slot_halfs = 2 * stage_rows * D + 4 * stage_rows;
-  const int R = p.ring2;
+  const int R = FIX ? dkdv_ring(D, NJT, JT, SJC).r : p.ring2;
   const int ahead = R - 2;
-  const int KR2 = p.KB * 32;                 // key rows of the workgroup
-  const int NB = p.nb2;                      // row-operand buffers (rows whose K/V tiles are in flight)
+  const int KR2 = KB * 32;                   // key rows of the workgroup
+  const int NB = FIX ? dkdv_ring(D, NJT, JT, SJC).nb : p.nb2;                      // row-operand buffers (rows whose K/V tiles are in flight)
   half_t* ktiles = smem + R * slot_halfs;    // [NB][K tile | V tile], KR2 x D each
   half_t* scratch = ktiles + NB * 2 * KR2 * D;  // cross-slab dK/dV partials, kept in fp16 to fit in LDS
   FragOffsets<D> fo;
@@ -526,10 +590,10 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   // workgroup's K and V rows of that row (read as B operands at the start of the row)
   // Stages are issued in order; the cursor keeps the row pointers so that issuing costs scalar adds.
   int cur_ir = 0, cur_t = 0;  // (row, step) of the next stage to issue
-  const half_t* qcur = qbase + (int64_t)i0 * p.qs[2] + (int64_t)p.jr0 * p.qs[3];
-  const half_t* docur = dobase + (int64_t)i0 * p.dos[2] + (int64_t)p.jr0 * p.dos[3];
-  const half_t* kcur = kbase + (int64_t)i0 * p.ks[2] + (int64_t)(kg * p.KB * 32) * p.ks[3];
-  const half_t* vcur = vbase + (int64_t)i0 * p.vs[2] + (int64_t)(kg * p.KB * 32) * p.vs[3];
+  const half_t* qcur = qbase + (int64_t)i0 * p.qs[2] + (int64_t)(FIX ? 0 : p.jr0) * p.qs[3];
+  const half_t* docur = dobase + (int64_t)i0 * p.dos[2] + (int64_t)(FIX ? 0 : p.jr0) * p.dos[3];
+  const half_t* kcur = kbase + (int64_t)i0 * p.ks[2] + (int64_t)(FIX ? 0 : kg * KB * 32) * p.ks[3];
+  const half_t* vcur = vbase + (int64_t)i0 * p.vs[2] + (int64_t)(FIX ? 0 : kg * KB * 32) * p.vs[3];
   const uint32_t* acur = p.aux + (((int64_t)bh * p.L1 + i0) * p.L2p + p.jr0) * 2;
   const int64_t qstep = (int64_t)JT * p.qs[3], dostep = (int64_t)JT * p.dos[3];
   // (a row length that is not a multiple of the tile: rows beyond it are copies of the last real
@@ -575,6 +639,45 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
       acur += 2 * p.L2p;
     }
   };
+  // FIX: pieces of 16 rows (one copy each), dealt to the eight waves; the cursors stand at the start of the row
+  constexpr int PQ = FIX ? SJC : 0, PK = FIX ? 4 / (FIX ? SJC : 1) : 0;  // per wave: Q and dO pieces of a stage; K and V pieces of a row
+  const uint32_t crow = (uint32_t)lane >> 2, ccol = (uint32_t)swz_slot<D>(lane >> 2, lane & 3) * 16u;
+  auto piece = [&](const half_t* row, uint32_t stride2, int first, uint32_t dst) {
+    uint32_t cr = crow;
+    asm volatile("" : "+v"(cr));  // (offsets kept over the rows would take the registers of the tiles)
+    dma16s(min((uint32_t)first + cr, (uint32_t)last) * stride2 + ccol, uniform_ptr(row), __builtin_amdgcn_readfirstlane(dst));
+  };
+  auto stage_fix = [&](auto tc, int slot) {
+    constexpr int t = decltype(tc)::value;
+    const uint32_t dst = lds0 + (uint32_t)(slot * slot_halfs) * 2u;
+    if constexpr (t == 0) {
+      const uint32_t kd = ldsk + (uint32_t)((cur_ir % NB) * 2 * KR2 * D) * 2u;
+#pragma unroll
+      for (int u = 0; u < PK; ++u) {
+        const int tr = (wave + 8 * u) * 16;  // of the K rows and then the V rows
+        const bool isk = tr < KR2;
+        piece(isk ? kcur : vcur, (uint32_t)(2 * (isk ? p.ks[3] : p.vs[3])), kg * KR2 + (isk ? tr : tr - KR2), kd + (uint32_t)tr * (D * 2));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PQ; ++u) {
+      const int tr = (wave + 8 * u) * 16;  // of the Q rows and then the dO rows
+      const bool isq = tr < stage_rows;
+      const int w = isq ? tr : tr - stage_rows;
+      piece(isq ? qcur : docur, (uint32_t)(2 * (isq ? p.qs[3] : p.dos[3])), p.jr0 + w / JT * JW + t * JT + w % JT, dst + (uint32_t)tr * (D * 2));
+    }
+    // (lse, delta): 2 * SJ copies of 16 lanes; the waves beyond them repeat one (the same bytes to the same place), so that
+    // all waves have the same number in flight
+    const int c = wave % (2 * SJ), which = c / SJ, sl = c % SJ;
+    const uint32_t* src = acur + (t * JT + sl * JW) * 2 + which * JT;
+    const uint32_t la = __builtin_amdgcn_readfirstlane(dst + (uint32_t)(2 * stage_rows * D) * 2u + (uint32_t)(sl * JT * 2 + which * JT) * 4u);
+    if (lane < JT / 4) dma16s((uint32_t)lane * 16u, uniform_ptr(src), la);
+    if constexpr (t == STEPS - 1) {
+      ++cur_ir;
+      qcur += p.qs[2]; docur += p.dos[2]; kcur += p.ks[2]; vcur += p.vs[2];
+      acur += 2 * p.L2p;
+    }
+  };
   auto stage_copies = [&](int sidx) { return ndma + ((sidx % STEPS == 0) ? nkdma : 0); };
 
   // K and V B-operand fragments of this wave's 32 keys for one row (from the staged rows)
@@ -582,7 +685,13 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   const bool PAIRX = (SJ == 2) && (STEPS >= 2);  // balanced exchange between the two slabs of a key block
   float keep[16 * DT];
 
-  for (int s0 = 0; s0 <= ahead && s0 < nstage; ++s0) stage(s0);
+  if constexpr (FIX) {
+    static_for<0, dkdv_ring(D, NJT, JT, SJC).r - 1>([&](auto sc) {
+      if (decltype(sc)::value < nstage) stage_fix(std::integral_constant<int, decltype(sc)::value % STEPS>{}, decltype(sc)::value);
+    });
+  } else {
+    for (int s0 = 0; s0 <= ahead && s0 < nstage; ++s0) stage(s0);
+  }
   wait_vmem_all();
   __syncthreads();
 
@@ -609,8 +718,8 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) { dk[dt][r] = 0.f; dv[dt][r] = 0.f; }
 
-#pragma unroll
-    for (int t = 0; t < STEPS; ++t) {
+    static_for<0, STEPS>([&](auto tc) {
+      constexpr int t = decltype(tc)::value;
       const int sidx = ir * STEPS + t;
       const half_t* cQ = smem + cur * slot_halfs;
       const half_t* cDO = cQ + stage_rows * D;
@@ -619,6 +728,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         const int jt = t * G + g;
+        if constexpr (FIX) __builtin_amdgcn_sched_barrier(0);  // (as in the dQ kernel)
         floatx16 s, dp;
 #pragma unroll
         for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
@@ -651,14 +761,16 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
           // odd query of pairs s, then of pairs s + 4)
           [[maybe_unused]] uint32_t kb[4];
           if constexpr (DROP) {
-            const int qd = l32 & 3, jtile = p.jr0 + jslab * JW + jt * 32 + 4 * hh;
+            int ln = lane;
+            if constexpr (FIX) asm volatile("" : "+v"(ln));  // (the generator's counters are not kept over the rows)
+            const int qd = ln & 3, jtile = p.jr0 + jslab * JW + jt * 32 + 4 * (ln >> 5), kl = k0 + (ln & 31);
             const uint32_t rowid = (uint32_t)(bh * p.L1 + i0 + ir);
-            const u32pair blkA = keep_block(p.drop, rowid, jtile + 8 * (qd >> 1) + 2 * (qd & 1), k0 + l32);          // pair m = q
-            const u32pair blkB = keep_block(p.drop, rowid, jtile + 8 * ((qd + 4) >> 1) + 2 * (qd & 1), k0 + l32);    // pair m = q + 4
-            kb[0] = quad_transpose_bytes(blkA.x, lane);
-            kb[1] = quad_transpose_bytes(blkA.y, lane);
-            kb[2] = quad_transpose_bytes(blkB.x, lane);
-            kb[3] = quad_transpose_bytes(blkB.y, lane);
+            const u32pair blkA = keep_block(p.drop, rowid, jtile + 8 * (qd >> 1) + 2 * (qd & 1), kl);          // pair m = q
+            const u32pair blkB = keep_block(p.drop, rowid, jtile + 8 * ((qd + 4) >> 1) + 2 * (qd & 1), kl);    // pair m = q + 4
+            kb[0] = quad_transpose_bytes(blkA.x, ln);
+            kb[1] = quad_transpose_bytes(blkA.y, ln);
+            kb[2] = quad_transpose_bytes(blkB.x, ln);
+            kb[3] = quad_transpose_bytes(blkB.y, ln);
           }
 #pragma unroll
           for (int rg = 0; rg < 4; ++rg) {
@@ -719,16 +831,28 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
         }
       }
       const int nxt = sidx + 1 + ahead;
-      if (nxt < nstage) {
-        stage(fill);
-        fill = (fill + 1 == R) ? 0 : fill + 1;
-      }
       cur = (cur + 1 == R) ? 0 : cur + 1;
-      int pending = 0;  // copies of the stages issued after the one the next step reads
-      for (int s2 = sidx + 2; s2 <= nxt && s2 < nstage; ++s2) pending += stage_copies(s2);
-      wait_vmem_coarse(pending);
+      if constexpr (FIX) {
+        constexpr int AHEAD = dkdv_ring(D, NJT, JT, SJC).r - 2;
+        if (nxt < nstage) {
+          stage_fix(std::integral_constant<int, (t + 1 + AHEAD) % STEPS>{}, fill);
+          fill = (fill + 1 == R) ? 0 : fill + 1;
+          constexpr int firsts = (AHEAD >= 1 && (t + 2) % STEPS == 0 ? 1 : 0) + (AHEAD >= 2 && (t + 3) % STEPS == 0 ? 1 : 0);
+          wait_vmem_leq(AHEAD * (PQ + 1) + firsts * PK);
+        } else {
+          wait_vmem_all();
+        }
+      } else {
+        if (nxt < nstage) {
+          stage(fill);
+          fill = (fill + 1 == R) ? 0 : fill + 1;
+        }
+        int pending = 0;  // copies of the stages issued after the one the next step reads
+        for (int s2 = sidx + 2; s2 <= nxt && s2 < nstage; ++s2) pending += stage_copies(s2);
+        wait_vmem_coarse(pending);
+      }
       __syncthreads();
-    }
+    });
 
     if (PAIRX) {
       const u32x2* in = reinterpret_cast<const u32x2*>(scratch) + (size_t)(wave ^ 1) * (4 * DT * 64) + lane;

@@ -176,6 +176,24 @@ hipError_t launch_short(BwdParams p, const ShortPlan& pl, int D, int dtype, bool
 bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl);
 hipError_t launch_dkdv1(BwdParams p, const Dkdv1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st);
 
+// Stage buffers and row-operand buffers that 160 KB hold beside the exchange records: of the dQ/dBias kernel with SK slabs
+// of NKT tiles, G1 of them to a stage, and of the dK/dV kernel with SJ slabs of NJT tiles, JT queries to a stage; eight
+// waves each (the kernels with that geometry fixed and the launch plan agree on it).
+struct Ring { int r, nb; };
+constexpr Ring fit_ring(int steps, int slot, int row, int records) {
+  for (int r = 4; r >= 3; --r) {
+    const int nb = (r + steps - 1) / steps;
+    if (r * slot + nb * row + records <= 160 * 1024) return Ring{r, nb};
+  }
+  return Ring{0, 0};
+}
+constexpr Ring dq_ring(int D, int NKT, int G1, int SK) {
+  return fit_ring(NKT / G1, 4 * SK * G1 * 32 * D, 4 * (8 / SK) * 32 * D, SK > 1 ? 8 * 16 * (D / 32) * 64 * (D == 32 ? 4 : 2) : 0);
+}
+constexpr Ring dkdv_ring(int D, int NJT, int JT, int SJ) {
+  return fit_ring(NJT / (JT / 32), 4 * SJ * JT * D + 8 * SJ * JT, 4 * (8 / SJ) * 32 * D, (SJ - 1) * (8 / SJ) * 32 * (D / 32) * 64 * 2);
+}
+
 // L2 is the length the tiles cover (a multiple of 128), `row` the true row length.
 // `feat`: 0 the fp16 kernels; 1 the plan is for bf16 inputs or the precise mode, 2 for dropout (general
 // kernels only, smaller instance sets).
