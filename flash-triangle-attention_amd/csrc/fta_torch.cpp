@@ -2,11 +2,12 @@
 // kernels read in place.  A call checks its arguments, allocates outputs and launches, without going through
 // the Python interpreter, and its backward runs in the autograd thread without taking the interpreter lock
 // for more than one flag.  Anything it does not take -- wrong types or shapes, layouts that need a copy,
-// another device than the current one -- it leaves to the Python path by returning None, which copies or
-// raises as documented there.
+// another device than the current one, a thread whose operations something else watches -- it leaves to the
+// Python path by returning None, which copies, records or raises as documented there.
 #include <ATen/autocast_mode.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
 #include <atomic>
@@ -35,6 +36,14 @@ bool plain(const Tensor& t, int device) {
          !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchGradWrapper,
                                                    c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchVmapMode,
                                                    c10::DispatchKey::Functionalize}));
+}
+// Whether something watches or rewrites this thread's operations: jit tracing, a Python dispatch mode, a functorch
+// transform (which need not show in this call's tensors).  The launches below are no operations, so a trace would hold
+// the allocations of the outputs alone, and replay them.
+bool watched() {
+  return torch::jit::tracer::isTracing() ||
+         c10::impl::tls_local_dispatch_key_set().included_.has_any(
+             c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchDynamicLayerFrontMode, c10::DispatchKey::Functionalize}));
 }
 bool wants_grad(std::initializer_list<const Tensor*> ts) {
   if (!at::GradMode::is_enabled()) return false;
@@ -136,6 +145,7 @@ struct Attention : public torch::autograd::Function<Attention> {
 py::object attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, double scale, double dropout_p,
                      int64_t seed, py::dict globals) {
   const py::object none = py::none();
+  if (watched()) return none;
   const at::ScalarType dt = q.scalar_type();
   if ((dt != at::kHalf && dt != at::kBFloat16) || k.scalar_type() != dt || v.scalar_type() != dt || b.scalar_type() != dt) return none;
   if (q.dim() != 5 || b.dim() != 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes() || !q.is_cuda()) return none;
@@ -247,6 +257,7 @@ struct Block : public torch::autograd::Function<Block> {
 py::object block(const Tensor& z, const std::optional<Tensor>& key_mask, const std::vector<std::optional<Tensor>>& weights, int64_t H,
                  int64_t D, bool starting, double eps, double dropout_p, int64_t seed, py::dict globals) {
   const py::object none = py::none();
+  if (watched()) return none;
   const at::ScalarType dt = z.scalar_type();
   if ((dt != at::kHalf && dt != at::kBFloat16 && dt != at::kFloat) || z.dim() != 4 || z.size(1) != z.size(2) || z.numel() == 0) return none;
   if (!z.is_cuda() || at::autocast::is_autocast_enabled(at::kCUDA) || weights.size() != 10) return none;

@@ -185,8 +185,9 @@ class _attention(torch.autograd.Function):
             seed = _draw_seed() if float(dropout_p) > 0.0 else 0
         ctx.n_extra = len(extra)
         # same preconditions as upstream forward (:557-561)
-        HEAD_DIM_Q, HEAD_DIM_K = q.shape[-1], k.shape[-1]
-        HEAD_DIM_V = v.shape[-1]
+        # (int: under torch.jit.trace a size is a traced value, which is in no set of numbers)
+        HEAD_DIM_Q, HEAD_DIM_K = int(q.shape[-1]), int(k.shape[-1])
+        HEAD_DIM_V = int(v.shape[-1])
         assert HEAD_DIM_Q == HEAD_DIM_K and HEAD_DIM_K == HEAD_DIM_V
         assert HEAD_DIM_K in {16, 32, 64, 128, 256}
         assert q.dtype == k.dtype == v.dtype == b_pw.dtype
@@ -199,7 +200,7 @@ class _attention(torch.autograd.Function):
         if not q.is_cuda:
             raise ValueError("attention() needs tensors on the GPU; there is no CPU path")
         assert q.dim() == 5 and k.shape == q.shape and v.shape == q.shape
-        B, H, L1, L2, D = q.shape
+        B, H, L1, L2, D = map(int, q.shape)
         assert tuple(b_pw.shape) == (B, H, L2, L2), "bias must be (B, H, L2, L2)"
         dtype = q.dtype
 

@@ -1,0 +1,61 @@
+"""What the C++ host path has to leave to the Python path, and what attention() and the block then do there: a call whose
+operations something watches (tracing, dispatch modes, functorch)."""
+import pytest
+import torch
+
+from oracle import tt_attn_oracle as orc
+
+gpu = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _operands(seed, L2=96):
+    return orc.make_inputs(1, 2, 5, L2, 32, seed=seed, device=DEV)
+
+
+def _block(C=64, D=32, H=2, **kw):
+    from triangle_attention import TriangleAttention
+    torch.manual_seed(1)
+    return TriangleAttention(C, D, H, **kw).to(DEV)
+
+
+def _pair(seed, L=48, C=64):
+    return torch.randn(1, L, L, C, device=DEV, generator=torch.Generator(DEV).manual_seed(seed))
+
+
+@gpu
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+def test_a_traced_call_runs_the_kernels_on_replay():
+    """The trace is replayed on other inputs than it was recorded on, twice, so that no buffer can hold the answer."""
+    from flash_tt_attn import attention
+    blk = _block().eval()
+    with torch.no_grad():
+        op = torch.jit.trace(lambda q, k, v, b: attention(q, k, v, b, 0.3), _operands(1)[:4], check_trace=False)
+        mod = torch.jit.trace(blk, (_pair(1),), check_trace=False)
+        for seed in (2, 3):
+            x, z = _operands(seed)[:4], _pair(seed)
+            assert torch.equal(op(*x), attention(*x, 0.3))
+            # (the fused block against separate layers: fp32 with the attention in fp16, as in the block's own tests)
+            assert orc.rel_l2(mod(z), blk(z)) <= 1e-3
+
+
+@gpu
+def test_a_dispatch_mode_sees_the_operations_of_the_block():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Log(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    blk, z, seen = _block(), _pair(1), []
+    with Log(), torch.no_grad():
+        blk(z)
+    assert any("native_layer_norm" in str(f) for f in seen)
+
+
+@gpu
+def test_functorch_transforms_are_refused_also_where_they_only_enclose_the_call():
+    from flash_tt_attn import attention
+    x = _operands(1)[:4]
+    with pytest.raises(RuntimeError, match="functorch"):
+        torch.vmap(lambda t: t.sum() + attention(*x, 0.3).sum())(torch.ones(3, 2, device=DEV))
