@@ -30,9 +30,10 @@ bool readable(const Tensor& t) {
     if (s[i] % 8 != 0) return false;
   return true;
 }
-// A plain tensor on the current GPU: no subclass or transform that has to see the operations.
+// A plain tensor on the current GPU: no subclass or transform that has to see the operations, and no tangent (the
+// operator has no forward-mode derivative: the Python function says so, here the output would come without one).
 bool plain(const Tensor& t, int device) {
-  return t.is_cuda() && t.device().index() == device && t.layout() == at::kStrided &&
+  return t.is_cuda() && t.device().index() == device && t.layout() == at::kStrided && !t._fw_grad(/*level=*/0).defined() &&
          !t.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Python, c10::DispatchKey::FuncTorchGradWrapper,
                                                    c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchVmapMode,
                                                    c10::DispatchKey::Functionalize}));

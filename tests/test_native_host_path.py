@@ -1,7 +1,8 @@
 """What the C++ host path has to leave to the Python path, and what attention() and the block then do there: a call whose
-operations something watches (tracing, dispatch modes, functorch)."""
+operations something watches (tracing, dispatch modes, functorch), tensors with a tangent."""
 import pytest
 import torch
+import torch.autograd.forward_ad as fwad
 
 from oracle import tt_attn_oracle as orc
 
@@ -59,3 +60,23 @@ def test_functorch_transforms_are_refused_also_where_they_only_enclose_the_call(
     x = _operands(1)[:4]
     with pytest.raises(RuntimeError, match="functorch"):
         torch.vmap(lambda t: t.sum() + attention(*x, 0.3).sum())(torch.ones(3, 2, device=DEV))
+
+
+@gpu
+@pytest.mark.parametrize("which", ["q", "k", "v", "bias", "z", "weight"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_forward_mode_derivatives_are_refused_not_dropped(which, grad):
+    from flash_tt_attn import attention
+    dual = lambda t: fwad.make_dual(t.detach(), torch.ones_like(t))
+    x, blk, z = list(_operands(1)[:4]), _block().requires_grad_(False), _pair(1)
+    with fwad.dual_level(), torch.set_grad_enabled(grad), pytest.raises(NotImplementedError, match="jvp"):
+        if which in ("z", "weight"):
+            if which == "weight":
+                blk.linear_v._parameters["weight"] = dual(blk.linear_v.weight)
+            blk(dual(z) if which == "z" else z)
+        else:
+            n = ("q", "k", "v", "bias").index(which)
+            x[n] = dual(x[n])
+            if grad:
+                x[n - 1].requires_grad_(True)
+            attention(*x, 0.3)
