@@ -38,6 +38,9 @@ bool plain(const Tensor& t, int device) {
                                                    c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchVmapMode,
                                                    c10::DispatchKey::Functionalize}));
 }
+// A torch.Tensor or Parameter itself.  A subclass, which may do without __torch_dispatch__, keeps its type through
+// the Python path.
+bool exact_tensor(py::handle h) { return THPVariable_CheckExact(h.ptr()); }
 // Whether something watches or rewrites this thread's operations: jit tracing, a Python dispatch mode, a functorch
 // transform (which need not show in this call's tensors).  The launches below are no operations, so a trace would hold
 // the allocations of the outputs alone, and replay them.
@@ -143,9 +146,13 @@ struct Attention : public torch::autograd::Function<Attention> {
   }
 };
 
-py::object attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, double scale, double dropout_p,
-                     int64_t seed, py::dict globals) {
+py::object attention(py::handle qh, py::handle kh, py::handle vh, py::handle bh, double scale, double dropout_p, int64_t seed,
+                     py::dict globals) {
   const py::object none = py::none();
+  for (const py::handle h : {qh, kh, vh, bh})
+    if (!exact_tensor(h)) return none;
+  const Tensor &q = THPVariable_Unpack(qh.ptr()), &k = THPVariable_Unpack(kh.ptr()), &v = THPVariable_Unpack(vh.ptr()),
+               &b = THPVariable_Unpack(bh.ptr());
   if (watched()) return none;
   const at::ScalarType dt = q.scalar_type();
   if ((dt != at::kHalf && dt != at::kBFloat16) || k.scalar_type() != dt || v.scalar_type() != dt || b.scalar_type() != dt) return none;
@@ -255,9 +262,11 @@ struct Block : public torch::autograd::Function<Block> {
   }
 };
 
-py::object block(const Tensor& z, const std::optional<Tensor>& key_mask, const std::vector<std::optional<Tensor>>& weights, int64_t H,
-                 int64_t D, bool starting, double eps, double dropout_p, int64_t seed, py::dict globals) {
+py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std::vector<py::object>& weights, int64_t H, int64_t D,
+                 bool starting, double eps, double dropout_p, int64_t seed, py::dict globals) {
   const py::object none = py::none();
+  if (!exact_tensor(zh)) return none;
+  const Tensor& z = THPVariable_Unpack(zh.ptr());
   if (watched()) return none;
   const at::ScalarType dt = z.scalar_type();
   if ((dt != at::kHalf && dt != at::kBFloat16 && dt != at::kFloat) || z.dim() != 4 || z.size(1) != z.size(2) || z.numel() == 0) return none;
@@ -268,11 +277,12 @@ py::object block(const Tensor& z, const std::optional<Tensor>& key_mask, const s
   const int64_t HD = H * D, rows[10] = {c.C, c.C, HD, HD, HD, H, HD, HD, c.C, c.C}, cols[10] = {0, 0, c.C, c.C, c.C, c.C, c.C, 0, HD, 0};
   Tensor w[10];
   for (int n = 0; n < 10; ++n) {
-    if (!weights[n].has_value()) {
+    if (weights[n].is_none()) {
       if (n != 7 && n != 9) return none;
       continue;
     }
-    w[n] = *weights[n];
+    if (!exact_tensor(weights[n])) return none;
+    w[n] = THPVariable_Unpack(weights[n].ptr());
     if (w[n].scalar_type() != dt || !plain(w[n], dev) || !w[n].is_contiguous() || reinterpret_cast<uintptr_t>(w[n].data_ptr()) % 16 != 0)
       return none;
     if (w[n].dim() != (cols[n] ? 2 : 1) || w[n].size(0) != rows[n] || (cols[n] && w[n].size(1) != cols[n])) return none;

@@ -160,7 +160,7 @@ class _attention(torch.autograd.Function):
             native = _native or _load_native()
             try:
                 o = native(*args[:4], *map(float, args[4:6]), *args[6:], globals=_GLOBALS)
-            except TypeError:  # (not tensors, or a seed beyond 63 bits)
+            except TypeError:  # (a seed that is no integer of 63 bits)
                 o = None
             if o is not None:
                 return o

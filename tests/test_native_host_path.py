@@ -1,5 +1,6 @@
 """What the C++ host path has to leave to the Python path, and what attention() and the block then do there: a call whose
-operations something watches (tracing, dispatch modes, functorch), tensors with a tangent."""
+operations something watches (tracing, dispatch modes, functorch), tensors with a tangent,
+tensor subclasses."""
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
@@ -80,3 +81,16 @@ def test_forward_mode_derivatives_are_refused_not_dropped(which, grad):
             if grad:
                 x[n - 1].requires_grad_(True)
             attention(*x, 0.3)
+
+
+@gpu
+def test_tensor_subclasses_keep_their_type():
+    from flash_tt_attn import attention
+
+    class Sub(torch.Tensor):
+        pass
+    x, blk, z = list(_operands(1)[:4]), _block(), _pair(1)
+    got, plain = attention(x[0].as_subclass(Sub), *x[1:], 0.3), attention(*x, 0.3)
+    assert type(got) is Sub and type(plain) is torch.Tensor and torch.equal(got.as_subclass(torch.Tensor), plain)
+    assert type(blk(z.as_subclass(Sub))) is Sub
+    assert type(attention(torch.nn.Parameter(x[0]), *x[1:], 0.3)) is torch.Tensor
