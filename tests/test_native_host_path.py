@@ -1,6 +1,6 @@
 """What the C++ host path has to leave to the Python path, and what attention() and the block then do there: a call whose
 operations something watches (tracing, dispatch modes, functorch), tensors with a tangent,
-tensor subclasses."""
+tensor subclasses, sizes that are not built."""
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
@@ -94,3 +94,13 @@ def test_tensor_subclasses_keep_their_type():
     assert type(got) is Sub and type(plain) is torch.Tensor and torch.equal(got.as_subclass(torch.Tensor), plain)
     assert type(blk(z.as_subclass(Sub))) is Sub
     assert type(attention(torch.nn.Parameter(x[0]), *x[1:], 0.3)) is torch.Tensor
+
+
+@gpu
+@pytest.mark.parametrize("C,D,H", [(64, 16, 4), (64, 16, 8), (128, 128, 1)])
+def test_a_refused_head_dim_leaves_other_calls_of_its_length_alone(C, D, H):
+    z = _pair(1, 71 + H, C)  # (a length no other test asks for)
+    with pytest.raises(ValueError, match="not built"):
+        _block(C, D, H)(z)
+    z = z[..., :64].contiguous()
+    assert _block()._fused(z, None, None) is not None
