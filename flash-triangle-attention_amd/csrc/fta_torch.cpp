@@ -81,7 +81,7 @@ fta_options make_options(at::ScalarType dtype, double dropout_p, uint64_t seed, 
 // Whether rows of L2 keys run forward and backward with these options: asked once per length and kind.
 bool length_supported(int64_t L2, int64_t D, const fta_options& o) {
   static std::atomic<uint8_t> known[2][2][2][FTA_MAX_L2 + 1];  // head dim, type, dropout: 0 unknown, 1 no, 2 yes
-  if (L2 < 1 || L2 > FTA_MAX_L2 || (D != 32 && D != 64)) return false;  // (what has no place in the table is not asked for)
+  if (L2 < 1 || L2 > FTA_MAX_L2 || (D != 32 && D != 64) || !(o.dropout_p < 1.f)) return false;  // (not what the table is about)
   auto& k = known[D == 64][o.dtype == FTA_DTYPE_BF16][o.dropout_p > 0.f][L2];
   uint8_t v = k.load(std::memory_order_relaxed);
   if (v == 0) {

@@ -195,7 +195,7 @@ class _attention(torch.autograd.Function):
             raise ValueError(f"head dim {HEAD_DIM_K} is not built for gfx950 (supported: {SUPPORTED_HEAD_DIMS})")
         if q.dtype not in (torch.float16, torch.bfloat16):
             raise ValueError("only float16 and bfloat16 inputs are supported")
-        if not (0.0 <= float(dropout_p) < 1.0):
+        if not (0.0 <= float(dropout_p) and ctypes.c_float(float(dropout_p)).value < 1.0):  # (the library takes it in fp32)
             raise ValueError("dropout_p must be in [0, 1)")
         if not q.is_cuda:
             raise ValueError("attention() needs tensors on the GPU; there is no CPU path")

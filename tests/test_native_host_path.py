@@ -104,3 +104,12 @@ def test_a_refused_head_dim_leaves_other_calls_of_its_length_alone(C, D, H):
         _block(C, D, H)(z)
     z = z[..., :64].contiguous()
     assert _block()._fused(z, None, None) is not None
+
+
+def test_a_dropout_probability_that_rounds_to_one_is_refused_as_such():
+    """(not as a length that is not built, which would be kept for the length)"""
+    import flash_tt_attn as fta
+    x = torch.zeros(1, 1, 1, 8, 32, dtype=torch.float16)
+    for p in (1.0, 1.0 - 1e-9, float("nan"), -0.1):
+        with pytest.raises(ValueError, match="dropout_p"):
+            fta.attention(x, x, x, torch.zeros(1, 1, 8, 8, dtype=torch.float16), 0.1, p, 3)
