@@ -263,7 +263,7 @@ struct Block : public torch::autograd::Function<Block> {
 };
 
 py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std::vector<py::object>& weights, int64_t H, int64_t D,
-                 bool starting, double eps, double dropout_p, int64_t seed, py::dict globals) {
+                 bool starting, double eps, double dropout_p, std::optional<int64_t> given_seed, py::dict globals) {
   const py::object none = py::none();
   if (!exact_tensor(zh)) return none;
   const Tensor& z = THPVariable_Unpack(zh.ptr());
@@ -272,7 +272,7 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
   if ((dt != at::kHalf && dt != at::kBFloat16 && dt != at::kFloat) || z.dim() != 4 || z.size(1) != z.size(2) || z.numel() == 0) return none;
   if (!z.is_cuda() || at::autocast::is_autocast_enabled(at::kCUDA) || weights.size() != 10) return none;
   const int dev = (int)c10::hip::current_device();
-  const BlockCall c{z.size(3), H, D, seed, starting ? 1 : 0, eps, dropout_p};
+  BlockCall c{z.size(3), H, D, given_seed.value_or(0), starting ? 1 : 0, eps, dropout_p};
   if (!plain(z, dev) || !readable(z) || !(dropout_p >= 0.0 && dropout_p < 1.0)) return none;
   const int64_t HD = H * D, rows[10] = {c.C, c.C, HD, HD, HD, H, HD, HD, c.C, c.C}, cols[10] = {0, 0, c.C, c.C, c.C, c.C, c.C, 0, HD, 0};
   Tensor w[10];
@@ -294,9 +294,12 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
       return none;
     mask = key_mask->to(dt).contiguous();
   }
-  const fta_block b = block_args(z, mask, w, c, false);
-  fta_options opt = make_options(dt, dropout_p, (uint64_t)seed, false);
-  if (!length_supported(b.L, D, opt) || fta_block_check(&b) != FTA_OK) return none;
+  fta_block b = block_args(z, mask, w, c, false);
+  if (!length_supported(b.L, D, make_options(dt, dropout_p, 0, false)) || fta_block_check(&b) != FTA_OK) return none;
+  if (dropout_p > 0.0 && !given_seed) {  // (drawn only now that the call is taken: the Python path draws its own)
+    c.seed = py::cast<int64_t>(globals["_draw_seed"]());
+    b.seed = (uint64_t)c.seed;
+  }
   if (!wants_grad({&z, &w[0], &w[1], &w[2], &w[3], &w[4], &w[5], &w[6], &w[7], &w[8], &w[9]})) {
     Tensor out, state;
     at::AutoDispatchBelowADInplaceOrView below;
@@ -304,7 +307,7 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
     return py::cast(out);
   }
   auto opt_t = [](const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
-  return py::cast(Block::apply(z, opt_t(mask), w[0], w[1], w[2], w[3], w[4], w[5], w[6], opt_t(w[7]), w[8], opt_t(w[9]), c.C, H, D, seed,
+  return py::cast(Block::apply(z, opt_t(mask), w[0], w[1], w[2], w[3], w[4], w[5], w[6], opt_t(w[7]), w[8], opt_t(w[9]), c.C, H, D, c.seed,
                                c.starting, eps, dropout_p, (int64_t) reinterpret_cast<intptr_t>(globals.ptr())));
 }
 

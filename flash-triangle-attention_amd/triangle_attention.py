@@ -101,11 +101,9 @@ class TriangleAttention(nn.Module):
             return None
         scope = _attention.forward.__globals__  # (the module that holds the PRECISE_BACKWARD switch)
         p = self.dropout_p if self.training else 0.0
-        if p > 0.0 and seed is None:
-            seed = scope["_draw_seed"]()
         try:
             return fta_lib.native().block(z, key_mask, weights, self.n_heads, self.c_hidden, self.starting, norm.eps, p,
-                                          seed if p > 0.0 else 0, scope)
+                                          seed if p > 0.0 else 0, scope)  # (no seed: one is drawn if the call is taken)
         except TypeError:  # (a seed beyond 63 bits, a mask that is no tensor)
             return None
 

@@ -21,6 +21,12 @@ def _block(C=64, D=32, H=2, **kw):
     return TriangleAttention(C, D, H, **kw).to(DEV)
 
 
+def _separate(blk):
+    """The same block as separate layers around attention(): a subclass does not take the fused kernels."""
+    from triangle_attention import TriangleAttention
+    return type("Separate", (TriangleAttention,), {})(blk.c_z, blk.c_hidden, blk.n_heads, blk.starting, blk.dropout_p).to(DEV)
+
+
 def _pair(seed, L=48, C=64):
     return torch.randn(1, L, L, C, device=DEV, generator=torch.Generator(DEV).manual_seed(seed))
 
@@ -113,3 +119,23 @@ def test_a_dropout_probability_that_rounds_to_one_is_refused_as_such():
     for p in (1.0, 1.0 - 1e-9, float("nan"), -0.1):
         with pytest.raises(ValueError, match="dropout_p"):
             fta.attention(x, x, x, torch.zeros(1, 1, 8, 8, dtype=torch.float16), 0.1, p, 3)
+
+
+@gpu
+@pytest.mark.parametrize("autocast", [False, True])
+def test_a_call_draws_one_dropout_seed_whichever_path_takes_it(autocast):
+    """The generator ends where one draw leaves it, and the mask is that draw's, on the fused path and on the separate
+    layers (which the fused path leaves an autocast call to)."""
+    z, blk = _pair(1), _block(dropout_p=0.25)
+    sep = _separate(blk)
+    sep.load_state_dict(blk.state_dict())
+    outs, states = [], []
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        for m in (blk, sep):
+            torch.manual_seed(5)
+            outs.append(m(z).float())
+            states.append(torch.get_rng_state())
+    torch.manual_seed(5)
+    torch.randint(0, 2 ** 62, (1,))
+    assert all(torch.equal(s, torch.get_rng_state()) for s in states)
+    assert (blk._fused(z, None, 7) is not None) and orc.rel_l2(*outs) <= 1e-3
