@@ -91,10 +91,14 @@ class TriangleAttention(nn.Module):
             m = self._modules.get(name)
             if type(m) is not kind or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
                 return None
-            weights.append(m._parameters.get("weight"))
+            own = m._parameters
+            # (a forward of the instance's own, as wrappers put there; a weight or bias that is no parameter any more)
+            if "forward" in m.__dict__ or "weight" not in own or "bias" not in own:
+                return None
+            weights.append(own["weight"])
             if has_bias:
-                weights.append(m._parameters.get("bias"))
-            elif m._parameters.get("bias") is not None:
+                weights.append(own["bias"])
+            elif own["bias"] is not None:
                 return None
         norm = self._modules["layer_norm"]
         if norm.normalized_shape != (z.shape[-1],):

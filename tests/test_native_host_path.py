@@ -1,6 +1,6 @@
 """What the C++ host path has to leave to the Python path, and what attention() and the block then do there: a call whose
 operations something watches (tracing, dispatch modes, functorch), tensors with a tangent,
-tensor subclasses, sizes that are not built."""
+tensor subclasses, sizes that are not built, submodules that are not as the block made them."""
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
@@ -139,3 +139,47 @@ def test_a_call_draws_one_dropout_seed_whichever_path_takes_it(autocast):
     torch.randint(0, 2 ** 62, (1,))
     assert all(torch.equal(s, torch.get_rng_state()) for s in states)
     assert (blk._fused(z, None, 7) is not None) and orc.rel_l2(*outs) <= 1e-3
+
+
+def _own_forward(blk):
+    lin = blk.linear_v
+    lin.forward = lambda x: 2.0 * torch.nn.functional.linear(x, lin.weight)
+
+
+def _plain_bias(blk):
+    for lin in (blk.linear_g, blk.linear_o):
+        value = lin.bias.detach() + 1.0
+        del lin.bias
+        lin.bias = value
+
+
+def _bias_of_a_projection(blk):
+    lin = blk.linear_q
+    del lin.bias
+    lin.bias = torch.ones(lin.out_features, device=DEV)
+
+
+def _plain_weight(blk):
+    lin = blk.linear_b
+    value = 2.0 * lin.weight.detach()
+    del lin.weight
+    lin.weight = value
+
+
+def _buffer_bias(blk):
+    value = blk.linear_g.bias.detach() + 1.0
+    del blk.linear_g.bias
+    blk.linear_g.register_buffer("bias", value)
+
+
+@gpu
+@pytest.mark.parametrize("change", [_own_forward, _plain_bias, _bias_of_a_projection, _plain_weight, _buffer_bias])
+def test_changed_submodules_are_used_as_they_are(change):
+    blk, z = _block(), _pair(1)
+    sep = _separate(blk)
+    sep.load_state_dict(blk.state_dict())
+    with torch.no_grad():
+        before = blk(z)
+        change(blk)
+        change(sep)
+        assert torch.equal(blk(z), sep(z)) and orc.rel_l2(blk(z), before) > 1e-2
