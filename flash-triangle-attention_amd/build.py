@@ -2,7 +2,9 @@
 
     python flash-triangle-attention_amd/build.py [--force]
 
-hipcc cross-compiles without a GPU, so this runs anywhere the ROCm toolchain is installed.
+hipcc cross-compiles without a GPU, so this runs anywhere the ROCm toolchain is installed.  The extension module
+fta_native.so (the C++ host path from torch tensors) is built for the torch at hand; without torch the C library and its
+demo are built alone.
 """
 from __future__ import annotations
 
@@ -11,6 +13,11 @@ import subprocess
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
+if HERE not in sys.path:
+    sys.path.insert(0, HERE)
+
+import fta_lib  # noqa: E402
+
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "libfta.so")
@@ -34,24 +41,36 @@ FLAGS = [
 ]
 
 
+def torch_version() -> "str | None":
+    try:
+        import torch
+    except ImportError:
+        return None
+    return torch.__version__
+
+
 def needs_build() -> bool:
-    if not os.path.exists(LIB) or not os.path.exists(DEMO) or not os.path.exists(NATIVE):
+    version = torch_version()
+    built = [LIB, DEMO] + ([NATIVE] if version is not None else [])
+    if not all(os.path.exists(f) for f in built) or (version is not None and fta_lib.native_torch_version(NATIVE) != version):
         return True
-    t = min(os.path.getmtime(LIB), os.path.getmtime(NATIVE))
+    t = min(os.path.getmtime(f) for f in built)
     deps = [os.path.join(CSRC, f) for f in os.listdir(CSRC)] + [os.path.join(INCLUDE, "fta.h")]
     return any(os.path.getmtime(d) > t for d in deps)
 
 
-def native_commands(hipcc: str, obj: str) -> tuple[list, list]:
-    """Compile and link commands of the extension module (host code only)."""
+def native_commands(hipcc: str, obj: str) -> "tuple[list, list] | None":
+    """Compile and link commands of the extension module (host code only); None without torch."""
     import sysconfig
 
+    if torch_version() is None:
+        return None
     import torch
     root = os.path.dirname(torch.__file__)
     inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
            sysconfig.get_paths()["include"], os.path.join(os.path.dirname(os.path.dirname(hipcc)), "include"), INCLUDE]
     compile_cmd = [hipcc, "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=fta_native",
-                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-everything"]
+                   f'-DFTA_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-Wno-everything"]
     for d in inc:
         compile_cmd += ["-I", d]
     compile_cmd += ["-c", os.path.join(CSRC, NATIVE_SOURCE), "-o", obj]
@@ -73,8 +92,11 @@ def build(force: bool = True, verbose: bool = False) -> str:
         for c in cmds:
             print(" ".join(c))
     native_obj = os.path.join(OBJDIR, "fta_torch.o")
-    native_compile, native_link = native_commands(hipcc, native_obj)
-    cmds.append(native_compile)
+    native = native_commands(hipcc, native_obj)
+    if native is not None:
+        cmds.append(native[0])
+    else:
+        print("no torch: building libfta.so and the demo without fta_native.so", file=sys.stderr)
     procs = [subprocess.Popen(c, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True) for c in cmds]
     failed = False
     for pr in procs:
@@ -91,10 +113,11 @@ def build(force: bool = True, verbose: bool = False) -> str:
     if res.returncode != 0:
         sys.stderr.write(res.stdout + res.stderr)
         raise RuntimeError("hipcc failed linking libfta.so")
-    res = subprocess.run(native_link, capture_output=True, text=True)
-    if res.returncode != 0:
-        sys.stderr.write(res.stdout + res.stderr)
-        raise RuntimeError("linking fta_native.so failed")
+    if native is not None:
+        res = subprocess.run(native[1], capture_output=True, text=True)
+        if res.returncode != 0:
+            sys.stderr.write(res.stdout + res.stderr)
+            raise RuntimeError("linking fta_native.so failed")
     # the C-ABI demo: a plain C++ program (HIP runtime only) linked against the library next to it
     demo = [hipcc, "--offload-arch=gfx950", "-O2", "-std=c++17", "-Wno-unused-command-line-argument", "-I", INCLUDE,
             os.path.join(CSRC, DEMO_SOURCE), "-o", DEMO, "-L", HERE, "-lfta", "-Wl,-rpath,$ORIGIN"]

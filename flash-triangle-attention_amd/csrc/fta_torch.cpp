@@ -315,6 +315,7 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
 
 PYBIND11_MODULE(fta_native, m) {
   m.doc() = "C++ host path of attention() and TriangleAttention; None = not taken, use the Python path";
+  m.attr("built_for") = "fta_native built for torch " FTA_TORCH_VERSION;  // (read from the file before it is loaded, too)
   m.def("attention", &attention, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("b_pw"), py::arg("sm_scale"),
         py::arg("dropout_p") = 0.0, py::arg("seed") = 0, py::kw_only(), py::arg("globals"));
   m.def("block", &block);

@@ -144,7 +144,8 @@ _native = None
 
 def _load_native():
     global _native
-    _native = fta_lib.native().attention
+    mod = fta_lib.native()
+    _native = mod.attention if mod is not None else (lambda *args, **kwargs: None)
     return _native
 
 

@@ -86,6 +86,9 @@ class TriangleAttention(nn.Module):
         sizes, autocast, mixed types, hooked, parametrised or replaced submodules, a subclass."""
         if type(self) is not TriangleAttention or not z.is_cuda or _has_any_global_hook():
             return None
+        native = fta_lib.native()
+        if native is None:
+            return None
         weights = []
         for name, kind, has_bias in _SUBMODULES:
             m = self._modules.get(name)
@@ -106,8 +109,8 @@ class TriangleAttention(nn.Module):
         scope = _attention.forward.__globals__  # (the module that holds the PRECISE_BACKWARD switch)
         p = self.dropout_p if self.training else 0.0
         try:
-            return fta_lib.native().block(z, key_mask, weights, self.n_heads, self.c_hidden, self.starting, norm.eps, p,
-                                          seed if p > 0.0 else 0, scope)  # (no seed: one is drawn if the call is taken)
+            return native.block(z, key_mask, weights, self.n_heads, self.c_hidden, self.starting, norm.eps, p,
+                                seed if p > 0.0 else 0, scope)  # (no seed: one is drawn if the call is taken)
         except TypeError:  # (a seed beyond 63 bits, a mask that is no tensor)
             return None
 

@@ -1,4 +1,5 @@
-"""What the C++ host path has to leave to the Python path, and what attention() and the block then do there: a call whose
+"""What the C++ host path has to leave to the Python path, and what attention() and the block then do there (also
+where the module is missing or was built for another torch): a call whose
 operations something watches (tracing, dispatch modes, functorch), tensors with a tangent,
 tensor subclasses, sizes that are not built, submodules that are not as the block made them."""
 import pytest
@@ -183,3 +184,70 @@ def test_changed_submodules_are_used_as_they_are(change):
         change(blk)
         change(sep)
         assert torch.equal(blk(z), sep(z)) and orc.rel_l2(blk(z), before) > 1e-2
+
+
+def _native_file(kind, tmp_path):
+    import fta_lib
+    path = tmp_path / "fta_native.so"
+    if kind == "other torch":
+        data = open(fta_lib.NATIVE_PATH, "rb").read()
+        assert data.count(fta_lib._BUILT_FOR + torch.__version__.encode()) == 1
+        path.write_bytes(data.replace(fta_lib._BUILT_FOR, fta_lib._BUILT_FOR + b"9."))
+    elif kind == "not a library":
+        path.write_bytes(fta_lib._BUILT_FOR + torch.__version__.encode() + b"\0")
+    return str(path)
+
+
+@pytest.fixture(params=["missing", "other torch", "not a library"])
+def no_native(request, tmp_path, monkeypatch):
+    import fta_lib
+    import flash_tt_attn
+    monkeypatch.setattr(fta_lib, "NATIVE_PATH", _native_file(request.param, tmp_path))
+    monkeypatch.setattr(fta_lib, "_native", None)
+    monkeypatch.setattr(flash_tt_attn, "_native", None)
+    with pytest.warns(RuntimeWarning, match="Python path"):
+        assert fta_lib.native() is None
+
+
+def test_without_the_module_calls_take_the_python_path(no_native):
+    import warnings
+    import flash_tt_attn as fta
+    x = torch.zeros(1, 1, 1, 8, 32, dtype=torch.float16)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")  # (said once)
+        with pytest.raises(ValueError, match="no CPU path"):
+            fta.attention(x, x, x, torch.zeros(1, 1, 8, 8, dtype=torch.float16), 0.1)
+
+
+@gpu
+def test_without_the_module_the_results_are_the_same(no_native, monkeypatch):
+    import fta_lib
+    import flash_tt_attn as fta
+    x, dout, blk, z = _operands(1)[:4], _operands(1)[4], _block(), _pair(1)
+
+    def results():
+        q = x[0].clone().requires_grad_(True)
+        o = fta.attention(q, *x[1:], 0.3)
+        return o, *torch.autograd.grad(o, q, dout), blk(z)
+    slow = results()
+    monkeypatch.undo()
+    assert fta_lib.native() is not None
+    fast = results()
+    assert all(torch.equal(a, b) for a, b in zip(slow[:2], fast[:2])) and orc.rel_l2(slow[2], fast[2]) <= 1e-3
+
+
+def test_the_build_follows_the_torch_at_hand(monkeypatch):
+    import importlib.util
+    import os
+    import fta_lib
+    spec = importlib.util.spec_from_file_location("fta_build", os.path.join(fta_lib.HERE, "build.py"))
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    assert fta_lib.native_torch_version(build.NATIVE) == torch.__version__
+    before = build.needs_build()
+    monkeypatch.setattr(build, "torch_version", lambda: "9.9")
+    assert build.needs_build()  # the module there is for another one
+    monkeypatch.setattr(build, "torch_version", lambda: None)
+    assert build.native_commands("hipcc", "x.o") is None
+    monkeypatch.setattr(build, "NATIVE", "/nowhere/fta_native.so")
+    assert build.needs_build() <= before  # without torch its absence is no reason to build
