@@ -20,6 +20,8 @@
 // Bound: memory (eight tensors of 64 bytes per pair and head against some 130 vector instructions per 32 x 32 tile,
 // about half of the memory time at 128 keys).  Two workgroups of four waves share a CU, one's loads under the other's
 // products.  B4 H8 L128 D32 fp16: 80 us where the delta, dQ/dBias and dK/dV kernels took 14 + 70 + 51.
+#include <type_traits>
+
 #include "fta_kernels.h"
 #include "fta_common.h"
 
@@ -56,14 +58,18 @@ __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(D 
   fo.init(lane);
   fx.init(lane);
 
-  // stationary bias, in the order of the rounds: tile r holds keys of block (wave + r) % NT
+  // stationary bias, in the order of the rounds: tile r holds keys of block (wave + r) % NT.  The values are the forward's,
+  // of the kernel that made lse (hand-scheduled at D = 32 without dropout, else the general one): where every key of a
+  // query is masked the weights are differences to that very floor.
+  constexpr bool FWD1 = (D == 32 && !DROP);
+  typedef typename std::conditional<FWD1, F16, T>::type BT;
   uint32_t bias_reg[NT][8];
   float dbacc[NT][16];
   load_bias_tiles<NT, 1, true, true>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], wave * 32, p.L2, T::kNegInf2,
                                      reinterpret_cast<char*>(xchg + wave * 2 * XT), lane, [=](int c) { return (wave + c) % NT * 32; },
                                      [&](int r, int g, u32x2 v) {
-                                       bias_reg[r][2 * g] = v[0];
-                                       bias_reg[r][2 * g + 1] = v[1];
+                                       bias_reg[r][2 * g] = FWD1 ? fwd1_bias_pair<T>(v[0]) : T::finite2(v[0]);
+                                       bias_reg[r][2 * g + 1] = FWD1 ? fwd1_bias_pair<T>(v[1]) : T::finite2(v[1]);
                                      });
 #pragma unroll
   for (int r = 0; r < NT; ++r)
@@ -148,8 +154,8 @@ __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(D 
       for (int e = 0; e < 16; e += 2) {
         uint32_t& bb = bias_reg[r][e >> 1];
         asm volatile("" : "+v"(bb));  // (converted where it is used: kept in fp32 over the rows it would take twice the registers)
-        float p0 = exp2_fast(__builtin_fmaf(__builtin_fmaf(s[e], scale, T::lo(bb)), kLog2e, nl));
-        float p1 = exp2_fast(__builtin_fmaf(__builtin_fmaf(s[e + 1], scale, T::hi(bb)), kLog2e, nl));
+        float p0 = exp2_fast(__builtin_fmaf(__builtin_fmaf(s[e], scale, BT::lo(bb)), kLog2e, nl));
+        float p1 = exp2_fast(__builtin_fmaf(__builtin_fmaf(s[e + 1], scale, BT::hi(bb)), kLog2e, nl));
         float e0 = dp[e], e1 = dp[e + 1], w0 = p0, w1 = p1;
         if constexpr (DROP) {
           const bool k0 = keep_byte(p.drop, keep[e >> 2], e & 3), k1 = keep_byte(p.drop, keep[e >> 2], (e & 3) + 1);

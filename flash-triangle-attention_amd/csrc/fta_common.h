@@ -71,14 +71,18 @@ __device__ __forceinline__ uint32_t bias_log2_half2(uint32_t u) {
   return pack_rn(__builtin_fmaxf((float)h[0] * kLog2e, kBiasFloorLog2), __builtin_fmaxf((float)h[1] * kLog2e, kBiasFloorLog2));
 }
 
-// The forward adds the bias on the vector ALU, where -inf is harmless unless EVERY key a query has
-// seen so far is masked (the running maximum is then -inf and the exponent becomes inf - inf).
-// With -inf replaced by the lowest finite fp16 the masked keys still get weight exp(-65504 - m) = 0
-// as soon as one unmasked key has been seen, and a leading run of masked keys is rescaled away
-// like any other early partial sum.
+// The bias as it is added on the vector ALU (natural units), kept at or above kMaskedBias: -inf would be harmless there
+// unless EVERY key a query has seen so far is masked (the running maximum is then -inf and the exponent becomes
+// inf - inf).  At the floor a masked key still gets weight exp(-59904 - m) = 0 as soon as one unmasked key has been
+// seen, and a leading run of masked keys is rescaled away like any other early partial sum.  A query whose keys are ALL at
+// the floor attends by its scores alone (to their rounding beside the floor, 2^-8), as it would with a finite mask value:
+// the floor is one value, exact in fp16 and in bf16, for the forward and for every backward kernel, because the backward
+// forms its weights from the forward's logsumexp.  (bf16 had a floor of -2^30, beside which the rounding of the
+// exponent alone is 2^6: the weights of such a query came out of the backward wrong by up to 2^64.)
+constexpr float kMaskedBias = -59904.0f;
 __device__ __forceinline__ uint32_t finite_half2(uint32_t u) {
   half2_t h = __builtin_bit_cast(half2_t, u);
-  const half2_t lowest = {(half_t)-65504.0f, (half_t)-65504.0f};
+  const half2_t lowest = {(half_t)kMaskedBias, (half_t)kMaskedBias};
   h = __builtin_elementwise_max(h, lowest);
   return __builtin_bit_cast(uint32_t, h);
 }
@@ -163,11 +167,7 @@ struct F16 {
   static __device__ __forceinline__ half8_t scale8(half8_t x, float f) { return scale_half8(x, f); }
   static __device__ __forceinline__ uint32_t bias_log2(uint32_t u) { return bias_log2_half2(u); }  // -> fp16 pair
   // The bias pair as it is (natural units: nothing is rounded), kept above the floor that stands for -inf.
-  static __device__ __forceinline__ uint32_t bias_nat(uint32_t u) {
-    half2_t h = __builtin_bit_cast(half2_t, u);
-    const half2_t floor2 = {(half_t)kBiasFloorLog2, (half_t)kBiasFloorLog2};
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(h, floor2));
-  }
+  static __device__ __forceinline__ uint32_t bias_nat(uint32_t u) { return finite_half2(u); }
   // The product kept to 22 bits: hi = the rounded product, lo = what the rounding dropped, itself
   // rounded.  An MFMA over hi plus one over lo gives the scores the precision of an fp32 product
   // (the precise mode, where scores of several tens would feel the 11-bit rounding of hi alone).
@@ -225,13 +225,8 @@ struct BF16 {
     const bf16x2_t ones = {(__bf16)1.0f, (__bf16)1.0f};
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, u), ones, acc, false);
   }
-  // The floor of a bf16 bias is -2^30.  While every key seen so far sits at the floor the forward
-  // takes exp2(s * log2e - fl(m * log2e)) with s = m: what is left is the rounding error of the second
-  // product, half an ulp of 1.5e9 = 64 at most, so those weights stay below 2^64 and are rescaled to
-  // nothing by the first real key.  (A floor of -1e30 left an error of 1e22 there: inf, then NaN.)
-  static constexpr float kFloor = -1073741824.0f;
   static __device__ __forceinline__ uint32_t finite2(uint32_t u) {
-    return pack(__builtin_fmaxf(lo(u), kFloor), __builtin_fmaxf(hi(u), kFloor));
+    return pack(__builtin_fmaxf(lo(u), kMaskedBias), __builtin_fmaxf(hi(u), kMaskedBias));
   }
   // Eight bf16 times an fp32 factor, rounded to nearest even.  The results feed MFMAs written as
   // assembly: the closing statement makes the values complete there and puts the two idle issue slots
@@ -282,6 +277,29 @@ struct BF16 {
   static constexpr float kOneHotInv = 128.0f;
   static __device__ __forceinline__ uint32_t add2(uint32_t a, uint32_t b) { return pack(lo(a) + lo(b), hi(a) + hi(b)); }
 };
+
+// The bias as the hand-scheduled forward kernels take it, whatever the element type: an fp16 pair at or above
+// kMaskedBias.  (bf16 biases beyond 65504 are held there: the general kernels take them as they are.)
+template <class T>
+__device__ __forceinline__ uint32_t fwd1_bias_pair(uint32_t u) {
+  if constexpr (T::is_bf16) {
+    // (in place, with one temporary: 128 of these run with the register file full)
+    uint32_t t;
+    asm volatile(
+        "v_lshlrev_b32 %1, 16, %0\n\t"
+        "v_and_b32 %0, 0xffff0000, %0\n\t"
+        "v_max_f32 %1, %2, %1\n\t"
+        "v_max_f32 %0, %2, %0\n\t"
+        "v_min_f32 %1, %3, %1\n\t"
+        "v_min_f32 %0, %3, %0\n\t"
+        "v_cvt_pk_f16_f32 %0, %1, %0"
+        : "+v"(u), "=&v"(t)
+        : "s"(kMaskedBias), "s"(65504.0f));
+    return u;
+  } else {
+    return finite_half2(u);
+  }
+}
 
 // ---- dropout ---------------------------------------------------------------------------------------
 // Counter-based random bytes: a function of (seed, row, query, key) alone, so that the forward and

@@ -78,27 +78,4 @@ __device__ __forceinline__ void fwd1_scaled_pair(float& x0, float& x1, float s0,
   }
 }
 
-// The bias as the vector ALU takes it: an fp16 pair, finite (a masked key keeps the lowest fp16 value
-// and gets weight exactly 0 once the reference has seen a real key).
-template <class T>
-__device__ __forceinline__ uint32_t fwd1_bias_pair(uint32_t u) {
-  if constexpr (T::is_bf16) {
-    // (in place, with one temporary: 128 of these run with the register file full)
-    uint32_t t;
-    asm volatile(
-        "v_lshlrev_b32 %1, 16, %0\n\t"
-        "v_and_b32 %0, 0xffff0000, %0\n\t"
-        "v_max_f32 %1, %2, %1\n\t"
-        "v_max_f32 %0, %2, %0\n\t"
-        "v_min_f32 %1, %3, %1\n\t"
-        "v_min_f32 %0, %3, %0\n\t"
-        "v_cvt_pk_f16_f32 %0, %1, %0"
-        : "+v"(u), "=&v"(t)
-        : "s"(-65504.0f), "s"(65504.0f));
-    return u;
-  } else {
-    return finite_half2(u);
-  }
-}
-
 }  // namespace fta

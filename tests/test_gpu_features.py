@@ -134,6 +134,51 @@ def test_masks_that_cover_all_keys_a_wave_has_seen(dtype, B, H, L1, L2, D, lo, h
     _compare(got, _oracle(q, k, v, b, sm, do), dtype, f"mask {lo}..{hi} L{L2} D{D}")
 
 
+_ALL_MASKED = [
+    # one-kernel backward
+    (64, 32, "plain"), (128, 32, "plain"), (128, 64, "plain"), (128, 32, "dropout"), (128, 64, "dropout"), (64, 32, "precise"), (128, 64, "precise"),
+    # general backward kernels
+    (256, 32, "dropout"), (512, 32, "dropout"), (1024, 32, "dropout"), (256, 64, "dropout"), (512, 64, "precise"),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("mask", ["-inf", "lowest"])
+@pytest.mark.parametrize("L2,D,mode", _ALL_MASKED)
+def test_queries_whose_keys_are_all_masked_attend_by_their_scores(L2, D, mode, mask, dtype):
+    """With the same mask value on every key of a query (-inf, or the type's lowest) its softmax is that of the scores
+    alone, in the output and in every gradient; other queries have the same value on some keys, which get weight 0.
+    The weights of such a query are differences beside the floor that stands for the mask, where fp32 holds a
+    score to 2^-9 and the logsumexp, a base-2 logarithm, to 2^-8: 5e-3 of a weight at most, half the tolerance."""
+    import flash_tt_attn as fta
+    if mode == "precise" and dtype == torch.bfloat16:
+        pytest.skip("a mode of fp16")
+    B, H, L1, sm = 1, 2, 3, 1.0 / math.sqrt(D)
+    rows = [0, 7, L2 - 1]
+    q, k, v, b, do = _inputs(B, H, L1, L2, D, 3, dtype)
+    low = float("-inf") if mask == "-inf" else torch.finfo(dtype).min
+    b[..., L2 // 2:L2 // 2 + 5] = low
+    ref_b = b.float()
+    ref_b[..., L2 // 2:L2 // 2 + 5] = float("-inf")
+    b[:, :, rows] = low
+    ref_b[:, :, rows] = 0.0
+    extra, kw, scale = (), {}, 1.0
+    if mode == "dropout":
+        keep, scale = dm.keep_mask(1234, 0.25, B, H, L1, L2)
+        extra, kw = (0.25, 1234), dict(keep=torch.from_numpy(keep).to(DEV), keep_scale=scale)
+    fta.PRECISE_BACKWARD = mode == "precise"
+    try:
+        got = _run(q, k, v, b, sm, do, *extra)
+    finally:
+        fta.PRECISE_BACKWARD = False
+    ref = _oracle(q, k, v, ref_b, sm, do, **kw)
+    got["o"], ref["o"] = (got["o"].detach().float() / scale).to(dtype), ref["o"] / scale  # (as the other dropout tests)
+    _compare(got, ref, dtype, f"all masked L{L2} D{D} {mode}")
+    for n in ("o", "dq", "db"):  # the masked queries by themselves
+        e = orc.rel_l2(got[n][..., rows, :], ref[n][..., rows, :])
+        assert e <= TOL[dtype][1], f"{n} of the masked queries: rel-L2 {e}"
+
+
 @pytest.fixture
 def general_kernels():
     """Selects the general backward kernels where the pipelined ones would run (library test hook)."""
