@@ -381,7 +381,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
     }
     // (a query beyond L2 gets the constant that makes its weights exactly 0 in both backward kernels)
     // (lse is stored as a base-2 logarithm)
-    const float nl = qvalid ? (NAT ? -lse_n * 0.6931471805599453f : -lse_n) : kBiasFloorLog2, nd = -sum_both_halves(dpart);
+    const float nl = qvalid ? (NAT ? -lse_n * 0.6931471805599453f : folded_lse(lse_n)) : kBiasFloorLog2, nd = -sum_both_halves(dpart);
     const uint32_t ws = split_2048(nl), wd = split_2048(nd);
     // the dK/dV kernel takes the constants from here (the look-ahead past the chunk's last row
     // works on the last row again and stores the same values once more)

@@ -87,6 +87,14 @@ __device__ __forceinline__ uint32_t finite_half2(uint32_t u) {
   return __builtin_bit_cast(uint32_t, h);
 }
 
+// -lse for the kernels that add bias * log2(e) through the matrix core.  A logsumexp below the floor of that bias belongs to
+// a query that has no key above it: forward and backward then hold the masked keys at different values, -59904 log2(e)
+// and -60000, and the difference goes into the constant, so that the weights are again those of the scores alone
+// (without it the exponent is +26423 and the gradients inf and NaN).  Where all of a query's biases lie between
+// the two floors, -59904 and -41588, the weights come out as 0.
+constexpr float kMaskedShiftLog2 = (float)(-(double)kMaskedBias * 1.4426950408889634 + (double)kBiasFloorLog2);
+__device__ __forceinline__ float folded_lse(float lse) { return lse < kBiasFloorLog2 ? -kMaskedShiftLog2 - lse : -lse; }
+
 // Eight halfs times an fp32 factor, rounded to nearest: the mixed-precision FMA converts, multiplies
 // and rounds in one instruction per element (the product is rounded once, to fp16).  The results
 // usually feed an MFMA, which may not read a register in the two issue slots after a vector-ALU

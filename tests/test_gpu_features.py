@@ -137,6 +137,9 @@ def test_masks_that_cover_all_keys_a_wave_has_seen(dtype, B, H, L1, L2, D, lo, h
 _ALL_MASKED = [
     # one-kernel backward
     (64, 32, "plain"), (128, 32, "plain"), (128, 64, "plain"), (128, 32, "dropout"), (128, 64, "dropout"), (64, 32, "precise"), (128, 64, "precise"),
+    # hand-scheduled backward (one and several key ranges; the precise instances in natural units)
+    (256, 32, "plain"), (384, 32, "plain"), (512, 32, "plain"), (1024, 32, "plain"), (256, 64, "plain"), (384, 64, "plain"), (512, 64, "plain"),
+    (256, 32, "precise"), (512, 32, "precise"),
     # general backward kernels
     (256, 32, "dropout"), (512, 32, "dropout"), (1024, 32, "dropout"), (256, 64, "dropout"), (512, 64, "precise"),
 ]
