@@ -24,7 +24,7 @@ LdsLimit g_lds_limit[kMaxKernels];  // per kernel: the limit already set on each
 int g_lds_kernels = 0;
 }  // namespace
 
-int forced_general_mask() { return g_forced_general.load(std::memory_order_relaxed); }
+bool forced_general() { return g_forced_general.load(std::memory_order_relaxed) != 0; }
 
 hipError_t ensure_dynamic_lds(const void* kern, size_t smem) {
   if (smem <= 48 * 1024) return hipSuccess;  // within every kernel's default limit
@@ -152,7 +152,7 @@ const fta::FwdPlan& cached_plan_fwd(int B, int H, int L1, int L2, int D, int fea
 const fta::BwdPlan& cached_plan_bwd(int B, int H, int L1, int L2, int D, int feat = 0) {
   thread_local PlanKey key{-1, 0, 0, 0, 0, 0};
   thread_local fta::BwdPlan plan;
-  const PlanKey k{B, H, L1, L2, D, fta::forced_general_mask() | (feat * 4)};
+  const PlanKey k{B, H, L1, L2, D, (fta::forced_general() ? 1 : 0) | (feat * 4)};
   if (!(key == k)) {
     const int lp = len_supported(L2, D, feat) ? padded_len_bwd(L2, D, feat) : 0;
     plan = (lp != 0) ? fta::plan_bwd(B, H, L1, lp, D, L2, feat) : fta::BwdPlan{};
@@ -199,7 +199,7 @@ int parse_options(const fta_options* o, Opts& out) {
 // the feature instances (level 1).
 bool both_hand_scheduled(int B, int H, int L1, int L2, int D) {
   const fta::BwdPlan& pl = cached_plan_bwd(B, H, L1, L2, D, 0);
-  return pl.valid && pl.use_dq1 && pl.use_dkdv1;
+  return pl.valid && pl.use_hand;
 }
 bool bf16_fast_plan(const Opts& opt, int B, int H, int L1, int L2, int D) {
   return opt.bf16_plain && both_hand_scheduled(B, H, L1, L2, D);
@@ -365,14 +365,14 @@ int fta_describe_plan_ex(int B, int H, int L1, int L2, int D, float sm_scale, co
   if (b.use_short) {
     snprintf(dq, sizeof dq, "fta_bwd_short_kernel<%d,%d> launches=1 grid=%ld block=%d lds=%zu", D, b.sh.NT, bh * b.sh.nchunks, b.sh.threads, b.sh.smem);
     memcpy(dkdv, dq, sizeof dkdv);
-  } else if (b.use_dq1)
+  } else if (b.use_hand)
     snprintf(dq, sizeof dq, "fta_bwd_dq1_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, b.dq1.SK, b.dq1.nlaunch,
              bh * b.dq1.nqg * b.dq1.nchunks, b.dq1.threads, b.dq1.smem);
   else
     snprintf(dq, sizeof dq, "fta_bwd_dq_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, (D == 32 && b.NKT == 4) ? 2 : 1, b.nlaunch,
              bh * b.nqg * b.nchunks, b.threads, b.smem);
   if (b.use_short) {
-  } else if (b.use_dkdv1)
+  } else if (b.use_hand)
     snprintf(dkdv, sizeof dkdv, "fta_bwd_dkdv1_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, b.dkdv1.NJT,
              b.dkdv1.nlaunch, bh * b.dkdv1.nkg * b.dkdv1.nchunks, b.dkdv1.threads, b.dkdv1.smem);
   else
@@ -387,7 +387,7 @@ int fta_describe_plan_ex(int B, int H, int L1, int L2, int D, float sm_scale, co
                          (f.fwd1 == 1 && opt.drop.thresh == 0) ? "fta_fwd1_kernel" : (f.fwd1 == 2 && opt.drop.thresh == 0) ? "fta_fwd2_kernel" : "fta_fwd_kernel", D, f.NKT, f.KT,
                          bh * f.nqg * f.nchunks, f.threads, f.smem, f.L2p, dq, dkdv, b.delta_bytes, b.partial_bytes, b.aux_bytes, b.L2p, tn,
                          opt.drop.thresh != 0 ? 1 : 0, level != 0 ? 1 : 0,
-                         ((level == 0 && opt.bf16_plain && b.use_dq1 && b.use_dkdv1 && fta::bf16_scale_needs_split(sm_scale)) ||
+                         ((level == 0 && opt.bf16_plain && b.use_hand && fta::bf16_scale_needs_split(sm_scale)) ||
                           (level == 0 && opt.f16_precise)) ? 1 : 0,
                          (level == 0 && opt.f16_precise) ? 1 : 0);
   return (n < 0 || (size_t)n >= out_bytes) ? FTA_ERR_WORKSPACE : FTA_OK;

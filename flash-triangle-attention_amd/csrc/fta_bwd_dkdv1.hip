@@ -676,7 +676,6 @@ bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl) {
   if (D != 32 && D != 64) return false;
   if (L2 % 128 != 0 || L2 < 256 || L2 / 128 > 4 * kMaxRanges) return false;
   if (D == 64 && (L2 + 255) / 256 > kMaxRanges) return false;
-  if (forced_general_mask() & 2) return false;  // the general kernel was asked for (tests)
   pl.nlaunch = dkdv1_ranges(L2, D, pl.range);
   pl.JR = pl.range[0];
   pl.NJT = pl.JR / 32;

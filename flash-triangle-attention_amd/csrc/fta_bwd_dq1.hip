@@ -862,7 +862,6 @@ bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl) {
   if (D != 32 && D != 64) return false;
   if (L2 % 128 != 0 || L2 < 256) return false;
   if (L2 / 128 > 4 * kMaxRanges) return false;
-  if (forced_general_mask() & 1) return false;  // the general kernel was asked for (tests)
   pl.nlaunch = dq1_ranges(L2, D, pl.range);
   const int nqb = L2 / 32;
   pl.threads = 256;

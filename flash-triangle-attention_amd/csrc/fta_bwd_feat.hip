@@ -1,8 +1,6 @@
-// Backward: the kernel instances for bf16 inputs, for dropout (fp16 and bf16) and for the fp16
-// "precise" mode (scale, bias and row constants in fp32 on the vector ALU instead of fp16 roundings
-// on their way into the matrix core).  Same four stages
-// as launch_bwd; the row constants and the bias are applied on the vector ALU (no MFMA folding), the
-// tail handling is always compiled in, and dK/dV has 64 or 32 queries per staged tile (plan_bwd knows).
+// Backward: the instances of the general kernels (fta_bwd_kernels.h).  They run for dropout, for bf16 inputs and the precise
+// mode of fp16 where the hand-scheduled kernels have no instances (plan_bwd knows), and in tests; dK/dV has 64
+// queries per staged tile, or 32 (D = 64).
 //
 // Dropout is bound by the vector ALU (the mask alone is two generator calls and 16 compares per tile and lane), so what
 // counts is instructions per score and that all four SIMDs of a CU have two waves.  B1 H4 L300 D32 bf16, dropout 0.25:
@@ -19,12 +17,11 @@ template <class T, bool DROP>
 static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t st, hipEvent_t* ev) {
   auto mark = [&](int i) { if (ev != nullptr) (void)hipEventRecord(ev[i], st); };
   hipError_t e = hipSuccess;
-  p.aug_cinv = 0.f;
-  {  // 0. delta and the raw {lse, delta} pairs
+  {  // 0. delta and the {lse, delta} pairs
     const int64_t nthr = (int64_t)p.B * p.H * p.L1 * p.L2p * (D / 8);
     dim3 grid((unsigned)((nthr + 255) / 256)), block(256);
-    if (D == 32) hipLaunchKernelGGL((fta_bwd_delta_kernel<T, 32, true>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((fta_bwd_delta_kernel<T, 64, true>), grid, block, 0, st, p);
+    if (D == 32) hipLaunchKernelGGL((fta_bwd_delta_kernel<T, 32>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((fta_bwd_delta_kernel<T, 64>), grid, block, 0, st, p);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   mark(1);
@@ -36,11 +33,11 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
       if (pl.NKT == 3) {  // key ranges of 384 keys with dropout: fixed geometry
         if constexpr (DROP)
           if (D == 32 && pl.threads == 512 && pl.SK == 4 && pl.ring == dq_ring(32, 3, 1, 4).r && pl.nb == dq_ring(32, 3, 1, 4).nb)
-            e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 0, 512, true, 3, 4>, p, grid, block, pl.smem, st);
+            e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 3, 4>, p, grid, block, pl.smem, st);
       } else if (D == 32) {
-        e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2, 0, 512, true>, p, grid, block, pl.smem, st);
+        e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2>, p, grid, block, pl.smem, st);
       } else {
-        e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 64, 1, 0, 512, true>, p, grid, block, pl.smem, st);
+        e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 64, 1>, p, grid, block, pl.smem, st);
       }
       if (e != hipSuccess) return e;
     }
@@ -54,16 +51,16 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
       e = hipErrorInvalidConfiguration;
 #define FTA_DKDV_FEAT_CASE(DD, NN, JJ) \
   if (e == hipErrorInvalidConfiguration && D == DD && pl.NJT == NN && pl.JT == JJ) \
-    e = launch_kernel(fta_bwd_dkdv_kernel<T, false, DROP, DD, NN, JJ, true>, p, grid, block, pl.smem2, st);
+    e = launch_kernel(fta_bwd_dkdv_kernel<T, DROP, DD, NN, JJ>, p, grid, block, pl.smem2, st);
       if constexpr (DROP) {  // fixed geometry: query ranges of 256, 384, 512 and 1024 queries
 #define FTA_DKDV_FIX_CASE(NN, SS)                                                                                        \
   if (D == 32 && pl.threads2 == 512 && pl.NJT == NN && pl.JT == 64 && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, 64, SS).r &&  \
       pl.nb2 == dkdv_ring(32, NN, 64, SS).nb)                                                                            \
-    e = launch_kernel(fta_bwd_dkdv_kernel<T, false, true, 32, NN, 64, true, SS>, p, grid, block, pl.smem2, st);
+    e = launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, NN, 64, SS>, p, grid, block, pl.smem2, st);
         FTA_DKDV_FIX_CASE(6, 2) FTA_DKDV_FIX_CASE(8, 1) FTA_DKDV_FIX_CASE(8, 2) FTA_DKDV_FIX_CASE(8, 4)
 #undef FTA_DKDV_FIX_CASE
       }
-      FTA_DKDV_FEAT_CASE(32, 8, 64) FTA_DKDV_FEAT_CASE(32, 4, 64) FTA_DKDV_FEAT_CASE(32, 8, 32) FTA_DKDV_FEAT_CASE(32, 4, 32)
+      FTA_DKDV_FEAT_CASE(32, 8, 64) FTA_DKDV_FEAT_CASE(32, 4, 64)
       FTA_DKDV_FEAT_CASE(64, 4, 64) FTA_DKDV_FEAT_CASE(64, 4, 32)
 #undef FTA_DKDV_FEAT_CASE
       if (e != hipSuccess) return e;
@@ -71,12 +68,7 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
     p.jr0 = 0;
   }
   mark(3);
-  {  // 3. dBias: sum the chunk partials
-    const int64_t total4 = (int64_t)p.B * p.H * p.L2 * ((p.L2 + 3) / 4);
-    dim3 grid((unsigned)((total4 + 255) / 256)), block(256);
-    hipLaunchKernelGGL(fta_dbias_reduce_kernel<T>, grid, block, 0, st, p);
-    e = hipGetLastError();
-  }
+  e = launch_dbias_reduce(p, T::is_bf16 ? kBF16 : kF16, st);  // 3. sums the chunk partials
   mark(4);
   return e;
 }

@@ -4,6 +4,9 @@
 //     delta = rowsum(O*dO)                       dP = dO V^T         dS = P*(dP - delta)
 //     dQ = sm_scale * dS K     dK = sm_scale * dS^T Q     dV = P^T dO     dBias = sum_i dS
 //
+// The general kernels: they run for dropout, for bf16 tensors and the precise mode of fp16 where the hand-scheduled ones
+// (fta_bwd_dq1.hip, fta_bwd_dkdv1.hip) have no instances, and in tests.  Scale, bias and row constants are applied on the
+// vector ALU in fp32, and rows of any length are masked.
 // Four launches (the same bias-stationary idea as the forward kernel, one per orientation):
 //   0. fta_bwd_delta_kernel -- delta = rowsum(O*dO), fp32 (upstream: _attn_bwd_preprocess).
 //   1. fta_bwd_dq_kernel   -- queries are accumulator COLUMNS (one query per lane).  A wave owns
@@ -27,12 +30,10 @@
 namespace fta {
 
 // ------------------------------------------------------------------------------------------------
-// 0. delta[b,h,i,j] = sum_d O*dO.  D/8 lanes per row, one 16-byte chunk each.  Also packs the
-//    per-query constants that the later kernels fold into their MFMAs (p.aux).
+// 0. delta[b,h,i,j] = sum_d O*dO.  D/8 lanes per row, one 16-byte chunk each.  Also pairs it with lse for
+//    the dK/dV kernel (p.aux).
 // ------------------------------------------------------------------------------------------------
-// RAW: aux gets the plain fp32 pair {lse, delta} per query (what the kernels that subtract the row
-// constants on the vector ALU read) instead of the fp16 splits that the MFMA folding takes.
-template <class T, int D, bool RAW>
+template <class T, int D>
 __global__ void __launch_bounds__(256) fta_bwd_delta_kernel(const BwdParams p) {
   constexpr int CPR = D / 8;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -61,37 +62,27 @@ __global__ void __launch_bounds__(256) fta_bwd_delta_kernel(const BwdParams p) {
   for (int m = 1; m < CPR; m <<= 1) d += __shfl_xor(d, m);
   if (row < nrow && col == 0) {
     p.delta[row] = d;
-    // the folded per-query constants of the dK/dV kernel: fp16 (hi, lo) splits of -lse (log2 domain)
-    // and -delta, see split_2048().  A query beyond the row's true length gets -lse = kBiasFloorLog2:
-    // its P is exactly 0, so the rows staged for it (copies of the last real query) add nothing to dK, dV.
-    // Dropout's factor c = 1/(1 - p) (1 without) goes into the raw pair: with P' = c P = exp(t - (lse - log c)), a kept
+    // The row constants of the dK/dV kernel, {lse, delta} in fp32.  A query beyond the row's true length gets
+    // -kBiasFloorLog2 for lse: its P is exactly 0, so the rows staged for it (copies of the last real query) add nothing to
+    // dK, dV.  Dropout's factor c = 1/(1 - p) (1 without) goes into the pair: with P' = c P = exp(t - (lse - log c)), a kept
     // weight is P' and dS = P' (mask dP - delta / c), so that neither takes a multiplication per score.
-    if constexpr (RAW)
-      *reinterpret_cast<float2*>(p.aux + row * 2) = float2{(real ? p.lse[lrow] : -kBiasFloorLog2) - __builtin_amdgcn_logf(p.drop.scale), d / p.drop.scale};
-    else
-      *reinterpret_cast<u32x2*>(p.aux + row * 2) = u32x2{split_2048(real ? -p.lse[lrow] : kBiasFloorLog2), split_2048(-d)};
+    *reinterpret_cast<float2*>(p.aux + row * 2) = float2{(real ? p.lse[lrow] : -kBiasFloorLog2) - __builtin_amdgcn_logf(p.drop.scale), d / p.drop.scale};
   }
 }
 
 // ------------------------------------------------------------------------------------------------
 // 1. dQ + dBias partials
 // ------------------------------------------------------------------------------------------------
-template <class T, bool DROP, int D, int G1, int AUGC, int MAXT, bool TAIL, int NKT = 4, int SKC = 0>
-__global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
-  // T: element type.  The MFMA folding of the row constants and of the pre-scaled bias is an fp16
-  // device; bf16 inputs and DROP (whose mask sits between dP and the subtraction of delta) use AUGC = 0.
-  static_assert(AUGC == 0 || (!T::is_bf16 && !DROP), "folded constants: fp16 without dropout only");
-  // TAIL: the row's true length is not the tiled length (separate instances, so that the others pay
-  // nothing for the clamped copies and predicated stores)
-  // AUGC: which per-query constants are folded into the MFMAs here: 0 none, 1 -delta, 2 -delta and -lse
-  constexpr bool AUG = (AUGC == 2);
-  // SKC: the number of slabs where it is known at compile time (eight waves, TAIL): the geometry is then constant, every
+template <class T, bool DROP, int D, int G1, int NKT = 4, int SKC = 0>
+__global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
+  // T: element type.
+  // SKC: the number of slabs where it is known at compile time (eight waves): the geometry is then constant, every
   // wave issues the same number of copies per stage, and their offsets are formed from two registers.  With the geometry
   // in kernel arguments a third of the instructions per tile moved or made scalars (slabs of 96 keys, B1 H4 L300 with
   // dropout: 162 against 118 us).  Slabs of 128 keys have no registers for it: 70 spilled, 2.41 against 2.51 ms a training
   // pass at B1 H8 L512, so those keep the run-time geometry.
   constexpr bool FIX = (SKC != 0);
-  static_assert(!FIX || (TAIL && D == 32), "fixed geometry");
+  static_assert(!FIX || D == 32, "fixed geometry");
   // NKT: 32-key tiles per wave slab (128 keys; with dropout also 96, where that makes four slabs of a key range)
   constexpr int STEPS = NKT / G1;   // stages per row (>= 2: the LDS reduction buffer relies on it)
   constexpr int KS = D / 16;
@@ -142,18 +133,9 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
     for (int tt = 0; tt < NKT; ++tt) {
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg) {
-        u32x2 v = TAIL ? load_bias4(bbh, p.bs[2], q0 + l32, key0 + 4 * hh + tt * 32 + rg * 8, p.L2, T::kNegInf2)
-                       : *reinterpret_cast<const u32x2*>(bbh + (int64_t)(q0 + l32) * p.bs[2] + key0 + 4 * hh + tt * 32 + rg * 8);
-        if (AUG) {  // exponent is taken in base 2: keep bias * log2(e)
-          v[0] = bias_log2_half2(v[0]);
-          v[1] = bias_log2_half2(v[1]);
-        }
-        else {  // (added on the vector ALU: -inf is fine there, but keep it finite like the forward does)
-          v[0] = T::finite2(v[0]);
-          v[1] = T::finite2(v[1]);
-        }
-        bias_reg[tt][2 * rg] = v[0];
-        bias_reg[tt][2 * rg + 1] = v[1];
+        const u32x2 v = load_bias4(bbh, p.bs[2], q0 + l32, key0 + 4 * hh + tt * 32 + rg * 8, p.L2, T::kNegInf2);
+        bias_reg[tt][2 * rg] = T::finite2(v[0]);
+        bias_reg[tt][2 * rg + 1] = T::finite2(v[1]);
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) dbacc[tt][r] = 0.f;
@@ -162,10 +144,7 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
 
   // K/V staging: asynchronous global -> LDS copies into a ring of stage buffers
   const int nstage = nrows * STEPS;
-  DmaPlan<2> plk, plv;
-  dma_plan<D, 2>(plk, stage_rows, G1 * 32, NKT * 32, p.ks[3], wave, lane, nwaves);
-  dma_plan<D, 2>(plv, stage_rows, G1 * 32, NKT * 32, p.vs[3], wave, lane, nwaves);
-  const int ndma = plk.n + plv.n;  // K/V copies this wave issues per stage
+  const int ndma = 2 * dma_rows_count(stage_rows, D, wave, nwaves);  // K/V copies this wave issues per stage
   const int nqdma = 2 * dma_rows_count(QR, D, wave, nwaves);  // extra copies in a row's first stage
   const uint32_t lds0 = lds_addr_of(smem);
   const uint32_t ldsq = lds_addr_of(qtiles);
@@ -177,33 +156,22 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   const half_t* vcur = vbase + (int64_t)i0 * p.vs[2] + (int64_t)(FIX ? 0 : p.kr0) * p.vs[3];
   const half_t* qcur = qbase + (int64_t)i0 * p.qs[2] + (int64_t)(FIX ? 0 : qg * QB * 32) * p.qs[3];
   const half_t* docur = dobase + (int64_t)i0 * p.dos[2] + (int64_t)(FIX ? 0 : qg * QB * 32) * p.dos[3];
-  const int64_t kstep = (int64_t)(G1 * 32) * p.ks[3], vstep = (int64_t)(G1 * 32) * p.vs[3];
   // (a row length that is not a multiple of the tile: rows beyond it are copies of the last real
   // key or query; such keys are masked through the bias, such queries are never stored)
-  constexpr bool tail = TAIL;
-  const int last = TAIL ? p.L2 - 1 : 0x7fffffff;
+  const int last = p.L2 - 1;
   auto stage = [&](int slot) {
     const uint32_t dst = lds0 + (uint32_t)(slot * buf_halfs) * 2u;
     const uint32_t qd = ldsq + (uint32_t)((cur_ir % NB) * 2 * QR * D) * 2u;
-    if constexpr (!tail) {
-      dma_issue(plk, kcur + cur_t * kstep, dst);
-      dma_issue(plv, vcur + cur_t * vstep, dst + (uint32_t)(stage_rows * D) * 2u);
-      if (cur_t == 0) {
-        dma_rows<D>(qcur, p.qs[3], QR, qd, wave, lane, nwaves);
-        dma_rows<D>(docur, p.dos[3], QR, qd + (uint32_t)(QR * D) * 2u, wave, lane, nwaves);
-      }
-    } else {
-      // (kcur and vcur point at key kr0 of the row, qcur and docur at the workgroup's first query:
-      // the clamped copies count rows from the start of the row)
-      dma_tile_clamped<D>(kcur - (int64_t)p.kr0 * p.ks[3], p.ks[3], stage_rows, G1 * 32, NKT * 32, p.kr0 + cur_t * (G1 * 32), last, dst,
-                          wave, lane, nwaves);
-      dma_tile_clamped<D>(vcur - (int64_t)p.kr0 * p.vs[3], p.vs[3], stage_rows, G1 * 32, NKT * 32, p.kr0 + cur_t * (G1 * 32), last,
-                          dst + (uint32_t)(stage_rows * D) * 2u, wave, lane, nwaves);
-      if (cur_t == 0) {
-        dma_tile_clamped<D>(qcur - (int64_t)(qg * QR) * p.qs[3], p.qs[3], QR, QR, 0, qg * QR, last, qd, wave, lane, nwaves);
-        dma_tile_clamped<D>(docur - (int64_t)(qg * QR) * p.dos[3], p.dos[3], QR, QR, 0, qg * QR, last,
-                            qd + (uint32_t)(QR * D) * 2u, wave, lane, nwaves);
-      }
+    // (kcur and vcur point at key kr0 of the row, qcur and docur at the workgroup's first query:
+    // the clamped copies count rows from the start of the row)
+    dma_tile_clamped<D>(kcur - (int64_t)p.kr0 * p.ks[3], p.ks[3], stage_rows, G1 * 32, NKT * 32, p.kr0 + cur_t * (G1 * 32), last, dst,
+                        wave, lane, nwaves);
+    dma_tile_clamped<D>(vcur - (int64_t)p.kr0 * p.vs[3], p.vs[3], stage_rows, G1 * 32, NKT * 32, p.kr0 + cur_t * (G1 * 32), last,
+                        dst + (uint32_t)(stage_rows * D) * 2u, wave, lane, nwaves);
+    if (cur_t == 0) {
+      dma_tile_clamped<D>(qcur - (int64_t)(qg * QR) * p.qs[3], p.qs[3], QR, QR, 0, qg * QR, last, qd, wave, lane, nwaves);
+      dma_tile_clamped<D>(docur - (int64_t)(qg * QR) * p.dos[3], p.dos[3], QR, QR, 0, qg * QR, last,
+                          qd + (uint32_t)(QR * D) * 2u, wave, lane, nwaves);
     }
     if (++cur_t == STEPS) {
       cur_t = 0;
@@ -268,7 +236,6 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
   __syncthreads();
 
   const float scale = p.scale;
-  const float sl2 = p.scale * kLog2e;
   [[maybe_unused]] const float drop_log2 = __builtin_amdgcn_logf(p.drop.scale), drop_inv = 1.0f / p.drop.scale;
   int cur = 0;                    // ring slot of the stage being read
   int fill = (ahead + 1) % R;     // ring slot the next issued stage goes to
@@ -285,16 +252,6 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
     lse_c = lse_n;
     delta_c = delta_n;
     if (ir + 1 < nrows) rowload(ir + 1);
-    // AUG: the per-query constants -lse/(scale*log2e) and -delta enter through one extra 16-wide
-    // MFMA contraction step (value = 2048*hi + lo, two fp16) instead of per-element subtractions
-    half8_t augS = {0, 0, 0, 0, 0, 0, 0, 0}, augD = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (p.aug_cinv != 0.f) {
-      const uint32_t ws = split_2048(lse_c * p.aug_cinv), wd = split_2048(-delta_c);
-      u32x4 bs = {hh ? 0u : ws, 0u, 0u, 0u}, bd = {hh ? 0u : wd, 0u, 0u, 0u};
-      if (AUGC == 2) augS = as_half8(bs);
-      if (AUGC >= 1) augD = as_half8(bd);
-    }
-
 #pragma unroll
     for (int tt = 0; tt < NKT; ++tt)
 #pragma unroll
@@ -326,8 +283,6 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
         for (int ks = 0; ks < KS; ++ks) s = T::mfma(lds_frag<D>(cK, row0 + g * 32, fo, ks), qf[ks], s);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) dp = T::mfma(lds_frag<D>(cV, row0 + g * 32, fo, ks), dof[ks], dp);
-        if constexpr (AUGC == 2) s = mfma32(aug_ones(), augS, s);
-        if constexpr (AUGC >= 1) dp = mfma32(aug_ones(), augD, dp);
         uint32_t dsp[8];
         [[maybe_unused]] uint32_t kb[4];  // DROP: the keep bytes of this lane's four groups of four keys
         if constexpr (DROP) {
@@ -338,25 +293,15 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
           const uint32_t bb = bias_reg[tt][r >> 1];
-          float p0, p1, d0, d1;
-          if (AUG) {
-            p0 = exp2_fast(__builtin_fmaf(s[r], sl2, T::lo(bb)));
-            p1 = exp2_fast(__builtin_fmaf(s[r + 1], sl2, T::hi(bb)));
-            d0 = p0 * dp[r];
-            d1 = p1 * dp[r + 1];
-          } else {
-            const float t0 = __builtin_fmaf(s[r], scale, T::lo(bb));
-            const float t1 = __builtin_fmaf(s[r + 1], scale, T::hi(bb));
-            p0 = exp2_fast(__builtin_fmaf(t0, kLog2e, nl));
-            p1 = exp2_fast(__builtin_fmaf(t1, kLog2e, nl));
-            float e0 = dp[r], e1 = dp[r + 1];
-            if constexpr (DROP) {  // (1 - p) dP
-              e0 = keep_byte(p.drop, kb[r >> 2], r & 3) ? e0 : 0.f;
-              e1 = keep_byte(p.drop, kb[r >> 2], (r & 3) + 1) ? e1 : 0.f;
-            }
-            d0 = (AUGC == 1) ? p0 * e0 : p0 * (e0 - delta_c);
-            d1 = (AUGC == 1) ? p1 * e1 : p1 * (e1 - delta_c);
+          const float t0 = __builtin_fmaf(s[r], scale, T::lo(bb));
+          const float t1 = __builtin_fmaf(s[r + 1], scale, T::hi(bb));
+          const float p0 = exp2_fast(__builtin_fmaf(t0, kLog2e, nl)), p1 = exp2_fast(__builtin_fmaf(t1, kLog2e, nl));
+          float e0 = dp[r], e1 = dp[r + 1];
+          if constexpr (DROP) {  // (1 - p) dP
+            e0 = keep_byte(p.drop, kb[r >> 2], r & 3) ? e0 : 0.f;
+            e1 = keep_byte(p.drop, kb[r >> 2], (r & 3) + 1) ? e1 : 0.f;
           }
+          const float d0 = p0 * (e0 - delta_c), d1 = p1 * (e1 - delta_c);
           dbacc[tt][r] += d0;
           dbacc[tt][r + 1] += d1;
           dsp[r >> 1] = T::pack_fast(d0, d1);
@@ -476,16 +421,11 @@ __global__ void __launch_bounds__(MAXT) fta_bwd_dq_kernel(const BwdParams p) {
 // ------------------------------------------------------------------------------------------------
 // 2. dK + dV
 // ------------------------------------------------------------------------------------------------
-// T: element type.  FOLD: scale, bias and the row constants -lse, -delta enter through the matrix
-// core (an fp16 device: pre-scaled K, one-hot bias steps, fp16 splits in aux); without it they are
-// applied on the vector ALU in fp32 from the raw {lse, delta} pairs in aux, which is what bf16
-// inputs and DROP (whose mask sits between dP and the subtraction of delta) need.
-// SJC: the number of query slabs where it is known at compile time, as in the dQ kernel.
-template <class T, bool FOLD, bool DROP, int D, int NJT, int JT, bool TAIL, int SJC = 0>
+// T: element type.  SJC: the number of query slabs where it is known at compile time, as in the dQ kernel.
+template <class T, bool DROP, int D, int NJT, int JT, int SJC = 0>
 __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
-  static_assert(!FOLD || (!T::is_bf16 && !DROP), "folded constants: fp16 without dropout only");
   constexpr bool FIX = (SJC != 0);
-  static_assert(!FIX || (TAIL && D == 32 && JT == 64), "fixed geometry");
+  static_assert(!FIX || (D == 32 && JT == 64), "fixed geometry");
   constexpr int G = JT / 32;                // 32-query tiles per stage (JT queries per slab and stage)
   constexpr int STEPS = NJT / G;
   constexpr int JW = NJT * 32;              // queries per wave slab
@@ -527,37 +467,12 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   half_t* dkbase = p.dk + b * p.dks[0] + h * p.dks[1];
   half_t* dvbase = p.dv + b * p.dvs[0] + h * p.dvs[1];
 
-  // stationary bias^T, pre-multiplied by log2(e), held as MFMA A operands: the tile's bias is added
-  // to the scores by the matrix core, S += biasA_u * Eb_u, with Eb_u the one-hot B operand that
-  // routes contraction slot s of step u to key column 16u + s.  biasA[jt][u] of lane (j = l%32, hh)
-  // holds bias[jr0 + jslab*JW + jt*32 + j][k0 + 16u + 8hh .. +7].
+  // stationary bias^T in the accumulator layout, as packed pairs of the element type: biasA[jt] words 0..7 hold the rows
+  // (queries) 8*(r/4) + 4*hh + r%4, r = 0..15, of key k0 + l%32.  One 2-byte load per element, once per chunk (the key
+  // of a lane is fixed, its queries are a bias row apart).
   u32x4 biasA[NJT][2];
-  half8_t Eb[2];
   const half_t* bbh = p.bias + b * p.bs[0] + h * p.bs[1];
-  if constexpr (FOLD) {
-#pragma unroll
-    for (int jt = 0; jt < NJT; ++jt) {
-      const int j = p.jr0 + jslab * JW + jt * 32 + l32;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        // (keys and queries beyond the row's true length: see load_bias4; neither is ever stored)
-        const u32x2 lo = TAIL ? load_bias4(bbh, p.bs[2], j, k0 + 8 * hh + 16 * u, p.L2)
-                              : *reinterpret_cast<const u32x2*>(bbh + (int64_t)j * p.bs[2] + k0 + 8 * hh + 16 * u);
-        const u32x2 hi = TAIL ? load_bias4(bbh, p.bs[2], j, k0 + 8 * hh + 16 * u + 4, p.L2)
-                              : *reinterpret_cast<const u32x2*>(bbh + (int64_t)j * p.bs[2] + k0 + 8 * hh + 16 * u + 4);
-        biasA[jt][u] = u32x4{bias_log2_half2(lo[0]), bias_log2_half2(lo[1]), bias_log2_half2(hi[0]),
-                             bias_log2_half2(hi[1])};
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int x = 0; x < 8; ++x) Eb[u][x] = (16 * u + 8 * hh + x == l32) ? (half_t)1.0f : (half_t)0.0f;
-  } else {
-    // Without the folding the bias tile sits in the accumulator layout, as packed pairs of the element
-    // type: biasA[jt] words 0..7 hold the rows (queries) 8*(r/4) + 4*hh + r%4, r = 0..15, of key k0 + l%32.
-    // One 2-byte load per element, once per chunk (the key of a lane is fixed, its queries are a
-    // bias row apart).
+  {
     const int kk = (k0 + l32 < p.L2) ? k0 + l32 : p.L2 - 1;   // (a key beyond the row: never stored)
 #pragma unroll
     for (int jt = 0; jt < NJT; ++jt) {
@@ -579,10 +494,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   // lse and delta: one copy instruction moves 64 floats x 4 = one slab's JT floats need JT/4 lanes.
   const int nstage = nrows * STEPS;
   const int nld = 2 * SJ;  // (lse|delta) x slab copy instructions per stage, dealt round-robin
-  DmaPlan<4> plq, pld;
-  dma_plan<D, 4>(plq, stage_rows, JT, JW, p.qs[3], wave, lane, nwaves);
-  dma_plan<D, 4>(pld, stage_rows, JT, JW, p.dos[3], wave, lane, nwaves);
-  const int ndma = plq.n + pld.n + ((nld > wave) ? (nld - wave + nwaves - 1) / nwaves : 0);
+  const int ndma = 2 * dma_rows_count(stage_rows, D, wave, nwaves) + ((nld > wave) ? (nld - wave + nwaves - 1) / nwaves : 0);
   const int nkdma = 2 * dma_rows_count(KR2, D, wave, nwaves);  // extra copies in a row's first stage
   const uint32_t lds0 = lds_addr_of(smem);
   const uint32_t ldsk = lds_addr_of(ktiles);
@@ -595,38 +507,26 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   const half_t* kcur = kbase + (int64_t)i0 * p.ks[2] + (int64_t)(FIX ? 0 : kg * KB * 32) * p.ks[3];
   const half_t* vcur = vbase + (int64_t)i0 * p.vs[2] + (int64_t)(FIX ? 0 : kg * KB * 32) * p.vs[3];
   const uint32_t* acur = p.aux + (((int64_t)bh * p.L1 + i0) * p.L2p + p.jr0) * 2;
-  const int64_t qstep = (int64_t)JT * p.qs[3], dostep = (int64_t)JT * p.dos[3];
   // (a row length that is not a multiple of the tile: rows beyond it are copies of the last real
   // key or query; P of such queries is 0 through their row constant, such keys are never stored)
-  constexpr bool tail = TAIL;
-  const int last = TAIL ? p.L2 - 1 : 0x7fffffff;
+  const int last = p.L2 - 1;
   auto stage = [&](int slot) {
     const int j0 = cur_t * JT;  // first query of slab 0 in this stage, relative to the launch's range
     const uint32_t dst = lds0 + (uint32_t)(slot * slot_halfs) * 2u;
-    if constexpr (!tail) {
-      if (cur_t == 0) {
-        const uint32_t kd = ldsk + (uint32_t)((cur_ir % NB) * 2 * KR2 * D) * 2u;
-        dma_rows<D>(kcur, p.ks[3], KR2, kd, wave, lane, nwaves);
-        dma_rows<D>(vcur, p.vs[3], KR2, kd + (uint32_t)(KR2 * D) * 2u, wave, lane, nwaves);
-      }
-      dma_issue(plq, qcur + cur_t * qstep, dst);
-      dma_issue(pld, docur + cur_t * dostep, dst + (uint32_t)(stage_rows * D) * 2u);
-    } else {
-      // (the clamped copies count rows from the start of the row)
-      if (cur_t == 0) {
-        const uint32_t kd = ldsk + (uint32_t)((cur_ir % NB) * 2 * KR2 * D) * 2u;
-        dma_tile_clamped<D>(kcur - (int64_t)(kg * KR2) * p.ks[3], p.ks[3], KR2, KR2, 0, kg * KR2, last, kd, wave, lane, nwaves);
-        dma_tile_clamped<D>(vcur - (int64_t)(kg * KR2) * p.vs[3], p.vs[3], KR2, KR2, 0, kg * KR2, last, kd + (uint32_t)(KR2 * D) * 2u,
-                            wave, lane, nwaves);
-      }
-      dma_tile_clamped<D>(qcur - (int64_t)p.jr0 * p.qs[3], p.qs[3], stage_rows, JT, JW, p.jr0 + j0, last, dst, wave, lane, nwaves);
-      dma_tile_clamped<D>(docur - (int64_t)p.jr0 * p.dos[3], p.dos[3], stage_rows, JT, JW, p.jr0 + j0, last,
-                          dst + (uint32_t)(stage_rows * D) * 2u, wave, lane, nwaves);
+    // (the clamped copies count rows from the start of the row)
+    if (cur_t == 0) {
+      const uint32_t kd = ldsk + (uint32_t)((cur_ir % NB) * 2 * KR2 * D) * 2u;
+      dma_tile_clamped<D>(kcur - (int64_t)(kg * KR2) * p.ks[3], p.ks[3], KR2, KR2, 0, kg * KR2, last, kd, wave, lane, nwaves);
+      dma_tile_clamped<D>(vcur - (int64_t)(kg * KR2) * p.vs[3], p.vs[3], KR2, KR2, 0, kg * KR2, last, kd + (uint32_t)(KR2 * D) * 2u,
+                          wave, lane, nwaves);
     }
+    dma_tile_clamped<D>(qcur - (int64_t)p.jr0 * p.qs[3], p.qs[3], stage_rows, JT, JW, p.jr0 + j0, last, dst, wave, lane, nwaves);
+    dma_tile_clamped<D>(docur - (int64_t)p.jr0 * p.dos[3], p.dos[3], stage_rows, JT, JW, p.jr0 + j0, last,
+                        dst + (uint32_t)(stage_rows * D) * 2u, wave, lane, nwaves);
     const uint32_t ld = dst + (uint32_t)(2 * stage_rows * D) * 2u;
     for (int c = wave; c < nld; c += nwaves) {
       const int which = c / SJ, sl = c % SJ;
-      // one (hi,lo) word pair per query row, written by the delta pre-pass: JT rows = JT/2 lanes
+      // one {lse, delta} pair per query row, written by the delta pre-pass: JT rows = JT/2 lanes
       // x 16 B, copied in two halves
       const uint32_t* src = acur + (j0 + sl * JW) * 2 + which * JT;
       const uint32_t la = __builtin_amdgcn_readfirstlane(ld + (uint32_t)(sl * JT * 2 + which * JT) * 4u);
@@ -696,7 +596,6 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   __syncthreads();
 
   const float scale = p.scale;
-  const float sl2 = p.scale * kLog2e;
   int cur = 0;                    // ring slot of the stage being read
   int fill = (ahead + 1) % R;     // ring slot the next issued stage goes to
 
@@ -705,9 +604,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
       const half_t* kt = ktiles + (ir % NB) * 2 * KR2 * D;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        // FOLD: K times sm_scale*log2(e), the scores come out of the MFMAs as base-2 exponents
-        if constexpr (FOLD) kf[ks] = scale_half8(lds_frag<D>(kt, kb * 32, fo, ks), sl2);
-        else kf[ks] = lds_frag<D>(kt, kb * 32, fo, ks);
+        kf[ks] = lds_frag<D>(kt, kb * 32, fo, ks);
         vf[ks] = lds_frag<D>(kt + KR2 * D, kb * 32, fo, ks);
       }
     }
@@ -737,66 +634,49 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) dp = T::mfma(lds_frag<D>(cDO, row0 + g * 32, fo, ks), vf[ks], dp);
         uint32_t pp[8], dsp[8];
-        if constexpr (FOLD) {
+        // {lse, delta} of the lane's 16 queries: four groups of four consecutive queries, 32 bytes each
+        const float* cF = reinterpret_cast<const float*>(cL) + (g * 32 + 4 * hh) * 2;
+        // DROP: the eight blocks of this tile (query pairs m = 0..7: accumulator rows 2m, 2m+1) are the
+        // same for the four lanes of a key group; each lane computes pairs q and q + 4 (q = its place in
+        // the group) and the bytes change lanes: kb[w] holds this lane's key, byte s of word w (the even and the
+        // odd query of pairs s, then of pairs s + 4)
+        [[maybe_unused]] uint32_t kb[4];
+        if constexpr (DROP) {
+          int ln = lane;
+          if constexpr (FIX) asm volatile("" : "+v"(ln));  // (the generator's counters are not kept over the rows)
+          const int qd = ln & 3, jtile = p.jr0 + jslab * JW + jt * 32 + 4 * (ln >> 5), kl = k0 + (ln & 31);
+          const uint32_t rowid = (uint32_t)(bh * p.L1 + i0 + ir);
+          const u32pair blkA = keep_block(p.drop, rowid, jtile + 8 * (qd >> 1) + 2 * (qd & 1), kl);          // pair m = q
+          const u32pair blkB = keep_block(p.drop, rowid, jtile + 8 * ((qd + 4) >> 1) + 2 * (qd & 1), kl);    // pair m = q + 4
+          kb[0] = quad_transpose_bytes(blkA.x, ln);
+          kb[1] = quad_transpose_bytes(blkA.y, ln);
+          kb[2] = quad_transpose_bytes(blkB.x, ln);
+          kb[3] = quad_transpose_bytes(blkB.y, ln);
+        }
 #pragma unroll
-          for (int u = 0; u < 2; ++u) s = mfma32(as_half8(biasA[jt][u]), Eb[u], s);
-          // row constants of the tile's 32 queries (A-operand rows): one word pair per lane
-          const u32x2 a = *reinterpret_cast<const u32x2*>(cL + (g * 32 + l32) * 2);
-          u32x4 as = {hh ? 0u : a[0], 0u, 0u, 0u}, ad = {hh ? 0u : a[1], 0u, 0u, 0u};
-          s = mfma32(as_half8(as), aug_ones(), s);
-          dp = mfma32(as_half8(ad), aug_ones(), dp);
+        for (int rg = 0; rg < 4; ++rg) {
+          const float4 c01 = *reinterpret_cast<const float4*>(cF + rg * 16);       // lse0 delta0 lse1 delta1
+          const float4 c23 = *reinterpret_cast<const float4*>(cF + rg * 16 + 4);
+          const float lse4[4] = {c01.x, c01.z, c23.x, c23.z}, del4[4] = {c01.y, c01.w, c23.y, c23.w};
 #pragma unroll
-          for (int r = 0; r < 16; r += 2) {
-            const float p0 = exp2_fast(s[r]);
-            const float p1 = exp2_fast(s[r + 1]);
-            pp[r >> 1] = pack_rtz(p0, p1);
-            dsp[r >> 1] = pack_rtz(p0 * dp[r], p1 * dp[r + 1]);
-          }
-        } else {
-          // {lse, delta} of the lane's 16 queries: four groups of four consecutive queries, 32 bytes each
-          const float* cF = reinterpret_cast<const float*>(cL) + (g * 32 + 4 * hh) * 2;
-          // DROP: the eight blocks of this tile (query pairs m = 0..7: accumulator rows 2m, 2m+1) are the
-          // same for the four lanes of a key group; each lane computes pairs q and q + 4 (q = its place in
-          // the group) and the bytes change lanes: kb[w] holds this lane's key, byte s of word w (the even and the
-          // odd query of pairs s, then of pairs s + 4)
-          [[maybe_unused]] uint32_t kb[4];
-          if constexpr (DROP) {
-            int ln = lane;
-            if constexpr (FIX) asm volatile("" : "+v"(ln));  // (the generator's counters are not kept over the rows)
-            const int qd = ln & 3, jtile = p.jr0 + jslab * JW + jt * 32 + 4 * (ln >> 5), kl = k0 + (ln & 31);
-            const uint32_t rowid = (uint32_t)(bh * p.L1 + i0 + ir);
-            const u32pair blkA = keep_block(p.drop, rowid, jtile + 8 * (qd >> 1) + 2 * (qd & 1), kl);          // pair m = q
-            const u32pair blkB = keep_block(p.drop, rowid, jtile + 8 * ((qd + 4) >> 1) + 2 * (qd & 1), kl);    // pair m = q + 4
-            kb[0] = quad_transpose_bytes(blkA.x, ln);
-            kb[1] = quad_transpose_bytes(blkA.y, ln);
-            kb[2] = quad_transpose_bytes(blkB.x, ln);
-            kb[3] = quad_transpose_bytes(blkB.y, ln);
-          }
-#pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
-            const float4 c01 = *reinterpret_cast<const float4*>(cF + rg * 16);       // lse0 delta0 lse1 delta1
-            const float4 c23 = *reinterpret_cast<const float4*>(cF + rg * 16 + 4);
-            const float lse4[4] = {c01.x, c01.z, c23.x, c23.z}, del4[4] = {c01.y, c01.w, c23.y, c23.w};
-#pragma unroll
-            for (int e = 0; e < 4; e += 2) {
-              const int r = 4 * rg + e;
-              const uint32_t bb = (r < 8) ? biasA[jt][0][r >> 1] : biasA[jt][1][(r - 8) >> 1];
-              const float t0 = __builtin_fmaf(s[r], scale, T::lo(bb)), t1 = __builtin_fmaf(s[r + 1], scale, T::hi(bb));
-              float p0 = exp2_fast(__builtin_fmaf(t0, kLog2e, -lse4[e])), p1 = exp2_fast(__builtin_fmaf(t1, kLog2e, -lse4[e + 1]));
-              float e0 = dp[r], e1 = dp[r + 1];
-              float w0 = p0, w1 = p1;  // the weights that dV sees
-              if constexpr (DROP) {
-                const int m = 2 * rg + e / 2;  // the query pair of rows r, r+1
-                const bool k0b = keep_byte(p.drop, kb[m < 4 ? 0 : 2], m & 3), k1b = keep_byte(p.drop, kb[m < 4 ? 1 : 3], m & 3);
-                w0 = k0b ? p0 : 0.f;
-                w1 = k1b ? p1 : 0.f;
-                e0 = k0b ? e0 : 0.f;
-                e1 = k1b ? e1 : 0.f;
-                asm("" : "+v"(w0), "+v"(w1));  // (otherwise each is converted by itself, selected and packed: twice the instructions)
-              }
-              pp[r >> 1] = T::pack_fast(w0, w1);
-              dsp[r >> 1] = T::pack_fast(p0 * (e0 - del4[e]), p1 * (e1 - del4[e + 1]));
+          for (int e = 0; e < 4; e += 2) {
+            const int r = 4 * rg + e;
+            const uint32_t bb = (r < 8) ? biasA[jt][0][r >> 1] : biasA[jt][1][(r - 8) >> 1];
+            const float t0 = __builtin_fmaf(s[r], scale, T::lo(bb)), t1 = __builtin_fmaf(s[r + 1], scale, T::hi(bb));
+            float p0 = exp2_fast(__builtin_fmaf(t0, kLog2e, -lse4[e])), p1 = exp2_fast(__builtin_fmaf(t1, kLog2e, -lse4[e + 1]));
+            float e0 = dp[r], e1 = dp[r + 1];
+            float w0 = p0, w1 = p1;  // the weights that dV sees
+            if constexpr (DROP) {
+              const int m = 2 * rg + e / 2;  // the query pair of rows r, r+1
+              const bool k0b = keep_byte(p.drop, kb[m < 4 ? 0 : 2], m & 3), k1b = keep_byte(p.drop, kb[m < 4 ? 1 : 3], m & 3);
+              w0 = k0b ? p0 : 0.f;
+              w1 = k1b ? p1 : 0.f;
+              e0 = k0b ? e0 : 0.f;
+              e1 = k1b ? e1 : 0.f;
+              asm("" : "+v"(w0), "+v"(w1));  // (otherwise each is converted by itself, selected and packed: twice the instructions)
             }
+            pp[r >> 1] = T::pack_fast(w0, w1);
+            dsp[r >> 1] = T::pack_fast(p0 * (e0 - del4[e]), p1 * (e1 - del4[e + 1]));
           }
         }
         // dV^T += dO^T P ; dK^T += Q^T dS   (contraction over the 32 queries of the tile)

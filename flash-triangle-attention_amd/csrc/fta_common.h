@@ -54,12 +54,6 @@ __device__ __forceinline__ uint32_t pack_rn(float a, float b) {
 
 __device__ __forceinline__ half2_t as_half2(uint32_t u) { return __builtin_bit_cast(half2_t, u); }
 
-// Packed fp16 pair times an fp32 factor, rounded back to fp16 (round to nearest).
-__device__ __forceinline__ uint32_t scale_half2(uint32_t u, float f) {
-  half2_t h = __builtin_bit_cast(half2_t, u);
-  return pack_rn((float)h[0] * f, (float)h[1] * f);
-}
-
 // The stationary bias of the kernels that add it through the matrix core: bias * log2(e) as fp16, kept
 // FINITE.  A masked key (-inf, or anything whose product with log2(e) leaves the fp16 range, such as
 // the usual -1e9 cast to fp16) would otherwise meet the zeros of the one-hot selector inside a
@@ -517,22 +511,7 @@ __device__ __forceinline__ void dma_plan(DmaPlan<MAXU>& pl, int rows, int T, int
   }
 }
 
-// One-off copy of a small tile (rows x D halfs, tile row r = global row r) computed on the fly;
-// returns how many copies this wave issued.  Used for the per-row operand rows (a few KB).
-template <int D>
-__device__ __forceinline__ int dma_rows(const void* sbase, int64_t gstride, int rows, uint32_t lds_tile_addr, int wave,
-                                        int lane, int nwaves) {
-  constexpr int CPR = D / 8;
-  const int ninstr = rows * CPR / 64;
-  int n = 0;
-  for (int j = wave; j < ninstr; j += nwaves, ++n) {
-    const int p = j * 64 + lane;
-    const int row = p / CPR, slot = p % CPR;
-    const uint32_t voff = (uint32_t)(((int64_t)row * gstride + swz_slot<D>(row, slot) * 8) * 2);
-    dma16s(voff, sbase, __builtin_amdgcn_readfirstlane(lds_tile_addr + (uint32_t)j * 1024u));
-  }
-  return n;
-}
+// How many of the 1 KB copies that a tile of `rows` rows of D halfs takes fall to this wave.
 __device__ __forceinline__ int dma_rows_count(int rows, int D, int wave, int nwaves) {
   const int ninstr = rows * (D / 8) / 64;
   return (ninstr > wave) ? (ninstr - wave + nwaves - 1) / nwaves : 0;

@@ -78,10 +78,10 @@ struct BwdParams {
   const half_t* q; const half_t* k; const half_t* v; const half_t* bias;
   const half_t* o; const float* lse; const half_t* dout;
   half_t* dq; half_t* dk; half_t* dv; half_t* dbias;
-  float* delta;        // (B,H,L1,L2) fp32 workspace, written by the dQ kernel, read by the dK/dV kernel
+  float* delta;        // (B,H,L1,L2) fp32 workspace, written by the delta kernel, read by the general dQ kernel
   float* partial;      // (nchunks,B*H,L2,L2) fp32 workspace: per-chunk sums of dS over L1 rows
-  uint32_t* aux;       // (B,H,L1,L2,2) workspace: packed fp16 (hi,lo) splits of -lse (log2 domain) and -delta
-  float aug_cinv;      // -1/(scale*log2e), or 0 when the constants are not folded into the MFMAs
+  uint32_t* aux;       // (B,H,L1,L2,2) workspace: the row constants lse and delta for the dK/dV kernel, as fp16 (hi,lo) splits
+                       // of -lse (log2 domain) and -delta (hand-scheduled) or in fp32 (general)
   int64_t qs[4], ks[4], vs[4], os[4], dos[4], dqs[4], dks[4], dvs[4];
   int64_t bs[3], dbs[3];
   int B, H, L1, L2;    // L2: the true row length; lse is (B,H,L1,L2)
@@ -146,9 +146,8 @@ struct BwdPlan {
   int NJT, JT, SJ, KB, nkg, nchunks2, rows_per_chunk2, threads2, JR, nlaunch2, ring2, nb2;
   size_t smem2;
   size_t delta_bytes, partial_bytes, aux_bytes;
-  bool use_dq1;        // the dQ/dBias stage runs the one-wave-per-SIMD kernel
+  bool use_hand;       // the hand-scheduled one-wave-per-SIMD kernels run
   Dq1Plan dq1;
-  bool use_dkdv1;      // the dK/dV stage runs the one-wave-per-SIMD kernel
   Dkdv1Plan dkdv1;
   bool use_short;      // rows of up to 128 keys: all gradients in one kernel
   ShortPlan sh;
@@ -199,6 +198,7 @@ constexpr Ring dkdv_ring(int D, int NJT, int JT, int SJ) {
 // kernels only, smaller instance sets).
 BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat);
 hipError_t launch_bwd(BwdParams p, const BwdPlan& pl, int D, int dtype, hipStream_t st, hipEvent_t* ev = nullptr);
+hipError_t launch_dbias_reduce(const BwdParams& p, int dtype, hipStream_t st);
 hipError_t launch_bwd_feat(const BwdParams& p, const BwdPlan& pl, int D, int dtype, hipStream_t st, hipEvent_t* ev);
 
 // feat: the plan is for bf16 inputs or dropout, which have a smaller set of kernel instances
@@ -219,9 +219,8 @@ inline hipError_t launch_kernel(K kern, const P& p, dim3 grid, dim3 block, size_
   return hipGetLastError();
 }
 
-// Bit 0: the dQ/dBias stage runs the general kernel even where the pipelined one applies; bit 1: the
-// same for dK/dV (set through fta_debug_select_kernels, for tests of the general kernels).
-int forced_general_mask();
+// The backward runs the general kernels even where others apply (set through fta_debug_select_kernels, for tests).
+bool forced_general();
 hipError_t launch_fwd(FwdParams p, const FwdPlan& pl, int D, int dtype, hipStream_t st);
 // The hand-scheduled forward (fta_fwd1_kernel.h): D = 32, tiled length 64 ... 1792, no dropout.
 bool plan_fwd1(int B, int H, int L1, int L2, int D, FwdPlan& pl);

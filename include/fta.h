@@ -149,9 +149,9 @@ int fta_describe_plan(int B, int H, int L1, int L2, int D, char* out, size_t out
 int fta_describe_plan_ex(int B, int H, int L1, int L2, int D, float sm_scale, const fta_options* options, char* out,
                          size_t out_bytes);
 
-/* Test hook, no counterpart upstream: bit 0 of `general_mask` makes the dQ/dBias stage run the general
- * (two waves per SIMD) kernel even where the pipelined one applies, bit 1 the same for dK/dV.
- * Process-wide; returns the previous mask.  The workspace size depends on it: set it before
+/* Test hook, no counterpart upstream: with bit 0 or 1 of `general_mask` set the backward runs the general
+ * (two waves per SIMD) kernels also where the hand-scheduled ones or the one-kernel form of short rows
+ * apply.  Process-wide; returns the previous mask.  The workspace size depends on it: set it before
  * fta_bwd_workspace_bytes.  Exists so that tests reach the general kernels at every length. */
 int fta_debug_select_kernels(int general_mask);
 
