@@ -100,14 +100,6 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
   return pl;
 }
 
-hipError_t launch_dbias_reduce(const BwdParams& p, int dtype, hipStream_t st) {
-  const int64_t total4 = (int64_t)p.B * p.H * p.L2 * ((p.L2 + 3) / 4);
-  dim3 grid((unsigned)((total4 + 255) / 256)), block(256);
-  if (dtype == kBF16) hipLaunchKernelGGL(fta_dbias_reduce_kernel<BF16>, grid, block, 0, st, p);
-  else hipLaunchKernelGGL(fta_dbias_reduce_kernel<F16>, grid, block, 0, st, p);
-  return hipGetLastError();
-}
-
 hipError_t launch_bwd(BwdParams p, const BwdPlan& pl, int D, int dtype, hipStream_t st, hipEvent_t* ev) {
   // ev (optional, 5 events): recorded before stage 0 and after each of the four stages
   auto mark = [&](int i) { if (ev != nullptr) (void)hipEventRecord(ev[i], st); };

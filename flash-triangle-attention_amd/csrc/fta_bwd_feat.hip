@@ -13,6 +13,14 @@
 
 namespace fta {
 
+hipError_t launch_dbias_reduce(const BwdParams& p, int dtype, hipStream_t st) {
+  const int64_t total4 = (int64_t)p.B * p.H * p.L2 * ((p.L2 + 3) / 4);
+  dim3 grid((unsigned)((total4 + 255) / 256)), block(256);
+  if (dtype == kBF16) hipLaunchKernelGGL(fta_dbias_reduce_kernel<BF16>, grid, block, 0, st, p);
+  else hipLaunchKernelGGL(fta_dbias_reduce_kernel<F16>, grid, block, 0, st, p);
+  return hipGetLastError();
+}
+
 template <class T, bool DROP>
 static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t st, hipEvent_t* ev) {
   auto mark = [&](int i) { if (ev != nullptr) (void)hipEventRecord(ev[i], st); };

@@ -82,6 +82,11 @@ struct BwdParams {
   float* partial;      // (nchunks,B*H,L2,L2) fp32 workspace: per-chunk sums of dS over L1 rows
   uint32_t* aux;       // (B,H,L1,L2,2) workspace: the row constants lse and delta for the dK/dV kernel, as fp16 (hi,lo) splits
                        // of -lse (log2 domain) and -delta (hand-scheduled) or in fp32 (general)
+  // (eight bytes that the hand-scheduled kernels do not read, in front of the strides: without them the compiler loads the
+  // strides in larger pieces than it has scalar registers for, and 190 lane reads instead of 57 fetch them back in dq1)
+  int dbias_f32;       // dbias is written as fp32 (B,H,L2,L2) instead of the element type
+  float partial_scale; // what the reduction multiplies the summed partials by (1, or 128 behind the bf16
+                       // hand-scheduled dQ/dBias kernel, whose one-hot selector is worth 2^-7: see kOneHotInv)
   int64_t qs[4], ks[4], vs[4], os[4], dos[4], dqs[4], dks[4], dvs[4];
   int64_t bs[3], dbs[3];
   int B, H, L1, L2;    // L2: the true row length; lse is (B,H,L1,L2)
@@ -110,9 +115,6 @@ struct BwdParams {
                        // instances that mask a row's tail run, which read the bias entry by entry where they must
   int nat;             // (host side) the hand-scheduled backward kernels' precise instances run: exponents in
                        // natural units, scaled operands as (hi, lo) pairs
-  int dbias_f32;       // dbias is written as fp32 (B,H,L2,L2) instead of the element type
-  float partial_scale; // what the reduction multiplies the summed partials by (1, or 128 behind the bf16
-                       // hand-scheduled dQ/dBias kernel, whose one-hot selector is worth 2^-7: see kOneHotInv)
 };
 
 
