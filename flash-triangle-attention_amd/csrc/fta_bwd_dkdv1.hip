@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       const int j = p.jr0 + jt * 32 + l32;
       const half_t* row = bias_bh + (int64_t)(TAIL ? min(j, p.L2 - 1) : j) * p.bs[2];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) raw[jt][u] = bias_piece_load<TAIL>(row, k0 + 8 * hh + 16 * u, p.L2, T::kNegInf2, false);
+      for (int u = 0; u < 2; ++u) raw[jt][u] = bias_piece_load<TAIL>(row, k0 + 8 * hh + 16 * u, p.L2, false);
     }
 #pragma unroll
     for (int jt = 0; jt < NJT; ++jt)
@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       for (int u = 0; u < 2; ++u) {
         u32x4 v = raw[jt][u];
         if constexpr (TAIL)
-          if (k0 + 32 > p.L2) v = bias_piece_fix(v, k0 + 8 * hh + 16 * u, p.L2, T::kNegInf2);
+          if (k0 + 32 > p.L2) v = bias_piece_fix(v, k0 + 8 * hh + 16 * u, p.L2, T::kNegInf2, false);  // (keys that are never stored)
         if constexpr (NAT) biasA[jt][u] = u32x4{T::bias_nat(v[0]), T::bias_nat(v[1]), T::bias_nat(v[2]), T::bias_nat(v[3])};
         else biasA[jt][u] = u32x4{T::bias_log2(v[0]), T::bias_log2(v[1]), T::bias_log2(v[2]), T::bias_log2(v[3])};
         asm volatile("" : "+a"(biasA[jt][u]));

@@ -420,13 +420,13 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
     // the bias, while those copies fly; it changes lanes in the ring slot that nothing is copied to yet
     static_assert(4 * 4096 <= SLOT_H * 2, "4 KB for every wave's bias");
     u32x2 even = {0u, 0u};
-    load_bias_tiles<NKT / 2, 2, TAIL, false>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], q0, p.L2, T::kNegInf2,
+    load_bias_tiles<NKT / 2, 2, TAIL, false>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], q0, p.L2, F16::kBeyond2,
                                              smem_raw + (R - 1) * SLOT_H * 2 + wave * 4096, lane, [=](int c) { return key0 + 64 * c; },
+                                             [](uint32_t u) { if constexpr (NAT) return T::bias_nat(u); else return T::bias_log2(u); },
                                              [&](int tt, int g, u32x2 v) {
                                                if (g % 2 == 0) { even = v; return; }
                                                u32x4& d = bias4[tt][g / 2];
-                                               if constexpr (NAT) d = u32x4{T::bias_nat(even[0]), T::bias_nat(even[1]), T::bias_nat(v[0]), T::bias_nat(v[1])};
-                                               else d = u32x4{T::bias_log2(even[0]), T::bias_log2(even[1]), T::bias_log2(v[0]), T::bias_log2(v[1])};
+                                               d = u32x4{even[0], even[1], v[0], v[1]};
                                                asm volatile("" : "+a"(d));  // parked in accumulation registers for the whole kernel
                                              });
   }

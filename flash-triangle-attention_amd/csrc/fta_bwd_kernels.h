@@ -133,9 +133,11 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
     for (int tt = 0; tt < NKT; ++tt) {
 #pragma unroll
       for (int rg = 0; rg < 4; ++rg) {
-        const u32x2 v = load_bias4(bbh, p.bs[2], q0 + l32, key0 + 4 * hh + tt * 32 + rg * 8, p.L2, T::kNegInf2);
-        bias_reg[tt][2 * rg] = T::finite2(v[0]);
-        bias_reg[tt][2 * rg + 1] = T::finite2(v[1]);
+        const int kk = key0 + 4 * hh + tt * 32 + rg * 8;
+        u32x2 v = load_bias4(bbh, p.bs[2], q0 + l32, kk, p.L2);
+        v = beyond_row(u32x2{T::finite2(v[0]), T::finite2(v[1])}, kk, p.L2, T::kBeyond2);
+        bias_reg[tt][2 * rg] = v[0];
+        bias_reg[tt][2 * rg + 1] = v[1];
       }
 #pragma unroll
       for (int r = 0; r < 16; ++r) dbacc[tt][r] = 0.f;

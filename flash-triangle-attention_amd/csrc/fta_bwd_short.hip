@@ -65,11 +65,12 @@ __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(D 
   typedef typename std::conditional<FWD1, F16, T>::type BT;
   uint32_t bias_reg[NT][8];
   float dbacc[NT][16];
-  load_bias_tiles<NT, 1, true, true>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], wave * 32, p.L2, T::kNegInf2,
+  load_bias_tiles<NT, 1, true, true>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], wave * 32, p.L2, BT::kBeyond2,
                                      reinterpret_cast<char*>(xchg + wave * 2 * XT), lane, [=](int c) { return (wave + c) % NT * 32; },
+                                     [](uint32_t u) { return FWD1 ? fwd1_bias_pair<T>(u) : T::finite2(u); },
                                      [&](int r, int g, u32x2 v) {
-                                       bias_reg[r][2 * g] = FWD1 ? fwd1_bias_pair<T>(v[0]) : T::finite2(v[0]);
-                                       bias_reg[r][2 * g + 1] = FWD1 ? fwd1_bias_pair<T>(v[1]) : T::finite2(v[1]);
+                                       bias_reg[r][2 * g] = v[0];
+                                       bias_reg[r][2 * g + 1] = v[1];
                                      });
 #pragma unroll
   for (int r = 0; r < NT; ++r)

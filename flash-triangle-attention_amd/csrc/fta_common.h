@@ -74,6 +74,8 @@ __device__ __forceinline__ uint32_t bias_log2_half2(uint32_t u) {
 // forms its weights from the forward's logsumexp.  (bf16 had a floor of -2^30, beside which the rounding of the
 // exponent alone is 2^6: the weights of such a query came out of the backward wrong by up to 2^64.)
 constexpr float kMaskedBias = -59904.0f;
+// The keys that a row's last tile has beyond the row (copies of the last real one) stand still lower, at kBeyond2 of the
+// element type, a packed pair of -65280: beside masked keys, too, their weight is exactly 0.
 __device__ __forceinline__ uint32_t finite_half2(uint32_t u) {
   half2_t h = __builtin_bit_cast(half2_t, u);
   const half2_t lowest = {(half_t)kMaskedBias, (half_t)kMaskedBias};
@@ -154,6 +156,7 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 struct F16 {
   static constexpr bool is_bf16 = false;
   static constexpr uint32_t kNegInf2 = 0xFC00FC00u;  // packed pair of -inf
+  static constexpr uint32_t kBeyond2 = 0xFBF8FBF8u;  // packed pair of -65280
   static __device__ __forceinline__ floatx16 mfma(half8_t a, half8_t b, floatx16 c) { return mfma32(a, b, c); }
   static __device__ __forceinline__ float lo(uint32_t u) { return (float)as_half2(u)[0]; }
   static __device__ __forceinline__ float hi(uint32_t u) { return (float)as_half2(u)[1]; }
@@ -209,6 +212,7 @@ struct F16 {
 struct BF16 {
   static constexpr bool is_bf16 = true;
   static constexpr uint32_t kNegInf2 = 0xFF80FF80u;
+  static constexpr uint32_t kBeyond2 = 0xC77FC77Fu;
   static __device__ __forceinline__ floatx16 mfma(half8_t a, half8_t b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
   }
@@ -546,28 +550,33 @@ __device__ __forceinline__ void dma_tile_clamped(const void* rowbase, int64_t gs
 }
 
 // Four consecutive bias entries bias[j][k .. k+3] (k a multiple of 4) as two packed pairs; keys at or
-// beyond L2 (the row's true length) read as -inf, queries beyond it read the last query's row.  One
+// beyond L2 (the row's true length) read as any value (beyond_row()), queries beyond it read the last query's row.  One
 // 8-byte load where the four entries exist and sit on an 8-byte boundary; entry by entry at the end of
 // a row whose length is not a multiple of 4 and in rows that start on a 2-byte boundary (such a
 // length, or a strided view).
-__device__ __forceinline__ u32x2 load_bias4(const half_t* bias_bh, int64_t jstride, int j, int k, int L2,
-                                            uint32_t neg_inf2 = 0xFC00FC00u) {
+__device__ __forceinline__ u32x2 load_bias4(const half_t* bias_bh, int64_t jstride, int j, int k, int L2) {
   const int jj = j < L2 ? j : L2 - 1;
-  if (k >= L2) return u32x2{neg_inf2, neg_inf2};
+  if (k >= L2) return u32x2{0u, 0u};
   const half_t* src = bias_bh + (int64_t)jj * jstride + k;
   if (k + 4 <= L2 && (reinterpret_cast<uintptr_t>(src) & 7u) == 0) return *reinterpret_cast<const u32x2*>(src);
   const uint16_t* s16 = reinterpret_cast<const uint16_t*>(src);
   uint32_t e[4];
 #pragma unroll
-  for (int n = 0; n < 4; ++n) e[n] = (k + n < L2) ? (uint32_t)s16[n] : (neg_inf2 & 0xFFFFu);
+  for (int n = 0; n < 4; ++n) e[n] = (k + n < L2) ? (uint32_t)s16[n] : 0u;
   return u32x2{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
+}
+// The pairs of keys k .. k+3 with those at or beyond L2 put to `beyond2` (see kMaskedBias).
+__device__ __forceinline__ u32x2 beyond_row(u32x2 v, int k, int L2, uint32_t beyond2) {
+  const int left = L2 - k;  // real ones
+  return u32x2{left <= 0 ? beyond2 : left == 1 ? (v[0] & 0xFFFFu) | (beyond2 << 16) : v[0],
+               left <= 2 ? beyond2 : left == 3 ? (v[1] & 0xFFFFu) | (beyond2 << 16) : v[1]};
 }
 
 // Eight consecutive bias entries from key k of a row, as whole-row loads want them: entries k .. k+7 of a row that holds
-// them, any other piece (TAIL) as the row's last eight entries, which bias_piece_fix() shifts into place; keys at or
-// beyond L2 come out as -inf.  Any 2-byte boundary.  (Rows of fewer than eight keys are read entry by entry.)
+// them, any other piece (TAIL) as the row's last eight entries, which bias_piece_fix() shifts into place, with `beyond2` for
+// the keys at or beyond L2.  Any 2-byte boundary.  (Rows of fewer than eight keys are read entry by entry.)
 template <bool TAIL>
-__device__ __forceinline__ u32x4 bias_piece_load(const half_t* row, int k, int L2, uint32_t neg_inf2, bool short_rows) {
+__device__ __forceinline__ u32x4 bias_piece_load(const half_t* row, int k, int L2, bool short_rows) {
   u32x4 v;
   if constexpr (!TAIL) {
     v = *reinterpret_cast<const u32x4*>(row + k);
@@ -576,34 +585,39 @@ __device__ __forceinline__ u32x4 bias_piece_load(const half_t* row, int k, int L
   } else {
     uint32_t e[8];
 #pragma unroll
-    for (int n = 0; n < 8; ++n) e[n] = k + n < L2 ? (uint32_t)reinterpret_cast<const uint16_t*>(row)[k + n] : (neg_inf2 & 0xFFFFu);
+    for (int n = 0; n < 8; ++n) e[n] = k + n < L2 ? (uint32_t)reinterpret_cast<const uint16_t*>(row)[k + n] : 0u;
     v = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
   }
   return v;
 }
-__device__ __forceinline__ u32x4 bias_piece_fix(u32x4 v, int k, int L2, uint32_t neg_inf2) {
+__device__ __forceinline__ u32x4 bias_piece_fix(u32x4 v, int k, int L2, uint32_t beyond2, bool short_rows) {
+  if (short_rows && L2 < 8) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n) v[n] = k + 2 * n >= L2 ? beyond2 : k + 2 * n + 1 >= L2 ? (v[n] & 0xFFFFu) | (beyond2 << 16) : v[n];
+    return v;
+  }
   const int sh = k + 8 <= L2 ? 0 : (k - (L2 - 8) < 8 ? k - (L2 - 8) : 8);  // entries to drop at the front
-  if (sh & 4) v = u32x4{v[2], v[3], neg_inf2, neg_inf2};
-  if (sh & 2) v = u32x4{v[1], v[2], v[3], neg_inf2};
+  if (sh & 4) v = u32x4{v[2], v[3], beyond2, beyond2};
+  if (sh & 2) v = u32x4{v[1], v[2], v[3], beyond2};
   if (sh & 1)
     v = u32x4{__builtin_amdgcn_alignbit(v[1], v[0], 16), __builtin_amdgcn_alignbit(v[2], v[1], 16), __builtin_amdgcn_alignbit(v[3], v[2], 16),
-              __builtin_amdgcn_alignbit(neg_inf2, v[3], 16)};
-  if (sh & 8) v = u32x4{neg_inf2, neg_inf2, neg_inf2, neg_inf2};
+              __builtin_amdgcn_alignbit(beyond2, v[3], 16)};
+  if (sh & 8) v = u32x4{beyond2, beyond2, beyond2, beyond2};
   return v;
 }
 
 // The stationary bias of a wave: 32 queries from q0 against NC chunks of 32*CT keys (chunk c from key first_key(c)),
-// handed to `sink(tile, group, pair)` in the S^T accumulator layout (keys 8*group + 4*hh + 0..3 of the tile's 32, of query
-// l%32, as two packed pairs; tile c*CT + t).  Loaded that way, 8 bytes per lane, an instruction touches 32 rows and every
+// passed through `conv` and handed to `sink(tile, group, pair)` in the S^T accumulator layout (keys
+// 8*group + 4*hh + 0..3 of the tile's 32, of query l%32, as two packed pairs; tile c*CT + t).  Loaded that way, 8 bytes per lane, an instruction touches 32 rows and every
 // 128-byte line is asked for by eight of them, more lines than the L1 holds between two: at 512 keys the set-up of a
 // workgroup took 16 us.  Instead four or eight lanes load a row's keys as one piece of a line, all of them in flight at
 // once, and the pieces change lanes through 2 or 4 KB (CT) of LDS that belong to the wave (no barrier: a wave's LDS operations are
 // executed in order).
-// TAIL: rows of L2 keys that may end inside the tile (keys beyond it read as -inf, queries beyond it as the last query's
-// row), on any 2-byte boundary; SHORT: of fewer than eight keys, too.
-template <int NC, int CT, bool TAIL, bool SHORT, class Key, class Sink>
-__device__ __forceinline__ void load_bias_tiles(const half_t* bias_bh, int64_t jstride, int q0, int L2, uint32_t neg_inf2, char* lds, int lane,
-                                                Key&& first_key, Sink&& sink) {
+// TAIL: rows of L2 keys that may end inside the tile (keys beyond it come out as `beyond2`, queries beyond it as the last
+// query's row), on any 2-byte boundary; SHORT: of fewer than eight keys, too.
+template <int NC, int CT, bool TAIL, bool SHORT, class Key, class Conv, class Sink>
+__device__ __forceinline__ void load_bias_tiles(const half_t* bias_bh, int64_t jstride, int q0, int L2, uint32_t beyond2, char* lds, int lane,
+                                                Key&& first_key, Conv&& conv, Sink&& sink) {
   static_assert(CT == 1 || CT == 2, "chunks of 32 or 64 keys");
   constexpr int PR = 4 * CT, RI = 64 / PR, NI = 32 / RI;  // pieces per row, rows per instruction, instructions per chunk
   const int rowi = lane / PR, piece = lane % PR, l32 = lane & 31, hh = lane >> 5;
@@ -614,20 +628,29 @@ __device__ __forceinline__ void load_bias_tiles(const half_t* bias_bh, int64_t j
     const int j = q0 + RI * i + rowi;
     const half_t* row = bias_bh + (int64_t)(TAIL ? (j < L2 ? j : L2 - 1) : j) * jstride;
 #pragma unroll
-    for (int c = 0; c < NC; ++c) raw[c][i] = bias_piece_load<TAIL>(row, first_key(c) + 8 * piece, L2, neg_inf2, SHORT);
+    for (int c = 0; c < NC; ++c) raw[c][i] = bias_piece_load<TAIL>(row, first_key(c) + 8 * piece, L2, SHORT);
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    if constexpr (TAIL)
-      if (first_key(c) + 32 * CT > L2 && (!SHORT || L2 >= 8))  // the row ends in this chunk, or before it
+    // (TAIL: converted before the pieces of the row's end are put in place, which `conv` would not leave as they are;
+    // else on the way out of LDS)
+    if constexpr (TAIL) {
 #pragma unroll
-        for (int i = 0; i < NI; ++i) raw[c][i] = bias_piece_fix(raw[c][i], first_key(c) + 8 * piece, L2, neg_inf2);
+      for (int i = 0; i < NI; ++i) raw[c][i] = u32x4{conv(raw[c][i][0]), conv(raw[c][i][1]), conv(raw[c][i][2]), conv(raw[c][i][3])};
+      if (first_key(c) + 32 * CT > L2)  // the row ends in this chunk, or before it
+#pragma unroll
+        for (int i = 0; i < NI; ++i) raw[c][i] = bias_piece_fix(raw[c][i], first_key(c) + 8 * piece, L2, beyond2, SHORT);
+    }
 #pragma unroll
     for (int i = 0; i < NI; ++i) *reinterpret_cast<u32x4*>(lds + slot(RI * i + rowi, piece)) = raw[c][i];
 #pragma unroll
     for (int t = 0; t < CT; ++t)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) sink(c * CT + t, g, *reinterpret_cast<const u32x2*>(lds + slot(l32, 4 * t + g) + 8 * hh));
+      for (int g = 0; g < 4; ++g) {
+        const u32x2 v = *reinterpret_cast<const u32x2*>(lds + slot(l32, 4 * t + g) + 8 * hh);
+        if constexpr (TAIL) sink(c * CT + t, g, v);
+        else sink(c * CT + t, g, u32x2{conv(v[0]), conv(v[1])});
+      }
   }
 }
 

@@ -172,11 +172,11 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_wav
   });
   uint32_t bias_reg[NKT][8];
   static_assert(8 * 4096 <= 2 * SLOT_B, "4 KB for every wave's bias");
-  load_bias_tiles<NKT / 2, 2, TAIL, false>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], q0, p.L2, T::kNegInf2, smem_raw + 2 * SLOT_B + wave * 4096,
-                                           lane, [=](int c) { return key0 + 64 * c; },
+  load_bias_tiles<NKT / 2, 2, TAIL, false>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], q0, p.L2, F16::kBeyond2, smem_raw + 2 * SLOT_B + wave * 4096,
+                                           lane, [=](int c) { return key0 + 64 * c; }, fwd1_bias_pair<T>,
                                            [&](int tt, int rg, u32x2 v) {
-                                             bias_reg[tt][2 * rg] = fwd1_bias_pair<T>(v[0]);
-                                             bias_reg[tt][2 * rg + 1] = fwd1_bias_pair<T>(v[1]);
+                                             bias_reg[tt][2 * rg] = v[0];
+                                             bias_reg[tt][2 * rg + 1] = v[1];
                                            });
   q_issue(false);
   wait_vmem_all();

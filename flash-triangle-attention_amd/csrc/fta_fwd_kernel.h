@@ -91,11 +91,11 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
     char* turn = reinterpret_cast<char*>(smem + buf_halfs) + wave * 2048;
     auto key = [=](int c) { return slab * KW + 32 * c; };
     auto keep = [&](int tt, int rg, u32x2 v) {
-      bias_reg[tt][2 * rg] = T::finite2(v[0]);
-      bias_reg[tt][2 * rg + 1] = T::finite2(v[1]);
+      bias_reg[tt][2 * rg] = v[0];
+      bias_reg[tt][2 * rg + 1] = v[1];
     };
-    if (!tail && !p.odd_bias) load_bias_tiles<NKT, 1, false, false>(bbh, p.bs[2], q0, p.L2, T::kNegInf2, turn, lane, key, keep);
-    else load_bias_tiles<NKT, 1, true, NKT == 4>(bbh, p.bs[2], q0, p.L2, T::kNegInf2, turn, lane, key, keep);
+    if (!tail && !p.odd_bias) load_bias_tiles<NKT, 1, false, false>(bbh, p.bs[2], q0, p.L2, T::kBeyond2, turn, lane, key, T::finite2, keep);
+    else load_bias_tiles<NKT, 1, true, NKT == 4>(bbh, p.bs[2], q0, p.L2, T::kBeyond2, turn, lane, key, T::finite2, keep);
   }
 
   // ---- global -> LDS staging of one (row, step): S slabs x KT keys of K and V, copied

@@ -27,12 +27,16 @@
  *     power-of-two L (flash_tt_attn.py:618) and has no masking; here the kernels tile the row in
  *     multiples of 128 keys and mask the rest of the last tile themselves: no padded copies are needed.  The rows of one (b, h, l1) slice must lie within
  *     4 GiB of its first row: L2 * (l2 stride) < 2^31 elements.
- *   - bias may hold any fp16 value including -inf (the usual key mask: -inf, or -1e9 cast to fp16):
- *     a masked key gets weight exactly 0 and zero gradients, as upstream (flash_tt_attn.py:78,
- *     :344-346, :418-420).  Entries below -60000/log2(e) = -41589 are all treated as masked in the
- *     backward (their weight underflows to 0 long before).  A query whose keys are ALL masked has
- *     no defined softmax: upstream returns NaN for it, this library returns finite numbers of no
- *     meaning.  +inf and NaN entries are not supported.
+ *   - bias may hold any value of its type including -inf (the usual key mask: -inf, or -1e9, which is -inf
+ *     in fp16): a masked key gets weight exactly 0 and zero gradients, as upstream (flash_tt_attn.py:78,
+ *     :344-346, :418-420).  Entries below -59904 are taken as -59904 (their weight underflows to 0 long
+ *     before); below -60000/log2(e) = -41589 the hand-scheduled backward kernels treat all of them as
+ *     masked.  A query whose keys are ALL masked with the same value (-inf, or any below -59904) attends by
+ *     its scores alone, in the output and in the gradients, as it does upstream with a finite mask value
+ *     (with -inf upstream returns NaN); where all of a query's biases lie between -59904 and -41589 those
+ *     kernels give it no gradients.  bf16 entries beyond +65504 are taken as 65504 by the hand-scheduled
+ *     forward kernels (D = 32 up to 1792 keys, D = 64 from 129 to 512; not with dropout).  +inf and NaN entries
+ *     are not supported.
  *   - The library never allocates, frees or keeps pointers.  Outputs are fully overwritten.
  *     Launches are asynchronous on `stream` (a hipStream_t; NULL = the default stream).
  *   - Return value: 0 on success; a negative fta_status for an argument error (detected on

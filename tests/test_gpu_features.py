@@ -142,6 +142,11 @@ _ALL_MASKED = [
     (256, 32, "precise"), (512, 32, "precise"),
     # general backward kernels
     (256, 32, "dropout"), (512, 32, "dropout"), (1024, 32, "dropout"), (256, 64, "dropout"), (512, 64, "precise"),
+    # rows that end inside a tile: the keys beyond them weigh nothing beside masked ones either
+    (3, 32, "plain"), (7, 64, "plain"), (9, 32, "dropout"), (33, 32, "plain"), (64, 64, "plain"), (64, 32, "dropout"), (97, 32, "precise"), (101, 64, "dropout"),
+    (131, 32, "plain"), (200, 32, "plain"), (300, 32, "precise"), (457, 32, "plain"), (701, 32, "plain"), (1290, 32, "plain"), (1801, 32, "plain"),
+    (200, 64, "plain"), (333, 64, "plain"), (514, 64, "plain"), (901, 64, "precise"),
+    (131, 32, "dropout"), (300, 32, "dropout"), (514, 32, "dropout"), (202, 64, "dropout"), (514, 64, "dropout"),
 ]
 
 
@@ -157,7 +162,7 @@ def test_queries_whose_keys_are_all_masked_attend_by_their_scores(L2, D, mode, m
     if mode == "precise" and dtype == torch.bfloat16:
         pytest.skip("a mode of fp16")
     B, H, L1, sm = 1, 2, 3, 1.0 / math.sqrt(D)
-    rows = [0, 7, L2 - 1]
+    rows = sorted({0, 7 % L2, L2 - 1})
     q, k, v, b, do = _inputs(B, H, L1, L2, D, 3, dtype)
     low = float("-inf") if mask == "-inf" else torch.finfo(dtype).min
     b[..., L2 // 2:L2 // 2 + 5] = low
