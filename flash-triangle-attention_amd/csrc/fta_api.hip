@@ -119,8 +119,8 @@ struct PlanKey {
 // The length the tiles of one direction cover for rows of L2 keys: the smallest multiple of 128 (forward: 64) that is at
 // least L2 and that the direction has a workgroup shape for (0 if there is none up to FTA_MAX_L2).  The
 // two directions need not agree (nothing they exchange is laid out by it: lse has the row's true length):
-// the backward has a shape for every multiple of 128, the forward skips a few (D = 32: 11 and 25 blocks
-// of 128 keys; D = 64: odd numbers of blocks from 5 on), and a row is only supported where both have one.
+// the backward has a shape for every multiple of 128, the forward skips a few (D = 32: from 1792 keys on,
+// the first 17 blocks of 128; D = 64: 11 and 13 blocks), and a row is only supported where both have one.
 // (`feat`: 1 for the backward's vector-ALU instances, 2 for dropout, which has fewer instances in both
 // directions)
 int padded_len_fwd(int L2, int D, int feat) {
@@ -311,9 +311,9 @@ const char* fta_strerror(int status) {
     case FTA_ERR_NULL_POINTER: return "null pointer argument";
     case FTA_ERR_MISALIGNED: return "pointer is not 16-byte aligned";
     case FTA_ERR_HEAD_DIM: return "head dimension must be 32 or 64";
-    case FTA_ERR_SEQ_LEN: return "L2 must be a multiple of 4 within the range built for this head dim (fta_seq_len_supported) and L1 >= 1";
+    case FTA_ERR_SEQ_LEN: return "L2 must be within the range built for this head dim (fta_seq_len_supported) and L1 >= 1";
     case FTA_ERR_BATCH: return "B and H must be >= 1";
-    case FTA_ERR_STRIDE: return "stride is negative, not a multiple of 8 elements (4 for bias), makes an output overlap itself, or puts the rows of a slice more than 4 GiB apart";
+    case FTA_ERR_STRIDE: return "stride is negative, not a multiple of 8 elements (5-D tensors), makes an output overlap itself, or puts the rows of a slice more than 4 GiB apart";
     case FTA_ERR_WORKSPACE: return "workspace is smaller than fta_bwd_workspace_bytes()";
     case FTA_ERR_SCALE: return "sm_scale is not finite";
     case FTA_ERR_NO_DEVICE: return "no usable gfx950 device";

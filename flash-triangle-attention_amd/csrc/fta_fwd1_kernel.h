@@ -37,7 +37,8 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // S: key slabs.  Rows beyond 512 keys do not fit one wave's bias registers: S = 2 or 4 waves of an eight-wave workgroup
 // take the keys of one query block in slabs of 32*NKT and merge their (m, l, O) through LDS, in fp32, once per row:
 // every slab finishes 16/S of the accumulator registers.  A stage then holds 64 keys of every slab.
-// (B1 H4 L701 bf16: 596 -> 515 us, B1 H4 L1536 fp16: 5180 -> 4300 us against the general kernel)
+// (against the general kernel, rocprofv3, middle half of 60 launches: B1 H4 L701 bf16 656 -> 466 us, B1 H4 L1536 fp16
+// 5200 -> 4100)
 template <class T, int NKT, bool TAIL, int W, int G = 4, int S = 1>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_waves_per_eu(2, 2))) fta_fwd1_kernel(const FwdParams p) {
   static_assert(W == 2 || W == 4 || W == 8, "one or two waves per SIMD from the same workgroup (rows of up to 64 keys: two waves)");

@@ -81,9 +81,10 @@ class TriangleAttention(nn.Module):
         return out if self.starting else out.transpose(1, 2)
 
     def _fused(self, z, key_mask, seed):
-        """The whole block in the kernels of csrc/fta_block.hip (three launches forward, eleven backward), for
-        plain fp16, bf16 or fp32 modules of the sizes built there; None where this does not apply: other
-        sizes, autocast, mixed types, hooked, parametrised or replaced submodules, a subclass."""
+        """The whole block in the kernels of csrc/fta_block.hip (three launches forward, eight backward), for
+        plain fp16, bf16 or fp32 modules of the sizes built there (c_z and n_heads * c_hidden of 64 or 128);
+        None where this does not apply: other sizes, autocast, mixed types, a call that something traces
+        or transforms, hooked, parametrised, wrapped or replaced submodules, a subclass."""
         if type(self) is not TriangleAttention or not z.is_cuda or _has_any_global_hook():
             return None
         native = fta_lib.native()

@@ -35,8 +35,9 @@
  *     its scores alone, in the output and in the gradients, as it does upstream with a finite mask value
  *     (with -inf upstream returns NaN); where all of a query's biases lie between -59904 and -41589 those
  *     kernels give it no gradients.  bf16 entries beyond +65504 are taken as 65504 by the hand-scheduled
- *     forward kernels (D = 32 up to 1792 keys, D = 64 from 129 to 512; not with dropout).  +inf and NaN entries
- *     are not supported.
+ *     forward kernels (D = 32 up to 1792 keys, D = 64 from 129 to 512; not with dropout).  Entries above
+ *     60000/log2(e) = 41588 leave the range in which the hand-scheduled backward holds bias * log2(e): not supported
+ *     there, nor are +inf and NaN anywhere.
  *   - The library never allocates, frees or keeps pointers.  Outputs are fully overwritten.
  *     Launches are asynchronous on `stream` (a hipStream_t; NULL = the default stream).
  *   - Return value: 0 on success; a negative fta_status for an argument error (detected on

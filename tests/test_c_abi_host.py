@@ -199,7 +199,7 @@ def test_plan_description_with_options_names_the_kernels_that_run():
     assert "dq1" not in wide["dq"]["kernel"] and "dkdv1" not in wide["dkdv"]["kernel"]
     assert fta_lib.describe_plan(2, 8, 512, 512, 64, 0.125, bf16)["options"]["precise_or_vector_alu_backward"] == 0
     # the precise mode of fp16: at D = 32 the hand-scheduled kernels' instances with the operand pair and the
-    # exponent in natural units, at D = 64 and for short rows the vector-ALU backward
+    # exponent in natural units, at D = 64 and for short rows a backward on the vector ALU
     precise = fta_lib.Options(fta_lib.DTYPE_F16, 0, 0.0, 0, 1)
     p32 = fta_lib.describe_plan(4, 8, 512, 512, 32, 1.3, precise)
     assert p32["options"] == {"type": "F16", "dropout": 0, "precise_or_vector_alu_backward": 0, "scaled_operand_pair": 1, "natural_exponent": 1}

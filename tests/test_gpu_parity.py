@@ -198,8 +198,8 @@ def general_kernels():
 
 
 def test_general_backward_kernels(general_kernels):
-    # The pipelined one-wave-per-SIMD backward kernels cover every tiled length from 256 on at D=32; the
-    # general kernels otherwise only run for shorter rows, D=64 dK/dV and the feature paths.
+    # fp16 rows run the one-kernel backward (up to 128 keys) or the pipelined one-wave-per-SIMD kernels; the general
+    # kernels otherwise only run with dropout and, at D=64, for bf16 at large scales and the precise mode.
     import fta_lib
     assert "dq1" not in fta_lib.describe_plan(1, 2, 24, 512, 32)["dq"]["kernel"]
     assert "dkdv1" not in fta_lib.describe_plan(1, 2, 24, 512, 32)["dkdv"]["kernel"]
