@@ -11,6 +11,7 @@
 #include <torch/extension.h>
 
 #include <atomic>
+#include <unordered_set>
 
 #include "fta.h"
 
@@ -91,6 +92,13 @@ bool length_supported(int64_t L2, int64_t D, const fta_options& o) {
   return v == 2;
 }
 
+// The globals of the Python module a call came from, for its backward.  One reference per module is kept for good: the
+// backward may run after the module itself is gone.  (Called under the interpreter lock.)
+int64_t held(py::dict globals) {
+  static std::unordered_set<PyObject*> kept;
+  if (kept.insert(globals.ptr()).second) globals.inc_ref();
+  return (int64_t) reinterpret_cast<intptr_t>(globals.ptr());
+}
 // The module switch PRECISE_BACKWARD of the Python module whose globals these are, at this moment.
 bool precise_now(PyObject* globals) {
   py::gil_scoped_acquire gil;
@@ -171,7 +179,7 @@ py::object attention(py::handle qh, py::handle kh, py::handle vh, py::handle bh,
     if (attention_forward(q, k, v, b, scale, opt, o, lse) != FTA_OK) return none;
     return py::cast(o);
   }
-  return py::cast(Attention::apply(q, k, v, b, scale, dropout_p, seed, (int64_t) reinterpret_cast<intptr_t>(globals.ptr())));
+  return py::cast(Attention::apply(q, k, v, b, scale, dropout_p, seed, held(globals)));
 }
 
 // ---- the block -----------------------------------------------------------------------------------------
@@ -308,7 +316,7 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
   }
   auto opt_t = [](const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
   return py::cast(Block::apply(z, opt_t(mask), w[0], w[1], w[2], w[3], w[4], w[5], w[6], opt_t(w[7]), w[8], opt_t(w[9]), c.C, H, D, c.seed,
-                               c.starting, eps, dropout_p, (int64_t) reinterpret_cast<intptr_t>(globals.ptr())));
+                               c.starting, eps, dropout_p, held(globals)));
 }
 
 }  // namespace

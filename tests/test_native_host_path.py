@@ -251,3 +251,22 @@ def test_the_build_follows_the_torch_at_hand(monkeypatch):
     assert build.native_commands("hipcc", "x.o") is None
     monkeypatch.setattr(build, "NATIVE", "/nowhere/fta_native.so")
     assert build.needs_build() <= before  # without torch its absence is no reason to build
+
+
+@gpu
+def test_the_backward_outlives_the_module_it_came_from():
+    import gc
+    import importlib.util
+    import os
+    import fta_lib
+    import flash_tt_attn
+    q, k, v, b, dout = _operands(1)
+    q.requires_grad_(True)
+    spec = importlib.util.spec_from_file_location("fta_module_to_drop", os.path.join(fta_lib.HERE, "flash_tt_attn.py"))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    o = mod.attention(q, k, v, b, 0.3)
+    del mod, spec
+    gc.collect()
+    got, = torch.autograd.grad(o, q, dout)
+    assert torch.equal(got, torch.autograd.grad(flash_tt_attn.attention(q, k, v, b, 0.3), q, dout)[0])
