@@ -69,6 +69,12 @@ fta_tensor4 t4(const Tensor& t) {
 void check(int rc) {
   TORCH_CHECK(rc == FTA_OK, "libfta: ", fta_strerror(rc), " (status ", rc, ")");
 }
+// A forward call whose arguments the library refused (before any launch): left to the Python path, which raises its errors.
+struct Refused {};
+void check_forward(int rc) {
+  if (rc < 0) throw Refused{};
+  check(rc);
+}
 
 fta_options make_options(at::ScalarType dtype, double dropout_p, uint64_t seed, bool precise) {
   fta_options o{};
@@ -123,7 +129,7 @@ struct Attention : public torch::autograd::Function<Attention> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, double scale,
                         double dropout_p, int64_t seed, int64_t globals) {
     Tensor o, lse;
-    check(attention_forward(q, k, v, b, scale, make_options(q.scalar_type(), dropout_p, (uint64_t)seed, false), o, lse));
+    check_forward(attention_forward(q, k, v, b, scale, make_options(q.scalar_type(), dropout_p, (uint64_t)seed, false), o, lse));
     ctx->save_for_backward({q, k, v, o, b, lse});
     ctx->saved_data["scale"] = scale;
     ctx->saved_data["dropout_p"] = dropout_p;
@@ -173,13 +179,17 @@ py::object attention(py::handle qh, py::handle kh, py::handle vh, py::handle bh,
   if (!readable(q) || !readable(k) || !readable(v) || b.stride(3) != 1) return none;
   const fta_options opt = make_options(dt, dropout_p, (uint64_t)seed, false);
   if (!length_supported(n[3], n[4], opt)) return none;
-  if (!wants_grad({&q, &k, &v, &b})) {
-    Tensor o, lse;
-    at::AutoDispatchBelowADInplaceOrView below;
-    if (attention_forward(q, k, v, b, scale, opt, o, lse) != FTA_OK) return none;
-    return py::cast(o);
+  try {
+    if (!wants_grad({&q, &k, &v, &b})) {
+      Tensor o, lse;
+      at::AutoDispatchBelowADInplaceOrView below;
+      check_forward(attention_forward(q, k, v, b, scale, opt, o, lse));
+      return py::cast(o);
+    }
+    return py::cast(Attention::apply(q, k, v, b, scale, dropout_p, seed, held(globals)));
+  } catch (const Refused&) {
+    return none;
   }
-  return py::cast(Attention::apply(q, k, v, b, scale, dropout_p, seed, held(globals)));
 }
 
 // ---- the block -----------------------------------------------------------------------------------------
@@ -229,7 +239,7 @@ struct Block : public torch::autograd::Function<Block> {
     const Tensor m = mask.value_or(Tensor());
     const BlockCall c{C, H, D, seed, starting, eps, dropout_p};
     Tensor out, state;
-    check(block_forward(z, block_args(z, m, w, c, false), starting, out, state));
+    check_forward(block_forward(z, block_args(z, m, w, c, false), starting, out, state));
     variable_list keep{z, m, state};
     for (const Tensor& t : w) keep.push_back(t);
     ctx->save_for_backward(keep);
@@ -308,15 +318,19 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
     c.seed = py::cast<int64_t>(globals["_draw_seed"]());
     b.seed = (uint64_t)c.seed;
   }
-  if (!wants_grad({&z, &w[0], &w[1], &w[2], &w[3], &w[4], &w[5], &w[6], &w[7], &w[8], &w[9]})) {
-    Tensor out, state;
-    at::AutoDispatchBelowADInplaceOrView below;
-    check(block_forward(z, b, c.starting, out, state));
-    return py::cast(out);
-  }
   auto opt_t = [](const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; };
-  return py::cast(Block::apply(z, opt_t(mask), w[0], w[1], w[2], w[3], w[4], w[5], w[6], opt_t(w[7]), w[8], opt_t(w[9]), c.C, H, D, c.seed,
-                               c.starting, eps, dropout_p, held(globals)));
+  try {
+    if (!wants_grad({&z, &w[0], &w[1], &w[2], &w[3], &w[4], &w[5], &w[6], &w[7], &w[8], &w[9]})) {
+      Tensor out, state;
+      at::AutoDispatchBelowADInplaceOrView below;
+      check_forward(block_forward(z, b, c.starting, out, state));
+      return py::cast(out);
+    }
+    return py::cast(Block::apply(z, opt_t(mask), w[0], w[1], w[2], w[3], w[4], w[5], w[6], opt_t(w[7]), w[8], opt_t(w[9]), c.C, H, D, c.seed,
+                                 c.starting, eps, dropout_p, held(globals)));
+  } catch (const Refused&) {
+    return none;
+  }
 }
 
 }  // namespace

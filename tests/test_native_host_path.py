@@ -270,3 +270,15 @@ def test_the_backward_outlives_the_module_it_came_from():
     gc.collect()
     got, = torch.autograd.grad(o, q, dout)
     assert torch.equal(got, torch.autograd.grad(flash_tt_attn.attention(q, k, v, b, 0.3), q, dout)[0])
+
+
+@gpu
+@pytest.mark.parametrize("grad", [False, True])
+def test_arguments_the_library_refuses_raise_its_error_with_and_without_grad(grad):
+    import fta_lib
+    from flash_tt_attn import attention
+    x = list(_operands(1)[:4])
+    x[0].requires_grad_(grad)
+    with pytest.raises(fta_lib.FtaError) as e:
+        attention(*x, float("inf"))
+    assert e.value.status == -8  # (the scale)
