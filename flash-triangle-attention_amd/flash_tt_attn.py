@@ -150,6 +150,12 @@ def _load_native():
 
 
 class _attention(torch.autograd.Function):
+    def __init_subclass__(cls, **kwargs):
+        """A subclass has the autograd machinery's own apply(), which runs the subclass's forward and backward."""
+        super().__init_subclass__(**kwargs)
+        if "apply" not in cls.__dict__:
+            cls.apply = classmethod(torch.autograd.Function.apply.__func__)
+
     @staticmethod
     def apply(*args):
         """The operator.  Tensors that the kernels read in place go through the C++ host path (an autograd

@@ -282,3 +282,20 @@ def test_arguments_the_library_refuses_raise_its_error_with_and_without_grad(gra
     with pytest.raises(fta_lib.FtaError) as e:
         attention(*x, float("inf"))
     assert e.value.status == -8  # (the scale)
+
+
+def test_a_subclass_of_the_function_runs_its_own_forward_and_backward():
+    import flash_tt_attn as fta
+
+    class Scaled(fta._attention):
+        @staticmethod
+        def forward(ctx, q, factor):
+            ctx.factor = factor
+            return q * factor
+
+        @staticmethod
+        def backward(ctx, do):
+            return do * ctx.factor, None
+    q = torch.ones(2, 3, requires_grad=True)
+    out = Scaled.apply(q, 3.0)
+    assert torch.equal(out, 3.0 * q) and torch.equal(torch.autograd.grad(out.sum(), q)[0], torch.full_like(q, 3.0))
