@@ -31,6 +31,9 @@ bool readable(const Tensor& t) {
     if (s[i] % 8 != 0) return false;
   return true;
 }
+// t if the kernels read it in place, else a copy of its own (contiguous() would leave a dense tensor off the 16-byte
+// boundary where it is: a gradient that the backward of a concatenation cut out, for instance).
+Tensor readable_copy(const Tensor& t) { return readable(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
 // A plain tensor on the current GPU: no subclass or transform that has to see the operations, and no tangent (the
 // operator has no forward-mode derivative: the Python function says so, here the output would come without one).
 bool plain(const Tensor& t, int device) {
@@ -140,9 +143,8 @@ struct Attention : public torch::autograd::Function<Attention> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
     const Tensor &q = s[0], &k = s[1], &v = s[2], &o = s[3], &b = s[4], &lse = s[5];
-    Tensor dout = grads[0];
-    TORCH_CHECK(dout.scalar_type() == q.scalar_type(), "the gradient has another type than the output");
-    if (!readable(dout)) dout = dout.contiguous();
+    TORCH_CHECK(grads[0].scalar_type() == q.scalar_type(), "the gradient has another type than the output");
+    const Tensor dout = readable_copy(grads[0]);
     c10::OptionalDeviceGuard guard(q.device());
     const fta_options opt = make_options(q.scalar_type(), ctx->saved_data["dropout_p"].toDouble(),
                                          (uint64_t)ctx->saved_data["seed"].toInt(),
@@ -253,8 +255,7 @@ struct Block : public torch::autograd::Function<Block> {
     const auto d = ctx->saved_data["d"].toDoubleVector();
     const BlockCall c{i[0], i[1], i[2], i[3], i[4], d[0], d[1]};
     const Tensor &z = s[0], &state = s[2];
-    Tensor dout = grads[0];
-    if (!readable(dout)) dout = dout.contiguous();
+    const Tensor dout = readable_copy(grads[0]);
     c10::OptionalDeviceGuard guard(z.device());
     const fta_block b = block_args(z, s[1], &s[3], c, precise_now(reinterpret_cast<PyObject*>(i[5])));
     Tensor dz = at::empty_like(z), dw[10];

@@ -243,8 +243,10 @@ class _attention(torch.autograd.Function):
         B, H, L1, L2, D = q.shape
         lib = fta_lib.load()
 
-        # upstream asserts a contiguous `do` with q's strides (:604-606); here any layout is taken
+        # upstream asserts a contiguous `do` with q's strides (:604-606); here any layout and alignment is taken
         do = _dense5(do)
+        if do.data_ptr() % 16 != 0:
+            do = do.clone(memory_format=torch.contiguous_format)
         dq = torch.empty_like(q)
         dk = torch.empty_like(k)
         dv = torch.empty_like(v)

@@ -299,3 +299,21 @@ def test_a_subclass_of_the_function_runs_its_own_forward_and_backward():
     q = torch.ones(2, 3, requires_grad=True)
     out = Scaled.apply(q, 3.0)
     assert torch.equal(out, 3.0 * q) and torch.equal(torch.autograd.grad(out.sum(), q)[0], torch.full_like(q, 3.0))
+
+
+@gpu
+@pytest.mark.parametrize("which", ["attention", "python path", "block"])
+def test_gradients_may_start_off_a_16_byte_boundary(which, monkeypatch):
+    """(what the backward of a concatenation hands on, for instance)"""
+    import flash_tt_attn as fta
+    if which == "python path":
+        monkeypatch.setattr(fta, "_native", lambda *a, **kw: None)
+    *x, dout = _operands(1)
+    run = lambda: fta.attention(*x, 0.3)
+    if which == "block":
+        blk, x, dout = _block(), [_pair(1)], _pair(2)
+        run = lambda: blk(x[0])
+    x[0].requires_grad_(True)
+    off = torch.empty(dout.numel() + 3, dtype=dout.dtype, device=DEV)[3:].view(dout.shape).copy_(dout)
+    assert off.data_ptr() % 16 != 0
+    assert torch.equal(*(torch.autograd.grad(run(), x[0], g)[0] for g in (off, dout)))
