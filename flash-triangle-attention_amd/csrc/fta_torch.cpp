@@ -34,6 +34,17 @@ bool readable(const Tensor& t) {
 // t if the kernels read it in place, else a copy of its own (contiguous() would leave a dense tensor off the 16-byte
 // boundary where it is: a gradient that the backward of a concatenation cut out, for instance).
 Tensor readable_copy(const Tensor& t) { return readable(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
+Tensor packed_copy(const Tensor& t) {
+  return t.is_contiguous() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0 ? t : t.clone(at::MemoryFormat::Contiguous);
+}
+// A tensor saved in the forward.  Hooks may have packed it and may return it with other strides, which the copies above
+// take; another tensor than they were given (kept in fewer bits, left on the host) must not reach a kernel, which
+// reads it by the sizes of the call.
+const Tensor& saved(const Tensor& t, at::IntArrayRef sizes, at::ScalarType dtype, const at::Device& device) {
+  TORCH_CHECK(t.defined() && t.layout() == at::kStrided && t.device() == device && t.scalar_type() == dtype && t.sizes() == sizes,
+              "a hook for saved tensors returned a tensor of another type, device or size than it was given");
+  return t;
+}
 // A plain tensor on the current GPU: no subclass or transform that has to see the operations, and no tangent (the
 // operator has no forward-mode derivative: the Python function says so, here the output would come without one).
 bool plain(const Tensor& t, int device) {
@@ -141,15 +152,21 @@ struct Attention : public torch::autograd::Function<Attention> {
     return o;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    at::NoGradGuard no_grad;
     const variable_list s = ctx->get_saved_variables();
-    const Tensor &q = s[0], &k = s[1], &v = s[2], &o = s[3], &b = s[4], &lse = s[5];
-    TORCH_CHECK(grads[0].scalar_type() == q.scalar_type(), "the gradient has another type than the output");
-    const Tensor dout = readable_copy(grads[0]);
-    c10::OptionalDeviceGuard guard(q.device());
+    const Tensor dout = readable_copy(grads[0]);  // (of the output's type, sizes and device: the engine sees to that)
+    const at::Device dev = dout.device();
+    const at::ScalarType dt = dout.scalar_type();
+    c10::OptionalDeviceGuard guard(dev);
+    const auto n = dout.sizes();
+    const Tensor q = readable_copy(saved(s[0], n, dt, dev)), k = readable_copy(saved(s[1], n, dt, dev)),
+                 v = readable_copy(saved(s[2], n, dt, dev)), o = readable_copy(saved(s[3], n, dt, dev)),
+                 lse = packed_copy(saved(s[5], n.slice(0, 4), at::kFloat, dev));
+    Tensor b = saved(s[4], {n[0], n[1], n[3], n[3]}, dt, dev);
+    if (b.stride(3) != 1) b = b.contiguous();
     const fta_options opt = make_options(q.scalar_type(), ctx->saved_data["dropout_p"].toDouble(),
                                          (uint64_t)ctx->saved_data["seed"].toInt(),
                                          precise_now(reinterpret_cast<PyObject*>(ctx->saved_data["globals"].toInt())));
-    const auto n = q.sizes();
     const int B = (int)n[0], H = (int)n[1], L1 = (int)n[2], L2 = (int)n[3], D = (int)n[4];
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), db = at::empty_like(b);
     const size_t bytes = fta_bwd_workspace_bytes_ex(B, H, L1, L2, D, &opt);
@@ -200,7 +217,18 @@ struct BlockCall {
   double eps, dropout_p;
 };
 
-// weights: norm weight, norm bias, q, k, v, b, gate weight, gate bias, output weight, output bias
+// The sizes of the weights: norm weight, norm bias, q, k, v, b, gate weight, gate bias, output weight, output bias.
+struct WeightSizes {
+  int64_t rows[10], cols[10];
+  explicit WeightSizes(const BlockCall& c)
+      : rows{c.C, c.C, c.H * c.D, c.H * c.D, c.H * c.D, c.H, c.H * c.D, c.H * c.D, c.C, c.C},
+        cols{0, 0, c.C, c.C, c.C, c.C, c.C, 0, c.H * c.D, 0} {}
+  c10::SmallVector<int64_t, 2> operator[](int n) const {
+    return cols[n] ? c10::SmallVector<int64_t, 2>{rows[n], cols[n]} : c10::SmallVector<int64_t, 2>{rows[n]};
+  }
+};
+
+// weights in that order
 fta_block block_args(const Tensor& z, const Tensor& mask, const Tensor* w, const BlockCall& c, bool precise) {
   fta_block b{};
   b.B = (int)z.size(0); b.L = (int)z.size(1); b.C = (int)c.C; b.H = (int)c.H; b.D = (int)c.D;
@@ -250,14 +278,23 @@ struct Block : public torch::autograd::Function<Block> {
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    at::NoGradGuard no_grad;
     const variable_list s = ctx->get_saved_variables();
     const auto i = ctx->saved_data["i"].toIntVector();
     const auto d = ctx->saved_data["d"].toDoubleVector();
     const BlockCall c{i[0], i[1], i[2], i[3], i[4], d[0], d[1]};
-    const Tensor &z = s[0], &state = s[2];
     const Tensor dout = readable_copy(grads[0]);
-    c10::OptionalDeviceGuard guard(z.device());
-    const fta_block b = block_args(z, s[1], &s[3], c, precise_now(reinterpret_cast<PyObject*>(i[5])));
+    const at::Device dev = dout.device();
+    const at::ScalarType dt = dout.scalar_type();
+    c10::OptionalDeviceGuard guard(dev);
+    const Tensor z = readable_copy(saved(s[0], dout.sizes(), dt, dev));
+    const Tensor mask = s[1].defined() ? packed_copy(saved(s[1], {z.size(0), z.size(1)}, dt, dev)) : Tensor();
+    const WeightSizes sizes(c);
+    Tensor w[10];
+    for (int n = 0; n < 10; ++n)
+      if (s[3 + n].defined()) w[n] = packed_copy(saved(s[3 + n], sizes[n], dt, dev));
+    const fta_block b = block_args(z, mask, w, c, precise_now(reinterpret_cast<PyObject*>(i[5])));
+    const Tensor state = packed_copy(saved(s[2], {(int64_t)fta_block_state_bytes(&b)}, at::kByte, dev));
     Tensor dz = at::empty_like(z), dw[10];
     if (!readable(dz)) dz = at::empty(z.sizes(), z.options());
     fta_block_grads g{};
@@ -265,8 +302,8 @@ struct Block : public torch::autograd::Function<Block> {
     node_strides(dz, c.starting, g.z_stride);
     void** dst[10] = {&g.norm_weight, &g.norm_bias, &g.wq, &g.wk, &g.wv, &g.wb, &g.wg, &g.bg, &g.wo, &g.bo};
     for (int n = 0; n < 10; ++n)
-      if (s[3 + n].defined()) {
-        dw[n] = at::empty(s[3 + n].sizes(), s[3 + n].options());
+      if (w[n].defined()) {
+        dw[n] = at::empty(w[n].sizes(), w[n].options());
         *dst[n] = dw[n].data_ptr();
       }
     const size_t bytes = fta_block_bwd_workspace_bytes(&b);
@@ -293,7 +330,7 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
   const int dev = (int)c10::hip::current_device();
   BlockCall c{z.size(3), H, D, given_seed.value_or(0), starting ? 1 : 0, eps, dropout_p};
   if (!plain(z, dev) || !readable(z) || !(dropout_p >= 0.0 && dropout_p < 1.0)) return none;
-  const int64_t HD = H * D, rows[10] = {c.C, c.C, HD, HD, HD, H, HD, HD, c.C, c.C}, cols[10] = {0, 0, c.C, c.C, c.C, c.C, c.C, 0, HD, 0};
+  const WeightSizes sizes(c);
   Tensor w[10];
   for (int n = 0; n < 10; ++n) {
     if (weights[n].is_none()) {
@@ -304,7 +341,7 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
     w[n] = THPVariable_Unpack(weights[n].ptr());
     if (w[n].scalar_type() != dt || !plain(w[n], dev) || !w[n].is_contiguous() || reinterpret_cast<uintptr_t>(w[n].data_ptr()) % 16 != 0)
       return none;
-    if (w[n].dim() != (cols[n] ? 2 : 1) || w[n].size(0) != rows[n] || (cols[n] && w[n].size(1) != cols[n])) return none;
+    if (w[n].sizes() != at::IntArrayRef(sizes[n])) return none;
   }
   Tensor mask;
   if (key_mask.has_value()) {

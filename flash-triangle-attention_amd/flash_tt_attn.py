@@ -240,7 +240,14 @@ class _attention(torch.autograd.Function):
         dtype = ctx.dtype
         assert do.dtype == dtype
         q, k, v, o, b_pw, logsumexp = ctx.saved_tensors
-        B, H, L1, L2, D = q.shape
+        B, H, L1, L2, D = do.shape
+        # (hooks for saved tensors may return them with other strides; another tensor than they were given must not reach
+        # a kernel, which reads it by these sizes)
+        for t, shape, kind in ((q, do.shape, dtype), (k, do.shape, dtype), (v, do.shape, dtype), (o, do.shape, dtype),
+                               (b_pw, (B, H, L2, L2), dtype), (logsumexp, (B, H, L1, L2), torch.float32)):
+            if t.device != do.device or t.dtype != kind or tuple(t.shape) != tuple(shape):
+                raise RuntimeError("a hook for saved tensors returned a tensor of another type, device or size than it was given")
+        q, k, v, o, b_pw, logsumexp = *map(_dense5, (q, k, v, o)), _dense4(b_pw), logsumexp.contiguous()
         lib = fta_lib.load()
 
         # upstream asserts a contiguous `do` with q's strides (:604-606); here any layout and alignment is taken

@@ -317,3 +317,55 @@ def test_gradients_may_start_off_a_16_byte_boundary(which, monkeypatch):
     off = torch.empty(dout.numel() + 3, dtype=dout.dtype, device=DEV)[3:].view(dout.shape).copy_(dout)
     assert off.data_ptr() % 16 != 0
     assert torch.equal(*(torch.autograd.grad(run(), x[0], g)[0] for g in (off, dout)))
+
+
+def _transposing_hooks():
+    """Saved tensors packed with their last two dimensions in the other order: the same values come back with other strides."""
+    return torch.autograd.graph.saved_tensors_hooks(lambda t: t.mT.contiguous().mT if t.dim() > 1 else t, lambda t: t)
+
+
+@gpu
+@pytest.mark.parametrize("which", ["attention", "python path", "block"])
+def test_tensors_saved_for_the_backward_may_come_back_in_another_layout(which, monkeypatch):
+    import flash_tt_attn as fta
+    if which == "python path":
+        monkeypatch.setattr(fta, "_native", lambda *a, **kw: None)
+    if which == "block":
+        blk, z = _block(), _pair(1).requires_grad_(True)
+        run, inputs, dout = lambda: blk(z, torch.ones(1, 48, device=DEV)), [z, *blk.parameters()], _pair(2)
+    else:
+        *x, dout = _operands(1)
+        inputs = [t.requires_grad_(True) for t in x]
+        run = lambda: fta.attention(*x, 0.3)
+    want = torch.autograd.grad(run(), inputs, dout)
+    with _transposing_hooks():
+        got = torch.autograd.grad(run(), inputs, dout)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+_OTHER = {"type": lambda t: t.to(torch.float8_e5m2 if t.dtype != torch.uint8 else torch.int8), "device": lambda t: t.cpu(),
+          "size": lambda t: t.flatten()[:1].clone()}
+
+
+@gpu
+@pytest.mark.parametrize("other", sorted(_OTHER))
+@pytest.mark.parametrize("nth", range(13))
+@pytest.mark.parametrize("which", ["attention", "python path", "block"])
+def test_saved_tensors_that_come_back_as_others_are_refused(which, nth, other, monkeypatch):
+    """One of them at a time, on the host: before anything is launched."""
+    import flash_tt_attn as fta
+    if which == "python path":
+        monkeypatch.setattr(fta, "_native", lambda *a, **kw: None)
+    blk, z, count = _block(), _pair(1), [0]
+    *x, dout = _operands(1)
+    x[0].requires_grad_(True)
+
+    def pack(t):
+        count[0] += 1
+        return _OTHER[other](t.detach()) if count[0] == nth + 1 else t
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        out = blk(z, torch.ones(1, 48, device=DEV)) if which == "block" else fta.attention(*x, 0.3)
+    assert count[0] == (13 if which == "block" else 6)
+    if nth < count[0]:
+        with pytest.raises(RuntimeError, match="hook for saved tensors"):
+            out.backward(torch.ones_like(out))
