@@ -25,6 +25,8 @@ import math
 import torch
 from torch import nn
 from torch.nn.modules.module import _has_any_global_hook
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 import fta_lib
 from flash_tt_attn import _attention, attention, reference_tt_attn
@@ -40,6 +42,12 @@ _KEY_MASK_BIAS = -30000.0
 _SUBMODULES = (("layer_norm", nn.LayerNorm, True), ("linear_q", nn.Linear, False), ("linear_k", nn.Linear, False),
                ("linear_v", nn.Linear, False), ("linear_b", nn.Linear, False), ("linear_g", nn.Linear, True),
                ("linear_o", nn.Linear, True))
+
+
+def _function_mode_on() -> bool:
+    """Whether a mode sees or rewrites the calls of torch functions (torch.device as a context or the default device is
+    one, too, but only says where new tensors go)."""
+    return torch._C._len_torch_function_stack() > 0 and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack())
 
 
 class TriangleAttention(nn.Module):
@@ -85,7 +93,7 @@ class TriangleAttention(nn.Module):
         plain fp16, bf16 or fp32 modules of the sizes built there (c_z and n_heads * c_hidden of 64 or 128);
         None where this does not apply: other sizes, autocast, mixed types, a call that something traces
         or transforms, hooked, parametrised, wrapped or replaced submodules, a subclass."""
-        if type(self) is not TriangleAttention or not z.is_cuda or _has_any_global_hook():
+        if type(self) is not TriangleAttention or not z.is_cuda or _has_any_global_hook() or _function_mode_on():
             return None
         native = fta_lib.native()
         if native is None:

@@ -369,3 +369,19 @@ def test_saved_tensors_that_come_back_as_others_are_refused(which, nth, other, m
     if nth < count[0]:
         with pytest.raises(RuntimeError, match="hook for saved tensors"):
             out.backward(torch.ones_like(out))
+
+
+@gpu
+def test_a_function_mode_sees_the_layers_of_the_block():
+    from torch.overrides import TorchFunctionMode
+
+    class Log(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    blk, z, seen = _block(), _pair(1), []
+    with Log(), torch.no_grad():
+        blk(z)
+    assert torch.nn.functional.linear in seen
+    with torch.device(DEV):  # (says where new tensors go: nothing the fused path hides from it)
+        assert blk._fused(z, None, None) is not None
