@@ -318,7 +318,7 @@ struct Block : public torch::autograd::Function<Block> {
   }
 };
 
-py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std::vector<py::object>& weights, int64_t H, int64_t D,
+py::object block(py::handle zh, py::handle key_mask, const std::vector<py::object>& weights, int64_t H, int64_t D,
                  bool starting, double eps, double dropout_p, std::optional<int64_t> given_seed, py::dict globals) {
   const py::object none = py::none();
   if (!exact_tensor(zh)) return none;
@@ -344,11 +344,11 @@ py::object block(py::handle zh, const std::optional<Tensor>& key_mask, const std
     if (w[n].sizes() != at::IntArrayRef(sizes[n])) return none;
   }
   Tensor mask;
-  if (key_mask.has_value()) {
-    if (key_mask->requires_grad() || !plain(*key_mask, dev) || key_mask->dim() != 2 || key_mask->size(0) != z.size(0) ||
-        key_mask->size(1) != z.size(1))
-      return none;
-    mask = key_mask->to(dt).contiguous();
+  if (!key_mask.is_none()) {
+    if (!exact_tensor(key_mask)) return none;
+    const Tensor& m = THPVariable_Unpack(key_mask.ptr());
+    if (m.requires_grad() || !plain(m, dev) || m.dim() != 2 || m.size(0) != z.size(0) || m.size(1) != z.size(1)) return none;
+    mask = m.to(dt).contiguous();
   }
   fta_block b = block_args(z, mask, w, c, false);
   if (!length_supported(b.L, D, make_options(dt, dropout_p, 0, false)) || fta_block_check(&b) != FTA_OK) return none;

@@ -120,7 +120,7 @@ class TriangleAttention(nn.Module):
         try:
             return native.block(z, key_mask, weights, self.n_heads, self.c_hidden, self.starting, norm.eps, p,
                                 seed if p > 0.0 else 0, scope)  # (no seed: one is drawn if the call is taken)
-        except TypeError:  # (a seed beyond 63 bits, a mask that is no tensor)
+        except TypeError:  # (a seed beyond 63 bits)
             return None
 
     def forward(self, z: torch.Tensor, key_mask: torch.Tensor | None = None, seed: int | None = None) -> torch.Tensor:

@@ -385,3 +385,12 @@ def test_a_function_mode_sees_the_layers_of_the_block():
     assert torch.nn.functional.linear in seen
     with torch.device(DEV):  # (says where new tensors go: nothing the fused path hides from it)
         assert blk._fused(z, None, None) is not None
+
+
+@gpu
+def test_a_mask_of_a_subclass_goes_to_the_separate_layers():
+    class Sub(torch.Tensor):
+        pass
+    blk, z, mask = _block(), _pair(1), torch.ones(1, 48, device=DEV)
+    assert blk._fused(z, mask, None) is not None and type(blk(z, mask)) is torch.Tensor
+    assert blk._fused(z, mask.as_subclass(Sub), None) is None
