@@ -7,6 +7,7 @@
 #include <ATen/autocast_mode.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
@@ -260,6 +261,16 @@ int block_forward(const Tensor& z, const fta_block& b, int64_t starting, Tensor&
   return fta_block_fwd(&b, out.data_ptr(), os, state.data_ptr(), current_stream(z));
 }
 
+// Gradients that are to be differentiated again, through a node that refuses it: the kernels' results have no graph, and a
+// loss made of them would lose that part of its gradient without a word.
+variable_list not_twice(variable_list grads) {
+  at::AutoGradMode enabled(true);
+  for (Tensor& t : grads)
+    if (t.defined()) t = t.detach().set_requires_grad(true);
+  const auto node = std::make_shared<torch::autograd::DelayedError>("TriangleAttention cannot be differentiated twice", (int64_t)grads.size());
+  return (*node)(std::move(grads));
+}
+
 struct Block : public torch::autograd::Function<Block> {
   static Tensor forward(AutogradContext* ctx, const Tensor& z, const std::optional<Tensor>& mask, const Tensor& w0, const Tensor& w1,
                         const Tensor& w2, const Tensor& w3, const Tensor& w4, const Tensor& w5, const Tensor& w6,
@@ -278,6 +289,7 @@ struct Block : public torch::autograd::Function<Block> {
     return out;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const bool create_graph = at::GradMode::is_enabled();
     at::NoGradGuard no_grad;
     const variable_list s = ctx->get_saved_variables();
     const auto i = ctx->saved_data["i"].toIntVector();
@@ -313,6 +325,7 @@ struct Block : public torch::autograd::Function<Block> {
     check(fta_block_bwd(&b, state.data_ptr(), dout.data_ptr(), ds, &g, ws.data_ptr(), bytes, current_stream(z)));
     variable_list out{dz, Tensor()};
     for (const Tensor& t : dw) out.push_back(t);
+    if (create_graph) out = not_twice(std::move(out));
     out.resize(2 + 10 + 8);
     return out;
   }

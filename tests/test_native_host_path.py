@@ -394,3 +394,14 @@ def test_a_mask_of_a_subclass_goes_to_the_separate_layers():
     blk, z, mask = _block(), _pair(1), torch.ones(1, 48, device=DEV)
     assert blk._fused(z, mask, None) is not None and type(blk(z, mask)) is torch.Tensor
     assert blk._fused(z, mask.as_subclass(Sub), None) is None
+
+
+@gpu
+def test_second_derivatives_of_the_block_are_refused_not_dropped():
+    blk, z = _block(), _pair(1).requires_grad_(True)
+    out = blk(z)
+    dz, = torch.autograd.grad(out.square().sum(), z, create_graph=True)
+    want, = torch.autograd.grad(blk(z).square().sum(), z)
+    assert torch.equal(dz, want)
+    with pytest.raises(RuntimeError, match="twice"):
+        (out.sum() + dz.square().sum()).backward()
