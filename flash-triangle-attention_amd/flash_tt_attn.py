@@ -206,6 +206,8 @@ class _attention(torch.autograd.Function):
             raise ValueError("dropout_p must be in [0, 1)")
         if not q.is_cuda:
             raise ValueError("attention() needs tensors on the GPU; there is no CPU path")
+        if not (k.device == v.device == b_pw.device == q.device):  # (a kernel must not see a host pointer)
+            raise ValueError("q, k, v and b_pw must be on the same device")
         assert q.dim() == 5 and k.shape == q.shape and v.shape == q.shape
         B, H, L1, L2, D = map(int, q.shape)
         assert tuple(b_pw.shape) == (B, H, L2, L2), "bias must be (B, H, L2, L2)"

@@ -405,3 +405,16 @@ def test_second_derivatives_of_the_block_are_refused_not_dropped():
     assert torch.equal(dz, want)
     with pytest.raises(RuntimeError, match="twice"):
         (out.sum() + dz.square().sum()).backward()
+
+
+@gpu
+@pytest.mark.parametrize("nth", [1, 2, 3])
+@pytest.mark.parametrize("device", ["cpu", "meta"])
+@pytest.mark.parametrize("grad", [False, True])
+def test_operands_on_another_device_are_refused(nth, device, grad):
+    from flash_tt_attn import attention
+    x = list(_operands(1)[:4])
+    x[nth] = x[nth].to(device)
+    x[0].requires_grad_(grad)
+    with pytest.raises(ValueError, match="same device"):
+        attention(*x, 0.3)
