@@ -91,8 +91,8 @@ class TriangleAttention(nn.Module):
     def _fused(self, z, key_mask, seed):
         """The whole block in the kernels of csrc/fta_block.hip (three launches forward, eight backward), for
         plain fp16, bf16 or fp32 modules of the sizes built there (c_z and n_heads * c_hidden of 64 or 128);
-        None where this does not apply: other sizes, autocast, mixed types, a call that something traces
-        or transforms, hooked, parametrised, wrapped or replaced submodules, a subclass."""
+        None where this does not apply: other sizes, autocast, mixed types, a call that something traces,
+        sees through a mode or transforms, hooked, parametrised, wrapped or replaced submodules, a subclass."""
         if type(self) is not TriangleAttention or not z.is_cuda or _has_any_global_hook() or _function_mode_on():
             return None
         native = fta_lib.native()

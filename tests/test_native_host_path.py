@@ -1,7 +1,8 @@
 """What the C++ host path has to leave to the Python path, and what attention() and the block then do there (also
 where the module is missing or was built for another torch): a call whose
-operations something watches (tracing, dispatch modes, functorch), tensors with a tangent,
-tensor subclasses, sizes that are not built, submodules that are not as the block made them."""
+operations something watches (tracing, dispatch and function modes, functorch), tensors with a tangent,
+tensor subclasses, sizes that are not built, submodules that are not as the block made them.  And what the
+backward of both paths is handed: gradients and saved tensors in any layout, or as others than they were."""
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
