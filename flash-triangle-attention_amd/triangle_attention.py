@@ -98,21 +98,24 @@ class TriangleAttention(nn.Module):
         native = fta_lib.native()
         if native is None:
             return None
-        weights = []
+        weights, modules = [], self._modules
         for name, kind, has_bias in _SUBMODULES:
-            m = self._modules.get(name)
-            if type(m) is not kind or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+            m = modules.get(name)
+            if type(m) is not kind:
                 return None
-            own = m._parameters
+            d = m.__dict__
+            if d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]:
+                return None
+            own = d["_parameters"]
             # (a forward of the instance's own, as wrappers put there; a weight or bias that is no parameter any more)
-            if "forward" in m.__dict__ or "weight" not in own or "bias" not in own:
+            if "forward" in d or "weight" not in own or "bias" not in own:
                 return None
             weights.append(own["weight"])
             if has_bias:
                 weights.append(own["bias"])
             elif own["bias"] is not None:
                 return None
-        norm = self._modules["layer_norm"]
+        norm = modules["layer_norm"]
         if norm.normalized_shape != (z.shape[-1],):
             return None
         scope = _attention.forward.__globals__  # (the module that holds the PRECISE_BACKWARD switch)
