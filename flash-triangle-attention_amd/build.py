@@ -21,8 +21,8 @@ import fta_lib  # noqa: E402
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "libfta.so")
-SOURCES = ["fta_api.hip", "fta_fwd.hip", "fta_fwd1.hip", "fta_fwd1_slabs.hip", "fta_fwd2.hip", "fta_fwd_feat.hip", "fta_bwd.hip", "fta_bwd_feat.hip", "fta_bwd_dq1.hip",
-           "fta_bwd_dkdv1.hip", "fta_bwd_short.hip", "fta_block.hip"]
+SOURCES = ["fta_api.hip", "fta_fwd.hip", "fta_fwd1.hip", "fta_fwd1_slabs.hip", "fta_fwd2.hip", "fta_fwd_feat.hip", "fta_bwd.hip", "fta_bwd_feat.hip", "fta_bwd_dq1.hip", "fta_bwd_dq1_bf16.hip",
+           "fta_bwd_dkdv1.hip", "fta_bwd_dkdv1_bf16.hip", "fta_bwd_short.hip", "fta_block.hip"]
 
 DEMO_SOURCE = "fta_c_demo.cpp"
 DEMO = os.path.join(HERE, "fta_c_demo")

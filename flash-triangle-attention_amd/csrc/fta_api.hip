@@ -117,7 +117,8 @@ struct PlanKey {
   bool operator==(const PlanKey& o) const { return B == o.B && H == o.H && L1 == o.L1 && L2 == o.L2 && D == o.D && mask == o.mask; }
 };
 // The length the tiles of one direction cover for rows of L2 keys: the smallest multiple of 128 (forward: 64) that is at
-// least L2 and that the direction has a workgroup shape for (0 if there is none up to FTA_MAX_L2).  The
+// least L2 and that the direction has a workgroup shape for (0 if there is none up to FTA_MAX_L2; the hand-scheduled
+// backward's tiles may end 64 short of it, see BwdPlan::Lt).  The
 // two directions need not agree (nothing they exchange is laid out by it: lse has the row's true length):
 // the backward has a shape for every multiple of 128, the forward skips a few (D = 32: from 1792 keys on,
 // the first 17 blocks of 128; D = 64: 11 and 13 blocks), and a row is only supported where both have one.
@@ -536,7 +537,7 @@ static int bwd_impl(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor
   copy4(p.qs, q->stride); copy4(p.ks, k->stride); copy4(p.vs, v->stride); copy4(p.os, o->stride);
   copy4(p.dos, dout->stride); copy4(p.dqs, dq->stride); copy4(p.dks, dk->stride); copy4(p.dvs, dv->stride);
   copy3(p.bs, bias->stride); copy3(p.dbs, dbias->stride);
-  p.B = B; p.H = H; p.L1 = L1; p.L2 = L2; p.L2p = pl.L2p;
+  p.B = B; p.H = H; p.L1 = L1; p.L2 = L2; p.L2p = pl.L2p; p.Lt = pl.Lt;
   p.scale = sm_scale;
   p.drop = opt.drop;
   p.dbias_f32 = opt.dbias_f32;

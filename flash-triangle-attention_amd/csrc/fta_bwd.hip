@@ -12,6 +12,22 @@ namespace fta {
 // ------------------------------------------------------------------------------------------------
 BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
   BwdPlan pl{};
+  pl.feat = feat != 0;
+  pl.use_short = !forced_general() && plan_short(B, H, L1, row, D, pl.sh);
+  // (the two go together: the pipelined dQ kernel makes delta itself and hands the row constants on to the dK/dV one in
+  // the packed form that only that one reads)
+  // Their tiles end at the next multiple of 64 keys: the work grows with the square of that length.  A training step at B1
+  // H4 D32 in fp16, tiles to the next multiple of 128 and key ranges of 512 + 256 -> this (us): L 129 to 192 85 -> 72, 257
+  // 160 -> 143, 320 194 -> 169, 385 366 -> 328, 448 435 -> 395, 513 985 -> 886, 576 1114 -> 996, 704 1859 -> 1716, 1281
+  // 11160 -> 10380.
+  auto hand = [&](int lt) { pl.Lt = lt; return plan_dq1(B, H, L1, lt, D, pl.dq1) && plan_dkdv1(B, H, L1, lt, D, pl.dkdv1); };
+  pl.use_hand = !pl.use_short && !feat && !forced_general() && (hand((row + 63) / 64 * 64) || hand(L2));
+  if (pl.use_short || pl.use_hand) {
+    pl.partial_bytes = (size_t)(pl.use_short ? pl.sh.nchunks : pl.dq1.nchunks) * B * H * L2 * L2 * sizeof(float);
+    pl.aux_bytes = pl.use_short ? 0 : (size_t)B * H * L1 * L2 * 2 * sizeof(uint32_t);
+    pl.valid = true;
+    return pl;
+  }
   const int nqb = L2 / 32;
   const size_t lds_max = 160 * 1024;
   // ---- dQ/dBias kernel: key range of at most 512 keys per launch, 128-key slabs
@@ -87,16 +103,10 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
   pl.rows_per_chunk2 = (L1 + pl.nchunks2 - 1) / pl.nchunks2;
   pl.nchunks2 = (L1 + pl.rows_per_chunk2 - 1) / pl.rows_per_chunk2;
 
-  pl.use_short = !forced_general() && plan_short(B, H, L1, row, D, pl.sh);
-  // (the two go together: the pipelined dQ kernel makes delta itself and hands the row constants on to the dK/dV one in
-  // the packed form that only that one reads)
-  pl.use_hand = !pl.use_short && !feat && !forced_general() && plan_dq1(B, H, L1, L2, D, pl.dq1) && plan_dkdv1(B, H, L1, L2, D, pl.dkdv1);
-  pl.delta_bytes = (pl.use_hand || pl.use_short) ? 0 : (size_t)B * H * L1 * L2 * sizeof(float);
-  const int maxchunks = pl.use_short ? pl.sh.nchunks : pl.use_hand ? pl.dq1.nchunks : pl.nchunks;  // of the dQ/dBias kernel that runs
-  pl.partial_bytes = (size_t)maxchunks * B * H * L2 * L2 * sizeof(float);
-  pl.aux_bytes = pl.use_short ? 0 : (size_t)B * H * L1 * L2 * 2 * sizeof(uint32_t);
+  pl.delta_bytes = (size_t)B * H * L1 * L2 * sizeof(float);
+  pl.partial_bytes = (size_t)pl.nchunks * B * H * L2 * L2 * sizeof(float);
+  pl.aux_bytes = (size_t)B * H * L1 * L2 * 2 * sizeof(uint32_t);
   pl.valid = ok2 && (pl.SK * pl.QB <= 8) && (pl.ring >= 3);
-  pl.feat = feat != 0;
   return pl;
 }
 

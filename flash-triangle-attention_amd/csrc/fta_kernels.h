@@ -92,6 +92,7 @@ struct BwdParams {
   int B, H, L1, L2;    // L2: the true row length; lse is (B,H,L1,L2)
   int L2p;             // the length the tiles cover (next supported multiple of 128); delta, partial and aux
                        // in the workspace are laid out with L2p
+  int Lt;              // the length that the hand-scheduled kernels' tiles cover (see BwdPlan)
   float scale;
   // dQ/dBias kernel geometry
   int SK;              // 128-key slabs per workgroup (waves sharing one query block)
@@ -120,6 +121,13 @@ struct BwdParams {
 
 // Geometry of the one-wave-per-SIMD dK/dV kernel (a wave owns 32 keys against the launch's query range).
 constexpr int kMaxRanges = 8;  // launches (key or query ranges) of a hand-scheduled backward stage: 4096 / 512
+// Cuts `units` into the fewest ranges of at most `most` units, larger ones first and none more than a unit larger than
+// another; the ranges, `unit` long each, go to `out` and their number is returned.
+inline int even_ranges(int units, int most, int unit, int* out) {
+  const int n = (units + most - 1) / most;
+  for (int r = 0; r < n; ++r) out[r] = (units / n + (r < units % n ? 1 : 0)) * unit;
+  return n;
+}
 struct Dq1Plan {
   int SK, QB, nqg, nchunks, rows_per_chunk, threads, KR, nlaunch, ring, nb;   // SK, QB, nqg, KR: of the first range
   int range[kMaxRanges];          // keys per launch
@@ -153,7 +161,8 @@ struct BwdPlan {
   Dkdv1Plan dkdv1;
   bool use_short;      // rows of up to 128 keys: all gradients in one kernel
   ShortPlan sh;
-  int L2p;             // the length the tiles cover (filled in by the C-ABI layer)
+  int L2p;             // the length the workspace is laid out with and the general kernels' tiles cover (filled in by the C-ABI layer)
+  int Lt;              // the length the hand-scheduled kernels' tiles cover: the next multiple of 64, not of 128, where they have the instances
   bool feat;           // planned for the feature instances (bf16, dropout, precise fp16)
   bool valid;
 };

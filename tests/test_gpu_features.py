@@ -459,6 +459,34 @@ def test_precise_backward_holds_the_tolerance_on_large_biases_and_scores(bias_st
     assert max(e_pre.values()) < max(e_def.values())
 
 
+# ---- the hand-scheduled backward at tiled lengths in steps of 64 -------------------------------------------
+
+@pytest.mark.parametrize("mode", ["fp16", "bf16", "bf16 operand pair", "precise"])
+@pytest.mark.parametrize("D,L2", [(32, L) for L in (129, 192, 193, 257, 320, 385, 448, 449, 513, 640, 703, 1088)]
+                         + [(64, L) for L in (129, 192, 257, 320, 400, 576, 640, 701, 832)])
+def test_backward_tiles_in_steps_of_64(D, L2, mode):
+    """Every number of tiles per wave (key ranges of 256 to 512 keys in two slabs, of 192 and 256 in one; D = 64: 160 to
+    256; query ranges of 192 to 512, at D = 64 256 to 384), odd numbers of them (stages of unequal length), groups of 128 queries or keys
+    that end beyond the tiled length, one to four ranges; rows that end inside a tile and whole ones."""
+    import fta_lib
+    import flash_tt_attn as fta
+    if D == 64 and mode in ("bf16 operand pair", "precise"):
+        pytest.skip("no such instances at head dim 64")
+    dtype = torch.bfloat16 if mode.startswith("bf16") else torch.float16
+    B, H, L1, sm = 1, 2, 5, 1.3 if mode == "bf16 operand pair" else 1.0 / math.sqrt(D)
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, 0.0, 0, 1 if mode == "precise" else 0)
+    plan = fta_lib.describe_plan(B, H, L1, L2, D, sm, opt)
+    assert "dq1" in plan["dq"]["kernel"] and "dkdv1" in plan["dkdv"]["kernel"]
+    print(f"case {mode} D={D} L2={L2}", flush=True)
+    q, k, v, b, do = _inputs(B, H, L1, L2, D, 41, dtype)
+    fta.PRECISE_BACKWARD = mode == "precise"
+    try:
+        got = _run(q, k, v, b, sm, do)
+    finally:
+        fta.PRECISE_BACKWARD = False
+    _compare(got, _oracle(q, k, v, b, sm, do), dtype, f"tiles of 64 {mode} D{D} L{L2}")
+
+
 # ---- everything at once, drawn at random -------------------------------------------------------------------
 
 def test_random_draws_over_types_masks_dropout_modes_and_layouts():
