@@ -119,7 +119,8 @@ __device__ __forceinline__ void dkdv1_lds_landed(u32x4 (&qf)[KS], u32x4 (&dof)[K
 // HL (D = 32): the scaled K fragments are kept as a (hi, lo) pair of values of the element type and S takes
 // one more MFMA per contraction step; NAT (fp16 with HL): exponents in natural units, the row constants as the
 // dQ kernel's NAT instance leaves them (see fta_bwd_dq1_kernel).
-template <class T, int D, int NJT, int TS, bool TAIL, bool HL = false, bool NAT = false>
+// LATER (D = 32): earlier query ranges' launches left partial dK, dV to add to (D = 64: told by jr0).
+template <class T, int D, int NJT, int TS, bool TAIL, bool HL = false, bool NAT = false, bool LATER = false>
 __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   static_assert(D == 32 || D == 64, "one or two 32-wide d tiles");
   static_assert(!HL || D == 32, "the (hi, lo) split exists at D = 32");
@@ -149,6 +150,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   static_assert(TS >= 4 && (TS - 1) * NG >= 2 * NQI + 1 + 2 * (KR * (D / 8) / 256),
                 "the iterations between two barriers must have a gap for every copy of a stage");
   static_assert(R * SLOT_B + NBK * KV_B <= 160 * 1024, "LDS");
+  static_assert(WIDE || NG >= 4 * DT, "a gap for every piece of an earlier range's row");
   static_assert(ACP == 1 || ACP == 2, "128 to 256 queries per stage");
 
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
@@ -228,7 +230,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   const int64_t step_q = hold_scalar(p.qs[2] * 2), step_do = hold_scalar(p.dos[2] * 2), step_k = hold_scalar(p.ks[2] * 2),
                 step_v = hold_scalar(p.vs[2] * 2), step_dk = hold_scalar(p.dks[2] * 2), step_dv = hold_scalar(p.dvs[2] * 2),
                 step_aux = hold_scalar((int64_t)p.L2p * 8);
-  const bool later_range = (p.jr0 != 0);  // earlier launches left partial dK, dV to add to
+  const bool later_range = (D == 32) ? LATER : (p.jr0 != 0);
   auto advance = [](auto*& ptr, int64_t bytes) {
     using P = std::remove_reference_t<decltype(ptr)>;
     ptr = (P)((const char*)ptr + bytes);
@@ -421,8 +423,23 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   // touches 32 different rows either way, and the address path is what the stage copies need too).
   half_t* dkcur = dkbase + (int64_t)i0 * p.dks[2];  // advance by one row per call
   half_t* dvcur = dvbase + (int64_t)i0 * p.dvs[2];
-  const uint32_t voff_dk = (uint32_t)(((int64_t)(k0 + l32) * p.dks[3] + 8 * hh) * 2);
-  const uint32_t voff_dv = (uint32_t)(((int64_t)(k0 + l32) * p.dvs[3] + 8 * hh) * 2);
+  const int kread = TAIL ? min(k0 + l32, p.L2 - 1) : k0 + l32;
+  const uint32_t voff_dk = (uint32_t)(((int64_t)kread * p.dks[3] + 8 * hh) * 2);
+  const uint32_t voff_dv = (uint32_t)(((int64_t)kread * p.dvs[3] + 8 * hh) * 2);
+  // What earlier query ranges left in the row comes in before the row's last barrier, whose wait covers it (loaded where it
+  // is added, a lone wave waits out the trip to memory at every row: the later ranges of B1 H4 L1536 took 1.79 ms against
+  // 1.57 of the first); into accumulation registers, which D = 64 has not enough of.
+  constexpr int OLD = 2 * DT;                                    // pieces of dK, and of dV
+  constexpr bool PRE = !WIDE && LATER;
+  constexpr int PRE_AT = STEPS == 1 ? 2 : (STEPS - 1) * TS - 2;  // the iteration that loads them
+  u32x4 oldk[OLD], oldv[OLD];
+#pragma unroll
+  for (int x = 0; x < OLD; ++x) oldk[x] = oldv[x] = u32x4{0u, 0u, 0u, 0u};
+  auto old_issue = [&](auto xc) {
+    constexpr int x = decltype(xc)::value;
+    if constexpr (x < OLD) load_piece<kA, 32 * x>(oldk[x], voff_dk, uniform_ptr(dkcur));
+    else if constexpr (x < 2 * OLD) load_piece<kA, 32 * (x - OLD)>(oldv[x - OLD], voff_dv, uniform_ptr(dvcur));
+  };
   auto swap_halves = [](uint32_t& x, uint32_t& y) {
     auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
     x = r[0];
@@ -456,8 +473,8 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       u32x4 ok[2 * DT], ov[2 * DT];
 #pragma unroll
       for (int x = 0; x < 2 * DT; ++x) {
-        ok[x] = *reinterpret_cast<const u32x4*>(dkr + 16 * x);
-        ov[x] = *reinterpret_cast<const u32x4*>(dvr + 16 * x);
+        ok[x] = PRE ? oldk[x] : *reinterpret_cast<const u32x4*>(dkr + 16 * x);
+        ov[x] = PRE ? oldv[x] : *reinterpret_cast<const u32x4*>(dvr + 16 * x);
       }
 #pragma unroll
       for (int x = 0; x < 2 * DT; ++x)
@@ -553,6 +570,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
           // (all reads go into the first NGR gaps: the last ones issued still have a few MFMAs to land behind)
           if constexpr (e < NGR) static_for<(e * NRD) / NGR, ((e + 1) * NRD) / NGR>(lds_read);
           // one copy of the stage whose slot the last barrier freed
+          if constexpr (PRE && g == PRE_AT) old_issue(std::integral_constant<int, e>{});
           constexpr int since = (g - (TS - 2) + NJT) % NJT;  // iterations since the row's first barrier
           if constexpr (since % TS != 0)
             stage_copy(std::integral_constant<int, (since / TS + 2) % STEPS>{}, std::integral_constant<int, (since % TS - 1) * NG + e>{});
@@ -659,6 +677,9 @@ template <class T, int D, bool HL, bool NAT>
 inline hipError_t launch_dkdv1_range(const BwdParams& p, int range, dim3 grid, size_t smem, hipStream_t st) {
   // (a last group of 128 keys that reaches beyond the row: the masking instances)
   const bool tl = (p.L2 != p.Lt) || (p.Lt % 128 != 0) || p.odd_bias;
+  // (later ranges: the masking instances for any row)
+#define FTA_DKDV1_LATER(NN, TS_)                                                                                   \
+  if (p.jr0 != 0 && range == 32 * NN) return launch_kernel(fta_bwd_dkdv1_kernel<T, D, NN, TS_, true, HL, NAT, true>, p, grid, dim3(256), smem, st);
 #define FTA_DKDV1_CASE(NN, TS_)                                                                                    \
   if (range == 32 * NN)                                                                                            \
     return tl ? launch_kernel(fta_bwd_dkdv1_kernel<T, D, NN, TS_, true, HL, NAT>, p, grid, dim3(256), smem, st)    \
@@ -666,9 +687,11 @@ inline hipError_t launch_dkdv1_range(const BwdParams& p, int range, dim3 grid, s
   if constexpr (D == 64) {
     FTA_DKDV1_CASE(8, 4) FTA_DKDV1_CASE(10, 5) FTA_DKDV1_CASE(12, 4)
   } else {
+    FTA_DKDV1_LATER(8, 8) FTA_DKDV1_LATER(10, 5) FTA_DKDV1_LATER(12, 6) FTA_DKDV1_LATER(14, 7) FTA_DKDV1_LATER(16, 8)
     FTA_DKDV1_CASE(6, 6) FTA_DKDV1_CASE(8, 8) FTA_DKDV1_CASE(10, 5) FTA_DKDV1_CASE(12, 6) FTA_DKDV1_CASE(14, 7) FTA_DKDV1_CASE(16, 8)
   }
 #undef FTA_DKDV1_CASE
+#undef FTA_DKDV1_LATER
   return hipErrorInvalidConfiguration;
 }
 

@@ -118,7 +118,8 @@ __device__ __forceinline__ uint32_t ds_pair(float s0, float s1, float dp0, float
 // NAT (fp16 with HL: the precise mode): the exponent is formed in natural units, so that the bias enters
 // as it is instead of rounded once more after the multiplication by log2(e); the vector ALU multiplies
 // by log2(e) in fp32 in front of the exponential (16 more instructions per tile)
-template <class T, int D, int SK, int NKT, bool TAIL, bool HL = false, bool NAT = false>
+// LATER (D = 32): earlier key ranges' launches left a partial dQ to add to (D = 64: told by kr0)
+template <class T, int D, int SK, int NKT, bool TAIL, bool HL = false, bool NAT = false, bool LATER = false>
 __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
   static_assert(!HL || D == 32, "the (hi, lo) split exists at D = 32");
   static_assert(!NAT || (HL && !T::is_bf16), "natural units come with the split, for fp16");
@@ -209,7 +210,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
   // keep whole argument blocks alive in scalar registers): byte steps from one row to the next.
   int64_t step_k = p.ks[2] * 2, step_v = p.vs[2] * 2, step_q = p.qs[2] * 2, step_do = p.dos[2] * 2, step_o = p.os[2] * 2,
           step_dq = p.dqs[2] * 2, step_lse = (int64_t)p.L2 * 4, step_aux = (int64_t)p.L2p * 8;
-  int later_range = (p.kr0 != 0) ? 1 : 0;  // an earlier launch left a partial dQ to add to
+  const bool later_range = (D == 32) ? LATER : (p.kr0 != 0);
   step_k = hold_scalar(step_k); step_v = hold_scalar(step_v); step_q = hold_scalar(step_q); step_do = hold_scalar(step_do);
   step_o = hold_scalar(step_o); step_dq = hold_scalar(step_dq); step_lse = hold_scalar(step_lse); step_aux = hold_scalar(step_aux);
   auto advance = [](auto*& ptr, int64_t bytes) {
@@ -501,9 +502,26 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
   // register pair (v_permlane32_swap) gives each lane the eight consecutive values of one group, so the
   // row goes out in 16-byte pieces (half as many store instructions).
   half_t* dqcur = dqbase + (int64_t)i0 * p.dqs[2];  // advances by one row per call
+  // What an earlier key range left in the row comes in ahead of the barrier before its use (loaded where it is added, a
+  // lone wave waits out the trip to memory at every row: the later ranges of B1 H4 L1536 took 1.94 ms against 1.61 of the
+  // first; with the same in dK/dV the step went from 14.95 to 14.48 ms).  It is issued in front of the copies of its iteration, so that the next barrier's wait covers it.  (D = 64 has no
+  // registers for it.)
+  constexpr bool PRE = (D == 32 && LATER);
+  constexpr bool PRE_NEXT = XCHG_RD < SYNC_B;     // the row computed now (it is stored in the next row's iterations), else the row before
+  constexpr int PRE_AT = PRE_NEXT ? SYNC_B : SYNC_A;
+  u32x4 old[XG / 2];
+#pragma unroll
+  for (int y = 0; y < XG / 2; ++y) old[y] = u32x4{0u, 0u, 0u, 0u};
   static_assert(XG % 2 == 0, "groups are exchanged in pairs");
   // lane (query, hh) ends up with group SK*(2y + hh) + slab of pair y: d = 8*SK*(2y + hh) + 8*slab .. +7
-  const uint32_t voff_dq = (uint32_t)(((int64_t)(q0 + l32) * p.dqs[3] + 8 * SK * hh + 8 * slab) * 2);
+  const uint32_t voff_dq = (uint32_t)(((int64_t)qread * p.dqs[3] + 8 * SK * hh + 8 * slab) * 2);
+  auto old_issue = [&]() {
+    const void* rb = uniform_ptr(dqcur);
+    static_for<0, XG / 2>([&](auto yc) {
+      constexpr int y = decltype(yc)::value;
+      load_piece<kV, 32 * SK * y>(old[y], voff_dq, rb);
+    });
+  };
   auto store_dq = [&](const float* vals) {
     half_t* dqr = reinterpret_cast<half_t*>(reinterpret_cast<char*>(dqcur) + voff_dq);
     advance(dqcur, step_dq);
@@ -519,9 +537,9 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
     }
     if (!qvalid) return;
     if (later_range) {  // one branch for the whole row
-      u32x4 old[XG / 2];
 #pragma unroll
-      for (int y = 0; y < XG / 2; ++y) old[y] = *reinterpret_cast<const u32x4*>(dqr + 16 * SK * y);
+      for (int y = 0; y < XG / 2; ++y)
+        if constexpr (!PRE) old[y] = *reinterpret_cast<const u32x4*>(dqr + 16 * SK * y);
 #pragma unroll
       for (int y = 0; y < XG / 2; ++y)
 #pragma unroll
@@ -691,6 +709,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
         static_for<(e * NRD) / NG, ((e + 1) * NRD) / NG>(lds_read);
         if constexpr (e == 0) lds_wait_older<((NRD / NG) > 15) ? 15 : NRD / NG>(kf, vf, ktlo_p, kthi_p);
         if constexpr (e == 0 && g == SYNC_A) rowconst_issue(ir + 1);
+        if constexpr (PRE && e == 0 && g == PRE_AT) old_issue();
         row_work(ec);
         if constexpr (has_part && e >= 1 && e <= 3)
           stage_part_copy(std::integral_constant<int, part_t>{}, std::integral_constant<int, part_k>{}, std::integral_constant<int, e - 1>{});
@@ -826,6 +845,12 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) acc[dt] = T::mfma(ktp[u][dt], db, acc[dt]);
   }
+  if constexpr (PRE && !PRE_NEXT) old_issue();
+  if constexpr (PRE) {
+    wait_vmem_all();
+#pragma unroll
+    for (int y = 0; y < XG / 2; ++y) asm volatile("" : "+v"(old[y]));
+  }
   split_groups(acc);
   if constexpr (SK == 2) {
     __syncthreads();
@@ -851,6 +876,9 @@ inline hipError_t launch_dq1_range(const BwdParams& p, int range, dim3 grid, siz
   const int nkt = range / (32 * p.SK);
   // (a last group of 128 queries that reaches beyond the row: the masking instances)
   const bool tl = (p.L2 != p.Lt) || (p.Lt % (32 * p.QB) != 0) || p.odd_bias;
+  // (later ranges: the masking instances for any row)
+#define FTA_DQ1_LATER(NN)                                                                                        \
+  if (p.kr0 != 0 && nkt == NN) return launch_kernel(fta_bwd_dq1_kernel<T, D, 2, NN, true, HL, NAT, true>, p, grid, dim3(256), smem, st);
 #define FTA_DQ1_CASE(SS, NN)                                                                                     \
   if (p.SK == SS && nkt == NN)                                                                                   \
     return tl ? launch_kernel(fta_bwd_dq1_kernel<T, D, SS, NN, true, HL, NAT>, p, grid, dim3(256), smem, st)     \
@@ -858,10 +886,12 @@ inline hipError_t launch_dq1_range(const BwdParams& p, int range, dim3 grid, siz
   if constexpr (D == 64) {
     FTA_DQ1_CASE(1, 5) FTA_DQ1_CASE(1, 6) FTA_DQ1_CASE(1, 7) FTA_DQ1_CASE(1, 8)
   } else {
+    FTA_DQ1_LATER(4) FTA_DQ1_LATER(5) FTA_DQ1_LATER(6) FTA_DQ1_LATER(7) FTA_DQ1_LATER(8)
     FTA_DQ1_CASE(1, 6) FTA_DQ1_CASE(1, 8)
     FTA_DQ1_CASE(2, 4) FTA_DQ1_CASE(2, 5) FTA_DQ1_CASE(2, 6) FTA_DQ1_CASE(2, 7) FTA_DQ1_CASE(2, 8)
   }
 #undef FTA_DQ1_CASE
+#undef FTA_DQ1_LATER
   return hipErrorInvalidConfiguration;
 }
 

@@ -146,4 +146,11 @@ __device__ __forceinline__ void mfma_acc_v_aa(floatx16& c, u32x4 a, half8_t b) {
   asm volatile(FTA_MFMA "%0, %1, %2, %0" : "+v"(c) : "a"(a), "v"(b));
 }
 
+// 16 bytes per lane from a uniform base.  The compiler does not see the load: the caller waits for it.
+template <int RF, int OFF>
+__device__ __forceinline__ void load_piece(u32x4& d, uint32_t voff, const void* base) {
+  if constexpr (RF == kA) asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=a"(d) : "v"(voff), "s"(base), "n"(OFF) : "memory");
+  else asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(d) : "v"(voff), "s"(base), "n"(OFF) : "memory");
+}
+
 }  // namespace fta
