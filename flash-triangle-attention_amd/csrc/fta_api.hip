@@ -116,7 +116,7 @@ struct PlanKey {
   int B, H, L1, L2, D, mask;
   bool operator==(const PlanKey& o) const { return B == o.B && H == o.H && L1 == o.L1 && L2 == o.L2 && D == o.D && mask == o.mask; }
 };
-// The length the tiles of one direction cover for rows of L2 keys: the smallest multiple of 128 (forward: 64) that is at
+// The length the tiles of one direction cover for rows of L2 keys: the smallest multiple of 128 (forward: 32) that is at
 // least L2 and that the direction has a workgroup shape for (0 if there is none up to FTA_MAX_L2; the hand-scheduled
 // backward's tiles may end 64 short of it, see BwdPlan::Lt).  The
 // two directions need not agree (nothing they exchange is laid out by it: lse has the row's true length):
@@ -125,10 +125,10 @@ struct PlanKey {
 // (`feat`: 1 for the backward's vector-ALU instances, 2 for dropout, which has fewer instances in both
 // directions)
 int padded_len_fwd(int L2, int D, int feat) {
-  for (int lp = (L2 + 63) / 64 * 64; lp <= FTA_MAX_L2; lp += 64) {
-    const fta::FwdPlan pl = fta::plan_fwd(1, 1, 1, lp, D, feat == 2);
+  for (int lp = (L2 + 31) / 32 * 32; lp <= FTA_MAX_L2; lp += 32) {
+    const fta::FwdPlan pl = fta::plan_fwd(1, 1, 1, lp, D, lp, feat == 2);
     // (shapes in between: the hand-scheduled kernel's, and rows of one slab with dropout at D = 32)
-    if (pl.valid && (lp % 128 == 0 || pl.fwd1 == 1 || (feat == 2 && D == 32 && pl.S == 1))) return lp;
+    if (pl.valid && (lp % 128 == 0 || pl.fwd1 == 1 || (feat == 2 && D == 32 && pl.S == 1 && lp % 64 == 0))) return lp;
   }
   return 0;
 }
@@ -144,7 +144,7 @@ const fta::FwdPlan& cached_plan_fwd(int B, int H, int L1, int L2, int D, int fea
   const PlanKey k{B, H, L1, L2, D, feat * 4};
   if (!(key == k)) {
     const int lp = len_supported(L2, D, feat) ? padded_len_fwd(L2, D, feat) : 0;
-    plan = (lp != 0) ? fta::plan_fwd(B, H, L1, lp, D, feat == 2) : fta::FwdPlan{};
+    plan = (lp != 0) ? fta::plan_fwd(B, H, L1, lp, D, L2, feat == 2) : fta::FwdPlan{};
     plan.L2p = lp;
     key = k;
   }

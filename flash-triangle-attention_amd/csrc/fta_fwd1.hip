@@ -6,20 +6,23 @@ namespace fta {
 
 // ---- host side ---------------------------------------------------------------------------------
 
-bool plan_fwd1(int B, int H, int L1, int L2, int D, FwdPlan& pl) {
-  if (D != 32 || L2 % 64 != 0 || L2 < 64 || L2 > 1792) return false;
+bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, FwdPlan& pl) {
+  if (D != 32 || L2 % 32 != 0 || L2 < 64 || L2 == 96 || L2 > 1792) return false;
   pl = FwdPlan{};
-  // rows beyond 512 keys in two slabs, beyond 1024 in four (three would leave two of the four SIMDs with one wave), each
-  // of an even number of tiles; four slabs of 512 keys have no registers left for the ends of rows
+  // rows beyond 512 keys in two slabs, beyond 1024 in four (three would leave two of the four SIMDs with one wave);
+  // four slabs of 512 keys have no registers left for the ends of rows.  Any number of tiles per slab: with even ones alone
+  // (bf16, B1 H4, us) L160 14.7 against 12.8 with five, L288 39.9 / 36.8, L416 90 / 85, L576 246 / 228, L701 420 / 396, L960
+  // 929 / 888, L1152 1738 / 1625, L1601 4750 / 4500
   pl.S = L2 <= 512 ? 1 : L2 <= 1024 ? 2 : 4;
-  pl.NKT = (L2 + 64 * pl.S - 1) / (64 * pl.S) * 2;
+  if (L2 % (32 * pl.S) != 0) return false;
+  pl.NKT = L2 / (32 * pl.S);
   // eight waves per workgroup where the queries divide that way and such workgroups still fill the chip
   // (see the kernel's comment; same-run A/B at B4 H8: 1.020 against 1.078 ms at L2 = 512, 0.183 against
   // 0.194 at 256; four-wave workgroups in four rounds instead of two gain 4 %), else four; rows of up to
   // 64 queries have two query blocks
   const bool fills = (long)B * H * (L2 / 256) * ((L1 + 7) / 8) >= 256;
   pl.QB = pl.S > 1 ? 8 / pl.S : (L2 % 256 == 0 && fills) ? 8 : L2 <= 64 ? 2 : 4;
-  pl.nqg = (L2 + 32 * pl.QB - 1) / (32 * pl.QB);
+  pl.nqg = (row + 32 * pl.QB - 1) / (32 * pl.QB);
   pl.threads = 64 * pl.QB * pl.S;
   // (stages of 256 keys, which an eight-wave workgroup has the LDS for, halve the barriers and measured
   // the same: 1.040-1.043 against 1.044-1.047 ms at B4 H8 L512; not instantiated)
@@ -40,6 +43,8 @@ bool plan_fwd1(int B, int H, int L1, int L2, int D, FwdPlan& pl) {
 hipError_t launch_fwd1(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 grid, dim3 block, hipStream_t st) {
   const bool tl = (p.L2 % (32 * pl.QB) != 0) || p.L2 != 32 * pl.NKT * pl.S || p.odd_bias;  // (the instances that mask a row's tail also read the bias entry by entry where they must)
   FTA_FWD1_CASE(2, 2, 2, 1)
+  FTA_FWD1_CASE(5, 4, 4, 1) FTA_FWD1_CASE(7, 4, 4, 1) FTA_FWD1_CASE(9, 4, 4, 1) FTA_FWD1_CASE(11, 4, 4, 1)
+  FTA_FWD1_CASE(13, 4, 4, 1) FTA_FWD1_CASE(15, 4, 4, 1)
   FTA_FWD1_CASE(4, 4, 4, 1) FTA_FWD1_CASE(6, 4, 4, 1) FTA_FWD1_CASE(8, 4, 4, 1) FTA_FWD1_CASE(10, 4, 4, 1)
   FTA_FWD1_CASE(12, 4, 4, 1) FTA_FWD1_CASE(14, 4, 4, 1) FTA_FWD1_CASE(16, 4, 4, 1)
   FTA_FWD1_CASE(8, 8, 4, 1) FTA_FWD1_CASE(16, 8, 4, 1)

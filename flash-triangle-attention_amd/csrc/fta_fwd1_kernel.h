@@ -24,8 +24,9 @@ namespace fta {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-// T: element type; NKT: 32-key tiles per row (even, 2 to 16: the score tiles alternate between two register
-// tuples, so an odd count would end a row on the wrong one); TAIL: the row's true length L2 is shorter
+// T: element type; NKT: 32-key tiles per row and slab (2 to 16: the score tiles alternate between two register
+// tuples, and an odd count moves the next row's first tile from one to the other at the end of a row, 16 instructions
+// where the tile it saves takes 64); TAIL: the row's true length L2 is shorter
 // than the 32*NKT keys the tiles cover, or than the workgroups' query blocks (keys beyond it masked, queries
 // beyond it computed on copies of the last one and not stored); W: waves (query blocks of 32) per workgroup, 4 or 8.
 // Two waves share a SIMD either way.  With W = 4 they belong to two independent workgroups, and the
@@ -52,10 +53,12 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
   constexpr int R = 4;                         // ring slots
   constexpr uint32_t TILE_B = S * KT * D * 2;  // bytes of a staged K (or V) tile: slab after slab
   constexpr uint32_t SLOT_B = 2 * TILE_B;      // K tile, then V tile
-  static_assert(NKT % 2 == 0 && NKT >= 2 && NKT <= 16, "an even number of tiles, bias within the register budget");
+  static_assert(NKT >= 2 && NKT <= 16, "bias within the register budget");
+  constexpr bool ODD = NKT % 2 != 0;
   // Stage w of a row: its tiles, and the copies a wave issues for it (of K, and as many of V).
   constexpr auto tiles_of = [](int w) { return (w + 1) * G <= NKT ? G : NKT - w * G; };
-  constexpr auto ncu_of = [=](int w) { return (S * 2 * tiles_of(w) + W - 1) / W; };
+  // (several slabs: a slab's rows keep their place in a stage that is not full; what is not a tile of the slab is copied and not read)
+  constexpr auto ncu_of = [=](int w) { return S > 1 ? NCU : (2 * tiles_of(w) + W - 1) / W; };
   // Iteration t issues the scores of tile tn = (t + 1) % NKT, and the tn % G-th share of the copies of the stage two
   // behind tile tn's: `first` to `end`, the K copies before the V copies.
   struct Share { int stage, first, end; };
@@ -144,10 +147,11 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
   // its row
   auto fill_copy = [&](auto wc, auto cc) {
     constexpr int w = decltype(wc)::value, c = decltype(cc)::value, nk = ncu_of(w);
-    constexpr bool TL = CLAMP && (w == NST - 1);
+    constexpr bool TL = S == 1 && CLAMP && (w == NST - 1);
     static_assert(c < 2 * nk, "a copy of the stage");
-    if constexpr (S > 1 && TAIL && w >= NST - S) {
-      // (fewer than 64*S keys are missing, so the last slab ends in one of its last S stages)
+    if constexpr (S > 1 && (TAIL ? w >= NST - S : w * G + G > NKT)) {
+      // (fewer than 64*S keys are missing, so the last slab ends in one of its last S stages; a stage that is not full
+      // reaches beyond the last slab)
       if constexpr (c < nk) dma16s_at<(uint32_t)c * W * 1024u>(min(goffk[c] + (uint32_t)(w * sstep_k), goffk_t[c]), kfill, fill_lds);
       else dma16s_at<TILE_B + (uint32_t)(c - nk) * W * 1024u>(min(goffv[c - nk] + (uint32_t)(w * sstep_v), goffv_t[c - nk]), vfill, fill_lds);
     } else if constexpr (c < nk) dma16s_at<(uint32_t)c * W * 1024u>(TL ? goffk_t[c] : goffk[c], kst, fill_lds);
@@ -200,12 +204,19 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
   });
   uint32_t bias_reg[NKT][8];
   static_assert(W * 4096 <= 2 * SLOT_B, "4 KB for every wave's bias");
-  load_bias_tiles<NKT / 2, 2, TAIL, NKT == 2>(p.bias + b * p.bs[0] + h * p.bs[1], p.bs[2], q0, p.L2, F16::kBeyond2,
-                                              smem_raw + 2 * SLOT_B + wave * 4096, lane, [=](int c) { return slab * KW + 64 * c; }, fwd1_bias_pair<T>,
-                                              [&](int tt, int rg, u32x2 v) {
-                                                bias_reg[tt][2 * rg] = v[0];
-                                                bias_reg[tt][2 * rg + 1] = v[1];
-                                              });
+  {
+    const half_t* bias_bh = p.bias + b * p.bs[0] + h * p.bs[1];
+    char* turn = smem_raw + 2 * SLOT_B + wave * 4096;
+    auto sink = [&](int tt, int rg, u32x2 v) {
+      bias_reg[tt][2 * rg] = v[0];
+      bias_reg[tt][2 * rg + 1] = v[1];
+    };
+    load_bias_tiles<NKT / 2, 2, TAIL, NKT == 2>(bias_bh, p.bs[2], q0, p.L2, F16::kBeyond2, turn, lane, [=](int c) { return slab * KW + 64 * c; },
+                                                fwd1_bias_pair<T>, sink);
+    if constexpr (ODD)
+      load_bias_tiles<1, 1, TAIL, false>(bias_bh, p.bs[2], q0, p.L2, F16::kBeyond2, turn, lane, [=](int) { return slab * KW + 32 * (NKT - 1); },
+                                         fwd1_bias_pair<T>, [&](int, int rg, u32x2 v) { sink(NKT - 1, rg, v); });
+  }
   q_issue(false);
   wait_vmem_all();
   __syncthreads();
@@ -402,8 +413,10 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
         constexpr int ahead = 2 * ncu_of((tn / G + 1) % NST);
         constexpr int allowed = (t == NKT - 1 && behind_q() < ahead) ? behind_q() : ahead;
         static_assert(allowed <= 15, "low bits of vmcnt");
-        // (S > 1, iteration 1: also this wave's record of the finished row is in LDS before the others pass the barrier)
-        __builtin_amdgcn_s_waitcnt((S > 1 && t == 1 ? 0x0070 : 0x0F70) | allowed);
+        // (S > 1, iteration 1: also this wave's record of the finished row is in LDS before the others pass the barrier;
+        // behind a stage of one tile: also the V^T reads of the iteration before, from the stage whose slot is filled now)
+        constexpr bool drain = (S > 1 && t == 1) || (t == NKT - 1 && tiles_of(NST - 1) == 1);
+        __builtin_amdgcn_s_waitcnt((drain ? 0x0070 : 0x0F70) | allowed);
         __builtin_amdgcn_s_barrier();
         kslot = (kslot + 1) & (R - 1);
 #pragma unroll
@@ -451,7 +464,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
       // V^T operands of tile t (for the next iteration)
       if constexpr (t % G == 0) {
 #pragma unroll
-        for (int x = 0; x < 2; ++x) aTc[x] = aT[x] + (uint32_t)kslot * SLOT_B;  // (tile t opens the stage the K reads entered one tile ago)
+        for (int x = 0; x < 2; ++x) aTc[x] = aT[x] + (uint32_t)(PUB ? (kslot - 1) & (R - 1) : kslot) * SLOT_B;  // (tile t opens the stage the K reads entered one tile ago)
       }
       vtl[0] = lds_issue_tr4<(t % G) * 32 * D * 2>(aTc[0]);
       vth[0] = lds_issue_tr4<(t % G) * 32 * D * 2>(aTc[1]);
@@ -520,6 +533,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
     // those of the row after are asked for
     l_done = l;
     m_done = m_ref;
+    if constexpr (ODD) s[0] = s[1];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = qn[ks];
     asm volatile("" : "+v"(qf[0]), "+v"(qf[1]));

@@ -92,7 +92,6 @@ struct BwdParams {
   int B, H, L1, L2;    // L2: the true row length; lse is (B,H,L1,L2)
   int L2p;             // the length the tiles cover (next supported multiple of 128); delta, partial and aux
                        // in the workspace are laid out with L2p
-  int Lt;              // the length that the hand-scheduled kernels' tiles cover (see BwdPlan)
   float scale;
   // dQ/dBias kernel geometry
   int SK;              // 128-key slabs per workgroup (waves sharing one query block)
@@ -116,6 +115,7 @@ struct BwdParams {
                        // instances that mask a row's tail run, which read the bias entry by entry where they must
   int nat;             // (host side) the hand-scheduled backward kernels' precise instances run: exponents in
                        // natural units, scaled operands as (hi, lo) pairs
+  int Lt;              // (host side) the length that the hand-scheduled kernels' tiles cover (see BwdPlan)
 };
 
 
@@ -213,7 +213,8 @@ hipError_t launch_dbias_reduce(const BwdParams& p, int dtype, hipStream_t st);
 hipError_t launch_bwd_feat(const BwdParams& p, const BwdPlan& pl, int D, int dtype, hipStream_t st, hipEvent_t* ev);
 
 // feat: the plan is for bf16 inputs or dropout, which have a smaller set of kernel instances
-FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, bool feat);
+// (`row`: the true row length)
+FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, int row, bool feat);
 
 // The kernels are gfx950 code objects: FTA_OK if the current device can run them (fta_api.hip).
 int check_device();
@@ -234,7 +235,7 @@ inline hipError_t launch_kernel(K kern, const P& p, dim3 grid, dim3 block, size_
 bool forced_general();
 hipError_t launch_fwd(FwdParams p, const FwdPlan& pl, int D, int dtype, hipStream_t st);
 // The hand-scheduled forward (fta_fwd1_kernel.h): D = 32, tiled length 64 ... 1792, no dropout.
-bool plan_fwd1(int B, int H, int L1, int L2, int D, FwdPlan& pl);
+bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, FwdPlan& pl);
 hipError_t launch_fwd1(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 grid, dim3 block, hipStream_t st);
 hipError_t launch_fwd1_slabs(const FwdParams& p, const FwdPlan& pl, int dtype, bool tl, dim3 grid, dim3 block, hipStream_t st);
 bool plan_fwd2(int B, int H, int L1, int L2, int D, FwdPlan& pl);

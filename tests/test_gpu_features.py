@@ -459,6 +459,25 @@ def test_precise_backward_holds_the_tolerance_on_large_biases_and_scores(bias_st
     assert max(e_pre.values()) < max(e_def.values())
 
 
+# ---- the hand-scheduled forward with an odd number of tiles per slab ----------------------------------------
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L1,L2,tiled", [(9, 129, 160), (5, 160, 160), (40, 224, 224), (3, 257, 288), (6, 288, 288), (8, 351, 352), (3, 416, 416), (7, 457, 480),
+                                         (3, 545, 576), (4, 576, 576), (5, 701, 704), (9, 704, 704), (3, 832, 832), (2, 950, 960),
+                                         (3, 1100, 1152), (2, 1152, 1152), (2, 1408, 1408), (2, 1601, 1664)])
+def test_forward_rows_of_an_odd_number_of_tiles(L1, L2, tiled, dtype):
+    """Stages of one tile (two barriers in a row) and of three, one, two and four slabs, whole rows and rows that end inside
+    a tile; the large scale takes the branch that raises a row's reference, in the tile that changes registers too."""
+    import fta_lib
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, 0.0, 0, 0)
+    plan = fta_lib.describe_plan(1, 2, L1, L2, 32, 1.0, opt)["fwd"]
+    assert plan["kernel"].startswith("fta_fwd1_kernel") and plan["tiled_length"] == tiled
+    for sm in (1.0 / math.sqrt(32), 1.3):
+        print(f"case odd tiles {L1}x{L2} {dtype} sm={sm:.2f}", flush=True)
+        q, k, v, b, do = _inputs(1, 2, L1, L2, 32, 43, dtype)
+        _compare(_run(q, k, v, b, sm, do), _oracle(q, k, v, b, sm, do), dtype, f"odd tiles {L1}x{L2}")
+
+
 # ---- the hand-scheduled backward at tiled lengths in steps of 64 -------------------------------------------
 
 @pytest.mark.parametrize("mode", ["fp16", "bf16", "bf16 operand pair", "precise"])
