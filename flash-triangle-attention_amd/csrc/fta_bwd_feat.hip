@@ -14,10 +14,14 @@
 namespace fta {
 
 hipError_t launch_dbias_reduce(const BwdParams& p, int dtype, hipStream_t st) {
-  const int64_t total4 = (int64_t)p.B * p.H * p.L2 * ((p.L2 + 3) / 4);
-  dim3 grid((unsigned)((total4 + 255) / 256)), block(256);
-  if (dtype == kBF16) hipLaunchKernelGGL(fta_dbias_reduce_kernel<BF16>, grid, block, 0, st, p);
-  else hipLaunchKernelGGL(fta_dbias_reduce_kernel<F16>, grid, block, 0, st, p);
+  const int in_bh = p.L2 * ((p.L2 + 3) / 4);
+  // shares of at least four chunks, until there are two waves for every SIMD
+  int split = 1;
+  while (split < 8 && (int64_t)p.B * p.H * in_bh * split < 2048 * 64 && p.nchunks >= 8 * split) split *= 2;
+  const int per_bh = (in_bh + 256 / split - 1) / (256 / split);
+  const dim3 grid((unsigned)(p.B * p.H * per_bh)), block(256);
+  if (dtype == kBF16) hipLaunchKernelGGL(fta_dbias_reduce_kernel<BF16>, grid, block, 0, st, p, split, per_bh);
+  else hipLaunchKernelGGL(fta_dbias_reduce_kernel<F16>, grid, block, 0, st, p, split, per_bh);
   return hipGetLastError();
 }
 

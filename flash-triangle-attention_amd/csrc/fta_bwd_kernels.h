@@ -835,24 +835,38 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
 // ------------------------------------------------------------------------------------------------
 // 3. dBias stage two: fixed-order sum of the chunk partials, fp32 -> fp16
 // ------------------------------------------------------------------------------------------------
+// `split` threads share a group of four consecutive keys of a row of the (B*H, L2, L2) result (the last group of a row may
+// hold fewer), each a share of the chunks: short rows have too few groups and too many chunks for one thread each (B1 H4
+// L128, 64 chunks: 17 us, a chain of 64 loads on a quarter of the chip; 4.7 with eight; L192 9.2 -> 4.9).  The partial sums are laid out
+// with the padded length L2p.  `per_bh` workgroups take one (b,h).
 template <class T>
-__global__ void __launch_bounds__(256) fta_dbias_reduce_kernel(const BwdParams p) {
-  // one thread per group of four consecutive keys of a row of the (B*H, L2, L2) result (the last group
-  // of a row may hold fewer); the partial sums are laid out with the padded length L2p
-  const int groups = (p.L2 + 3) / 4;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)p.B * p.H * p.L2 * groups) return;
-  const int k = 4 * (int)(idx % groups);
-  const int j = (int)((idx / groups) % p.L2);
-  const int bh = (int)(idx / ((int64_t)groups * p.L2));
+__global__ void __launch_bounds__(256) fta_dbias_reduce_kernel(const BwdParams p, int split, int per_bh) {
+  __shared__ float4 part[256];
+  const int groups = (p.L2 + 3) / 4, items = 256 / split, share = (int)threadIdx.x / items;
+  const int bh = (int)blockIdx.x / per_bh;
+  const int item = ((int)blockIdx.x - bh * per_bh) * items + (int)threadIdx.x % items;
+  const bool mine = item < p.L2 * groups;
+  const int j = mine ? item / groups : 0, k = mine ? 4 * (item - j * groups) : 0;
   const int n = min(4, p.L2 - k);
   float4 acc = {0.f, 0.f, 0.f, 0.f};
   const int64_t chunk_stride = (int64_t)p.B * p.H * p.L2p * p.L2p;
   const float* src = p.partial + ((int64_t)bh * p.L2p + j) * p.L2p + k;
-  for (int c = 0; c < p.nchunks; ++c) {
-    const float4 v = *reinterpret_cast<const float4*>(src + c * chunk_stride);
-    acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+  if (mine) {
+#pragma unroll 4
+    for (int c = share; c < p.nchunks; c += split) {
+      const float4 v = *reinterpret_cast<const float4*>(src + c * chunk_stride);
+      acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+    }
   }
+  if (split > 1) {  // the shares, in order
+    part[threadIdx.x] = acc;
+    __syncthreads();
+    for (int s = 1; s < split && share == 0; ++s) {
+      const float4 v = part[threadIdx.x + s * items];
+      acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+    }
+  }
+  if (!mine || share != 0) return;
   acc.x *= p.partial_scale; acc.y *= p.partial_scale; acc.z *= p.partial_scale; acc.w *= p.partial_scale;
   const int64_t off = (bh / p.H) * p.dbs[0] + (bh % p.H) * p.dbs[1] + (int64_t)j * p.dbs[2] + k;
   // (one vector store where the group is whole and its address allows it; rows of a length that is not a
