@@ -59,7 +59,7 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
     const int nb = (r + steps1 - 1) / steps1;  // rows whose operand tiles can be in flight at once
     if (r * slot1 + nb * qtile1 + part1 <= lds_max) { pl.ring = r; pl.nb = nb; pl.smem = r * slot1 + nb * qtile1 + part1; break; }
   }
-  pl.nchunks = balanced_chunks((long)B * H * pl.nqg, L1, 256);
+  pl.nchunks = balanced_chunks((long)B * H * pl.nqg, L1, 256, least_rows(L2));
   pl.rows_per_chunk = (L1 + pl.nchunks - 1) / pl.nchunks;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   // ---- dK/dV kernel: query slabs of at most 256 (D=32) / 128 (D=64) queries per wave (register
@@ -99,7 +99,7 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
       }
     }
   }
-  pl.nchunks2 = balanced_chunks((long)B * H * (ok2 ? pl.nkg : 1), L1, 256);
+  pl.nchunks2 = balanced_chunks((long)B * H * (ok2 ? pl.nkg : 1), L1, 256, least_rows(L2));
   pl.rows_per_chunk2 = (L1 + pl.nchunks2 - 1) / pl.nchunks2;
   pl.nchunks2 = (L1 + pl.rows_per_chunk2 - 1) / pl.rows_per_chunk2;
 

@@ -34,7 +34,7 @@ bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl) {
     pl.smem_range[n] = smem;
     if (smem > pl.smem) pl.smem = smem;
   }
-  const int nch = balanced_chunks((long)B * H * pl.nkg, L1, 256);  // one workgroup per CU
+  const int nch = balanced_chunks((long)B * H * pl.nkg, L1, 256, least_rows(L2));  // one workgroup per CU
   pl.rows_per_chunk = (L1 + nch - 1) / nch;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   return true;

@@ -91,7 +91,7 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int
   // L1-row chunks: enough workgroups to fill 256 CUs a few times over, rows >= 8 per chunk
   // (two of the 4-wave workgroups fit a CU, one of the larger ones)
   const long slots = (pl.threads <= 128 && pl.smem <= 40 * 1024) ? 1024 : (pl.threads <= 256 && pl.smem <= 80 * 1024) ? 512 : 256;
-  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, slots);
+  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, slots, pl.S > 1 ? 8 : least_rows(L2));
   pl.rows_per_chunk = (L1 + nch - 1) / nch;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   pl.valid = (pl.S * pl.QB <= 8) && (pl.KT != 0);

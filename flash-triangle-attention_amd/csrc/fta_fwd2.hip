@@ -541,7 +541,7 @@ bool plan_fwd2(int B, int H, int L1, int L2, int D, FwdPlan& pl) {
   pl.KT = 64;
   pl.smem = (size_t)4 * pl.S * 2 * 64 * 64 * 2 + (pl.S == 2 ? 8 * (2048 + 512) : 0);  // four slots; the merge records
   pl.alias_scratch = 0;
-  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, 256);  // one workgroup per CU
+  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, 256, least_rows(L2));  // one workgroup per CU
   pl.rows_per_chunk = (L1 + nch - 1) / nch;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   pl.fwd1 = 2;

@@ -72,6 +72,11 @@ inline int balanced_chunks(long base, int L1, long slots, int least = 8) {
   return best;
 }
 
+// The fewest rows of a chunk for rows of L2 keys: a workgroup's set-up loads one bias row per query, so that short rows
+// can be spread thinner over the chip than eight to a workgroup (B1 H4, us, eight -> this: forward at D = 64, L48 23.7 -> 9.5,
+// L192 48.1 -> 28.4; step with dropout at D = 32, L192 217 -> 138, L256 215 -> 170).
+inline int least_rows(int L2) { return L2 >= 512 ? 8 : L2 <= 128 ? 2 : L2 / 64; }
+
 // ---- backward ---------------------------------------------------------------------------------
 
 struct BwdParams {
