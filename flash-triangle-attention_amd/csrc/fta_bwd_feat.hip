@@ -39,7 +39,19 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
   mark(1);
   {  // 1. dQ, dBias partials
     dim3 grid((unsigned)(p.B * p.H * pl.nqg * pl.nchunks)), block((unsigned)pl.threads);
-    for (int n = 0; n < pl.nlaunch; ++n) {
+    if (pl.nranges > 0) {
+      if constexpr (DROP)
+        for (int n = 0, at = 0; n < pl.nranges; at += pl.range[n++]) {
+          const DropRange r = drop_range(pl.range[n]);
+          p.kr0 = at; p.ring = r.dq.r; p.nb = r.dq.nb;
+          e = pl.range[n] == 512   ? launch_kernel(fta_bwd_dq_kernel<T, true, 32, 2>, p, grid, block, r.smem, st)
+              : pl.range[n] == 384 ? launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 3, 4>, p, grid, block, r.smem, st)
+              : pl.range[n] == 256 ? launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 2, 4>, p, grid, block, r.smem, st)
+                                   : hipErrorInvalidConfiguration;
+          if (e != hipSuccess) return e;
+        }
+    }
+    for (int n = 0; n < (pl.nranges > 0 ? 0 : pl.nlaunch); ++n) {
       p.kr0 = n * pl.KR;
       e = hipErrorInvalidConfiguration;
       if (pl.NKT == 3) {  // key ranges of 384 keys with dropout: fixed geometry
@@ -58,21 +70,34 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
   mark(2);
   {  // 2. dK, dV
     dim3 grid((unsigned)(p.B * p.H * pl.nkg * pl.nchunks2)), block((unsigned)pl.threads2);
-    for (int n = 0; n < pl.nlaunch2; ++n) {
+    if (pl.nranges > 0) {
+      if constexpr (DROP)
+        for (int n = 0, at = 0; n < pl.nranges; at += pl.range[n++]) {
+          const DropRange r = drop_range(pl.range[n]);
+          p.jr0 = at;
+          e = pl.range[n] == 512   ? launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, 8, 64, 2>, p, grid, block, r.smem2, st)
+              : pl.range[n] == 384 ? launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, 6, 64, 2>, p, grid, block, r.smem2, st)
+              : pl.range[n] == 256 ? launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, 4, 64, 2>, p, grid, block, r.smem2, st)
+                                   : hipErrorInvalidConfiguration;
+          if (e != hipSuccess) return e;
+        }
+    }
+    for (int n = 0; n < (pl.nranges > 0 ? 0 : pl.nlaunch2); ++n) {
       p.jr0 = n * pl.JR;
       e = hipErrorInvalidConfiguration;
 #define FTA_DKDV_FEAT_CASE(DD, NN, JJ) \
   if (e == hipErrorInvalidConfiguration && D == DD && pl.NJT == NN && pl.JT == JJ) \
     e = launch_kernel(fta_bwd_dkdv_kernel<T, DROP, DD, NN, JJ>, p, grid, block, pl.smem2, st);
-      if constexpr (DROP) {  // fixed geometry: query ranges of 256, 384, 512 and 1024 queries
+      if constexpr (DROP) {  // fixed geometry: rows of 256, 384 and 512 queries
 #define FTA_DKDV_FIX_CASE(NN, SS)                                                                                        \
   if (D == 32 && pl.threads2 == 512 && pl.NJT == NN && pl.JT == 64 && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, 64, SS).r &&  \
       pl.nb2 == dkdv_ring(32, NN, 64, SS).nb)                                                                            \
     e = launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, NN, 64, SS>, p, grid, block, pl.smem2, st);
-        FTA_DKDV_FIX_CASE(6, 2) FTA_DKDV_FIX_CASE(8, 1) FTA_DKDV_FIX_CASE(8, 2) FTA_DKDV_FIX_CASE(8, 4)
+        FTA_DKDV_FIX_CASE(6, 2) FTA_DKDV_FIX_CASE(8, 1) FTA_DKDV_FIX_CASE(8, 2)
 #undef FTA_DKDV_FIX_CASE
       }
-      FTA_DKDV_FEAT_CASE(32, 8, 64) FTA_DKDV_FEAT_CASE(32, 4, 64)
+      if constexpr (!DROP) { FTA_DKDV_FEAT_CASE(32, 8, 64) }
+      FTA_DKDV_FEAT_CASE(32, 4, 64)
       FTA_DKDV_FEAT_CASE(64, 4, 64) FTA_DKDV_FEAT_CASE(64, 4, 32)
 #undef FTA_DKDV_FEAT_CASE
       if (e != hipSuccess) return e;

@@ -164,6 +164,8 @@ struct BwdPlan {
   bool use_hand;       // the hand-scheduled one-wave-per-SIMD kernels run
   Dq1Plan dq1;
   Dkdv1Plan dkdv1;
+  int nranges;         // dropout beyond 512 keys: ranges of their own geometry (see drop_range), else 0
+  int range[kMaxRanges];
   bool use_short;      // rows of up to 128 keys: all gradients in one kernel
   ShortPlan sh;
   int L2p;             // the length the workspace is laid out with and the general kernels' tiles cover (filled in by the C-ABI layer)
@@ -207,6 +209,19 @@ constexpr Ring dq_ring(int D, int NKT, int G1, int SK) {
 }
 constexpr Ring dkdv_ring(int D, int NJT, int JT, int SJ) {
   return fit_ring(NJT / (JT / 32), 4 * SJ * JT * D + 8 * SJ * JT, 4 * (8 / SJ) * 32 * D, (SJ - 1) * (8 / SJ) * 32 * (D / 32) * 64 * 2);
+}
+
+// One key range and one query range of the backward with dropout beyond 512 keys (D = 32): stage and row-operand
+// buffers and LDS bytes of the dQ/dBias kernel with four slabs and of the dK/dV kernel with two.
+struct DropRange { Ring dq, dkdv; size_t smem, smem2; };
+inline DropRange drop_range(int len) {
+  const int nkt = len / 128, g1 = nkt == 4 ? 2 : 1, njt = len / 64;
+  DropRange r;
+  r.dq = dq_ring(32, nkt, g1, 4);
+  r.dkdv = dkdv_ring(32, njt, 64, 2);
+  r.smem = (size_t)r.dq.r * (4 * 4 * g1 * 32 * 32) + (size_t)r.dq.nb * (4 * 2 * 32 * 32) + 8 * 16 * 64 * 4;
+  r.smem2 = (size_t)r.dkdv.r * (4 * 2 * 64 * 32 + 8 * 2 * 64) + (size_t)r.dkdv.nb * (4 * 4 * 32 * 32) + 4 * 32 * 64 * 2;
+  return r;
 }
 
 // L2 is the length the tiles cover (a multiple of 128), `row` the true row length.
