@@ -20,12 +20,20 @@
 // are loaded.  proj and dx have four to five times the weights: there the waves of a workgroup keep them in registers,
 // one or two tiles of output channels each, and share the rows through LDS (see "staged row tiles" below).
 //
-// fp32 blocks run the fp32 matrix instructions (v_mfma_f32_32x32x2_f32): nothing is rounded to 16 bits
-// that was not before (q, k, v, bias, o and their gradients).
+// fp32 blocks: the fp32 matrix instructions run at a sixteenth of the bf16 ones' rate and bounded every kernel (training pass
+// at 192 x 192 pairs: 283 us in these kernels).  So an fp32 operand is taken apart into three bf16 ones, x = x1 + x2 + x3, which
+// hold its 24 bits, and a product of two is six bf16 products summed in fp32 (x1 y1, x1 y2, x2 y1, x1 y3, x2 y2, x3 y1; what is
+// left out is below 2^-24 of the product).  Activations are taken apart where they enter LDS, weights on their way into
+// registers or LDS.  Against 64 bits (relative L2, 192 x 192 pairs, fp32 instructions / three parts): gate 8.0e-8 / 7.1e-8, out
+// 1.6e-7 / 1.3e-7, dz 2.9e-7 / 2.3e-7, weight gradients 4.0e-7 / 1.8e-7 (wo) to 3.6e-7 (wb): the matrix core sums 16 products
+// at once, the fp32 instruction two.  Infinity and values beyond the largest bf16 (3.39e38) have no three parts: what they
+// enter comes out as NaN.  Nothing is rounded to 16 bits in memory that was not before (q, k, v, bias, o and their gradients).
+// us per kernel at 192 x 192 pairs, before and after: proj 69 / 47, out 32 / 26, dout 29 / 28, dx 57 / 48, wgrad 82 / 55; a
+// training pass 352 / 265 (256 x 256: 498 / 394, 321 x 321: 838 / 670), inference 112 / 82 (457 x 457: 505 / 387).
 //
 // Measured, AlphaFold2's block (C 128, 4 heads of 32) at 384 x 384 pairs in bf16: a training pass 3.64 ms as separate
 // library calls around the attention, 0.52 with these; us per kernel (rocprofv3, mean of 30 launches): proj 56, out
-// 30, dout 43, dx 55, wgrad 88, reduce 10, norm_grad 5.
+// 30, dout 43, dx 54, wgrad 82, reduce 10, norm_grad 5.
 #include "fta_block.h"
 
 #include <type_traits>
@@ -45,16 +53,57 @@ template <> struct Frag<true> { float v[8]; };
 template <bool F32> struct Store { typedef uint16_t type; };
 template <> struct Store<true> { typedef float type; };
 
-template <class A>
-__device__ __forceinline__ floatx16 mma(const Frag<false>& a, const Frag<false>& b, floatx16 c) {
-  return A::mfma(as_half8(a.w), as_half8(b.w), c);
-}
-template <class A>
-__device__ __forceinline__ floatx16 mma(const Frag<true>& a, const Frag<true>& b, floatx16 c) {
-  // (element e of the two lane halves is one contraction pair: the same order for both operands)
+// The same as matrix core operands: the 16-bit values as they are, fp32 ones as three planes of bf16, largest first.
+template <bool F32> struct Op { u32x4 p[F32 ? 3 : 1]; };
+template <bool HERE = false>
+__device__ __forceinline__ Op<false> to_op(const Frag<false>& f) { return Op<false>{{f.w}}; }
+// (HERE: in place, every time.  Weights are the same in every pass of a loop, and their planes, taken out of it, do not fit
+// the registers.)
+template <bool HERE = false>
+__device__ __forceinline__ Op<true> to_op(const Frag<true>& f) {
+  Op<true> o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a.v[e], b.v[e], c, 0, 0, 0);
-  return c;
+  for (int e = 0; e < 4; ++e) {
+    float a = f.v[2 * e], b = f.v[2 * e + 1];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {  // (the differences are exact)
+      uint32_t w;
+      if constexpr (HERE) {
+        // (two idle slots behind the last of them, in front of an MFMA that the compiler may put there)
+        if (n == 0 && e < 3) asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(w) : "v"(a), "v"(b));
+        else if (n == 0) asm volatile("v_cvt_pk_bf16_f32 %0, %1, %2\n\ts_nop 1" : "=v"(w) : "v"(a), "v"(b));
+        else w = BF16::pack(a, b);
+      } else {
+        w = BF16::pack(a, b);
+      }
+      o.p[n][e] = w;
+      a -= BF16::lo(w);
+      b -= BF16::hi(w);
+    }
+  }
+  return o;
+}
+template <class A, int PA = 3, bool LONG = false>
+__device__ __forceinline__ floatx16 mma(const Op<false>& a, const Op<false>& b, floatx16 c) {
+  return A::mfma(as_half8(a.p[0]), as_half8(b.p[0]), c);
+}
+// (PA: planes of `a` that are not zero: two hold the 11 bits of an fp16 value.  LONG: a sum over many steps; the small
+// products are summed by themselves first, so that the long sum is rounded twice a step and not six times)
+template <class A, int PA = 3, bool LONG = false>
+__device__ __forceinline__ floatx16 mma(const Op<true>& a, const Op<true>& b, floatx16 c) {
+  constexpr int at[6][2] = {{2, 0}, {0, 2}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};
+  floatx16 t = c;
+  if constexpr (LONG)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] = 0.f;
+#pragma unroll
+  for (int n = PA == 3 ? 0 : 1; n < (LONG ? 5 : 6); ++n) t = BF16::mfma(as_half8(a.p[at[n][0]]), as_half8(b.p[at[n][1]]), t);
+  if constexpr (LONG) {
+    c = BF16::mfma(as_half8(a.p[0]), as_half8(b.p[0]), c);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) t[r] += c[r];
+  }
+  return t;
 }
 
 template <class A>
@@ -151,6 +200,23 @@ __device__ __forceinline__ Frag<F32> frag_zero() {
   return f;
 }
 
+// Operands in LDS: a 16-byte plane of 64 lanes each, three for fp32.
+template <bool F32> constexpr int kOpBytes = F32 ? 3072 : 1024;
+template <bool F32>
+__device__ __forceinline__ Op<F32> op_read(const char* ops, int idx, int lane) {
+  Op<F32> o;
+  const char* s = ops + (size_t)idx * kOpBytes<F32> + lane * 16;
+#pragma unroll
+  for (int n = 0; n < kOpBytes<F32> / 1024; ++n) o.p[n] = *reinterpret_cast<const u32x4*>(s + n * 1024);
+  return o;
+}
+template <bool F32>
+__device__ __forceinline__ void op_write(char* ops, int idx, int lane, const Op<F32>& o) {
+  char* d = ops + (size_t)idx * kOpBytes<F32> + lane * 16;
+#pragma unroll
+  for (int n = 0; n < kOpBytes<F32> / 1024; ++n) *reinterpret_cast<u32x4*>(d + n * 1024) = o.p[n];
+}
+
 // An accumulator tile (lane: column l % 32; register r: row 8*(r/4) + 4*hh + r%4) as two runs of eight
 // consecutive rows per lane: out[u][e] is row 16*u + 8*hh + e.
 __device__ __forceinline__ void rows8(const floatx16& acc, float (&out)[2][8]) {
@@ -174,7 +240,7 @@ __device__ __forceinline__ floatx16 zero16() {
 
 template <bool F32>
 __device__ __forceinline__ float sigmoid(float x) {
-  if constexpr (F32) return 1.0f / (1.0f + expf(-x));
+  if constexpr (F32) return __builtin_amdgcn_rcpf(1.0f + expf(-x));
   else return __builtin_amdgcn_rcpf(1.0f + exp2_fast(-kLog2e * x));
 }
 
@@ -235,7 +301,7 @@ __device__ __forceinline__ void normalise(float (&v)[8], float eps, float& mean,
   s = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) { v[e] -= mean; s = __builtin_fmaf(v[e], v[e], s); }
-  rstd = 1.0f / __builtin_sqrtf(row_sum<C / 8>(s) * (1.0f / C) + eps);
+  rstd = __builtin_amdgcn_rsqf(row_sum<C / 8>(s) * (1.0f / C) + eps);  // (to one unit in the last place; a root and a division are 25 instructions)
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] *= rstd;
 }
@@ -248,39 +314,45 @@ __device__ __forceinline__ void normalise(float (&v)[8], float eps, float& mean,
 // pieces of a row, which neighbouring threads write at once, over the banks.
 template <bool F32>
 __device__ __forceinline__ void piece_write(char* blk, int r, int c, const Frag<F32>& f) {
-  frag_write<F32>(blk, c / 2, (r ^ (c % 16)) + 32 * (c % 2), f);
+  op_write<F32>(blk, c / 2, (r ^ (c % 16)) + 32 * (c % 2), to_op(f));
 }
 template <bool F32>
-__device__ __forceinline__ Frag<F32> piece_frag(const char* blk, int ks, int l32, int hh) {
-  return frag_read<F32>(blk, ks, (l32 ^ ((2 * ks + hh) % 16)) + 32 * hh);
+__device__ __forceinline__ Op<F32> piece_frag(const char* blk, int ks, int l32, int hh) {
+  return op_read<F32>(blk, ks, (l32 ^ ((2 * ks + hh) % 16)) + 32 * hh);
 }
 
 // ---- forward: layer norm and projections --------------------------------------------------------------
 // A wave keeps the weights of one or two tiles of 32 output channels (4*HD/32 tiles of q, k, v, gate over eight
-// waves) in registers, 64 or 128 of them; the bias heads are one more tile, its weights in LDS, that the waves take
+// waves) in registers, 64 of them; the bias heads are one more tile, its weights in LDS, that the waves take
 // turns at.  The next stage's loads and its layer norm overlap this stage's products (two stage buffers).
+// fp32: a tile's three planes take 96 registers, so that a wave keeps one tile and two workgroups of the same die share the
+// output tiles of a row (each reads and normalises it); the bias heads are dot products of the threads that hold the row, in
+// the first of the two (a tile more for one of eight waves that meet at every stage's barrier costs half as much
+// again): 47 us at 192 x 192 pairs.  With both tiles' weights in fp32 and taken apart at every use, proj took 55, by fp32
+// matrix instructions 69.
 template <class A, bool F32, int C, int HD>
 __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
-  constexpr int KS = C / 16, NT = HD / 64;           // NT: tiles per wave
+  constexpr int PARTS = F32 ? HD / 64 : 1;           // workgroups that share a row's tiles
+  constexpr int KS = C / 16, NT = HD / 64 / PARTS;   // NT: tiles per wave
   constexpr int TR = F32 ? 32 : 64, RS = TR / 32;    // rows per stage (fp32: half, so that few rows still load the CUs evenly)
   constexpr int NP = (TR * C / 8 + 511) / 512;       // pieces per thread
-  constexpr int SUB = KS * kFragBytes<F32>, BUF = RS * SUB;
+  constexpr int SUB = KS * kOpBytes<F32>, BUF = RS * SUB;
   extern __shared__ char smem[];
   char* wbf = smem + 2 * BUF;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
   float* bgs = reinterpret_cast<float*>(wbf + SUB);
   float* msk = bgs + HD;  // what the mask adds to the bias of a stage's rows, two buffers
-  Frag<F32> w[NT][KS];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int n = (wave * NT + t) * 32 + l32, sec = n / HD;
-      w[t][ks] = load8<F32>(p.w[sec], (int64_t)(n - sec * HD) * C + ks * 16 + hh * 8);
-    }
-  for (int ks = wave; ks < KS; ks += 8)
-    frag_write<F32>(wbf, ks, lane, l32 < p.H ? load8<F32>(p.wb, (int64_t)l32 * C + ks * 16 + hh * 8) : frag_zero<F32>());
+  // (the parts of a row are a multiple of the dies apart where the launch fills the chip)
+  const int teams = (int)gridDim.x / PARTS, part = (int)blockIdx.x / teams;
+  auto tile_of = [=](int t) { return (t * 8 + wave) * PARTS + part; };  // (the gate's tiles, which have the sigmoid besides, spread over waves and parts)
   const int c8 = (tid % (C / 8)) * 8;
+  float wbv[F32 ? 4 : 1][8];  // (fp32) the bias heads' weights of this thread's channels
+  if constexpr (F32) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) wbv[h][e] = h < p.H ? load1<A, F32>(p.wb, h * C + c8 + e) : 0.f;
+  }
   float gam[8], bet[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) { gam[e] = load1<A, F32>(p.gamma, c8 + e); bet[e] = load1<A, F32>(p.beta, c8 + e); }
@@ -290,11 +362,12 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
   Frag<F32> z[NP];
   float mrow;
   const void* mask = p.mask != nullptr ? p.mask : p.gamma;  // (loaded either way, see the stores)
-  for (int c = tid; c < HD; c += 512) bgs[c] = p.bg != nullptr ? load1<A, F32>(p.bg, c) : 0.f;
+  int zst = 0;  // the stage in z
   auto fetch = [&](int st) {
     const int b = st / nst, p0 = (st - b * nst) * TR;
+    zst = st;
     {
-      const uint32_t q = (uint32_t)min(p0 + tid % TR, LL - 1), i = div_by_length(q, (uint32_t)p.L, inv_l);
+      const uint32_t q = (uint32_t)min(p0 + (F32 ? tid / (C / 8) : tid) % TR, LL - 1), i = div_by_length(q, (uint32_t)p.L, inv_l);
       mrow = load1<A, F32>(mask, p.mask != nullptr ? (int64_t)b * p.L + (q - i * (uint32_t)p.L) : 0);
     }
 #pragma unroll
@@ -307,7 +380,8 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
   auto put = [&](int buffer) {
     char* buf = smem + buffer * BUF;
     // 0 marks padded key positions, which no query may attend to
-    if (tid < TR) msk[buffer * TR + tid] = p.mask != nullptr ? (mrow - 1.0f) * 30000.0f : 0.f;
+    const float add = p.mask != nullptr ? (mrow - 1.0f) * 30000.0f : 0.f;
+    if (!F32 && tid < TR) msk[buffer * TR + tid] = add;
 #pragma unroll
     for (int n = 0; n < NP; ++n) {
       const int row = (tid + 512 * n) / (C / 8);
@@ -316,19 +390,46 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
       normalise<C>(v, p.eps, mean, rstd);
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = __builtin_fmaf(v[e], gam[e], bet[e]);
+      if constexpr (F32) {
+        if (part == 0) {
+          const int b = zst / nst, q = min((zst - b * nst) * TR + row, LL - 1), h = c8 / 8;
+          float own = 0.f;
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            float s = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s = __builtin_fmaf(v[e], wbv[g][e], s);
+            s = row_sum<C / 8>(s);
+            own = h == g ? s : own;
+          }
+          if (h < p.H && row < TR) store1<A, false>(p.bias, ((int64_t)b * p.H + h) * LL + q, own + add);
+        }
+      }
       Frag<F32> f;
       pack<A>(v, f);
       if (TR * C / 8 >= 512 || row < TR) piece_write<F32>(buf + (row / 32) * SUB, row % 32, c8 / 8, f);
     }
   };
-  int st = (int)blockIdx.x;
+  int st = (int)blockIdx.x - part * teams;
+  if (st < ntot) fetch(st);  // (in flight while the weights come in)
+  Op<F32> w[NT][KS];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int n = tile_of(t) * 32 + l32, sec = n / HD;
+      w[t][ks] = to_op(load8<F32>(p.w[sec], (int64_t)(n - sec * HD) * C + ks * 16 + hh * 8));
+    }
+  if constexpr (!F32)
+    for (int ks = wave; ks < KS; ks += 8)
+      op_write<F32>(wbf, ks, lane, to_op(l32 < p.H ? load8<F32>(p.wb, (int64_t)l32 * C + ks * 16 + hh * 8) : frag_zero<F32>()));
+  for (int c = tid; c < HD; c += 512) bgs[c] = p.bg != nullptr ? load1<A, F32>(p.bg, c) : 0.f;
   if (st < ntot) {
-    fetch(st);
     put(0);
-    fetch(min(st + (int)gridDim.x, ntot - 1));
+    fetch(min(st + teams, ntot - 1));
   }
   __syncthreads();
-  for (int it = 0; st < ntot; st += (int)gridDim.x, ++it) {
+  auto products = [&](int st, int it) {
     const char* buf = smem + (it & 1) * BUF;
     const int b = st / nst, p0 = (st - b * nst) * TR;
 #pragma unroll
@@ -341,13 +442,13 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
       for (int t = 0; t < NT; ++t) acc[t] = zero16();
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        const Frag<F32> x = piece_frag<F32>(buf + rs * SUB, ks, l32, hh);
+        const Op<F32> x = piece_frag<F32>(buf + rs * SUB, ks, l32, hh);
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[t] = mma<A>(w[t][ks], x, acc[t]);
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const int n = (wave * NT + t) * 32, sec = n / HD, col = n - sec * HD, h = col / p.D;
+        const int n = tile_of(t) * 32, sec = n / HD, col = n - sec * HD, h = col / p.D;
         const int64_t off = (((int64_t)b * p.H + h) * LL + q) * p.D + (col - h * p.D) + hh * 8;
         float y[2][8];
         rows8(acc[t], y);
@@ -366,11 +467,11 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
           }
         }
       }
-      if (wave == ((RS * it + rs) & 7)) {
+      if (!F32 && wave == ((RS * it + rs) & 7)) {
         floatx16 ab = zero16();
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-          ab = mma<A>(frag_read<F32>(wbf, ks, lane), piece_frag<F32>(buf + rs * SUB, ks, l32, hh), ab);
+          ab = mma<A>(op_read<F32>(wbf, ks, lane), piece_frag<F32>(buf + rs * SUB, ks, l32, hh), ab);
         const float add = msk[(it & 1) * TR + rs * 32 + l32];
         if (hh == 0)
 #pragma unroll
@@ -378,8 +479,17 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
             if (h < p.H) store1<A, false>(p.bias, ((int64_t)b * p.H + h) * LL + q, ab[h] + add);
       }
     }
+  };
+  // Half of the waves (one of the two that share a SIMD) prepare the next stage first and multiply then, the others the other
+  // way round, so that one wave's products run beside the other's layer norm.
+  auto prepare = [&](int st, int it) {
     put((it + 1) & 1);  // (behind the last stage: once more the last rows, into the buffer nobody reads)
-    fetch(min(st + 2 * (int)gridDim.x, ntot - 1));
+    fetch(min(st + 2 * teams, ntot - 1));
+  };
+  for (int it = 0; st < ntot; st += teams, ++it) {
+    if (wave >= 4) prepare(st, it);
+    products(st, it);
+    if (wave < 4) prepare(st, it);
     __syncthreads();
   }
 }
@@ -391,9 +501,9 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
   extern __shared__ char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
   const int nw = blockDim.x >> 6;
-  float* bos = reinterpret_cast<float*>(smem + (size_t)NT * KS * kFragBytes<F32>);
+  float* bos = reinterpret_cast<float*>(smem + (size_t)NT * KS * kOpBytes<F32>);
   for (int idx = wave; idx < NT * KS; idx += nw)
-    frag_write<F32>(smem, idx, lane, load8<F32>(p.wo, (int64_t)((idx / KS) * 32 + l32) * HD + (idx % KS) * 16 + hh * 8));
+    op_write<F32>(smem, idx, lane, to_op(load8<F32>(p.wo, (int64_t)((idx / KS) * 32 + l32) * HD + (idx % KS) * 16 + hh * 8)));
   for (int c = tid; c < C; c += blockDim.x) bos[c] = p.bo != nullptr ? load1<A, F32>(p.bo, c) : 0.f;
   __syncthreads();
 
@@ -416,7 +526,7 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
   for (; item < nitems; item += step) {
     const RowBlock cur = rb;
     const int g = item % p.cg;
-    Frag<F32> x[KS];
+    Op<F32> x[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       float a[8], b[8];
@@ -424,7 +534,9 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
       unpack<A>(o[ks], b);
 #pragma unroll
       for (int e = 0; e < 8; ++e) a[e] *= b[e];
-      pack<A>(a, x[ks]);
+      Frag<F32> f;
+      pack<A>(a, f);
+      x[ks] = to_op(f);
     }
     if (item + step < nitems) {
       rb = row_block(p, (item + step) / p.cg, lane);
@@ -434,7 +546,7 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
     for (int t = g; t < NT; t += p.cg) {
       floatx16 acc = zero16();
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) acc = mma<A>(frag_read<F32>(smem, t * KS + ks, lane), x[ks], acc);
+      for (int ks = 0; ks < KS; ++ks) acc = mma<A>(op_read<F32>(smem, t * KS + ks, lane), x[ks], acc);
       float y[2][8];
       rows8(acc, y);
 #pragma unroll
@@ -482,19 +594,22 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
     for (int e = 0; e < 8; ++e) v[e] = load1<A, F32>(p.wo, (int64_t)((idx % KS) * 16 + hh * 8 + e) * HD + (idx / KS) * 32 + l32);
     Frag<F32> f;
     pack<A>(v, f);
-    frag_write<F32>(smem, idx, lane, f);
+    op_write<F32>(smem, idx, lane, to_op(f));
   }
   __syncthreads();
 
   const int nitems = p.B * p.nper * p.cg, step = p.nwg * nw;
   int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * nw + wave);
   if (item >= nitems) return;
-  Frag<F32> x[KS];
+  Op<F32> x[KS];
   RowBlock rb = row_block(p, item / p.cg, lane);
   auto fetch = [&]() {
     const int64_t so = pair_off(p.douts, rb) + hh * 8;
+    Frag<F32> f[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) x[ks] = load8<F32>(p.dout, so + ks * 16);
+    for (int ks = 0; ks < KS; ++ks) f[ks] = load8<F32>(p.dout, so + ks * 16);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) x[ks] = to_op(f[ks]);
   };
   fetch();
   for (; item < nitems; item += step) {
@@ -509,7 +624,7 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
       for (int u = 0; u < 2; ++u) { gt[u] = load8<F32>(p.gate, off + 16 * u); o[u] = load8<false>(p.o, off + 16 * u); }
       floatx16 acc = zero16();
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) acc = mma<A>(frag_read<F32>(smem, t * KS + ks, lane), x[ks], acc);
+      for (int ks = 0; ks < KS; ++ks) acc = mma<A>(op_read<F32>(smem, t * KS + ks, lane), x[ks], acc);
       float y[2][8];
       rows8(acc, y);
 #pragma unroll
@@ -542,9 +657,10 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
 // ---- backward: input gradient and layer norm ----------------------------------------------------------
 // dx = sum of the five projections' input gradients, one product with 4*HD + 16 contraction elements (the bias
 // heads padded to one 16-wide step).  A wave keeps the transposed weights of 32 channels in registers (132 of them in
-// bf16; fp32: half of the contraction, 136), the rows' gradients go through LDS once, and dx comes back
-// through LDS in fp32 (one plane per share of the contraction) to the threads that hold the rows of z in the layer norm's layout: 8 channels
-// of a row each, so that dz leaves in whole lines.
+// bf16; fp32: half of the contraction as fp32, 136, taken apart at every use because its planes, 204, do not fit beside
+// the rest), the rows' gradients go through LDS once, and dx comes back through LDS in fp32 (one plane per share of the
+// contraction) to the threads that hold the rows of z in the layer norm's layout: 8 channels of a row each, so that dz
+// leaves in whole lines.
 template <class A, bool F32, int C, int HD>
 __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
   constexpr int TR = F32 ? 32 : 64, RS = TR / 32, NT = C / 32;
@@ -552,7 +668,7 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
   constexpr int KH = HD / 16, KALL = 4 * KH + 1, KW = (KALL + SPLIT - 1) / SPLIT;
   constexpr int NP = TR * HD / 8 / 512;                  // pieces per thread of a section
   constexpr int NZ = (TR * C / 8 + 511) / 512;           // pieces of z
-  constexpr int SUB = KALL * kFragBytes<F32>;
+  constexpr int SUB = KALL * kOpBytes<F32>;
   constexpr int XROW = C + 4;                            // floats per row of a dx plane
   static_assert(NP >= 1 || F32, "pieces");
   constexpr int NPP = NP > 0 ? NP : 1;
@@ -560,12 +676,6 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
   float* dxs = reinterpret_cast<float*>(smem + RS * SUB);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
   const int ct = wave % NT, rs = (wave / NT) % RS, share = wave / (NT * RS);
-  Frag<F32> w[KW];
-#pragma unroll
-  for (int k = 0; k < KW; ++k) {
-    const int ks = share * KW + k;
-    w[k] = ks < KALL ? frag_read<F32>(static_cast<const char*>(p.wt), ct * KALL + ks, lane) : frag_zero<F32>();
-  }
   const int c8 = (tid % (C / 8)) * 8;
   float gam[8];
 #pragma unroll
@@ -624,7 +734,14 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
     }
   };
   int st = (int)blockIdx.x;
-  if (st < ntot) { fetch(st); put(); }
+  if (st < ntot) fetch(st);  // (in flight while the weights come in)
+  Frag<F32> w[KW];
+#pragma unroll
+  for (int k = 0; k < KW; ++k) {
+    const int ks = share * KW + k;
+    w[k] = ks < KALL ? frag_read<F32>(static_cast<const char*>(p.wt), ct * KALL + ks, lane) : frag_zero<F32>();
+  }
+  if (st < ntot) put();
   __syncthreads();
   for (; st < ntot; st += (int)gridDim.x) {
     const int next = st + (int)gridDim.x;
@@ -635,7 +752,7 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
 #pragma unroll
     for (int k = 0; k < KW; ++k) {
       const int ks = SPLIT == 1 ? k : min(share * KW + k, KALL - 1);  // (a share's steps beyond the end: the last one again, with zero weights)
-      acc = mma<A>(w[k], piece_frag<F32>(smem + rs * SUB, ks, l32, hh), acc);
+      acc = mma<A>(to_op<true>(w[k]), piece_frag<F32>(smem + rs * SUB, ks, l32, hh), acc);
     }
     float* plane = dxs + ((size_t)share * TR + rs * 32 + l32) * XROW + ct * 32 + 4 * hh;
 #pragma unroll
@@ -688,38 +805,30 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
 //
 // Bound by memory latency and the vector ALU rather than bandwidth: a stage has 8 MFMAs per wave.  So all
 // addresses are a base plus the row, the next stage's loads are in flight during a stage, and two workgroups
-// share a CU.  Sections in separate workgroups keep a partial sum at 64 KB (one workgroup for all six: 264 KB, 67 MB to
+// share a CU.  fp32: the three planes of a stage take the LDS of two, so a stage is read, then replaced between two
+// barriers (82 -> 55 us at 192 x 192 pairs; taken apart at every use instead, by up to four waves each, 69).  Sections in separate workgroups keep a partial sum at 64 KB (one workgroup for all six: 264 KB, 67 MB to
 // write and read back over the chip, as much as the inputs at 384 x 384 pairs).
 //
 // One chunk's partial: the result tiles row-major [a][b], then (at C * HD) the row sums.
 __host__ __device__ inline size_t wgrad_part_floats(int C, int HD) { return (size_t)C * HD + (C > HD ? C : HD); }
 constexpr int kWgradSections = 6;
 
-// Sub-tile of 32 columns in LDS: 16-bit rows of 64 bytes, swizzled as the attention's staged tiles; fp32 rows
-// of 128 bytes as they are.
-template <bool F32> constexpr int kSubRow = F32 ? 128 : 64;
-template <bool F32>
-__device__ __forceinline__ void sub_write(char* tile, int row, int chunk, const Frag<F32>& f) {
-  if constexpr (F32) {
-    float4* d = reinterpret_cast<float4*>(tile + row * 128 + chunk * 32);
-    d[0] = make_float4(f.v[0], f.v[1], f.v[2], f.v[3]);
-    d[1] = make_float4(f.v[4], f.v[5], f.v[6], f.v[7]);
-  } else {
-    *reinterpret_cast<u32x4*>(tile + 2 * swz_off<32>(row, chunk)) = f.w;
-  }
+// Sub-tile of 32 columns in LDS: 16-bit rows of 64 bytes, swizzled as the attention's staged tiles; fp32: a plane of such
+// rows after the other (PL of the three).
+template <bool F32, int TR, int PL>
+__device__ __forceinline__ void sub_write(char* tile, int row, int chunk, const Op<F32>& o) {
+#pragma unroll
+  for (int n = 0; n < (F32 ? PL : 1); ++n) *reinterpret_cast<u32x4*>(tile + n * (TR * 64) + 2 * swz_off<32>(row, chunk)) = o.p[n];
 }
 // Column l % 32 of the sub-tile, contraction rows rowbase + 8*(e/4) + 4*hh + e%4.
-template <bool F32>
-__device__ __forceinline__ Frag<F32> sub_frag_t(const char* tile, int rowbase, const FragOffsets<32>& fo, int l32, int hh) {
-  Frag<F32> f;
-  if constexpr (F32) {
-    const float* s = reinterpret_cast<const float*>(tile) + (rowbase + 4 * hh) * 32 + l32;
+template <bool F32, int TR, int PL>
+__device__ __forceinline__ Op<F32> sub_frag_t(const char* tile, int rowbase, const FragOffsets<32>& fo) {
+  Op<F32> o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f.v[e] = s[(8 * (e / 4) + e % 4) * 32];
-  } else {
-    f.w = __builtin_bit_cast(u32x4, lds_frag_t<32>(reinterpret_cast<const half_t*>(tile), rowbase, fo, 0));
-  }
-  return f;
+  for (int n = 0; n < (F32 ? PL : 1); ++n)
+    o.p[n] = __builtin_bit_cast(u32x4, lds_frag_t<32>(reinterpret_cast<const half_t*>(tile + n * (TR * 64)), rowbase, fo, 0));
+  if constexpr (F32 && PL < 3) o.p[2] = u32x4{0, 0, 0, 0};
+  return o;
 }
 
 enum WgradKind { kWgradQkv, kWgradGate, kWgradOut, kWgradBias };
@@ -733,7 +842,9 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
   constexpr int PA = KIND == kWgradBias ? 0 : (TR * NA * 4 + 511) / 512;   // 8-element pieces per thread
   constexpr int PB = (TR * NB * 4 + 511) / 512;
   constexpr int PD = KIND == kWgradBias ? 4 : 0;        // dbias entries per thread (H <= 32)
-  constexpr int SUB = TR * kSubRow<F32>;                // bytes of a sub-tile
+  constexpr int PLA = KIND == kWgradQkv || KIND == kWgradBias ? 2 : 3;  // (fp32) planes of operand A: q, k, v's gradients are fp16
+  constexpr int SUB = (F32 ? 3 : 1) * TR * 64;          // bytes of a sub-tile
+  constexpr int BUFS = F32 ? 1 : 2;                     // stage buffers: two workgroups share a CU's LDS
   constexpr int DROW = TR + 8;                          // dbias: one row of TR entries per head
   constexpr int ABYTES = KIND == kWgradBias ? 32 * DROW * 2 : NA * SUB;
   constexpr int BUF = ABYTES + NB * SUB;
@@ -802,7 +913,7 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
     for (int n = 0; n < PA; ++n) {
       const int pc = tid + 512 * n, row = pc / (NA * 4), c = pc % (NA * 4);
       if (TR * NA * 4 >= 512 || row < TR) {
-        sub_write<F32>(buf + (c / 4) * SUB, row, c % 4, ra[n]);
+        sub_write<F32, TR, PLA>(buf + (c / 4) * SUB, row, c % 4, to_op(ra[n]));
         float v[8];
         unpack<A>(ra[n], v);
         const float one = row < left ? 1.0f : 0.0f;
@@ -835,7 +946,7 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
       Frag<F32> f;
       pack<A>(v, f);
       if (row >= left) f = frag_zero<F32>();
-      if (TR * NB * 4 >= 512 || row < TR) sub_write<F32>(buf + ABYTES + (c / 4) * SUB, row, c % 4, f);
+      if (TR * NB * 4 >= 512 || row < TR) sub_write<F32, TR, 3>(buf + ABYTES + (c / 4) * SUB, row, c % 4, to_op(f));
     }
   };
   auto frag_a = [&](const char* buf, int at, int k) {
@@ -848,12 +959,12 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
       if constexpr (F32) {
         Frag<true> f;
         unpack<A>(d, f.v);
-        return f;
+        return to_op(f);
       } else {
-        return d;
+        return to_op(d);
       }
     } else {
-      return sub_frag_t<F32>(buf + at * SUB, k * 16, fo, l32, hh);
+      return sub_frag_t<F32, TR, PLA>(buf + at * SUB, k * 16, fo);
     }
   };
 
@@ -868,18 +979,19 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
     if (first + 1 < last) fetch(first + 1);
     __syncthreads();
     for (int st = first; st < last; ++st) {
-      const char* buf = smem + ((st - first) & 1) * BUF;
+      const char* buf = smem + (BUFS == 2 ? (st - first) & 1 : 0) * BUF;
       if (own) {
 #pragma unroll
         for (int k = 0; k < TR / 16; ++k) {
-          const Frag<F32> fa = frag_a(buf, at, k);
+          const Op<F32> fa = frag_a(buf, at, k);
 #pragma unroll
           for (int n = 0; n < NT; ++n)
-            acc[n] = mma<A>(fa, sub_frag_t<F32>(buf + ABYTES + (wave / NA + n * (8 / NA)) * SUB, k * 16, fo, l32, hh), acc[n]);
+            acc[n] = mma<A, PLA, PLA == 3>(fa, sub_frag_t<F32, TR, 3>(buf + ABYTES + (wave / NA + n * (8 / NA)) * SUB, k * 16, fo), acc[n]);
         }
       }
+      if constexpr (BUFS == 1) __syncthreads();
       if (st + 1 < last) {
-        put(smem + ((st + 1 - first) & 1) * BUF, st + 1);
+        put(smem + (BUFS == 2 ? (st + 1 - first) & 1 : 0) * BUF, st + 1);
         if (st + 2 < last) fetch(st + 2);
       }
       __syncthreads();
@@ -1024,6 +1136,7 @@ constexpr int kCus = 256;
   else if (p.HD == 64) { FTA_BLOCK_TYPES(X, 128, 64) } else { FTA_BLOCK_TYPES(X, 128, 128) }
 
 inline size_t frag_bytes(int dtype) { return dtype == 2 ? kFragBytes<true> : kFragBytes<false>; }
+inline size_t op_bytes(int dtype) { return dtype == 2 ? kOpBytes<true> : kOpBytes<false>; }
 
 // Column groups: a wave works off a row block's output tiles alone where there are enough row blocks for the
 // eight waves of every CU, else neighbouring waves share them.
@@ -1042,28 +1155,29 @@ int workgroups(long items, int waves, int most) {
 hipError_t launch_block_proj(BlockParams p, int C, int dtype, hipStream_t st) {
   // two stage buffers of 64 rows (fp32: 32) and the bias projection's weights
   const int rows = dtype == 2 ? 32 : 64;
-  const size_t smem = (size_t)(2 * rows / 32 + 1) * (C / 16) * frag_bytes(dtype) + (p.HD + 2 * rows) * sizeof(float);
-  const dim3 grid((unsigned)workgroups((long)p.B * ((p.LL + rows - 1) / rows), 1, kCus)), block(512);
+  const size_t smem = (size_t)(2 * rows / 32 + 1) * (C / 16) * op_bytes(dtype) + (p.HD + 2 * rows) * sizeof(float);
+  const int parts = dtype == 2 ? p.HD / 64 : 1;
+  const dim3 grid((unsigned)(parts * workgroups((long)p.B * ((p.LL + rows - 1) / rows), 1, kCus / parts))), block(512);
 #define FTA_BLOCK_CASE(AA, FF, CC, HH) return launch_kernel(blk_proj_kernel<AA, FF, CC, HH>, p, grid, block, smem, st);
   FTA_BLOCK_C_HD(FTA_BLOCK_CASE)
 #undef FTA_BLOCK_CASE
 }
 
 hipError_t launch_block_out(BlockParams p, int C, int dtype, hipStream_t st) {
-  const size_t smem = (size_t)(C / 32) * (p.HD / 16) * frag_bytes(dtype) + C * sizeof(float);
+  const size_t smem = (size_t)(C / 32) * (p.HD / 16) * op_bytes(dtype) + C * sizeof(float);
   const long blocks = (long)p.B * p.nper;
   p.cg = column_groups(blocks, C / 32);
-  const dim3 grid((unsigned)workgroups(blocks * p.cg, 8, 2 * kCus)), block(512);
+  const dim3 grid((unsigned)workgroups(blocks * p.cg, 8, dtype == 2 ? kCus : 2 * kCus)), block(512);
 #define FTA_BLOCK_CASE(AA, FF, CC, HH) return launch_kernel(blk_out_kernel<AA, FF, CC, HH>, p, grid, block, smem, st);
   FTA_BLOCK_C_HD(FTA_BLOCK_CASE)
 #undef FTA_BLOCK_CASE
 }
 
 hipError_t launch_block_dout(BlockParams p, int C, int dtype, hipStream_t st) {
-  const size_t smem = (size_t)(p.HD / 32) * (C / 16) * frag_bytes(dtype);
+  const size_t smem = (size_t)(p.HD / 32) * (C / 16) * op_bytes(dtype);
   const long blocks = (long)p.B * p.nper;
   p.cg = column_groups(blocks, p.HD / 32);
-  p.nwg = workgroups(blocks * p.cg, 8, 2 * kCus);
+  p.nwg = workgroups(blocks * p.cg, 8, dtype == 2 ? kCus : 2 * kCus);
   const dim3 grid((unsigned)(p.nwg + 17)), block(512);  // (17: one fragment of the packed weights per wave at 4 x 33)
 #define FTA_BLOCK_CASE(AA, FF, CC, HH) return launch_kernel(blk_dout_kernel<AA, FF, CC, HH>, p, grid, block, smem, st);
   FTA_BLOCK_C_HD(FTA_BLOCK_CASE)
@@ -1072,7 +1186,7 @@ hipError_t launch_block_dout(BlockParams p, int C, int dtype, hipStream_t st) {
 
 hipError_t launch_block_dx(BlockParams p, int C, int dtype, hipStream_t st) {
   const int rows = dtype == 2 ? 32 : 64, split = 8 / (rows / 32 * (C / 32));
-  const size_t smem = (size_t)(rows / 32) * (4 * p.HD / 16 + 1) * frag_bytes(dtype) + (size_t)split * rows * (C + 4) * sizeof(float);
+  const size_t smem = (size_t)(rows / 32) * (4 * p.HD / 16 + 1) * op_bytes(dtype) + (size_t)split * rows * (C + 4) * sizeof(float);
   const dim3 grid((unsigned)workgroups((long)p.B * ((p.LL + rows - 1) / rows), 1, kCus)), block(512);
 #define FTA_BLOCK_CASE(AA, FF, CC, HH) return launch_kernel(blk_dx_kernel<AA, FF, CC, HH>, p, grid, block, smem, st);
   FTA_BLOCK_C_HD(FTA_BLOCK_CASE)
@@ -1081,8 +1195,8 @@ hipError_t launch_block_dx(BlockParams p, int C, int dtype, hipStream_t st) {
 
 hipError_t launch_block_wgrad(BlockParams p, int C, int dtype, hipStream_t st) {
   // (the largest section: both operands C or HD columns wide; the bias section has one row per head)
-  const int sub = dtype == 2 ? 32 * 128 : 64 * 64, n = (p.HD + C) / 32;
-  const size_t smem = (size_t)2 * n * sub;
+  const int n = (p.HD + C) / 32;
+  const size_t smem = dtype == 2 ? (size_t)n * 3 * 32 * 64 : (size_t)2 * n * 64 * 64;  // (fp32: one stage of three planes)
   const dim3 grid((unsigned)(kWgradSections * p.nchunks)), block(512);
   const dim3 rgrid((unsigned)(reduce_proj_groups(p.HD, p.H) + C / 4));
 #define FTA_BLOCK_CASE(AA, FF, CC, HH)                                                                       \

@@ -201,3 +201,69 @@ def test_block_imports_after_the_repo_root_alias_module():
             % (root, os.path.join(root, "flash_tt_attn.py"), os.path.join(root, "flash-triangle-attention_amd")))
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd="/")
     assert r.returncode == 0 and "TriangleAttention" in r.stdout, r.stderr
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L,C,H,D", [
+    (1, 1, 128, 4, 32),    # one row of a 32-row stage
+    (1, 33, 128, 4, 32),   # 1089 rows: a last stage of one row
+    (2, 40, 64, 2, 32), (1, 23, 64, 4, 32), (1, 41, 128, 1, 64), (1, 96, 128, 2, 64),
+    (1, 160, 128, 4, 32)])  # several stages per workgroup, both workgroups of a row
+def test_fp32_block_products_hold_fp32_precision(B, L, C, H, D):
+    """Every product of an fp32 block, formed again in float64 from the operands that the kernels left in the forward
+    state and the backward workspace.  Bound: an operand short of its third bf16 part is off by up to 2^-17 (typically
+    3e-6 of the result), sums of up to 25600 rows in fp32 by chunks stay below 6e-7: 1e-6."""
+    import ctypes
+
+    import fta_lib
+    lib = fta_lib.load()
+    torch.manual_seed(5)
+    HD, n, m = H * D, B * L * L * H * D, B * L * L * H
+    rn = lambda *s: torch.randn(*s, device="cuda:0")
+    z, dout = rn(B, L, L, C), rn(B, L, L, C)
+    w = {"norm_weight": 1 + 0.1 * rn(C), "norm_bias": 0.1 * rn(C), "bg": 0.1 * rn(HD), "bo": 0.1 * rn(C), "wb": rn(H, C) / C ** 0.5,
+         "wo": rn(C, HD) / HD ** 0.5, **{k: rn(HD, C) / C ** 0.5 for k in ("wq", "wk", "wv", "wg")}}
+    st = (ctypes.c_int64 * 3)(L * L * C, L * C, C)
+    blk = fta_lib.Block(B=B, L=L, C=C, H=H, D=D, dtype=fta_lib.DTYPE_F32, eps=1e-5, sm_scale=D ** -0.5, z=z.data_ptr(), z_stride=st)
+    state = torch.empty(lib.fta_block_state_bytes(ctypes.byref(blk)), dtype=torch.uint8, device="cuda:0")
+    ws = torch.empty(lib.fta_block_bwd_workspace_bytes(ctypes.byref(blk)), dtype=torch.uint8, device="cuda:0")
+    out, dz, g = torch.empty_like(z), torch.empty_like(z), {k: torch.empty_like(t) for k, t in w.items()}
+    grads = fta_lib.BlockGrads(z=dz.data_ptr(), z_stride=st)
+    for k in w:
+        setattr(blk, k, w[k].data_ptr())
+        setattr(grads, k, g[k].data_ptr())
+    fta_lib.check(lib.fta_block_fwd(ctypes.byref(blk), out.data_ptr(), st, state.data_ptr(), 0))
+    fta_lib.check(lib.fta_block_bwd(ctypes.byref(blk), state.data_ptr(), dout.data_ptr(), st, ctypes.byref(grads), ws.data_ptr(), ws.numel(), 0))
+    torch.cuda.synchronize()
+
+    def parts(buf, sizes):  # regions at multiples of 256 bytes
+        at, r = 0, []
+        for by in sizes:
+            r.append(buf[at:at + by])
+            at += (by + 255) // 256 * 256
+        return r
+    rows = lambda t, dt, d: t.view(dt).view(B, H, L, L, d).permute(0, 2, 3, 1, 4).reshape(-1, H * d).double()
+    q, k, v, o, bias, gate, _ = parts(state, [2 * n] * 4 + [2 * m, 4 * n, 4 * m])
+    _, dgp, dq, dk, dv, db = parts(ws, [2 * n, 4 * n, 2 * n, 2 * n, 2 * n, 2 * m])
+    o, gate, dgp = rows(o, torch.float16, D), rows(gate, torch.float32, D), rows(dgp, torch.float32, D)
+    dq, dk, dv, db = (rows(t, torch.float16, d) for t, d in ((dq, D), (dk, D), (dv, D), (db, 1)))
+    w = {k: t.double() for k, t in w.items()}
+    z, dout, dz, out = (t.reshape(-1, C).double() for t in (z, dout, dz, out))
+    mean, rstd = z.mean(-1, keepdim=True), (z.var(-1, unbiased=False, keepdim=True) + 1e-5).rsqrt()
+    xh = (z - mean) * rstd
+    x = xh * w["norm_weight"] + w["norm_bias"]
+    dx = dq @ w["wq"] + dk @ w["wk"] + dv @ w["wv"] + dgp @ w["wg"] + db @ w["wb"]
+    dxh = dx * w["norm_weight"]
+    pairs = {"gate": (gate, torch.sigmoid(x @ w["wg"].T + w["bg"])), "out": (out, (gate * o) @ w["wo"].T + w["bo"]),
+             "d gate": (dgp, (dout @ w["wo"]) * o * gate * (1 - gate)),
+             "dz": (dz, rstd * (dxh - dxh.mean(-1, keepdim=True) - xh * (dxh * xh).mean(-1, keepdim=True))),
+             "wq": (g["wq"], dq.T @ x), "wk": (g["wk"], dk.T @ x), "wv": (g["wv"], dv.T @ x), "wg": (g["wg"], dgp.T @ x),
+             "wb": (g["wb"], db.T @ x), "wo": (g["wo"], dout.T @ (gate * o)), "bg": (g["bg"], dgp.sum(0)), "bo": (g["bo"], dout.sum(0)),
+             "norm_weight": (g["norm_weight"], (dx * xh).sum(0)), "norm_bias": (g["norm_bias"], dx.sum(0))}
+    for name, (a, b) in pairs.items():
+        # (one pair: the softmax over one key passes nothing on to q, k and the bias)
+        assert _rel_l2(a, b) <= 1e-6 or (L == 1 and name in ("wq", "wk", "wb") and (a.double() - b).abs().max() <= 1e-6), name
+    # what proj rounds to the attention's type: half a unit of fp16
+    for name, got in (("wq", q), ("wk", k), ("wv", v)):
+        assert _rel_l2(rows(got, torch.float16, D), x @ w[name].T) <= 2 ** -11, name
+    assert _rel_l2(rows(bias, torch.float16, 1), x @ w["wb"].T) <= 2 ** -11
