@@ -1,4 +1,4 @@
-// Backward: the launch plan and the dispatch of the stages.  Rows of up to 128 keys run the one-kernel form
+// Backward: the launch plan and the dispatch of the stages.  Rows of up to 128 keys (D = 32: 192, with dropout 256) run the one-kernel form
 // (fta_bwd_short.hip), longer ones the hand-scheduled kernels (fta_bwd_dq1.hip, fta_bwd_dkdv1.hip) or the general ones
 // (fta_bwd_kernels.h, instances in fta_bwd_feat.hip).
 #include <stdlib.h>
@@ -13,11 +13,11 @@ namespace fta {
 BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
   BwdPlan pl{};
   pl.feat = feat != 0;
-  pl.use_short = !forced_general() && plan_short(B, H, L1, row, D, pl.sh);
+  pl.use_short = !forced_general() && plan_short(B, H, L1, row, D, feat, pl.sh);
   // (the two go together: the pipelined dQ kernel makes delta itself and hands the row constants on to the dK/dV one in
   // the packed form that only that one reads)
   // Their tiles end at the next multiple of 64 keys: the work grows with the square of that length.  A training step at B1
-  // H4 D32 in fp16, tiles to the next multiple of 128 and key ranges of 512 + 256 -> this (us): L 129 to 192 85 -> 72, 257
+  // H4 D32 in fp16, tiles to the next multiple of 128 and key ranges of 512 + 256 -> this (us): L 257
   // 160 -> 143, 320 194 -> 169, 385 366 -> 328, 448 435 -> 395, 513 985 -> 886, 576 1114 -> 996, 704 1859 -> 1716, 1281
   // 11160 -> 10380.
   auto hand = [&](int lt) { pl.Lt = lt; return plan_dq1(B, H, L1, lt, D, pl.dq1) && plan_dkdv1(B, H, L1, lt, D, pl.dkdv1); };
@@ -148,7 +148,7 @@ hipError_t launch_bwd(BwdParams p, const BwdPlan& pl, int D, int dtype, hipStrea
   hipError_t e = hipSuccess;
   mark(0);
   if (pl.use_short) {
-    // rows of up to 128 keys, any options: one kernel
+    // short rows, any options: one kernel
     mark(1);
     e = launch_short(p, pl.sh, D, dtype, pl.feat, st);  // (fp16 without dropout is planned at that level in precise mode only)
     if (e != hipSuccess) return e;

@@ -5,7 +5,7 @@
 namespace fta {
 
 // Query ranges of one launch each (a wave's stationary bias^T tile and the stage size are compiled in), in units of 64
-// queries and as even as the row divides.  D = 32: four to eight units (three for a row of 192 queries); D = 64: four or
+// queries and as even as the row divides.  D = 32: four to eight units; D = 64: four or
 // five (bias^T, dK and dV share the accumulation registers with the operands), or one range of six, which takes the last
 // register, for a row of 384 queries.
 static int dkdv1_ranges(int L2, int D, int* out) {
@@ -19,7 +19,7 @@ static int dkdv1_stage(int range, int D) {
 
 bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl) {
   if (D != 32 && D != 64) return false;
-  if (L2 % 64 != 0 || L2 < (D == 64 ? 256 : 192) || L2 > (D == 64 ? 256 : 512) * kMaxRanges) return false;
+  if (L2 % 64 != 0 || L2 < 256 || L2 > (D == 64 ? 256 : 512) * kMaxRanges) return false;
   if (D == 64 && (L2 == 448 || L2 == 704)) return false;  // (no cut into these ranges: tiled as 512 and 768)
   pl.nlaunch = dkdv1_ranges(L2, D, pl.range);
   pl.JR = pl.range[0];

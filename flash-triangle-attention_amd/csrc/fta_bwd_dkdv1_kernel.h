@@ -17,8 +17,8 @@
 //     dO^T), the MFMAs that consume P and dS of tile j-1 (dV^T += dO^T P, dK^T += Q^T dS), the MFMAs
 //     that produce S and dP of tile j+1, and between them the vector-ALU work of tile j
 //     (exp2, dS = P * dP, two fp16 packings).  The pipeline runs across stage and row boundaries.
-// Used for tiled lengths that are a multiple of 64 from 192 on (D = 64: from 256 on, without 448): a launch takes a
-// query range of 192 to 512 (NJT = 6 to 16; D = 64: 256 to 384) in one to three stages of 128 to 256 queries; otherwise
+// Used for tiled lengths that are a multiple of 64 from 256 on (D = 64: without 448): a launch takes a
+// query range of 256 to 512 (NJT = 8 to 16; D = 64: 256 to 384) in one to three stages of 128 to 256 queries; otherwise
 // the two-waves-per-SIMD kernel runs.
 #pragma once
 #include "fta_kernels.h"
@@ -688,7 +688,7 @@ inline hipError_t launch_dkdv1_range(const BwdParams& p, int range, dim3 grid, s
     FTA_DKDV1_CASE(8, 4) FTA_DKDV1_CASE(10, 5) FTA_DKDV1_CASE(12, 4)
   } else {
     FTA_DKDV1_LATER(8, 8) FTA_DKDV1_LATER(10, 5) FTA_DKDV1_LATER(12, 6) FTA_DKDV1_LATER(14, 7) FTA_DKDV1_LATER(16, 8)
-    FTA_DKDV1_CASE(6, 6) FTA_DKDV1_CASE(8, 8) FTA_DKDV1_CASE(10, 5) FTA_DKDV1_CASE(12, 6) FTA_DKDV1_CASE(14, 7) FTA_DKDV1_CASE(16, 8)
+    FTA_DKDV1_CASE(8, 8) FTA_DKDV1_CASE(10, 5) FTA_DKDV1_CASE(12, 6) FTA_DKDV1_CASE(14, 7) FTA_DKDV1_CASE(16, 8)
   }
 #undef FTA_DKDV1_CASE
 #undef FTA_DKDV1_LATER

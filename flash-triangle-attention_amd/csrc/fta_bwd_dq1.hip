@@ -5,7 +5,7 @@
 namespace fta {
 
 // Key ranges of one launch each, as even as the row divides: later ones add into the dQ that the first stored.
-// D = 32: two slabs of four to eight tiles (256 to 512 keys); rows of 192 and 256 keys, which one slab covers, take that
+// D = 32: two slabs of four to eight tiles (256 to 512 keys); rows of 256 keys, which one slab covers, take that
 // (128 queries per workgroup instead of 64, and no exchange between slabs).  D = 64: one slab of five to eight tiles.
 static int dq1_ranges(int L2, int D, int* out) {
   return D == 64 ? even_ranges(L2 / 32, 8, 32, out) : even_ranges(L2 / 64, 8, 64, out);
@@ -14,7 +14,7 @@ static int dq1_slabs(int L2, int D) { return (D == 64 || L2 <= 256) ? 1 : 2; }
 
 bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl) {
   if (D != 32 && D != 64) return false;
-  if (L2 % 64 != 0 || L2 < 192 || L2 > (D == 64 ? 256 : 512) * kMaxRanges) return false;
+  if (L2 % 64 != 0 || L2 < 256 || L2 > (D == 64 ? 256 : 512) * kMaxRanges) return false;
   pl.nlaunch = dq1_ranges(L2, D, pl.range);
   pl.threads = 256;
   pl.ring = (D == 64) ? 3 : 4;  // as compiled into the kernel
@@ -25,7 +25,7 @@ bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl) {
   pl.nqg = (L2 + 32 * pl.QB - 1) / (32 * pl.QB);
   pl.KR = pl.range[0];
   for (int n = 0; n < pl.nlaunch; ++n) {
-    const int nkt = pl.range[n] / (32 * pl.SK), ts = (D == 32 && pl.SK == 1) ? 2 * ((nkt + 2) / 4) : (nkt + 1) / 2;  // tiles of a slab's first stage
+    const int nkt = pl.range[n] / (32 * pl.SK), ts = (nkt + 1) / 2;  // tiles of a slab's first stage
     const size_t slot = (size_t)2 * pl.SK * (ts * 32) * D * 2;
     const size_t qbuf = ((size_t)2 * pl.QB * 32 * D) * 2;
     const size_t xchg = (pl.SK == 2) ? (size_t)4 * (4 * (4 * (D / 32) / 2)) * 64 * 4 : 0;

@@ -19,8 +19,8 @@
 //   * -lse and -delta always enter through the extra MFMA contraction step (see aug_ones());
 //     this kernel computes delta = rowsum(O * dO) itself (no pre-pass runs in front of it) and
 //     writes the packed constants for the dK/dV kernel.
-// Used for tiled lengths that are a multiple of 64 from 192 on: a launch takes a key range of 256 to 512 keys in two wave
-// slabs (D = 32; rows of 192 and 256 keys in one), or of 160 to 256 in one (D = 64); any softmax scale, zero included
+// Used for tiled lengths that are a multiple of 64 from 256 on: a launch takes a key range of 256 to 512 keys in two wave
+// slabs (D = 32; rows of 256 keys in one), or of 160 to 256 in one (D = 64); any softmax scale, zero included
 // (nothing divides by it).  Otherwise the two-waves-per-SIMD kernel runs.
 //
 // Tiled lengths in steps of 64 instead of 128 (the tiles' work grows with the square of the tiled length), and ranges as
@@ -124,8 +124,8 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
   static_assert(!HL || D == 32, "the (hi, lo) split exists at D = 32");
   static_assert(!NAT || (HL && !T::is_bf16), "natural units come with the split, for fp16");
   static_assert(NKT >= 4 && NKT <= 8, "slabs of 128 to 256 keys");
-  // tiles of a slab's two stages (one slab at D = 32: even numbers, so that the copies split evenly over the waves)
-  constexpr int TS0 = (D == 32 && SK == 1) ? 2 * ((NKT + 2) / 4) : (NKT + 1) / 2, TS1 = NKT - TS0;
+  // tiles of a slab's two stages
+  constexpr int TS0 = (NKT + 1) / 2, TS1 = NKT - TS0;
   constexpr int KS = D / 16;
   constexpr int DT = D / 32;
   constexpr int QB = 4 / SK;                   // query blocks of 32 per workgroup
@@ -887,7 +887,7 @@ inline hipError_t launch_dq1_range(const BwdParams& p, int range, dim3 grid, siz
     FTA_DQ1_CASE(1, 5) FTA_DQ1_CASE(1, 6) FTA_DQ1_CASE(1, 7) FTA_DQ1_CASE(1, 8)
   } else {
     FTA_DQ1_LATER(4) FTA_DQ1_LATER(5) FTA_DQ1_LATER(6) FTA_DQ1_LATER(7) FTA_DQ1_LATER(8)
-    FTA_DQ1_CASE(1, 6) FTA_DQ1_CASE(1, 8)
+    FTA_DQ1_CASE(1, 8)
     FTA_DQ1_CASE(2, 4) FTA_DQ1_CASE(2, 5) FTA_DQ1_CASE(2, 6) FTA_DQ1_CASE(2, 7) FTA_DQ1_CASE(2, 8)
   }
 #undef FTA_DQ1_CASE

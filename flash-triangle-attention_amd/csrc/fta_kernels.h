@@ -74,7 +74,7 @@ inline int balanced_chunks(long base, int L1, long slots, int least = 8) {
 
 // The fewest rows of a chunk for rows of L2 keys: a workgroup's set-up loads one bias row per query, so that short rows
 // can be spread thinner over the chip than eight to a workgroup (B1 H4, us, eight -> this: forward at D = 64, L48 23.7 -> 9.5,
-// L192 48.1 -> 28.4; step with dropout at D = 32, L192 217 -> 138, L256 215 -> 170).
+// L192 48.1 -> 28.4).
 inline int least_rows(int L2) { return L2 >= 512 ? 8 : L2 <= 128 ? 2 : L2 / 64; }
 
 // ---- backward ---------------------------------------------------------------------------------
@@ -146,7 +146,7 @@ struct Dkdv1Plan {
   size_t smem;                    // the largest
 };
 
-// Geometry of the one-kernel backward for rows of up to 128 keys (a workgroup holds a whole row).
+// Geometry of the one-kernel backward for rows of up to 128 keys, at D = 32 192 (with dropout 256); a workgroup holds a whole row.
 struct ShortPlan {
   int NT, nchunks, rows_per_chunk, threads;
   size_t smem;
@@ -166,7 +166,7 @@ struct BwdPlan {
   Dkdv1Plan dkdv1;
   int nranges;         // dropout beyond 512 keys: ranges of their own geometry (see drop_range), else 0
   int range[kMaxRanges];
-  bool use_short;      // rows of up to 128 keys: all gradients in one kernel
+  bool use_short;      // short rows: all gradients in one kernel
   ShortPlan sh;
   int L2p;             // the length the workspace is laid out with and the general kernels' tiles cover (filled in by the C-ABI layer)
   int Lt;              // the length the hand-scheduled kernels' tiles cover: the next multiple of 64, not of 128, where they have the instances
@@ -187,7 +187,7 @@ inline bool bf16_scale_needs_split(float sm_scale) { return !(fabsf(sm_scale) * 
 bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl);
 hipError_t launch_dq1(BwdParams p, const Dq1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st);
 
-bool plan_short(int B, int H, int L1, int L2, int D, ShortPlan& pl);
+bool plan_short(int B, int H, int L1, int L2, int D, int feat, ShortPlan& pl);
 hipError_t launch_short(BwdParams p, const ShortPlan& pl, int D, int dtype, bool precise, hipStream_t st);
 
 bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl);

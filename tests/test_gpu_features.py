@@ -399,6 +399,29 @@ def test_one_kernel_backward_of_short_rows(L1, L2, p, D, dtype):
     _compare(_run(q, k, v, b, sm, do, *extra), _oracle(q, k, v, b, sm, do, **kw), dtype, f"short {L1}x{L2}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L1,L2,p", [(1, 129, 0.0), (2, 160, 0.0), (5, 161, 0.0), (40, 192, 0.0), (300, 137, 0.0), (3, 150, 0.25), (7, 192, 0.1),
+                                     (4, 193, 0.25), (33, 224, 0.1), (3, 225, 0.25), (70, 256, 0.1)])
+def test_one_kernel_backward_of_rows_that_fill_a_compute_unit(L1, L2, p, dtype):
+    """D = 32, 129 to 192 keys (with dropout 256): the one-kernel backward with five to eight waves, the bias packed in
+    memory and the next row's tiles loaded ahead; at the edges of its 32-key blocks, with one and with several rows per
+    workgroup, and with bias, q and dO as views of other strides.  Tolerances as for the shorter rows."""
+    import fta_lib
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, p, 1234)
+    assert fta_lib.describe_plan(1, 2, L1, L2, 32, 0.2, opt)["dq"]["kernel"] == f"fta_bwd_short_kernel<32,{(L2 + 31) // 32}>"
+    B, H, sm = 1, 2, 0.2
+    q, k, v, b, do = _inputs(B, H, L1, L2, 32, 31, dtype)
+    extra, kw = (), {}
+    if p:
+        keep, scale = dm.keep_mask(1234, p, B, H, L1, L2)
+        extra, kw = (p, 1234), dict(keep=torch.from_numpy(keep).to(DEV), keep_scale=scale)
+    ref = _oracle(q, k, v, b, sm, do, **kw)
+    _compare(_run(q, k, v, b, sm, do, *extra), ref, dtype, f"one kernel {L1}x{L2}")
+    rows = lambda t: t.permute(0, 2, 3, 1, 4).contiguous().permute(0, 3, 1, 2, 4)  # (B, L1, L2, H, D) in memory
+    wide = torch.zeros(B, H, L2, L2 + 3, device=DEV, dtype=dtype)[..., :L2].copy_(b)
+    _compare(_run(rows(q), k, rows(v), wide, sm, rows(do), *extra), ref, dtype, f"one kernel {L1}x{L2}, strided")
+
+
 def test_dropout_zero_is_the_plain_path_and_lse_ignores_the_mask():
     import fta_lib, flash_tt_attn as fta
     lib = fta_lib.load()
@@ -498,11 +521,11 @@ def test_forward_rows_of_an_odd_number_of_tiles(L1, L2, tiled, dtype):
 # ---- the hand-scheduled backward at tiled lengths in steps of 64 -------------------------------------------
 
 @pytest.mark.parametrize("mode", ["fp16", "bf16", "bf16 operand pair", "precise"])
-@pytest.mark.parametrize("D,L2", [(32, L) for L in (129, 192, 193, 257, 320, 385, 448, 449, 513, 640, 703, 1088)]
+@pytest.mark.parametrize("D,L2", [(32, L) for L in (193, 256, 257, 320, 385, 448, 449, 513, 640, 703, 1088)]
                          + [(64, L) for L in (129, 192, 257, 320, 400, 576, 640, 701, 832)])
 def test_backward_tiles_in_steps_of_64(D, L2, mode):
-    """Every number of tiles per wave (key ranges of 256 to 512 keys in two slabs, of 192 and 256 in one; D = 64: 160 to
-    256; query ranges of 192 to 512, at D = 64 256 to 384), odd numbers of them (stages of unequal length), groups of 128 queries or keys
+    """Every number of tiles per wave (key ranges of 256 to 512 keys in two slabs, of 256 in one; D = 64: 160 to
+    256; query ranges of 256 to 512, at D = 64 256 to 384), odd numbers of them (stages of unequal length), groups of 128 queries or keys
     that end beyond the tiled length, one to four ranges; rows that end inside a tile and whole ones."""
     import fta_lib
     import flash_tt_attn as fta
