@@ -114,7 +114,10 @@ using fta::half_t;
 // last one is kept per thread.
 struct PlanKey {
   int B, H, L1, L2, D, mask;
-  bool operator==(const PlanKey& o) const { return B == o.B && H == o.H && L1 == o.L1 && L2 == o.L2 && D == o.D && mask == o.mask; }
+  size_t limit = 0;
+  bool operator==(const PlanKey& o) const {
+    return B == o.B && H == o.H && L1 == o.L1 && L2 == o.L2 && D == o.D && mask == o.mask && limit == o.limit;
+  }
 };
 // The length the tiles of one direction cover for rows of L2 keys: the smallest multiple of 128 (forward: 32) that is at
 // least L2 and that the direction has a workgroup shape for (0 if there is none up to FTA_MAX_L2; the hand-scheduled
@@ -150,13 +153,13 @@ const fta::FwdPlan& cached_plan_fwd(int B, int H, int L1, int L2, int D, int fea
   }
   return plan;
 }
-const fta::BwdPlan& cached_plan_bwd(int B, int H, int L1, int L2, int D, int feat = 0) {
+const fta::BwdPlan& cached_plan_bwd(int B, int H, int L1, int L2, int D, int feat = 0, size_t limit = 0) {
   thread_local PlanKey key{-1, 0, 0, 0, 0, 0};
   thread_local fta::BwdPlan plan;
-  const PlanKey k{B, H, L1, L2, D, (fta::forced_general() ? 1 : 0) | (feat * 4)};
+  const PlanKey k{B, H, L1, L2, D, (fta::forced_general() ? 1 : 0) | (feat * 4), limit};
   if (!(key == k)) {
     const int lp = len_supported(L2, D, feat) ? padded_len_bwd(L2, D, feat) : 0;
-    plan = (lp != 0) ? fta::plan_bwd(B, H, L1, lp, D, L2, feat) : fta::BwdPlan{};
+    plan = (lp != 0) ? fta::plan_bwd(B, H, L1, lp, D, L2, feat, limit) : fta::BwdPlan{};
     plan.L2p = lp;
     key = k;
   }
@@ -474,7 +477,7 @@ static int check_bwd_impl(const fta_tensor5* q, const fta_tensor5* k, const fta_
                           const fta_tensor4* bias, const fta_tensor5* o, const float* lse,
                           const fta_tensor5* dout, const fta_tensor5* dq, const fta_tensor5* dk,
                           const fta_tensor5* dv, const fta_tensor4* dbias, const void* workspace,
-                          size_t workspace_bytes, int B, int H, int L1, int L2, int D, float sm_scale, int feat) {
+                          size_t workspace_bytes, int B, int H, int L1, int L2, int D, float sm_scale, int feat, size_t limit = 0) {
   int rc = check_dims(B, H, L1, L2, D, sm_scale);
   if (rc != FTA_OK) return rc;
   const fta_tensor5* ins[5] = {q, k, v, o, dout};
@@ -490,7 +493,7 @@ static int check_bwd_impl(const fta_tensor5* q, const fta_tensor5* k, const fta_
   if (lse == nullptr || workspace == nullptr) return FTA_ERR_NULL_POINTER;
   if (reinterpret_cast<uintptr_t>(lse) % 16 != 0 || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
     return FTA_ERR_MISALIGNED;
-  const fta::BwdPlan pl = cached_plan_bwd(B, H, L1, L2, D, feat);
+  const fta::BwdPlan pl = cached_plan_bwd(B, H, L1, L2, D, feat, limit);
   if (!pl.valid) return FTA_ERR_SEQ_LEN;
   if (workspace_bytes < pl.delta_bytes + pl.partial_bytes + pl.aux_bytes) return FTA_ERR_WORKSPACE;
   return FTA_OK;
@@ -509,16 +512,16 @@ static int bwd_impl(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor
                     const fta_tensor5* dout, const fta_tensor5* dq, const fta_tensor5* dk,
                     const fta_tensor5* dv, const fta_tensor4* dbias, void* workspace,
                     size_t workspace_bytes, int B, int H, int L1, int L2, int D, float sm_scale,
-                    void* stream, hipEvent_t* ev, const Opts& opt = Opts{}) {
+                    void* stream, hipEvent_t* ev, const Opts& opt = Opts{}, size_t limit = 0) {
   int rc = check_dims(B, H, L1, L2, D, sm_scale);
   if (rc != FTA_OK) return rc;
   const int level = bwd_level(opt, B, H, L1, L2, D, sm_scale);
   rc = check_bwd_impl(q, k, v, bias, o, lse, dout, dq, dk, dv, dbias, workspace, workspace_bytes,
-                      B, H, L1, L2, D, sm_scale, level);
+                      B, H, L1, L2, D, sm_scale, level, limit);
   if (rc != FTA_OK) return rc;
   if (opt.dbias_f32 && reinterpret_cast<uintptr_t>(dbias->ptr) % 4 != 0) return FTA_ERR_MISALIGNED;
   if ((rc = fta::check_device()) != FTA_OK) return rc;
-  const fta::BwdPlan pl = cached_plan_bwd(B, H, L1, L2, D, level);
+  const fta::BwdPlan pl = cached_plan_bwd(B, H, L1, L2, D, level, limit);
   fta::BwdParams p{};
   p.q = static_cast<const half_t*>(q->ptr);
   p.k = static_cast<const half_t*>(k->ptr);
@@ -590,22 +593,23 @@ int fta_bwd_noalloc(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor
                     const fta_tensor5* dout, const fta_tensor5* dq, const fta_tensor5* dk,
                     const fta_tensor5* dv, const fta_tensor4* dbias,
                     int B, int H, int L1, int L2, int D, float sm_scale, void* stream) {
-  // sizes first (host only): what fta_bwd would need as workspace must fit the built-in buffer
+  // sizes first (host only): the scratch must fit the built-in buffer, with fewer chunks than fta_bwd takes where it has to
   int rc = check_dims(B, H, L1, L2, D, sm_scale);
   if (rc != FTA_OK) return rc;
-  const fta::BwdPlan& pl = cached_plan_bwd(B, H, L1, L2, D);
+  constexpr size_t limit = FTA_STATIC_WORKSPACE_BYTES;
+  const fta::BwdPlan& pl = cached_plan_bwd(B, H, L1, L2, D, 0, limit);
   if (!pl.valid) return FTA_ERR_SEQ_LEN;
   const size_t need = pl.delta_bytes + pl.partial_bytes + pl.aux_bytes;
-  if (need > (size_t)FTA_STATIC_WORKSPACE_BYTES) return FTA_ERR_STATIC_WORKSPACE;
+  if (need > limit) return FTA_ERR_STATIC_WORKSPACE;
   // argument checks with a stand-in workspace address (never dereferenced), still before any GPU call
-  rc = fta_check_bwd(q, k, v, bias, o, lse, dout, dq, dk, dv, dbias, reinterpret_cast<const void*>(uintptr_t{256}), need,
-                     B, H, L1, L2, D, sm_scale);
+  rc = check_bwd_impl(q, k, v, bias, o, lse, dout, dq, dk, dv, dbias, reinterpret_cast<const void*>(uintptr_t{256}), need,
+                      B, H, L1, L2, D, sm_scale, 0, limit);
   if (rc != FTA_OK) return rc;
   void* ws = nullptr;
   if ((rc = static_scratch(&ws)) != FTA_OK) return rc;
   // Every kernel writes its part of the scratch before anything reads it (delta, the dBias partial
   // sums of each chunk, the packed row constants): nothing has to start at zero, so nothing is cleared.
-  return bwd_impl(q, k, v, bias, o, lse, dout, dq, dk, dv, dbias, ws, need, B, H, L1, L2, D, sm_scale, stream, nullptr);
+  return bwd_impl(q, k, v, bias, o, lse, dout, dq, dk, dv, dbias, ws, need, B, H, L1, L2, D, sm_scale, stream, nullptr, Opts{}, limit);
 }
 
 int fta_bwd_profile(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor5* v,

@@ -10,7 +10,7 @@ namespace fta {
 // ------------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------------
-BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
+static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int feat) {
   BwdPlan pl{};
   pl.feat = feat != 0;
   pl.use_short = !forced_general() && plan_short(B, H, L1, row, D, feat, pl.sh);
@@ -135,6 +135,21 @@ BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat) {
   pl.partial_bytes = (size_t)pl.nchunks * B * H * L2 * L2 * sizeof(float);
   pl.aux_bytes = (size_t)B * H * L1 * L2 * 2 * sizeof(uint32_t);
   pl.valid = ok2 && (pl.SK * pl.QB <= 8) && (pl.ring >= 3);
+  return pl;
+}
+
+BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat, size_t limit) {
+  BwdPlan pl = plan_any_size(B, H, L1, L2, D, row, feat);
+  if (!pl.valid || limit == 0 || pl.delta_bytes + pl.partial_bytes + pl.aux_bytes <= limit) return pl;
+  // The chunks are as many as make the launch shortest, and each has a partial dBias of its own: as many as fit instead.
+  int& nch = pl.use_short ? pl.sh.nchunks : pl.use_hand ? pl.dq1.nchunks : pl.nchunks;
+  int& rows = pl.use_short ? pl.sh.rows_per_chunk : pl.use_hand ? pl.dq1.rows_per_chunk : pl.rows_per_chunk;
+  const size_t one = pl.partial_bytes / nch, rest = pl.delta_bytes + pl.aux_bytes;
+  if (rest + one > limit) return pl;
+  const int most = (int)((limit - rest) / one);
+  rows = (L1 + most - 1) / most;
+  nch = (L1 + rows - 1) / rows;
+  pl.partial_bytes = nch * one;
   return pl;
 }
 

@@ -226,8 +226,9 @@ inline DropRange drop_range(int len) {
 
 // L2 is the length the tiles cover (a multiple of 128), `row` the true row length.
 // `feat`: 0 the fp16 kernels; 1 the plan is for bf16 inputs or the precise mode, 2 for dropout (general
-// kernels only, smaller instance sets).
-BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat);
+// kernels only, smaller instance sets).  `limit`: at most that many bytes of workspace (0: any number) if the partial dBias of
+// one chunk fits.
+BwdPlan plan_bwd(int B, int H, int L1, int L2, int D, int row, int feat, size_t limit = 0);
 hipError_t launch_bwd(BwdParams p, const BwdPlan& pl, int D, int dtype, hipStream_t st, hipEvent_t* ev = nullptr);
 hipError_t launch_dbias_reduce(const BwdParams& p, int dtype, hipStream_t st);
 hipError_t launch_bwd_feat(const BwdParams& p, const BwdPlan& pl, int D, int dtype, hipStream_t st, hipEvent_t* ev);

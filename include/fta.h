@@ -214,9 +214,11 @@ int fta_bwd_ex(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor5* v,
  * results as fta_bwd without the workspace: the scratch (delta, dBias partial sums, packed row
  * constants) lives in a buffer of FTA_STATIC_WORKSPACE_BYTES that is part of the library's device
  * image -- every GPU the library runs on holds its own copy until the process ends.  The call
- * allocates and frees nothing.  Sizes whose fta_bwd_workspace_bytes() exceeds the buffer are
- * refused with FTA_ERR_STATIC_WORKSPACE before any GPU work (the benchmark shape B4 H8 L512 D32
- * needs 101 MB and fits).  All calls on one GPU share that GPU's buffer: two calls that overlap in
+ * allocates and frees nothing.  Where fta_bwd_workspace_bytes() exceeds the buffer, the L1 rows are
+ * cut into fewer chunks, each with a partial dBias of its own (dBias is then summed in another order
+ * than fta_bwd's); sizes that do not fit in one chunk either are refused with
+ * FTA_ERR_STATIC_WORKSPACE before any GPU work (the benchmark shape B4 H8 L512 D32 needs 101 MB and
+ * fits as it is).  All calls on one GPU share that GPU's buffer: two calls that overlap in
  * time on one GPU (different streams or threads) race on it; calls on one stream are ordered and
  * safe.  The first call on a device looks the buffer's address up (hipGetSymbolAddress); make that
  * call outside any graph capture. */

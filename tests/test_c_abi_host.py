@@ -262,3 +262,18 @@ def test_chunk_counts_fill_the_last_round_of_workgroups():
     # never fewer than 8 rows per chunk, never more chunks than rows allow
     d = fta_lib.describe_plan(1, 1, 16, 512, 32)
     assert d["dq"]["grid"] <= 8 * 2 and d["fwd"]["grid"] <= 4 * 2
+
+
+@pytest.mark.parametrize("B,H,L,D", [(4, 8, 400, 32), (4, 8, 448, 32), (2, 8, 420, 32), (8, 8, 280, 32), (1, 2, 900, 32), (1, 2, 1088, 32)])
+def test_the_backward_without_a_workspace_takes_fewer_chunks_where_more_do_not_fit(B, H, L, D):
+    """One chunk's partial dBias and the row constants fit the built-in buffer: the sizes are not refused, however many
+    chunks the launch would take by itself.  (The call ends at an argument error behind the check of the sizes.)"""
+    lib = fta_lib.load()
+    assert lib.fta_bwd_workspace_bytes(B, H, L, L, D) > fta_lib.STATIC_WORKSPACE_BYTES
+    t, b = _t5(B, H, L, L, D), _t4(B, H, L)
+    odd_lse = FAKE + 4
+    assert lib.fta_bwd_noalloc(t, t, t, b, t, odd_lse, t, t, t, t, b, B, H, L, L, D, 0.5, 0) == -2
+    # (row constants alone beyond it)
+    B, H, L = 4, 8, 1024
+    t, b = _t5(B, H, L, L, D), _t4(B, H, L)
+    assert lib.fta_bwd_noalloc(t, t, t, b, t, odd_lse, t, t, t, t, b, B, H, L, L, D, 0.5, 0) == -10

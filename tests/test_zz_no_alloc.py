@@ -62,6 +62,41 @@ def test_noalloc_backward_matches_the_workspace_backward_twice_in_a_row():
     _both(lib, fta_lib, 1, 1, 5, 128, 64, 0.3, seed=32)                    # smaller, general kernels, delta pre-pass
 
 
+@pytest.mark.parametrize("B,H,L1,L2,D", [(4, 8, 385, 385, 32), (1, 2, 900, 900, 32)])
+def test_noalloc_backward_with_fewer_chunks_than_the_workspace_backward(B, H, L1, L2, D):
+    """dQ, dK and dV do not depend on the chunks; dBias is summed in another order (fp32 sums of at most L1 terms, rounded to
+    fp16: half a unit in the last place of the result each, and another one where the two sums fall on either side)."""
+    import fta_lib
+    lib = fta_lib.load()
+    print(f"case noalloc chunks B={B} H={H} L1={L1} L2={L2} D={D}", flush=True)
+    need = lib.fta_bwd_workspace_bytes(B, H, L1, L2, D)
+    assert need > fta_lib.STATIC_WORKSPACE_BYTES
+    q, k, v, b, do = orc.make_inputs(B, H, L1, L2, D, seed=33, device=DEV)
+    t5 = lambda t: fta_lib.t5(t.data_ptr(), t.stride())
+    t4 = lambda t: fta_lib.t4(t.data_ptr(), t.stride())
+    o = torch.empty_like(q)
+    lse = torch.empty(B, H, L1, L2, device=DEV, dtype=torch.float32)
+    sm = 1.0 / math.sqrt(D)
+    fta_lib.check(lib.fta_fwd(t5(q), t5(k), t5(v), t4(b), t5(o), lse.data_ptr(), B, H, L1, L2, D, sm, 0))
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    outs = []
+    for noalloc in (False, True):
+        g = [torch.full_like(t, float("nan")) for t in (q, k, v, b)]
+        args = (t5(q), t5(k), t5(v), t4(b), t5(o), lse.data_ptr(), t5(do), t5(g[0]), t5(g[1]), t5(g[2]), t4(g[3]))
+        if noalloc:
+            fta_lib.check(lib.fta_bwd_noalloc(*args, B, H, L1, L2, D, sm, 0))
+        else:
+            fta_lib.check(lib.fta_bwd(*args, ws.data_ptr(), need, B, H, L1, L2, D, sm, 0))
+        torch.cuda.synchronize()
+        outs.append(g)
+    for name, a, c in zip(("dq", "dk", "dv"), *outs):
+        assert bool(torch.isfinite(c).all()) and torch.equal(a, c), name
+    a, c = (g[3].double() for g in outs)
+    assert bool(torch.isfinite(c).all())
+    assert float(((a - c).abs() / (c.abs() + 1e-2)).max()) <= 2.0 ** -9
+    assert float((a - c).norm() / c.norm()) <= 2.0 ** -11
+
+
 def test_noalloc_backward_refuses_sizes_beyond_its_buffer():
     import fta_lib
     lib = fta_lib.load()
