@@ -30,19 +30,32 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   }
   // Dropout at D = 32 beyond 512 keys: key and query ranges of 256, 384 and 512, as even as the row divides, every one by
   // eight waves (four slabs of 64, 96 or 128 keys; two of 128, 192 or 256 queries).  Cut into the widest equal pieces that
-  // divide the row, 640 keys take five launches of 128 and 768 queries three slabs, six waves: steps at B1 H4 in bf16 of 576,
-  // 640, 768, 896 and 1024 keys that way and as below 2.97 / 1.77, 3.33 / 2.07, 4.35 / 3.38, 7.07 / 5.52, 9.12 / 8.97 ms.
+  // divide the row, 640 keys take five launches of 128: steps at B1 H4 in bf16 of 576, 640, 896 and 1280 keys that way and as
+  // below 3.09 / 1.85, 3.46 / 2.18, 7.54 / 5.65, 18.4 / 16.6 ms.
+  // dK and dV are held in the tensors' type from one query range to the next, a rounding at each.  So dK/dV takes rows that
+  // 768 or 1024 divides in launches of as many queries, four slabs of 192 or 256: of 768, 1024, 2048, 2304 and
+  // 3072 queries its relative error in bf16 is 2.37, 2.36, 2.64, 2.88 and 2.88e-3, in ranges of up to 512 2.65, 2.63, 3.11,
+  // 3.40 and 3.53e-3; the steps are 1 to 3 % longer (768 3.60 / 3.53 ms, 1024 9.46 / 9.38, 1536 29.6 / 28.9, 2048 85.4 / 83.9).
   if (feat == 2 && D == 32 && L2 > 512 && L2 % 128 == 0 && L2 <= 512 * kMaxRanges) {
-    pl.nranges = even_ranges(L2 / 128, 4, 128, pl.range);
-    const int nblk = (row + 31) / 32, sk = 4, qb = 2, sj = 2, kb = 4;
+    pl.nranges = pl.nranges2 = even_ranges(L2 / 128, 4, 128, pl.range);
+    const int nblk = (row + 31) / 32, sk = 4, qb = 2;
+    int sj = 2, kb = 4;
     pl.NKT = pl.range[0] / 128; pl.SK = sk; pl.QB = qb; pl.KR = pl.range[0]; pl.nlaunch = pl.nranges;
-    pl.NJT = pl.range[0] / 64; pl.JT = 64; pl.SJ = sj; pl.KB = kb; pl.JR = pl.range[0]; pl.nlaunch2 = pl.nranges;
-    pl.threads = pl.threads2 = 512;
+    pl.NJT = pl.range[0] / 64; pl.JT = 64; pl.JR = pl.range[0]; pl.nlaunch2 = pl.nranges;
     for (int n = 0; n < pl.nranges; ++n) {
       const DropRange r = drop_range(pl.range[n]);
       if (r.smem > pl.smem) pl.smem = r.smem;
       if (r.smem2 > pl.smem2) pl.smem2 = r.smem2;
     }
+    const int wide = L2 % 1024 == 0 ? 1024 : L2 % 768 == 0 ? 768 : 0;
+    if (wide != 0) {
+      const Ring r = dkdv_ring(32, wide / 128, 64, 4);
+      sj = 4; kb = 2;
+      pl.nranges2 = 0; pl.NJT = wide / 128; pl.JR = wide; pl.nlaunch2 = L2 / wide;
+      pl.ring2 = r.r; pl.nb2 = r.nb; pl.smem2 = dkdv_smem(32, pl.NJT, 64, 4);
+    }
+    pl.SJ = sj; pl.KB = kb;
+    pl.threads = pl.threads2 = 512;
     pl.nqg = (nblk + qb - 1) / qb;
     pl.nkg = (nblk + kb - 1) / kb;
     const int nch = balanced_chunks((long)B * H * pl.nqg, L1, 256), nch2 = balanced_chunks((long)B * H * pl.nkg, L1, 256);

@@ -70,9 +70,9 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
   mark(2);
   {  // 2. dK, dV
     dim3 grid((unsigned)(p.B * p.H * pl.nkg * pl.nchunks2)), block((unsigned)pl.threads2);
-    if (pl.nranges > 0) {
+    if (pl.nranges2 > 0) {
       if constexpr (DROP)
-        for (int n = 0, at = 0; n < pl.nranges; at += pl.range[n++]) {
+        for (int n = 0, at = 0; n < pl.nranges2; at += pl.range[n++]) {
           const DropRange r = drop_range(pl.range[n]);
           p.jr0 = at;
           e = pl.range[n] == 512   ? launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, 8, 64, 2>, p, grid, block, r.smem2, st)
@@ -82,18 +82,18 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
           if (e != hipSuccess) return e;
         }
     }
-    for (int n = 0; n < (pl.nranges > 0 ? 0 : pl.nlaunch2); ++n) {
+    for (int n = 0; n < (pl.nranges2 > 0 ? 0 : pl.nlaunch2); ++n) {
       p.jr0 = n * pl.JR;
       e = hipErrorInvalidConfiguration;
 #define FTA_DKDV_FEAT_CASE(DD, NN, JJ) \
   if (e == hipErrorInvalidConfiguration && D == DD && pl.NJT == NN && pl.JT == JJ) \
     e = launch_kernel(fta_bwd_dkdv_kernel<T, DROP, DD, NN, JJ>, p, grid, block, pl.smem2, st);
-      if constexpr (DROP) {  // fixed geometry: rows of 256, 384 and 512 queries
+      if constexpr (DROP) {  // fixed geometry: 256, 384, 512, 768 and 1024 queries to a launch
 #define FTA_DKDV_FIX_CASE(NN, SS)                                                                                        \
   if (D == 32 && pl.threads2 == 512 && pl.NJT == NN && pl.JT == 64 && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, 64, SS).r &&  \
       pl.nb2 == dkdv_ring(32, NN, 64, SS).nb)                                                                            \
     e = launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, NN, 64, SS>, p, grid, block, pl.smem2, st);
-        FTA_DKDV_FIX_CASE(6, 2) FTA_DKDV_FIX_CASE(8, 1) FTA_DKDV_FIX_CASE(8, 2)
+        FTA_DKDV_FIX_CASE(6, 2) FTA_DKDV_FIX_CASE(8, 1) FTA_DKDV_FIX_CASE(8, 2) FTA_DKDV_FIX_CASE(6, 4) FTA_DKDV_FIX_CASE(8, 4)
 #undef FTA_DKDV_FIX_CASE
       }
       if constexpr (!DROP) { FTA_DKDV_FEAT_CASE(32, 8, 64) }

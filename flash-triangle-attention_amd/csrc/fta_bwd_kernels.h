@@ -458,7 +458,8 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   const int KR2 = KB * 32;                   // key rows of the workgroup
   const int NB = FIX ? dkdv_ring(D, NJT, JT, SJC).nb : p.nb2;                      // row-operand buffers (rows whose K/V tiles are in flight)
   half_t* ktiles = smem + R * slot_halfs;    // [NB][K tile | V tile], KR2 x D each
-  half_t* scratch = ktiles + NB * 2 * KR2 * D;  // cross-slab dK/dV partials, kept in fp16 to fit in LDS
+  typedef typename std::conditional<dkdv_share_bytes(NJT, SJC) == 4, float, half_t>::type Share;
+  Share* scratch = reinterpret_cast<Share*>(ktiles + NB * 2 * KR2 * D);  // cross-slab dK/dV partials, in fp16 where they would not fit in LDS
   FragOffsets<D> fo;
   fo.init(lane);
 
@@ -772,19 +773,19 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
       // sum the query slabs of one key block through LDS (own region; the next row's stage
       // barriers separate these reads from the next row's writes)
       if (jslab != 0) {
-        half_t* mine = scratch + ((size_t)(kb * (SJ - 1) + jslab - 1) * 32 * DT) * 64 + lane;
+        Share* mine = scratch + ((size_t)(kb * (SJ - 1) + jslab - 1) * 32 * DT) * 64 + lane;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            mine[(dt * 32 + r) * 64] = (half_t)dk[dt][r];
-            mine[(dt * 32 + 16 + r) * 64] = (half_t)dv[dt][r];
+            mine[(dt * 32 + r) * 64] = (Share)dk[dt][r];
+            mine[(dt * 32 + 16 + r) * 64] = (Share)dv[dt][r];
           }
       }
       __syncthreads();
       if (jslab == 0) {
         for (int s2 = 1; s2 < SJ; ++s2) {
-          const half_t* o2 = scratch + ((size_t)(kb * (SJ - 1) + s2 - 1) * 32 * DT) * 64 + lane;
+          const Share* o2 = scratch + ((size_t)(kb * (SJ - 1) + s2 - 1) * 32 * DT) * 64 + lane;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -801,15 +802,33 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
       half_t* dkr = dkbase + (int64_t)(i0 + ir) * p.dks[2] + (int64_t)(k0 + l32) * p.dks[3] + 8 * hh;
       half_t* dvr = dvbase + (int64_t)(i0 + ir) * p.dvs[2] + (int64_t)(k0 + l32) * p.dvs[3] + 8 * hh;
       const bool kreal = (k0 + l32 <= last);
+      // Later query ranges add to what the earlier launches stored: ahead of the one rounding of both with four slabs of
+      // known geometry, else rounded and then added (before it, in 32 bits, D = 64 spills more: 1276 -> 1458 us a training step
+      // at B1 H8 L300 in bf16).
+      constexpr bool IN32 = (SJC == 4);
 #pragma unroll
       for (int y = 0; y < 2 * DT; ++y) {
         const floatx16& ak = dk[y / 2];
         const floatx16& av = dv[y / 2];
         const int r0 = (y % 2) * 8;
-        const uint32_t kx0 = T::pack(ak[r0] * scale, ak[r0 + 1] * scale), kx1 = T::pack(ak[r0 + 2] * scale, ak[r0 + 3] * scale);
-        const uint32_t ky0 = T::pack(ak[r0 + 4] * scale, ak[r0 + 5] * scale), ky1 = T::pack(ak[r0 + 6] * scale, ak[r0 + 7] * scale);
-        const uint32_t vx0 = T::pack(av[r0], av[r0 + 1]), vx1 = T::pack(av[r0 + 2], av[r0 + 3]);
-        const uint32_t vy0 = T::pack(av[r0 + 4], av[r0 + 5]), vy1 = T::pack(av[r0 + 6], av[r0 + 7]);
+        float fk[8], fv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { fk[e] = ak[r0 + e] * scale; fv[e] = av[r0 + e]; }
+        if (IN32 && p.jr0 != 0 && kreal) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {  // (before the exchange a lane holds d = 16 y + 8 u + 4 hh .. +3)
+            const u32x2 ok = *reinterpret_cast<const u32x2*>(dkr + 16 * y + 8 * u - 4 * hh), ov = *reinterpret_cast<const u32x2*>(dvr + 16 * y + 8 * u - 4 * hh);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              fk[4 * u + e] += (e & 1) ? T::hi(ok[e >> 1]) : T::lo(ok[e >> 1]);
+              fv[4 * u + e] += (e & 1) ? T::hi(ov[e >> 1]) : T::lo(ov[e >> 1]);
+            }
+          }
+        }
+        const uint32_t kx0 = T::pack(fk[0], fk[1]), kx1 = T::pack(fk[2], fk[3]);
+        const uint32_t ky0 = T::pack(fk[4], fk[5]), ky1 = T::pack(fk[6], fk[7]);
+        const uint32_t vx0 = T::pack(fv[0], fv[1]), vx1 = T::pack(fv[2], fv[3]);
+        const uint32_t vy0 = T::pack(fv[4], fv[5]), vy1 = T::pack(fv[6], fv[7]);
         auto k0s = __builtin_amdgcn_permlane32_swap(kx0, ky0, false, false);
         auto k1s = __builtin_amdgcn_permlane32_swap(kx1, ky1, false, false);
         auto v0s = __builtin_amdgcn_permlane32_swap(vx0, vy0, false, false);
@@ -819,7 +838,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
         if (kreal) {
           u32x4* pk = reinterpret_cast<u32x4*>(dkr + 16 * y);
           u32x4* pv = reinterpret_cast<u32x4*>(dvr + 16 * y);
-          if (p.jr0 != 0) {  // later query ranges add to what the earlier launches stored
+          if (!IN32 && p.jr0 != 0) {
             const u32x4 ok = *pk, ov = *pv;
 #pragma unroll
             for (int e = 0; e < 4; ++e) { wk[e] = T::add2(wk[e], ok[e]); wv[e] = T::add2(wv[e], ov[e]); }

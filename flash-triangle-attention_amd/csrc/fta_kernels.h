@@ -165,6 +165,7 @@ struct BwdPlan {
   Dq1Plan dq1;
   Dkdv1Plan dkdv1;
   int nranges;         // dropout beyond 512 keys: ranges of their own geometry (see drop_range), else 0
+  int nranges2;        // the same for dK/dV, 0 where it takes launches of JR queries
   int range[kMaxRanges];
   bool use_short;      // short rows: all gradients in one kernel
   ShortPlan sh;
@@ -207,8 +208,16 @@ constexpr Ring fit_ring(int steps, int slot, int row, int records) {
 constexpr Ring dq_ring(int D, int NKT, int G1, int SK) {
   return fit_ring(NKT / G1, 4 * SK * G1 * 32 * D, 4 * (8 / SK) * 32 * D, SK > 1 ? 8 * 16 * (D / 32) * 64 * (D == 32 ? 4 : 2) : 0);
 }
+// (the slabs' shares of dK and dV are exchanged in fp16, of four slabs of 192 queries in fp32, for which LDS has room)
+constexpr int dkdv_share_bytes(int NJT, int SJ) { return NJT == 6 && SJ == 4 ? 4 : 2; }
+constexpr int dkdv_shares(int D, int NJT, int SJ) { return (SJ - 1) * (8 / SJ) * 32 * (D / 32) * 64 * dkdv_share_bytes(NJT, SJ); }
 constexpr Ring dkdv_ring(int D, int NJT, int JT, int SJ) {
-  return fit_ring(NJT / (JT / 32), 4 * SJ * JT * D + 8 * SJ * JT, 4 * (8 / SJ) * 32 * D, (SJ - 1) * (8 / SJ) * 32 * (D / 32) * 64 * 2);
+  return fit_ring(NJT / (JT / 32), 4 * SJ * JT * D + 8 * SJ * JT, 4 * (8 / SJ) * 32 * D, dkdv_shares(D, NJT, SJ));
+}
+
+constexpr size_t dkdv_smem(int D, int NJT, int JT, int SJ) {
+  const Ring r = dkdv_ring(D, NJT, JT, SJ);
+  return (size_t)r.r * (4 * SJ * JT * D + 8 * SJ * JT) + (size_t)r.nb * (4 * (8 / SJ) * 32 * D) + dkdv_shares(D, NJT, SJ);
 }
 
 // One key range and one query range of the backward with dropout beyond 512 keys (D = 32): stage and row-operand
@@ -220,7 +229,7 @@ inline DropRange drop_range(int len) {
   r.dq = dq_ring(32, nkt, g1, 4);
   r.dkdv = dkdv_ring(32, njt, 64, 2);
   r.smem = (size_t)r.dq.r * (4 * 4 * g1 * 32 * 32) + (size_t)r.dq.nb * (4 * 2 * 32 * 32) + 8 * 16 * 64 * 4;
-  r.smem2 = (size_t)r.dkdv.r * (4 * 2 * 64 * 32 + 8 * 2 * 64) + (size_t)r.dkdv.nb * (4 * 4 * 32 * 32) + 4 * 32 * 64 * 2;
+  r.smem2 = dkdv_smem(32, njt, 64, 2);
   return r;
 }
 

@@ -277,3 +277,17 @@ def test_the_backward_without_a_workspace_takes_fewer_chunks_where_more_do_not_f
     B, H, L = 4, 8, 1024
     t, b = _t5(B, H, L, L, D), _t4(B, H, L)
     assert lib.fta_bwd_noalloc(t, t, t, b, t, odd_lse, t, t, t, t, b, B, H, L, L, D, 0.5, 0) == -10
+
+
+def test_dropout_backward_cuts_no_row_into_more_query_ranges_than_it_has_to():
+    """D = 32: dK and dV are held in 16 bits between the launches over query ranges.  A launch covers 256, 384 or 512 queries,
+    or 768 or 1024 of rows that those divide."""
+    wide = {768: 1, 1024: 1, 1536: 2, 2048: 2, 2304: 3, 3072: 3, 3840: 5, 4096: 4}
+    for dtype in (fta_lib.DTYPE_F16, fta_lib.DTYPE_BF16):
+        opt = fta_lib.Options(dtype, 0, 0.25, 7, 0)
+        for tiled in range(640, 4097, 128):
+            for L2 in (tiled - 127, tiled - 64, tiled):
+                d = fta_lib.describe_plan(1, 4, L2, L2, 32, 0.17, opt)
+                assert d["dkdv"]["launches"] == wide.get(tiled, -(-tiled // 512)), (L2, d["dkdv"])
+                assert d["dq"]["launches"] == -(-tiled // 512), (L2, d["dq"])
+                assert 0 < d["dkdv"]["lds"] <= 160 * 1024

@@ -366,15 +366,17 @@ def test_dropout_at_the_tiled_lengths_of_head_dim_32(L1, L2, p, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("L1,L2,launches", [(5, 513, 2), (4, 640, 2), (9, 768, 2), (3, 801, 2), (4, 1024, 2), (3, 1100, 3)])
-def test_dropout_beyond_512_keys_in_ranges_of_their_own(L1, L2, launches, dtype):
-    """Key and query ranges of 256, 384 and 512 in one row, each by eight waves, summed over their launches; rows that end
-    inside a range's last blocks."""
+@pytest.mark.parametrize("L1,L2,launches,launches2", [(5, 513, 2, 2), (4, 640, 2, 2), (9, 768, 2, 1), (3, 801, 2, 2), (4, 1024, 2, 1), (3, 1100, 3, 3),
+                                                      (3, 2011, 4, 2)])
+def test_dropout_beyond_512_keys_in_ranges_of_their_own(L1, L2, launches, launches2, dtype):
+    """Key and query ranges of 256, 384 and 512 in one row, each by eight waves, summed over their launches, or 768 and 1024
+    queries to a launch where those are fewer; rows that end inside a range's last blocks."""
     import fta_lib
     B, H, p, sm = 1, 2, 0.2, 1.0 / math.sqrt(32)
     opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, p, 77, 0)
     plan = fta_lib.describe_plan(B, H, L1, L2, 32, sm, opt)
-    assert plan["dq"]["launches"] == plan["dkdv"]["launches"] == launches and plan["dq"]["block"] == plan["dkdv"]["block"] == 512
+    assert plan["dq"]["launches"] == launches and plan["dkdv"]["launches"] == launches2
+    assert plan["dq"]["block"] == plan["dkdv"]["block"] == 512
     print(f"case dropout ranges {L1}x{L2} {dtype}", flush=True)
     q, k, v, b, do = _inputs(B, H, L1, L2, 32, 47, dtype)
     keep, scale = dm.keep_mask(77, p, B, H, L1, L2)
