@@ -26,8 +26,9 @@
 // left out is below 2^-24 of the product).  Activations are taken apart where they enter LDS, weights on their way into
 // registers or LDS.  Against 64 bits (relative L2, 192 x 192 pairs, fp32 instructions / three parts): gate 8.0e-8 / 7.1e-8, out
 // 1.6e-7 / 1.3e-7, dz 2.9e-7 / 2.3e-7, weight gradients 4.0e-7 / 1.8e-7 (wo) to 3.6e-7 (wb): the matrix core sums 16 products
-// at once, the fp32 instruction two.  Infinity and values beyond the largest bf16 (3.39e38) have no three parts: what they
-// enter comes out as NaN.  Nothing is rounded to 16 bits in memory that was not before (q, k, v, bias, o and their gradients).
+// at once, the fp32 instruction two.  Infinity, and values that round to it in
+// bf16 (beyond 3.39e38), have no three parts: a tile whose sums are not all finite is formed again by the fp32 instruction,
+// so that infinities come out as they went in.  Nothing is rounded to 16 bits in memory that was not before (q, k, v, bias, o and their gradients).
 // us per kernel at 192 x 192 pairs, before and after: proj 69 / 47, out 32 / 26, dout 29 / 28, dx 57 / 48, wgrad 82 / 55; a
 // training pass 352 / 265 (256 x 256: 498 / 394, 321 x 321: 838 / 670), inference 112 / 82 (457 x 457: 505 / 387).
 //
@@ -104,6 +105,22 @@ __device__ __forceinline__ floatx16 mma(const Op<true>& a, const Op<true>& b, fl
     for (int r = 0; r < 16; ++r) t[r] += c[r];
   }
   return t;
+}
+
+// A tile of sums that are not all finite (for the whole wave): three parts of an infinite operand, or of a finite one that
+// rounds to infinity in bf16, sum to NaN whatever the product is.  The waves keep a flag, and one that has seen such a tile
+// forms all of its tiles again behind its loop, from the operands in memory, where the registers of the loop are free.
+__device__ __forceinline__ bool not_finite(const floatx16& c) {
+  float s = 0.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) s = __builtin_fmaf(c[r], 0.f, s);
+  return __builtin_amdgcn_ballot_w64(s != 0.f) != 0;
+}
+// One contraction step by the fp32 matrix instruction: element e of the two lane halves is one pair.
+__device__ __forceinline__ floatx16 mma_f32(const float (&a)[8], const float (&b)[8], floatx16 c) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], c, 0, 0, 0);
+  return c;
 }
 
 template <class A>
@@ -321,6 +338,38 @@ __device__ __forceinline__ Op<F32> piece_frag(const char* blk, int ks, int l32, 
   return op_read<F32>(blk, ks, (l32 ^ ((2 * ks + hh) % 16)) + 32 * hh);
 }
 
+// (fp32) A tile of projections by the fp32 instruction: the lane's pair row at element `row` of z, its weight row at
+// element `wrow` of w.
+template <int C>
+__device__ __forceinline__ floatx16 proj_tile_f32(const BlockParams& p, int64_t row, const void* w, int64_t wrow, int hh) {
+  float s = 0.f;
+#pragma clang loop unroll(disable)
+  for (int c = 0; c < C; c += 8) {
+    const Frag<true> z = load8<true>(p.z, row + c);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += z.v[e];
+  }
+  const float mean = s * (1.0f / C);
+  s = 0.f;
+#pragma clang loop unroll(disable)
+  for (int c = 0; c < C; c += 8) {
+    const Frag<true> z = load8<true>(p.z, row + c);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s = __builtin_fmaf(z.v[e] - mean, z.v[e] - mean, s);
+  }
+  const float rstd = 1.0f / __builtin_sqrtf(s * (1.0f / C) + p.eps);
+  floatx16 acc = zero16();
+#pragma clang loop unroll(disable)
+  for (int c = 8 * hh; c < C; c += 16) {
+    Frag<true> z = load8<true>(p.z, row + c);
+    const Frag<true> g = load8<true>(p.gamma, c), b = load8<true>(p.beta, c), a = load8<true>(w, wrow + c);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) z.v[e] = __builtin_fmaf((z.v[e] - mean) * rstd, g.v[e], b.v[e]);
+    acc = mma_f32(a.v, z.v, acc);
+  }
+  return acc;
+}
+
 // ---- forward: layer norm and projections --------------------------------------------------------------
 // A wave keeps the weights of one or two tiles of 32 output channels (4*HD/32 tiles of q, k, v, gate over eight
 // waves) in registers, 64 of them; the bias heads are one more tile, its weights in LDS, that the waves take
@@ -429,6 +478,29 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
     fetch(min(st + teams, ntot - 1));
   }
   __syncthreads();
+  // the tile of channels n .. n + 31 of pair row q (this lane's)
+  auto store_tile = [&](const floatx16& acc, int n, int b, int q) {
+    const int sec = n / HD, col = n - sec * HD, h = col / p.D;
+    const int64_t off = (((int64_t)b * p.H + h) * LL + q) * p.D + (col - h * p.D) + hh * 8;
+    float y[2][8];
+    rows8(acc, y);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (sec == 3) {
+        Frag<F32> f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[u][e] = sigmoid<F32>(y[u][e] + bgs[col + 16 * u + 8 * hh + e]);
+        pack<A>(y[u], f);
+        store8<F32>(p.gate, off + 16 * u, f);
+      } else {
+        Frag<false> f;
+        pack<A>(y[u], f);
+        store8<false>(p.qkv[sec], off + 16 * u, f);
+      }
+    }
+  };
+  [[maybe_unused]] bool bad = false;
+  [[maybe_unused]] const int st0 = st;
   auto products = [&](int st, int it) {
     const char* buf = smem + (it & 1) * BUF;
     const int b = st / nst, p0 = (st - b * nst) * TR;
@@ -448,24 +520,8 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const int n = tile_of(t) * 32, sec = n / HD, col = n - sec * HD, h = col / p.D;
-        const int64_t off = (((int64_t)b * p.H + h) * LL + q) * p.D + (col - h * p.D) + hh * 8;
-        float y[2][8];
-        rows8(acc[t], y);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          if (sec == 3) {
-            Frag<F32> f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) y[u][e] = sigmoid<F32>(y[u][e] + bgs[col + 16 * u + 8 * hh + e]);
-            pack<A>(y[u], f);
-            store8<F32>(p.gate, off + 16 * u, f);
-          } else {
-            Frag<false> f;
-            pack<A>(y[u], f);
-            store8<false>(p.qkv[sec], off + 16 * u, f);
-          }
-        }
+        if constexpr (F32) bad = bad || not_finite(acc[t]);
+        store_tile(acc[t], tile_of(t) * 32, b, q);
       }
       if (!F32 && wave == ((RS * it + rs) & 7)) {
         floatx16 ab = zero16();
@@ -492,6 +548,18 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
     if (wave < 4) prepare(st, it);
     __syncthreads();
   }
+  if constexpr (F32)
+    if (bad)
+#pragma clang loop unroll(disable)
+      for (st = st0; st < ntot; st += teams) {
+        const int b = st / nst, q = min((st - b * nst) * TR + l32, LL - 1);
+        const uint32_t i = div_by_length((uint32_t)q, (uint32_t)p.L, inv_l), j = (uint32_t)q - i * (uint32_t)p.L;
+#pragma clang loop unroll(disable)
+        for (int t = 0; t < NT; ++t) {
+          const int n = tile_of(t) * 32, sec = n / HD;
+          store_tile(proj_tile_f32<C>(p, b * p.zs[0] + (int64_t)i * p.zs[1] + (int64_t)j * p.zs[2], p.w[sec], (int64_t)(n - sec * HD + l32) * C, hh), n, b, q);
+        }
+      }
 }
 
 // ---- forward: gating and output projection ------------------------------------------------------------
@@ -522,6 +590,21 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
       o[ks] = load8<false>(p.o, off);
     }
   };
+  auto store_tile = [&](const floatx16& acc, int t, const RowBlock& r) {
+    const int64_t oo = pair_off(p.outs, r) + hh * 8;
+    float y[2][8];
+    rows8(acc, y);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[u][e] += bos[t * 32 + 16 * u + 8 * hh + e];
+      Frag<F32> f;
+      pack<A>(y[u], f);
+      if (r.valid) store8<F32>(p.out, oo + t * 32 + 16 * u, f);
+    }
+  };
+  [[maybe_unused]] bool bad = false;
+  [[maybe_unused]] const int item0 = item;
   fetch();
   for (; item < nitems; item += step) {
     const RowBlock cur = rb;
@@ -542,23 +625,36 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
       rb = row_block(p, (item + step) / p.cg, lane);
       fetch();
     }
-    const int64_t oo = pair_off(p.outs, cur) + hh * 8;
     for (int t = g; t < NT; t += p.cg) {
       floatx16 acc = zero16();
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) acc = mma<A>(op_read<F32>(smem, t * KS + ks, lane), x[ks], acc);
-      float y[2][8];
-      rows8(acc, y);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) y[u][e] += bos[t * 32 + 16 * u + 8 * hh + e];
-        Frag<F32> f;
-        pack<A>(y[u], f);
-        if (cur.valid) store8<F32>(p.out, oo + t * 32 + 16 * u, f);
-      }
+      if constexpr (F32) bad = bad || not_finite(acc);
+      store_tile(acc, t, cur);
     }
   }
+  if constexpr (F32)
+    if (bad)
+#pragma clang loop unroll(disable)
+      for (item = item0; item < nitems; item += step) {
+        const RowBlock cur = row_block(p, item / p.cg, lane);
+#pragma clang loop unroll(disable)
+        for (int t = item % p.cg; t < NT; t += p.cg) {
+          floatx16 acc = zero16();
+#pragma clang loop unroll(disable)
+          for (int ks = 0; ks < KS; ++ks) {
+            const int h = ks * 16 / p.D;
+            const int64_t off = head_off(p, cur, h) + (ks * 16 - h * p.D) + hh * 8;
+            Frag<true> v = load8<true>(p.gate, off);
+            float b[8];
+            unpack<A>(load8<false>(p.o, off), b);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v.v[e] *= b[e];
+            acc = mma_f32(load8<true>(p.wo, (int64_t)(t * 32 + l32) * HD + ks * 16 + hh * 8).v, v.v, acc);
+          }
+          store_tile(acc, t, cur);
+        }
+      }
 }
 
 // ---- backward: output projection and gate -------------------------------------------------------------
@@ -611,47 +707,79 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) x[ks] = to_op(f[ks]);
   };
+  auto head_at = [&](int t, const RowBlock& r) { const int h = t * 32 / p.D; return head_off(p, r, h) + (t * 32 - h * p.D) + hh * 8; };
+  auto operands = [&](int t, const RowBlock& r, Frag<F32> (&gt)[2], Frag<false> (&o)[2]) {
+    const int64_t off = head_at(t, r);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) { gt[u] = load8<F32>(p.gate, off + 16 * u); o[u] = load8<false>(p.o, off + 16 * u); }
+  };
+  auto store_tile = [&](const floatx16& acc, int t, const RowBlock& r, const Frag<F32> (&gt)[2], const Frag<false> (&o)[2]) {
+    const int64_t off = head_at(t, r);
+    float y[2][8];
+    rows8(acc, y);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float a[8], b[8], d[8];
+      unpack<A>(gt[u], a);
+      unpack<A>(o[u], b);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        d[e] = y[u][e] * b[e] * a[e] * (1.0f - a[e]);
+        y[u][e] *= a[e];
+      }
+      Frag<false> fo;
+      Frag<F32> fd;
+      pack<A>(y[u], fo);
+      pack<A>(d, fd);
+      if (r.valid) {
+        store8<false>(p.dog, off + 16 * u, fo);
+        store8<F32>(p.dgp, off + 16 * u, fd);
+      }
+    }
+  };
+  [[maybe_unused]] bool bad = false;
+  [[maybe_unused]] const int item0 = item;
   fetch();
   for (; item < nitems; item += step) {
     const RowBlock cur = rb;
     const int g = item % p.cg;
     for (int t = g; t < NT; t += p.cg) {
-      const int h = t * 32 / p.D;
-      const int64_t off = head_off(p, cur, h) + (t * 32 - h * p.D) + hh * 8;
       Frag<F32> gt[2];
       Frag<false> o[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) { gt[u] = load8<F32>(p.gate, off + 16 * u); o[u] = load8<false>(p.o, off + 16 * u); }
+      operands(t, cur, gt, o);
       floatx16 acc = zero16();
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) acc = mma<A>(op_read<F32>(smem, t * KS + ks, lane), x[ks], acc);
-      float y[2][8];
-      rows8(acc, y);
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        float a[8], b[8], d[8];
-        unpack<A>(gt[u], a);
-        unpack<A>(o[u], b);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          d[e] = y[u][e] * b[e] * a[e] * (1.0f - a[e]);
-          y[u][e] *= a[e];
-        }
-        Frag<false> fo;
-        Frag<F32> fd;
-        pack<A>(y[u], fo);
-        pack<A>(d, fd);
-        if (cur.valid) {
-          store8<false>(p.dog, off + 16 * u, fo);
-          store8<F32>(p.dgp, off + 16 * u, fd);
-        }
-      }
+      if constexpr (F32) bad = bad || not_finite(acc);
+      store_tile(acc, t, cur, gt, o);
     }
     if (item + step < nitems) {
       rb = row_block(p, (item + step) / p.cg, lane);
       fetch();
     }
   }
+  if constexpr (F32)
+    if (bad)
+#pragma clang loop unroll(disable)
+      for (item = item0; item < nitems; item += step) {
+        const RowBlock cur = row_block(p, item / p.cg, lane);
+        const int64_t so = pair_off(p.douts, cur) + hh * 8;
+#pragma clang loop unroll(disable)
+        for (int t = item % p.cg; t < NT; t += p.cg) {
+          Frag<F32> gt[2];
+          Frag<false> o[2];
+          operands(t, cur, gt, o);
+          floatx16 acc = zero16();
+#pragma clang loop unroll(disable)
+          for (int ks = 0; ks < KS; ++ks) {
+            float w[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) w[e] = load1<A, F32>(p.wo, (int64_t)(ks * 16 + hh * 8 + e) * HD + t * 32 + l32);
+            acc = mma_f32(w, load8<true>(p.dout, so + ks * 16).v, acc);
+          }
+          store_tile(acc, t, cur, gt, o);
+        }
+      }
 }
 
 // ---- backward: input gradient and layer norm ----------------------------------------------------------
@@ -743,17 +871,8 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
   }
   if (st < ntot) put();
   __syncthreads();
-  for (; st < ntot; st += (int)gridDim.x) {
-    const int next = st + (int)gridDim.x;
-#pragma unroll
-    for (int n = 0; n < NZ; ++n) z[n] = load8<F32>(p.z, pair_off_of(p.zs, st, n));
-    fetch(min(next, ntot - 1));
-    floatx16 acc = zero16();
-#pragma unroll
-    for (int k = 0; k < KW; ++k) {
-      const int ks = SPLIT == 1 ? k : min(share * KW + k, KALL - 1);  // (a share's steps beyond the end: the last one again, with zero weights)
-      acc = mma<A>(to_op<true>(w[k]), piece_frag<F32>(smem + rs * SUB, ks, l32, hh), acc);
-    }
+  // the sums of a stage through LDS to the rows' threads, and the layer norm's backward
+  auto finish = [&](const floatx16& acc, int st) {
     float* plane = dxs + ((size_t)share * TR + rs * 32 + l32) * XROW + ct * 32 + 4 * hh;
 #pragma unroll
     for (int g = 0; g < 4; ++g) *reinterpret_cast<float4*>(plane + 8 * g) = make_float4(acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]);
@@ -789,8 +908,51 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
       pack<A>(x, f);
       store8<F32>(p.dz, pair_off_of(p.dzs, st, n), f);
     }
+  };
+  [[maybe_unused]] bool bad = false;
+  for (; st < ntot; st += (int)gridDim.x) {
+    const int next = st + (int)gridDim.x;
+#pragma unroll
+    for (int n = 0; n < NZ; ++n) z[n] = load8<F32>(p.z, pair_off_of(p.zs, st, n));
+    fetch(min(next, ntot - 1));
+    floatx16 acc = zero16();
+#pragma unroll
+    for (int k = 0; k < KW; ++k) {
+      const int ks = SPLIT == 1 ? k : min(share * KW + k, KALL - 1);  // (a share's steps beyond the end: the last one again, with zero weights)
+      acc = mma<A>(to_op<true>(w[k]), piece_frag<F32>(smem + rs * SUB, ks, l32, hh), acc);
+    }
+    if constexpr (F32) bad = bad || not_finite(acc);
+    finish(acc, st);
     put();
     __syncthreads();
+  }
+  if constexpr (F32) {
+    if (!__syncthreads_or(bad)) return;
+#pragma clang loop unroll(disable)
+    for (st = (int)blockIdx.x; st < ntot; st += (int)gridDim.x) {
+#pragma unroll
+      for (int n = 0; n < NZ; ++n) z[n] = load8<F32>(p.z, pair_off_of(p.zs, st, n));
+      const int b = st / nst, q = min((st - b * nst) * TR + rs * 32 + l32, LL - 1);
+      floatx16 acc = zero16();
+#pragma clang loop unroll(disable)
+      for (int ks = share * KW; ks < min(share * KW + KW, KALL); ++ks) {
+        const int s = ks / KH, e8 = (ks % KH) * 16 + hh * 8, h = e8 / p.D;
+        const int64_t off = (((int64_t)b * p.H + h) * LL + q) * p.D + (e8 - h * p.D);
+        float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (s < 3) {
+          unpack<A>(load8<false>(p.dqkv[s], off), x);
+        } else if (s == 3) {
+          unpack<A>(load8<true>(p.dgp, off), x);
+        } else if (hh == 0) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            if (g < p.H) x[g] = load1<A, false>(p.db, ((int64_t)b * p.H + g) * LL + q);
+        }
+        acc = mma_f32(frag_read<true>(static_cast<const char*>(p.wt), ct * KALL + ks, lane).v, x, acc);
+      }
+      finish(acc, st);
+      __syncthreads();
+    }
   }
 }
 
@@ -995,6 +1157,55 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
         if (st + 2 < last) fetch(st + 2);
       }
       __syncthreads();
+    }
+  }
+  if constexpr (F32) {
+    bool again = not_finite(acc[0]);
+#pragma unroll
+    for (int n = 1; n < NT; ++n) again = again || not_finite(acc[n]);
+    if (own && again) {  // two rows at a time, one per lane half
+#pragma unroll
+      for (int n = 0; n < NT; ++n) acc[n] = zero16();
+      const int col = at * 32 + l32;
+#pragma clang loop unroll(disable)
+      for (int r = first * TR; r < last * TR; r += 2) {
+        const int st = r / TR, b = st / nst, row = (st - b * nst) * TR + r % TR + hh, q = min(row, LL - 1);
+        const int64_t hb = (int64_t)b * p.H * LL * p.D + (int64_t)q * p.D;
+        float x, y[NT];
+        if constexpr (KIND == kWgradOut) x = load1<A, true>(srca, pair_row(p.douts, b, q) + col);
+        else if constexpr (KIND == kWgradBias) x = l32 < p.H ? load1<A, false>(srca, ((int64_t)b * p.H + l32) * LL + q) : 0.f;
+        else x = load1<A, KIND == kWgradGate>(srca, hb + head_part(col));
+        if constexpr (KIND == kWgradOut) {
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            const int64_t off = hb + head_part((wave / NA + n * (8 / NA)) * 32 + l32);
+            y[n] = load1<A, true>(p.gate, off) * load1<A, false>(p.o, off);
+          }
+        } else {
+          const int64_t off = pair_row(p.zs, b, q) + l32;
+          float z[NB], s = 0.f;
+#pragma unroll
+          for (int m = 0; m < NB; ++m) { z[m] = load1<A, true>(p.z, off + 32 * m); s += z[m]; }
+#pragma unroll
+          for (int m = 1; m < 32; m *= 2) s += __shfl_xor(s, m);
+          const float mean = s * (1.0f / C);
+          s = 0.f;
+#pragma unroll
+          for (int m = 0; m < NB; ++m) { z[m] -= mean; s = __builtin_fmaf(z[m], z[m], s); }
+#pragma unroll
+          for (int m = 1; m < 32; m *= 2) s += __shfl_xor(s, m);
+          const float rstd = 1.0f / __builtin_sqrtf(s * (1.0f / C) + p.eps);
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            y[n] = 0.f;
+#pragma unroll
+            for (int m = 0; m < NB; ++m) y[n] = wave / NA + n * (8 / NA) == m ? z[m] * rstd : y[n];
+          }
+        }
+        if (row >= LL) x = 0.f;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, row < LL ? y[n] : 0.f, acc[n], 0, 0, 0);
+      }
     }
   }
   // partial of this chunk

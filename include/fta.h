@@ -249,7 +249,11 @@ int fta_bwd_profile(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor
  * stride for the channels, element strides (b, i, j) that are multiples of 8, where i is the attention's
  * row and j its key: the ending node is the same call with the last two swapped.  Weights are contiguous in
  * torch's (out features, in features) order, 16-byte aligned; mask (B, L), 1 for keys that exist, or NULL; bg and
- * bo may be NULL.  C and H*D are 64 or 128. */
+ * bo may be NULL.  C and H*D are 64 or 128.
+ * Blocks of fp32 tensors: every product is one of fp32 operands summed in fp32, infinities and the values next to the type's
+ * largest included.  (A tile of finite sums is formed from three bf16 parts of each operand, one that is not all finite
+ * again by the fp32 matrix instruction: such calls are slower.)  The weights' gradients but the output projection's
+ * are gamma * (d^T xhat) + beta * (sum of d), in which an infinite d may come out as NaN. */
 typedef struct fta_block {
   int B, L, C, H, D, dtype;
   float eps;       /* of the layer norm */

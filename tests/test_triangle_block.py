@@ -267,3 +267,57 @@ def test_fp32_block_products_hold_fp32_precision(B, L, C, H, D):
     for name, got in (("wq", q), ("wk", k), ("wv", v)):
         assert _rel_l2(rows(got, torch.float16, D), x @ w[name].T) <= 2 ** -11, name
     assert _rel_l2(rows(bias, torch.float16, 1), x @ w["wb"].T) <= 2 ** -11
+
+
+def _same_values(a, b, tol, name):
+    """NaN where NaN is, infinity of the same sign where infinity is, elsewhere the same values (relative L2)."""
+    a, b = a.double(), b.double()
+    assert torch.equal(a.isnan(), b.isnan()), f"{name}: {int(a.isnan().sum())} NaN for {int(b.isnan().sum())}"
+    for sign in (1, -1):
+        assert torch.equal(a == sign * float("inf"), b == sign * float("inf")), f"{name}: infinities"
+    ok = b.isfinite()
+    if bool(ok.any()):
+        scale = b[ok].abs().max().clamp_min(1e-30)  # (squares of the largest values overflow)
+        assert _rel_l2(a[ok] / scale, b[ok] / scale) <= tol, name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L,C,H,D", [(1, 33, 128, 4, 32), (2, 40, 64, 2, 32), (1, 41, 128, 1, 64), (1, 24, 64, 4, 32), (1, 160, 128, 4, 32)])
+@pytest.mark.parametrize("where", ["gate weight", "output weight", "largest output weight", "gradient", "largest gradient", "key weight", "norm weight"])
+def test_infinities_of_an_fp32_block_come_out_as_they_went_in(where, B, L, C, H, D):
+    """An infinite weight or incoming gradient, and finite ones next to the type's largest value, against the block as
+    separate fp32 layers around attention(): the same infinities, the same NaN, and the finite values as without them.  (The
+    gradients of the projections are gamma * (d^T xhat) + beta * (sum of d), with infinite d not what d^T x is: not compared.)"""
+    torch.manual_seed(6)
+    fused, plain = TriangleAttention(C, D, H).to("cuda:0"), _Unfused(C, D, H).to("cuda:0")
+    z = torch.randn(B, L, L, C, device="cuda:0")
+    dout = torch.randn_like(z)
+    inf, big = float("inf"), 3.4e38
+    with torch.no_grad():
+        if where == "gate weight":  # saturated gates: everything stays finite but the sums over this channel
+            fused.linear_g.weight[5, 7] = inf
+            fused.linear_g.weight[C // 2 - 1, 3] = -inf
+        elif where == "output weight":
+            fused.linear_o.weight[3, 9] = inf
+        elif where == "largest output weight":
+            fused.linear_o.weight[3, 9] = big
+        elif where == "key weight":
+            fused.linear_k.weight[1, 2] = -inf
+        elif where == "norm weight":
+            fused.layer_norm.weight[4] = inf
+        elif where == "gradient":
+            dout[0, L - 1, L - 2, 6] = -inf
+            dout[0, 1, 2, 8] = inf
+        else:
+            dout[0, 1, 2, 8] = -big
+    plain.load_state_dict(fused.state_dict())
+    res = []
+    for blk in (fused, plain):
+        zz = z.clone().requires_grad_(True)
+        out = blk(zz)
+        res.append([out, *torch.autograd.grad(out, [zz, *blk.parameters()], dout)])
+        torch.cuda.synchronize()
+    assert fused._fused(z, None, None) is not None
+    for name, a, b in zip(["out", "z", *(n for n, _ in fused.named_parameters())], *res):
+        if where != "gradient" or name in ("out", "z", "linear_o.weight", "linear_o.bias"):
+            _same_values(a, b, 1e-3, name)
