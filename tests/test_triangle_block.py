@@ -321,3 +321,32 @@ def test_infinities_of_an_fp32_block_come_out_as_they_went_in(where, B, L, C, H,
     for name, a, b in zip(["out", "z", *(n for n, _ in fused.named_parameters())], *res):
         if where != "gradient" or name in ("out", "z", "linear_o.weight", "linear_o.bias"):
             _same_values(a, b, 1e-3, name)
+
+
+@pytest.mark.gpu
+def test_gate_of_an_fp32_block_is_the_sigmoid_to_fp32_precision():
+    """With zero gate weights the logits are the bias, from saturated to subnormal gates.  Bound: exp, good to one unit in the
+    last place, and three roundings; an absolute 2^-149 where the gate is subnormal."""
+    import ctypes
+
+    import fta_lib
+    lib = fta_lib.load()
+    L, C, H, D = 3, 128, 4, 32
+    st = (ctypes.c_int64 * 3)(L * L * C, L * C, C)
+    zero, one = torch.zeros(C, C, device="cuda:0"), torch.ones(C, device="cuda:0")
+    z, out = torch.randn(1, L, L, C, device="cuda:0"), torch.empty(1, L, L, C, device="cuda:0")
+    for lo, hi in ((-88.6, -86.0), (-86.0, -20.0), (-20.0, 20.0), (-1.0, 1.0), (-110.0, -89.0)):
+        bg = torch.linspace(lo, hi, H * D, device="cuda:0")
+        blk = fta_lib.Block(B=1, L=L, C=C, H=H, D=D, dtype=fta_lib.DTYPE_F32, eps=1e-5, sm_scale=1.0, z=z.data_ptr(), z_stride=st,
+                            norm_weight=one.data_ptr(), norm_bias=one.data_ptr(), bg=bg.data_ptr(),
+                            **{k: zero.data_ptr() for k in ("wq", "wk", "wv", "wb", "wg", "wo")})
+        state = torch.empty(lib.fta_block_state_bytes(ctypes.byref(blk)), dtype=torch.uint8, device="cuda:0")
+        fta_lib.check(lib.fta_block_fwd(ctypes.byref(blk), out.data_ptr(), st, state.data_ptr(), 0))
+        torch.cuda.synchronize()
+        n = L * L * H * D
+        at = 4 * ((2 * n + 255) // 256 * 256) + (2 * L * L * H + 255) // 256 * 256
+        gate = state[at:at + 4 * n].view(torch.float32).view(H, L, L, D).permute(1, 2, 0, 3).reshape(L * L, H * D).cpu().double()
+        ref = torch.sigmoid(bg.cpu().double())
+        # (exp(-x) overflows at 88.7: the gate is 0 from there)
+        ref = torch.where(bg.cpu() < -88.72, torch.zeros_like(ref), ref)
+        assert ((gate - ref).abs() <= 5 * 2.0 ** -24 * ref + 2.0 ** -149).all(), (lo, hi, ((gate - ref).abs() / ref.clamp_min(2.0 ** -149)).max())
