@@ -98,13 +98,19 @@ def test_kernel_sources_have_no_scalar_register_hazards():
     assert {s: h for s, (h, _) in report.items() if h} == {}
     # the hand-scheduled kernels keep everything in registers: a reload would make the compiler wait for
     # every memory operation in flight, the stage copies included, in the middle of the schedule
-    for src in ("fta_fwd1.hip", "fta_fwd2.hip", "fta_bwd_dq1.hip", "fta_bwd_dkdv1.hip"):
+    for src in ("fta_fwd1.hip", "fta_fwd1_slabs.hip", "fta_fwd2.hip", "fta_bwd_dq1.hip", "fta_bwd_dq1_bf16.hip", "fta_bwd_dkdv1.hip",
+                "fta_bwd_dkdv1_bf16.hip", "fta_bwd_short.hip"):
         spilling = dict(report[src][1])
         if src == "fta_fwd2.hip":
             # known: the tail-masking instances of the two-slab D=64 forward (template arguments <T, 2, true>)
             # keep five bias registers of a row's last tile in scratch (three reloads per row)
             spilling = {k: v for k, v in spilling.items() if "Li2ELb1E" not in k}
-        if src == "fta_bwd_dkdv1.hip":
+        if src == "fta_bwd_short.hip":
+            # known: its widest instances with dropout (eight waves, D=32) keep a few values of a row in scratch; every reload
+            # waits for the next row's copies, which are in flight from the row's start
+            assert all(v <= 17 for k, v in spilling.items() if "Li32ELi8ELb1E" in k)
+            spilling = {k: v for k, v in spilling.items() if "Li32ELi8ELb1E" not in k}
+        if src.startswith("fta_bwd_dkdv1"):
             # known: the D=64 instances for 384 queries per launch (template arguments <T, 64, 12, 4, ...>) use
             # every vector and accumulation register and keep one loop-invariant pair in scratch (one
             # reload per row; three accesses per kernel); still 2.5x the general kernel's rate at that length
