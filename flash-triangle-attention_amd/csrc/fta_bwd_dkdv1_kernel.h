@@ -432,6 +432,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   constexpr int OLD = 2 * DT;                                    // pieces of dK, and of dV
   constexpr bool PRE = !WIDE && LATER;
   constexpr int PRE_AT = STEPS == 1 ? 2 : (STEPS - 1) * TS - 2;  // the iteration that loads them
+  static_assert(PRE_AT >= 2 && PRE_AT < NJT - 2, "behind the store of the row before, in front of the row's last barrier");
   u32x4 oldk[OLD], oldv[OLD];
 #pragma unroll
   for (int x = 0; x < OLD; ++x) oldk[x] = oldv[x] = u32x4{0u, 0u, 0u, 0u};
@@ -439,6 +440,11 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
     constexpr int x = decltype(xc)::value;
     if constexpr (x < OLD) load_piece<kA, 32 * x>(oldk[x], voff_dk, uniform_ptr(dkcur));
     else if constexpr (x < 2 * OLD) load_piece<kA, 32 * (x - OLD)>(oldv[x - OLD], voff_dv, uniform_ptr(dvcur));
+  };
+  // Behind the wait that covers them: no reader of the pieces may be moved in front of it, and no copy made of them before.
+  auto old_landed = [&]() {
+#pragma unroll
+    for (int x = 0; x < OLD; ++x) asm volatile("" : "+a"(oldk[x]), "+a"(oldv[x]));
   };
   auto swap_halves = [](uint32_t& x, uint32_t& y) {
     auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
@@ -516,6 +522,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       if constexpr (g % TS == TS - 2) {
         constexpr int tn = ((g + 2) / TS) % STEPS;           // part of the published stage
         sync_stage(std::integral_constant<int, (tn + 1) % STEPS>{});
+        if constexpr (PRE && g == NJT - 2) old_landed();
       }
       if constexpr (g == NJT - 1) row_operands(ir + 1, kf_n, kl_n, vf_n);  // the next row's K, V fragments
       // -- row change: dK, dV of the previous row are complete after iteration 0

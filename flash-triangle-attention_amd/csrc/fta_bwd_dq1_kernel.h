@@ -522,6 +522,11 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
       load_piece<kV, 32 * SK * y>(old[y], voff_dq, rb);
     });
   };
+  // Behind the wait that covers them: no reader of the pieces may be moved in front of it, and no copy made of them before.
+  auto old_landed = [&]() {
+#pragma unroll
+    for (int y = 0; y < XG / 2; ++y) asm volatile("" : "+v"(old[y]));
+  };
   auto store_dq = [&](const float* vals) {
     half_t* dqr = reinterpret_cast<half_t*>(reinterpret_cast<char*>(dqcur) + voff_dq);
     advance(dqcur, step_dq);
@@ -605,6 +610,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
       // in the iteration before it; elsewhere a later iteration, or the end of the row, has waited for them)
       if constexpr (DEEP && g == SYNC_B && TS1 == 2) lds_wait_older<0>(kf, vf, ktlo_p, kthi_p);
       if constexpr (g == SYNC_A || g == SYNC_B) sync_stage(gc, ir);
+      if constexpr (PRE && g == (PRE_NEXT ? SYNC_A : SYNC_B)) old_landed();
       if constexpr (g == NKT - 1) row_operands(ir + 1, qf_n, ql_n, dof_n, augS_n, augD_n);
       // -- row change: the accumulator of the previous row is complete after iteration 0
       //    (DEEP with two slabs does this work in pieces, in the gaps between MFMAs: row_work below)
@@ -848,8 +854,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
   if constexpr (PRE && !PRE_NEXT) old_issue();
   if constexpr (PRE) {
     wait_vmem_all();
-#pragma unroll
-    for (int y = 0; y < XG / 2; ++y) asm volatile("" : "+v"(old[y]));
+    old_landed();
   }
   split_groups(acc);
   if constexpr (SK == 2) {

@@ -26,6 +26,10 @@ that the compiler does not recognise as MFMAs:
   * a vector-memory store of more than 8 bytes has its data registers overwritten by a vector-ALU
     instruction in the two slots after it (the store still reads them there).
 
+  * the destination of a global load inside an asm block, which the compiler takes to be there when the
+    block ends, is read or written (copied, spilled, added ...) on some way through the branches before a
+    wait that covers the load.
+
     python isa_lint.py            # compiles every kernel source to assembly and checks it
 
 It also lists the kernels that spill registers to scratch memory (scratch_ops): the hand-scheduled
@@ -33,8 +37,8 @@ kernels must not -- the compiler waits for ALL outstanding memory operations bef
 value, the global->LDS copies in flight included.
 
 Slots are counted as the hardware counts wait states: one per instruction, N+1 for `s_nop N`.
-The scan is linear (labels and branches are ignored), which is what the hardware sees on the
-fall-through path and is conservative for the others.
+The scan for the slot distances is linear (labels and branches are ignored), which is what the hardware
+sees on the fall-through path and is conservative for the others.
 """
 from __future__ import annotations
 
@@ -127,11 +131,58 @@ def lint(asm: str) -> list[str]:
     hits += _lint_mfma(ins)
     hits += _lint_dot(ins)
     hits += _lint_wide_store(ins)
+    hits += _lint_asm_loads(asm)
     for (ln, s), (ln2, s2) in zip(ins, ins[1:]):
         if s.startswith(TRANS) and s2.startswith("v_") and not s2.startswith(TRANS) and not s2.startswith("v_mfma"):
             rest = s2.split(None, 1)[1].split(",", 1)
             if len(rest) > 1 and _vregs(_dest(s)) & _vregs(rest[1]):
                 hits.append(f"line {ln}: `{s}` result read by line {ln2}: `{s2}` in the next slot")
+    return hits
+
+
+ASM_LOAD = re.compile(r"global_load_(?!lds_)\w+\s")
+VMEM_COUNTED = re.compile(r"(global|buffer|flat|scratch)_(load|store|atomic)")
+
+
+def _lint_asm_loads(asm: str) -> list[str]:
+    """Follows every way from a global load of an asm block to the wait that covers it: `s_waitcnt vmcnt(N)` does once
+    N or more memory operations were issued behind the load (they complete in order)."""
+    ins, loads, labels, in_asm = [], [], {}, False
+    for ln, line in enumerate(asm.split("\n"), 1):
+        if "#ASMSTART" in line or "#ASMEND" in line:
+            in_asm = "#ASMSTART" in line
+            continue
+        s = line.split(";")[0].split("//")[0].strip()
+        if re.match(r"[.\w$]+:$", s):
+            labels[s[:-1]] = len(ins)
+        elif s and not s.startswith("."):
+            if in_asm and ASM_LOAD.match(s):
+                loads.append(len(ins))
+            ins.append((ln, s))
+    hits = []
+    for i in loads:
+        dst = _vregs(_dest(ins[i][1]))
+        fewest: dict[int, int] = {}           # instruction -> fewest memory operations behind the load on any way there
+        todo = [(i + 1, 0)]
+        while todo:
+            j, behind = todo.pop()
+            while j < len(ins) and fewest.get(j, behind + 1) > behind:
+                fewest[j] = behind
+                ln, s = ins[j]
+                m = re.match(r"s_waitcnt\b.*vmcnt\((\d+)\)", s)
+                if s.startswith("s_endpgm") or (m and int(m.group(1)) <= behind):
+                    break
+                if not s.startswith("s_") and _vregs(s) & dst:
+                    hits.append(f"line {ins[i][0]}: `{ins[i][1]}` may be in flight where line {ln}: `{s}` touches its destination")
+                    break
+                behind += bool(VMEM_COUNTED.match(s))
+                if s.startswith(("s_branch", "s_cbranch")):
+                    to = labels.get(s.split()[1])
+                    if to is not None:
+                        todo.append((to, behind))
+                    if s.startswith("s_branch"):
+                        break
+                j += 1
     return hits
 
 

@@ -4,9 +4,10 @@ A memory instruction or an MFMA inside an asm block is invisible to the compiler
 the assembly of every kernel source is checked for (1) a vector-memory instruction reading a scalar
 register that a vector-ALU instruction wrote fewer than 5 slots earlier, (2) a global->LDS copy
 reading M0 right after the scalar instruction that wrote it, (3) an MFMA result touched fewer than 11
-slots after the MFMA, (4) an MFMA operand written by the vector ALU fewer than 2 slots before and
+slots after the MFMA, (4) an MFMA operand written by the vector ALU fewer than 2 slots before,
 (5) a dot-product result read by another vector-ALU opcode fewer than 3 slots later (or overwritten
-by one fewer than 4 slots later).
+by one fewer than 4 slots later) and (6) the destination of an asm block's global load touched before a
+wait that covers the load.
 The checker itself is pinned on hand-written listings."""
 import isa_lint
 
@@ -132,3 +133,32 @@ def test_checker_on_wide_store_data():
     narrow = "global_store_dwordx2 v131, v[34:35], s[10:11]\nv_mul_f32_e32 v34, v8, v38\n"
     assert len(isa_lint.lint(bad)) == 1
     assert isa_lint.lint(late) == [] and isa_lint.lint(other) == [] and isa_lint.lint(narrow) == []
+
+
+def _asm(line):
+    return f"\t;;#ASMSTART\n\t{line}\n\t;;#ASMEND\n"
+
+
+def test_checker_on_loads_that_the_compiler_does_not_see():
+    load = _asm("global_load_dwordx4 v[8:11], v1, s[2:3] offset:16")
+    copy = _asm("global_load_lds_dwordx4 v2, s[4:5]")
+    add, wait = "\tv_pk_add_f16 v12, v9, v13\n", "\ts_waitcnt vmcnt({})\n"
+    assert len(isa_lint.lint(load + add)) == 1
+    assert isa_lint.lint(load + wait.format(0) + add) == []
+    # the loads of ordinary code have the compiler's own waits
+    assert isa_lint.lint("\tglobal_load_dwordx4 v[8:11], v1, s[2:3]\n\ts_waitcnt lgkmcnt(0)\n" + add) == []
+    # a wait that lets more operations stay in flight than were issued behind the load
+    assert len(isa_lint.lint(load + copy * 2 + wait.format(3) + add)) == 1
+    assert isa_lint.lint(load + copy * 3 + wait.format(3) + add) == []
+    # moved, spilled or overwritten before it is there
+    assert len(isa_lint.lint(load + "\tv_accvgpr_write_b32 a0, v10\n")) == 1
+    assert len(isa_lint.lint(load + "\tscratch_store_dword off, v11, off\n")) == 1
+    assert len(isa_lint.lint(load + "\tv_mov_b32_e32 v8, 0\n")) == 1
+    assert len(isa_lint.lint(_asm("global_load_dwordx4 a[8:11], v1, s[2:3]") + "\tv_accvgpr_read_b32 v0, a8\n")) == 1
+    # over the back edge of a loop: the reader stands in front of the load
+    loop = "\ts_nop 0\n.LBB0_1:\n{}" + add + load + "\ts_cbranch_scc1 .LBB0_1\n" + wait.format(0) + "\ts_endpgm\n"
+    assert len(isa_lint.lint(loop.format(""))) == 1
+    assert isa_lint.lint(loop.format(wait.format(0))) == []
+    # one of two ways round the wait
+    assert len(isa_lint.lint(load + "\ts_cbranch_execz .LBB0_2\n" + wait.format(0) + ".LBB0_2:\n" + add)) == 1
+    assert isa_lint.lint(load + "\ts_branch .LBB0_2\n" + add + ".LBB0_2:\n" + wait.format(0) + add) == []
