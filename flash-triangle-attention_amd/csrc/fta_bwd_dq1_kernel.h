@@ -893,7 +893,8 @@ inline hipError_t launch_dq1_range(const BwdParams& p, int range, dim3 grid, siz
   } else {
     FTA_DQ1_LATER(4) FTA_DQ1_LATER(5) FTA_DQ1_LATER(6) FTA_DQ1_LATER(7) FTA_DQ1_LATER(8)
     FTA_DQ1_CASE(1, 8)
-    FTA_DQ1_CASE(2, 4) FTA_DQ1_CASE(2, 5) FTA_DQ1_CASE(2, 6) FTA_DQ1_CASE(2, 7) FTA_DQ1_CASE(2, 8)
+    // (a first range is the row's longest: five units of 64 keys at least)
+    FTA_DQ1_CASE(2, 5) FTA_DQ1_CASE(2, 6) FTA_DQ1_CASE(2, 7) FTA_DQ1_CASE(2, 8)
   }
 #undef FTA_DQ1_CASE
 #undef FTA_DQ1_LATER
