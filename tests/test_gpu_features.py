@@ -137,11 +137,12 @@ def test_masks_that_cover_all_keys_a_wave_has_seen(dtype, B, H, L1, L2, D, lo, h
 _ALL_MASKED = [
     # one-kernel backward
     (64, 32, "plain"), (128, 32, "plain"), (128, 64, "plain"), (128, 32, "dropout"), (128, 64, "dropout"), (64, 32, "precise"), (128, 64, "precise"),
+    (256, 32, "dropout"),
     # hand-scheduled backward (one and several key ranges; the precise instances in natural units)
     (256, 32, "plain"), (384, 32, "plain"), (512, 32, "plain"), (1024, 32, "plain"), (256, 64, "plain"), (384, 64, "plain"), (512, 64, "plain"),
     (256, 32, "precise"), (512, 32, "precise"),
     # general backward kernels
-    (256, 32, "dropout"), (512, 32, "dropout"), (1024, 32, "dropout"), (256, 64, "dropout"), (512, 64, "precise"),
+    (512, 32, "dropout"), (1024, 32, "dropout"), (256, 64, "dropout"), (512, 64, "precise"),
     # rows that end inside a tile: the keys beyond them weigh nothing beside masked ones either
     (3, 32, "plain"), (7, 64, "plain"), (9, 32, "dropout"), (33, 32, "plain"), (64, 64, "plain"), (64, 32, "dropout"), (97, 32, "precise"), (101, 64, "dropout"),
     (131, 32, "plain"), (200, 32, "plain"), (300, 32, "precise"), (457, 32, "plain"), (701, 32, "plain"), (1290, 32, "plain"), (1801, 32, "plain"),
@@ -241,8 +242,8 @@ def test_bf16_either_side_of_the_scale_that_selects_the_backward_kernels(sm):
 def test_bf16_large_scale_keeps_the_accuracy_of_a_small_one(L1, L2, D):
     """sm_scale = 1.3 (upstream's benchmark scale, flash_tt_attn.py:783) against 1/sqrt(D) on the same
     inputs: the gradients of the large scale are no further from the oracle than 2x those of the small
-    one (with the scaled operands rounded to 8 bits once, dQ and dK were 4x off).  1152 = 512 + 384 + 256
-    runs every range size of the (hi, lo) instances, 300 their masked tail."""
+    one (with the scaled operands rounded to 8 bits once, dQ and dK were 4x off).  1152 takes three ranges of
+    384 in the (hi, lo) instances (their other range sizes: test_backward_tiles_in_steps_of_64), 300 a masked tail."""
     print(f"case bf16 scales L1={L1} L2={L2} D={D}", flush=True)
     q, k, v, b, do = _inputs(1, 2, L1, L2, D, 36, torch.bfloat16)
     errs = {}
@@ -256,8 +257,9 @@ def test_bf16_large_scale_keeps_the_accuracy_of_a_small_one(L1, L2, D):
 
 
 def test_bf16_precise_mode_and_sum_over_key_ranges():
-    """The precise switch routes bf16 to the vector-ALU instances; L2 = 1152 = 512 + 384 + 256 runs every
-    range size of the pipelined kernels with the bf16 read-modify-write of dQ, dK, dV between launches."""
+    """The precise switch routes bf16 to the vector-ALU instances; without it L2 = 1152 runs three ranges of 384 of the
+    hand-scheduled kernels with the bf16 read-modify-write of dQ, dK, dV between launches (the other range sizes:
+    test_backward_tiles_in_steps_of_64)."""
     import flash_tt_attn as fta
     sm = 1.0 / math.sqrt(32)
     q, k, v, b, do = _inputs(1, 2, 12, 1152, 32, 33, torch.bfloat16)
@@ -478,9 +480,10 @@ def test_dropout_without_a_seed_draws_one_and_lengths_beyond_what_is_built_raise
 def test_precise_backward_holds_the_tolerance_on_large_biases_and_scores(bias_std, std, sm, L1, L2, D):
     """Bias spread 30 or score spread ~60: the default backward kernels round log2(e)*bias and the
     scaled Q/K to fp16 on their way into the matrix core and leave the 1e-2 gradient bar there
-    (documented); the precise mode does not and holds it: at D = 32 and rows of 256 keys and more through
-    the hand-scheduled kernels' instances with the operand pair and the exponent in natural units (every
-    key range size, tails, several ranges), elsewhere through the vector-ALU kernels."""
+    (documented); the precise mode does not and holds it: at D = 32 and rows beyond 192 keys through
+    the hand-scheduled kernels' instances with the operand pair and the exponent in natural units (tails, one
+    range and several), at 128 through the one-kernel backward (more of that one below), at D = 64 through the
+    vector-ALU kernels."""
     import flash_tt_attn as fta
     B, H = 1, 2
     if D == 64:
@@ -499,6 +502,29 @@ def test_precise_backward_holds_the_tolerance_on_large_biases_and_scores(bias_st
     assert torch.equal(default["o"], precise["o"])
     _compare(precise, ref, torch.float16, f"precise bias_std{bias_std} std{std}")
     assert max(e_pre.values()) < max(e_def.values())
+
+
+@pytest.mark.parametrize("L1,L2", [(4, 97), (5, 131), (3, 160), (40, 192)])
+def test_precise_instances_of_the_one_kernel_backward(L1, L2):
+    """The one-kernel backward (here with four, five and six waves) keeps everything per score in fp32 either way; its
+    precise instances round P and dS to nearest on their way into the matrix core instead of toward zero: dQ, dK and dV come
+    closer, the bias gradient, summed unrounded, is the same."""
+    import fta_lib
+    import flash_tt_attn as fta
+    B, H, sm = 1, 2, 1.0 / math.sqrt(32)
+    opt = fta_lib.Options(fta_lib.DTYPE_F16, 0, 0.0, 0, 1)
+    assert fta_lib.describe_plan(B, H, L1, L2, 32, sm, opt)["dq"]["kernel"] == f"fta_bwd_short_kernel<32,{(L2 + 31) // 32}>"
+    q, k, v, b, do = orc.make_inputs(B, H, L1, L2, 32, seed=17, bias_std=30.0, device=DEV)
+    ref, default = _oracle(q, k, v, b, sm, do), _run(q, k, v, b, sm, do)
+    fta.PRECISE_BACKWARD = True
+    try:
+        precise = _run(q, k, v, b, sm, do)
+    finally:
+        fta.PRECISE_BACKWARD = False
+    _compare(precise, ref, torch.float16, f"precise one kernel L{L2}")
+    for n in ("dq", "dk", "dv"):
+        assert orc.rel_l2(precise[n], ref[n]) < orc.rel_l2(default[n], ref[n]), n
+    assert torch.equal(precise["db"], default["db"])
 
 
 # ---- the hand-scheduled forward with an odd number of tiles per slab ----------------------------------------
@@ -523,11 +549,11 @@ def test_forward_rows_of_an_odd_number_of_tiles(L1, L2, tiled, dtype):
 # ---- the hand-scheduled backward at tiled lengths in steps of 64 -------------------------------------------
 
 @pytest.mark.parametrize("mode", ["fp16", "bf16", "bf16 operand pair", "precise"])
-@pytest.mark.parametrize("D,L2", [(32, L) for L in (193, 256, 257, 320, 385, 448, 449, 513, 640, 703, 1088)]
+@pytest.mark.parametrize("D,L2", [(32, L) for L in (193, 256, 257, 320, 385, 448, 449, 513, 640, 703, 896, 1024, 1088)]
                          + [(64, L) for L in (129, 192, 257, 320, 400, 576, 640, 701, 832)])
 def test_backward_tiles_in_steps_of_64(D, L2, mode):
-    """Every number of tiles per wave (key ranges of 256 to 512 keys in two slabs, of 256 in one; D = 64: 160 to
-    256; query ranges of 256 to 512, at D = 64 256 to 384), odd numbers of them (stages of unequal length), groups of 128 queries or keys
+    """Every number of tiles per wave (key ranges of 256 to 512 keys in two slabs, first and later ones: 513, 640, 703, 896
+    and 1024 have later ranges of 256, 320, 384 (1088), 448 and 512; of 256 in one; D = 64: 160 to 256; query ranges of 256 to 512, at D = 64 256 to 384), odd numbers of them (stages of unequal length), groups of 128 queries or keys
     that end beyond the tiled length, one to four ranges; rows that end inside a tile and whole ones."""
     import fta_lib
     import flash_tt_attn as fta
