@@ -101,14 +101,18 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
   // ---- global -> LDS staging of one (row, step): S slabs x KT keys of K and V, copied
   // asynchronously straight into LDS (no registers); the tile row r holds key
   // (r / KT) * KW + t * KT + r % KT.
-  // (the widest D = 64 slab has no registers left for the plan: kept, the compiler spills it and reloads it
-  // in front of every stage, and a reload waits for every copy in flight -- 10.4 against 6.3 ms at B1 H2
-  // L1792; that instance forms the offsets at each stage, like the tail path)
+  // (the wide D = 64 slabs have no registers left for the whole plan: kept, the compiler spills it and reloads it
+  // in front of every stage, and a reload waits for every copy in flight -- 448 keys: 10.4 against 6.3 ms at B1 H2
+  // L1792; 384 keys, three and four slabs: 5.06 against 3.46 at B1 H4 L1152, 9.82 against 7.32 at L1536.  The former form
+  // the offsets at each stage, like the tail path; the latter, too, but with two slabs, whose waves have two copies of a tile and
+  // not four, keep them: 3.07 against 3.23 at B2 H8 L768)
   constexpr bool PLAN = !(D == 64 && NKT >= 14);
-  DmaPlan<4> plk, plv;
+  constexpr int COPIES = (D == 64 && !DROP && KT == 64 && NKT == 12) ? 2 : 4;
+  const bool planned = PLAN && (COPIES == 4 || stage_rows * (D / 8) / 64 <= COPIES * nwaves);
+  DmaPlan<COPIES> plk, plv;
   if constexpr (PLAN) {
-    dma_plan<D, 4>(plk, stage_rows, KT, KW, p.ks[3], wave, lane, nwaves);
-    dma_plan<D, 4>(plv, stage_rows, KT, KW, p.vs[3], wave, lane, nwaves);
+    dma_plan<D, COPIES>(plk, stage_rows, KT, KW, p.ks[3], wave, lane, nwaves);
+    dma_plan<D, COPIES>(plv, stage_rows, KT, KW, p.vs[3], wave, lane, nwaves);
   }
   // Stages are issued in order; the cursor keeps the row pointers so that issuing costs scalar adds.
   int cur_t = 0;
@@ -126,7 +130,7 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
     const int cur_buf = (STEPS & 1) ? buf_ct : buf_rt;
     buf_rt ^= 1;
     // (stages that end inside the row in every slab take the offsets computed once)
-    if (PLAN && (!tail || (S - 1) * KW + (cur_t + 1) * KT <= p.L2)) {
+    if (planned && (!tail || (S - 1) * KW + (cur_t + 1) * KT <= p.L2)) {
       dma_issue(plk, kcur + cur_t * kstep, ldsK[cur_buf]);
       dma_issue(plv, vcur + cur_t * vstep, ldsV[cur_buf]);
     } else {
