@@ -106,7 +106,10 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
   // L1792; 384 keys, three and four slabs: 5.06 against 3.46 at B1 H4 L1152, 9.82 against 7.32 at L1536.  The former form
   // the offsets at each stage, like the tail path; the latter, too, but with two slabs, whose waves have two copies of a tile and
   // not four, keep them: 3.07 against 3.23 at B2 H8 L768)
-  constexpr bool PLAN = !(D == 64 && NKT >= 14);
+  // With dropout slabs of 512 keys at D = 32 and of 256 at D = 64 form them at each stage, too: 318 against 270 us at B1 H4 L512, 2.64
+  // against 2.13 ms at L1024, D = 64 48 / 45 us at L256, 400 / 340 at L512, 4.58 / 3.05 ms at L1024; slabs of 384 and 448 keys
+  // at D = 32, which spill as well, are 2 % faster with the plan.
+  constexpr bool PLAN = !(D == 64 && NKT >= 14) && !(DROP && KT == 64 && NKT >= (D == 64 ? 8 : 16));
   constexpr int COPIES = (D == 64 && !DROP && KT == 64 && NKT == 12) ? 2 : 4;
   const bool planned = PLAN && (COPIES == 4 || stage_rows * (D / 8) / 64 <= COPIES * nwaves);
   DmaPlan<COPIES> plk, plv;
