@@ -58,7 +58,7 @@ def read_clock_and_power():
 
 
 PROFILE_SUMMARY = os.path.join(ROOT, "profiles", "fta_kernels_b4h8_l512_d32.txt")
-FETCH_UNIT_BYTES = 2048.0   # FETCH_SIZE reads 1 per 2 KiB on this pool (copy kernels of the same runs, see the summary)
+FETCH_UNIT_BYTES = 2048.0   # FETCH_SIZE reads 1 per 2 KiB (copy kernels of the same runs, see the summary)
 WRITE_UNIT_BYTES = 1024.0
 
 

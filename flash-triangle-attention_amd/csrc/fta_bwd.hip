@@ -32,6 +32,11 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   // eight waves (four slabs of 64, 96 or 128 keys; two of 128, 192 or 256 queries).  Cut into the widest equal pieces that
   // divide the row, 640 keys take five launches of 128: steps at B1 H4 in bf16 of 576, 640, 896 and 1280 keys that way and as
   // below 3.09 / 1.85, 3.46 / 2.18, 7.54 / 5.65, 18.4 / 16.6 ms.
+  // Longer rows at B1 H1: 1408 9.45 / 5.88, 1664 15.7 / 9.43, 1792 12.3 / 11.3, 2176 38.7 / 26.0, 2304 36.8 / 32.3, 3328 103 / 99.3, 3840 166 / 148,
+  // 1152, 2560 and 4096 equal.  Five, seven and nine times 384 keys are the exception: in ranges of 384 dQ/dBias takes 2.67 us a key
+  // at 1920, in ranges of 512, whose geometry comes from the arguments (known at compile time it spills), 3.03 (dK/dV 2.73 and 2.65), and a
+  // step 1 to 4 % longer (1920 19.7 / 20.0, 2688 45.5 / 46.4, 3456 112 / 116); but dQ, too, is held in the tensors' type between launches,
+  // and those are one or two fewer here.
   // dK and dV are held in the tensors' type from one query range to the next, a rounding at each.  So dK/dV takes rows that
   // 768 or 1024 divides in launches of as many queries, four slabs of 192 or 256: of 768, 1024, 2048, 2304 and
   // 3072 queries its relative error in bf16 is 2.37, 2.36, 2.64, 2.88 and 2.88e-3, in ranges of up to 512 2.65, 2.63, 3.11,
@@ -105,8 +110,8 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   // ---- dK/dV kernel: query slabs of at most 256 (D=32) / 128 (D=64) queries per wave (register
   // budget); up to SJ slabs share a workgroup, longer rows take several launches over query ranges
-  // (the dropout instances spill 42 registers with 256 queries per wave and still measure 4 % faster per
-  // step than with 128, which halves the reuse of a workgroup's K/V rows)
+  // (the dropout instances with 256 queries per wave touch scratch memory twice per row; with 128, which halves the reuse of a
+  // workgroup's K/V rows, a step took 4 % longer, also when the former spilled 42 registers)
   const int jwmax = (D == 32) ? 256 : 128;
   int jw = 0;
   for (int c = jwmax; c >= 128; c -= 128)

@@ -88,7 +88,9 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
 #define FTA_DKDV_FEAT_CASE(DD, NN, JJ) \
   if (e == hipErrorInvalidConfiguration && D == DD && pl.NJT == NN && pl.JT == JJ) \
     e = launch_kernel(fta_bwd_dkdv_kernel<T, DROP, DD, NN, JJ>, p, grid, block, pl.smem2, st);
-      if constexpr (DROP) {  // fixed geometry: 256, 384, 512, 768 and 1024 queries to a launch
+      // fixed geometry: 384, 512, 768 and 1024 queries to a launch.  (Rows of up to 256 queries at D = 32 run the one-kernel
+      // backward; <8, 64, 1> and <4, 64> are theirs where fta_debug_select_kernels asks for the general kernels)
+      if constexpr (DROP) {
 #define FTA_DKDV_FIX_CASE(NN, SS)                                                                                        \
   if (D == 32 && pl.threads2 == 512 && pl.NJT == NN && pl.JT == 64 && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, 64, SS).r &&  \
       pl.nb2 == dkdv_ring(32, NN, 64, SS).nb)                                                                            \

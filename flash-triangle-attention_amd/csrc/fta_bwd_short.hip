@@ -29,9 +29,9 @@
 // in LDS, the next row's coming in during the first four rounds.  The bias has no registers left: a wave packs its
 // tiles, converted and in the order of the rounds, where it will write its part of the partial bias gradient at the end, and loads
 // a tile of 2 KB per round (from L2, a round ahead).  Bound: the chain of a round (exchange read, S and dP, exponentials,
-// exchange write, barrier), 1.8 us for two tiles per SIMD of which the vector ALU is busy 40 % and the matrix core 15.
+// exchange write, barrier), 1.8 us (260 us for 24 rows of six rounds) for two tiles per SIMD of which the vector ALU is busy 40 % and the matrix core 15.
 // Backward kernels, two (dQ/dBias, dK/dV) -> this, us: B4 H8 L192 fp16 346 -> 260, B1 H4 L192 51 -> 43; training steps B4 H8
-// L160 317 -> 227, L192 425 -> 339, B1 H4 L192 with dropout 220 -> 82, B2 H4 L256 with dropout 300 -> 236.  B1 H4 L224
+// L160 332 -> 227, L192 441 -> 339, B1 H4 L192 with dropout 220 -> 83, B2 H4 L256 with dropout 300 -> 236.  B1 H4 L224
 // 85 -> 85 and B2 H4 L256 160 -> 174: without dropout the two kernels take over at 192 keys (their tiles then fill whole slabs
 // of 256, and this one's waves have the second barrier).
 // Measured and left: the two waves of a SIMD half a round apart (L192 339 -> 404), the own Q and dO in registers (as fast).

@@ -99,8 +99,9 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int
 }
 
 FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, int row, bool feat) {
-  // L2 here is the length the tiles cover (a multiple of 128, or of 64 where a rule below takes it).  Slab widths are tried in this order,
-  // the first that has a built instance and a stage length that fits is taken:
+  // L2 here is the length the tiles cover: a multiple of 128, or of 32 or 64 where the hand-scheduled kernel or a rule below takes it
+  // (padded_len_fwd tries them in steps of 32).  The hand-scheduled kernels first; then slab widths are tried in this order, the first that
+  // has a built instance and a stage length that fits is taken:
   const int kwmax = (D == 32) ? 512 : 256;  // the widest that keeps the stationary bias within the register budget
   FwdPlan pl{};
   if (!feat && plan_fwd1(B, H, L1, L2, D, row, pl)) return pl;

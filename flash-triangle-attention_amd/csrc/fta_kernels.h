@@ -73,8 +73,12 @@ inline int balanced_chunks(long base, int L1, long slots, int least = 8) {
 }
 
 // The fewest rows of a chunk for rows of L2 keys: a workgroup's set-up loads one bias row per query, so that short rows
-// can be spread thinner over the chip than eight to a workgroup (B1 H4, us, eight -> this: forward at D = 64, L48 23.7 -> 9.5,
-// L192 48.1 -> 28.4).
+// can be spread thinner over the chip than eight to a workgroup.  B1 H4, us, eight -> this: forward at D = 64 of 48, 128, 192,
+// 256, 384, 448 keys 23.8 -> 9.7, 23.6 -> 10.0, 48.4 -> 29.9, 51.2 -> 35.0, 114 -> 112, 216 -> 213; with dropout at D = 32 of
+// 64, 192, 256, 384 24.1 -> 9.8, 50.4 -> 23.4, 42.2 -> 35.6, 114 -> 114; training steps at D = 32 (dK/dV) of 200, 256, 384, 448
+// 92 -> 87, 98 -> 97, 256 -> 252, 402 -> 404, with dropout of 300, 384, 448 324 -> 312, 444 -> 445, 851 -> 852; at D = 64 of
+// 160, 256, 384 141 -> 110, 166 -> 155, 518 -> 520, with dropout of 192, 256, 384 285 -> 217, 314 -> 284, 1205 -> 1206.  Where B * H
+// fills the chip nothing changes (B4 H8 of 192, 256 and 384 keys within 0.7 %).  From 512 keys on it is eight.
 inline int least_rows(int L2) { return L2 >= 512 ? 8 : L2 <= 128 ? 2 : L2 / 64; }
 
 // ---- backward ---------------------------------------------------------------------------------

@@ -2,7 +2,7 @@
 
 TEST INFRASTRUCTURE ONLY.  Nothing in the shipped package imports this module; only
 tests/, __graft_entry__.smoke() and the cpu_baseline leg of bench.py use it, and only
-as the checker.
+as the reference.
 
 Every function restates one piece of the upstream single-file reference
 (flash_tt_attn.py) and says which lines it follows:

@@ -1,4 +1,4 @@
-"""bench.py on a machine without a GPU: the flags of the driver's contract parse, more than one GPU is
+"""bench.py on a machine without a GPU: the flags of its contract parse, more than one GPU is
 refused with a message (this build runs on one), and the clock/power reader copes with missing files."""
 import os
 import subprocess
