@@ -141,13 +141,13 @@ int padded_len_bwd(int L2, int D, int feat) {
   return 0;
 }
 bool len_supported(int L2, int D, int feat) { return padded_len_fwd(L2, D, feat) != 0 && padded_len_bwd(L2, D, feat) != 0; }
-const fta::FwdPlan& cached_plan_fwd(int B, int H, int L1, int L2, int D, int feat = 0) {
+const fta::FwdPlan& cached_plan_fwd(int B, int H, int L1, int L2, int D, int feat = 0, bool scattered = false) {
   thread_local PlanKey key{-1, 0, 0, 0, 0, 0};
   thread_local fta::FwdPlan plan;
-  const PlanKey k{B, H, L1, L2, D, feat * 4};
+  const PlanKey k{B, H, L1, L2, D, (scattered ? 1 : 0) | (feat * 4)};
   if (!(key == k)) {
     const int lp = len_supported(L2, D, feat) ? padded_len_fwd(L2, D, feat) : 0;
-    plan = (lp != 0) ? fta::plan_fwd(B, H, L1, lp, D, L2, feat == 2) : fta::FwdPlan{};
+    plan = (lp != 0) ? fta::plan_fwd(B, H, L1, lp, D, L2, feat == 2, scattered) : fta::FwdPlan{};
     plan.L2p = lp;
     key = k;
   }
@@ -439,7 +439,7 @@ int fta_fwd_ex(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor5* v,
   p.lse = lse;
   copy4(p.qs, q->stride); copy4(p.ks, k->stride); copy4(p.vs, v->stride); copy4(p.os, o->stride);
   copy3(p.bs, bias->stride);
-  const fta::FwdPlan pl = cached_plan_fwd(B, H, L1, L2, D, opt.feat_fwd);
+  const fta::FwdPlan pl = cached_plan_fwd(B, H, L1, L2, D, opt.feat_fwd, k->stride[3] != D);
   p.B = B; p.H = H; p.L1 = L1; p.L2 = L2; p.L2p = pl.L2p;
   p.odd_bias = bias_rows_unaligned(bias) ? 1 : 0;
   p.head_inner = (H > 1 && k->stride[1] < k->stride[3]) ? 1 : 0;

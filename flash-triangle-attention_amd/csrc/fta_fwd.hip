@@ -98,13 +98,13 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int
   return pl;
 }
 
-FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, int row, bool feat) {
+FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, int row, bool feat, bool scattered) {
   // L2 here is the length the tiles cover: a multiple of 128, or of 32 or 64 where the hand-scheduled kernel or a rule below takes it
   // (padded_len_fwd tries them in steps of 32).  The hand-scheduled kernels first; then slab widths are tried in this order, the first that
   // has a built instance and a stage length that fits is taken:
   const int kwmax = (D == 32) ? 512 : 256;  // the widest that keeps the stationary bias within the register budget
   FwdPlan pl{};
-  if (!feat && plan_fwd1(B, H, L1, L2, D, row, pl)) return pl;
+  if (!feat && plan_fwd1(B, H, L1, L2, D, row, scattered, pl)) return pl;
   if (!feat && plan_fwd2(B, H, L1, L2, D, pl)) return pl;
   auto take = [&](int kw, bool wide = false) {
     if (pl.valid || kw < 128 || (kw > kwmax && !wide) || kw % 32 != 0 || L2 % kw != 0) return;

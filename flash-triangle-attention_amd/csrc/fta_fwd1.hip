@@ -6,7 +6,7 @@ namespace fta {
 
 // ---- host side ---------------------------------------------------------------------------------
 
-bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, FwdPlan& pl) {
+bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, bool scattered, FwdPlan& pl) {
   if (D != 32 || L2 % 32 != 0 || L2 < 64 || L2 == 96 || L2 > 1792) return false;
   pl = FwdPlan{};
   // rows beyond 512 keys in two slabs, beyond 1024 in four (three would leave two of the four SIMDs with one wave);
@@ -16,16 +16,15 @@ bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, FwdPlan& pl) {
   pl.S = L2 <= 512 ? 1 : L2 <= 1024 ? 2 : 4;
   if (L2 % (32 * pl.S) != 0) return false;
   pl.NKT = L2 / (32 * pl.S);
-  // eight waves per workgroup where the queries divide that way and such workgroups still fill the chip
-  // (see the kernel's comment; same-run A/B at B4 H8: 1.020 against 1.078 ms at L2 = 512, 0.183 against
-  // 0.194 at 256; four-wave workgroups in four rounds instead of two gain 4 %), else four; rows of up to
-  // 64 queries have two query blocks
-  const bool fills = (long)B * H * (L2 / 256) * ((L1 + 7) / 8) >= 256;
-  pl.QB = pl.S > 1 ? 8 / pl.S : (L2 % 256 == 0 && fills) ? 8 : L2 <= 64 ? 2 : 4;
+  // eight waves per workgroup where a query block's keys are several slabs, else four, two workgroups to a CU (see the kernel's
+  // comment); rows of up to 64 queries have two query blocks.  256 keys that do not lie next to each other in memory (heads
+  // interleaved, or a transposed view: half a line each): the eight query blocks of a row in one workgroup, where such workgroups fill the chip, so that half as
+  // many ask for a line (B2 H4, us, four / eight waves: heads interleaved in bf16 46.7 / 46.0, a training pass 179 / 177, transposed 47.9 / 47.2; contiguous
+  // 42.0 / 42.4, B4 H8 146 / 150; 512 keys, heads interleaved, 1033 / 1069)
+  const bool row_of_eight = L2 == 256 && scattered && (long)B * H * ((L1 + 7) / 8) >= 256;
+  pl.QB = pl.S > 1 ? 8 / pl.S : L2 <= 64 ? 2 : row_of_eight ? 8 : 4;
   pl.nqg = (row + 32 * pl.QB - 1) / (32 * pl.QB);
   pl.threads = 64 * pl.QB * pl.S;
-  // (stages of 256 keys, which an eight-wave workgroup has the LDS for, halve the barriers and measured
-  // the same: 1.040-1.043 against 1.044-1.047 ms at B4 H8 L512; not instantiated)
   pl.KT = (L2 <= 64 || pl.S > 1) ? 64 : 128;
   pl.smem = (size_t)4 * 2 * pl.S * pl.KT * 32 * 2;  // four slots of a K and a V tile of KT keys per slab
   if (pl.S > 1) pl.smem += pl.S == 4 ? 8 * (3072 + 512) + 1024 : 8 * (4096 + 512);  // the merge records
@@ -46,8 +45,8 @@ hipError_t launch_fwd1(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 gr
   FTA_FWD1_CASE(5, 4, 4, 1) FTA_FWD1_CASE(7, 4, 4, 1) FTA_FWD1_CASE(9, 4, 4, 1) FTA_FWD1_CASE(11, 4, 4, 1)
   FTA_FWD1_CASE(13, 4, 4, 1) FTA_FWD1_CASE(15, 4, 4, 1)
   FTA_FWD1_CASE(4, 4, 4, 1) FTA_FWD1_CASE(6, 4, 4, 1) FTA_FWD1_CASE(8, 4, 4, 1) FTA_FWD1_CASE(10, 4, 4, 1)
+  FTA_FWD1_CASE(8, 8, 4, 1)
   FTA_FWD1_CASE(12, 4, 4, 1) FTA_FWD1_CASE(14, 4, 4, 1) FTA_FWD1_CASE(16, 4, 4, 1)
-  FTA_FWD1_CASE(8, 8, 4, 1) FTA_FWD1_CASE(16, 8, 4, 1)
   return launch_fwd1_slabs(p, pl, dtype, tl, grid, block, st);
 }
 

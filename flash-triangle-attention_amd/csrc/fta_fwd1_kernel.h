@@ -28,13 +28,18 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // tuples, and an odd count moves the next row's first tile from one to the other at the end of a row, 16 instructions
 // where the tile it saves takes 64); TAIL: the row's true length L2 is shorter
 // than the 32*NKT keys the tiles cover, or than the workgroups' query blocks (keys beyond it masked, queries
-// beyond it computed on copies of the last one and not stored); W: waves (query blocks of 32) per workgroup, 4 or 8.
-// Two waves share a SIMD either way.  With W = 4 they belong to two independent workgroups, and the
-// hardware lets the older one issue first whenever both are ready, which in a kernel bound by the
-// vector ALU is nearly always: measured with a clock around every workgroup, the older workgroup of a CU
-// finishes its 128 rows after 750 us and the younger one, left with a SIMD to itself that a lone wave
-// cannot fill, after 1250.  With W = 8 the two waves of a SIMD are in one workgroup and meet at every
-// stage barrier, so neither runs ahead, and the K/V stage is copied into LDS once for eight query blocks.
+// beyond it computed on copies of the last one and not stored); W: waves (query blocks of 32) per workgroup: 4, or 2 for rows of up to 64
+// keys, and 8 with several slabs (and for some rows of 256 keys, see plan_fwd1).
+// Two waves share a SIMD either way.  With one slab they belong to independent workgroups, and the hardware lets the
+// older one issue first whenever both are ready, which in a kernel bound by the vector ALU is nearly always: measured with
+// a clock around every workgroup (B4 H8 L512), the older workgroup of a CU finished its 128 rows after 750 us and the
+// younger one, left with a SIMD to itself that a lone wave cannot fill, after 1250.  So a wave's priority falls from half row to
+// half row, in turns of two rows: the one that is ahead yields until the other has caught up, neither is ever more than two rows
+// ahead, and their barriers stay uncoupled.  Without / with it, us: B1 H4 L150 13.1 / 12.5, L200 20.4 / 18.4, L300 42.7 / 40.3, L384
+// 66.8 / 63.0, L457 in bf16 113 / 109, B2 H4 L320 88.7 / 84, B4 H8 L128 31.2 / 30.3, L384 at scale 1.3 510 / 489.  One workgroup of eight
+// waves, where the two waves of a SIMD meet at every stage barrier, gives B4 H8 L512 1037 and 1117 us (scale 1.3), B1 H4 L512 137.6; this 989,
+// 1051 and 131.4.  Four steps over the whole chunk instead: 1027, 1087, 134.1; a step a row in turns of four: 984, 1055, 131.0, but 2 % more
+// at 128 keys; four steps within a row: equal, 3 % more at 384 keys.
 // S: key slabs.  Rows beyond 512 keys do not fit one wave's bias registers: S = 2 or 4 waves of an eight-wave workgroup
 // take the keys of one query block in slabs of 32*NKT and merge their (m, l, O) through LDS, in fp32, once per row:
 // every slab finishes 16/S of the accumulator registers.  A stage then holds 64 keys of every slab.
@@ -42,9 +47,9 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // 5200 -> 4100)
 template <class T, int NKT, bool TAIL, int W, int G = 4, int S = 1>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_waves_per_eu(2, 2))) fta_fwd1_kernel(const FwdParams p) {
-  static_assert(W == 2 || W == 4 || W == 8, "one or two waves per SIMD from the same workgroup (rows of up to 64 keys: two waves)");
+  static_assert(S > 1 ? W == 8 : W == 4 || (W == 8 && NKT == 8) || (W == 2 && NKT == 2), "one or two waves per SIMD from the same workgroup");
   static_assert(S == 1 ? G == 4 || (G == 2 && NKT == 2) : G == 2, "stages of 128 keys; of 64 for such rows and for several slabs");
-  static_assert(S == 1 || ((S == 2 || S == 4) && W == 8 && NKT >= 6), "slabs: four query blocks in two, or two in four; the merge takes the first three iterations of a row");
+  static_assert(S == 1 || ((S == 2 || S == 4) && NKT >= 6), "slabs: four query blocks in two, or two in four; the merge takes the first three iterations of a row");
   constexpr int D = 32, KS = 2;
   constexpr int NCU = S * 2 * G / W;           // copies per wave and stage of K, and of V (a stage has 2*G pieces of 1 KB of each per slab)
   constexpr int KT = 32 * G;                   // keys per stage and slab
@@ -406,6 +411,14 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
       constexpr bool PUB = (tn % G == 0);         // tile t+1 opens a stage: publish it first
       floatx16& sc = s[t & 1];
       floatx16& sn = s[(t + 1) & 1];
+      if constexpr (W < 8 && t == 0) {  // (see W above)
+        if (ir & 1) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(3);
+      }
+      if constexpr (W < 8 && t == NKT / 2) {
+        if (ir & 1) __builtin_amdgcn_s_setprio(0);
+        else __builtin_amdgcn_s_setprio(2);
+      }
 
       if constexpr (PUB) {
         // everything but the copies of the stage after it has landed (copies retire in order; the last wait of
@@ -522,7 +535,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
             ph[r >> 1] = T::pack(p0, p1);
             lt = T::sum2(ph[r >> 1], lt);
           }
-          asm volatile("s_nop 1" : "+v"(acc), "+v"(ph[0]), "+v"(ph[1]), "+v"(ph[2]), "+v"(ph[3]), "+v"(ph[4]), "+v"(ph[5]),
+          asm volatile("s_nop 3" : "+v"(acc), "+v"(lt), "+v"(ph[0]), "+v"(ph[1]), "+v"(ph[2]), "+v"(ph[3]), "+v"(ph[4]), "+v"(ph[5]),
                        "+v"(ph[6]), "+v"(ph[7]));
         }
         l += lt;

@@ -248,7 +248,7 @@ hipError_t launch_bwd_feat(const BwdParams& p, const BwdPlan& pl, int D, int dty
 
 // feat: the plan is for bf16 inputs or dropout, which have a smaller set of kernel instances
 // (`row`: the true row length)
-FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, int row, bool feat);
+FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, int row, bool feat, bool scattered = false);
 
 // The kernels are gfx950 code objects: FTA_OK if the current device can run them (fta_api.hip).
 int check_device();
@@ -269,7 +269,7 @@ inline hipError_t launch_kernel(K kern, const P& p, dim3 grid, dim3 block, size_
 bool forced_general();
 hipError_t launch_fwd(FwdParams p, const FwdPlan& pl, int D, int dtype, hipStream_t st);
 // The hand-scheduled forward (fta_fwd1_kernel.h): D = 32, tiled length 64 ... 1792, no dropout.
-bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, FwdPlan& pl);
+bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, bool scattered, FwdPlan& pl);
 hipError_t launch_fwd1(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 grid, dim3 block, hipStream_t st);
 hipError_t launch_fwd1_slabs(const FwdParams& p, const FwdPlan& pl, int dtype, bool tl, dim3 grid, dim3 block, hipStream_t st);
 bool plan_fwd2(int B, int H, int L1, int L2, int D, FwdPlan& pl);

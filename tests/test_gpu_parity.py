@@ -572,3 +572,20 @@ def test_head_dim_64_forward_of_one_and_two_slabs_with_masked_key_ranges(L2, mas
         got = _run(q, k, v, b, sm, do)
         assert all(bool(torch.isfinite(got[n].float()).all()) for n in got)
         _compare(got, _oracle(q, k, v, b, sm, do), f"D64 L{L2} mask {masked} sm {sm}")
+
+
+@pytest.mark.parametrize("L1,L2", [(64, 256), (57, 256), (64, 255), (63, 500), (128, 64)])
+def test_forward_is_the_same_however_the_rows_lie_in_memory(L1, L2):
+    """Rows of 256 keys run in workgroups of four or of eight query blocks, by whether a row's keys are neighbours in memory.  A
+    wave's arithmetic is the same in both, so contiguous, head-interleaved and transposed tensors give the same bits."""
+    B, H, D = 4, 8, 32
+    print(f"case memory order L1={L1} L2={L2}", flush=True)
+    q, k, v, b, do = orc.make_inputs(B, H, L1, L2, D, seed=9, device=DEV)
+    want = _run(q, k, v, b, 1.3, do)
+    _compare(want, _oracle(q, k, v, b, 1.3, do), f"L{L1}x{L2}")
+    for order in ((0, 2, 3, 1, 4), (0, 1, 3, 2, 4)):  # heads interleaved; L1 and L2 swapped
+        back = tuple(order.index(n) for n in range(5))
+        q2, k2, v2 = (t.permute(order).contiguous().permute(back) for t in (q, k, v))
+        got = _run(q2, k2, v2, b, 1.3, do)
+        assert torch.equal(got["o"], want["o"]), order
+        _compare(got, {n: t.float() for n, t in want.items()}, f"order {order}")
