@@ -16,18 +16,22 @@ bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, bool scattered, Fwd
   pl.S = L2 <= 512 ? 1 : L2 <= 1024 ? 2 : 4;
   if (L2 % (32 * pl.S) != 0) return false;
   pl.NKT = L2 / (32 * pl.S);
-  // eight waves per workgroup where a query block's keys are several slabs, else four, two workgroups to a CU (see the kernel's
-  // comment); rows of up to 64 queries have two query blocks.  256 keys that do not lie next to each other in memory (heads
+  // four waves per workgroup, two workgroups to a CU (see the kernel's comment); eight where a query block's keys are four slabs; rows of up to
+  // 64 queries have two query blocks.  256 keys that do not lie next to each other in memory (heads
   // interleaved, or a transposed view: half a line each): the eight query blocks of a row in one workgroup, where such workgroups fill the chip, so that half as
   // many ask for a line (B2 H4, us, four / eight waves: heads interleaved in bf16 46.7 / 46.0, a training pass 179 / 177, transposed 47.9 / 47.2; contiguous
   // 42.0 / 42.4, B4 H8 146 / 150; 512 keys, heads interleaved, 1033 / 1069)
+  // Two slabs of such keys, where four query blocks to a workgroup leave no more of them empty than two: the same (us, two / four query blocks:
+  // transposed B1 H4 L640 306 / 302, B2 H8 L640 1209 / 1181, B1 H4 L768 506 / 501; L900 862 / 882, L960 944 / 954, contiguous L640 1128 / 1138).
+  const int nblk = (row + 31) / 32;
+  const bool four_blocks = scattered && L2 % 128 == 0 && nblk % 4 == 0;
   const bool row_of_eight = L2 == 256 && scattered && (long)B * H * ((L1 + 7) / 8) >= 256;
-  pl.QB = pl.S > 1 ? 8 / pl.S : L2 <= 64 ? 2 : row_of_eight ? 8 : 4;
+  pl.QB = pl.S == 2 && four_blocks ? 4 : pl.S > 1 || L2 <= 64 ? 2 : row_of_eight ? 8 : 4;
   pl.nqg = (row + 32 * pl.QB - 1) / (32 * pl.QB);
   pl.threads = 64 * pl.QB * pl.S;
   pl.KT = (L2 <= 64 || pl.S > 1) ? 64 : 128;
   pl.smem = (size_t)4 * 2 * pl.S * pl.KT * 32 * 2;  // four slots of a K and a V tile of KT keys per slab
-  if (pl.S > 1) pl.smem += pl.S == 4 ? 8 * (3072 + 512) + 1024 : 8 * (4096 + 512);  // the merge records
+  if (pl.S > 1) pl.smem += pl.S == 4 ? 8 * (3072 + 512) + 1024 : pl.S * pl.QB * (2048 + 512);  // the merge records
   pl.alias_scratch = 0;
   // two waves per SIMD: one, two or four workgroups per CU.  At least a row per 64 keys in a chunk: a workgroup's set-up
   // loads one bias row per query, so short rows can be spread thinner (B1 H4 L64: 14.9 us with 8 rows, 5 with 1)

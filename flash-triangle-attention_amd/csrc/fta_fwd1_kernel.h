@@ -40,14 +40,18 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // waves, where the two waves of a SIMD meet at every stage barrier, gives B4 H8 L512 1037 and 1117 us (scale 1.3), B1 H4 L512 137.6; this 989,
 // 1051 and 131.4.  Four steps over the whole chunk instead: 1027, 1087, 134.1; a step a row in turns of four: 984, 1055, 131.0, but 2 % more
 // at 128 keys; four steps within a row: equal, 3 % more at 384 keys.
-// S: key slabs.  Rows beyond 512 keys do not fit one wave's bias registers: S = 2 or 4 waves of an eight-wave workgroup
+// S: key slabs.  Rows beyond 512 keys do not fit one wave's bias registers: S = 2 or 4 waves of a workgroup
 // take the keys of one query block in slabs of 32*NKT and merge their (m, l, O) through LDS, in fp32, once per row:
-// every slab finishes 16/S of the accumulator registers.  A stage then holds 64 keys of every slab.
+// every slab finishes 16/S of the accumulator registers.  A stage then holds 64 keys of every slab.  Two slabs: workgroups of two query
+// blocks, two to a CU, whose records of the merge leave out what a wave keeps (10 KB; with them whole a second workgroup does not fit LDS).
+// Barriers of two workgroups do not couple, and a row's last query group is at most one block short; K and V are copied into LDS
+// once for two query blocks instead of four.  B1 H4, us, one workgroup of four query blocks / two of two: L540 219 / 196, L660 in bf16 368 /
+// 330, L701 in bf16 409 / 382, L768 at scale 1.3 523 / 489, L900 in bf16 813 / 762, L1000 996 / 980, B2 H4 L1024 2059 / 1988 (transposed: see plan_fwd1).
 // (against the general kernel, rocprofv3, middle half of 60 launches: B1 H4 L701 bf16 656 -> 466 us, B1 H4 L1536 fp16
 // 5200 -> 4100)
 template <class T, int NKT, bool TAIL, int W, int G = 4, int S = 1>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdgpu_waves_per_eu(2, 2))) fta_fwd1_kernel(const FwdParams p) {
-  static_assert(S > 1 ? W == 8 : W == 4 || (W == 8 && NKT == 8) || (W == 2 && NKT == 2), "one or two waves per SIMD from the same workgroup");
+  static_assert(S == 4 ? W == 8 : W == 4 || (S == 2 && W == 8) || (S == 1 && W == 8 && NKT == 8) || (S == 1 && W == 2 && NKT == 2), "one or two waves per SIMD from the same workgroup");
   static_assert(S == 1 ? G == 4 || (G == 2 && NKT == 2) : G == 2, "stages of 128 keys; of 64 for such rows and for several slabs");
   static_assert(S == 1 || ((S == 2 || S == 4) && NKT >= 6), "slabs: four query blocks in two, or two in four; the merge takes the first three iterations of a row");
   constexpr int D = 32, KS = 2;
@@ -104,15 +108,19 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
 
   // ---- stage copies: a stage is 32*G K rows and 32*G V rows of 64 bytes, 1 KB per wave instruction,
   // NCU K and NCU V copies per wave; copy u of wave w carries the 16-byte pieces (w + W*u)*64 .. +63.
-  uint32_t goffk[NCU], goffv[NCU];
+  // (S = 2: a copy covers rows of one slab, and a wave's next one the same rows of the other: one offset, and the slabs' distance in
+  // the base.  With four slabs, where registers are left, that is 2 % slower)
+  constexpr int NGO = S == 2 ? 1 : NCU;
+  uint32_t goffk[NGO], goffv[NGO];
   constexpr bool CLAMP = TAIL || NKT % G != 0;
-  [[maybe_unused]] uint32_t goffk_t[NCU], goffv_t[NCU];  // CLAMP: the row's last stage (rows beyond the last key are copies of it); S > 1: the last key's row
+  [[maybe_unused]] uint32_t goffk_t[NGO], goffv_t[NGO];  // CLAMP: the row's last stage (rows beyond the last key are copies of it); S = 4: the last key's row
+  [[maybe_unused]] const uint32_t ctail = (uint32_t)swz_slot<D>(lane >> 2, lane & 3) * 16u;  // S = 2: this lane's piece of a row, the same in every copy (16 rows each)
 #pragma unroll
-  for (int u = 0; u < NCU; ++u) {
+  for (int u = 0; u < NGO; ++u) {
     const int pidx = (wave + W * u) * 64 + lane, prow = pidx >> 2, chunkk = swz_slot<D>(prow, pidx & 3), row = (prow / KT) * KW + prow % KT;
     goffk[u] = (uint32_t)(((int64_t)row * p.ks[3] + chunkk * 8) * 2);
     goffv[u] = (uint32_t)(((int64_t)row * p.vs[3] + chunkk * 8) * 2);
-    if constexpr (CLAMP) {
+    if constexpr (CLAMP && S != 2) {
       const int grow = S > 1 ? last : min((NST - 1) * KT + row, last) - (NST - 1) * KT;
       goffk_t[u] = (uint32_t)(((int64_t)grow * p.ks[3] + chunkk * 8) * 2);
       goffv_t[u] = (uint32_t)(((int64_t)grow * p.vs[3] + chunkk * 8) * 2);
@@ -122,6 +130,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
   const uint32_t wofs = (uint32_t)wave * 1024u;
   int64_t rstep_k = hold_scalar(p.ks[2] * 2), rstep_v = hold_scalar(p.vs[2] * 2);            // bytes from one row to the next
   int64_t sstep_k = hold_scalar(p.ks[3] * 2 * KT), sstep_v = hold_scalar(p.vs[3] * 2 * KT);  // from one stage to the next
+  [[maybe_unused]] const int64_t ustep_k = (int64_t)KW * p.ks[3] * 2, ustep_v = (int64_t)KW * p.vs[3] * 2;
   // fill cursor: the stage the copies currently go to (row pointer, LDS slot); it runs ahead of the row
   // being computed and stops advancing at the chunk's last row (whose data is then copied again into
   // slots nothing reads any more: the loop stays free of "is there a next stage" branches)
@@ -148,6 +157,13 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
     fill_lds = lds0 + wofs + (uint32_t)fill_slot * SLOT_B;
     fill_slot = (fill_slot + 1) & (R - 1);
   };
+  // S = 2: the smaller of `off` + `step` and this lane's piece of the last key's row (formed at every use: the sums would be kept over the rows)
+  [[maybe_unused]] uint32_t lastk = (uint32_t)(last * p.ks[3] * 2), lastv = (uint32_t)(last * p.vs[3] * 2);
+  auto clamped = [&](uint32_t off, uint32_t step, uint32_t lastrow) {
+    uint32_t a, b;
+    asm volatile("v_add_u32 %0, %2, %3\n\tv_add_u32 %1, %4, %5\n\tv_min_u32 %0, %0, %1" : "=&v"(a), "=&v"(b) : "s"(step), "v"(off), "s"(lastrow), "v"(ctail));
+    return a;
+  };
   // copy c (first the K copies, then the V copies) of the stage begun last, which is stage number w of
   // its row
   auto fill_copy = [&](auto wc, auto cc) {
@@ -157,8 +173,14 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
     if constexpr (S > 1 && (TAIL ? w >= NST - S : w * G + G > NKT)) {
       // (fewer than 64*S keys are missing, so the last slab ends in one of its last S stages; a stage that is not full
       // reaches beyond the last slab)
-      if constexpr (c < nk) dma16s_at<(uint32_t)c * W * 1024u>(min(goffk[c] + (uint32_t)(w * sstep_k), goffk_t[c]), kfill, fill_lds);
-      else dma16s_at<TILE_B + (uint32_t)(c - nk) * W * 1024u>(min(goffv[c - nk] + (uint32_t)(w * sstep_v), goffv_t[c - nk]), vfill, fill_lds);
+      if constexpr (S == 4) {
+        if constexpr (c < nk) dma16s_at<(uint32_t)c * W * 1024u>(min(goffk[c] + (uint32_t)(w * sstep_k), goffk_t[c]), kfill, fill_lds);
+        else dma16s_at<TILE_B + (uint32_t)(c - nk) * W * 1024u>(min(goffv[c - nk] + (uint32_t)(w * sstep_v), goffv_t[c - nk]), vfill, fill_lds);
+      } else if constexpr (c < nk) dma16s_at<(uint32_t)c * W * 1024u>(clamped(goffk[0], (uint32_t)(w * sstep_k + c * ustep_k), lastk), kfill, fill_lds);
+      else dma16s_at<TILE_B + (uint32_t)(c - nk) * W * 1024u>(clamped(goffv[0], (uint32_t)(w * sstep_v + (c - nk) * ustep_v), lastv), vfill, fill_lds);
+    } else if constexpr (S == 2) {
+      if constexpr (c < nk) dma16s_at<(uint32_t)c * W * 1024u>(goffk[0], kst + c * ustep_k, fill_lds);
+      else dma16s_at<TILE_B + (uint32_t)(c - nk) * W * 1024u>(goffv[0], vst + (c - nk) * ustep_v, fill_lds);
     } else if constexpr (c < nk) dma16s_at<(uint32_t)c * W * 1024u>(TL ? goffk_t[c] : goffk[c], kst, fill_lds);
     else dma16s_at<TILE_B + (uint32_t)(c - nk) * W * 1024u>(TL ? goffv_t[c - nk] : goffv[c - nk], vst, fill_lds);
   };
@@ -302,13 +324,12 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
     lcur += p.L2;
   };
 
-  // S > 1: the finished row's accumulator changes waves in two steps.  Record of a wave: its (l, m) at 4 KB (S = 2) or
-  // 3 KB (S = 4), in front of it the accumulator in groups of four registers, 1 KB each; with four slabs LDS has no room
-  // for the wave's own group, which stays in registers, and group g of slab s is in place (g - s - 1) % 4 (its own goes
-  // to a place that nothing reads).
-  constexpr uint32_t REC_B = (S == 4 ? 3072u : 4096u) + 512u;
+  // S > 1: the finished row's accumulator changes waves in two steps.  A wave's record holds the accumulator registers that
+  // others finish, in groups of four, 1 KB each, and its (l, m) behind them; its own stay in registers.  S = 2: slab s finishes
+  // registers 8*s .. +7.  S = 4: group s; group g of slab s is in place (g - s - 1) % 4 (its own goes to a place that nothing reads).
+  constexpr uint32_t REC_B = (S == 4 ? 3072u : 2048u) + 512u;
   const uint32_t rec0 = lds0 + R * SLOT_B;
-  [[maybe_unused]] float keep[4];
+  [[maybe_unused]] float keep[16 / (S > 1 ? S : 4)];
   [[maybe_unused]] uint32_t ostride = (uint32_t)p.os[3] * 2u;
   if constexpr (S > 1) asm volatile("" : "+s"(ostride));
   auto lane_now = []() {  // (see store_lse)
@@ -320,10 +341,23 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
     if constexpr (S > 1) {
       const uint32_t ln = lane_now(), rec = rec0 + (uint32_t)wave * REC_B;
       const float lt = sum_both_halves(l_done), m2 = m_done * kLog2e;
+      auto half = [&](auto own) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        uint32_t at = rec + (uint32_t)g * 1024u;
-        if constexpr (S == 4) at = (g == slab) ? rec0 + W * REC_B : rec + (uint32_t)((g - slab - 1) & 3) * 1024u;
+        for (int g = 0; g < 2; ++g) {
+          constexpr int o = decltype(own)::value;
+          const floatx4 v = {acc[8 - o + 4 * g], acc[9 - o + 4 * g], acc[10 - o + 4 * g], acc[11 - o + 4 * g]};
+          asm volatile("ds_write_b128 %0, %1 offset:%2" : : "v"(rec + ln * 16u), "v"(v), "n"(g * 1024) : "memory");
+#pragma unroll
+          for (int e = 0; e < 4; ++e) keep[4 * g + e] = acc[o + 4 * g + e];
+        }
+      };
+      if constexpr (S == 2) {
+        if (slab == 0) half(std::integral_constant<int, 0>{});
+        else half(std::integral_constant<int, 8>{});
+      }
+#pragma unroll
+      for (int g = 0; g < (S == 4 ? 4 : 0); ++g) {
+        const uint32_t at = (g == slab) ? rec0 + W * REC_B : rec + (uint32_t)((g - slab - 1) & 3) * 1024u;
         const floatx4 v = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
         asm volatile("ds_write_b128 %0, %1" : : "v"(at + ln * 16u), "v"(v) : "memory");
       }
@@ -361,14 +395,11 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
       const float inv = __builtin_amdgcn_rcpf(tot);
       float o[16 / S];
       if constexpr (S == 2) {
+        const float ck = slab ? c[1] : c[0], cx = slab ? c[0] : c[1];
+        floatx4 a[2];
+        asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:1024\n\ts_waitcnt lgkmcnt(0)" : "=&v"(a[0]), "=&v"(a[1]) : "v"(team + (uint32_t)(slab ^ 1) * REC_B + ln * 16u) : "memory");
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          floatx4 a, b2;
-          const uint32_t at = team + (uint32_t)(2 * slab + g) * 1024u + ln * 16u;
-          asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:%3\n\ts_waitcnt lgkmcnt(0)" : "=&v"(a), "=&v"(b2) : "v"(at), "n"(REC_B) : "memory");
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o[4 * g + e] = (a[e] * c[0] + b2[e] * c[1]) * inv;
-        }
+        for (int e = 0; e < 8; ++e) o[e] = __builtin_fmaf(keep[e], ck, a[e / 4][e % 4] * cx) * inv;  // (the same rounding in every instance)
       } else {
         const float ck = (slab & 2) ? ((slab & 1) ? c[S - 1] : c[S - 2]) : ((slab & 1) ? c[S - 3] : c[S - 4]);
 #pragma unroll

@@ -574,9 +574,9 @@ def test_head_dim_64_forward_of_one_and_two_slabs_with_masked_key_ranges(L2, mas
         _compare(got, _oracle(q, k, v, b, sm, do), f"D64 L{L2} mask {masked} sm {sm}")
 
 
-@pytest.mark.parametrize("L1,L2", [(64, 256), (57, 256), (64, 255), (63, 500), (128, 64)])
+@pytest.mark.parametrize("L1,L2", [(64, 256), (57, 256), (64, 255), (63, 500), (128, 64), (9, 640), (5, 701), (5, 1024), (4, 1000)])
 def test_forward_is_the_same_however_the_rows_lie_in_memory(L1, L2):
-    """Rows of 256 keys run in workgroups of four or of eight query blocks, by whether a row's keys are neighbours in memory.  A
+    """Rows of 256 keys run in workgroups of four or of eight query blocks, some rows of 513 to 1024 in two or four, by whether a row's keys are neighbours in memory.  A
     wave's arithmetic is the same in both, so contiguous, head-interleaved and transposed tensors give the same bits."""
     B, H, D = 4, 8, 32
     print(f"case memory order L1={L1} L2={L2}", flush=True)
