@@ -54,10 +54,10 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
     }
     const int wide = L2 % 1024 == 0 ? 1024 : L2 % 768 == 0 ? 768 : 0;
     if (wide != 0) {
-      const Ring r = dkdv_ring(32, wide / 128, 64, 4);
+      const Ring r = dkdv_ring(32, wide / 128, 64, 4, 8);
       sj = 4; kb = 2;
       pl.nranges2 = 0; pl.NJT = wide / 128; pl.JR = wide; pl.nlaunch2 = L2 / wide;
-      pl.ring2 = r.r; pl.nb2 = r.nb; pl.smem2 = dkdv_smem(32, pl.NJT, 64, 4);
+      pl.ring2 = r.r; pl.nb2 = r.nb; pl.smem2 = dkdv_smem(32, pl.NJT, 64, 4, 8);
     }
     pl.SJ = sj; pl.KB = kb;
     pl.threads = pl.threads2 = 512;
@@ -82,19 +82,20 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
     if (L2 % c == 0) { kr = c; break; }
   pl.KR = kr;
   pl.nlaunch = L2 / kr;
-  // Dropout at D = 32, key ranges of 384 keys: four slabs of 96 keys instead of three of 128, so that eight waves and
-  // not six share a CU's four SIMDs, and the query (key) blocks that hold nothing of the row have no workgroup.
+  // Dropout at D = 32, key ranges of 384 keys: four slabs of 96 keys instead of three of 128, so that the four SIMDs of a CU have
+  // as many waves each, and the query (key) blocks that hold nothing of the row have no workgroup.
   const bool three = (feat == 2 && D == 32 && kr == 384);
   const int nblk = (feat == 2) ? (row + 31) / 32 : nqb;
   pl.NKT = three ? 3 : 4;
   pl.SK = kr / (32 * pl.NKT);
-  int qb = 8 / pl.SK;
+  const bool four = (feat == 2 && D == 32 && pl.SK == 4);  // workgroups of four waves, two to a CU (see fta_bwd_feat.hip)
+  int qb = (four ? 4 : 8) / pl.SK;
   if (qb < 1) qb = 1;
   while (qb > 1 && nqb % qb != 0) --qb;
   pl.QB = qb;
   pl.nqg = (nblk + qb - 1) / qb;
   pl.threads = 64 * pl.SK * pl.QB;
-  const int G1 = (D == 32 && !three) ? 2 : 1;
+  const int G1 = (D == 32 && !four) ? 2 : 1;
   const int stage_rows = pl.SK * G1 * 32;
   const size_t slot1 = (size_t)2 * stage_rows * D * 2;
   const int steps1 = pl.NKT / G1;
@@ -103,9 +104,9 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   pl.ring = 0;
   for (int r = 4; r >= 3; --r) {
     const int nb = (r + steps1 - 1) / steps1;  // rows whose operand tiles can be in flight at once
-    if (r * slot1 + nb * qtile1 + part1 <= lds_max) { pl.ring = r; pl.nb = nb; pl.smem = r * slot1 + nb * qtile1 + part1; break; }
+    if (r * slot1 + nb * qtile1 + part1 <= lds_max / (four ? 2 : 1)) { pl.ring = r; pl.nb = nb; pl.smem = r * slot1 + nb * qtile1 + part1; break; }
   }
-  pl.nchunks = balanced_chunks((long)B * H * pl.nqg, L1, 256, least_rows(L2));
+  pl.nchunks = balanced_chunks((long)B * H * pl.nqg, L1, four ? 512 : 256, least_rows(L2));
   pl.rows_per_chunk = (L1 + pl.nchunks - 1) / pl.nchunks;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   // ---- dK/dV kernel: query slabs of at most 256 (D=32) / 128 (D=64) queries per wave (register
@@ -116,7 +117,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   int jw = 0;
   for (int c = jwmax; c >= 128; c -= 128)
     if (L2 % c == 0) { jw = c; break; }
-  // (dropout, lengths that three slabs of 128 queries would cut: two slabs of 192, for eight waves instead of six)
+  // (dropout, lengths that three slabs of 128 queries would cut: two slabs of 192, as many waves for every SIMD)
   const bool two192 = (feat == 2 && D == 32 && jw == 128 && L2 % 384 == 0);
   if (two192) jw = 192;
   pl.NJT = jw / 32;
@@ -125,7 +126,8 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   bool ok2 = false;
   for (int sj = (nslab < sjmax ? nslab : sjmax); sj >= 1 && !ok2; --sj) {
     if (nslab % sj != 0) continue;
-    int kb = 8 / sj;
+    const bool four2 = (feat == 2 && D == 32 && sj == 2 && jw >= 192);
+    int kb = (four2 ? 4 : 8) / sj;
     if (kb < 1) continue;
     while (kb > 1 && nqb % kb != 0) --kb;
     for (int jt = 64; jt >= 32 && !ok2; jt /= 2) {
@@ -137,7 +139,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
       const int steps2 = (jw / 32) / (jt / 32);
       for (int r = 4; r >= 3 && !ok2; --r) {
         const int nb = (r + steps2 - 1) / steps2;
-        if (r * slot2 + nb * ktile2 + scratch2 > lds_max) continue;
+        if (r * slot2 + nb * ktile2 + scratch2 > lds_max / (four2 ? 2 : 1)) continue;
         pl.SJ = sj; pl.KB = kb; pl.nkg = (nblk + kb - 1) / kb; pl.threads2 = 64 * sj * kb; pl.JT = jt;
         pl.ring2 = r; pl.nb2 = nb; pl.smem2 = r * slot2 + nb * ktile2 + scratch2;
         pl.JR = sj * jw; pl.nlaunch2 = L2 / pl.JR;
@@ -145,7 +147,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
       }
     }
   }
-  pl.nchunks2 = balanced_chunks((long)B * H * (ok2 ? pl.nkg : 1), L1, 256, least_rows(L2));
+  pl.nchunks2 = balanced_chunks((long)B * H * (ok2 ? pl.nkg : 1), L1, feat == 2 && D == 32 && pl.threads2 == 256 ? 512 : 256, least_rows(L2));
   pl.rows_per_chunk2 = (L1 + pl.nchunks2 - 1) / pl.nchunks2;
   pl.nchunks2 = (L1 + pl.rows_per_chunk2 - 1) / pl.rows_per_chunk2;
 

@@ -9,6 +9,12 @@
 // lane that made it, 145 with two slabs of 192 and the bytes of a key group transposed once per tile.  With the geometry
 // fixed at compile time where eight waves share the row: training passes of 386 to 325 us there (dQ/dBias 118), 350 to 299
 // at B2 H4 L256 and 2.41 to 2.18 ms at B1 H8 L512 (dK/dV alone).
+//
+// Rows of 257 to 512 keys run in workgroups of four waves (one query block in four slabs, or two key blocks in two), two to a CU, whose
+// priorities change in turns (see fta_fwd1_kernel): one's products and waits run beside the other's vector part, where eight waves of one
+// workgroup meet at every stage, and a row's last group is at most one block short.  K and V, or Q and dO, are copied into LDS twice
+// as often for it.  Training steps at B1 H4, us, before and after: L270 284 / 242, L300 in bf16 318 / 274, L330 372 / 337, L384 436 / 402, L400 787 / 738,
+// L512 in bf16 1073 / 1044, B4 H8 L300 2262 / 2060; without the turns L300 302, L384 443, L512 1107.
 #include "fta_bwd_kernels.h"
 
 namespace fta {
@@ -56,8 +62,10 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
       e = hipErrorInvalidConfiguration;
       if (pl.NKT == 3) {  // key ranges of 384 keys with dropout: fixed geometry
         if constexpr (DROP)
-          if (D == 32 && pl.threads == 512 && pl.SK == 4 && pl.ring == dq_ring(32, 3, 1, 4).r && pl.nb == dq_ring(32, 3, 1, 4).nb)
-            e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 3, 4>, p, grid, block, pl.smem, st);
+          if (D == 32 && pl.threads == 256 && pl.SK == 4 && pl.ring == dq_ring(32, 3, 1, 4, 4).r && pl.nb == dq_ring(32, 3, 1, 4, 4).nb)
+            e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 3, 4, 4>, p, grid, block, pl.smem, st);
+      } else if (DROP && D == 32 && pl.SK == 4) {
+        if constexpr (DROP) e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 4, 0, 4>, p, grid, block, pl.smem, st);
       } else if (D == 32) {
         e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2>, p, grid, block, pl.smem, st);
       } else {
@@ -91,11 +99,11 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
       // fixed geometry: 384, 512, 768 and 1024 queries to a launch.  (Rows of up to 256 queries at D = 32 run the one-kernel
       // backward; <8, 64, 1> and <4, 64> are theirs where fta_debug_select_kernels asks for the general kernels)
       if constexpr (DROP) {
-#define FTA_DKDV_FIX_CASE(NN, SS)                                                                                        \
-  if (D == 32 && pl.threads2 == 512 && pl.NJT == NN && pl.JT == 64 && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, 64, SS).r &&  \
-      pl.nb2 == dkdv_ring(32, NN, 64, SS).nb)                                                                            \
-    e = launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, NN, 64, SS>, p, grid, block, pl.smem2, st);
-        FTA_DKDV_FIX_CASE(6, 2) FTA_DKDV_FIX_CASE(8, 1) FTA_DKDV_FIX_CASE(8, 2) FTA_DKDV_FIX_CASE(6, 4) FTA_DKDV_FIX_CASE(8, 4)
+#define FTA_DKDV_FIX_CASE(NN, SS, WW)                                                                                            \
+  if (D == 32 && pl.threads2 == 64 * WW && pl.NJT == NN && pl.JT == 64 && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, 64, SS, WW).r && \
+      pl.nb2 == dkdv_ring(32, NN, 64, SS, WW).nb)                                                                                \
+    e = launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, NN, 64, SS, WW>, p, grid, block, pl.smem2, st);
+        FTA_DKDV_FIX_CASE(6, 2, 4) FTA_DKDV_FIX_CASE(8, 1, 8) FTA_DKDV_FIX_CASE(8, 2, 4) FTA_DKDV_FIX_CASE(6, 4, 8) FTA_DKDV_FIX_CASE(8, 4, 8)
 #undef FTA_DKDV_FIX_CASE
       }
       if constexpr (!DROP) { FTA_DKDV_FEAT_CASE(32, 8, 64) }

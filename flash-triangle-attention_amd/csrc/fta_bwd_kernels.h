@@ -73,10 +73,10 @@ __global__ void __launch_bounds__(256) fta_bwd_delta_kernel(const BwdParams p) {
 // ------------------------------------------------------------------------------------------------
 // 1. dQ + dBias partials
 // ------------------------------------------------------------------------------------------------
-template <class T, bool DROP, int D, int G1, int NKT = 4, int SKC = 0>
-__global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
+template <class T, bool DROP, int D, int G1, int NKT = 4, int SKC = 0, int NW = 8>
+__global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams p) {
   // T: element type.
-  // SKC: the number of slabs where it is known at compile time (eight waves): the geometry is then constant, every
+  // SKC: the number of slabs where it is known at compile time (NW waves): the geometry is then constant, every
   // wave issues the same number of copies per stage, and their offsets are formed from two registers.  With the geometry
   // in kernel arguments a third of the instructions per tile moved or made scalars (slabs of 96 keys, B1 H4 L300 with
   // dropout: 162 against 118 us).  Slabs of 128 keys have no registers for it: 70 spilled, 2.41 against 2.51 ms a training
@@ -92,8 +92,8 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = FIX ? 8 : blockDim.x >> 6;
-  const int SK = FIX ? SKC : p.SK, QB = FIX ? 8 / (FIX ? SKC : 1) : p.QB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = FIX ? NW : blockDim.x >> 6;
+  const int SK = FIX ? SKC : p.SK, QB = FIX ? NW / (FIX ? SKC : 1) : p.QB;
   const int slab = wave % SK, qb = wave / SK;
   const int hh = lane >> 5, l32 = lane & 31;
 
@@ -107,10 +107,10 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
   const int key0 = p.kr0 + slab * (NKT * 32);
   const int stage_rows = SK * G1 * 32;       // K (and V) rows per stage: G1 tiles for every slab
   const int buf_halfs = 2 * stage_rows * D;  // one ring slot: K tile then V tile
-  const int R = FIX ? dq_ring(D, NKT, G1, SKC).r : p.ring;  // ring slots; R - 2 stages are in flight beyond the next one
+  const int R = FIX ? dq_ring(D, NKT, G1, SKC, NW).r : p.ring;  // ring slots; R - 2 stages are in flight beyond the next one
   const int ahead = R - 2;
   const int QR = QB * 32;                    // query rows of the workgroup
-  const int NB = FIX ? dq_ring(D, NKT, G1, SKC).nb : p.nb;  // row-operand buffers (rows whose Q/dO tiles are in flight)
+  const int NB = FIX ? dq_ring(D, NKT, G1, SKC, NW).nb : p.nb;  // row-operand buffers (rows whose Q/dO tiles are in flight)
   half_t* qtiles = smem + R * buf_halfs;     // [NB][Q tile | dO tile], QR x D each
   // cross-slab dQ partials: fp32 for D=32; fp16 for D=64, where fp32 would not fit in LDS
   typedef typename std::conditional<D == 32, float, half_t>::type part_t;
@@ -181,8 +181,8 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
       kcur += p.ks[2]; vcur += p.vs[2]; qcur += p.qs[2]; docur += p.dos[2];
     }
   };
-  // FIX: pieces of 16 rows (one copy each), dealt to the eight waves; the cursors stand at the start of the row
-  constexpr int PK = FIX ? SKC * G1 * 2 / 8 : 0, PQ = FIX ? 32 / (FIX ? SKC : 1) / 8 : 0;  // per wave: K (and V) pieces of a stage; Q and dO pieces of a row
+  // FIX: pieces of 16 rows (one copy each), dealt to the waves; the cursors stand at the start of the row
+  constexpr int PK = FIX ? SKC * G1 * 2 / NW : 0, PQ = FIX ? 4 / (FIX ? SKC : 1) : 0;  // per wave: K (and V) pieces of a stage; Q and dO pieces of a row
   const uint32_t crow = (uint32_t)lane >> 2, ccol = (uint32_t)swz_slot<D>(lane >> 2, lane & 3) * 16u;
   auto piece = [&](const half_t* row, uint32_t stride2, int first, uint32_t dst) {
     uint32_t cr = crow;
@@ -194,7 +194,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
     const uint32_t dst = lds0 + (uint32_t)(slot * buf_halfs) * 2u;
 #pragma unroll
     for (int u = 0; u < PK; ++u) {
-      const int tr = (wave + 8 * u) * 16, first = p.kr0 + tr / (G1 * 32) * (NKT * 32) + t * (G1 * 32) + tr % (G1 * 32);
+      const int tr = (wave + NW * u) * 16, first = p.kr0 + tr / (G1 * 32) * (NKT * 32) + t * (G1 * 32) + tr % (G1 * 32);
       piece(kcur, (uint32_t)(2 * p.ks[3]), first, dst + (uint32_t)tr * (D * 2));
       piece(vcur, (uint32_t)(2 * p.vs[3]), first, dst + (uint32_t)(stage_rows + tr) * (D * 2));
     }
@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
       const uint32_t qd = ldsq + (uint32_t)((cur_ir % NB) * 2 * QR * D) * 2u;
 #pragma unroll
       for (int u = 0; u < PQ; ++u) {
-        const int tr = (wave + 8 * u) * 16;  // of the Q rows and then the dO rows
+        const int tr = (wave + NW * u) * 16;  // of the Q rows and then the dO rows
         const bool isq = tr < QR;
         const int w = isq ? tr : tr - QR;
         piece(isq ? qcur : docur, (uint32_t)(2 * (isq ? p.qs[3] : p.dos[3])), qg * QR + w, qd + (uint32_t)tr * (D * 2));
@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
   };
 
   if constexpr (FIX) {
-    static_for<0, dq_ring(D, NKT, G1, SKC).r - 1>([&](auto sc) {
+    static_for<0, dq_ring(D, NKT, G1, SKC, NW).r - 1>([&](auto sc) {
       if (decltype(sc)::value < nstage) stage_fix(std::integral_constant<int, decltype(sc)::value % STEPS>{}, decltype(sc)::value);
     });
   } else {
@@ -270,6 +270,14 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
 
     static_for<0, STEPS>([&](auto tc) {
       constexpr int t = decltype(tc)::value;
+      if constexpr (NW == 4 && t == 0) {  // (turns between the workgroups that share a SIMD, as in fta_fwd1_kernel)
+        if (ir & 1) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(3);
+      }
+      if constexpr (NW == 4 && t == (STEPS + 1) / 2) {
+        if (ir & 1) __builtin_amdgcn_s_setprio(0);
+        else __builtin_amdgcn_s_setprio(2);
+      }
       const int sidx = ir * STEPS + t;
       const half_t* cK = smem + cur * buf_halfs;
       const half_t* cV = cK + stage_rows * D;
@@ -329,7 +337,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
       const int nxt = sidx + 1 + ahead;
       cur = (cur + 1 == R) ? 0 : cur + 1;
       if constexpr (FIX) {
-        constexpr int AHEAD = dq_ring(D, NKT, G1, SKC).r - 2;
+        constexpr int AHEAD = dq_ring(D, NKT, G1, SKC, NW).r - 2;
         if (nxt < nstage) {
           stage_fix(std::integral_constant<int, (t + 1 + AHEAD) % STEPS>{}, fill);
           fill = (fill + 1 == R) ? 0 : fill + 1;
@@ -423,9 +431,9 @@ __global__ void __launch_bounds__(512) fta_bwd_dq_kernel(const BwdParams p) {
 // ------------------------------------------------------------------------------------------------
 // 2. dK + dV
 // ------------------------------------------------------------------------------------------------
-// T: element type.  SJC: the number of query slabs where it is known at compile time, as in the dQ kernel.
-template <class T, bool DROP, int D, int NJT, int JT, int SJC = 0>
-__global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
+// T: element type.  SJC: the number of query slabs where it is known at compile time (NW waves), as in the dQ kernel.
+template <class T, bool DROP, int D, int NJT, int JT, int SJC = 0, int NW = 8>
+__global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParams p) {
   constexpr bool FIX = (SJC != 0);
   static_assert(!FIX || (D == 32 && JT == 64), "fixed geometry");
   constexpr int G = JT / 32;                // 32-query tiles per stage (JT queries per slab and stage)
@@ -438,8 +446,8 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];
   half_t* smem = reinterpret_cast<half_t*>(smem_raw);
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = FIX ? 8 : blockDim.x >> 6;
-  const int SJ = FIX ? SJC : p.SJ, KB = FIX ? 8 / (FIX ? SJC : 1) : p.KB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = FIX ? NW : blockDim.x >> 6;
+  const int SJ = FIX ? SJC : p.SJ, KB = FIX ? NW / (FIX ? SJC : 1) : p.KB;
   const int jslab = wave % SJ, kb = wave / SJ;
   const int hh = lane >> 5, l32 = lane & 31;
 
@@ -453,10 +461,10 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   const int stage_rows = SJ * JT;
   // one ring slot: Q tile, dO tile (halfs), then lse and delta of the same rows (floats)
   const int slot_halfs = 2 * stage_rows * D + 4 * stage_rows;
-  const int R = FIX ? dkdv_ring(D, NJT, JT, SJC).r : p.ring2;
+  const int R = FIX ? dkdv_ring(D, NJT, JT, SJC, NW).r : p.ring2;
   const int ahead = R - 2;
   const int KR2 = KB * 32;                   // key rows of the workgroup
-  const int NB = FIX ? dkdv_ring(D, NJT, JT, SJC).nb : p.nb2;                      // row-operand buffers (rows whose K/V tiles are in flight)
+  const int NB = FIX ? dkdv_ring(D, NJT, JT, SJC, NW).nb : p.nb2;                      // row-operand buffers (rows whose K/V tiles are in flight)
   half_t* ktiles = smem + R * slot_halfs;    // [NB][K tile | V tile], KR2 x D each
   typedef typename std::conditional<dkdv_share_bytes(NJT, SJC) == 4, float, half_t>::type Share;
   Share* scratch = reinterpret_cast<Share*>(ktiles + NB * 2 * KR2 * D);  // cross-slab dK/dV partials, in fp16 where they would not fit in LDS
@@ -542,8 +550,8 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
       acur += 2 * p.L2p;
     }
   };
-  // FIX: pieces of 16 rows (one copy each), dealt to the eight waves; the cursors stand at the start of the row
-  constexpr int PQ = FIX ? SJC : 0, PK = FIX ? 4 / (FIX ? SJC : 1) : 0;  // per wave: Q and dO pieces of a stage; K and V pieces of a row
+  // FIX: pieces of 16 rows (one copy each), dealt to the waves; the cursors stand at the start of the row
+  constexpr int PQ = FIX ? SJC * 8 / NW : 0, PK = FIX ? 4 / (FIX ? SJC : 1) : 0;  // per wave: Q and dO pieces of a stage; K and V pieces of a row
   const uint32_t crow = (uint32_t)lane >> 2, ccol = (uint32_t)swz_slot<D>(lane >> 2, lane & 3) * 16u;
   auto piece = [&](const half_t* row, uint32_t stride2, int first, uint32_t dst) {
     uint32_t cr = crow;
@@ -557,14 +565,14 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
       const uint32_t kd = ldsk + (uint32_t)((cur_ir % NB) * 2 * KR2 * D) * 2u;
 #pragma unroll
       for (int u = 0; u < PK; ++u) {
-        const int tr = (wave + 8 * u) * 16;  // of the K rows and then the V rows
+        const int tr = (wave + NW * u) * 16;  // of the K rows and then the V rows
         const bool isk = tr < KR2;
         piece(isk ? kcur : vcur, (uint32_t)(2 * (isk ? p.ks[3] : p.vs[3])), kg * KR2 + (isk ? tr : tr - KR2), kd + (uint32_t)tr * (D * 2));
       }
     }
 #pragma unroll
     for (int u = 0; u < PQ; ++u) {
-      const int tr = (wave + 8 * u) * 16;  // of the Q rows and then the dO rows
+      const int tr = (wave + NW * u) * 16;  // of the Q rows and then the dO rows
       const bool isq = tr < stage_rows;
       const int w = isq ? tr : tr - stage_rows;
       piece(isq ? qcur : docur, (uint32_t)(2 * (isq ? p.qs[3] : p.dos[3])), p.jr0 + w / JT * JW + t * JT + w % JT, dst + (uint32_t)tr * (D * 2));
@@ -589,7 +597,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
   float keep[16 * DT];
 
   if constexpr (FIX) {
-    static_for<0, dkdv_ring(D, NJT, JT, SJC).r - 1>([&](auto sc) {
+    static_for<0, dkdv_ring(D, NJT, JT, SJC, NW).r - 1>([&](auto sc) {
       if (decltype(sc)::value < nstage) stage_fix(std::integral_constant<int, decltype(sc)::value % STEPS>{}, decltype(sc)::value);
     });
   } else {
@@ -620,6 +628,14 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
 
     static_for<0, STEPS>([&](auto tc) {
       constexpr int t = decltype(tc)::value;
+      if constexpr (NW == 4 && t == 0) {  // (turns between the workgroups that share a SIMD, as in fta_fwd1_kernel)
+        if (ir & 1) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(3);
+      }
+      if constexpr (NW == 4 && t == (STEPS + 1) / 2) {
+        if (ir & 1) __builtin_amdgcn_s_setprio(0);
+        else __builtin_amdgcn_s_setprio(2);
+      }
       const int sidx = ir * STEPS + t;
       const half_t* cQ = smem + cur * slot_halfs;
       const half_t* cDO = cQ + stage_rows * D;
@@ -716,7 +732,7 @@ __global__ void __launch_bounds__(512) fta_bwd_dkdv_kernel(const BwdParams p) {
       const int nxt = sidx + 1 + ahead;
       cur = (cur + 1 == R) ? 0 : cur + 1;
       if constexpr (FIX) {
-        constexpr int AHEAD = dkdv_ring(D, NJT, JT, SJC).r - 2;
+        constexpr int AHEAD = dkdv_ring(D, NJT, JT, SJC, NW).r - 2;
         if (nxt < nstage) {
           stage_fix(std::integral_constant<int, (t + 1 + AHEAD) % STEPS>{}, fill);
           fill = (fill + 1 == R) ? 0 : fill + 1;

@@ -202,26 +202,31 @@ hipError_t launch_dkdv1(BwdParams p, const Dkdv1Plan& pl, int D, int dtype, bool
 // of NKT tiles, G1 of them to a stage, and of the dK/dV kernel with SJ slabs of NJT tiles, JT queries to a stage; eight
 // waves each (the kernels with that geometry fixed and the launch plan agree on it).
 struct Ring { int r, nb; };
-constexpr Ring fit_ring(int steps, int slot, int row, int records) {
+constexpr Ring fit_ring(int steps, int slot, int row, int records, int waves) {
   for (int r = 4; r >= 3; --r) {
     const int nb = (r + steps - 1) / steps;
-    if (r * slot + nb * row + records <= 160 * 1024) return Ring{r, nb};
+    if (r * slot + nb * row + records <= waves * 20 * 1024) return Ring{r, nb};
   }
   return Ring{0, 0};
 }
-constexpr Ring dq_ring(int D, int NKT, int G1, int SK) {
-  return fit_ring(NKT / G1, 4 * SK * G1 * 32 * D, 4 * (8 / SK) * 32 * D, SK > 1 ? 8 * 16 * (D / 32) * 64 * (D == 32 ? 4 : 2) : 0);
+constexpr int dq_records(int D, int SK, int waves) { return SK > 1 ? waves * 16 * (D / 32) * 64 * (D == 32 ? 4 : 2) : 0; }
+constexpr Ring dq_ring(int D, int NKT, int G1, int SK, int waves) {
+  return fit_ring(NKT / G1, 4 * SK * G1 * 32 * D, 4 * (waves / SK) * 32 * D, dq_records(D, SK, waves), waves);
+}
+constexpr size_t dq_smem(int D, int NKT, int G1, int SK, int waves) {
+  const Ring r = dq_ring(D, NKT, G1, SK, waves);
+  return (size_t)r.r * (4 * SK * G1 * 32 * D) + (size_t)r.nb * (4 * (waves / SK) * 32 * D) + dq_records(D, SK, waves);
 }
 // (the slabs' shares of dK and dV are exchanged in fp16, of four slabs of 192 queries in fp32, for which LDS has room)
 constexpr int dkdv_share_bytes(int NJT, int SJ) { return NJT == 6 && SJ == 4 ? 4 : 2; }
-constexpr int dkdv_shares(int D, int NJT, int SJ) { return (SJ - 1) * (8 / SJ) * 32 * (D / 32) * 64 * dkdv_share_bytes(NJT, SJ); }
-constexpr Ring dkdv_ring(int D, int NJT, int JT, int SJ) {
-  return fit_ring(NJT / (JT / 32), 4 * SJ * JT * D + 8 * SJ * JT, 4 * (8 / SJ) * 32 * D, dkdv_shares(D, NJT, SJ));
+constexpr int dkdv_shares(int D, int NJT, int SJ, int waves) { return (SJ - 1) * (waves / SJ) * 32 * (D / 32) * 64 * dkdv_share_bytes(NJT, SJ); }
+constexpr Ring dkdv_ring(int D, int NJT, int JT, int SJ, int waves) {
+  return fit_ring(NJT / (JT / 32), 4 * SJ * JT * D + 8 * SJ * JT, 4 * (waves / SJ) * 32 * D, dkdv_shares(D, NJT, SJ, waves), waves);
 }
 
-constexpr size_t dkdv_smem(int D, int NJT, int JT, int SJ) {
-  const Ring r = dkdv_ring(D, NJT, JT, SJ);
-  return (size_t)r.r * (4 * SJ * JT * D + 8 * SJ * JT) + (size_t)r.nb * (4 * (8 / SJ) * 32 * D) + dkdv_shares(D, NJT, SJ);
+constexpr size_t dkdv_smem(int D, int NJT, int JT, int SJ, int waves) {
+  const Ring r = dkdv_ring(D, NJT, JT, SJ, waves);
+  return (size_t)r.r * (4 * SJ * JT * D + 8 * SJ * JT) + (size_t)r.nb * (4 * (waves / SJ) * 32 * D) + dkdv_shares(D, NJT, SJ, waves);
 }
 
 // One key range and one query range of the backward with dropout beyond 512 keys (D = 32): stage and row-operand
@@ -229,12 +234,7 @@ constexpr size_t dkdv_smem(int D, int NJT, int JT, int SJ) {
 struct DropRange { Ring dq, dkdv; size_t smem, smem2; };
 inline DropRange drop_range(int len) {
   const int nkt = len / 128, g1 = nkt == 4 ? 2 : 1, njt = len / 64;
-  DropRange r;
-  r.dq = dq_ring(32, nkt, g1, 4);
-  r.dkdv = dkdv_ring(32, njt, 64, 2);
-  r.smem = (size_t)r.dq.r * (4 * 4 * g1 * 32 * 32) + (size_t)r.dq.nb * (4 * 2 * 32 * 32) + 8 * 16 * 64 * 4;
-  r.smem2 = dkdv_smem(32, njt, 64, 2);
-  return r;
+  return DropRange{dq_ring(32, nkt, g1, 4, 8), dkdv_ring(32, njt, 64, 2, 8), dq_smem(32, nkt, g1, 4, 8), dkdv_smem(32, njt, 64, 2, 8)};
 }
 
 // L2 is the length the tiles cover (a multiple of 128), `row` the true row length.

@@ -368,6 +368,23 @@ def test_dropout_at_the_tiled_lengths_of_head_dim_32(L1, L2, p, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L1,L2", [(61, 257), (8, 288), (33, 289), (17, 353), (64, 384), (9, 400), (40, 481), (7, 512)])
+def test_dropout_backward_in_workgroups_of_four_waves(L1, L2, dtype):
+    """257 to 512 keys: one query block or two key blocks to a workgroup, two workgroups to a CU; groups that end in a block of one
+    query, odd numbers of key blocks, chunks of one and of several rows (whose turns of priority are two rows long)."""
+    import fta_lib
+    B, H, p, sm = 2, 3, 0.15, 1.0 / math.sqrt(32)
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, p, 77, 0)
+    plan = fta_lib.describe_plan(B, H, L1, L2, 32, sm, opt)
+    assert plan["dq"]["block"] == plan["dkdv"]["block"] == 256
+    print(f"case dropout four waves {L1}x{L2} {dtype}", flush=True)
+    q, k, v, b, do = _inputs(B, H, L1, L2, 32, 53, dtype)
+    keep, scale = dm.keep_mask(77, p, B, H, L1, L2)
+    ref = _oracle(q, k, v, b, sm, do, keep=torch.from_numpy(keep).to(DEV), keep_scale=scale)
+    _compare(_run(q, k, v, b, sm, do, p, 77), ref, dtype, f"dropout four waves {L1}x{L2}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("L1,L2,launches,launches2", [(5, 513, 2, 2), (4, 640, 2, 2), (9, 768, 2, 1), (3, 801, 2, 2), (4, 1024, 2, 1), (3, 1100, 3, 3),
                                                       (3, 2011, 4, 2)])
 def test_dropout_beyond_512_keys_in_ranges_of_their_own(L1, L2, launches, launches2, dtype):
