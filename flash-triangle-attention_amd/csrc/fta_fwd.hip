@@ -32,7 +32,7 @@ static bool fwd_instance_exists(int D, int NKT, int KT, bool feat) {
 }
 
 // The plan for rows cut into slabs of kw keys (invalid if no built instance and stage length fit).
-static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int kw) {
+static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, int row, bool feat, int kw) {
   FwdPlan pl{};
   pl.NKT = kw / 32;
   pl.S = L2 / kw;
@@ -41,12 +41,16 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int
   // (their barriers do not couple: measured 5 to 20 % faster than one of 8); several slabs want the
   // 8 waves of one workgroup behind each staged tile.
   // (D = 32 with a number of query blocks that four does not divide: workgroups of two waves, four to a CU)
-  const int maxw = (pl.S == 1 && D == 32) ? (nqb % 4 == 0 ? 4 : 2) : 8;
+  // (dropout, bound by the vector ALU, wants two workgroups of four waves and their turns of priority with two slabs, too: training steps at
+  // B1 H4 of 600, 750 and 1024 keys 1936 / 1881, 3396 / 3314 and 8651 / 8397 us, at D = 64 of 200 and 400 keys 241 / 238 and 1516 / 1488.  Without,
+  // two slabs at D = 64 are bound by the copies into LDS, which twice as many workgroups double: 640 keys 489 / 511, 768 795 / 900)
+  const bool halves = feat && pl.S <= 2;
+  const int maxw = (pl.S == 1 && D == 32) ? (nqb % 4 == 0 ? 4 : 2) : halves ? 4 : 8;
   int qb = maxw / pl.S;
   if (qb < 1) qb = 1;
   while (qb > 1 && nqb % qb != 0) --qb;
   pl.QB = qb;
-  pl.nqg = nqb / qb;
+  pl.nqg = ((row + 31) / 32 + qb - 1) / qb;
   pl.threads = 64 * pl.S * pl.QB;
   // keys per staged tile: as many as LDS allows (longer stages = longer prefetch distance).  The
   // records of the slab merge get a region of their own where that fits next to the tile chosen;
@@ -79,7 +83,7 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, bool feat, int
       if (kw % kt != 0) continue;
       const size_t bufs = (size_t)2 * 2 * pl.S * kt * D * sizeof(uint16_t);
       const size_t smem = bufs + (alias ? 0 : scratch);
-      if (bufs + (alias ? 0 : scratch_room) > 160 * 1024) continue;
+      if (bufs + (alias ? 0 : scratch_room) > (halves ? 80 : 160) * 1024) continue;
       if (alias && scratch > bufs / 2) continue;  // the records must fit one stage buffer
       if (pl.S * kt * (D / 8) / 64 > 4 * (pl.threads / 64)) continue;  // the kernel's copy plan holds 4 copies per wave and tile
       if (!fwd_instance_exists(D, pl.NKT, kt, feat)) continue;
@@ -108,7 +112,7 @@ FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, int row, bool feat, bool s
   if (!feat && plan_fwd2(B, H, L1, L2, D, pl)) return pl;
   auto take = [&](int kw, bool wide = false) {
     if (pl.valid || kw < 128 || (kw > kwmax && !wide) || kw % 32 != 0 || L2 % kw != 0) return;
-    pl = plan_fwd_slab(B, H, L1, L2, D, feat, kw);
+    pl = plan_fwd_slab(B, H, L1, L2, D, row, feat, kw);
   };
   auto pow2 = [](int n) { return n >= 1 && n <= 8 && (n & (n - 1)) == 0; };
   // 0. D=64 (not the dropout instances): slabs of up to 448 keys (14 tiles of bias still fit the registers,

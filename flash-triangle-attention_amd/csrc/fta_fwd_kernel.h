@@ -199,14 +199,14 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
 
 #pragma unroll
     for (int t = 0; t < STEPS; ++t) {
-      // One slab: independent workgroups share the SIMDs, and a wave's priority falls from half row to half row, in turns of two
+      // Workgroups of less than eight waves share the SIMDs: a wave's priority falls from half row to half row, in turns of two
       // rows, so that the older workgroup does not run ahead (see fta_fwd1_kernel): with dropout B1 H4 L300 76 against 70 us, L450 a
-      // training step 960 / 935, without at D = 64 B4 H8 L100 40.2 / 39.2.  (Waves of several slabs, in one workgroup: up to 2 % slower.)
-      if (S == 1 && t == 0) {
+      // training step 960 / 935, without at D = 64 B4 H8 L100 40.2 / 39.2.  (Eight waves in one workgroup: up to 2 % slower.)
+      if (nthreads < 512 && t == 0) {
         if (ir & 1) __builtin_amdgcn_s_setprio(1);
         else __builtin_amdgcn_s_setprio(3);
       }
-      if (S == 1 && t == (STEPS + 1) / 2) {
+      if (nthreads < 512 && t == (STEPS + 1) / 2) {
         if (ir & 1) __builtin_amdgcn_s_setprio(0);
         else __builtin_amdgcn_s_setprio(2);
       }
