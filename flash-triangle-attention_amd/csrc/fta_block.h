@@ -22,6 +22,7 @@ struct BlockParams {
   void* dog; void* dgp;                   // dO (16-bit type), gradient of the gate before the sigmoid (block's type)
   const void* dqkv[3]; const void* db;    // attention gradients
   void* wt;                               // packed transposed projection weights, in MFMA operand order
+  float2* stats;                          // the layer norm's {mean, reciprocal deviation} of every pair row
   float* part;                            // weight-gradient partial sums, one block of wgrad_part_floats() per section and chunk
   float* red;                             // contributions to the layer norm's gradients, (groups, 2, C)
   void* dw[4]; void* dwb; void* dbg; void* dwo; void* dbo; void* dgamma; void* dbeta;

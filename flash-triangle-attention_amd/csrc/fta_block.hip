@@ -29,12 +29,12 @@
 // at once, the fp32 instruction two.  Infinity, and values that round to it in
 // bf16 (beyond 3.39e38), have no three parts: a tile whose sums are not all finite is formed again by the fp32 instruction,
 // so that infinities come out as they went in.  Nothing is rounded to 16 bits in memory that was not before (q, k, v, bias, o and their gradients).
-// us per kernel at 192 x 192 pairs, before and after: proj 69 / 47, out 32 / 26, dout 29 / 28, dx 57 / 48, wgrad 82 / 55; a
+// us per kernel at 192 x 192 pairs, before and after: proj 69 / 47, out 32 / 26, dout 29 / 28, dx 57 / 48, wgrad 82 / 50; a
 // training pass 352 / 265 (256 x 256: 498 / 394, 321 x 321: 838 / 670), inference 112 / 82 (457 x 457: 505 / 387).
 //
 // Measured, AlphaFold2's block (C 128, 4 heads of 32) at 384 x 384 pairs in bf16: a training pass 3.64 ms as separate
 // library calls around the attention, 0.52 with these; us per kernel (rocprofv3, mean of 30 launches): proj 56, out
-// 30, dout 43, dx 54, wgrad 82, reduce 10, norm_grad 5.
+// 30, dout 43, dx 47, wgrad 66, reduce 11, norm_grad 5.
 #include "fta_block.h"
 
 #include <type_traits>
@@ -898,6 +898,10 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
       float x[8], g[8], mean, rstd;
       unpack<A>(z[n], x);
       normalise<C>(x, p.eps, mean, rstd);
+      if (c8 == 0) {
+        const int b = st / nst, q = min((st - b * nst) * TR + row, LL - 1);
+        p.stats[(int64_t)b * LL + q] = float2{mean, rstd};
+      }
 #pragma unroll
       for (int e = 0; e < 8; ++e) g[e] = 0.f;
 #pragma unroll
@@ -973,21 +977,24 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
 // ---- backward: weight gradients -----------------------------------------------------------------------
 // Six products with the pair rows as contraction: section s = 0..3 is (d of projection s)^T xhat, with xhat
 // the normalised row without gamma and beta (the reduction applies those: one product serves the weight, gamma
-// and beta), section 4 is dout^T (gate * o), section 5 the bias projection's.  A workgroup works off one chunk of
+// and beta), section 4 is dout^T (gate * o), section 5 the bias projection's, which the workgroups of section 0 form beside
+// theirs (by workgroups of its own, which loaded and normalised z for H columns, the launch took 80 us at 384 x 384 pairs in bf16 and 56
+// at 192 x 192 in fp32; so 67 and 50).  A workgroup works off one chunk of
 // rows of one section: stages of 64 rows (32 in fp32) are formed in registers, written to LDS as 32-column
 // sub-tiles and read back transposed as MFMA operands; its waves own up to two 32 x 32 tiles of the result
-// each.  The sums over the rows (bias gradients) are kept by the threads that load the rows.  The
-// sections of a chunk sit on one die, whose L2 serves z to five of them.
+// each.  The sums over the rows (bias gradients) are products with ones, in fp32 kept by the threads that load the rows; a row's mean
+// and deviation come from blk_dx_kernel.  The sections of a chunk sit on one die, whose L2 serves z to four of them.
 //
-// Bound by memory latency and the vector ALU rather than bandwidth: a stage has 8 MFMAs per wave.  So all
+// Bound by memory: 300 MB in, z counted once, at 384 x 384 pairs in bf16 (4.5 TB/s).  A stage has 8 MFMAs per wave.  All
 // addresses are a base plus the row, the next stage's loads are in flight during a stage, and two workgroups
 // share a CU.  fp32: the three planes of a stage take the LDS of two, so a stage is read, then replaced between two
-// barriers (82 -> 55 us at 192 x 192 pairs; taken apart at every use instead, by up to four waves each, 69).  Sections in separate workgroups keep a partial sum at 64 KB (one workgroup for all six: 264 KB, 67 MB to
+// barriers (with six sections 82 -> 55 us at 192 x 192 pairs; taken apart at every use instead, by up to four waves each, 69).  Sections in separate workgroups keep a partial sum at 64 KB (one workgroup for all six: 264 KB, 67 MB to
 // write and read back over the chip, as much as the inputs at 384 x 384 pairs).
 //
 // One chunk's partial: the result tiles row-major [a][b], then (at C * HD) the row sums.
 __host__ __device__ inline size_t wgrad_part_floats(int C, int HD) { return (size_t)C * HD + (C > HD ? C : HD); }
-constexpr int kWgradSections = 6;
+constexpr int kWgradSections = 6;   // of partial sums; the workgroups of section 0 form section 5, too
+constexpr int wgrad_bias_bytes(int TR) { return 4 * (TR + 8) * 2; }  // dbias in a stage: a padded row per head
 
 // Sub-tile of 32 columns in LDS: 16-bit rows of 64 bytes, swizzled as the attention's staged tiles; fp32: a plane of such
 // rows after the other (PL of the three).
@@ -1007,23 +1014,24 @@ __device__ __forceinline__ Op<F32> sub_frag_t(const char* tile, int rowbase, con
   return o;
 }
 
-enum WgradKind { kWgradQkv, kWgradGate, kWgradOut, kWgradBias };
+enum WgradKind { kWgradQkv, kWgradGate, kWgradOut };
 
-template <class A, bool F32, int C, int HD, int KIND>
+// BIAS: the bias heads' gradient, too, which are H more rows of operand A
+template <class A, bool F32, int C, int HD, int KIND, bool BIAS = false>
 __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int chunk, char* smem) {
-  constexpr int NA = KIND == kWgradOut ? C / 32 : KIND == kWgradBias ? 1 : HD / 32;
+  constexpr int NA = KIND == kWgradOut ? C / 32 : HD / 32;
   constexpr int NB = KIND == kWgradOut ? HD / 32 : C / 32;
   constexpr int NT = (NA * NB + 7) / 8;                 // result tiles per wave
   constexpr int TR = F32 ? 32 : 64;                     // rows per stage
-  constexpr int PA = KIND == kWgradBias ? 0 : (TR * NA * 4 + 511) / 512;   // 8-element pieces per thread
+  constexpr int PA = (TR * NA * 4 + 511) / 512;         // 8-element pieces per thread
   constexpr int PB = (TR * NB * 4 + 511) / 512;
-  constexpr int PD = KIND == kWgradBias ? 4 : 0;        // dbias entries per thread (H <= 32)
-  constexpr int PLA = KIND == kWgradQkv || KIND == kWgradBias ? 2 : 3;  // (fp32) planes of operand A: q, k, v's gradients are fp16
+  static_assert(4 * TR <= 512 && NA <= 4 && NB <= 4, "a thread has one dbias entry; a wave one tile more");
+  constexpr int PLA = KIND == kWgradQkv ? 2 : 3;  // (fp32) planes of operand A: q, k, v's gradients are fp16
   constexpr int SUB = (F32 ? 3 : 1) * TR * 64;          // bytes of a sub-tile
   constexpr int BUFS = F32 ? 1 : 2;                     // stage buffers: two workgroups share a CU's LDS
   constexpr int DROW = TR + 8;                          // dbias: one row of TR entries per head
-  constexpr int ABYTES = KIND == kWgradBias ? 32 * DROW * 2 : NA * SUB;
-  constexpr int BUF = ABYTES + NB * SUB;
+  constexpr int ABYTES = NA * SUB;
+  constexpr int BUF = ABYTES + NB * SUB + (BIAS ? wgrad_bias_bytes(TR) : 0);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
   const int LL = (int)p.LL, nst = (LL + TR - 1) / TR;   // stages per batch entry
   const int ntot = p.B * nst, per = (ntot + p.nchunks - 1) / p.nchunks;
@@ -1031,13 +1039,14 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
   FragOffsets<32> fo;
   fo.init(lane);
 
-  const void* srca = KIND == kWgradQkv ? p.dqkv[sec] : KIND == kWgradGate ? p.dgp : KIND == kWgradOut ? p.dout : p.db;
-  Frag<F32> ra[PA > 0 ? PA : 1], rx[PB];
+  const void* srca = KIND == kWgradQkv ? p.dqkv[sec] : KIND == kWgradGate ? p.dgp : p.dout;
+  Frag<F32> ra[PA], rx[PB];
   Frag<false> ro[PB];
-  uint16_t rd[PD > 0 ? PD : 1];
+  float2 rs[PB];
+  uint16_t rd = 0;
   // where this thread's pieces sit: row of the stage, and the offset of their first element inside row 0
   auto head_part = [&](int c8) { const int h = c8 / p.D; return ((int64_t)h * LL) * p.D + (c8 - h * p.D); };
-  int64_t ao[PA > 0 ? PA : 1], bo[PB];
+  int64_t ao[PA], bo[PB];
 #pragma unroll
   for (int n = 0; n < PA; ++n) {
     const int c8 = ((tid + 512 * n) % (NA * 4)) * 8;
@@ -1072,37 +1081,36 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
         ro[n] = load8<false>(p.o, hb + (int64_t)q * p.D + bo[n]);
       } else {
         rx[n] = load8<F32>(p.z, pair_row(p.zs, b, q) + bo[n]);
+        rs[n] = p.stats[(int64_t)b * LL + q];
       }
     }
-#pragma unroll
-    for (int n = 0; n < PD; ++n) {
-      const int e = tid + 512 * n, h = e / TR, q = min(p0 + e % TR, LL - 1);
-      if (h < p.H) rd[n] = static_cast<const uint16_t*>(srca)[((int64_t)b * p.H + h) * LL + q];
+    if constexpr (BIAS) {
+      const int h = tid / TR, q = min(p0 + tid % TR, LL - 1);
+      if (h < p.H) rd = static_cast<const uint16_t*>(p.db)[((int64_t)b * p.H + h) * LL + q];
     }
   };
   // forms operand B (gate * o, or the normalised row: the lanes of a row are neighbours) and writes both to LDS;
   // rows beyond the end are zero in operand B
-  float csum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // of this thread's columns of operand A (dbias: of its entry)
+  [[maybe_unused]] float csum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // (fp32) of this thread's columns of operand A
+  [[maybe_unused]] float dsum = 0.f;                                            // of this thread's dbias entry
   auto put = [&](char* buf, int st) {
     const int left = LL - (st % nst) * TR;
 #pragma unroll
     for (int n = 0; n < PA; ++n) {
       const int pc = tid + 512 * n, row = pc / (NA * 4), c = pc % (NA * 4);
       if (TR * NA * 4 >= 512 || row < TR) {
+        if (row >= left) ra[n] = frag_zero<F32>();
         sub_write<F32, TR, PLA>(buf + (c / 4) * SUB, row, c % 4, to_op(ra[n]));
-        float v[8];
-        unpack<A>(ra[n], v);
-        const float one = row < left ? 1.0f : 0.0f;
+        if constexpr (F32)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) csum[e] = __builtin_fmaf(v[e], one, csum[e]);
+          for (int e = 0; e < 8; ++e) csum[e] += ra[n].v[e];
       }
     }
-#pragma unroll
-    for (int n = 0; n < PD; ++n) {
-      const int e = tid + 512 * n, h = e / TR;
+    if constexpr (BIAS) {
+      const int h = tid / TR;
       if (h < p.H) {
-        reinterpret_cast<uint16_t*>(buf)[h * DROW + e % TR] = rd[n];
-        csum[n] += e % TR < left ? A::lo((uint32_t)rd[n]) : 0.f;
+        reinterpret_cast<uint16_t*>(buf + ABYTES + NB * SUB)[h * DROW + tid % TR] = rd;
+        dsum += tid % TR < left ? A::lo((uint32_t)rd) : 0.f;
       }
     }
 #pragma unroll
@@ -1116,8 +1124,8 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] *= w[e];
       } else {
-        float mean, rstd;
-        normalise<C>(v, p.eps, mean, rstd);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (v[e] - rs[n].x) * rs[n].y;
       }
       Frag<F32> f;
       pack<A>(v, f);
@@ -1125,30 +1133,36 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
       if (TR * NB * 4 >= 512 || row < TR) sub_write<F32, TR, 3>(buf + ABYTES + (c / 4) * SUB, row, c % 4, to_op(f));
     }
   };
-  auto frag_a = [&](const char* buf, int at, int k) {
-    if constexpr (KIND == kWgradBias) {
-      const char* s = buf + ((size_t)(l32 < p.H ? l32 : 0) * DROW + k * 16 + 4 * hh) * 2;
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(s), hi = *reinterpret_cast<const u32x2*>(s + 16);
-      Frag<false> d;
-      d.w = u32x4{lo[0], lo[1], hi[0], hi[1]};
-      if (l32 >= p.H) d = frag_zero<false>();
-      if constexpr (F32) {
-        Frag<true> f;
-        unpack<A>(d, f.v);
-        return to_op(f);
-      } else {
-        return to_op(d);
-      }
+  // the bias heads as operand A: column l % 32 is head l % 32
+  auto frag_d = [&](const char* buf, int k) {
+    const char* s = buf + ABYTES + NB * SUB + ((size_t)(l32 < p.H ? l32 : 0) * DROW + k * 16 + 4 * hh) * 2;
+    const u32x2 lo = *reinterpret_cast<const u32x2*>(s), hi = *reinterpret_cast<const u32x2*>(s + 16);
+    Frag<false> d;
+    d.w = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    if (l32 >= p.H) d = frag_zero<false>();
+    if constexpr (F32) {
+      Frag<true> f;
+      unpack<A>(d, f.v);
+      return to_op(f);
     } else {
-      return sub_frag_t<F32, TR, PLA>(buf + at * SUB, k * 16, fo);
+      return to_op(d);
     }
   };
 
-  floatx16 acc[NT];
+  auto head_tile = [&](const char* buf, int k, floatx16 c) {
+    return mma<A, 2, false>(frag_d(buf, k), sub_frag_t<F32, TR, 3>(buf + ABYTES + (wave - 4) * SUB, k * 16, fo), c);
+  };
+  floatx16 acc[NT], more = zero16();
 #pragma unroll
   for (int n = 0; n < NT; ++n) acc[n] = zero16();
   const int at = wave % NA;             // (NA divides 8: the same rows for both tiles of a wave)
   const bool own = wave < NA * NB;      // (fewer than eight tiles: the other waves only help staging)
+  // one tile more: the row sums of operand A, as a product with ones (waves 0 .. NA - 1; fp32: by the threads that load the rows, since
+  // three parts of an infinite entry would not sum to it), the bias heads' tiles (waves 4 .. 4 + NB - 1)
+  const bool sums = !F32 && wave < NA, heads = BIAS && wave >= 4 && wave < 4 + NB;
+  u32x4 ones;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) ones[e] = A::is_bf16 ? 0x3F803F80u : 0x3C003C00u;
   if (first < last) {
     fetch(first);
     put(smem, first);
@@ -1159,11 +1173,20 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
       if (own) {
 #pragma unroll
         for (int k = 0; k < TR / 16; ++k) {
-          const Op<F32> fa = frag_a(buf, at, k);
+          const Op<F32> fa = sub_frag_t<F32, TR, PLA>(buf + at * SUB, k * 16, fo);
 #pragma unroll
           for (int n = 0; n < NT; ++n)
             acc[n] = mma<A, PLA, PLA == 3>(fa, sub_frag_t<F32, TR, 3>(buf + ABYTES + (wave / NA + n * (8 / NA)) * SUB, k * 16, fo), acc[n]);
+          if (sums) more = A::mfma(as_half8(fa.p[0]), as_half8(ones), more);
+          if (NA * NB >= 8 && heads) more = head_tile(buf, k, more);
         }
+        // (no unfinished product over the branches: the listings are checked line by line)
+        if constexpr (BIAS) asm volatile("s_nop 15" : "+v"(more), "+v"(acc[NT - 1]));
+      }
+      if (NA * NB < 8 && heads) {
+#pragma unroll
+        for (int k = 0; k < TR / 16; ++k) more = head_tile(buf, k, more);
+        asm volatile("s_nop 15" : "+v"(more));
       }
       if constexpr (BUFS == 1) __syncthreads();
       if (st + 1 < last) {
@@ -1177,7 +1200,9 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
     bool again = not_finite(acc[0]);
 #pragma unroll
     for (int n = 1; n < NT; ++n) again = again || not_finite(acc[n]);
-    if (own && again) {  // two rows at a time, one per lane half
+    if (heads) again = again || not_finite(more);
+    if ((own || heads) && again) {  // two rows at a time, one per lane half
+      more = zero16();
 #pragma unroll
       for (int n = 0; n < NT; ++n) acc[n] = zero16();
       const int col = at * 32 + l32;
@@ -1186,8 +1211,8 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
         const int st = r / TR, b = st / nst, row = (st - b * nst) * TR + r % TR + hh, q = min(row, LL - 1);
         const int64_t hb = (int64_t)b * p.H * LL * p.D + (int64_t)q * p.D;
         float x, y[NT];
+        [[maybe_unused]] float xd = 0.f, yd = 0.f;
         if constexpr (KIND == kWgradOut) x = load1<A, true>(srca, pair_row(p.douts, b, q) + col);
-        else if constexpr (KIND == kWgradBias) x = l32 < p.H ? load1<A, false>(srca, ((int64_t)b * p.H + l32) * LL + q) : 0.f;
         else x = load1<A, KIND == kWgradGate>(srca, hb + head_part(col));
         if constexpr (KIND == kWgradOut) {
 #pragma unroll
@@ -1215,37 +1240,56 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
 #pragma unroll
             for (int m = 0; m < NB; ++m) y[n] = wave / NA + n * (8 / NA) == m ? z[m] * rstd : y[n];
           }
+          if constexpr (BIAS) {
+            if (l32 < p.H && row < LL) xd = load1<A, false>(p.db, ((int64_t)b * p.H + l32) * LL + q);
+#pragma unroll
+            for (int m = 0; m < NB; ++m) yd = wave - 4 == m && row < LL ? z[m] * rstd : yd;
+          }
         }
         if (row >= LL) x = 0.f;
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, row < LL ? y[n] : 0.f, acc[n], 0, 0, 0);
+        if constexpr (BIAS) more = __builtin_amdgcn_mfma_f32_32x32x2f32(xd, yd, more, 0, 0, 0);
+        asm volatile("s_nop 15" : "+v"(acc[0]), "+v"(acc[NT - 1]), "+v"(more));  // (the same)
       }
     }
   }
   // partial of this chunk
   float* out = p.part + ((size_t)sec * p.nchunks + chunk) * wgrad_part_floats(C, HD);
-  const int rows = KIND == kWgradBias ? p.H : NA * 32;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int a = at * 32 + 8 * (r / 4) + 4 * hh + r % 4;
-    if (a >= rows || !own) continue;
+    if (!own) continue;
 #pragma unroll
     for (int n = 0; n < NT; ++n) out[(size_t)a * (NB * 32) + (wave / NA + n * (8 / NA)) * 32 + l32] = acc[n][r];
+    if (sums && l32 == 0) out[(size_t)C * HD + a] = more[r];
   }
   float* ssum = reinterpret_cast<float*>(smem);  // (the last stage has been read: every wave is past its barrier)
-  constexpr int PER = KIND == kWgradBias ? TR : 512 / (NA * 4);
-  if constexpr (KIND == kWgradBias) {
-#pragma unroll
-    for (int n = 0; n < PD; ++n) ssum[tid + 512 * n] = csum[n];
-  } else {
+  constexpr int PER = 512 / (NA * 4);
+  if constexpr (F32) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) ssum[((tid % (NA * 4)) * 8 + e) * (PER + 1) + tid / (NA * 4)] = csum[e];
+    __syncthreads();
+    if (tid < NA * 32) {
+      float s = 0.f;
+      for (int k = 0; k < PER; ++k) s += ssum[tid * (PER + 1) + k];
+      out[(size_t)C * HD + tid] = s;
+    }
   }
-  __syncthreads();
-  if (tid < rows) {
-    float s = 0.f;
-    for (int k = 0; k < PER; ++k) s += ssum[KIND == kWgradBias ? tid * TR + k : tid * (PER + 1) + k];
-    out[(size_t)C * HD + tid] = s;
+  if constexpr (BIAS) {
+    float* out5 = p.part + ((size_t)5 * p.nchunks + chunk) * wgrad_part_floats(C, HD);
+    if (heads && hh == 0)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (r < p.H) out5[r * (NB * 32) + (wave - 4) * 32 + l32] = more[r];
+    if constexpr (F32) __syncthreads();
+    ssum[tid] = dsum;
+    __syncthreads();
+    if (tid < p.H) {
+      float s = 0.f;
+      for (int k = 0; k < TR; ++k) s += ssum[tid * TR + k];
+      out5[(size_t)C * HD + tid] = s;
+    }
   }
 }
 
@@ -1253,11 +1297,11 @@ template <class A, bool F32, int C, int HD>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) blk_wgrad_kernel(BlockParams p) {
   extern __shared__ char smem[];
   const int slot = (int)blockIdx.x / kXcds;
-  const int sec = slot % kWgradSections, chunk = (slot / kWgradSections) * kXcds + (int)blockIdx.x % kXcds;
-  if (sec < 3) wgrad_body<A, F32, C, HD, kWgradQkv>(p, sec, chunk, smem);
+  const int sec = slot % (kWgradSections - 1), chunk = (slot / (kWgradSections - 1)) * kXcds + (int)blockIdx.x % kXcds;
+  if (sec == 0) wgrad_body<A, F32, C, HD, kWgradQkv, true>(p, sec, chunk, smem);
+  else if (sec < 3) wgrad_body<A, F32, C, HD, kWgradQkv>(p, sec, chunk, smem);
   else if (sec == 3) wgrad_body<A, F32, C, HD, kWgradGate>(p, sec, chunk, smem);
-  else if (sec == 4) wgrad_body<A, F32, C, HD, kWgradOut>(p, sec, chunk, smem);
-  else wgrad_body<A, F32, C, HD, kWgradBias>(p, sec, chunk, smem);
+  else wgrad_body<A, F32, C, HD, kWgradOut>(p, sec, chunk, smem);
 }
 
 // Sums the chunks in a fixed order: a workgroup takes four rows of the projections' gradients (4*HD, then H of the
@@ -1421,8 +1465,9 @@ hipError_t launch_block_dx(BlockParams p, int C, int dtype, hipStream_t st) {
 hipError_t launch_block_wgrad(BlockParams p, int C, int dtype, hipStream_t st) {
   // (the largest section: both operands C or HD columns wide; the bias section has one row per head)
   const int n = (p.HD + C) / 32;
-  const size_t smem = dtype == 2 ? (size_t)n * 3 * 32 * 64 : (size_t)2 * n * 64 * 64;  // (fp32: one stage of three planes)
-  const dim3 grid((unsigned)(kWgradSections * p.nchunks)), block(512);
+  // (fp32: one stage of three planes)
+  const size_t smem = dtype == 2 ? (size_t)n * 3 * 32 * 64 + wgrad_bias_bytes(32) : (size_t)2 * (n * 64 * 64 + wgrad_bias_bytes(64));
+  const dim3 grid((unsigned)((kWgradSections - 1) * p.nchunks)), block(512);
   const dim3 rgrid((unsigned)(reduce_proj_groups(p.HD, p.H) + C / 4));
 #define FTA_BLOCK_CASE(AA, FF, CC, HH)                                                                       \
   {                                                                                                          \
@@ -1446,7 +1491,7 @@ size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 // Byte offsets of the forward state and the backward workspace.
 struct BlockLayout {
   size_t q, k, v, bias, o, gate, lse, state;
-  size_t dog, dgp, dq, dk, dv, db, wt, part, red, attn, attn_bytes, total;
+  size_t dog, dgp, dq, dk, dv, db, wt, stats, part, red, attn, attn_bytes, total;
   int nchunks;
 };
 bool block_supported(const fta_block& b) {
@@ -1473,11 +1518,12 @@ BlockLayout block_layout(const fta_block& b) {
   at = 0;
   l.dog = take(2 * n); l.dgp = take(es * n); l.dq = take(2 * n); l.dk = take(2 * n); l.dv = take(2 * n); l.db = take(2 * m);
   l.wt = take((size_t)(b.C / 32) * (4 * HD / 16 + 1) * frag_bytes(b.dtype));
-  // Chunks of the weight-gradient kernel, a multiple of the dies: six sections of 80 are 480 workgroups, of which two
-  // fit a CU (56: 118 us at 384 x 384 pairs in bf16, 40: 110, 80: 91).  A chunk keeps at least four stages, so that its partial sums (64 KB at C = H*D = 128) are not
+  l.stats = take((size_t)b.B * LL * sizeof(float2));
+  // Chunks of the weight-gradient kernel, a multiple of the dies: five sections of 96 are 480 workgroups, of which two
+  // fit a CU (with six sections 56: 118 us at 384 x 384 pairs in bf16, 40: 110, 80: 91).  A chunk keeps at least four stages, so that its partial sums (64 KB at C = H*D = 128) are not
   // what the launch spends its time on.
   const size_t rows = b.dtype == FTA_DTYPE_F32 ? 32 : 64, stages = b.B * ((LL + rows - 1) / rows);
-  l.nchunks = kXcds * (int)(stages < 64 ? 1 : stages > 32 * 10 ? 10 : stages / 32);
+  l.nchunks = kXcds * (int)(stages < 64 ? 1 : stages > 32 * 12 ? 12 : stages / 32);
   l.part = take((size_t)kWgradSections * l.nchunks * wgrad_part_floats(b.C, (int)HD) * sizeof(float));
   l.red = take((size_t)reduce_proj_groups((int)HD, b.H) * 2 * b.C * sizeof(float));
   const fta_options opt = attn_options(b);
@@ -1595,6 +1641,7 @@ int fta_block_bwd(const fta_block* b, const void* state, const void* dout, const
   p.dog = w + l.dog; p.dgp = w + l.dgp;
   p.dqkv[0] = w + l.dq; p.dqkv[1] = w + l.dk; p.dqkv[2] = w + l.dv; p.db = w + l.db;
   p.wt = w + l.wt;
+  p.stats = reinterpret_cast<float2*>(w + l.stats);
   p.part = reinterpret_cast<float*>(w + l.part);
   p.red = reinterpret_cast<float*>(w + l.red);
   p.dw[0] = g->wq; p.dw[1] = g->wk; p.dw[2] = g->wv; p.dw[3] = g->wg;
