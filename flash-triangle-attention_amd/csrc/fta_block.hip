@@ -553,15 +553,17 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
   // Half of the waves (one of the two that share a SIMD) prepare the next stage first and multiply then, the others the other
   // way round, so that one wave's products run beside the other's layer norm.
   auto prepare = [&](int st, int it) {
-    put((it + 1) & 1);  // (behind the last stage: once more the last rows, into the buffer nobody reads)
-    fetch(min(st + 2 * teams, ntot - 1));
+    put((it + 1) & 1);
+    fetch(min(st + 2 * teams, ntot - 1));  // (behind the last stage: once more the last rows, which nobody waits for)
   };
-  for (int it = 0; st < ntot; st += teams, ++it) {
+  int it = 0;
+  for (; st + teams < ntot; st += teams, ++it) {
     if (wave >= 4) prepare(st, it);
     products(st, it);
     if (wave < 4) prepare(st, it);
     __syncthreads();
   }
+  if (st < ntot) products(st, it);
   if constexpr (F32)
     if (bad)
 #pragma clang loop unroll(disable)
@@ -941,6 +943,7 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
     }
     if constexpr (F32) bad = bad || not_finite(acc);
     finish(acc, st);
+    if (next >= ntot) break;
     put();
     __syncthreads();
   }
