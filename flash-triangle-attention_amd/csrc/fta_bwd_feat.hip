@@ -35,7 +35,8 @@ template <class T, bool DROP>
 static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t st, hipEvent_t* ev) {
   auto mark = [&](int i) { if (ev != nullptr) (void)hipEventRecord(ev[i], st); };
   hipError_t e = hipSuccess;
-  {  // 0. delta and the {lse, delta} pairs
+  const bool own = DROP && D == 32 && pl.NKT == 3 && pl.nranges == 0;  // the dQ kernel's instance for 384 keys forms them itself
+  if (!own) {  // 0. delta and the {lse, delta} pairs
     const int64_t nthr = (int64_t)p.B * p.H * p.L1 * p.L2p * (D / 8);
     dim3 grid((unsigned)((nthr + 255) / 256)), block(256);
     if (D == 32) hipLaunchKernelGGL((fta_bwd_delta_kernel<T, 32>), grid, block, 0, st, p);
