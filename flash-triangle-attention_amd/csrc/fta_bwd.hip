@@ -119,19 +119,19 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
     if (L2 % c == 0) { jw = c; break; }
   // (dropout, lengths that three slabs of 128 queries would cut: two slabs of 192, as many waves for every SIMD)
   const bool two192 = (feat == 2 && D == 32 && jw == 128 && L2 % 384 == 0);
-  if (two192) jw = 192;
+  if (two192) jw = row <= 320 ? 160 : 192;
   pl.NJT = jw / 32;
-  const int nslab = L2 / jw;
+  const int nslab = two192 ? 2 : L2 / jw;
   const int sjmax = two192 ? 2 : 4;
   bool ok2 = false;
   for (int sj = (nslab < sjmax ? nslab : sjmax); sj >= 1 && !ok2; --sj) {
     if (nslab % sj != 0) continue;
-    const bool four2 = (feat == 2 && D == 32 && sj == 2 && jw >= 192);
+    const bool four2 = (feat == 2 && D == 32 && sj == 2 && jw >= 160);
     int kb = (four2 ? 4 : 8) / sj;
     if (kb < 1) continue;
     while (kb > 1 && nqb % kb != 0) --kb;
     for (int jt = 64; jt >= 32 && !ok2; jt /= 2) {
-      if (jw % jt != 0) continue;
+      if (jw % jt != 0) continue;  // (160 queries: stages of 32)
       const int stage_rows2 = sj * jt;
       const size_t slot2 = (size_t)2 * stage_rows2 * D * 2 + (size_t)2 * stage_rows2 * 4;
       const size_t scratch2 = (size_t)(sj - 1) * kb * 32 * (D / 32) * 64 * 2;  // fp16 partials
@@ -142,7 +142,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
         if (r * slot2 + nb * ktile2 + scratch2 > lds_max / (four2 ? 2 : 1)) continue;
         pl.SJ = sj; pl.KB = kb; pl.nkg = (nblk + kb - 1) / kb; pl.threads2 = 64 * sj * kb; pl.JT = jt;
         pl.ring2 = r; pl.nb2 = nb; pl.smem2 = r * slot2 + nb * ktile2 + scratch2;
-        pl.JR = sj * jw; pl.nlaunch2 = L2 / pl.JR;
+        pl.JR = sj * jw; pl.nlaunch2 = two192 ? 1 : L2 / pl.JR;
         ok2 = true;
       }
     }

@@ -100,11 +100,12 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
       // fixed geometry: 384, 512, 768 and 1024 queries to a launch.  (Rows of up to 256 queries at D = 32 run the one-kernel
       // backward; <8, 64, 1> and <4, 64> are theirs where fta_debug_select_kernels asks for the general kernels)
       if constexpr (DROP) {
-#define FTA_DKDV_FIX_CASE(NN, SS, WW)                                                                                            \
-  if (D == 32 && pl.threads2 == 64 * WW && pl.NJT == NN && pl.JT == 64 && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, 64, SS, WW).r && \
-      pl.nb2 == dkdv_ring(32, NN, 64, SS, WW).nb)                                                                                \
-    e = launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, NN, 64, SS, WW>, p, grid, block, pl.smem2, st);
-        FTA_DKDV_FIX_CASE(6, 2, 4) FTA_DKDV_FIX_CASE(8, 1, 8) FTA_DKDV_FIX_CASE(8, 2, 4) FTA_DKDV_FIX_CASE(6, 4, 8) FTA_DKDV_FIX_CASE(8, 4, 8)
+#define FTA_DKDV_FIX_CASE(NN, JJ, SS, WW)                                                                                        \
+  if (D == 32 && pl.threads2 == 64 * WW && pl.NJT == NN && pl.JT == JJ && pl.SJ == SS && pl.ring2 == dkdv_ring(32, NN, JJ, SS, WW).r && \
+      pl.nb2 == dkdv_ring(32, NN, JJ, SS, WW).nb)                                                                                \
+    e = launch_kernel(fta_bwd_dkdv_kernel<T, true, 32, NN, JJ, SS, WW>, p, grid, block, pl.smem2, st);
+        FTA_DKDV_FIX_CASE(5, 32, 2, 4) FTA_DKDV_FIX_CASE(6, 64, 2, 4) FTA_DKDV_FIX_CASE(8, 64, 1, 8) FTA_DKDV_FIX_CASE(8, 64, 2, 4)
+        FTA_DKDV_FIX_CASE(6, 64, 4, 8) FTA_DKDV_FIX_CASE(8, 64, 4, 8)
 #undef FTA_DKDV_FIX_CASE
       }
       if constexpr (!DROP) { FTA_DKDV_FEAT_CASE(32, 8, 64) }

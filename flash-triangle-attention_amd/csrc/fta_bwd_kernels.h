@@ -473,7 +473,7 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
 template <class T, bool DROP, int D, int NJT, int JT, int SJC = 0, int NW = 8>
 __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParams p) {
   constexpr bool FIX = (SJC != 0);
-  static_assert(!FIX || (D == 32 && JT == 64), "fixed geometry");
+  static_assert(!FIX || (D == 32 && (JT == 64 || JT == 32)), "fixed geometry");
   constexpr int G = JT / 32;                // 32-query tiles per stage (JT queries per slab and stage)
   constexpr int STEPS = NJT / G;
   constexpr int JW = NJT * 32;              // queries per wave slab
@@ -589,7 +589,7 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParam
     }
   };
   // FIX: pieces of 16 rows (one copy each), dealt to the waves; the cursors stand at the start of the row
-  constexpr int PQ = FIX ? SJC * 8 / NW : 0, PK = FIX ? 4 / (FIX ? SJC : 1) : 0;  // per wave: Q and dO pieces of a stage; K and V pieces of a row
+  constexpr int PQ = FIX ? SJC * JT / 8 / NW : 0, PK = FIX ? 4 / (FIX ? SJC : 1) : 0;  // per wave: Q and dO pieces of a stage; K and V pieces of a row
   const uint32_t crow = (uint32_t)lane >> 2, ccol = (uint32_t)swz_slot<D>(lane >> 2, lane & 3) * 16u;
   auto piece = [&](const half_t* row, uint32_t stride2, int first, uint32_t dst) {
     uint32_t cr = crow;
