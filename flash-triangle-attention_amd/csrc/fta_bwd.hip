@@ -20,7 +20,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   // H4 D32 in fp16, tiles to the next multiple of 128 and key ranges of 512 + 256 -> this (us): L 257
   // 160 -> 143, 320 194 -> 169, 385 366 -> 328, 448 435 -> 395, 513 985 -> 886, 576 1114 -> 996, 704 1859 -> 1716, 1281
   // 11160 -> 10380.
-  auto hand = [&](int lt) { pl.Lt = lt; return plan_dq1(B, H, L1, lt, D, pl.dq1) && plan_dkdv1(B, H, L1, lt, D, pl.dkdv1); };
+  auto hand = [&](int lt) { pl.Lt = lt; return plan_dq1(B, H, L1, lt, row, D, pl.dq1) && plan_dkdv1(B, H, L1, lt, D, pl.dkdv1); };
   pl.use_hand = !pl.use_short && !feat && !forced_general() && (hand((row + 63) / 64 * 64) || hand(L2));
   if (pl.use_short || pl.use_hand) {
     pl.partial_bytes = (size_t)(pl.use_short ? pl.sh.nchunks : pl.dq1.nchunks) * B * H * L2 * L2 * sizeof(float);

@@ -12,9 +12,15 @@ static int dq1_ranges(int L2, int D, int* out) {
 }
 static int dq1_slabs(int L2, int D) { return (D == 64 || L2 <= 256) ? 1 : 2; }
 
-bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl) {
+bool plan_dq1(int B, int H, int L1, int L2, int row, int D, Dq1Plan& pl) {
   if (D != 32 && D != 64) return false;
-  if (L2 % 64 != 0 || L2 < 256 || L2 > (D == 64 ? 256 : 512) * kMaxRanges) return false;
+  // D = 64: the tiles end at the row's next multiple of 32 keys, whatever length dK/dV takes (that ends with the same
+  // group of 128 queries, so the aux it reads is all written).  257 to 288 keys stay at two ranges of
+  // 160, as 128 keys are less than the shortest instance.  Training step, before -> now: 150 keys 109 -> 90 us (8 -> 5 tiles),
+  // 200 keys 128 -> 123 (8 -> 7), 2x4 heads of 400 keys 1635 -> 1580 (2 x 8 -> 7 + 6).  D = 32 pairs its slabs: 64 keys.
+  if (D == 64 && row > 128) L2 = (row > 256 && row <= 288) ? 320 : (row + 31) / 32 * 32;
+  pl.Lt = L2;
+  if (L2 % (D == 64 ? 32 : 64) != 0 || L2 < (D == 64 ? 160 : 256) || L2 > (D == 64 ? 256 : 512) * kMaxRanges) return false;
   pl.nlaunch = dq1_ranges(L2, D, pl.range);
   pl.threads = 256;
   pl.ring = (D == 64) ? 3 : 4;  // as compiled into the kernel
@@ -34,7 +40,9 @@ bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl) {
     if (pl.smem_range[n] > pl.smem) pl.smem = pl.smem_range[n];
   }
   // every launch cuts L1 into the same chunks (the dBias partial sums are indexed by chunk)
-  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, 256);  // one workgroup per CU
+  // (one workgroup per CU; short rows in chunks of fewer rows where eight would leave CUs idle, as in dK/dV: B1 H4 of 150 keys
+  // at D = 64 240 workgroups instead of 152, 200 keys 232 instead of 200: at D = 32 80.3 -> 79.4 us a training step)
+  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, 256, least_rows(L2));
   pl.rows_per_chunk = (L1 + nch - 1) / nch;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   return true;
@@ -43,7 +51,7 @@ bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl) {
 hipError_t launch_dq1(BwdParams p, const Dq1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st) {
   p.nchunks = pl.nchunks; p.rows_per_chunk = pl.rows_per_chunk;
   p.ring = pl.ring; p.nb = pl.nb;
-  p.SK = pl.SK; p.QB = pl.QB; p.nqg = pl.nqg;
+  p.SK = pl.SK; p.QB = pl.QB; p.nqg = pl.nqg; p.Lt = pl.Lt;
   const dim3 grid((unsigned)(p.B * p.H * pl.nqg * pl.nchunks));
   p.kr0 = 0;
   for (int n = 0; n < pl.nlaunch; ++n) {

@@ -142,6 +142,7 @@ struct Dq1Plan {
   int range[kMaxRanges];          // keys per launch
   size_t smem_range[kMaxRanges];
   size_t smem;                    // the largest
+  int Lt;                         // the length its tiles cover (D = 64: the next multiple of 32 keys)
 };
 struct Dkdv1Plan {
   int NJT, JR, nlaunch, nkg, nchunks, rows_per_chunk, threads;   // NJT, JR: of the first range
@@ -189,7 +190,7 @@ constexpr float kBf16PlainMaxScaleLog2 = 0.5f;
 inline bool bf16_scale_needs_split(float sm_scale) { return !(fabsf(sm_scale) * 1.4426950408889634f <= kBf16PlainMaxScaleLog2); }
 
 // Geometry of the one-wave-per-SIMD dQ/dBias kernel (256-key wave slabs).
-bool plan_dq1(int B, int H, int L1, int L2, int D, Dq1Plan& pl);
+bool plan_dq1(int B, int H, int L1, int L2, int row, int D, Dq1Plan& pl);
 hipError_t launch_dq1(BwdParams p, const Dq1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st);
 
 bool plan_short(int B, int H, int L1, int L2, int D, int feat, ShortPlan& pl);

@@ -591,6 +591,17 @@ def test_backward_tiles_in_steps_of_64(D, L2, mode):
     _compare(got, _oracle(q, k, v, b, sm, do), dtype, f"tiles of 64 {mode} D{D} L{L2}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L2", [160, 161, 255, 288, 289, 415, 449, 545, 641, 1025])
+def test_dq_at_head_dim_64_tiles_to_the_next_32_keys(L2, dtype):
+    """dQ/dBias at D = 64 ends its key tiles at the next multiple of 32, dK/dV at its own length: one tile more or less
+    than a whole range, whole rows of an odd number of tiles, the two ranges of 160 below 288, uneven ranges, and a last
+    group of 128 queries that only dK/dV reads to its end.  Chunks of fewer rows than eight at L1 = 5."""
+    print(f"case dq tiles D=64 L2={L2} {dtype}", flush=True)
+    q, k, v, b, do = _inputs(1, 2, 5, L2, 64, 44, dtype)
+    _compare(_run(q, k, v, b, 0.125, do), _oracle(q, k, v, b, 0.125, do), dtype, f"dq tiles D64 L{L2}")
+
+
 # ---- everything at once, drawn at random -------------------------------------------------------------------
 
 def test_random_draws_over_types_masks_dropout_modes_and_layouts():
