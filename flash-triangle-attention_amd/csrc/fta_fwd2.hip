@@ -24,11 +24,11 @@ namespace fta {
 // T: element type; S: key slabs per row (waves sharing a query block); TAIL: the row's true length L2 is
 // shorter than the 32*NKT*S keys the tiles cover (keys beyond it masked, K/V rows and queries beyond it
 // are copies of the last one; such queries are not stored); NKT: tiles per slab (8: slabs of 256 keys; 6: of
-// 192, for rows tiled as 384 keys).
+// 192, for rows tiled as 192 or 384 keys).
 template <class T, int S, bool TAIL, int NKT = 8>
 __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) fta_fwd2_kernel(const FwdParams p) {
   constexpr int D = 64, KS = 4, DT = 2;
-  static_assert(NKT == 8 || (NKT == 6 && S == 2), "slabs of 256 keys, or two of 192");
+  static_assert(NKT == 8 || NKT == 6, "slabs of 256 keys or of 192");
   constexpr int G = 2;                         // tiles per stage
   constexpr int KT = 32 * G;                   // keys per slab and stage
   constexpr int NST = NKT / G;                 // stages per row
@@ -531,12 +531,12 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_wav
 // ---- host side ---------------------------------------------------------------------------------
 
 bool plan_fwd2(int B, int H, int L1, int L2, int D, FwdPlan& pl) {
-  if (D != 64 || (L2 != 256 && L2 != 384 && L2 != 512)) return false;
+  if (D != 64 || (L2 != 192 && L2 != 256 && L2 != 384 && L2 != 512)) return false;
   pl = FwdPlan{};
-  pl.NKT = (L2 == 384) ? 6 : 8;
-  pl.S = (L2 == 256) ? 1 : 2;
+  pl.NKT = (L2 % 192 == 0) ? 6 : 8;
+  pl.S = (L2 <= 256) ? 1 : 2;
   pl.QB = 8 / pl.S;
-  pl.nqg = L2 / (32 * pl.QB);
+  pl.nqg = (L2 + 32 * pl.QB - 1) / (32 * pl.QB);
   pl.threads = 512;
   pl.KT = 64;
   pl.smem = (size_t)4 * pl.S * 2 * 64 * 64 * 2 + (pl.S == 2 ? 8 * (2048 + 512) : 0);  // four slots; the merge records
@@ -550,7 +550,7 @@ bool plan_fwd2(int B, int H, int L1, int L2, int D, FwdPlan& pl) {
 }
 
 hipError_t launch_fwd2(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 grid, dim3 block, hipStream_t st) {
-  const bool tl = (p.L2 != p.L2p) || p.odd_bias;
+  const bool tl = (p.L2 != p.L2p) || (p.L2p % (32 * pl.QB) != 0) || p.odd_bias;
 #define FTA_FWD2_CASE(SS, NN)                                                                           \
   if (pl.S == SS && pl.NKT == NN) {                                                                     \
     if (dtype == kBF16)                                                                                 \
@@ -560,6 +560,12 @@ hipError_t launch_fwd2(const FwdParams& p, const FwdPlan& pl, int dtype, dim3 gr
               : launch_kernel(fta_fwd2_kernel<F16, SS, false, NN>, p, grid, block, pl.smem, st);        \
   }
   FTA_FWD2_CASE(1, 8) FTA_FWD2_CASE(2, 8) FTA_FWD2_CASE(2, 6)
+  // (129 to 192 keys: six tiles instead of eight, and rows split finer over the chip, as a row of fewer keys asks for fewer rows
+  // per workgroup; the last two of the eight query blocks lie beyond the row, hence only masking instances.  Forward, fp16, us,
+  // tiled as 256 -> as 192: B1 H4 of 129 / 150 / 192 keys 27.4 / 27.2 / 28.4 -> 19.0 / 19.0 / 21.1, B4 H8 of 160 keys 136 -> 116)
+  if (pl.S == 1 && pl.NKT == 6)
+    return dtype == kBF16 ? launch_kernel(fta_fwd2_kernel<BF16, 1, true, 6>, p, grid, block, pl.smem, st)
+                          : launch_kernel(fta_fwd2_kernel<F16, 1, true, 6>, p, grid, block, pl.smem, st);
 #undef FTA_FWD2_CASE
   return hipErrorInvalidConfiguration;
 }

@@ -602,6 +602,22 @@ def test_dq_at_head_dim_64_tiles_to_the_next_32_keys(L2, dtype):
     _compare(_run(q, k, v, b, 0.125, do), _oracle(q, k, v, b, 0.125, do), dtype, f"dq tiles D64 L{L2}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L1,L2", [(7, 129), (3, 160), (4, 161), (1, 191), (9, 192)])
+def test_forward_at_head_dim_64_of_129_to_192_keys(L1, L2, dtype):
+    """One slab of six tiles: two of the eight query blocks beyond the row, whole rows, one key more than a tile; one row,
+    and chunks of unequal numbers of rows.  The keys of the first and of the last tile masked out by the bias."""
+    import fta_lib
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, 0.0, 0, 0)
+    plan = fta_lib.describe_plan(2, 2, L1, L2, 64, 0.125, opt)["fwd"]
+    assert plan["kernel"].startswith("fta_fwd2_kernel") and plan["tiled_length"] == 192
+    for masked in ((0, 0), (0, 32), (L2 - 32, L2)):
+        print(f"case D=64 {L1}x{L2} {dtype} masked {masked}", flush=True)
+        q, k, v, b, do = _inputs(2, 2, L1, L2, 64, 45, dtype)
+        b[..., masked[0]:masked[1]] = -1e4
+        _compare(_run(q, k, v, b, 0.125, do), _oracle(q, k, v, b, 0.125, do), dtype, f"D64 L{L2} masked {masked}")
+
+
 # ---- everything at once, drawn at random -------------------------------------------------------------------
 
 def test_random_draws_over_types_masks_dropout_modes_and_layouts():
