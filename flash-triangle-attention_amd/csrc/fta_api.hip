@@ -130,8 +130,8 @@ struct PlanKey {
 int padded_len_fwd(int L2, int D, int feat) {
   for (int lp = (L2 + 31) / 32 * 32; lp <= FTA_MAX_L2; lp += 32) {
     const fta::FwdPlan pl = fta::plan_fwd(1, 1, 1, lp, D, lp, feat == 2);
-    // (shapes in between: the hand-scheduled kernel's, and rows of one slab with dropout at D = 32)
-    if (pl.valid && (lp % 128 == 0 || pl.fwd1 != 0 || (feat == 2 && D == 32 && pl.S == 1 && lp % 64 == 0))) return lp;
+    // (shapes in between: the hand-scheduled kernels', the shortest at D = 64, and rows of one slab with dropout at D = 32)
+    if (pl.valid && (lp % 128 == 0 || pl.fwd1 != 0 || (D == 64 && lp < 128) || (feat == 2 && D == 32 && pl.S == 1 && lp % 64 == 0))) return lp;
   }
   return 0;
 }

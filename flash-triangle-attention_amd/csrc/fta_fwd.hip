@@ -71,7 +71,7 @@ static FwdPlan plan_fwd_slab(int B, int H, int L1, int L2, int D, int row, bool 
   // allow; two slabs of 320 or 448 keys: 2.5 against 3.6 ms at L2 = 640 and 6.4 against 9.3 ms at 896
   // with stages of 64 keys)
   int cands[6], nc = 0;
-  if (pl.NKT == 9 || pl.NKT == 15) cands[nc++] = 96;
+  if (pl.NKT == 3 || pl.NKT == 9 || pl.NKT == 15) cands[nc++] = 96;
   if (pl.NKT == 10) cands[nc++] = 160;
   if (pl.NKT == 14) cands[nc++] = 224;
   for (int kt = kt_first; kt >= 64; kt /= 2) cands[nc++] = kt;
@@ -111,10 +111,14 @@ FwdPlan plan_fwd(int B, int H, int L1, int L2, int D, int row, bool feat, bool s
   if (!feat && plan_fwd1(B, H, L1, L2, D, row, scattered, pl)) return pl;
   if (!feat && plan_fwd2(B, H, L1, L2, D, pl)) return pl;
   auto take = [&](int kw, bool wide = false) {
-    if (pl.valid || kw < 128 || (kw > kwmax && !wide) || kw % 32 != 0 || L2 % kw != 0) return;
+    if (pl.valid || kw < 64 || (kw > kwmax && !wide) || kw % 32 != 0 || L2 % kw != 0) return;
     pl = plan_fwd_slab(B, H, L1, L2, D, row, feat, kw);
   };
   auto pow2 = [](int n) { return n >= 1 && n <= 8 && (n & (n - 1)) == 0; };
+  // D=64 (not the dropout instances), rows of up to 96 keys: one slab of two or three tiles, a stage a row and a wave per query block.
+  // Forward in us, as 128 keys -> this: B1 H4 of 32 / 64 / 80 / 96 keys 9.35 / 9.2 / 9.7 / 10.1 -> 6.8 / 6.75 / 8.45 / 8.3, B4 H8 of 64
+  // 20.5 -> 14.3, of 96 in bf16 38.0 -> 32.6.
+  if (D == 64 && !feat && (L2 == 64 || L2 == 96)) take(L2);
   // 0. D=64 (not the dropout instances): slabs of up to 448 keys (14 tiles of bias still fit the registers,
   //    with a few spilled at 14) where they cut the row into two or four: fewer, wider slabs mean more
   //    query blocks behind each staged tile and longer stages

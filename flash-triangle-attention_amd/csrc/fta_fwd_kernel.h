@@ -23,7 +23,7 @@
 // that the hand-scheduled kernel takes, D = 64 up to 128 and beyond 512 keys.
 #define FTA_FWD_INSTANCES(X) \
   X(32, 12, 64) X(32, 15, 96) X(32, 16, 64) \
-  X(64, 4, 64) X(64, 8, 64) X(64, 8, 32) X(64, 10, 64) X(64, 12, 64) X(64, 12, 32) X(64, 14, 64)
+  X(64, 2, 64) X(64, 3, 96) X(64, 4, 64) X(64, 8, 64) X(64, 8, 32) X(64, 10, 64) X(64, 12, 64) X(64, 12, 32) X(64, 14, 64)
 
 // The (D, NKT) instances built with dropout (64 keys per staged tile).
 #define FTA_FWD_FEAT_INSTANCES(X) X(32, 4) X(32, 6) X(32, 8) X(32, 10) X(32, 12) X(32, 14) X(32, 16) X(64, 4) X(64, 8)
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
       bias_reg[tt][2 * rg + 1] = v[1];
     };
     if (!tail && !p.odd_bias) load_bias_tiles<NKT, 1, false, false>(bbh, p.bs[2], q0, p.L2, T::kBeyond2, turn, lane, key, T::finite2, keep);
-    else load_bias_tiles<NKT, 1, true, NKT == 4>(bbh, p.bs[2], q0, p.L2, T::kBeyond2, turn, lane, key, T::finite2, keep);
+    else load_bias_tiles<NKT, 1, true, NKT == (D == 64 && !DROP ? 2 : 4)>(bbh, p.bs[2], q0, p.L2, T::kBeyond2, turn, lane, key, T::finite2, keep);
   }
 
   // ---- global -> LDS staging of one (row, step): S slabs x KT keys of K and V, copied

@@ -618,6 +618,22 @@ def test_forward_at_head_dim_64_of_129_to_192_keys(L1, L2, dtype):
         _compare(_run(q, k, v, b, 0.125, do), _oracle(q, k, v, b, 0.125, do), dtype, f"D64 L{L2} masked {masked}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("L1,L2,tiled", [(3, 3, 64), (5, 7, 64), (2, 8, 64), (9, 33, 64), (5, 64, 64), (6, 65, 96), (1, 95, 96), (7, 96, 96),
+                                         (3, 97, 128)])
+def test_forward_at_head_dim_64_of_up_to_96_keys(L1, L2, tiled, dtype):
+    """One slab of two or three tiles, a stage a row: rows shorter than a piece of the bias, ends inside a tile and on one,
+    one row and odd numbers of rows (the buffers change places from row to row).  (Of a row of one key dQ, dK and dBias
+    are 0 whatever the inputs, and a relative error has no meaning: three keys are the shortest here.)"""
+    import fta_lib
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, 0.0, 0, 0)
+    plan = fta_lib.describe_plan(2, 3, L1, L2, 64, 0.125, opt)["fwd"]
+    assert plan["tiled_length"] == tiled
+    print(f"case D=64 {L1}x{L2} {dtype}", flush=True)
+    q, k, v, b, do = _inputs(2, 3, L1, L2, 64, 46, dtype)
+    _compare(_run(q, k, v, b, 0.125, do), _oracle(q, k, v, b, 0.125, do), dtype, f"D64 L{L2} {dtype}")
+
+
 # ---- everything at once, drawn at random -------------------------------------------------------------------
 
 def test_random_draws_over_types_masks_dropout_modes_and_layouts():
