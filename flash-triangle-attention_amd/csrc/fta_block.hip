@@ -248,6 +248,81 @@ __device__ __forceinline__ void rows8(const floatx16& acc, float (&out)[2][8]) {
     }
 }
 
+// The two runs of a lane's row on their way to memory or back.  An access of run u by all lanes takes 32 bytes out of every row, a half
+// or a quarter of the lines it touches.  So the lanes of rows r and r + 16 exchange (the second half of theirs for the first of the other's):
+// a lane then has one part of both rows, and an access takes 64 consecutive bytes of each of 16 rows.  at0, at1: the elements
+// of rows r % 16 and 16 + r % 16 where the lane half's runs begin (row_pair).
+__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {
+  auto s = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = s[0];
+  b = s[1];
+}
+__device__ __forceinline__ void row_pair(int64_t at, int64_t& at0, int64_t& at1) {
+  uint32_t lo0 = (uint32_t)at, lo1 = lo0, hi0 = (uint32_t)((uint64_t)at >> 32), hi1 = hi0;
+  swap16(lo0, lo1);
+  swap16(hi0, hi1);
+  at0 = (int64_t)((uint64_t)hi0 << 32 | lo0);
+  at1 = (int64_t)((uint64_t)hi1 << 32 | lo1);
+}
+template <bool F32>
+__device__ __forceinline__ void load_runs(const void* base, int64_t at0, int64_t at1, int lane, Frag<F32>& f0, Frag<F32>& f1) {
+  const int odd = (lane >> 4) & 1;
+  if constexpr (F32) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const uint32_t* d = static_cast<const uint32_t*>(base) + 16 * u + 4 * odd;
+      const u32x4 a = *reinterpret_cast<const u32x4*>(d + at0), b = *reinterpret_cast<const u32x4*>(d + at1);
+      Frag<F32>& f = u == 0 ? f0 : f1;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        uint32_t x = a[e], y = b[e];
+        swap16(x, y);
+        f.v[e] = __builtin_bit_cast(float, x);
+        f.v[4 + e] = __builtin_bit_cast(float, y);
+      }
+    }
+  } else {
+    const uint16_t* d = static_cast<const uint16_t*>(base) + 16 * odd;
+    const u32x4 a = *reinterpret_cast<const u32x4*>(d + at0), b = *reinterpret_cast<const u32x4*>(d + at1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t x = a[e], y = b[e];
+      swap16(x, y);
+      f0.w[e] = x;
+      f1.w[e] = y;
+    }
+  }
+}
+template <bool F32>
+__device__ __forceinline__ void store_runs(void* base, int64_t at0, int64_t at1, int lane, Frag<F32> (&f)[2]) {
+  const int odd = (lane >> 4) & 1;
+  if constexpr (F32) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      uint32_t w[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) w[e] = __builtin_bit_cast(uint32_t, f[u].v[e]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) swap16(w[e], w[4 + e]);
+      uint32_t* d = static_cast<uint32_t*>(base) + 16 * u + 4 * odd;
+      *reinterpret_cast<u32x4*>(d + at0) = u32x4{w[0], w[1], w[2], w[3]};
+      *reinterpret_cast<u32x4*>(d + at1) = u32x4{w[4], w[5], w[6], w[7]};
+    }
+  } else {
+    u32x4 a = f[0].w, b = f[1].w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t x = a[e], y = b[e];
+      swap16(x, y);
+      a[e] = x;
+      b[e] = y;
+    }
+    uint16_t* d = static_cast<uint16_t*>(base) + 16 * odd;
+    *reinterpret_cast<u32x4*>(d + at0) = a;
+    *reinterpret_cast<u32x4*>(d + at1) = b;
+  }
+}
+
 __device__ __forceinline__ floatx16 zero16() {
   floatx16 v;
 #pragma unroll
@@ -279,15 +354,12 @@ __device__ __forceinline__ uint32_t div_by_length(uint32_t q, uint32_t L, float 
 struct RowBlock {
   int b;          // batch entry (wave-uniform)
   uint32_t p;     // this lane's row: i * L + j, the last one of the batch entry beyond the end
-  bool valid;
   uint32_t i, j;
 };
 __device__ __forceinline__ RowBlock row_block(const BlockParams& p, int blk, int lane) {
   RowBlock r;
   r.b = blk / p.nper;
-  const uint32_t p0 = (uint32_t)(blk - r.b * p.nper) * 32u + (uint32_t)(lane & 31);
-  r.valid = p0 < (uint32_t)p.LL;
-  r.p = r.valid ? p0 : (uint32_t)p.LL - 1u;
+  r.p = min((uint32_t)(blk - r.b * p.nper) * 32u + (uint32_t)(lane & 31), (uint32_t)p.LL - 1u);
   r.i = div_by_length(r.p, (uint32_t)p.L, 1.0f / (float)p.L);
   r.j = r.p - r.i * (uint32_t)p.L;
   return r;
@@ -492,25 +564,29 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
     fetch(min(st + teams, ntot - 1));
   }
   __syncthreads();
-  // the tile of channels n .. n + 31 of pair row q (this lane's)
-  auto store_tile = [&](const floatx16& acc, int n, int b, int q) {
+  // the tile of channels n .. n + 31 of pair rows q0 .. q0 + 31
+  // (rows beyond the end repeat the last one, and store the same values to the same place: with no branch
+  // around the stores the waits for the next stage's loads do not have to wait for them as well)
+  auto store_tile = [&](const floatx16& acc, int n, int b, int q0) {
     const int sec = n / HD, col = n - sec * HD, h = col / p.D;
-    const int64_t off = (((int64_t)b * p.H + h) * LL + q) * p.D + (col - h * p.D) + hh * 8;
+    const int64_t off = ((int64_t)b * p.H + h) * LL * p.D + (col - h * p.D) + hh * 8;
+    const int64_t at0 = off + (int64_t)min(q0 + (lane & 15), LL - 1) * p.D, at1 = off + (int64_t)min(q0 + 16 + (lane & 15), LL - 1) * p.D;
     float y[2][8];
     rows8(acc, y);
+    if (sec == 3) {
+      Frag<F32> f[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (sec == 3) {
-        Frag<F32> f;
+      for (int u = 0; u < 2; ++u) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) y[u][e] = sigmoid<F32>(y[u][e] + bgs[col + 16 * u + 8 * hh + e]);
-        pack<A>(y[u], f);
-        store8<F32>(p.gate, off + 16 * u, f);
-      } else {
-        Frag<false> f;
-        pack<A>(y[u], f);
-        store8<false>(p.qkv[sec], off + 16 * u, f);
+        pack<A>(y[u], f[u]);
       }
+      store_runs<F32>(p.gate, at0, at1, lane, f);
+    } else {
+      Frag<false> f[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) pack<A>(y[u], f[u]);
+      store_runs<false>(p.qkv[sec], at0, at1, lane, f);
     }
   };
   [[maybe_unused]] bool bad = false;
@@ -520,9 +596,6 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
     const int b = st / nst, p0 = (st - b * nst) * TR;
 #pragma unroll
     for (int rs = 0; rs < RS; ++rs) {
-      // (rows beyond the end repeat the last one, and store the same values to the same place: with no branch
-      // around the stores the waits for the next stage's loads do not have to wait for them as well)
-      const int q = min(p0 + rs * 32 + l32, LL - 1);
       floatx16 acc[NT];
 #pragma unroll
       for (int t = 0; t < NT; ++t) acc[t] = zero16();
@@ -535,7 +608,7 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         if constexpr (F32) bad = bad || not_finite(acc[t]);
-        store_tile(acc[t], tile_of(t) * 32, b, q);
+        store_tile(acc[t], tile_of(t) * 32, b, p0 + rs * 32);
       }
       if (!F32 && wave == ((RS * it + rs) & 7)) {
         floatx16 ab = zero16();
@@ -543,6 +616,7 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
         for (int ks = 0; ks < KS; ++ks)
           ab = mma<A>(op_read<F32>(wbf, ks, lane), piece_frag<F32>(buf + rs * SUB, ks, l32, hh), ab);
         const float add = msk[(it & 1) * TR + rs * 32 + l32];
+        const int q = min(p0 + rs * 32 + l32, LL - 1);
         if (hh == 0)
 #pragma unroll
           for (int h = 0; h < 4; ++h)
@@ -568,12 +642,12 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
     if (bad)
 #pragma clang loop unroll(disable)
       for (st = st0; st < ntot; st += teams) {
-        const int b = st / nst, q = min((st - b * nst) * TR + l32, LL - 1);
+        const int b = st / nst, q0 = (st - b * nst) * TR, q = min(q0 + l32, LL - 1);
         const uint32_t i = div_by_length((uint32_t)q, (uint32_t)p.L, inv_l), j = (uint32_t)q - i * (uint32_t)p.L;
 #pragma clang loop unroll(disable)
         for (int t = 0; t < NT; ++t) {
           const int n = tile_of(t) * 32, sec = n / HD;
-          store_tile(proj_tile_f32<C>(p, b * p.zs[0] + (int64_t)i * p.zs[1] + (int64_t)j * p.zs[2], p.w[sec], (int64_t)(n - sec * HD + l32) * C, hh), n, b, q);
+          store_tile(proj_tile_f32<C>(p, b * p.zs[0] + (int64_t)i * p.zs[1] + (int64_t)j * p.zs[2], p.w[sec], (int64_t)(n - sec * HD + l32) * C, hh), n, b, q0);
         }
       }
 }
@@ -599,11 +673,12 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
   RowBlock rb = row_block(p, item / p.cg, lane);
   auto fetch = [&]() {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
+    for (int ks = 0; ks < KS; ks += 2) {
       const int h = ks * 16 / p.D;
-      const int64_t off = head_off(p, rb, h) + (ks * 16 - h * p.D) + hh * 8;
-      gt[ks] = load8<F32>(p.gate, off);
-      o[ks] = load8<false>(p.o, off);
+      int64_t at0, at1;
+      row_pair(head_off(p, rb, h) + (ks * 16 - h * p.D) + hh * 8, at0, at1);
+      load_runs<F32>(p.gate, at0, at1, lane, gt[ks], gt[ks + 1]);
+      load_runs<false>(p.o, at0, at1, lane, o[ks], o[ks + 1]);
     }
   };
   auto store_tile = [&](const floatx16& acc, int t, const RowBlock& r) {
@@ -616,7 +691,7 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
       for (int e = 0; e < 8; ++e) y[u][e] += bos[t * 32 + 16 * u + 8 * hh + e];
       Frag<F32> f;
       pack<A>(y[u], f);
-      if (r.valid) store8<F32>(p.out, oo + t * 32 + 16 * u, f);
+      store8<F32>(p.out, oo + t * 32 + 16 * u, f);  // (rows beyond the end: once more the last one)
     }
   };
   [[maybe_unused]] bool bad = false;
@@ -725,14 +800,18 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
   };
   auto head_at = [&](int t, const RowBlock& r) { const int h = t * 32 / p.D; return head_off(p, r, h) + (t * 32 - h * p.D) + hh * 8; };
   auto operands = [&](int t, const RowBlock& r, Frag<F32> (&gt)[2], Frag<false> (&o)[2]) {
-    const int64_t off = head_at(t, r);
-#pragma unroll
-    for (int u = 0; u < 2; ++u) { gt[u] = load8<F32>(p.gate, off + 16 * u); o[u] = load8<false>(p.o, off + 16 * u); }
+    int64_t at0, at1;
+    row_pair(head_at(t, r), at0, at1);
+    load_runs<F32>(p.gate, at0, at1, lane, gt[0], gt[1]);
+    load_runs<false>(p.o, at0, at1, lane, o[0], o[1]);
   };
   auto store_tile = [&](const floatx16& acc, int t, const RowBlock& r, const Frag<F32> (&gt)[2], const Frag<false> (&o)[2]) {
-    const int64_t off = head_at(t, r);
+    int64_t at0, at1;
+    row_pair(head_at(t, r), at0, at1);
     float y[2][8];
     rows8(acc, y);
+    Frag<false> fo[2];
+    Frag<F32> fd[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       float a[8], b[8], d[8];
@@ -743,15 +822,11 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
         d[e] = y[u][e] * b[e] * a[e] * (1.0f - a[e]);
         y[u][e] *= a[e];
       }
-      Frag<false> fo;
-      Frag<F32> fd;
-      pack<A>(y[u], fo);
-      pack<A>(d, fd);
-      if (r.valid) {
-        store8<false>(p.dog, off + 16 * u, fo);
-        store8<F32>(p.dgp, off + 16 * u, fd);
-      }
+      pack<A>(y[u], fo[u]);
+      pack<A>(d, fd[u]);
     }
+    store_runs<false>(p.dog, at0, at1, lane, fo);  // (rows beyond the end: once more the last one)
+    store_runs<F32>(p.dgp, at0, at1, lane, fd);
   };
   [[maybe_unused]] bool bad = false;
   [[maybe_unused]] const int item0 = item;
