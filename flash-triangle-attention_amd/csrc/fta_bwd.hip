@@ -83,19 +83,21 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   pl.KR = kr;
   pl.nlaunch = L2 / kr;
   // Dropout at D = 32, key ranges of 384 keys: four slabs of 96 keys instead of three of 128, so that the four SIMDs of a CU have
-  // as many waves each, and the query (key) blocks that hold nothing of the row have no workgroup.
+  // as many waves each, and the query (key) blocks that hold nothing of the row have no workgroup.  These are
+  // workgroups of four waves, two to a CU (see fta_bwd_feat.hip).  Four slabs of 128 keys stay in one workgroup of eight: its stages of 64
+  // keys leave no LDS for a second, and in stages of 32 keys four waves took longer (us a training step, four / eight waves in dQ/dBias:
+  // B1 H4 L400 738 / 735, L450 in bf16 953 / 931, L512 in bf16 1048 / 1020, B2 H8 L420 in bf16 2957 / 2885, B4 H8 L512 8152 / 8047).
   const bool three = (feat == 2 && D == 32 && kr == 384);
   const int nblk = (feat == 2) ? (row + 31) / 32 : nqb;
   pl.NKT = three ? 3 : 4;
   pl.SK = kr / (32 * pl.NKT);
-  const bool four = (feat == 2 && D == 32 && pl.SK == 4);  // workgroups of four waves, two to a CU (see fta_bwd_feat.hip)
-  int qb = (four ? 4 : 8) / pl.SK;
+  int qb = (three ? 4 : 8) / pl.SK;
   if (qb < 1) qb = 1;
   while (qb > 1 && nqb % qb != 0) --qb;
   pl.QB = qb;
   pl.nqg = (nblk + qb - 1) / qb;
   pl.threads = 64 * pl.SK * pl.QB;
-  const int G1 = (D == 32 && !four) ? 2 : 1;
+  const int G1 = (D == 32 && !three) ? 2 : 1;
   const int stage_rows = pl.SK * G1 * 32;
   const size_t slot1 = (size_t)2 * stage_rows * D * 2;
   const int steps1 = pl.NKT / G1;
@@ -104,9 +106,9 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   pl.ring = 0;
   for (int r = 4; r >= 3; --r) {
     const int nb = (r + steps1 - 1) / steps1;  // rows whose operand tiles can be in flight at once
-    if (r * slot1 + nb * qtile1 + part1 <= lds_max / (four ? 2 : 1)) { pl.ring = r; pl.nb = nb; pl.smem = r * slot1 + nb * qtile1 + part1; break; }
+    if (r * slot1 + nb * qtile1 + part1 <= lds_max / (three ? 2 : 1)) { pl.ring = r; pl.nb = nb; pl.smem = r * slot1 + nb * qtile1 + part1; break; }
   }
-  pl.nchunks = balanced_chunks((long)B * H * pl.nqg, L1, four ? 512 : 256, least_rows(L2));
+  pl.nchunks = balanced_chunks((long)B * H * pl.nqg, L1, three ? 512 : 256, least_rows(L2));
   pl.rows_per_chunk = (L1 + pl.nchunks - 1) / pl.nchunks;
   pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
   // ---- dK/dV kernel: query slabs of at most 256 (D=32) / 128 (D=64) queries per wave (register

@@ -10,11 +10,11 @@
 // fixed at compile time where eight waves share the row: training passes of 386 to 325 us there (dQ/dBias 118), 350 to 299
 // at B2 H4 L256 and 2.41 to 2.18 ms at B1 H8 L512 (dK/dV alone).
 //
-// Rows of 257 to 512 keys run in workgroups of four waves (one query block in four slabs, or two key blocks in two), two to a CU, whose
-// priorities change in turns (see fta_fwd1_kernel): one's products and waits run beside the other's vector part, where eight waves of one
+// Rows of 257 to 512 keys run in workgroups of four waves (dQ/dBias up to 384 keys, see plan_any_size: one query block in four
+// slabs; dK/dV: two key blocks in two), two to a CU, whose priorities change in turns (see fta_fwd1_kernel): one's products and waits run beside the other's vector part, where eight waves of one
 // workgroup meet at every stage, and a row's last group is at most one block short.  K and V, or Q and dO, are copied into LDS twice
-// as often for it.  Training steps at B1 H4, us, before and after: L270 284 / 242, L300 in bf16 318 / 274, L330 372 / 337, L384 436 / 402, L400 787 / 738,
-// L512 in bf16 1073 / 1044, B4 H8 L300 2262 / 2060; without the turns L300 302, L384 443, L512 1107.
+// as often for it.  Training steps at B1 H4, us, before and after: L270 284 / 242, L300 in bf16 318 / 274, L330 372 / 337, L384 436 / 402, L400 787 / 735,
+// L512 in bf16 1073 / 1020, B4 H8 L300 2262 / 2060; without the turns L300 302, L384 443.
 #include "fta_bwd_kernels.h"
 
 namespace fta {
@@ -65,8 +65,6 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
         if constexpr (DROP)
           if (D == 32 && pl.threads == 256 && pl.SK == 4 && pl.ring == dq_ring(32, 3, 1, 4, 4).r && pl.nb == dq_ring(32, 3, 1, 4, 4).nb)
             e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 3, 4, 4>, p, grid, block, pl.smem, st);
-      } else if (DROP && D == 32 && pl.SK == 4) {
-        if constexpr (DROP) e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 4, 0, 4>, p, grid, block, pl.smem, st);
       } else if (D == 32) {
         e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2>, p, grid, block, pl.smem, st);
       } else {

@@ -221,8 +221,7 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
   float lse_c, lse_n = 0.f, delta_c, delta_n = 0.f;
   // Four waves of known geometry (dropout, 257 to 384 keys): they form delta themselves, from O fragments fetched a row ahead, and leave the
   // row constants {lse - log2 c, delta / c}, c = 1/(1 - p), for the dK/dV kernel.  A kernel of its own in front of this one, which
-  // reads dO once more, takes 15 us at B1 H4 L300 in bf16; training steps there 275 / 262 us, L384 406 / 391.  (Four slabs of 128 keys:
-  // 1 % shorter in bf16, 2 % longer in fp16 at L450 and L512.)
+  // reads dO once more, takes 15 us at B1 H4 L300 in bf16; training steps there 275 / 262 us, L384 406 / 391.
   constexpr bool OWN = FIX && NW == 4;
   static_assert(!OWN || (DROP && D == 32), "row constants of dropout");
   [[maybe_unused]] u32x4 on[KS];
