@@ -101,7 +101,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   const int stage_rows = pl.SK * G1 * 32;
   const size_t slot1 = (size_t)2 * stage_rows * D * 2;
   const int steps1 = pl.NKT / G1;
-  const size_t part1 = (pl.SK > 1) ? (size_t)(pl.threads / 64) * 16 * (D / 32) * 64 * ((D == 32) ? 4 : 2) : 0;
+  const size_t part1 = dq_records(D, pl.SK, pl.threads / 64);
   const size_t qtile1 = (size_t)2 * pl.QB * 32 * D * 2;  // Q and dO rows of the workgroup, one L1 row
   pl.ring = 0;
   for (int r = 4; r >= 3; --r) {
@@ -136,7 +136,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
       if (jw % jt != 0) continue;  // (160 queries: stages of 32)
       const int stage_rows2 = sj * jt;
       const size_t slot2 = (size_t)2 * stage_rows2 * D * 2 + (size_t)2 * stage_rows2 * 4;
-      const size_t scratch2 = (size_t)(sj - 1) * kb * 32 * (D / 32) * 64 * 2;  // fp16 partials
+      const size_t scratch2 = dkdv_shares(D, sj, sj * kb);
       const size_t ktile2 = (size_t)2 * kb * 32 * D * 2;  // K and V rows of the workgroup, one L1 row
       const int steps2 = (jw / 32) / (jt / 32);
       for (int r = 4; r >= 3 && !ok2; --r) {

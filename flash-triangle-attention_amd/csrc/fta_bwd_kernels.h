@@ -112,9 +112,13 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
   const int QR = QB * 32;                    // query rows of the workgroup
   const int NB = FIX ? dq_ring(D, NKT, G1, SKC, NW).nb : p.nb;  // row-operand buffers (rows whose Q/dO tiles are in flight)
   half_t* qtiles = smem + R * buf_halfs;     // [NB][Q tile | dO tile], QR x D each
-  // cross-slab dQ partials: fp32 for D=32; fp16 for D=64, where fp32 would not fit in LDS
-  typedef typename std::conditional<D == 32, float, half_t>::type part_t;
-  part_t* scratch = reinterpret_cast<part_t*>(qtiles + NB * 2 * QR * D);
+  // cross-slab dQ partials, fp32.  D = 64: without the groups of four registers that a wave finishes itself, for which LDS has no
+  // room beside three stages of four slabs (48 KB of records instead of 64, 160 KB in all); group g of slab s is in
+  // place g / SK * (SK - 1) + (g - s - 1) % SK.  (In fp16, as they were there, bf16 gradients beyond 65504 came out infinite, and half of
+  // those near 6e-8 was lost.)
+  constexpr int RECORD = dq_record_regs(D) * 64;  // floats of a wave
+  float* scratch = reinterpret_cast<float*>(qtiles + NB * 2 * QR * D);
+  auto wrap = [&](int n) { return n < 0 ? n + SK : n; };
   FragOffsets<D> fo;
   fo.init(lane);
 
@@ -357,11 +361,17 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
       }
       if (t == STEPS - 1 && SK > 1) {
         // every slab publishes its partial dQ^T tile: scratch[wave][register][lane]
-        part_t* mine = scratch + (size_t)wave * (16 * DT * 64) + lane;
+        float* mine = scratch + (size_t)wave * RECORD + lane;
+        int turn = 0, ph = 0;  // D = 64: gi / SK * (SK - 1) and gi % SK
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int gi = 0; gi < 4 * DT; ++gi) {
+          if (D == 32 || ph != slab) {
+            float* at = mine + (D == 32 ? gi : turn + wrap(ph - slab - 1)) * 256;
 #pragma unroll
-          for (int r = 0; r < 16; ++r) mine[(dt * 16 + r) * 64] = (part_t)acc[dt][r];
+            for (int e = 0; e < 4; ++e) at[e * 64] = acc[gi / 4][(gi % 4) * 4 + e];
+          }
+          if (++ph == SK) { ph = 0; turn += SK - 1; }
+        }
       }
       // (the next row's constants are waited for here, where everything in flight is due at this step's end: at the row's end the
       // compiler would wait for the stores of dQ, too, and for every copy)
@@ -398,6 +408,7 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
     // dQ: the SK slab waves of a query block each finish a share of the 8-byte output groups
     half_t* dqr = dqbase + (int64_t)(i0 + ir) * p.dqs[2] + (int64_t)(q0 + l32) * p.dqs[3] + 4 * hh;
     const bool qreal = (q0 + l32 <= last);
+    int turn = 0;  // D = 64: gi / SK * (SK - 1) of the groups below
     if (SK == 1) {
       // One slab: the wave has the whole row.  The two lanes of a query hold alternating runs of four d
       // values; one exchange per register pair gives each eight consecutive ones, and the row goes out in
@@ -431,9 +442,14 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
 #pragma unroll
         for (int e = 0; e < 4; ++e) v4[e] = 0.f;
         for (int s2 = 0; s2 < SK; ++s2) {
-          const part_t* o2 = scratch + (size_t)(qb * SK + s2) * (16 * DT * 64) + (gi * 4) * 64 + lane;
+          const float* o2 = scratch + (size_t)(qb * SK + s2) * RECORD + (D == 32 ? gi : turn + wrap(slab - s2 - 1)) * 256 + lane;
+          if (D == 64 && s2 == slab) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v4[e] += (float)o2[e * 64];
+            for (int e = 0; e < 4; ++e) v4[e] += acc[gi / 4][(gi % 4) * 4 + e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v4[e] += o2[e * 64];
+          }
         }
       } else {
 #pragma unroll
@@ -451,6 +467,7 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
         u32x2 w = {T::pack(v4[0], v4[1]), T::pack(v4[2], v4[3])};
         *dst = w;
       }
+      turn += SK - 1;
     }
   }
 
@@ -503,8 +520,10 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParam
   const int KR2 = KB * 32;                   // key rows of the workgroup
   const int NB = FIX ? dkdv_ring(D, NJT, JT, SJC, NW).nb : p.nb2;                      // row-operand buffers (rows whose K/V tiles are in flight)
   half_t* ktiles = smem + R * slot_halfs;    // [NB][K tile | V tile], KR2 x D each
-  typedef typename std::conditional<dkdv_share_bytes(NJT, SJC) == 4, float, half_t>::type Share;
-  Share* scratch = reinterpret_cast<Share*>(ktiles + NB * 2 * KR2 * D);  // cross-slab dK/dV partials, in fp16 where they would not fit in LDS
+  // cross-slab dK/dV partials, fp32.  (In fp16, as they were, bf16 gradients beyond 65504 came out infinite, and half of those near
+  // 6e-8 was lost.  Steps with dropout at B1 H4, us, fp16 / fp32: D = 32 of 384 keys 393 / 394, 1024 8448 / 8320, D = 64 of 384 keys in bf16 1224 /
+  // 1121, of 512, which is left with three stages instead of four, 2024 / 2060.)
+  float* scratch = reinterpret_cast<float*>(ktiles + NB * 2 * KR2 * D);
   FragOffsets<D> fo;
   fo.init(lane);
 
@@ -749,9 +768,9 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParam
       }
       if (PAIRX && t == STEPS - 1) {
         // two query slabs per key block: each wave finishes half of the dK/dV accumulator groups
-        // (4 rows each; group 2x + jslab) and hands the other half, as fp16, to its partner; the
+        // (4 rows each; group 2x + jslab) and hands the other half to its partner; the
         // barrier that ends this stage publishes them
-        u32x2* out = reinterpret_cast<u32x2*>(scratch) + (size_t)wave * (4 * DT * 64) + lane;
+        float4* out = reinterpret_cast<float4*>(scratch) + (size_t)wave * (4 * DT * 64) + lane;
 #pragma unroll
         for (int x = 0; x < 4 * DT; ++x) {
           float a[4], c[4];
@@ -763,7 +782,7 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParam
             keep[4 * x + e] = jslab ? c[e] : a[e];
             a[e] = jslab ? a[e] : c[e];
           }
-          out[x * 64] = u32x2{pack_rn(a[0], a[1]), pack_rn(a[2], a[3])};
+          out[x * 64] = float4{a[0], a[1], a[2], a[3]};
         }
       }
       const int nxt = sidx + 1 + ahead;
@@ -791,14 +810,16 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParam
     });
 
     if (PAIRX) {
-      const u32x2* in = reinterpret_cast<const u32x2*>(scratch) + (size_t)(wave ^ 1) * (4 * DT * 64) + lane;
+      const float4* in = reinterpret_cast<const float4*>(scratch) + (size_t)(wave ^ 1) * (4 * DT * 64) + lane;
       half_t* dkr = dkbase + (int64_t)(i0 + ir) * p.dks[2] + (int64_t)(k0 + l32) * p.dks[3] + 4 * hh + 8 * jslab;
       half_t* dvr = dvbase + (int64_t)(i0 + ir) * p.dvs[2] + (int64_t)(k0 + l32) * p.dvs[3] + 4 * hh + 8 * jslab;
 #pragma unroll
       for (int x = 0; x < 4 * DT; ++x) {
-        const u32x2 w = in[x * 64];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) keep[4 * x + e] += (float)as_half2(w[e >> 1])[e & 1];
+        const float4 w = in[x * 64];
+        keep[4 * x] += w.x;
+        keep[4 * x + 1] += w.y;
+        keep[4 * x + 2] += w.z;
+        keep[4 * x + 3] += w.w;
       }
 #pragma unroll
       for (int x = 0; x < 2 * DT; ++x)
@@ -826,25 +847,25 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParam
       // sum the query slabs of one key block through LDS (own region; the next row's stage
       // barriers separate these reads from the next row's writes)
       if (jslab != 0) {
-        Share* mine = scratch + ((size_t)(kb * (SJ - 1) + jslab - 1) * 32 * DT) * 64 + lane;
+        float* mine = scratch + ((size_t)(kb * (SJ - 1) + jslab - 1) * 32 * DT) * 64 + lane;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            mine[(dt * 32 + r) * 64] = (Share)dk[dt][r];
-            mine[(dt * 32 + 16 + r) * 64] = (Share)dv[dt][r];
+            mine[(dt * 32 + r) * 64] = dk[dt][r];
+            mine[(dt * 32 + 16 + r) * 64] = dv[dt][r];
           }
       }
       __syncthreads();
       if (jslab == 0) {
         for (int s2 = 1; s2 < SJ; ++s2) {
-          const Share* o2 = scratch + ((size_t)(kb * (SJ - 1) + s2 - 1) * 32 * DT) * 64 + lane;
+          const float* o2 = scratch + ((size_t)(kb * (SJ - 1) + s2 - 1) * 32 * DT) * 64 + lane;
 #pragma unroll
           for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-              dk[dt][r] += (float)o2[(dt * 32 + r) * 64];
-              dv[dt][r] += (float)o2[(dt * 32 + 16 + r) * 64];
+              dk[dt][r] += o2[(dt * 32 + r) * 64];
+              dv[dt][r] += o2[(dt * 32 + 16 + r) * 64];
             }
         }
       }

@@ -210,7 +210,9 @@ constexpr Ring fit_ring(int steps, int slot, int row, int records, int waves) {
   }
   return Ring{0, 0};
 }
-constexpr int dq_records(int D, int SK, int waves) { return SK > 1 ? waves * 16 * (D / 32) * 64 * (D == 32 ? 4 : 2) : 0; }
+// (registers of its partial dQ that a wave publishes to the other slabs: all, at D = 64 those that they finish, of up to four slabs three quarters)
+constexpr int dq_record_regs(int D) { return D == 32 ? 16 : 24; }
+constexpr int dq_records(int D, int SK, int waves) { return SK > 1 ? waves * dq_record_regs(D) * 64 * 4 : 0; }
 constexpr Ring dq_ring(int D, int NKT, int G1, int SK, int waves) {
   return fit_ring(NKT / G1, 4 * SK * G1 * 32 * D, 4 * (waves / SK) * 32 * D, dq_records(D, SK, waves), waves);
 }
@@ -218,16 +220,14 @@ constexpr size_t dq_smem(int D, int NKT, int G1, int SK, int waves) {
   const Ring r = dq_ring(D, NKT, G1, SK, waves);
   return (size_t)r.r * (4 * SK * G1 * 32 * D) + (size_t)r.nb * (4 * (waves / SK) * 32 * D) + dq_records(D, SK, waves);
 }
-// (the slabs' shares of dK and dV are exchanged in fp16, of four slabs of 192 queries in fp32, for which LDS has room)
-constexpr int dkdv_share_bytes(int NJT, int SJ) { return NJT == 6 && SJ == 4 ? 4 : 2; }
-constexpr int dkdv_shares(int D, int NJT, int SJ, int waves) { return (SJ - 1) * (waves / SJ) * 32 * (D / 32) * 64 * dkdv_share_bytes(NJT, SJ); }
+constexpr int dkdv_shares(int D, int SJ, int waves) { return (SJ - 1) * (waves / SJ) * 32 * (D / 32) * 64 * 4; }
 constexpr Ring dkdv_ring(int D, int NJT, int JT, int SJ, int waves) {
-  return fit_ring(NJT / (JT / 32), 4 * SJ * JT * D + 8 * SJ * JT, 4 * (waves / SJ) * 32 * D, dkdv_shares(D, NJT, SJ, waves), waves);
+  return fit_ring(NJT / (JT / 32), 4 * SJ * JT * D + 8 * SJ * JT, 4 * (waves / SJ) * 32 * D, dkdv_shares(D, SJ, waves), waves);
 }
 
 constexpr size_t dkdv_smem(int D, int NJT, int JT, int SJ, int waves) {
   const Ring r = dkdv_ring(D, NJT, JT, SJ, waves);
-  return (size_t)r.r * (4 * SJ * JT * D + 8 * SJ * JT) + (size_t)r.nb * (4 * (waves / SJ) * 32 * D) + dkdv_shares(D, NJT, SJ, waves);
+  return (size_t)r.r * (4 * SJ * JT * D + 8 * SJ * JT) + (size_t)r.nb * (4 * (waves / SJ) * 32 * D) + dkdv_shares(D, SJ, waves);
 }
 
 // One key range and one query range of the backward with dropout beyond 512 keys (D = 32): stage and row-operand

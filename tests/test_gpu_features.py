@@ -634,6 +634,44 @@ def test_forward_at_head_dim_64_of_up_to_96_keys(L1, L2, tiled, dtype):
     _compare(_run(q, k, v, b, 0.125, do), _oracle(q, k, v, b, 0.125, do), dtype, f"D64 L{L2} {dtype}")
 
 
+# ---- magnitudes of bf16 gradients -------------------------------------------------------------------------
+
+def _check_gradients_scale_with_dout(q, k, v, b, sm, do, *extra):
+    """The gradients are linear in dO, and bf16 has the exponents of fp32: dO times a power of two scales every product and sum
+    exactly, so the gradients are the same bits but for their exponent (a mean over a long pair tensor leaves some of 1e-8, and less).
+    Weights near 2^-126 times a small dO vanish: less than 2^-126 of each of L2 products with factors of up to 2^6."""
+    want = _run(q, k, v, b, sm, do, *extra)
+    for e in (-40, -24, 20, 40):
+        got = _run(q, k, v, b, sm, do * 2.0 ** e, *extra)
+        for n in ("dq", "dk", "dv", "db"):
+            off = (got[n].double() - want[n].double() * 2.0 ** e).abs().max().item()
+            assert off <= k.shape[3] * 2.0 ** -120, f"{n} at 2^{e}: {orc.rel_l2(got[n].double() * 2.0 ** -e, want[n].double()):.2e}"
+
+
+@pytest.mark.parametrize("D,L2,sm,p", [
+    (32, 300, 0.17, 0.15), (32, 384, 0.17, 0.15), (32, 450, 1.3, 0.15), (32, 600, 0.17, 0.15), (32, 768, 0.17, 0.15), (32, 1000, 0.17, 0.15),
+    (32, 1408, 0.17, 0.15), (64, 100, 0.17, 0.15), (64, 150, 0.17, 0.15), (64, 300, 0.17, 0.15), (64, 512, 0.17, 0.15), (64, 600, 0.17, 0.15),
+    (64, 200, 1.3, 0.0), (64, 384, 1.3, 0.0), (64, 500, 1.3, 0.0), (64, 1024, 1.3, 0.0)])
+def test_bf16_gradients_of_any_magnitude_from_the_general_kernels(D, L2, sm, p):
+    """Shares of dQ, dK and dV that slabs hand to each other, in every number of slabs."""
+    print(f"case magnitudes D={D} L2={L2} sm={sm} p={p}", flush=True)
+    q, k, v, b, do = _inputs(1, 2, 3, L2, D, 61, torch.bfloat16)
+    _check_gradients_scale_with_dout(q, k, v, b, sm, do, *((p, 7) if p else ()))
+
+
+@pytest.mark.parametrize("D,L2", [(32, 384), (32, 512), (32, 640), (32, 1024), (64, 256), (64, 384), (64, 512)])
+def test_bf16_gradients_of_any_magnitude_from_the_general_kernels_at_every_scale(D, L2):
+    import fta_lib
+    lib = fta_lib.load()
+    print(f"case magnitudes D={D} L2={L2} general", flush=True)
+    q, k, v, b, do = _inputs(1, 2, 3, L2, D, 62, torch.bfloat16)
+    before = lib.fta_debug_select_kernels(3)
+    try:
+        _check_gradients_scale_with_dout(q, k, v, b, 0.17, do)
+    finally:
+        lib.fta_debug_select_kernels(before)
+
+
 # ---- everything at once, drawn at random -------------------------------------------------------------------
 
 def test_random_draws_over_types_masks_dropout_modes_and_layouts():
