@@ -9,7 +9,7 @@
 //   * bias^T (fp16, times log2(e)) sits in accumulation registers as MFMA A operands for the whole
 //     L1 chunk (8 registers per tile) and is added to the scores by the matrix core;
 //   * the row constants -lse and -delta are read from LDS as they are stored (one 8-byte pair per
-//     query) and added by one extra contraction step each: the B operand is {2048, 1} on the two
+//     query) and added by one extra contraction step each: the B operand is {2048, 1} (-delta in bf16: {1, 1}) on the two
 //     contraction slots where the A operand carries the constant's (hi, lo) halves, zero elsewhere,
 //     so no vector-ALU instruction prepares them;
 //   * the walk over the tiles of a row is software-pipelined two tiles deep: iteration j issues the
@@ -203,22 +203,18 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       }
   }
   // constant B operands: the one-hot selectors that route contraction slot s of step u to key column
-  // 16u + s, and the {2048, 1} pairs that pick up the (hi, lo) halves of -lse (words 0 of the
-  // constant pair: slots 0, 1) and of -delta (word 1: slots 2, 3); only the lanes 0..31 own those slots
+  // 16u + s, and the pairs of factors that pick up the halves of -lse (words 0 of the
+  // constant pair: slots 0, 1) and of -delta (word 1: slots 2, 3; see aug_ones); only the lanes 0..31 own those slots
   u32x4 Eb[2], onesS, onesD;
   {
-    half8_t eb[2], os, od;
+    half8_t eb[2];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int x = 0; x < 8; ++x) eb[u][x] = (16 * u + 8 * hh + x == l32) ? (half_t)1.0f : (half_t)0.0f;
-#pragma unroll
-    for (int x = 0; x < 8; ++x) {
-      os[x] = (hh == 0 && x == 0) ? (half_t)2048.0f : (hh == 0 && x == 1) ? (half_t)1.0f : (half_t)0.0f;
-      od[x] = (hh == 0 && x == 2) ? (half_t)2048.0f : (hh == 0 && x == 3) ? (half_t)1.0f : (half_t)0.0f;
-    }
     Eb[0] = __builtin_bit_cast(u32x4, eb[0]); Eb[1] = __builtin_bit_cast(u32x4, eb[1]);
-    onesS = __builtin_bit_cast(u32x4, os); onesD = __builtin_bit_cast(u32x4, od);
+    onesS = u32x4{hh == 0 ? kLseOnes : 0u, 0u, 0u, 0u};
+    onesD = u32x4{0u, hh == 0 ? T::kDeltaOnes : 0u, 0u, 0u};
   }
   // (opaque, settled operands)
   asm volatile("s_nop 1" : "+v"(Eb[0]), "+v"(Eb[1]), "+v"(onesS), "+v"(onesD));
@@ -401,7 +397,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
     mfma_rf<F16, kA, kV, kV, 0>(s_cur, biasA[0][0], Eb[0]);
     mfma_rf<F16, kA, kV, kV, 0>(s_cur, biasA[0][1], Eb[1]);
     mfma_rf<F16, kV, kV, kV, 1>(s_cur, cst, onesS);
-    mfma_rf<F16, kV, kV, kV, 1>(dp_cur, cst, onesD);
+    mfma_rf<T, kV, kV, kV, 1>(dp_cur, cst, onesD);
     asm volatile("s_nop 15\n\ts_nop 7" : "+v"(s_cur), "+v"(dp_cur));  // results land before anything reads them
     // operands of tile 1, settled here so that the loop's waits need not cover them
 #pragma unroll
@@ -628,7 +624,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       });
       mfma_rf<F16, kA, kV, kV, 0>(s_nxt, biasA[gn][0], Eb[0]);
       after(std::integral_constant<int, NM2 + PS * KS>{});
-      mfma_rf<F16, kV, kV, kV, 0>(dp_nxt, cstn, onesD);
+      mfma_rf<T, kV, kV, kV, 0>(dp_nxt, cstn, onesD);
       after(std::integral_constant<int, NM2 + PS * KS + 1>{});
       mfma_rf<F16, kA, kV, kV, 0>(s_nxt, biasA[gn][1], Eb[1]);
       after(std::integral_constant<int, NM2 + PS * KS + 2>{});

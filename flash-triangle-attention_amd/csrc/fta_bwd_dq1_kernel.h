@@ -349,13 +349,13 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
     }
   };
 
-  half8_t ones = aug_ones();
+  half8_t ones = aug_ones<T>();
   asm volatile("" : "+v"(ones));  // kept in registers: not re-created in front of each use
 
   // operands of one row: Q and dO fragments of this wave's query block and the packed constants
   half8_t qf[KS], dof[KS], qf_n[KS], dof_n[KS];
   half8_t ql[HL ? KS : 1], ql_n[HL ? KS : 1];  // (HL) what the rounding of the scaled Q dropped
-  // (the packed constants sit in slot 0 of the lanes 0..31 of an otherwise zero B operand; the
+  // (the packed constants sit in one word of the lanes 0..31 of an otherwise zero B operand; the
   // operands are built once per row and made opaque, so that no instruction rewrites them right
   // in front of the MFMA that reads them)
   u32x4 augS, augD, augS_n = {0u, 0u, 0u, 0u}, augD_n = {0u, 0u, 0u, 0u};
@@ -387,7 +387,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
     // (a query beyond L2 gets the constant that makes its weights exactly 0 in both backward kernels)
     // (lse is stored as a base-2 logarithm)
     const float nl = qvalid ? (NAT ? -lse_n * 0.6931471805599453f : folded_lse(lse_n)) : kBiasFloorLog2, nd = -sum_both_halves(dpart);
-    const uint32_t ws = split_2048(nl), wd = split_2048(nd);
+    const uint32_t ws = split_2048(nl), wd = T::delta_pair(nd);
     // the dK/dV kernel takes the constants from here (the look-ahead past the chunk's last row
     // works on the last row again and stores the same values once more)
     if (ir > 0 && ir < nrows) advance(auxcur, step_aux);
@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
       asm volatile("s_nop 1" : "+v"(cS), "+v"(cD));
     } else {
       as = u32x4{hh ? 0u : ws, 0u, 0u, 0u};
-      ad = u32x4{hh ? 0u : wd, 0u, 0u, 0u};
+      ad = u32x4{0u, hh ? 0u : wd, 0u, 0u};
       asm volatile("" : "+v"(as), "+v"(ad));
     }
   };
@@ -481,7 +481,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
     mfma_acc_v_ba(s_cur, E[1], bias4[0][1]);
     if constexpr (!CIN) {
       mfma_acc_v_late(s_cur, ones, as_half8(augS));
-      mfma_acc_v_late(dp_cur, ones, as_half8(augD));
+      mfma_acc_v_late<T>(dp_cur, ones, as_half8(augD));
     }
     asm volatile("s_nop 15\n\ts_nop 7" : "+v"(s_cur), "+v"(dp_cur));  // results land before anything reads them
 #pragma unroll
@@ -799,7 +799,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
       } else {
         mfma_acc_v_ba(s_nxt, E[0], bias4[gn][0]);
         after(std::integral_constant<int, NM2 + 2 * KS>{});
-        mfma_acc_v(dp_nxt, ones, as_half8(ad));
+        mfma_acc_v<T>(dp_nxt, ones, as_half8(ad));
         after(std::integral_constant<int, NM2 + 2 * KS + 1>{});
         mfma_acc_v_ba(s_nxt, E[1], bias4[gn][1]);
         after(std::integral_constant<int, NM2 + 2 * KS + 2>{});

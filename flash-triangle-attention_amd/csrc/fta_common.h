@@ -32,12 +32,15 @@ __device__ __forceinline__ floatx16 mfma32(half8_t a, half8_t b, floatx16 c) {
 
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// MFMA operand {2048, 1, 0, ..., 0} on contraction slots 0 and 1: with the other operand holding
-// split_2048(c) on the same slots (and zeros on slots 8..15, which the lanes 32..63 own), one extra
-// 16-wide contraction step adds the constant c to every element of the accumulator column/row.
+// Row constants -lse and -delta that enter through the matrix core: one extra 16-wide contraction step adds the constant c to every
+// element of an accumulator column or row, with c as a pair of 16-bit values on two contraction slots of one operand and
+// their factors on the same slots of the other, zeros elsewhere.  -lse: split_2048(c), fp16 for every element type, against {2048, 1} on
+// slots 0 and 1.  -delta has the range of the incoming gradient: T::delta_pair(c) against T::kDeltaOnes on slots 2 and 3, through
+// T's MFMA.  (Either pair meets zeros of the other's step: a finite fp16 is finite read as bf16, a bf16 below 2^121 read as fp16.)
+constexpr uint32_t kLseOnes = 0x3C006800u;
+template <class T>
 __device__ __forceinline__ half8_t aug_ones() {
-  half8_t v = {(_Float16)2048.0f, (_Float16)1.0f, 0, 0, 0, 0, 0, 0};
-  return v;
+  return __builtin_bit_cast(half8_t, u32x4{kLseOnes, T::kDeltaOnes, 0u, 0u});
 }
 
 // Two floats -> packed fp16 pair (round toward zero), as raw bits.
@@ -113,7 +116,7 @@ __device__ __forceinline__ half8_t scale_half8(half8_t x, float f) {
 }
 
 // c = 2048*hi + lo with hi, lo fp16: about 22 significant bits over the range |c| < 1.3e8.
-// Returned as the packed pair (hi in the low half); the matching MFMA operand is aug_ones().
+// Returned as the packed pair (hi in the low half); the matching MFMA operand holds {2048, 1}.
 __device__ __forceinline__ uint32_t split_2048(float c) {
   const half_t hi = (half_t)(c * (1.0f / 2048.0f));
   const half_t lo = (half_t)__builtin_fmaf(-2048.0f, (float)hi, c);
@@ -203,6 +206,9 @@ struct F16 {
   }
   // 1 / (what the fp16 bit pattern of 1.0 is worth as an operand of this type's MFMA)
   static constexpr float kOneHotInv = 1.0f;
+  // -delta as a pair for the matrix core, and the pair of its factors (see aug_ones)
+  static __device__ __forceinline__ uint32_t delta_pair(float c) { return split_2048(c); }
+  static constexpr uint32_t kDeltaOnes = kLseOnes;
   // Element-wise sum of two packed pairs, rounded once (what adding in fp32 and rounding gives too).
   static __device__ __forceinline__ uint32_t add2(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, as_half2(a) + as_half2(b));
@@ -281,6 +287,14 @@ struct BF16 {
   // The one-hot selectors are shared with the fp16 MFMAs that add the bias: fp16 1.0 = 0x3C00, which a
   // bf16 MFMA reads as 2^-7 exactly.  Sums taken through such a selector are scaled back by 128.
   static constexpr float kOneHotInv = 128.0f;
+  // -delta as hi + lo in bf16: 17 significant bits at every magnitude.  (As split_2048's fp16 pair a delta below 2^-8 kept fewer, one near
+  // 6e-8 none, and one beyond 1.3e8 was infinite: with dO of 6e-8 dK was off by 5 %, at D = 64 dQ and dBias, too.  At unit dO the
+  // gradients' errors against 64 bits are the same, means of 96 inputs within 2e-5 of each other; so are the times.)
+  static __device__ __forceinline__ uint32_t delta_pair(float c) {
+    const uint32_t h = pack(c, 0.0f);
+    return pack(lo(h), c - lo(h));
+  }
+  static constexpr uint32_t kDeltaOnes = 0x3F803F80u;
   static __device__ __forceinline__ uint32_t add2(uint32_t a, uint32_t b) { return pack(lo(a) + lo(b), hi(a) + hi(b)); }
 };
 

@@ -672,6 +672,17 @@ def test_bf16_gradients_of_any_magnitude_from_the_general_kernels_at_every_scale
         lib.fta_debug_select_kernels(before)
 
 
+@pytest.mark.parametrize("D,L2,sm", [(32, 200, 0.17), (32, 256, 1.3), (32, 383, 0.17), (32, 512, 0.17), (32, 512, 1.3), (32, 700, 0.17), (32, 1100, 1.3),
+                                     (64, 150, 0.17), (64, 256, 0.17), (64, 401, 0.17), (64, 1024, 0.17)])
+def test_bf16_gradients_of_any_magnitude_from_the_hand_scheduled_kernels(D, L2, sm):
+    """Delta, which the matrix core adds as a pair of 16-bit values."""
+    import fta_lib
+    assert "dq1" in fta_lib.describe_plan(1, 2, 3, L2, D, sm, fta_lib.Options(fta_lib.DTYPE_BF16, 0, 0.0, 0, 0))["dq"]["kernel"]
+    print(f"case magnitudes D={D} L2={L2} sm={sm}", flush=True)
+    q, k, v, b, do = _inputs(1, 2, 3, L2, D, 63, torch.bfloat16)
+    _check_gradients_scale_with_dout(q, k, v, b, sm, do)
+
+
 # ---- everything at once, drawn at random -------------------------------------------------------------------
 
 def test_random_draws_over_types_masks_dropout_modes_and_layouts():
