@@ -1168,7 +1168,7 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
     }
   };
   // forms operand B (gate * o, or the normalised row: the lanes of a row are neighbours) and writes both to LDS;
-  // rows beyond the end are zero in operand B
+  // rows beyond the end are zero in both
   [[maybe_unused]] float csum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // (fp32) of this thread's columns of operand A
   [[maybe_unused]] float dsum = 0.f;                                            // of this thread's dbias entry
   auto put = [&](char* buf, int st) {
@@ -1187,8 +1187,9 @@ __device__ __forceinline__ void wgrad_body(const BlockParams& p, int sec, int ch
     if constexpr (BIAS) {
       const int h = tid / TR;
       if (h < p.H) {
-        reinterpret_cast<uint16_t*>(buf + ABYTES + NB * SUB)[h * DROW + tid % TR] = rd;
-        dsum += tid % TR < left ? A::lo((uint32_t)rd) : 0.f;
+        const uint16_t d = tid % TR < left ? rd : (uint16_t)0;  // (an infinite one times operand B's zeros would be NaN)
+        reinterpret_cast<uint16_t*>(buf + ABYTES + NB * SUB)[h * DROW + tid % TR] = d;
+        dsum += A::lo((uint32_t)d);
       }
     }
 #pragma unroll
@@ -1541,7 +1542,7 @@ hipError_t launch_block_dx(BlockParams p, int C, int dtype, hipStream_t st) {
 }
 
 hipError_t launch_block_wgrad(BlockParams p, int C, int dtype, hipStream_t st) {
-  // (the largest section: both operands C or HD columns wide; the bias section has one row per head)
+  // (the largest section: both operands C or HD columns wide, and a row of dbias per head)
   const int n = (p.HD + C) / 32;
   // (fp32: one stage of three planes)
   const size_t smem = dtype == 2 ? (size_t)n * 3 * 32 * 64 + wgrad_bias_bytes(32) : (size_t)2 * (n * 64 * 64 + wgrad_bias_bytes(64));

@@ -1,6 +1,8 @@
 """The AlphaFold2 triangle-attention block around attention(): the pure-PyTorch form of the block on
 the CPU (structure, ending = starting on the transposed pair tensor, key mask), and on the GPU the
 block with the HIP kernels against that form, outputs and every gradient."""
+import math
+
 import pytest
 import torch
 
@@ -321,6 +323,40 @@ def test_infinities_of_an_fp32_block_come_out_as_they_went_in(where, B, L, C, H,
     for name, a, b in zip(["out", "z", *(n for n, _ in fused.named_parameters())], *res):
         if where != "gradient" or name in ("out", "z", "linear_o.weight", "linear_o.bias"):
             _same_values(a, b, 1e-3, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("B,L,C,H,D", [(1, 33, 128, 4, 32), (2, 41, 64, 2, 32), (1, 35, 128, 2, 64), (1, 40, 128, 4, 32)])
+def test_an_infinite_bias_gradient_of_the_last_pair_makes_infinite_weight_gradients(B, L, C, H, D, dtype):
+    """The bias gradient, fp16, overflows at the last pair alone (every row adds to it, and its softmax weight, half, is that of all
+    other keys together).  The bias weights' gradient is then infinite wherever norm weight * xhat and norm bias agree in sign, also where
+    the pairs do not fill the last stage of 64 (32 in fp32) rows, which repeats the last pair."""
+    torch.manual_seed(8)
+    blk = TriangleAttention(C, D, H).to("cuda:0", dtype)
+    z = 0.01 * torch.randn(B, L, L, C, device="cuda:0")
+    z[:, :, L - 1, 1] = 6.0       # this key's value, the same in every row
+    z[:, L - 1, L - 1, 0] = 6.0   # the last pair's bias
+    with torch.no_grad():
+        for lin in (blk.linear_q, blk.linear_k, blk.linear_v, blk.linear_b):
+            lin.weight.zero_()
+        x0 = torch.nn.functional.layer_norm(z[0, L - 1, L - 1].double(), (C,))[0].item()
+        blk.linear_b.weight[:, 0] = math.log(L - 1.0) / (x0 + 1.0)  # (beside the other pairs' bias of about -1 times the same)
+        blk.linear_v.weight[:, 1] = 1.0
+        blk.layer_norm.bias.fill_(-1.0)
+        blk.linear_g.weight.zero_()
+        blk.linear_o.weight.copy_(torch.eye(C, H * D))
+    zz = z.to(dtype).requires_grad_(True)
+    out = blk(zz)
+    dout = torch.zeros_like(out)
+    dout[:, :, L - 1] = 300.0
+    wb, wv = torch.autograd.grad(out, (blk.linear_b.weight, blk.linear_v.weight), dout)
+    torch.cuda.synchronize()
+    assert blk._fused(zz, None, None) is not None
+    assert bool(wv.isfinite().all())
+    live = (C + D - 1) // D  # heads that the output projection reads
+    assert bool((wb[:live, 2:] == -float("inf")).all()), wb
+    assert bool(wb[live:].isfinite().all())
 
 
 @pytest.mark.gpu
