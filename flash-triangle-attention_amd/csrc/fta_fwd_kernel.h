@@ -199,14 +199,15 @@ __global__ void __launch_bounds__(512) fta_fwd_kernel(const FwdParams p) {
 
 #pragma unroll
     for (int t = 0; t < STEPS; ++t) {
-      // Workgroups of less than eight waves share the SIMDs: a wave's priority falls from half row to half row, in turns of two
-      // rows, so that the older workgroup does not run ahead (see fta_fwd1_kernel): with dropout B1 H4 L300 76 against 70 us, L450 a
-      // training step 960 / 935, without at D = 64 B4 H8 L100 40.2 / 39.2.  (Eight waves in one workgroup: up to 2 % slower.)
-      if (nthreads < 512 && t == 0) {
+      // Workgroups of up to four waves share the SIMDs: a wave's priority falls from half row to half row (rows of one stage: from row to
+      // row), in turns of two rows, so that the older workgroup does not run ahead (see fta_fwd1_kernel): with dropout B1 H4 L300 76 against 70 us,
+      // L450 a training step 960 / 935, without at D = 64 B4 H8 L100 40.2 / 39.2.  More waves sit alone on a CU and lose by it, us with / without: five
+      // to seven with dropout L1100 3693 / 3614, D = 64 L384 203 / 198, L1280 x 150 1143 / 1134, without L2304 x 100 1038 / 1022; eight up to 2 %.
+      if (nthreads <= 256 && t == 0) {
         if (ir & 1) __builtin_amdgcn_s_setprio(1);
         else __builtin_amdgcn_s_setprio(3);
       }
-      if (nthreads < 512 && t == (STEPS + 1) / 2) {
+      if (nthreads <= 256 && t == (STEPS + 1) / 2) {
         if (ir & 1) __builtin_amdgcn_s_setprio(0);
         else __builtin_amdgcn_s_setprio(2);
       }
