@@ -153,6 +153,10 @@ const fta::FwdPlan& cached_plan_fwd(int B, int H, int L1, int L2, int D, int fea
   }
   return plan;
 }
+// The plan of a call: the argument check and the launch ask for the same one.
+const fta::FwdPlan& call_plan_fwd(const fta_tensor5* k, int B, int H, int L1, int L2, int D, int feat) {
+  return cached_plan_fwd(B, H, L1, L2, D, feat, k->stride[3] != D);
+}
 const fta::BwdPlan& cached_plan_bwd(int B, int H, int L1, int L2, int D, int feat = 0, size_t limit = 0) {
   thread_local PlanKey key{-1, 0, 0, 0, 0, 0};
   thread_local fta::BwdPlan plan;
@@ -411,7 +415,7 @@ static int check_fwd_impl(const fta_tensor5* q, const fta_tensor5* k, const fta_
     if ((rc = check_row_span(t, L2)) != FTA_OK) return rc;
   if (lse == nullptr) return FTA_ERR_NULL_POINTER;
   if (reinterpret_cast<uintptr_t>(lse) % 16 != 0) return FTA_ERR_MISALIGNED;
-  if (!cached_plan_fwd(B, H, L1, L2, D, feat).valid) return FTA_ERR_SEQ_LEN;
+  if (!call_plan_fwd(k, B, H, L1, L2, D, feat).valid) return FTA_ERR_SEQ_LEN;
   return FTA_OK;
 }
 
@@ -439,7 +443,7 @@ int fta_fwd_ex(const fta_tensor5* q, const fta_tensor5* k, const fta_tensor5* v,
   p.lse = lse;
   copy4(p.qs, q->stride); copy4(p.ks, k->stride); copy4(p.vs, v->stride); copy4(p.os, o->stride);
   copy3(p.bs, bias->stride);
-  const fta::FwdPlan pl = cached_plan_fwd(B, H, L1, L2, D, opt.feat_fwd, k->stride[3] != D);
+  const fta::FwdPlan pl = call_plan_fwd(k, B, H, L1, L2, D, opt.feat_fwd);
   p.B = B; p.H = H; p.L1 = L1; p.L2 = L2; p.L2p = pl.L2p;
   p.odd_bias = bias_rows_unaligned(bias) ? 1 : 0;
   p.head_inner = (H > 1 && k->stride[1] < k->stride[3]) ? 1 : 0;
