@@ -368,6 +368,10 @@ int fta_describe_plan_ex(int B, int H, int L1, int L2, int D, float sm_scale, co
   const fta::BwdPlan b = cached_plan_bwd(B, H, L1, L2, D, level);
   if (!b.valid) return FTA_ERR_SEQ_LEN;
   const long bh = (long)B * H;
+  const fta::FwdPlan fs = cached_plan_fwd(B, H, L1, L2, D, opt.feat_fwd, true);
+  char scattered[96] = "";
+  if (fs.threads != f.threads || fs.nqg * fs.nchunks != f.nqg * f.nchunks || fs.smem != f.smem)
+    snprintf(scattered, sizeof scattered, " scattered_grid=%ld scattered_block=%d scattered_lds=%zu", bh * fs.nqg * fs.nchunks, fs.threads, fs.smem);
   const char* tn = (opt.dtype == fta::kBF16) ? "BF16" : "F16";
   char dq[160], dkdv[160];
   if (b.use_short) {
@@ -387,13 +391,13 @@ int fta_describe_plan_ex(int B, int H, int L1, int L2, int D, float sm_scale, co
     snprintf(dkdv, sizeof dkdv, "fta_bwd_dkdv_kernel<%d,%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, b.NJT, b.JT,
              b.nlaunch2, bh * b.nkg * b.nchunks2, b.threads2, b.smem2);
   const int n = snprintf(out, out_bytes,
-                         "fwd: %s<%d,%d,%d> launches=1 grid=%ld block=%d lds=%zu tiled_length=%d\n"
+                         "fwd: %s<%d,%d,%d> launches=1 grid=%ld block=%d lds=%zu tiled_length=%d%s\n"
                          "dq: %s\n"
                          "dkdv: %s\n"
                          "workspace: delta=%zu partial=%zu aux=%zu tiled_length=%d\n"
                          "options: type=%s dropout=%d precise_or_vector_alu_backward=%d scaled_operand_pair=%d natural_exponent=%d\n",
                          (f.fwd1 == 1 && opt.drop.thresh == 0) ? "fta_fwd1_kernel" : (f.fwd1 == 2 && opt.drop.thresh == 0) ? "fta_fwd2_kernel" : "fta_fwd_kernel", D, f.NKT, f.KT,
-                         bh * f.nqg * f.nchunks, f.threads, f.smem, f.L2p, dq, dkdv, b.delta_bytes, b.partial_bytes, b.aux_bytes, b.L2p, tn,
+                         bh * f.nqg * f.nchunks, f.threads, f.smem, f.L2p, scattered, dq, dkdv, b.delta_bytes, b.partial_bytes, b.aux_bytes, b.L2p, tn,
                          opt.drop.thresh != 0 ? 1 : 0, level != 0 ? 1 : 0,
                          ((level == 0 && opt.bf16_plain && b.use_hand && fta::bf16_scale_needs_split(sm_scale)) ||
                           (level == 0 && opt.f16_precise)) ? 1 : 0,

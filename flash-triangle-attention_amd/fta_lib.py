@@ -154,7 +154,8 @@ def strerror(status: int) -> str:
 
 def describe_plan(B: int, H: int, L1: int, L2: int, D: int, sm_scale: float = 1.0, options: "Options | None" = None) -> dict:
     """Kernel instance, launch count, grid, block and LDS bytes per stage, and the workspace parts, for a
-    call with these sizes, softmax scale and options (None: fp16, no dropout)."""
+    call with these sizes, softmax scale and options (None: fp16, no dropout).  "fwd" has scattered_grid, scattered_block and scattered_lds
+    where keys that are not neighbours in memory run other workgroups."""
     buf = ctypes.create_string_buffer(1024)
     check(load().fta_describe_plan_ex(B, H, L1, L2, D, float(sm_scale), ctypes.byref(options) if options is not None else None,
                                       buf, len(buf)))

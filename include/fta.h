@@ -140,8 +140,10 @@ int fta_seq_len_supported_ex(int L2, int D, const fta_options* options);
 
 /* Writes, as text, which kernel instance each stage would run for these sizes, with launch count,
  * grid, block and LDS bytes, and the parts of the backward workspace (one line per stage: "fwd: ...",
- * "dq: ...", "dkdv: ...", "workspace: ..."; `tiled_length` on the "fwd" and "workspace" lines is the
- * multiple of 128 keys that the forward's, respectively the backward's, tiles cover).  Host only.  No counterpart upstream (its Triton
+ * "dq: ...", "dkdv: ...", "workspace: ..."; `tiled_length` is the length that the forward's tiles cover, a multiple of 32
+ * keys, and on the "workspace" line the multiple of 128 that the backward's workspace is laid out with).  The forward of
+ * keys that are not neighbours in memory (stride[3] of k is not D: interleaved heads, transposed views) runs other
+ * workgroups at some lengths: the "fwd" line then has scattered_grid, scattered_block and scattered_lds, too.  Host only.  No counterpart upstream (its Triton
  * autotuner prints its choice with TRITON_PRINT_AUTOTUNING); for logs, tests and bug reports.
  * FTA_ERR_WORKSPACE if `out_bytes` is too small (512 is enough). */
 int fta_describe_plan(int B, int H, int L1, int L2, int D, char* out, size_t out_bytes);

@@ -246,6 +246,25 @@ def test_plan_description_is_consistent_for_every_supported_length():
     assert lib.fta_describe_plan(4, 8, 512, 512, 32, None, 0) == -1
 
 
+def test_plan_description_of_keys_that_are_not_neighbours_in_memory():
+    """Interleaved heads and transposed views: rows of 225 to 256 keys that fill the chip and some of 513 to 1024 run larger workgroups,
+    which the description names beside those of contiguous tensors."""
+    for dims, block, scattered in (((4, 8, 256, 256, 32), 256, 512), ((4, 8, 230, 230, 32), 256, 512), ((2, 4, 230, 230, 32), 256, None), ((1, 1, 8, 256, 32), 256, None),
+                                   ((1, 4, 224, 224, 32), 256, None), ((1, 4, 512, 512, 32), 256, None), ((1, 4, 640, 640, 32), 256, 512),
+                                   ((1, 4, 701, 701, 32), 256, None), ((1, 4, 768, 768, 32), 256, 512), ((1, 4, 1024, 1024, 32), 256, 512),
+                                   ((1, 4, 1536, 1536, 32), 512, None), ((2, 8, 512, 512, 64), 512, None)):
+        fwd = fta_lib.describe_plan(*dims)["fwd"]
+        assert fwd["block"] == block and fwd.get("scattered_block") == scattered, (dims, fwd)
+        if scattered is not None:
+            B, H, L1, L2, _ = dims
+            blocks = (scattered // 64) // (1 if L2 <= 512 else 2)  # query blocks of 32 to a workgroup
+            groups = -(-L2 // (32 * blocks))
+            assert fwd["scattered_grid"] % (B * H * groups) == 0 and fwd["scattered_grid"] // (B * H * groups) <= L1
+            assert 0 < fwd["scattered_lds"] <= 160 * 1024
+    buf = ctypes.create_string_buffer(512)  # the size the header promises to be enough
+    assert fta_lib.load().fta_describe_plan(64, 64, 4000, 1024, 32, buf, 512) == 0 and b"scattered_block=512" in buf.value
+
+
 def test_chunk_counts_fill_the_last_round_of_workgroups():
     """With few (b,h) slices the L1-chunk count decides how full the last round of workgroups on the
     256 CUs is; the planner picks counts that fill it where the sizes allow."""
