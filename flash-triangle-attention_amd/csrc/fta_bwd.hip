@@ -90,6 +90,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   const bool three = (feat == 2 && D == 32 && kr == 384);
   const int nblk = (feat == 2) ? (row + 31) / 32 : nqb;
   pl.NKT = three ? 3 : 4;
+  pl.own_delta = three;
   pl.SK = kr / (32 * pl.NKT);
   int qb = (three ? 4 : 8) / pl.SK;
   if (qb < 1) qb = 1;
@@ -153,7 +154,7 @@ static BwdPlan plan_any_size(int B, int H, int L1, int L2, int D, int row, int f
   pl.rows_per_chunk2 = (L1 + pl.nchunks2 - 1) / pl.nchunks2;
   pl.nchunks2 = (L1 + pl.rows_per_chunk2 - 1) / pl.rows_per_chunk2;
 
-  pl.delta_bytes = (size_t)B * H * L1 * L2 * sizeof(float);
+  pl.delta_bytes = pl.own_delta ? 0 : (size_t)B * H * L1 * L2 * sizeof(float);
   pl.partial_bytes = (size_t)pl.nchunks * B * H * L2 * L2 * sizeof(float);
   pl.aux_bytes = (size_t)B * H * L1 * L2 * 2 * sizeof(uint32_t);
   pl.valid = ok2 && (pl.SK * pl.QB <= 8) && (pl.ring >= 3);

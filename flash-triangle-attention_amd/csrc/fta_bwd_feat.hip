@@ -35,8 +35,7 @@ template <class T, bool DROP>
 static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t st, hipEvent_t* ev) {
   auto mark = [&](int i) { if (ev != nullptr) (void)hipEventRecord(ev[i], st); };
   hipError_t e = hipSuccess;
-  const bool own = DROP && D == 32 && pl.NKT == 3 && pl.nranges == 0;  // the dQ kernel's instance for 384 keys forms them itself
-  if (!own) {  // 0. delta and the {lse, delta} pairs
+  if (!pl.own_delta) {  // 0. delta and the {lse, delta} pairs
     const int64_t nthr = (int64_t)p.B * p.H * p.L1 * p.L2p * (D / 8);
     dim3 grid((unsigned)((nthr + 255) / 256)), block(256);
     if (D == 32) hipLaunchKernelGGL((fta_bwd_delta_kernel<T, 32>), grid, block, 0, st, p);
@@ -61,9 +60,9 @@ static hipError_t bwd_feat_t(BwdParams p, const BwdPlan& pl, int D, hipStream_t 
     for (int n = 0; n < (pl.nranges > 0 ? 0 : pl.nlaunch); ++n) {
       p.kr0 = n * pl.KR;
       e = hipErrorInvalidConfiguration;
-      if (pl.NKT == 3) {  // key ranges of 384 keys with dropout: fixed geometry
+      if (pl.own_delta) {  // key ranges of 384 keys with dropout: fixed geometry
         if constexpr (DROP)
-          if (D == 32 && pl.threads == 256 && pl.SK == 4 && pl.ring == dq_ring(32, 3, 1, 4, 4).r && pl.nb == dq_ring(32, 3, 1, 4, 4).nb)
+          if (D == 32 && pl.NKT == 3 && pl.threads == 256 && pl.SK == 4 && pl.ring == dq_ring(32, 3, 1, 4, 4).r && pl.nb == dq_ring(32, 3, 1, 4, 4).nb)
             e = launch_kernel(fta_bwd_dq_kernel<T, true, 32, 1, 3, 4, 4>, p, grid, block, pl.smem, st);
       } else if (D == 32) {
         e = launch_kernel(fta_bwd_dq_kernel<T, DROP, 32, 2>, p, grid, block, pl.smem, st);

@@ -176,6 +176,7 @@ struct BwdPlan {
   ShortPlan sh;
   int L2p;             // the length the workspace is laid out with and the general kernels' tiles cover (filled in by the C-ABI layer)
   int Lt;              // the length the hand-scheduled kernels' tiles cover: the next multiple of 64, not of 128, where they have the instances
+  bool own_delta;      // dropout: the dQ/dBias kernel forms delta and the row constants itself, no kernel runs in front of it
   bool feat;           // planned for the feature instances (bf16, dropout, precise fp16)
   bool valid;
 };

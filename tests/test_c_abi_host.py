@@ -265,6 +265,15 @@ def test_plan_description_of_keys_that_are_not_neighbours_in_memory():
     assert fta_lib.load().fta_describe_plan(64, 64, 4000, 1024, 32, buf, 512) == 0 and b"scattered_block=512" in buf.value
 
 
+def test_the_dropout_backward_asks_for_delta_where_a_kernel_writes_it():
+    """D = 32, 257 to 384 keys: dQ/dBias forms delta itself; the one-kernel backward below never stores it."""
+    for L2, need in ((200, False), (256, False), (257, False), (320, False), (384, False), (385, True), (512, True), (700, True), (768, True)):
+        opt = fta_lib.Options(fta_lib.DTYPE_BF16, 0, 0.25, 7, 0)
+        ws = fta_lib.describe_plan(1, 4, 37, L2, 32, 0.17, opt)["workspace"]
+        assert ws["delta"] == (4 * 37 * ws["tiled_length"] * 4 if need else 0), (L2, ws)
+        assert ws["delta"] + ws["partial"] + ws["aux"] == fta_lib.load().fta_bwd_workspace_bytes_ex(1, 4, 37, L2, 32, ctypes.byref(opt))
+
+
 def test_chunk_counts_fill_the_last_round_of_workgroups():
     """With few (b,h) slices the L1-chunk count decides how full the last round of workgroups on the
     256 CUs is; the planner picks counts that fill it where the sizes allow."""
