@@ -19,10 +19,12 @@ bool plan_fwd1(int B, int H, int L1, int L2, int D, int row, bool scattered, Fwd
   // four waves per workgroup, two workgroups to a CU (see the kernel's comment); eight where a query block's keys are four slabs; rows of up to
   // 64 queries have two query blocks.  256 keys that do not lie next to each other in memory (heads
   // interleaved, or a transposed view: half a line each): the eight query blocks of a row in one workgroup, where such workgroups fill the chip, so that half as
-  // many ask for a line (B2 H4, us, four / eight waves: heads interleaved in bf16 46.7 / 46.0, a training pass 179 / 177, transposed 47.9 / 47.2; contiguous
-  // 42.0 / 42.4, B4 H8 146 / 150; 512 keys, heads interleaved, 1033 / 1069)
+  // many ask for a line (bf16, inputs not in the caches, us, four / eight waves: heads interleaved B2 H4 46.9 / 45.6, B4 H8 167.8 / 163.5, 240 keys
+  // 154.5 / 153.3, transposed 164.1 / 161.9, a training pass 696 / 694; with inputs that stay in the caches equal at 256, 141 / 145 at 240;
+  // contiguous B2 H4 42.0 / 42.4, B4 H8 146 / 150; 512 keys, heads interleaved, 1033 / 1069)
   // Two slabs of such keys, where four query blocks to a workgroup leave no more of them empty than two: the same (us, two / four query blocks:
-  // transposed B1 H4 L640 306 / 302, B2 H8 L640 1209 / 1181, B1 H4 L768 506 / 501; L900 862 / 882, L960 944 / 954, contiguous L640 1128 / 1138).
+  // transposed B1 H4 L640 294 / 292, L1024 1070 / 1046, heads interleaved L768 477 / 475, B2 H8 L890 2999 / 2963; L900 862 / 882, L960 944 / 954, contiguous
+  // L640 1128 / 1138; with inputs that stay in the caches L640 286 / 296, L1024 999 / 1080).
   const int nblk = (row + 31) / 32;
   const bool four_blocks = scattered && L2 % 128 == 0 && nblk % 4 == 0;
   const bool row_of_eight = L2 == 256 && scattered && (long)B * H * ((L1 + 7) / 8) >= 256;

@@ -34,9 +34,10 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // older one issue first whenever both are ready, which in a kernel bound by the vector ALU is nearly always: measured with
 // a clock around every workgroup (B4 H8 L512), the older workgroup of a CU finished its 128 rows after 750 us and the
 // younger one, left with a SIMD to itself that a lone wave cannot fill, after 1250.  So a wave's priority falls from half row to
-// half row, in turns of two rows: the one that is ahead yields until the other has caught up, neither is ever more than two rows
-// ahead, and their barriers stay uncoupled.  Without / with it, us: B1 H4 L150 13.1 / 12.5, L200 20.4 / 18.4, L300 42.7 / 40.3, L384
-// 66.8 / 63.0, L457 in bf16 113 / 109, B2 H4 L320 88.7 / 84, B4 H8 L128 31.2 / 30.3, L384 at scale 1.3 510 / 489.  One workgroup of eight
+// half row, in turns of two rows: the one that is ahead by less than two yields until the other has caught up (two rows apart they are equals
+// again; and one that waits lets the other issue, whatever their priorities), and their barriers stay uncoupled.  Without / with it, us: B1 H4 L150
+// 13.1 / 12.5, L200 20.4 / 18.4, L300 42.7 / 40.3, L384 66.8 / 63.0, L457 in bf16 113 / 109, B2 H4 L320 88.7 / 84, B4 H8 L128 31.7 / 31.9 (inputs in
+// the caches 27.0 / 26.6), L192 89.7 / 85.6, L384 at scale 1.3 510 / 489.  One workgroup of eight
 // waves, where the two waves of a SIMD meet at every stage barrier, gives B4 H8 L512 1037 and 1117 us (scale 1.3), B1 H4 L512 137.6; this 989,
 // 1051 and 131.4.  Four steps over the whole chunk instead: 1027, 1087, 134.1; a step a row in turns of four: 984, 1055, 131.0, but 2 % more
 // at 128 keys; four steps within a row: equal, 3 % more at 384 keys.
@@ -566,6 +567,7 @@ __global__ void __attribute__((amdgpu_flat_work_group_size(64 * W, 64 * W), amdg
             ph[r >> 1] = T::pack(p0, p1);
             lt = T::sum2(ph[r >> 1], lt);
           }
+          // (the row sum's dot product is read by another opcode from here on: three slots; the packed weights by the matrix core: two)
           asm volatile("s_nop 3" : "+v"(acc), "+v"(lt), "+v"(ph[0]), "+v"(ph[1]), "+v"(ph[2]), "+v"(ph[3]), "+v"(ph[4]), "+v"(ph[5]),
                        "+v"(ph[6]), "+v"(ph[7]));
         }

@@ -200,9 +200,10 @@ hipError_t launch_short(BwdParams p, const ShortPlan& pl, int D, int dtype, bool
 bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl);
 hipError_t launch_dkdv1(BwdParams p, const Dkdv1Plan& pl, int D, int dtype, bool hilo, bool nat, hipStream_t st);
 
-// Stage buffers and row-operand buffers that 160 KB hold beside the exchange records: of the dQ/dBias kernel with SK slabs
-// of NKT tiles, G1 of them to a stage, and of the dK/dV kernel with SJ slabs of NJT tiles, JT queries to a stage; eight
-// waves each (the kernels with that geometry fixed and the launch plan agree on it).
+// Stage buffers and row-operand buffers that a workgroup's share of LDS holds beside the exchange records, 160 KB for eight waves and
+// 80 for four: of the dQ/dBias kernel with SK slabs
+// of NKT tiles, G1 of them to a stage, and of the dK/dV kernel with SJ slabs of NJT tiles, JT queries to a stage
+// (the kernels with that geometry fixed and the launch plan agree on it).
 struct Ring { int r, nb; };
 constexpr Ring fit_ring(int steps, int slot, int row, int records, int waves) {
   for (int r = 4; r >= 3; --r) {

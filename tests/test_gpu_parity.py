@@ -578,7 +578,9 @@ def test_head_dim_64_forward_of_one_and_two_slabs_with_masked_key_ranges(L2, mas
 def test_forward_is_the_same_however_the_rows_lie_in_memory(L1, L2):
     """Rows of 256 keys run in workgroups of four or of eight query blocks, some rows of 513 to 1024 in two or four, by whether a row's keys are neighbours in memory.  A
     wave's arithmetic is the same in both, so contiguous, head-interleaved and transposed tensors give the same bits."""
+    import fta_lib
     B, H, D = 4, 8, 32
+    assert ("scattered_block" in fta_lib.describe_plan(B, H, L1, L2, D)["fwd"]) == (L2 in (255, 256, 640, 1000, 1024))
     print(f"case memory order L1={L1} L2={L2}", flush=True)
     q, k, v, b, do = orc.make_inputs(B, H, L1, L2, D, seed=9, device=DEV)
     want = _run(q, k, v, b, 1.3, do)
