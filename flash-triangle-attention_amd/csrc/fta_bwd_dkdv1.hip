@@ -5,13 +5,18 @@
 namespace fta {
 
 // Query ranges of one launch each (a wave's stationary bias^T tile and the stage size are compiled in), in units of 64
-// queries and as even as the row divides.  D = 32: four to eight units; D = 64: four or
-// five (bias^T, dK and dV share the accumulation registers with the operands), or one range of six, which takes the last
-// register, for a row of 384 queries.
+// queries and as even as the row divides: four to eight units.  D = 64 has no instance of seven (14 tiles divide into stages of seven,
+// of which LDS holds no three): seven and six are cut as eight and five, two sevens as eight and six, and three or more ranges that are
+// not equal as ranges of four and five (as before there were wider ones: 1408 keys 25.6 ms a step).
 static int dkdv1_ranges(int L2, int D, int* out) {
-  return even_ranges(L2 / 64, D == 32 ? 8 : L2 == 384 ? 6 : 5, 64, out);
+  const int units = L2 / 64;
+  const int n = even_ranges(units, 8, 64, out);
+  if (D == 32) return n;
+  if (n <= 2 ? units == 15 : (units % n != 0 || out[0] == 448)) return even_ranges(units, 5, 64, out);
+  if (n == 2 && out[0] == 448) { out[0] += 64; out[1] -= 64; }
+  return n;
 }
-// queries per stage: half of the range where that is at most 256 (D = 64: 160), else a third; a short one at once
+// queries per stage: half of the range where that is at most 256, a short one at once; D = 64: 128, of a range of 320 160
 static int dkdv1_stage(int range, int D) {
   if (D == 64 && range % 128 == 0) return 128;
   return range > 256 ? range / 2 : range;
@@ -20,7 +25,7 @@ static int dkdv1_stage(int range, int D) {
 bool plan_dkdv1(int B, int H, int L1, int L2, int D, Dkdv1Plan& pl) {
   if (D != 32 && D != 64) return false;
   if (L2 % 64 != 0 || L2 < 256 || L2 > (D == 64 ? 256 : 512) * kMaxRanges) return false;
-  if (D == 64 && (L2 == 448 || L2 == 704)) return false;  // (no cut into these ranges: tiled as 512 and 768)
+  if (D == 64 && L2 == 448) return false;  // (seven units: tiled as 512)
   pl.nlaunch = dkdv1_ranges(L2, D, pl.range);
   pl.JR = pl.range[0];
   pl.NJT = pl.JR / 32;

@@ -18,8 +18,14 @@
 //     that produce S and dP of tile j+1, and between them the vector-ALU work of tile j
 //     (exp2, dS = P * dP, two fp16 packings).  The pipeline runs across stage and row boundaries.
 // Used for tiled lengths that are a multiple of 64 from 256 on (D = 64: without 448): a launch takes a
-// query range of 256 to 512 (NJT = 8 to 16; D = 64: 256 to 384) in one to three stages of 128 to 256 queries; otherwise
+// query range of 256 to 512 (NJT = 8 to 16; D = 64: not 448) in one to four stages of 128 to 256 queries; otherwise
 // the two-waves-per-SIMD kernel runs.
+//
+// D = 64 bound: a launch reads K and V and writes dK and dV whole, so that what a row costs beside its tiles is memory: at B2 H8 L512 two
+// launches of 256 queries moved 6.4 GB (two of 967 us), one of 512 moves 3.2 GB (1210 us; without copies, stores and LDS reads, timing only,
+// 930: 20 MFMAs a tile under the power cap).  It takes 128 accumulation registers for bias^T, so that an operand's registers
+// are filled again behind the MFMA that consumes it instead of being held twice (by itself, at 256 queries, within 1 %).  Training steps
+// (us): L512 4235 -> 3800, B1 H4 L701 3357 -> 3060, L1024 in bf16 9470 -> 8590, L1536 30790 -> 29030.
 #pragma once
 #include "fta_kernels.h"
 #include "fta_pipe.h"
@@ -80,7 +86,7 @@ __device__ __forceinline__ u32x4 lds_issue_pair2(uint32_t addr) {
 // Waits until every LDS read issued so far has landed and ties the registers they fill to that point
 // (SETTLE: plus the idle slot that keeps the first vector-ALU reader of the tile that the previous
 // iteration's last MFMA completed far enough behind it).  D = 64 (KS = 4) keeps the Q, dO operands in
-// accumulation registers.
+// accumulation registers and waits in this way at the end of a row only.
 template <int KS, int DT, bool SETTLE>
 __device__ __forceinline__ void dkdv1_lds_landed(u32x4 (&qf)[KS], u32x4 (&dof)[KS], u32x4& cstn, u32x2 (&qtlo_p)[2][DT],
                                                  u32x2 (&qthi_p)[2][DT], u32x2 (&dtlo_p)[2][DT], u32x2 (&dthi_p)[2][DT]) {
@@ -94,19 +100,30 @@ __device__ __forceinline__ void dkdv1_lds_landed(u32x4 (&qf)[KS], u32x4 (&dof)[K
                    : "+v"(qf[0]), "+v"(qf[1]), "+v"(dof[0]), "+v"(dof[1]), "+v"(cstn), "+v"(qtlo_p[0][0]), "+v"(qthi_p[0][0]),
                      "+v"(qtlo_p[1][0]), "+v"(qthi_p[1][0]), "+v"(dtlo_p[0][0]), "+v"(dthi_p[0][0]), "+v"(dtlo_p[1][0]), "+v"(dthi_p[1][0]));
   } else {
-    if constexpr (SETTLE)
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 0"
-                   : "+a"(qf[0]), "+a"(qf[1]), "+a"(qf[2]), "+a"(qf[3]), "+a"(dof[0]), "+a"(dof[1]), "+a"(dof[2]), "+a"(dof[3]), "+v"(cstn),
-                     "+v"(qtlo_p[0][0]), "+v"(qthi_p[0][0]), "+v"(qtlo_p[0][1]), "+v"(qthi_p[0][1]), "+v"(qtlo_p[1][0]), "+v"(qthi_p[1][0]),
-                     "+v"(qtlo_p[1][1]), "+v"(qthi_p[1][1]), "+v"(dtlo_p[0][0]), "+v"(dthi_p[0][0]), "+v"(dtlo_p[0][1]), "+v"(dthi_p[0][1]),
-                     "+v"(dtlo_p[1][0]), "+v"(dthi_p[1][0]), "+v"(dtlo_p[1][1]), "+v"(dthi_p[1][1]));
-    else
-      asm volatile("s_waitcnt lgkmcnt(0)"
-                   : "+a"(qf[0]), "+a"(qf[1]), "+a"(qf[2]), "+a"(qf[3]), "+a"(dof[0]), "+a"(dof[1]), "+a"(dof[2]), "+a"(dof[3]), "+v"(cstn),
-                     "+v"(qtlo_p[0][0]), "+v"(qthi_p[0][0]), "+v"(qtlo_p[0][1]), "+v"(qthi_p[0][1]), "+v"(qtlo_p[1][0]), "+v"(qthi_p[1][0]),
-                     "+v"(qtlo_p[1][1]), "+v"(qthi_p[1][1]), "+v"(dtlo_p[0][0]), "+v"(dthi_p[0][0]), "+v"(dtlo_p[0][1]), "+v"(dthi_p[0][1]),
-                     "+v"(dtlo_p[1][0]), "+v"(dthi_p[1][0]), "+v"(dtlo_p[1][1]), "+v"(dthi_p[1][1]));
+    static_assert(!SETTLE, "D = 64 waits for the operands one by one");
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+a"(qf[0]), "+a"(qf[1]), "+a"(qf[2]), "+a"(qf[3]), "+a"(dof[0]), "+a"(dof[1]), "+a"(dof[2]), "+a"(dof[3]), "+v"(cstn),
+                   "+v"(qtlo_p[0][0]), "+v"(qthi_p[0][0]), "+v"(qtlo_p[0][1]), "+v"(qthi_p[0][1]), "+v"(qtlo_p[1][0]), "+v"(qthi_p[1][0]),
+                   "+v"(qtlo_p[1][1]), "+v"(qthi_p[1][1]), "+v"(dtlo_p[0][0]), "+v"(dthi_p[0][0]), "+v"(dtlo_p[0][1]), "+v"(dthi_p[0][1]),
+                   "+v"(dtlo_p[1][0]), "+v"(dthi_p[1][0]), "+v"(dtlo_p[1][1]), "+v"(dthi_p[1][1]));
   }
+}
+
+// D = 64: the registers of an operand are filled again behind the MFMA that consumes it, so that the reads complete in the
+// order of their use, one iteration later.  Three waits an iteration (25 reads; the counter holds 15): for the operands that P and dS of
+// step 0 meet, reads 0 to 7, with 17 issued behind them; for step 1's and the first Q, dO fragments, up to read 17, with 7 + 8 behind it;
+// for the rest, up to read 24, with 18 behind it.
+template <int DT, int N>
+__device__ __forceinline__ void dkdv1_wait_step(u32x2 (&qtlo)[DT], u32x2 (&qthi)[DT], u32x2 (&dtlo)[DT], u32x2 (&dthi)[DT]) {
+  if constexpr (DT == 2)
+    asm volatile("s_waitcnt lgkmcnt(%8)\n\ts_nop 0"
+                 : "+v"(qtlo[0]), "+v"(qthi[0]), "+v"(qtlo[1]), "+v"(qthi[1]), "+v"(dtlo[0]), "+v"(dthi[0]), "+v"(dtlo[1]), "+v"(dthi[1])
+                 : "n"(N));
+}
+template <int KS>
+__device__ __forceinline__ void dkdv1_wait_rest(u32x4 (&qf)[KS], u32x4 (&dof)[KS], u32x4& cst) {
+  if constexpr (KS == 4)
+    asm volatile("s_waitcnt lgkmcnt(14)" : "+a"(qf[1]), "+a"(qf[2]), "+a"(qf[3]), "+a"(dof[1]), "+a"(dof[2]), "+a"(dof[3]), "+v"(cst));
 }
 
 // T: element type; TS: tiles (of 32 queries) per stage; TAIL: the row's true length L2 is shorter than the
@@ -129,6 +146,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   constexpr int DT = D / 32;
   constexpr bool WIDE = (D == 64);
   constexpr int OPF = WIDE ? kA : kV;          // register file of the MFMA-only operands
+  constexpr int KVF = WIDE && NJT <= 12 ? kA : kV;  // of the row's K and V fragments
   constexpr int STEPS = NJT / TS;              // stages per row
   constexpr int JT = TS * 32;                  // queries per stage
   constexpr int KR = 128;                      // keys per workgroup
@@ -146,10 +164,11 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   constexpr int NRD = 2 * KS + 1 + 8 * DT;     // LDS reads per iteration
   constexpr int NG = NM - 8;                   // gaps: MFMAs that no vector-ALU pair follows
   constexpr int NGR = (NG > 8) ? 8 : NG;       // gaps that take LDS reads
-  static_assert(NJT % TS == 0 && STEPS >= 1 && STEPS <= 3, "whole stages; the ring holds three");
+  static_assert(NJT % TS == 0 && STEPS >= 1 && STEPS <= 4, "whole stages");
   static_assert(TS >= 4 && (TS - 1) * NG >= 2 * NQI + 1 + 2 * (KR * (D / 8) / 256),
                 "the iterations between two barriers must have a gap for every copy of a stage");
   static_assert(R * SLOT_B + NBK * KV_B <= 160 * 1024, "LDS");
+  static_assert(!WIDE || 2 * NQI + 1 + 2 * (KR * (D / 8) / 256) <= 2 * NG, "no copy behind a row's stores and in front of the next barrier");
   static_assert(WIDE || NG >= 4 * DT, "a gap for every piece of an earlier range's row");
   static_assert(ACP == 1 || ACP == 2, "128 to 256 queries per stage");
 
@@ -239,14 +258,21 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   // row pointers stop advancing and the last row is copied again into slots that nothing reads any
   // more, which keeps the loop free of "is there a next stage" branches.
   int row_iss = 0;
-  uint32_t goffq[STEPS][NQI], goffdo[STEPS][NQI], goffk[NKI], goffv[NKI], goffa[STEPS];  // [part of the row][copy]
+  // D = 64: one set of offsets for every part, from the part's first query (TAIL: the last part, the only one that can reach
+  // beyond the row, has its own); D = 32: a set per part, from the range's first query.
+  constexpr int NOFF = WIDE ? (TAIL ? 2 : 1) : STEPS;
+  auto part_of = [](int t) constexpr { return !WIDE ? t : TAIL && t == STEPS - 1 ? 1 : 0; };
+  uint32_t goffq[NOFF][NQI], goffdo[NOFF][NQI], goffk[NKI], goffv[NKI], goffa[WIDE ? 1 : STEPS];  // [part of the row][copy]
 #pragma unroll
-  for (int t = 0; t < STEPS; ++t) {
+  for (int t = 0; t < NOFF; ++t) {
 #pragma unroll
     for (int u = 0; u < NQI; ++u) {
       const int pidx = (wave + 4 * u) * 64 + lane, row = pidx / (D / 8), chunkc = swz_slot<D>(row, pidx % (D / 8));
-      int grow = min(row, JT - 1) + t * JT;
-      if constexpr (TAIL) grow = min(p.jr0 + grow, p.L2 - 1) - min(p.jr0, p.L2 - 1);  // (see qcur)
+      int grow = min(row, JT - 1) + (WIDE ? 0 : t * JT);
+      if constexpr (TAIL && WIDE) {
+        const int first = p.jr0 + (t == 1 || STEPS == 1 ? (STEPS - 1) * JT : 0);  // (a real query: the tiles end less than 128 beyond the row)
+        grow = min(first + grow, p.L2 - 1) - first;
+      } else if constexpr (TAIL) grow = min(p.jr0 + grow, p.L2 - 1) - min(p.jr0, p.L2 - 1);  // (see qcur)
       goffq[t][u] = (uint32_t)(((int64_t)grow * p.qs[3] + chunkc * 8) * 2);
       goffdo[t][u] = (uint32_t)(((int64_t)grow * p.dos[3] + chunkc * 8) * 2);
     }
@@ -255,7 +281,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
     // it), which keeps the copy counts of the waves equal
     // (past the pairs of the stage, the last two again)
     const int at = ((wave >> 1) % ACP) * 1024 + lane * 16;
-    goffa[t] = (uint32_t)(t * (JT * 8) + (JT * 8 % 1024 != 0 ? min(at, JT * 8 - 16) : at));
+    if (!WIDE || t == 0) goffa[t] = (uint32_t)((WIDE ? 0 : t * (JT * 8)) + (JT * 8 % 1024 != 0 ? min(at, JT * 8 - 16) : at));
   }
 #pragma unroll
   for (int u = 0; u < NKI; ++u) {
@@ -282,6 +308,9 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   // on), stage_copy<t, c>() issues copy c of a stage of part t; the loop issues them one per gap
   // between MFMAs, over the iterations that follow the barrier.
   uint32_t iss_dst = 0, iss_kd = 0, iss_ad = 0;
+  const int64_t step_qt = hold_scalar(WIDE ? (int64_t)JT * p.qs[3] * 2 : 0), step_dot = hold_scalar(WIDE ? (int64_t)JT * p.dos[3] * 2 : 0);
+  const half_t* qpart = qcur;    // (D = 64) where the part being issued starts
+  const half_t* dopart = docur;
   auto stage_begin = [&](auto tc, bool first) {
     constexpr int t = decltype(tc)::value;
     if constexpr (t == 0) {
@@ -291,6 +320,9 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       }
       iss_kd = ldskv + (uint32_t)cur_kb * KV_B + wofs;
       cur_kb = (cur_kb + 1 == NBK) ? 0 : cur_kb + 1;
+      if constexpr (WIDE) { qpart = qcur; dopart = docur; }
+    } else if constexpr (WIDE) {
+      advance(qpart, step_qt); advance(dopart, step_dot);
     }
     iss_dst = lds0 + (uint32_t)cur_slot * SLOT_B + wofs;
     iss_ad = lds0 + (uint32_t)cur_slot * SLOT_B + (uint32_t)CST_B + (uint32_t)((wave >> 1) % ACP) * 1024u;
@@ -298,9 +330,9 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   };
   auto stage_copy = [&](auto tc, auto cc) {  // copy number c of a stage of part t (nothing if it has fewer)
     constexpr int t = decltype(tc)::value, c = decltype(cc)::value;
-    if constexpr (c < NQI) dma16s_at<(uint32_t)c * 4096u>(goffq[t][c], uniform_ptr(qcur), iss_dst);
-    else if constexpr (c < 2 * NQI) dma16s_at<(uint32_t)(JTP * D * 2) + (uint32_t)(c - NQI) * 4096u>(goffdo[t][c - NQI], uniform_ptr(docur), iss_dst);
-    else if constexpr (c == 2 * NQI) dma16s_at<0u>(goffa[t], uniform_ptr(acur), iss_ad);
+    if constexpr (c < NQI) dma16s_at<(uint32_t)c * 4096u>(goffq[part_of(t)][c], uniform_ptr(WIDE ? qpart : qcur), iss_dst);
+    else if constexpr (c < 2 * NQI) dma16s_at<(uint32_t)(JTP * D * 2) + (uint32_t)(c - NQI) * 4096u>(goffdo[part_of(t)][c - NQI], uniform_ptr(WIDE ? dopart : docur), iss_dst);
+    else if constexpr (c == 2 * NQI) dma16s_at<0u>(goffa[WIDE ? 0 : t], uniform_ptr(WIDE ? acur + t * (JT * 2) : acur), iss_ad);
     else if constexpr (t == 0 && c < 2 * NQI + 1 + NKI) dma16s_at<(uint32_t)(c - 2 * NQI - 1) * 4096u>(goffk[c - 2 * NQI - 1], uniform_ptr(kcur), iss_kd);
     else if constexpr (t == 0 && c < 2 * NQI + 1 + 2 * NKI)
       dma16s_at<(uint32_t)(KR * D * 2) + (uint32_t)(c - 2 * NQI - 1 - NKI) * 4096u>(goffv[c - 2 * NQI - 1 - NKI], uniform_ptr(vcur), iss_kd);
@@ -312,8 +344,10 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
   };
   // Publishes the stage issued last (waits for all copies issued so far), then picks the slot that
   // became free for the next one, whose copies the following iterations issue.
-  auto sync_stage = [&](auto tc) {
-    wait_vmem_all();
+  // `stores`: the youngest of them, which a row's end has just issued (D = 64), are not waited for.
+  auto sync_stage = [&](auto tc, bool stores) {
+    if (WIDE && stores) __builtin_amdgcn_s_waitcnt(0x0F70 | (4 * DT));
+    else wait_vmem_all();
     __syncthreads();
     stage_begin(tc, false);
   };
@@ -334,7 +368,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
         kk[ks] = __builtin_bit_cast(u32x4, T::scale8(lds_frag<D>(kt, wave * 32, fo, ks), sl2));
       }
       vv[ks] = __builtin_bit_cast(u32x4, lds_frag<D>(kt + KR * D, wave * 32, fo, ks));
-      if constexpr (WIDE) asm volatile("" : "+a"(kk[ks]), "+a"(vv[ks]));
+      if constexpr (KVF == kA) asm volatile("" : "+a"(kk[ks]), "+a"(vv[ks]));
     }
   };
 
@@ -381,18 +415,19 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
     const u32x4 cst = {w[0], w[1], w[0], w[1]};
     // (freshly scaled, or freshly moved: see mfma_acc_v_late)
     if constexpr (KS == 2) asm volatile("s_nop 1" : "+v"(kf[0]), "+v"(kf[1]));
+    else if constexpr (KVF == kV) asm volatile("s_nop 1" : "+v"(kf[0]), "+v"(kf[1]), "+v"(kf[2]), "+v"(kf[3]), "+v"(vf[0]), "+v"(vf[1]), "+v"(vf[2]), "+v"(vf[3]));
     else asm volatile("s_nop 1" : "+a"(kf[0]), "+a"(kf[1]), "+a"(kf[2]), "+a"(kf[3]), "+a"(vf[0]), "+a"(vf[1]), "+a"(vf[2]), "+a"(vf[3]));
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const u32x4 aq = __builtin_bit_cast(u32x4, lds_frag<D>(cQ, 0, fo, ks)), ado = __builtin_bit_cast(u32x4, lds_frag<D>(cDO, 0, fo, ks));
       if (ks == 0) {
-        mfma_rf<T, kV, OPF, kV, 3>(s_cur, aq, kf[ks]);
-        mfma_rf<T, kV, OPF, kV, 3>(dp_cur, ado, vf[ks]);
+        mfma_rf<T, kV, KVF, kV, 3>(s_cur, aq, kf[ks]);
+        mfma_rf<T, kV, KVF, kV, 3>(dp_cur, ado, vf[ks]);
       } else {
-        mfma_rf<T, kV, OPF, kV, 0>(s_cur, aq, kf[ks]);
-        mfma_rf<T, kV, OPF, kV, 0>(dp_cur, ado, vf[ks]);
+        mfma_rf<T, kV, KVF, kV, 0>(s_cur, aq, kf[ks]);
+        mfma_rf<T, kV, KVF, kV, 0>(dp_cur, ado, vf[ks]);
       }
-      if constexpr (HL) mfma_rf<T, kV, OPF, kV, 0>(s_cur, aq, kl[ks]);
+      if constexpr (HL) mfma_rf<T, kV, KVF, kV, 0>(s_cur, aq, kl[ks]);
     }
     mfma_rf<F16, kA, kV, kV, 0>(s_cur, biasA[0][0], Eb[0]);
     mfma_rf<F16, kA, kV, kV, 0>(s_cur, biasA[0][1], Eb[1]);
@@ -517,7 +552,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       // -- publish the stage that tile g+2 starts: its operands are read two iterations ahead
       if constexpr (g % TS == TS - 2) {
         constexpr int tn = ((g + 2) / TS) % STEPS;           // part of the published stage
-        sync_stage(std::integral_constant<int, (tn + 1) % STEPS>{});
+        sync_stage(std::integral_constant<int, (tn + 1) % STEPS>{}, WIDE && g == TS - 2 && ir > 0 && !(TAIL && k0 >= p.L2));
         if constexpr (PRE && g == NJT - 2) old_landed();
       }
       if constexpr (g == NJT - 1) row_operands(ir + 1, kf_n, kl_n, vf_n);  // the next row's K, V fragments
@@ -540,6 +575,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
           constexpr int u = i / (4 * DT), w = i % (4 * DT), dt = (w % (2 * DT)) / 2;
           constexpr bool isq = (w >= 2 * DT), hi = (w & 1) != 0;
           constexpr int off = offc + 16 * u * D * 2 + (isq ? 0 : offdo);
+          // (2m and 2m + 1: the operand of MFMA m of the next iteration)
           if constexpr (!isq && !hi) dtlo[u][dt] = lds_issue_tr4<off>(aT[dt][0] + sc);
           else if constexpr (!isq) dthi[u][dt] = lds_issue_tr4<off>(aT[dt][1] + sc);
           else if constexpr (!hi) qtlo[u][dt] = lds_issue_tr4<off>(aT[dt][0] + sc);
@@ -547,8 +583,8 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
         } else if constexpr (i < 8 * DT + 2 * KS) {
           constexpr int ks = (i - 8 * DT) / 2;
           if constexpr (WIDE) {
-            if constexpr (i % 2 == 0) qfr[ks] = lds_issue_b128_a<off2>(aQ[ks] + s2);
-            else dofr[ks] = lds_issue_b128_a<off2 + offdo>(aQ[ks] + s2);
+            if constexpr (i % 2 == 0) qf[ks] = lds_issue_b128_a<off2>(aQ[ks] + s2);
+            else dof[ks] = lds_issue_b128_a<off2 + offdo>(aQ[ks] + s2);
           } else {
             if constexpr (i % 2 == 0) qfr[ks] = lds_issue_b128<off2>(aQ[ks] + s2);
             else dofr[ks] = lds_issue_b128<off2 + offdo>(aQ[ks] + s2);
@@ -567,11 +603,18 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       };
       auto after = [&](auto mc) {
         constexpr int m = decltype(mc)::value;
+        if constexpr (WIDE) {
+          if constexpr (m < 8) {
+            lds_read(std::integral_constant<int, 2 * m>{});
+            lds_read(std::integral_constant<int, 2 * m + 1>{});
+          } else if constexpr (m < 16) lds_read(std::integral_constant<int, 8 + m>{});
+          else if constexpr (m == NM - 1) lds_read(std::integral_constant<int, NRD - 1>{});
+        }
         static_for<(8 * m) / NM, (8 * (m + 1)) / NM>(valu_pair);
         if constexpr ((8 * m) / NM == (8 * (m + 1)) / NM) {
           constexpr int e = m - (8 * m) / NM;
           // (all reads go into the first NGR gaps: the last ones issued still have a few MFMAs to land behind)
-          if constexpr (e < NGR) static_for<(e * NRD) / NGR, ((e + 1) * NRD) / NGR>(lds_read);
+          if constexpr (!WIDE && e < NGR) static_for<(e * NRD) / NGR, ((e + 1) * NRD) / NGR>(lds_read);
           // one copy of the stage whose slot the last barrier freed
           if constexpr (PRE && g == PRE_AT) old_issue(std::integral_constant<int, e>{});
           constexpr int since = (g - (TS - 2) + NJT) % NJT;  // iterations since the row's first barrier
@@ -579,19 +622,24 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
             stage_copy(std::integral_constant<int, (since / TS + 2) % STEPS>{}, std::integral_constant<int, (since % TS - 1) * NG + e>{});
         }
       };
-      // -- everything the previous iteration read has landed
-      dkdv1_lds_landed<KS, DT, true>(qf, dof, cstn, qtlo_p, qthi_p, dtlo_p, dthi_p);
+      // -- everything the previous iteration read has landed (D = 64: what the next MFMAs consume, see dkdv1_wait_step)
+      if constexpr (!WIDE) dkdv1_lds_landed<KS, DT, true>(qf, dof, cstn, qtlo_p, qthi_p, dtlo_p, dthi_p);
       u32x4 qtp[2][DT], dotp[2][DT];
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
+      auto operands = [&](auto uc) {
+        constexpr int u = decltype(uc)::value;
+        if constexpr (WIDE) dkdv1_wait_step<DT, 14 - u>(qtlo_p[u], qthi_p[u], dtlo_p[u], dthi_p[u]);
+        if constexpr (WIDE && u == 1) asm volatile("" : "+a"(qf[0]), "+a"(dof[0]));
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
           qtp[u][dt] = u32x4{qtlo_p[u][dt][0], qtlo_p[u][dt][1], qthi_p[u][dt][0], qthi_p[u][dt][1]};
           dotp[u][dt] = u32x4{dtlo_p[u][dt][0], dtlo_p[u][dt][1], dthi_p[u][dt][0], dthi_p[u][dt][1]};
         }
+      };
+      if constexpr (!WIDE) static_for<0, 2>(operands);
       // -- MFMAs that consume P and dS of tile g-1: dV^T += dO^T P, dK^T += Q^T dS
       static_for<0, 2>([&](auto uc) {
         constexpr int u = decltype(uc)::value;
+        if constexpr (WIDE) operands(uc);
         // (g == 1: starts the new row's accumulators; g == 0: the compiler may have just moved them)
         constexpr int mode = (g == 1 && u == 0) ? 2 : (g == 0 && u == 0) ? 1 : 0;
         const u32x4 pb = {pp_prev[4 * u], pp_prev[4 * u + 1], pp_prev[4 * u + 2], pp_prev[4 * u + 3]};
@@ -613,13 +661,14 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       const u32x4* vv = (g == NJT - 1) ? vf_n : vf;
       static_for<0, KS>([&](auto kc) {
         constexpr int ks = decltype(kc)::value;
-        mfma_rf<T, OPF, OPF, kV, (ks == 0) ? 3 : 0>(s_nxt, qf[ks], kk[ks]);
+        if constexpr (WIDE && ks == 1) dkdv1_wait_rest(qf, dof, cstn);
+        mfma_rf<T, OPF, KVF, kV, (ks == 0) ? 3 : 0>(s_nxt, qf[ks], kk[ks]);
         after(std::integral_constant<int, NM2 + PS * ks>{});
         if constexpr (HL) {
-          mfma_rf<T, OPF, OPF, kV, 0>(s_nxt, qf[ks], klo[ks]);
+          mfma_rf<T, OPF, KVF, kV, 0>(s_nxt, qf[ks], klo[ks]);
           after(std::integral_constant<int, NM2 + PS * ks + 1>{});
         }
-        mfma_rf<T, OPF, OPF, kV, (ks == 0) ? 3 : 0>(dp_nxt, dof[ks], vv[ks]);
+        mfma_rf<T, OPF, KVF, kV, (ks == 0) ? 3 : 0>(dp_nxt, dof[ks], vv[ks]);
         after(std::integral_constant<int, NM2 + PS * ks + PS - 1>{});
       });
       mfma_rf<F16, kA, kV, kV, 0>(s_nxt, biasA[gn][0], Eb[0]);
@@ -642,8 +691,9 @@ __global__ void __launch_bounds__(256) fta_bwd_dkdv1_kernel(const BwdParams p) {
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) { qtlo_p[u][dt] = qtlo[u][dt]; qthi_p[u][dt] = qthi[u][dt]; dtlo_p[u][dt] = dtlo[u][dt]; dthi_p[u][dt] = dthi[u][dt]; }
+      if constexpr (!WIDE)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) { qf[ks] = qfr[ks]; dof[ks] = dofr[ks]; }
+        for (int ks = 0; ks < KS; ++ks) { qf[ks] = qfr[ks]; dof[ks] = dofr[ks]; }
       cstn = cst;
     });
     // (nothing may copy registers with reads still in flight: settle them before the loop turns)
@@ -688,7 +738,7 @@ inline hipError_t launch_dkdv1_range(const BwdParams& p, int range, dim3 grid, s
     return tl ? launch_kernel(fta_bwd_dkdv1_kernel<T, D, NN, TS_, true, HL, NAT>, p, grid, dim3(256), smem, st)    \
               : launch_kernel(fta_bwd_dkdv1_kernel<T, D, NN, TS_, false, HL, NAT>, p, grid, dim3(256), smem, st);
   if constexpr (D == 64) {
-    FTA_DKDV1_CASE(8, 4) FTA_DKDV1_CASE(10, 5) FTA_DKDV1_CASE(12, 4)
+    FTA_DKDV1_CASE(8, 4) FTA_DKDV1_CASE(10, 5) FTA_DKDV1_CASE(12, 4) FTA_DKDV1_CASE(16, 4)
   } else {
     FTA_DKDV1_LATER(8, 8) FTA_DKDV1_LATER(10, 5) FTA_DKDV1_LATER(12, 6) FTA_DKDV1_LATER(14, 7) FTA_DKDV1_LATER(16, 8)
     FTA_DKDV1_CASE(8, 8) FTA_DKDV1_CASE(10, 5) FTA_DKDV1_CASE(12, 6) FTA_DKDV1_CASE(14, 7) FTA_DKDV1_CASE(16, 8)
