@@ -378,7 +378,7 @@ int fta_describe_plan_ex(int B, int H, int L1, int L2, int D, float sm_scale, co
     snprintf(dq, sizeof dq, "fta_bwd_short_kernel<%d,%d> launches=1 grid=%ld block=%d lds=%zu", D, b.sh.NT, bh * b.sh.nchunks, b.sh.threads, b.sh.smem);
     memcpy(dkdv, dq, sizeof dkdv);
   } else if (b.use_hand)
-    snprintf(dq, sizeof dq, "fta_bwd_dq1_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, b.dq1.SK, b.dq1.nlaunch,
+    snprintf(dq, sizeof dq, "fta_bwd_dq1%s_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", b.dq1.wide ? "w" : "", D, b.dq1.SK, b.dq1.nlaunch,
              bh * b.dq1.nqg * b.dq1.nchunks, b.dq1.threads, b.dq1.smem);
   else
     snprintf(dq, sizeof dq, "fta_bwd_dq_kernel<%d,%d> launches=%d grid=%ld block=%d lds=%zu", D, (D == 32 && b.NKT == 4) ? 2 : 1, b.nlaunch,

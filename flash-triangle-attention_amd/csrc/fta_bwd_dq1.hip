@@ -1,6 +1,6 @@
 // dQ and dBias, hand-scheduled: the launch plan, the dispatch and the fp16 instances (the kernel is in fta_bwd_dq1_kernel.h; the
 // bf16 instances are compiled in fta_bwd_dq1_bf16.hip).
-#include "fta_bwd_dq1_kernel.h"
+#include "fta_bwd_dq1w_kernel.h"
 
 namespace fta {
 
@@ -12,8 +12,33 @@ static int dq1_ranges(int L2, int D, int* out) {
 }
 static int dq1_slabs(int L2, int D) { return (D == 64 || L2 <= 256) ? 1 : 2; }
 
+// D = 64, rows of more than 384 keys: ranges of 256, 384 or 512 keys in one workgroup's two slabs, tiled to the next multiple of 128.  Q, dO and
+// O are read, and dQ written, once a range, and a range of up to 256 keys, as below, is half as long: training steps (us), those ranges / these:
+// B2 H8 400 keys 2823 / 2726, 448 in bf16 3170 / 3000, 460 3425 / 3215, 512 3895 / 3610 (dQ/dBias 1750 / 1360); B1 H4 530 1808 / 1652, 640 2293 / 2160,
+// 701 in bf16 3283 / 3109, 1024 8660 / 8000, 1536 29.4 / 27.2 ms.  Three or more ranges that are not equal stay as below (1408 keys: six launches), and
+// so do 257 to 384 keys, whose two ranges of up to 192 the two slabs of one would tile no shorter.
+static bool plan_dq1w(int B, int H, int L1, int L2, int row, Dq1Plan& pl) {
+  const int units = (row + 127) / 128;
+  const int n = row > 384 && row <= 512 * kMaxRanges ? even_ranges(units, 4, 128, pl.range) : 0;
+  if (n == 0 || (n > 2 && units % n != 0)) return false;
+  pl.Lt = units * 128;
+  pl.nlaunch = n;
+  pl.threads = 256;
+  pl.ring = 4; pl.nb = 1; pl.SK = 2; pl.QB = 2;
+  pl.nqg = (L2 + 63) / 64;
+  pl.KR = pl.range[0];
+  pl.smem = 160 * 1024;  // four stages of 32 KB, Q and dO rows of 16 KB, exchange records of 16 KB
+  for (int r = 0; r < n; ++r) pl.smem_range[r] = pl.smem;
+  const int nch = balanced_chunks((long)B * H * pl.nqg, L1, 256, least_rows(L2));
+  pl.rows_per_chunk = (L1 + nch - 1) / nch;
+  pl.nchunks = (L1 + pl.rows_per_chunk - 1) / pl.rows_per_chunk;
+  return true;
+}
+
 bool plan_dq1(int B, int H, int L1, int L2, int row, int D, Dq1Plan& pl) {
   if (D != 32 && D != 64) return false;
+  pl.wide = D == 64 && plan_dq1w(B, H, L1, L2, row, pl);
+  if (pl.wide) return true;
   // D = 64: the tiles end at the row's next multiple of 32 keys, whatever length dK/dV takes (that ends with the same
   // group of 128 queries, so the aux it reads is all written).  257 to 288 keys stay at two ranges of
   // 160, as 128 keys are less than the shortest instance.  Training step, before -> now: 150 keys 109 -> 90 us (8 -> 5 tiles),
@@ -56,6 +81,8 @@ hipError_t launch_dq1(BwdParams p, const Dq1Plan& pl, int D, int dtype, bool hil
   p.kr0 = 0;
   for (int n = 0; n < pl.nlaunch; ++n) {
     hipError_t e = hipErrorInvalidConfiguration;
+    if (pl.wide) e = dtype == kBF16 ? launch_dq1w_bf16(p, pl.range[n], grid, pl.smem, st) : launch_dq1w_range<F16>(p, pl.range[n], grid, pl.smem, st);
+    else
     // (nat: the caller asks for it at D = 32 with fp16 tensors only)
     if (nat) e = (dtype == kF16 && D == 32) ? launch_dq1_range<F16, 32, true, true>(p, pl.range[n], grid, pl.smem_range[n], st) : e;
     else if (dtype == kBF16) e = launch_dq1_bf16(p, pl.range[n], D, hilo, grid, pl.smem_range[n], st);

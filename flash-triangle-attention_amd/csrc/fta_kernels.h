@@ -142,7 +142,8 @@ struct Dq1Plan {
   int range[kMaxRanges];          // keys per launch
   size_t smem_range[kMaxRanges];
   size_t smem;                    // the largest
-  int Lt;                         // the length its tiles cover (D = 64: the next multiple of 32 keys)
+  int Lt;                         // the length its tiles cover (D = 64: the next multiple of 32 keys, `wide` of 128)
+  bool wide;                      // D = 64: ranges of up to 512 keys in two slabs (fta_bwd_dq1w_kernel.h)
 };
 struct Dkdv1Plan {
   int NJT, JR, nlaunch, nkg, nchunks, rows_per_chunk, threads;   // NJT, JR: of the first range

@@ -104,13 +104,16 @@ def test_head_dim_64_rows_of_an_odd_number_of_128_key_blocks(L1, L2):
     assert d["fwd"]["tiled_length"] == (384 if short else 1536)
 
 
-@pytest.mark.parametrize("L1,L2,queries", [(9, 449, 1), (5, 512, 1), (3, 576, 2), (3, 700, 2), (2, 830, 2), (3, 893, 2), (2, 960, 3), (2, 1024, 2)])
-def test_head_dim_64_query_ranges_of_up_to_512(L1, L2, queries):
-    """D=64, dK/dV: rows of 449 to 512 keys in one launch (16 tiles of the bias in a wave's accumulation registers, four
-    stages to a row), longer ones in ranges of 256, 320, 384 and 512 queries (eight and five units of 64 for 13, eight and six for 14)."""
+@pytest.mark.parametrize("L1,L2,keys,queries", [(1, 385, 1, 1), (9, 449, 1, 1), (5, 512, 1, 1), (3, 513, 2, 2), (3, 576, 2, 2), (3, 700, 2, 2), (2, 830, 2, 2),
+                                                (3, 893, 2, 2), (2, 960, 2, 3), (2, 1024, 2, 2), (1, 1152, 3, 3)])
+def test_head_dim_64_key_and_query_ranges_of_up_to_512(L1, L2, keys, queries):
+    """D=64.  dK/dV: rows of 385 to 512 keys in one launch (16 tiles of the bias in a wave's accumulation registers, four
+    stages to a row), longer ones in ranges of 256, 320, 384 and 512 queries (eight and five units of 64 for 13, eight and six for 14).
+    dQ/dBias: ranges of 256, 384 and 512 keys in two slabs (four, six and eight tiles), the second slab ending up to 127 keys beyond the row."""
     _case(2, 2, L1, L2, 64, 0.125, seed=29)
     import fta_lib
     d = fta_lib.describe_plan(2, 2, L1, L2, 64)
+    assert d["dq"]["kernel"].startswith("fta_bwd_dq1") and d["dq"]["launches"] == keys
     assert d["dkdv"]["kernel"].startswith("fta_bwd_dkdv1_kernel") and d["dkdv"]["launches"] == queries
 
 
