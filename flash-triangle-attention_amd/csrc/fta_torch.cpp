@@ -5,6 +5,7 @@
 // another device than the current one, a thread whose operations something else watches -- it leaves to the
 // Python path by returning None, which copies, records or raises as documented there.
 #include <ATen/autocast_mode.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
@@ -128,12 +129,19 @@ bool precise_now(PyObject* globals) {
 }
 
 // ---- attention -----------------------------------------------------------------------------------------
+// Outputs of the forward, straight from the allocator: nothing watches this thread's operations here (see `watched`), every element is
+// overwritten, and two trips through the dispatcher were a fifth of what a call costs the host.  A dense tensor's strides
+// are kept, as at::empty_like keeps them; any other layout is left to that.
+Tensor output_like(const Tensor& t) {
+  if (!t.is_non_overlapping_and_dense()) return at::empty_like(t);
+  return Tensor(at::detail::empty_strided_cuda(t.sizes(), t.strides(), t.scalar_type(), t.device()));
+}
 int attention_forward(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& b, double scale, const fta_options& opt,
                       Tensor& o, Tensor& lse) {
-  o = at::empty_like(q);  // keeps q's (possibly permuted) strides
+  o = output_like(q);
   if (!readable(o)) o = at::empty(q.sizes(), q.options());
   const auto n = q.sizes();
-  lse = at::empty({n[0], n[1], n[2], n[3]}, q.options().dtype(at::kFloat));
+  lse = Tensor(at::detail::empty_cuda({n[0], n[1], n[2], n[3]}, at::kFloat, q.device(), std::nullopt));
   const fta_tensor5 tq = t5(q), tk = t5(k), tv = t5(v), to = t5(o);
   const fta_tensor4 tb = t4(b);
   return fta_fwd_ex(&tq, &tk, &tv, &tb, &to, lse.data_ptr<float>(), (int)n[0], (int)n[1], (int)n[2], (int)n[3], (int)n[4],
@@ -390,6 +398,6 @@ PYBIND11_MODULE(fta_native, m) {
   m.doc() = "C++ host path of attention() and TriangleAttention; None = not taken, use the Python path";
   m.attr("built_for") = "fta_native built for torch " FTA_TORCH_VERSION;  // (read from the file before it is loaded, too)
   m.def("attention", &attention, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("b_pw"), py::arg("sm_scale"),
-        py::arg("dropout_p") = 0.0, py::arg("seed") = 0, py::kw_only(), py::arg("globals"));
+        py::arg("dropout_p") = 0.0, py::arg("seed") = 0, py::arg("globals"));
   m.def("block", &block);
 }

@@ -162,13 +162,16 @@ class _attention(torch.autograd.Function):
         function of its own, csrc/fta_torch.cpp): the interpreted path below costs 15 us a call, as much as
         the kernel at 64 keys.  What that path does not take -- and the precise mode -- comes here."""
         if 5 <= len(args) <= 7 and not PRECISE_BACKWARD:
-            if len(args) == 6 and float(args[5]) > 0.0:
-                args = args + (_draw_seed(),)
             native = _native or _load_native()
-            try:
-                o = native(*args[:4], *map(float, args[4:6]), *args[6:], globals=_GLOBALS)
-            except TypeError:  # (a seed that is no integer of 63 bits)
-                o = None
+            if len(args) == 5 and type(args[4]) is float:  # (the plain call, without keywords and conversions)
+                o = native(*args, 0.0, 0, _GLOBALS)
+            else:
+                if len(args) == 6 and float(args[5]) > 0.0:
+                    args = args + (_draw_seed(),)
+                try:
+                    o = native(*args[:4], *map(float, args[4:6]), *args[6:], globals=_GLOBALS)
+                except TypeError:  # (a seed that is no integer of 63 bits)
+                    o = None
             if o is not None:
                 return o
         return super(_attention, _attention).apply(*args)

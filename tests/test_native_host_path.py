@@ -417,3 +417,21 @@ def test_operands_on_another_device_are_refused(nth, device, grad):
     x[0].requires_grad_(grad)
     with pytest.raises(ValueError, match="same device"):
         attention(*x, 0.3)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["contiguous", "projection", "ending", "every other row", "one of two batches"])
+def test_the_output_has_the_strides_that_empty_like_gives(layout):
+    """The forward's output keeps a dense tensor's strides, whatever their order; of a tensor with gaps it takes the order."""
+    import flash_tt_attn as fta
+    q = {"contiguous": lambda: torch.randn(2, 4, 6, 40, 32), "projection": lambda: torch.randn(2, 6, 40, 4, 32).permute(0, 3, 1, 2, 4),
+         "ending": lambda: torch.randn(2, 4, 40, 6, 32).transpose(2, 3), "every other row": lambda: torch.randn(2, 4, 12, 40, 32)[:, :, ::2],
+         "one of two batches": lambda: torch.randn(4, 6, 4, 40, 32).permute(0, 2, 1, 3, 4)[::2]}[layout]()
+    storage = torch.empty(q.untyped_storage().nbytes() // 4, dtype=torch.float16, device="cuda").normal_()
+    q = storage.as_strided(q.shape, q.stride(), q.storage_offset())
+    b = torch.randn(2, 4, 40, 40, device="cuda", dtype=torch.float16)
+    for grad in (False, True):
+        o = fta.attention(q.detach().requires_grad_(grad), q, q, b, 0.2)
+        assert o.stride() == torch.empty_like(q).stride() and o.storage_offset() == 0
+        ref = torch.nn.functional.scaled_dot_product_attention(q.float().cpu(), q.float().cpu(), q.float().cpu(), b.float().cpu()[:, :, None], scale=0.2)
+        assert (o.detach().float().cpu() - ref).abs().max() <= 1e-2
