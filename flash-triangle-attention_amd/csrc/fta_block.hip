@@ -481,17 +481,6 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
   const int teams = (int)gridDim.x / PARTS, part = (int)blockIdx.x / teams;
   auto tile_of = [=](int t) { return (t * 8 + wave) * PARTS + part; };  // (the gate's tiles, which have the sigmoid besides, spread over waves and parts)
   const int c8 = (tid % (C / 8)) * 8;
-  float wbv[F32 ? 4 : 1][8];  // (fp32) the bias heads' weights of this thread's channels
-  if constexpr (F32) {
-#pragma unroll
-    for (int h = 0; h < 4; ++h)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) wbv[h][e] = h < p.H ? load1<A, F32>(p.wb, h * C + c8 + e) : 0.f;
-  }
-  float gam[8], bet[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) { gam[e] = load1<A, F32>(p.gamma, c8 + e); bet[e] = load1<A, F32>(p.beta, c8 + e); }
-
   const int LL = (int)p.LL, nst = (LL + TR - 1) / TR, ntot = p.B * nst;
   const float inv_l = 1.0f / (float)p.L;
   Frag<F32> z[NP];
@@ -512,6 +501,8 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
       z[n] = load8<F32>(p.z, b * p.zs[0] + (int64_t)i * p.zs[1] + (int64_t)j * p.zs[2] + c8);
     }
   };
+  float wbv[F32 ? 4 : 1][8];  // (fp32) the bias heads' weights of this thread's channels (of the last head for heads there are not)
+  float gam[8], bet[8];
   auto put = [&](int buffer) {
     char* buf = smem + buffer * BUF;
     // 0 marks padded key positions, which no query may attend to
@@ -545,24 +536,43 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
       if (TR * C / 8 >= 512 || row < TR) piece_write<F32>(buf + (row / 32) * SUB, row % 32, c8 / 8, f);
     }
   };
+  // Every load that the first stage waits for is issued here, with no branch and no other load's result in between.
+  // (With a pointer per lane, the bias heads' weights under a branch each and the gate's bias behind the weights, four latencies followed
+  // each other and a workgroup's first products began after 27k of its 86k cycles at 192 x 192 pairs in fp32.)
   int st = (int)blockIdx.x - part * teams;
-  if (st < ntot) fetch(st);  // (in flight while the weights come in)
-  Op<F32> w[NT][KS];
+  fetch(min(st, ntot - 1));
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+  for (int e = 0; e < 8; ++e) { gam[e] = load1<A, F32>(p.gamma, c8 + e); bet[e] = load1<A, F32>(p.beta, c8 + e); }
+  if constexpr (F32) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int n = tile_of(t) * 32 + l32, sec = n / HD;
-      w[t][ks] = to_op(load8<F32>(p.w[sec], (int64_t)(n - sec * HD) * C + ks * 16 + hh * 8));
-    }
-  if constexpr (!F32)
-    for (int ks = wave; ks < KS; ks += 8)
-      op_write<F32>(wbf, ks, lane, to_op(l32 < p.H ? load8<F32>(p.wb, (int64_t)l32 * C + ks * 16 + hh * 8) : frag_zero<F32>()));
-  for (int c = tid; c < HD; c += 512) bgs[c] = p.bg != nullptr ? load1<A, F32>(p.bg, c) : 0.f;
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) wbv[h][e] = load1<A, F32>(p.wb, min(h, p.H - 1) * C + c8 + e);
+  }
+  Frag<F32> wraw[NT][KS];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int n0 = tile_of(t) * 32, sec = n0 / HD;  // (a tile is of one projection)
+    const void* ws = p.w[sec];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) wraw[t][ks] = load8<F32>(ws, (int64_t)(n0 - sec * HD + l32) * C + ks * 16 + hh * 8);
+  }
+  static_assert(KS <= 8 && HD <= 512, "a wave has one step of the bias heads' weights, a thread one entry of the gate's bias");
+  [[maybe_unused]] Frag<F32> wbr;
+  if constexpr (!F32) wbr = load8<F32>(p.wb, (int64_t)min(l32, p.H - 1) * C + min(wave, KS - 1) * 16 + hh * 8);
+  const float bg = load1<A, F32>(p.bg != nullptr ? p.bg : p.gamma, p.bg != nullptr ? min(tid, HD - 1) : 0);
   if (st < ntot) {
     put(0);
     fetch(min(st + teams, ntot - 1));
   }
+  Op<F32> w[NT][KS];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) w[t][ks] = to_op(wraw[t][ks]);
+  if constexpr (!F32)
+    if (wave < KS) op_write<F32>(wbf, wave, lane, to_op(l32 < p.H ? wbr : frag_zero<F32>()));
+  if (tid < HD) bgs[tid] = p.bg != nullptr ? bg : 0.f;
   __syncthreads();
   // the tile of channels n .. n + 31 of pair rows q0 .. q0 + 31
   // (rows beyond the end repeat the last one, and store the same values to the same place: with no branch
@@ -658,19 +668,23 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
   constexpr int KS = HD / 16, NT = C / 32;
   extern __shared__ char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
-  const int nw = blockDim.x >> 6;
+  constexpr int NW = 8, NF = NT * KS / NW;  // waves; weight fragments that a wave brings
+  static_assert(NT * KS % NW == 0 && C <= 64 * NW, "shares of the weights");
   float* bos = reinterpret_cast<float*>(smem + (size_t)NT * KS * kOpBytes<F32>);
-  for (int idx = wave; idx < NT * KS; idx += nw)
-    op_write<F32>(smem, idx, lane, to_op(load8<F32>(p.wo, (int64_t)((idx / KS) * 32 + l32) * HD + (idx % KS) * 16 + hh * 8)));
-  for (int c = tid; c < C; c += blockDim.x) bos[c] = p.bo != nullptr ? load1<A, F32>(p.bo, c) : 0.f;
-  __syncthreads();
-
-  const int nitems = p.B * p.nper * p.cg, step = (int)gridDim.x * nw;
-  int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * nw + wave);
-  if (item >= nitems) return;
+  // The weights and the first rows are asked for together (a fragment at a time, and the rows behind the barrier, were six latencies in
+  // a row: at 192 x 192 pairs a wave has one or two row blocks)
+  Frag<F32> wf[NF];
+#pragma unroll
+  for (int n = 0; n < NF; ++n) {
+    const int idx = wave + NW * n;
+    wf[n] = load8<F32>(p.wo, (int64_t)((idx / KS) * 32 + l32) * HD + (idx % KS) * 16 + hh * 8);
+  }
+  float bo = load1<A, F32>(p.bo != nullptr ? p.bo : p.wo, p.bo != nullptr ? min(tid, C - 1) : 0);
+  const int nitems = p.B * p.nper * p.cg, step = (int)gridDim.x * NW;
+  int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * NW + wave);
   Frag<F32> gt[KS];
   Frag<false> o[KS];
-  RowBlock rb = row_block(p, item / p.cg, lane);
+  RowBlock rb = row_block(p, min(item, nitems - 1) / p.cg, lane);
   auto fetch = [&]() {
 #pragma unroll
     for (int ks = 0; ks < KS; ks += 2) {
@@ -681,6 +695,13 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
       load_runs<false>(p.o, at0, at1, lane, o[ks], o[ks + 1]);
     }
   };
+  fetch();
+  asm volatile("" : "+v"(bo));  // (not asked for under the branch below)
+#pragma unroll
+  for (int n = 0; n < NF; ++n) op_write<F32>(smem, wave + NW * n, lane, to_op(wf[n]));
+  if (tid < C) bos[tid] = p.bo != nullptr ? bo : 0.f;
+  __syncthreads();
+  if (item >= nitems) return;
   auto store_tile = [&](const floatx16& acc, int t, const RowBlock& r) {
     const int64_t oo = pair_off(p.outs, r) + hh * 8;
     float y[2][8];
@@ -696,7 +717,6 @@ __global__ void __launch_bounds__(512) blk_out_kernel(BlockParams p) {
   };
   [[maybe_unused]] bool bad = false;
   [[maybe_unused]] const int item0 = item;
-  fetch();
   for (; item < nitems; item += step) {
     const RowBlock cur = rb;
     const int g = item % p.cg;
@@ -756,11 +776,12 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
   constexpr int KS = C / 16, NT = HD / 32;
   extern __shared__ char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, hh = lane >> 5;
-  const int nw = blockDim.x >> 6;
+  constexpr int NW = 8, NF = NT * KS / NW;  // (as in blk_out_kernel)
+  static_assert(NT * KS % NW == 0, "shares of the weights");
   if ((int)blockIdx.x >= p.nwg) {
     constexpr int ksall = 4 * HD / 16 + 1;
     const int npack = (int)gridDim.x - p.nwg;
-    for (int idx = ((int)blockIdx.x - p.nwg) * nw + wave; idx < (C / 32) * ksall; idx += npack * nw) {
+    for (int idx = ((int)blockIdx.x - p.nwg) * NW + wave; idx < (C / 32) * ksall; idx += npack * NW) {
       const int ct = idx / ksall, ks = idx % ksall, c = ct * 32 + l32;
       float v[8];
 #pragma unroll
@@ -775,29 +796,32 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
     }
     return;
   }
-  for (int idx = wave; idx < NT * KS; idx += nw) {
-    float v[8];
+  float wv[NF][8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = load1<A, F32>(p.wo, (int64_t)((idx % KS) * 16 + hh * 8 + e) * HD + (idx / KS) * 32 + l32);
-    Frag<F32> f;
-    pack<A>(v, f);
-    op_write<F32>(smem, idx, lane, to_op(f));
-  }
-  __syncthreads();
-
-  const int nitems = p.B * p.nper * p.cg, step = p.nwg * nw;
-  int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * nw + wave);
-  if (item >= nitems) return;
-  Op<F32> x[KS];
-  RowBlock rb = row_block(p, item / p.cg, lane);
+  for (int n = 0; n < NF; ++n)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int idx = wave + NW * n;
+      wv[n][e] = load1<A, F32>(p.wo, (int64_t)((idx % KS) * 16 + hh * 8 + e) * HD + (idx / KS) * 32 + l32);
+    }
+  const int nitems = p.B * p.nper * p.cg, step = p.nwg * NW;
+  int item = __builtin_amdgcn_readfirstlane((int)blockIdx.x * NW + wave);
+  Frag<F32> f[KS];  // the next row block
+  RowBlock rb = row_block(p, min(item, nitems - 1) / p.cg, lane);
   auto fetch = [&]() {
     const int64_t so = pair_off(p.douts, rb) + hh * 8;
-    Frag<F32> f[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) f[ks] = load8<F32>(p.dout, so + ks * 16);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) x[ks] = to_op(f[ks]);
   };
+  fetch();
+#pragma unroll
+  for (int n = 0; n < NF; ++n) {
+    Frag<F32> fw;
+    pack<A>(wv[n], fw);
+    op_write<F32>(smem, wave + NW * n, lane, to_op(fw));
+  }
+  __syncthreads();
+  if (item >= nitems) return;
   auto head_at = [&](int t, const RowBlock& r) { const int h = t * 32 / p.D; return head_off(p, r, h) + (t * 32 - h * p.D) + hh * 8; };
   auto operands = [&](int t, const RowBlock& r, Frag<F32> (&gt)[2], Frag<false> (&o)[2]) {
     int64_t at0, at1;
@@ -830,10 +854,16 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
   };
   [[maybe_unused]] bool bad = false;
   [[maybe_unused]] const int item0 = item;
-  fetch();
   for (; item < nitems; item += step) {
     const RowBlock cur = rb;
     const int g = item % p.cg;
+    Op<F32> x[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) x[ks] = to_op(f[ks]);
+    if (item + step < nitems) {
+      rb = row_block(p, (item + step) / p.cg, lane);
+      fetch();
+    }
     for (int t = g; t < NT; t += p.cg) {
       Frag<F32> gt[2];
       Frag<false> o[2];
@@ -843,10 +873,6 @@ __global__ void __launch_bounds__(512) blk_dout_kernel(BlockParams p) {
       for (int ks = 0; ks < KS; ++ks) acc = mma<A>(op_read<F32>(smem, t * KS + ks, lane), x[ks], acc);
       if constexpr (F32) bad = bad || not_finite(acc);
       store_tile(acc, t, cur, gt, o);
-    }
-    if (item + step < nitems) {
-      rb = row_block(p, (item + step) / p.cg, lane);
-      fetch();
     }
   }
   if constexpr (F32)
