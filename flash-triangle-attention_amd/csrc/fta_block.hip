@@ -36,6 +36,7 @@
 // library calls around the attention, 0.52 with these; us per kernel (rocprofv3, mean of 30 launches): proj 56, out
 // 30, dout 43, dx 47, wgrad 66, reduce 11, norm_grad 5.
 #include "fta_block.h"
+#include "fta_pipe.h"
 
 #include <type_traits>
 
@@ -77,6 +78,8 @@ __device__ __forceinline__ Op<true> to_op(const Frag<true>& f) {
       } else {
         w = BF16::pack(a, b);
       }
+      // (the compiler would convert each half once more by itself, to subtract it)
+      if (n < 2) asm("" : "+v"(w));
       o.p[n][e] = w;
       a -= BF16::lo(w);
       b -= BF16::hi(w);
@@ -84,13 +87,13 @@ __device__ __forceinline__ Op<true> to_op(const Frag<true>& f) {
   }
   return o;
 }
-template <class A, int PA = 3, bool LONG = false>
+template <class A, int PA = 3, bool LONG = false, int PB = 3>
 __device__ __forceinline__ floatx16 mma(const Op<false>& a, const Op<false>& b, floatx16 c) {
   return A::mfma(as_half8(a.p[0]), as_half8(b.p[0]), c);
 }
-// (PA: planes of `a` that are not zero: two hold the 11 bits of an fp16 value.  LONG: a sum over many steps; the small
+// (PA, PB: planes of `a` and `b` that are not zero: two hold the 11 bits of an fp16 value.  LONG: a sum over many steps; the small
 // products are summed by themselves first, so that the long sum is rounded twice a step and not six times)
-template <class A, int PA = 3, bool LONG = false>
+template <class A, int PA = 3, bool LONG = false, int PB = 3>
 __device__ __forceinline__ floatx16 mma(const Op<true>& a, const Op<true>& b, floatx16 c) {
   constexpr int at[6][2] = {{2, 0}, {0, 2}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};
   floatx16 t = c;
@@ -98,7 +101,8 @@ __device__ __forceinline__ floatx16 mma(const Op<true>& a, const Op<true>& b, fl
 #pragma unroll
     for (int r = 0; r < 16; ++r) t[r] = 0.f;
 #pragma unroll
-  for (int n = PA == 3 ? 0 : 1; n < (LONG ? 5 : 6); ++n) t = BF16::mfma(as_half8(a.p[at[n][0]]), as_half8(b.p[at[n][1]]), t);
+  for (int n = 0; n < (LONG ? 5 : 6); ++n)
+    if (at[n][0] < PA && at[n][1] < PB) t = BF16::mfma(as_half8(a.p[at[n][0]]), as_half8(b.p[at[n][1]]), t);
   if constexpr (LONG) {
     c = BF16::mfma(as_half8(a.p[0]), as_half8(b.p[0]), c);
 #pragma unroll
@@ -219,19 +223,20 @@ __device__ __forceinline__ Frag<F32> frag_zero() {
 
 // Operands in LDS: a 16-byte plane of 64 lanes each, three for fp32.
 template <bool F32> constexpr int kOpBytes = F32 ? 3072 : 1024;
-template <bool F32>
+// (PL: the fp32 planes that are not zero)
+template <bool F32, int PL = 3>
 __device__ __forceinline__ Op<F32> op_read(const char* ops, int idx, int lane) {
   Op<F32> o;
   const char* s = ops + (size_t)idx * kOpBytes<F32> + lane * 16;
 #pragma unroll
-  for (int n = 0; n < kOpBytes<F32> / 1024; ++n) o.p[n] = *reinterpret_cast<const u32x4*>(s + n * 1024);
+  for (int n = 0; n < (F32 ? PL : 1); ++n) o.p[n] = *reinterpret_cast<const u32x4*>(s + n * 1024);
   return o;
 }
-template <bool F32>
+template <bool F32, int PL = 3>
 __device__ __forceinline__ void op_write(char* ops, int idx, int lane, const Op<F32>& o) {
   char* d = ops + (size_t)idx * kOpBytes<F32> + lane * 16;
 #pragma unroll
-  for (int n = 0; n < kOpBytes<F32> / 1024; ++n) *reinterpret_cast<u32x4*>(d + n * 1024) = o.p[n];
+  for (int n = 0; n < (F32 ? PL : 1); ++n) *reinterpret_cast<u32x4*>(d + n * 1024) = o.p[n];
 }
 
 // An accumulator tile (lane: column l % 32; register r: row 8*(r/4) + 4*hh + r%4) as two runs of eight
@@ -415,13 +420,13 @@ __device__ __forceinline__ void normalise(float (&v)[8], float eps, float& mean,
 // next ones), and sits in LDS as MFMA B operands, one 16-byte slot per (row, 8 elements) and plane.  Slot
 // of row r, piece c of a 32-row sub-block: ((c / 2) * 64 + (r ^ (c % 16)) + 32 * (c % 2)): the XOR spreads the
 // pieces of a row, which neighbouring threads write at once, over the banks.
-template <bool F32>
+template <bool F32, int PL = 3>
 __device__ __forceinline__ void piece_write(char* blk, int r, int c, const Frag<F32>& f) {
-  op_write<F32>(blk, c / 2, (r ^ (c % 16)) + 32 * (c % 2), to_op(f));
+  op_write<F32, PL>(blk, c / 2, (r ^ (c % 16)) + 32 * (c % 2), to_op(f));
 }
-template <bool F32>
+template <bool F32, int PL = 3>
 __device__ __forceinline__ Op<F32> piece_frag(const char* blk, int ks, int l32, int hh) {
-  return op_read<F32>(blk, ks, (l32 ^ ((2 * ks + hh) % 16)) + 32 * hh);
+  return op_read<F32, PL>(blk, ks, (l32 ^ ((2 * ks + hh) % 16)) + 32 * hh);
 }
 
 // (fp32) A tile of projections by the fp32 instruction: the lane's pair row at element `row` of z, its weight row at
@@ -962,7 +967,7 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
           Frag<F32> f;
           if constexpr (F32) unpack<A>(d[s][n], f.v);
           else f = d[s][n];
-          piece_write<F32>(blk, row % 32, s * (HD / 8) + c, f);
+          piece_write<F32, 2>(blk, row % 32, s * (HD / 8) + c, f);
         }
         piece_write<F32>(blk, row % 32, 3 * (HD / 8) + c, dg[n]);
       }
@@ -975,17 +980,20 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
       Frag<F32> f;
       pack<A>(v, f);
       const int row = tid % TR;
-      piece_write<F32>(smem + (row / 32) * SUB, row % 32, 4 * (HD / 8) + tid / TR, f);
+      piece_write<F32, 2>(smem + (row / 32) * SUB, row % 32, 4 * (HD / 8) + tid / TR, f);
     }
   };
   int st = (int)blockIdx.x;
-  if (st < ntot) fetch(st);  // (in flight while the weights come in)
+  fetch(min(st, ntot - 1));  // (in flight while the weights come in)
+  // A share takes every SPLIT-th step, so that all have the same number from the fp16 gradients, whose third plane is zero.  The last step is
+  // one share's (the others': the last one again, with zero weights).
+  static_assert(3 * KH % SPLIT == 0 && KH % SPLIT == 0, "even shares of every section");
+  auto step_of = [=](int k) { return SPLIT == 1 ? k : min(k * SPLIT + share, KALL - 1); };
+  constexpr int KP = 3 * KH / SPLIT;   // a share's steps from the fp16 gradients of q, k and v
   Frag<F32> w[KW];
 #pragma unroll
-  for (int k = 0; k < KW; ++k) {
-    const int ks = share * KW + k;
-    w[k] = ks < KALL ? frag_read<F32>(static_cast<const char*>(p.wt), ct * KALL + ks, lane) : frag_zero<F32>();
-  }
+  for (int k = 0; k < KW; ++k) w[k] = frag_read<F32>(static_cast<const char*>(p.wt), ct * KALL + step_of(k), lane);
+  if (SPLIT > 1 && share > 0) w[KW - 1] = frag_zero<F32>();
   if (st < ntot) put();
   __syncthreads();
   // the sums of a stage through LDS to the rows' threads, and the layer norm's backward
@@ -1035,12 +1043,26 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
     const int next = st + (int)gridDim.x;
 #pragma unroll
     for (int n = 0; n < NZ; ++n) z[n] = load8<F32>(p.z, pair_off_of(p.zs, st, n));
-    fetch(min(next, ntot - 1));
+    if constexpr (!F32) fetch(min(next, ntot - 1));
     floatx16 acc = zero16();
+    if constexpr (F32) {
+      // (the next step's operands are read during this one's products; the registers for that are the next stage's rows', which are
+      // asked for behind the products)
+      auto operand = [&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        return piece_frag<F32, (k < KP || k == KW - 1) ? 2 : 3>(smem + rs * SUB, step_of(k), l32, hh);
+      };
+      Op<F32> x = operand(std::integral_constant<int, 0>{});
+      static_for<0, KW>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        const Op<F32> cur = x;
+        if constexpr (k + 1 < KW) x = operand(std::integral_constant<int, k + 1>{});
+        acc = mma<A, 3, false, (k < KP || k == KW - 1) ? 2 : 3>(to_op<true>(w[k]), cur, acc);
+      });
+      fetch(min(next, ntot - 1));
+    } else {
 #pragma unroll
-    for (int k = 0; k < KW; ++k) {
-      const int ks = SPLIT == 1 ? k : min(share * KW + k, KALL - 1);  // (a share's steps beyond the end: the last one again, with zero weights)
-      acc = mma<A>(to_op<true>(w[k]), piece_frag<F32>(smem + rs * SUB, ks, l32, hh), acc);
+      for (int k = 0; k < KW; ++k) acc = mma<A>(to_op<true>(w[k]), piece_frag<F32>(smem + rs * SUB, step_of(k), l32, hh), acc);
     }
     if constexpr (F32) bad = bad || not_finite(acc);
     finish(acc, st);
@@ -1057,7 +1079,7 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
       const int b = st / nst, q = min((st - b * nst) * TR + rs * 32 + l32, LL - 1);
       floatx16 acc = zero16();
 #pragma clang loop unroll(disable)
-      for (int ks = share * KW; ks < min(share * KW + KW, KALL); ++ks) {
+      for (int ks = share; ks < KALL; ks += SPLIT) {
         const int s = ks / KH, e8 = (ks % KH) * 16 + hh * 8, h = e8 / p.D;
         const int64_t off = (((int64_t)b * p.H + h) * LL + q) * p.D + (e8 - h * p.D);
         float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
