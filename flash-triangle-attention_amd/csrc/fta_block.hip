@@ -670,8 +670,8 @@ __global__ void __launch_bounds__(512) blk_proj_kernel(BlockParams p) {
 // ---- forward: gating and output projection ------------------------------------------------------------
 // The first item (a column group of a row block) of a wave, in steps of all waves: neighbouring waves take the groups of a row block, then
 // comes the next workgroup, so that where the items are no multiple of the waves, the last ones are spread over all CUs.  (Workgroup after
-workgroup, the first 32 of 256 had two items per wave and the others one at 192 x 192 pairs in fp32: out 24.0 / 19.4 us, dout 24.4 / 21.2;
-at 384 x 384 in bf16 27.0 / 25.9 and 39.2 / 36.5.)
+// workgroup, the first 32 of 256 had two items per wave and the others one at 192 x 192 pairs in fp32: out 24.0 / 19.4 us, dout 24.4 / 21.2;
+// at 384 x 384 in bf16 27.0 / 25.9 and 39.2 / 36.5.)
 __device__ __forceinline__ int first_item(int cg, int nwg, int wave) {
   return __builtin_amdgcn_readfirstlane(((wave / cg) * nwg + (int)blockIdx.x) * cg + wave % cg);
 }
