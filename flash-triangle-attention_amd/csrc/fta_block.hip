@@ -30,13 +30,15 @@
 // bf16 (beyond 3.39e38), have no three parts: a tile whose sums are not all finite is formed again by the fp32 instruction,
 // so that infinities come out as they went in.  Nothing is rounded to 16 bits in memory that was not before (q, k, v, bias, o and their gradients).
 // us per kernel at 192 x 192 pairs, before and after: proj 69 / 47, out 32 / 26, dout 29 / 28, dx 57 / 48, wgrad 82 / 50; a
-// training pass 352 / 265 (256 x 256: 498 / 394, 321 x 321: 838 / 670), inference 112 / 82 (457 x 457: 505 / 387).
+// training pass 352 / 265 (256 x 256: 498 / 394, 321 x 321: 838 / 670), inference 112 / 82 (457 x 457: 505 / 387).  A workgroup there has few
+// rows, so that what it waits for before the first of them counts: with every load that the first row needs asked for at once, row blocks dealt to the
+// workgroups in turn and dx's operands read a step ahead proj 41, out 19, dout 21, dx 40, wgrad 46; a training pass 238 (beside 267; 256 x 256: 383
+// beside 416, 321 x 321 645 beside 690), inference 80 beside 90 (457 x 457: 370 beside 384).
 //
 // Measured, AlphaFold2's block (C 128, 4 heads of 32) at 384 x 384 pairs in bf16: a training pass 3.64 ms as separate
-// library calls around the attention, 0.52 with these; us per kernel (rocprofv3, mean of 30 launches): proj 56, out
-// 30, dout 43, dx 47, wgrad 66, reduce 11, norm_grad 5.
+// library calls around the attention, 0.47 with these; us per kernel (rocprofv3, median of 40 launches): proj 49, out
+// 26, dout 37, dx 46, wgrad 62, reduce 10, norm_grad 5.
 #include "fta_block.h"
-#include "fta_pipe.h"
 
 #include <type_traits>
 
@@ -44,6 +46,7 @@
 
 #include "fta_common.h"
 #include "fta_kernels.h"
+#include "fta_pipe.h"
 
 namespace fta {
 namespace {
@@ -992,11 +995,12 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
   };
   int st = (int)blockIdx.x;
   fetch(min(st, ntot - 1));  // (in flight while the weights come in)
-  // A share takes every SPLIT-th step, so that all have the same number from the fp16 gradients, whose third plane is zero.  The last step is
-  // one share's (the others': the last one again, with zero weights).
+  // A share takes every SPLIT-th step, so that all have the same number from the fp16 gradients, whose third plane is zero, and begins with the
+  // gate's: dz against 64 bits at 192 x 192 pairs in fp32 1.91e-7, with the gate's behind q, k and v, which are larger, 2.33e-7 (half of the
+  // contraction in a row for each share 2.27e-7).  The last step is one share's (the others': the last one again, with zero weights).
   static_assert(3 * KH % SPLIT == 0 && KH % SPLIT == 0, "even shares of every section");
-  auto step_of = [=](int k) { return SPLIT == 1 ? k : min(k * SPLIT + share, KALL - 1); };
-  constexpr int KP = 3 * KH / SPLIT;   // a share's steps from the fp16 gradients of q, k and v
+  constexpr int KG = KH / SPLIT;   // a share's steps of a section
+  auto step_of = [=](int k) { return SPLIT == 1 ? k : k < KG ? (k + 3 * KG) * SPLIT + share : k < 4 * KG ? (k - KG) * SPLIT + share : KALL - 1; };
   Frag<F32> w[KW];
 #pragma unroll
   for (int k = 0; k < KW; ++k) w[k] = frag_read<F32>(static_cast<const char*>(p.wt), ct * KALL + step_of(k), lane);
@@ -1057,14 +1061,14 @@ __global__ void __launch_bounds__(512) blk_dx_kernel(BlockParams p) {
       // asked for behind the products)
       auto operand = [&](auto kc) {
         constexpr int k = decltype(kc)::value;
-        return piece_frag<F32, (k < KP || k == KW - 1) ? 2 : 3>(smem + rs * SUB, step_of(k), l32, hh);
+        return piece_frag<F32, (k >= KG) ? 2 : 3>(smem + rs * SUB, step_of(k), l32, hh);
       };
       Op<F32> x = operand(std::integral_constant<int, 0>{});
       static_for<0, KW>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
         const Op<F32> cur = x;
         if constexpr (k + 1 < KW) x = operand(std::integral_constant<int, k + 1>{});
-        acc = mma<A, 3, false, (k < KP || k == KW - 1) ? 2 : 3>(to_op<true>(w[k]), cur, acc);
+        acc = mma<A, 3, false, (k >= KG) ? 2 : 3>(to_op<true>(w[k]), cur, acc);
       });
       fetch(min(next, ntot - 1));
     } else {
@@ -1473,12 +1477,25 @@ __global__ void __launch_bounds__(1024) blk_reduce_kernel(BlockParams p) {
   __syncthreads();
   float dg[4] = {0.f, 0.f, 0.f, 0.f}, db[4] = {0.f, 0.f, 0.f, 0.f};
   if (grp == 0 && valid) {
-    float g[4] = {a.x, a.y, a.z, a.w};
-    for (int k = 1; k < groups; ++k) {
-      const float4 v = part[tid + k * quads];
-      g[0] += v.x; g[1] += v.y; g[2] += v.z; g[3] += v.w;
-      sum += psum[tid + k * quads];
+    // (four sums side by side: twice as many groups in a row round once more often than half as many did)
+    float g4[4][4], s4[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      s4[u] = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) g4[u][e] = 0.f;
     }
+    for (int k = 0; k < groups; k += 4)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float4 v = part[tid + (k + u) * quads];
+        g4[u][0] += v.x; g4[u][1] += v.y; g4[u][2] += v.z; g4[u][3] += v.w;
+        s4[u] += psum[tid + (k + u) * quads];
+      }
+    float g[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) g[e] = (g4[0][e] + g4[1][e]) + (g4[2][e] + g4[3][e]);
+    sum = (s4[0] + s4[1]) + (s4[2] + s4[3]);
     if (proj) {
       void* dst = sec < 4 ? p.dw[sec] : p.dwb;
       const void* w = sec < 4 ? p.w[sec] : p.wb;

@@ -159,6 +159,14 @@ def test_fused_block_kernels_against_separate_operations(C, H, D, B, L, starting
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("L,dtype", [(192, torch.float32), (257, torch.float32), (363, torch.bfloat16)])
+def test_row_blocks_beyond_a_round_of_the_waves(L, dtype):
+    """The output and gate-gradient kernels deal row blocks of 32 pairs to the workgroups in turn.  2304 halves of row blocks, 2065 and 4118 whole
+    ones for 2048, 2048 and 4096 waves: a second round that few of the waves have.  Same tolerance as above."""
+    test_fused_block_kernels_against_separate_operations(128, 4, 32, 1, L, True, False, 0.0, dtype)
+
+
+@pytest.mark.gpu
 def test_block_dropout_draws_a_fresh_mask_per_call_and_replays_a_given_seed():
     torch.manual_seed(3)
     dev = "cuda:0"
