@@ -8,7 +8,10 @@
 //   * the registers of an operand are filled again right behind the MFMA that consumes it: 16 reads an iteration, in the order of
 //     their use one iteration later, so that each wait leaves the last 12 in flight;
 //   * slab s finishes d = 32 s .. +31 of the row: its operands of K^T are addressed so that acc[0] is its own half of d and
-//     acc[1] the partner's, which goes through LDS once a row (the halves meet in fp32).
+//     acc[1] the partner's, which goes through LDS once a row (the halves meet in fp32).  A wave writes its record in iteration 0 of the next row
+//     and its partner reads it in iterations 2 and 3; barriers open every even iteration.  So write -> read has the barrier of iteration 2 between, and
+//     read -> next row's write that of iteration 0.  The last row's record is written behind the loop: six and eight tiles have the
+//     barrier of iteration 4 between the read and that, four tiles need one of their own there.
 //
 // Bound: matrix core and power (18 MFMAs a tile), issue (166 instructions) and memory in about equal parts: 1360 us at B2 H8 L512, 1200 cycles a
 // tile.  Two launches over 256 keys each, of workgroups of 128 queries, read Q, dO, O and wrote dQ twice: 2 x 876 us.
@@ -508,6 +511,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1w_kernel(const BwdParams p) {
     for (int dt = 0; dt < DT; ++dt) acc[dt] = T::mfma(as_half8(u32x4{ktlo[u][dt][0], ktlo[u][dt][1], kthi[u][dt][0], kthi[u][dt][1]}), db, acc[dt]);
   }
   if constexpr (LATER) old_issue();
+  if constexpr (NKT == 4) __syncthreads();  // (the partner has read the record of the row before: no barrier of the loop lies behind iteration 3)
   {
     float* out = reinterpret_cast<float*>(smem_raw + R * SLOT_B + 2 * QTILE_B) + wave * 1024 + ln * 4;
     const float* in = reinterpret_cast<const float*>(smem_raw + R * SLOT_B + 2 * QTILE_B) + (wave ^ 1) * 1024 + ln * 4;

@@ -30,6 +30,11 @@ that the compiler does not recognise as MFMAs:
     block ends, is read or written (copied, spilled, added ...) on some way through the branches before a
     wait that covers the load.
 
+and for the records through which the waves of a two-slab dQ/dBias kernel hand each other their shares of a row:
+
+  * on some way through the branches a wave's read of its partner's record is followed by a write to its own record of the
+    next row with no barrier between: the partner, which reads that record, may not be that far.
+
     python isa_lint.py            # compiles every kernel source to assembly and checks it
 
 It also lists the kernels that spill registers to scratch memory (scratch_ops): the hand-scheduled
@@ -132,6 +137,7 @@ def lint(asm: str) -> list[str]:
     hits += _lint_dot(ins)
     hits += _lint_wide_store(ins)
     hits += _lint_asm_loads(asm)
+    hits += _lint_exchange(asm)
     for (ln, s), (ln2, s2) in zip(ins, ins[1:]):
         if s.startswith(TRANS) and s2.startswith("v_") and not s2.startswith(TRANS) and not s2.startswith("v_mfma"):
             rest = s2.split(None, 1)[1].split(",", 1)
@@ -183,6 +189,71 @@ def _lint_asm_loads(asm: str) -> list[str]:
                     if s.startswith("s_branch"):
                         break
                 j += 1
+    return hits
+
+
+# Per kernel with a record exchange: its reads of the partner's record and its writes of its own, told from the other LDS accesses
+# by their form.  (fta_bwd_dq1w_kernel: the operands that it reads 16 bytes at a time lie multiples of 4 KB apart.)
+EXCHANGES = {
+    re.compile(r"_ZN3fta19fta_bwd_dq1w_kernel"): (re.compile(r"ds_read_b128 .*offset:(0x400|1024|0x800|2048|0xc00|3072)$"), re.compile(r"ds_write_b128 ")),
+}
+
+
+def _kernels(asm: str):
+    """Name and lines (with their numbers) of every kernel of a listing."""
+    name, lines = None, []
+    for ln, line in enumerate(asm.split("\n"), 1):
+        m = re.match(r"(_Z\w+):", line)
+        if m:
+            name, lines = m.group(1), []
+        elif name is not None and ".end_amdhsa_kernel" in line:
+            yield name, lines
+            name = None
+        elif name is not None:
+            lines.append((ln, line.split(";")[0].split("//")[0].strip()))
+
+
+def exchange_kernels(asm: str) -> list[str]:
+    """The kernels of a listing whose record exchange is checked."""
+    return [name for name, _ in _kernels(asm) for k in EXCHANGES if k.match(name)]
+
+
+def _lint_exchange(asm: str) -> list[str]:
+    """Follows every way from a read of the partner's record to the first barrier: no record is written on it."""
+    hits = []
+    for name, lines in _kernels(asm):
+        forms = [f for k, f in EXCHANGES.items() if k.match(name)]
+        if not forms:
+            continue
+        is_read, is_write = forms[0]
+        ins, labels = [], {}
+        for ln, s in lines:
+            if re.match(r"[.\w$]+:$", s):
+                labels[s[:-1]] = len(ins)
+            elif s and not s.startswith("."):
+                ins.append((ln, s))
+        reads = [i for i, (_, s) in enumerate(ins) if is_read.match(s)]
+        if not reads or not any(is_write.match(s) for _, s in ins):
+            hits.append(f"{name}: no record exchange found")
+        for i in reads:
+            seen, todo = set(), [i + 1]
+            while todo:
+                j = todo.pop()
+                while j < len(ins) and j not in seen:
+                    seen.add(j)
+                    ln, s = ins[j]
+                    if s.startswith(("s_barrier", "s_endpgm")):
+                        break
+                    if is_write.match(s):
+                        hits.append(f"{name}: line {ln}: `{s}` may overwrite a record behind line {ins[i][0]}: `{ins[i][1]}` with no barrier between")
+                        break
+                    if s.startswith(("s_branch", "s_cbranch")):
+                        to = labels.get(s.split()[1])
+                        if to is not None:
+                            todo.append(to)
+                        if s.startswith("s_branch"):
+                            break
+                    j += 1
     return hits
 
 

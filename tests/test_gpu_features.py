@@ -603,6 +603,32 @@ def test_dq_at_head_dim_64_tiles_to_the_next_32_keys(L2, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["contiguous", "projection", "ending"])
+@pytest.mark.parametrize("L1,L2", [(20, 577), (17, 513), (19, 640), (20, 700)])
+def test_dq_at_head_dim_64_later_ranges_over_several_rows_and_chunks(L1, L2, layout, dtype):
+    """dQ/dBias at D = 64 of two ranges, 384 + 256 keys (four tiles a slab in the later one: a wave reads its partner's share of a row in the
+    row's last iteration) and 384 + 384: three chunks of several rows each, in every layout that the projections leave; plain, and with the
+    whole later range or its first slab masked.  Every run gives the same bits."""
+    import fta_lib
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, 0.0, 0, 0)
+    plan = fta_lib.describe_plan(1, 2, L1, L2, 64, 0.125, opt)["dq"]
+    assert plan["kernel"].startswith("fta_bwd_dq1w_kernel") and plan["launches"] == 2
+    assert plan["grid"] >= 2 * 2 * ((L2 + 63) // 64)   # (two chunks or more)
+    order = {"contiguous": (0, 1, 2, 3, 4), "projection": (0, 2, 3, 1, 4), "ending": (0, 1, 3, 2, 4)}[layout]
+    q, k, v, b, do = _inputs(1, 2, L1, L2, 64, 46, dtype)
+    q, k, v, do = (t.permute(order).contiguous().permute([order.index(d) for d in range(5)]) for t in (q, k, v, do))
+    assert layout == "contiguous" or not q.is_contiguous()
+    for masked in ((0, 0), (384, L2), (384, 512)):
+        print(f"case later ranges D=64 {L1}x{L2} {layout} {dtype} masked {masked}", flush=True)
+        bm = b.clone()
+        bm[..., masked[0]:masked[1]] = -math.inf
+        got, again = _run(q, k, v, bm, 0.125, do), _run(q, k, v, bm, 0.125, do)
+        _compare(got, _oracle(q, k, v, bm, 0.125, do), dtype, f"later ranges D64 {L1}x{L2} {layout} masked {masked}")
+        for n in got:
+            assert torch.equal(got[n], again[n]), n
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("L1,L2", [(7, 129), (3, 160), (4, 161), (1, 191), (9, 192)])
 def test_forward_at_head_dim_64_of_129_to_192_keys(L1, L2, dtype):
     """One slab of six tiles: two of the eight query blocks beyond the row, whole rows, one key more than a tile; one row,

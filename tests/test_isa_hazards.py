@@ -173,3 +173,23 @@ def test_checker_on_loads_that_the_compiler_does_not_see():
     # one of two ways round the wait
     assert len(isa_lint.lint(load + "\ts_cbranch_execz .LBB0_2\n" + wait.format(0) + ".LBB0_2:\n" + add)) == 1
     assert isa_lint.lint(load + "\ts_branch .LBB0_2\n" + add + ".LBB0_2:\n" + wait.format(0) + add) == []
+
+
+def test_checker_on_records_between_waves():
+    kernel = "_ZN3fta19fta_bwd_dq1w_kernelX:\n{}\ts_endpgm\n\t.end_amdhsa_kernel\n"
+    read, write, barrier = "\tds_read_b128 v[0:3], v9 offset:0x800\n", "\tds_write_b128 v8, a[0:3]\n", "\ts_barrier\n"
+    operand = "\tds_read_b128 v[4:7], v9 offset:0x4000\n"
+    assert isa_lint.exchange_kernels(kernel.format("")) == ["_ZN3fta19fta_bwd_dq1w_kernelX"]
+    assert len(isa_lint.lint(kernel.format(read + operand + write))) == 1
+    assert isa_lint.lint(kernel.format(read + barrier + write)) == []
+    assert isa_lint.lint(kernel.format(barrier + write + operand + barrier + read)) == []
+    # the next row's write, over the back edge of the row loop, and the last row's, behind the loop
+    loop = ".LBB0_1:\n{}" + write + barrier + read + "{}\ts_cbranch_scc1 .LBB0_1\n{}" + write + barrier + read
+    assert isa_lint.lint(kernel.format(loop.format("", barrier, ""))) == []
+    assert isa_lint.lint(kernel.format(loop.format(barrier, "", barrier))) == []
+    assert len(isa_lint.lint(kernel.format(loop.format("", "", barrier)))) == 1
+    assert len(isa_lint.lint(kernel.format(loop.format(barrier, "", "")))) == 1
+    # a kernel that is named but has no exchange in a form that the checker knows
+    assert len(isa_lint.lint(kernel.format(operand + barrier))) == 1
+    # other kernels hand nothing over in this way
+    assert isa_lint.lint(kernel.replace("dq1w", "dkdv").format(read + write)) == []
