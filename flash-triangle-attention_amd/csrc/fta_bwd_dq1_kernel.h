@@ -149,7 +149,10 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
   constexpr bool DEEP = (D == 32);
   constexpr int SYNC_A = DEEP ? TS0 - 2 : TS0 - 1, SYNC_B = SYNC_A + TS1;  // iterations that publish a stage
   // (DEEP with two slabs) iteration in which a wave fetches its partner's share of the previous dQ row:
-  // the share is written during iteration 1, and a stage barrier has to lie between the two
+  // the share is written during iteration 1, and a stage barrier has to lie between the two.  Another one has to lie between the read and
+  // the next write to that record: in the loop the next row's first (SYNC_A, 0 to 2, opens an iteration and iteration 1 writes behind it if it is 0 or
+  // 1; with SYNC_A = 2 the read in iteration 3 has SYNC_B, 5 or 6, behind it).  The last row's share is written behind the
+  // loop: where the read is in the iteration that SYNC_B opens (4, 5 and 6 tiles) the loop has no barrier left, and the epilogue brings one.
   constexpr int XCHG_RD = (SYNC_A >= 2) ? 3 : SYNC_B;
   constexpr int NRD = 2 * KS + 4 * DT;         // LDS reads per iteration
   constexpr int NG = CIN ? 4 : NM - 8;         // fillers per iteration (without CIN: the MFMAs that no vector-ALU pair follows)
@@ -856,6 +859,7 @@ __global__ void __launch_bounds__(256) fta_bwd_dq1_kernel(const BwdParams p) {
     wait_vmem_all();
     old_landed();
   }
+  if constexpr (SK == 2 && XCHG_RD == SYNC_B) __syncthreads();  // (the partner has read the record of the row before)
   split_groups(acc);
   if constexpr (SK == 2) {
     __syncthreads();

@@ -193,8 +193,10 @@ def _lint_asm_loads(asm: str) -> list[str]:
 
 
 # Per kernel with a record exchange: its reads of the partner's record and its writes of its own, told from the other LDS accesses
-# by their form.  (fta_bwd_dq1w_kernel: the operands that it reads 16 bytes at a time lie multiples of 4 KB apart.)
+# by their form.  (fta_bwd_dq1w_kernel: the operands that it reads 16 bytes at a time lie multiples of 4 KB apart.
+# fta_bwd_dq1_kernel<T, 32, 2, ...>: nothing else is moved by pairs of single floats.)
 EXCHANGES = {
+    re.compile(r"_ZN3fta18fta_bwd_dq1_kernelINS_(3F16|4BF16)ELi32ELi2E"): (re.compile(r"ds_read2st64_b32 "), re.compile(r"ds_write2st64_b32 ")),
     re.compile(r"_ZN3fta19fta_bwd_dq1w_kernel"): (re.compile(r"ds_read_b128 .*offset:(0x400|1024|0x800|2048|0xc00|3072)$"), re.compile(r"ds_write_b128 ")),
 }
 

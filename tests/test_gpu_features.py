@@ -591,6 +591,31 @@ def test_backward_tiles_in_steps_of_64(D, L2, mode):
     _compare(got, _oracle(q, k, v, b, sm, do), dtype, f"tiles of 64 {mode} D{D} L{L2}")
 
 
+@pytest.mark.parametrize("mode", ["fp16", "bf16", "bf16 operand pair", "precise"])
+@pytest.mark.parametrize("L1,L2,launches", [(41, 257, 1), (40, 384, 1), (20, 576, 2), (19, 640, 2), (21, 703, 2), (20, 768, 2)])
+def test_dq_at_head_dim_32_in_two_slabs_over_several_rows_and_chunks(L1, L2, launches, mode):
+    """dQ/dBias at D = 32 of four, five and six tiles a slab, where a wave reads its partner's share of a row behind the last barrier of the
+    next one: first and later ranges, several chunks of several rows each.  Every run gives the same bits."""
+    import fta_lib
+    import flash_tt_attn as fta
+    dtype = torch.bfloat16 if mode.startswith("bf16") else torch.float16
+    B, H, sm = 1, 2, 1.3 if mode == "bf16 operand pair" else 1.0 / math.sqrt(32)
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, 0.0, 0, 1 if mode == "precise" else 0)
+    plan = fta_lib.describe_plan(B, H, L1, L2, 32, sm, opt)["dq"]
+    assert plan["kernel"].startswith("fta_bwd_dq1_kernel<32,2>") and plan["launches"] == launches
+    assert plan["grid"] >= 2 * H * ((L2 + 63) // 64)   # (two chunks or more)
+    print(f"case two slabs {mode} D=32 {L1}x{L2}", flush=True)
+    q, k, v, b, do = _inputs(B, H, L1, L2, 32, 47, dtype)
+    fta.PRECISE_BACKWARD = mode == "precise"
+    try:
+        got, again = _run(q, k, v, b, sm, do), _run(q, k, v, b, sm, do)
+    finally:
+        fta.PRECISE_BACKWARD = False
+    _compare(got, _oracle(q, k, v, b, sm, do), dtype, f"two slabs {mode} D32 {L1}x{L2}")
+    for n in got:
+        assert torch.equal(got[n], again[n]), n
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("L2", [160, 161, 255, 288, 289, 415, 449, 545, 641, 1025])
 def test_dq_at_head_dim_64_tiles_to_the_next_32_keys(L2, dtype):

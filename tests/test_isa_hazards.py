@@ -191,5 +191,11 @@ def test_checker_on_records_between_waves():
     assert len(isa_lint.lint(kernel.format(loop.format(barrier, "", "")))) == 1
     # a kernel that is named but has no exchange in a form that the checker knows
     assert len(isa_lint.lint(kernel.format(operand + barrier))) == 1
+    # the kernel for head dim 32, whose records are moved by pairs of floats; with one slab it has none
+    floats = kernel.replace("_ZN3fta19fta_bwd_dq1w_kernelX", "_ZN3fta18fta_bwd_dq1_kernelINS_3F16ELi32ELi2ELi5E")
+    read, write = "\tds_read2st64_b32 v[0:1], v9 offset1:1\n", "\tds_write2st64_b32 v8, v2, v3 offset1:1\n"
+    assert len(isa_lint.lint(floats.format(read + write))) == 1
+    assert isa_lint.lint(floats.format(write + barrier + read + barrier + write)) == []
+    assert isa_lint.lint(floats.replace("Li32ELi2E", "Li32ELi1E").format("")) == []
     # other kernels hand nothing over in this way
     assert isa_lint.lint(kernel.replace("dq1w", "dkdv").format(read + write)) == []
