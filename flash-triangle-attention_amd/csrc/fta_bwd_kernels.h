@@ -128,10 +128,26 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
   const half_t* dobase = p.dout + b * p.dos[0] + h * p.dos[1];
   half_t* dqbase = p.dq + b * p.dqs[0] + h * p.dqs[1];
 
-  // stationary bias tile (fp16 pairs) and dBias accumulators (fp32), accumulator layout; loaded behind the first copies, which fly
-  // meanwhile (so is the bias of the dK/dV kernel: a training pass with dropout at B1 H4 L300 in bf16 248.5 / 247.2 us)
+  // stationary bias tile (fp16 pairs) and dBias accumulators (fp32), accumulator layout
   uint32_t bias_reg[NKT][8];
   floatx16 dbacc[NKT];
+  {
+    const half_t* bbh = p.bias + b * p.bs[0] + h * p.bs[1];
+#pragma unroll
+    for (int tt = 0; tt < NKT; ++tt) {
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) {
+        const int kk = key0 + 4 * hh + tt * 32 + rg * 8;
+        u32x2 v = load_bias4(bbh, p.bs[2], q0 + l32, kk, p.L2);
+        v = beyond_row(u32x2{T::finite2(v[0]), T::finite2(v[1])}, kk, p.L2, T::kBeyond2);
+        bias_reg[tt][2 * rg] = v[0];
+        bias_reg[tt][2 * rg + 1] = v[1];
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dbacc[tt][r] = 0.f;
+    }
+  }
+
   // K/V staging: asynchronous global -> LDS copies into a ring of stage buffers
   const int nstage = nrows * STEPS;
   const int ndma = 2 * dma_rows_count(stage_rows, D, wave, nwaves);  // K/V copies this wave issues per stage
@@ -235,22 +251,6 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dq_kernel(const BwdParams 
     for (int s0 = 0; s0 <= ahead && s0 < nstage; ++s0) stage(s0);
   }
   rowload(0);
-  {
-    const half_t* bbh = p.bias + b * p.bs[0] + h * p.bs[1];
-#pragma unroll
-    for (int tt = 0; tt < NKT; ++tt) {
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const int kk = key0 + 4 * hh + tt * 32 + rg * 8;
-        u32x2 v = load_bias4(bbh, p.bs[2], q0 + l32, kk, p.L2);
-        v = beyond_row(u32x2{T::finite2(v[0]), T::finite2(v[1])}, kk, p.L2, T::kBeyond2);
-        bias_reg[tt][2 * rg] = v[0];
-        bias_reg[tt][2 * rg + 1] = v[1];
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dbacc[tt][r] = 0.f;
-    }
-  }
   wait_vmem_all();
   __syncthreads();
 
@@ -539,6 +539,24 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParam
   // of a lane is fixed, its queries are a bias row apart).
   u32x4 biasA[NJT][2];
   const half_t* bbh = p.bias + b * p.bs[0] + h * p.bs[1];
+  {
+    const int kk = (k0 + l32 < p.L2) ? k0 + l32 : p.L2 - 1;   // (a key beyond the row: never stored)
+#pragma unroll
+    for (int jt = 0; jt < NJT; ++jt) {
+      uint32_t w[8];
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        const int j0 = p.jr0 + jslab * JW + jt * 32 + 8 * (r / 4) + 4 * hh + r % 4;
+        const int ja = (j0 < p.L2) ? j0 : p.L2 - 1, jb = (j0 + 1 < p.L2) ? j0 + 1 : p.L2 - 1;
+        const uint32_t a = *reinterpret_cast<const uint16_t*>(bbh + (int64_t)ja * p.bs[2] + kk);
+        const uint32_t c = *reinterpret_cast<const uint16_t*>(bbh + (int64_t)jb * p.bs[2] + kk);
+        w[r >> 1] = T::finite2(a | (c << 16));
+      }
+      biasA[jt][0] = u32x4{w[0], w[1], w[2], w[3]};
+      biasA[jt][1] = u32x4{w[4], w[5], w[6], w[7]};
+    }
+  }
+
   // Q/dO/lse/delta staging: asynchronous global -> LDS copies into a ring of stage buffers.
   // lse and delta: one copy instruction moves 64 floats x 4 = one slab's JT floats need JT/4 lanes.
   const int nstage = nrows * STEPS;
@@ -640,23 +658,6 @@ __global__ void __launch_bounds__(64 * NW, 2) fta_bwd_dkdv_kernel(const BwdParam
     });
   } else {
     for (int s0 = 0; s0 <= ahead && s0 < nstage; ++s0) stage(s0);
-  }
-  {
-    const int kk = (k0 + l32 < p.L2) ? k0 + l32 : p.L2 - 1;   // (a key beyond the row: never stored)
-#pragma unroll
-    for (int jt = 0; jt < NJT; ++jt) {
-      uint32_t w[8];
-#pragma unroll
-      for (int r = 0; r < 16; r += 2) {
-        const int j0 = p.jr0 + jslab * JW + jt * 32 + 8 * (r / 4) + 4 * hh + r % 4;
-        const int ja = (j0 < p.L2) ? j0 : p.L2 - 1, jb = (j0 + 1 < p.L2) ? j0 + 1 : p.L2 - 1;
-        const uint32_t a = *reinterpret_cast<const uint16_t*>(bbh + (int64_t)ja * p.bs[2] + kk);
-        const uint32_t c = *reinterpret_cast<const uint16_t*>(bbh + (int64_t)jb * p.bs[2] + kk);
-        w[r >> 1] = T::finite2(a | (c << 16));
-      }
-      biasA[jt][0] = u32x4{w[0], w[1], w[2], w[3]};
-      biasA[jt][1] = u32x4{w[4], w[5], w[6], w[7]};
-    }
   }
   wait_vmem_all();
   __syncthreads();
