@@ -570,8 +570,9 @@ def test_forward_rows_of_an_odd_number_of_tiles(L1, L2, tiled, dtype):
                          + [(64, L) for L in (129, 192, 257, 320, 400, 576, 640, 701, 832)])
 def test_backward_tiles_in_steps_of_64(D, L2, mode):
     """Every number of tiles per wave (key ranges of 256 to 512 keys in two slabs, first and later ones: 513, 640, 703, 896
-    and 1024 have later ranges of 256, 320, 384 (1088), 448 and 512; of 256 in one; D = 64: 160 to 256; query ranges of 256 to 512, at D = 64 256 to 384), odd numbers of them (stages of unequal length), groups of 128 queries or keys
-    that end beyond the tiled length, one to four ranges; rows that end inside a tile and whole ones."""
+    and 1024 have later ranges of 256, 320, 384 (1088), 448 and 512; of 256 in one; D = 64: 160 to 256 in one slab up to 384 keys, 256, 384 and 512 in
+    two beyond; query ranges of 256 to 512, at D = 64 without 448), odd numbers of them (stages of unequal length), groups of 128 queries or keys
+    that end beyond the tiled length, one to three ranges; rows that end inside a tile and whole ones."""
     import fta_lib
     import flash_tt_attn as fta
     if D == 64 and mode in ("bf16 operand pair", "precise"):
@@ -617,11 +618,16 @@ def test_dq_at_head_dim_32_in_two_slabs_over_several_rows_and_chunks(L1, L2, lau
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("L2", [160, 161, 255, 288, 289, 415, 449, 545, 641, 1025])
+@pytest.mark.parametrize("L2", [160, 161, 255, 288, 289, 353, 384, 1153, 1281, 1408, 1700, 415, 449, 545, 641, 1025])
 def test_dq_at_head_dim_64_tiles_to_the_next_32_keys(L2, dtype):
-    """dQ/dBias at D = 64 ends its key tiles at the next multiple of 32, dK/dV at its own length: one tile more or less
-    than a whole range, whole rows of an odd number of tiles, the two ranges of 160 below 288, uneven ranges, and a last
-    group of 128 queries that only dK/dV reads to its end.  Chunks of fewer rows than eight at L1 = 5."""
+    """dQ/dBias at D = 64 in one slab ends its key tiles at the next multiple of 32, dK/dV at its own length: one tile more or less
+    than a whole range, whole rows of an odd number of tiles, the two ranges of 160 below 288, uneven ranges (five to seven from 1153 keys
+    on), and a last group of 128 queries that only dK/dV reads to its end.  In two slabs (385 to 1152 keys among these) the tiles end at the
+    next multiple of 128.  Chunks of fewer rows than eight at L1 = 5."""
+    import fta_lib
+    opt = fta_lib.Options(fta_lib.DTYPE_BF16 if dtype == torch.bfloat16 else fta_lib.DTYPE_F16, 0, 0.0, 0, 0)
+    kernel = fta_lib.describe_plan(1, 2, 5, L2, 64, 0.125, opt)["dq"]["kernel"]
+    assert kernel.startswith("fta_bwd_dq1w_kernel" if 384 < L2 <= 1152 else "fta_bwd_dq1_kernel<64,1>")
     print(f"case dq tiles D=64 L2={L2} {dtype}", flush=True)
     q, k, v, b, do = _inputs(1, 2, 5, L2, 64, 44, dtype)
     _compare(_run(q, k, v, b, 0.125, do), _oracle(q, k, v, b, 0.125, do), dtype, f"dq tiles D64 L{L2}")

@@ -113,7 +113,7 @@ def test_head_dim_64_key_and_query_ranges_of_up_to_512(L1, L2, keys, queries):
     _case(2, 2, L1, L2, 64, 0.125, seed=29)
     import fta_lib
     d = fta_lib.describe_plan(2, 2, L1, L2, 64)
-    assert d["dq"]["kernel"].startswith("fta_bwd_dq1") and d["dq"]["launches"] == keys
+    assert d["dq"]["kernel"].startswith("fta_bwd_dq1w_kernel") and d["dq"]["launches"] == keys
     assert d["dkdv"]["kernel"].startswith("fta_bwd_dkdv1_kernel") and d["dkdv"]["launches"] == queries
 
 
@@ -158,12 +158,12 @@ def _masked_bias(b, L2, where, value):
 
 @pytest.mark.parametrize("value", ["-inf", "-1e9", "-60000"])
 @pytest.mark.parametrize("where", ["trailing", "leading", "ragged"])
-@pytest.mark.parametrize("D,L2", [(32, 256), (32, 384), (32, 512), (64, 256), (64, 384), (64, 512)])
+@pytest.mark.parametrize("D,L2", [(32, 256), (32, 384), (32, 512), (64, 256), (64, 384), (64, 512), (64, 640), (64, 768)])
 def test_key_mask_written_into_the_bias(D, L2, where, value):
     """A key-padding mask in the bias (-inf, -1e9 cast to fp16, -60000) on part of every row: the
     masked keys get weight 0 and zero gradients, as upstream (flash_tt_attn.py:78, :344-346,
-    :418-420); everything stays finite and within the usual tolerances.  L2 = 256/512 run the
-    pipelined backward kernels, 384 the general ones."""
+    :418-420); everything stays finite and within the usual tolerances.  All of them run the hand-scheduled backward kernels
+    (640 and 768 keys in two launches; at D=64 their later range ends with masked keys)."""
     B, H, L1, sm = 1, 2, 9, 1.0 / math.sqrt(D)
     print(f"case mask D={D} L2={L2} {where} {value}", flush=True)
     q, k, v, b, do = orc.make_inputs(B, H, L1, L2, D, seed=13, device=DEV)
