@@ -32,8 +32,8 @@
 // us per kernel at 192 x 192 pairs, before and after: proj 69 / 47, out 32 / 26, dout 29 / 28, dx 57 / 48, wgrad 82 / 50; a
 // training pass 352 / 265 (256 x 256: 498 / 394, 321 x 321: 838 / 670), inference 112 / 82 (457 x 457: 505 / 387).  A workgroup there has few
 // rows, so that what it waits for before the first of them counts: with every load that the first row needs asked for at once, row blocks dealt to the
-// workgroups in turn and dx's operands read a step ahead proj 41, out 19, dout 21, dx 40, wgrad 46; a training pass 238 (beside 267; 256 x 256: 383
-// beside 416, 321 x 321 645 beside 690), inference 80 beside 90 (457 x 457: 370 beside 384).
+// workgroups in turn and dx's operands read a step ahead proj 41, out 19, dout 21, dx 40, wgrad 46; a training pass 246 (beside 272; 150 x 150: 181
+// beside 200, 256 x 256: 383 beside 413, 321 x 321: 645 beside 690), inference 73 beside 84 (457 x 457: 374 beside 384).
 //
 // Measured, AlphaFold2's block (C 128, 4 heads of 32) at 384 x 384 pairs in bf16: a training pass 3.64 ms as separate
 // library calls around the attention, 0.47 with these; us per kernel (rocprofv3, median of 40 launches): proj 49, out

@@ -7,7 +7,9 @@ namespace fta {
 // Query ranges of one launch each (a wave's stationary bias^T tile and the stage size are compiled in), in units of 64
 // queries and as even as the row divides: four to eight units.  D = 64 has no instance of seven (14 tiles divide into stages of seven,
 // of which LDS holds no three): seven and six are cut as eight and five, two sevens as eight and six, and three or more ranges that are
-// not equal as ranges of four and five (as before there were wider ones: 1408 keys 25.6 ms a step).
+// not equal, or equal to seven, as ranges of four and five.  That is the slower side: as ranges of four and five / of eight, six and five (ms a
+// step, dQ/dBias the same) B1 H4 1088 keys 12.2 / 11.7, 1153 15.7 / 15.2, 1280 18.3 / 17.7, 1408 25.9 / 24.2, B1 H2 1664 in bf16 22.0 / 20.8,
+// 1792 25.1 / 23.8.
 static int dkdv1_ranges(int L2, int D, int* out) {
   const int units = L2 / 64;
   const int n = even_ranges(units, 8, 64, out);

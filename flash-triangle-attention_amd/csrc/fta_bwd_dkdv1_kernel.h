@@ -22,10 +22,12 @@
 // the two-waves-per-SIMD kernel runs.
 //
 // D = 64 bound: a launch reads K and V and writes dK and dV whole, so that what a row costs beside its tiles is memory: at B2 H8 L512 two
-// launches of 256 queries moved 6.4 GB (two of 967 us), one of 512 moves 3.2 GB (1210 us; without copies, stores and LDS reads, timing only,
-// 930: 20 MFMAs a tile under the power cap).  It takes 128 accumulation registers for bias^T, so that an operand's registers
-// are filled again behind the MFMA that consumes it instead of being held twice (by itself, at 256 queries, within 1 %).  Training steps
-// (us): L512 4235 -> 3800, B1 H4 L701 3357 -> 3060, L1024 in bf16 9470 -> 8590, L1536 30790 -> 29030.
+// launches of 256 queries moved 6.4 GB (2 x 873 us in a kernel trace), one of 512 moves 3.2 GB (1305 us on the same device, 1.30 to 1.34 ms over
+// devices; without copies, stores and LDS reads, timing only, three quarters of that: 20 MFMAs a tile under the power cap).  It takes 128
+// accumulation registers for bias^T, so that an operand's registers are filled again behind the MFMA that consumes it instead of being held twice
+// (by itself within 1 %: 256 keys at B1 H4 in fp16 151.8 / 152.5 us a step, 320 371 / 374, 384 512 / 513).  Training steps (us) before, with
+// this, and with the wide dQ/dBias kernel as well: B2 H8 L512 through transposed views 4435, 3940, 3755; B1 H4 L701 3357, 3060, 3089 (the last on
+// another device), L1024 in bf16 9470, 8590, 8146, L1536 30790, 29030, 26616.
 #pragma once
 #include "fta_kernels.h"
 #include "fta_pipe.h"

@@ -14,9 +14,11 @@ static int dq1_slabs(int L2, int D) { return (D == 64 || L2 <= 256) ? 1 : 2; }
 
 // D = 64, rows of more than 384 keys: ranges of 256, 384 or 512 keys in one workgroup's two slabs, tiled to the next multiple of 128.  Q, dO and
 // O are read, and dQ written, once a range, and a range of up to 256 keys, as below, is half as long: training steps (us), those ranges / these:
-// B2 H8 400 keys 2823 / 2726, 448 in bf16 3170 / 3000, 460 3425 / 3215, 512 3895 / 3610 (dQ/dBias 1750 / 1360); B1 H4 530 1808 / 1652, 640 2293 / 2160,
-// 701 in bf16 3283 / 3109, 1024 8660 / 8000, 1536 29.4 / 27.2 ms.  Three or more ranges that are not equal stay as below (1408 keys: six launches), and
-// so do 257 to 384 keys, whose two ranges of up to 192 the two slabs of one would tile no shorter.
+// B2 H8 400 keys 2823 / 2726, 448 in bf16 3170 / 3000, 460 3425 / 3215, 512 3895 / 3610 (dQ/dBias 2 x 856 / 1408); B1 H4 530 1808 / 1652, 640 2293 / 2160,
+// 701 in bf16 3283 / 3109, 1024 8660 / 8000, 1536 29.4 / 27.2 ms.  257 to 384 keys stay as below: the two slabs of one would tile their two ranges of
+// up to 192 no shorter.  Three or more ranges that are not equal stay as below, too, in five to seven launches, although that is the slower side: as
+// below / in unequal ranges of these (ms a step) B1 H4 1153 keys 15.7 / 15.0, 1280 18.3 / 17.4, 1408 25.9 / 24.2, B1 H2 1664 in bf16 22.0 / 20.8,
+// 1792 25.1 / 23.8.
 static bool plan_dq1w(int B, int H, int L1, int L2, int row, Dq1Plan& pl) {
   const int units = (row + 127) / 128;
   const int n = row > 384 && row <= 512 * kMaxRanges ? even_ranges(units, 4, 128, pl.range) : 0;

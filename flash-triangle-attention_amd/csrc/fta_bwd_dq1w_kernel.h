@@ -13,8 +13,9 @@
 //     read -> next row's write that of iteration 0.  The last row's record is written behind the loop: six and eight tiles have the
 //     barrier of iteration 4 between the read and that, four tiles need one of their own there.
 //
-// Bound: matrix core and power (18 MFMAs a tile), issue (166 instructions) and memory in about equal parts: 1360 us at B2 H8 L512, 1200 cycles a
-// tile.  Two launches over 256 keys each, of workgroups of 128 queries, read Q, dO, O and wrote dQ twice: 2 x 876 us.
+// Bound: matrix core and power (18 MFMAs a tile), issue (166 instructions) and memory in about equal parts: 1.40 to 1.45 ms at B2 H8 L512
+// (averages of kernel traces over devices), 1200 cycles a tile.  Two launches over 256 keys each, of workgroups of 128 queries, read Q, dO, O and
+// wrote dQ twice: 2 x 856 us on the device where this takes 1408.
 #pragma once
 #include "fta_bwd_dq1_kernel.h"
 

@@ -82,7 +82,9 @@ __global__ void __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(D 
   fo.init(lane);
   fx.init(lane);
 
-  // bias (in registers or packed in memory, see above; loaded behind the first row's copies, one latency less at the start: training passes 111.5 / 110.2 us at B4 H8 L128) in the order of the rounds: tile r holds keys of block (wave + r) % NT.  The values are the forward's,
+  // bias (in registers or packed in memory, see above) in the order of the rounds: tile r holds keys of block (wave + r) % NT.  It is
+  // loaded behind the first row's copies, which saves a latency at the start (training passes, in front of them / behind: B4 H8 L128 99.1 / 96.9 us,
+  // B2 H8 L192 in bf16 154.6 / 150.6).  The values are the forward's,
   // of the kernel that made lse (hand-scheduled at D = 32 without dropout, else the general one): where every key of a
   // query is masked the weights are differences to that very floor.
   constexpr bool FWD1 = (D == 32 && !DROP);
